@@ -1,20 +1,23 @@
-"""Build recipe for libfastcache_hip.so (hipcc, gfx950 only).
+"""Build recipe for libfastcache_hip.so (hipcc, gfx950 only) and _host.so (g++, against torch's headers).
 
 ``python -m fastcache_amd.build`` compiles every ``csrc/*.hip`` file into one shared library
-next to this file.  hipcc cross-compiles without a GPU, so the library is built on the
-development host and travels with the source tree.
+next to this file, and ``csrc/fc_host.cpp`` (the host path that takes torch tensors) into a CPython module beside
+it.  hipcc cross-compiles without a GPU, so both are built on the development host and travel with the source tree.
 """
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libfastcache_hip.so"
+HOST_SRC = CSRC / "fc_host.cpp"
+HOST_PATH = PKG_DIR / "_host.so"
 OBJ_DIR = PKG_DIR / "csrc" / "build"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -45,22 +48,52 @@ def _compile_one(src: Path, verbose: bool) -> Path:
     return obj
 
 
-def build_library(verbose: bool = False, jobs: int = 4) -> Path:
-    """Compile and link the library unconditionally; returns its path."""
-    OBJ_DIR.mkdir(parents=True, exist_ok=True)
-    srcs = sources()
-    if not srcs:
-        raise RuntimeError(f"no HIP sources under {CSRC}")
-    with ThreadPoolExecutor(max_workers=jobs) as pool:
-        objs = list(pool.map(lambda s: _compile_one(s, verbose), srcs))
-    tmp = LIB_PATH.with_suffix(".so.tmp")
-    cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
+def _compile_host(verbose: bool) -> Path:
+    import torch
+    from torch.utils import cpp_extension
+    obj = OBJ_DIR / "fc_host.o"
+    includes = [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-isystem{d}" for d in includes),
+           "-c", str(HOST_SRC), "-o", str(obj)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SRC.name}:\n{res.stdout}\n{res.stderr}")
+    return obj
+
+
+def _link(cmd, target: Path, verbose: bool) -> None:
+    tmp = target.with_suffix(".so.tmp")
+    cmd = [*cmd, "-shared", "-fPIC", "-o", str(tmp)]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
-    os.replace(tmp, LIB_PATH)
+    os.replace(tmp, target)
+
+
+def _link_host(obj: Path, verbose: bool) -> None:
+    """The module finds the kernel library beside itself; torch's libraries are loaded before it is imported."""
+    from torch.utils import cpp_extension
+    _link([os.environ.get("CXX", "g++"), str(obj), *(f"-L{d}" for d in cpp_extension.library_paths()), f"-L{PKG_DIR}",
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN"],
+          HOST_PATH, verbose)
+
+
+def build_library(verbose: bool = False, jobs: int = 4) -> Path:
+    """Compile and link the library and the host module unconditionally; returns the library's path."""
+    OBJ_DIR.mkdir(parents=True, exist_ok=True)
+    srcs = sources()
+    if not srcs:
+        raise RuntimeError(f"no HIP sources under {CSRC}")
+    with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_compile_host, verbose)
+        objs = list(pool.map(lambda s: _compile_one(s, verbose), srcs))
+    _link([HIPCC, f"--offload-arch={ARCH}", *map(str, objs), "-Wl,-soname," + LIB_PATH.name], LIB_PATH, verbose)
+    _link_host(host.result(), verbose)
     return LIB_PATH
 
 

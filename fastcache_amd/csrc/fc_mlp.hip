@@ -100,16 +100,17 @@ __device__ __forceinline__ void ml_wave_sync() {
 // RAG: every sequence has its own segment: seg_start_v / seg_len_v / dst_start_v [batch] in device memory; c_rows is
 // then the largest row count any sequence can have (it bounds the loops), and a sequence whose segment gives fewer
 // than min_rows rows is left to the copy kernel below.
+// The body works on ONE layer of one plane: `slayer` / `dlayer` and the weight pointers carry the layer already; a
+// workgroup takes the column groups cg0, cg0 + cg_step, ... below ncg.
 template <int DTYPE, int SRC_T, int DST_T, bool W1R, bool RAG>
-__global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView src, KvView dst, const char* __restrict__ w1,
-                                                            const char* __restrict__ b1, const char* __restrict__ w2,
-                                                            const char* __restrict__ b2, const char* __restrict__ w3,
-                                                            const char* __restrict__ b3, int cf, int seg_start,
-                                                            int c_rows, int dst_start, int wpc, int ncols, int ncg,
-                                                            const int* __restrict__ seg_start_v,
-                                                            const int* __restrict__ seg_len_v,
-                                                            const int* __restrict__ dst_start_v, int min_rows) {
-  extern __shared__ __align__(16) char lds[];
+__device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvView& dst, const char* slayer, char* dlayer,
+                                         const char* __restrict__ w1l, const char* __restrict__ b1l,
+                                         const char* __restrict__ w2l, const char* __restrict__ b2l,
+                                         const char* __restrict__ w3l, const char* __restrict__ b3l, int cf,
+                                         int seg_start, int c_rows, int dst_start, int wpc, int ncols, int ncg, int cg0,
+                                         int cg_step, const int* __restrict__ seg_start_v,
+                                         const int* __restrict__ seg_len_v, const int* __restrict__ dst_start_v,
+                                         int min_rows) {
   char* w1buf = lds;                       // 2 x ML_WBYTES
   char* w2buf = lds + 2 * ML_WBYTES;       // permuted
   char* w3buf = lds + 3 * ML_WBYTES;       // permuted
@@ -118,7 +119,6 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
   char* xsw = lds + 4 * ML_WBYTES + 3 * 128 * 4 + 2 * ML_TBLTOT * 4 + (threadIdx.x >> 6) * ML_XS;
   int* wave_rows = reinterpret_cast<int*>(lds + 4 * ML_WBYTES + 3 * 128 * 4 + 2 * ML_TBLTOT * 4 + ML_WAVES * ML_XS);
 
-  const int l = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, lhalf = lane >> 5;
   const int lq = lane >> 2, lp = lane & 3;   // memory-side layout: row lq (and 16 + lq), 16-byte piece lp of 64 bytes
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
   const int sub = wave % wpc;
   const int H = src.num_kv_heads;
   const int K1 = cf * 128;
-  // the column this wavefront works on; a workgroup takes column groups blockIdx.x, blockIdx.x + gridDim.x, ...
+  // the column this wavefront works on; set per column group
   int col = 0, b = 0, h = 0;
   bool col_ok = false;
 
@@ -167,8 +167,6 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
 
   // ---- resident weights: W2, W3 with the k permutation, biases as fp32 ------------------------------
   {
-    const char* w2l = w2 + (long long)l * 128 * 128 * 2;
-    const char* w3l = w3 + (long long)l * 128 * 128 * 2;
     // 8-byte pieces: piece p of a row holds k = 4p .. 4p+3; inside each group of 4 pieces the order
     // becomes [0, 2, 1, 3]
     for (int i = tid; i < 128 * 32; i += ML_THREADS) {
@@ -180,14 +178,13 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
     }
     for (int i = tid; i < 384; i += ML_THREADS) {
       const int which = i >> 7, n = i & 127;
-      const char* bp = which == 0 ? b1 : which == 1 ? b2 : b3;
-      bias[i] = ml_to_float<DTYPE>(*reinterpret_cast<const unsigned short*>(bp + ((long long)l * 128 + n) * 2));
+      const char* bp = which == 0 ? b1l : which == 1 ? b2l : b3l;
+      bias[i] = ml_to_float<DTYPE>(*reinterpret_cast<const unsigned short*>(bp + n * 2));
     }
   }
 
   // W1 chunk kc covers columns [kc*128, kc*128+128) of W1[l]: 2048 pieces of 16 bytes
   constexpr int WCH = 2048 / ML_THREADS;
-  const char* w1l = w1 + (long long)l * 128 * K1 * 2;
   u32x4 wpre[WCH];
   auto w1_load = [&](int kc) {
 #pragma unroll
@@ -371,14 +368,14 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
       w1_store(1);
     }
   }
-  for (int cg = blockIdx.x; cg < ncg; cg += gridDim.x) {
-    if (cg != (int)blockIdx.x) __syncthreads();   // every wavefront is done with the previous group's tables and W1 buffers
+  for (int cg = cg0; cg < ncg; cg += cg_step) {
+    if (cg != cg0) __syncthreads();   // every wavefront is done with the previous group's tables and W1 buffers
     col = cg * cols_per_wg + wave / wpc;
     col_ok = col < ncols;
     b = col_ok ? col / H : 0;
     h = col_ok ? col - (col / H) * H : 0;
-    sbase = src.base + ((long long)l * src.stride_layer + (long long)h * src.stride_head) * 2 + lp * 16;
-    dbase = dst.base + ((long long)l * dst.stride_layer + (long long)h * dst.stride_head) * 2 + lp * 16;
+    sbase = slayer + (long long)h * src.stride_head * 2 + lp * 16;
+    dbase = dlayer + (long long)h * dst.stride_head * 2 + lp * 16;
     if constexpr (RAG) {
       // The sequence's own segment.  Numbers from device memory are cut to what the host validated: the views'
       // max_seq_len (which their block tables cover) and the launch's row bound.
@@ -413,6 +410,76 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
     // the streaming variant is launched with one column group per workgroup (its groups are long, and the
     // loop would cost it registers it does not have)
     if (!W1R) break;
+  }
+}
+
+template <int DTYPE, int SRC_T, int DST_T, bool W1R, bool RAG>
+__global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView src, KvView dst, const char* __restrict__ w1,
+                                                            const char* __restrict__ b1, const char* __restrict__ w2,
+                                                            const char* __restrict__ b2, const char* __restrict__ w3,
+                                                            const char* __restrict__ b3, int cf, int seg_start,
+                                                            int c_rows, int dst_start, int wpc, int ncols, int ncg,
+                                                            const int* __restrict__ seg_start_v,
+                                                            const int* __restrict__ seg_len_v,
+                                                            const int* __restrict__ dst_start_v, int min_rows) {
+  extern __shared__ __align__(16) char lds[];
+  const long long l = blockIdx.y;
+  mlp_body<DTYPE, SRC_T, DST_T, W1R, RAG>(
+      lds, src, dst, src.base + l * src.stride_layer * 2, dst.base + l * dst.stride_layer * 2, w1 + l * 128 * cf * 256,
+      b1 + l * 256, w2 + l * 128 * 256, b2 + l * 256, w3 + l * 128 * 256, b3 + l * 256, cf, seg_start, c_rows, dst_start,
+      wpc, ncols, ncg, blockIdx.x, gridDim.x, seg_start_v, seg_len_v, dst_start_v, min_rows);
+}
+
+// ---- a list of per-layer tensors, both planes and every segment in ONE launch ---------------------------------
+// A HuggingFace cache is a list of (K, V) tensors, one pair per layer; one prompt of it is little work per tensor (32
+// columns of 288 rows: 12 us of kernel), so what a launch per (layer, plane, segment) costs is the launches.  The
+// source addresses travel in the kernel's arguments (no table upload).  blockIdx.y = (segment, plane, layer); each
+// segment has its own split of the columns, and a segment's remainder rows (or all rows of one too short to compress)
+// are copied behind its compressed rows by the same workgroup: source and destination are different tensors, so
+// nothing has to be ordered.
+#define ML_LIST_LAYERS 64
+#define ML_LIST_SEGS 2
+struct MlpList {
+  const char* src[2][ML_LIST_LAYERS];           // [plane][layer]
+  const char* w[ML_LIST_SEGS][2][6];            // [segment][plane]: w1, b1, w2, b2, w3, b3, all layers stacked
+  int seg_start[ML_LIST_SEGS], c_rows[ML_LIST_SEGS], rem[ML_LIST_SEGS], dst_start[ML_LIST_SEGS];
+  int wpc[ML_LIST_SEGS], ncg[ML_LIST_SEGS], gx[ML_LIST_SEGS];
+};
+
+template <int DTYPE, bool W1R>
+__global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_list_kernel(KvView ksrc, KvView vsrc, KvView kdst, KvView vdst,
+                                                                           MlpList a, int cf, int ncols) {
+  extern __shared__ __align__(16) char lds[];
+  const int L = ksrc.num_layers;
+  const int job = (int)blockIdx.y / L, l = (int)blockIdx.y - job * L;
+  const int seg = job >> 1, p = job & 1;
+  const int gx = a.gx[seg];
+  if ((int)blockIdx.x >= gx) return;
+  const KvView& src = p ? vsrc : ksrc;
+  const KvView& dst = p ? vdst : kdst;
+  const char* slayer = a.src[p][l];
+  char* dlayer = dst.base + (long long)l * dst.stride_layer * 2;
+  const int c = a.c_rows[seg], wpc = a.wpc[seg], ncg = a.ncg[seg];
+  const long long ll = l;
+  if (c > 0)
+    mlp_body<DTYPE, 0, 0, W1R, false>(lds, src, dst, slayer, dlayer, a.w[seg][p][0] + ll * 128 * cf * 256,
+                                      a.w[seg][p][1] + ll * 256, a.w[seg][p][2] + ll * 128 * 256, a.w[seg][p][3] + ll * 256,
+                                      a.w[seg][p][4] + ll * 128 * 256, a.w[seg][p][5] + ll * 256, cf, a.seg_start[seg], c,
+                                      a.dst_start[seg], wpc, ncols, ncg, blockIdx.x, gx, nullptr, nullptr, nullptr, 0);
+  const int rem = a.rem[seg];
+  if (rem > 0) {   // 16 lanes per row
+    const int cols_per_wg = ML_WAVES / wpc, sub = threadIdx.x & 15;
+    const int s0 = a.seg_start[seg] + c * cf, d0 = a.dst_start[seg] + c;
+    for (int cg = blockIdx.x; cg < ncg; cg += gx) {
+      const int c0 = cg * cols_per_wg, rows = min(cols_per_wg, ncols - c0) * rem;
+      for (int i = threadIdx.x >> 4; i < rows; i += ML_THREADS / 16) {
+        const int col = c0 + i / rem, t = i - (i / rem) * rem;
+        const int b = col / src.num_kv_heads, h = col - b * src.num_kv_heads;
+        const long long so = (long long)b * src.stride_batch + (long long)h * src.stride_head + (long long)(s0 + t) * src.stride_token;
+        const long long dof = (long long)b * dst.stride_batch + (long long)h * dst.stride_head + (long long)(d0 + t) * dst.stride_token;
+        *reinterpret_cast<uint4*>(dlayer + dof * 2 + sub * 16) = *reinterpret_cast<const uint4*>(slayer + so * 2 + sub * 16);
+      }
+    }
   }
 }
 
@@ -592,6 +659,100 @@ extern "C" int fc_ccm_mlp_ragged(const fc_kv_view* src, const fc_kv_view* dst, c
                    src->stride_layer == dst->stride_layer && src->stride_batch == dst->stride_batch;
   hipLaunchKernelGGL(mlp_tail_copy_kernel, dim3(src->num_kv_heads, src->batch, src->num_layers), dim3(256), 0, st,
                      fc_make_view(src), fc_make_view(dst), cf, min_rows, c, seg_start, seg_len, dst_start, same);
+  FC_CHECK_LAUNCH(who);
+  return FC_OK;
+}
+
+extern "C" int fc_ccm_mlp_layers(const void* const* k_layers, const void* const* v_layers, const fc_kv_view* k_src,
+                                 const fc_kv_view* v_src, const fc_kv_view* k_dst, const fc_kv_view* v_dst,
+                                 const fc_mlp_weights* weights, int32_t num_segments, const int32_t* seg_start,
+                                 const int32_t* seg_len, const int32_t* dst_start, int32_t cf, int32_t min_rows,
+                                 void* stream) {
+  const char* who = "fc_ccm_mlp_layers";
+  FC_REQUIRE(k_layers && v_layers && k_src && v_src && k_dst && v_dst && weights && seg_start && seg_len && dst_start,
+             FC_EINVAL, "%s: null pointer", who);
+  FC_REQUIRE(num_segments >= 1 && num_segments <= ML_LIST_SEGS, FC_EINVAL, "%s: %d segments (1 or 2)", who, num_segments);
+  FC_REQUIRE(min_rows >= 0, FC_EINVAL, "%s: negative min_rows", who);
+  FC_REQUIRE(k_src->num_layers <= ML_LIST_LAYERS, FC_EUNSUPPORTED, "%s: %d layers (at most %d)", who, k_src->num_layers,
+             ML_LIST_LAYERS);
+  const fc_kv_view* views[2][2] = {{k_src, k_dst}, {v_src, v_dst}};
+  int rc;
+  for (int p = 0; p < 2; ++p)
+    for (int s = 0; s < num_segments; ++s)
+      if ((rc = ml_check(who, views[p][0], views[p][1], &weights[s * 2 + p], cf))) return rc;
+  FC_REQUIRE(!k_src->block_tables && !v_src->block_tables && !k_dst->block_tables && !v_dst->block_tables, FC_EINVAL,
+             "%s: dense tensors only", who);
+  FC_REQUIRE(k_src->dtype == v_src->dtype && k_src->num_layers == v_src->num_layers && k_src->batch == v_src->batch &&
+                 k_src->num_kv_heads == v_src->num_kv_heads,
+             FC_EINVAL, "%s: K and V disagree", who);
+  MlpList a;
+  for (int p = 0; p < 2; ++p)
+    for (int l = 0; l < k_src->num_layers; ++l) {
+      a.src[p][l] = (const char*)(p ? v_layers : k_layers)[l];
+      FC_REQUIRE(a.src[p][l] && ((uintptr_t)a.src[p][l] & 15) == 0, FC_EINVAL, "%s: layer %d not 16-byte aligned", who, l);
+    }
+  const int ncols = k_src->batch * k_src->num_kv_heads;
+  const int lp = 2 * k_src->num_layers;     // (plane, layer) pairs per segment
+  int gmax = 0;
+  for (int s = 0; s < num_segments; ++s) {
+    const int64_t n = seg_len[s], c0 = n / cf;
+    const int c = c0 < min_rows ? 0 : (int)c0;
+    FC_REQUIRE(n >= 0 && seg_start[s] >= 0 && dst_start[s] >= 0 && seg_start[s] + n <= k_src->max_seq_len &&
+                   seg_start[s] + n <= v_src->max_seq_len,
+               FC_EINVAL, "%s: segment %d outside the source", who, s);
+    a.rem[s] = (int)(n - (int64_t)c * cf);
+    FC_REQUIRE((int64_t)dst_start[s] + c + a.rem[s] <= k_dst->max_seq_len &&
+                   (int64_t)dst_start[s] + c + a.rem[s] <= v_dst->max_seq_len,
+               FC_EINVAL, "%s: segment %d outside the destination", who, s);
+    a.seg_start[s] = seg_start[s];
+    a.dst_start[s] = dst_start[s];
+    a.c_rows[s] = c;
+    for (int p = 0; p < 2; ++p) {
+      const fc_mlp_weights& w = weights[s * 2 + p];
+      const void* ws[6] = {w.w1, w.b1, w.w2, w.b2, w.w3, w.b3};
+      for (int i = 0; i < 6; ++i) a.w[s][p][i] = (const char*)ws[i];
+    }
+    // How many wavefronts share a column and how many column groups a workgroup walks: the pair with the fewest
+    // rounds * (groups * time per group + start-up), the same coarse model as the single launch's.
+    const int ncu = ml_compute_units() > 0 ? ml_compute_units() : 256;
+    double best = -1.0;
+    a.wpc[s] = 1;
+    a.ncg[s] = (ncols + ML_WAVES - 1) / ML_WAVES;
+    a.gx[s] = a.ncg[s];
+    for (int wpc = 1; wpc <= ML_WAVES && (wpc == 1 || ML_ROWS * wpc < 2 * c); wpc *= 2) {
+      const int cpw = ML_WAVES / wpc, ncg = (ncols + cpw - 1) / cpw;
+      const int n_iter = (c + ML_ROWS * wpc - 1) / (ML_ROWS * wpc);
+      const double t_group = 1.5 * n_iter * (cf + 2), t_start = 4.0;
+      for (int per = 1; per <= ncg && per <= (cf <= 2 ? 64 : 1); ++per) {
+        const int g = (ncg + per - 1) / per;
+        const long long rounds = ((long long)g * lp + ncu - 1) / ncu;
+        const double cost = (double)rounds * (((ncg + g - 1) / g) * t_group + t_start);
+        if (best < 0 || cost < best) {
+          best = cost;
+          a.wpc[s] = wpc;
+          a.ncg[s] = ncg;
+          a.gx[s] = g;
+        }
+      }
+    }
+    if (c + a.rem[s] > 0 && a.gx[s] > gmax) gmax = a.gx[s];
+  }
+  if (gmax == 0) return FC_OK;
+  FC_REQUIRE(lp * num_segments <= 65535, FC_EUNSUPPORTED, "%s: grid too large", who);
+  dim3 grid(gmax, lp * num_segments);
+  KvView ks = fc_make_view(k_src), vs = fc_make_view(v_src), kd = fc_make_view(k_dst), vd = fc_make_view(v_dst);
+#define ML_LIST(DT, WR)                                                                                              \
+  do {                                                                                                               \
+    FC_ALLOW_LDS((mlp_list_kernel<DT, WR>), ML_LDS);                                                                 \
+    hipLaunchKernelGGL((mlp_list_kernel<DT, WR>), grid, dim3(ML_THREADS), ML_LDS, (hipStream_t)stream, ks, vs, kd, vd, a, \
+                       cf, ncols);                                                                                   \
+  } while (0)
+  if (k_src->dtype == FC_BF16) {
+    if (cf <= 2) ML_LIST(FC_BF16, true); else ML_LIST(FC_BF16, false);
+  } else {
+    if (cf <= 2) ML_LIST(FC_F16, true); else ML_LIST(FC_F16, false);
+  }
+#undef ML_LIST
   FC_CHECK_LAUNCH(who);
   return FC_OK;
 }

@@ -86,19 +86,33 @@ class _CCMBase(nn.Module):
     # -- weights ------------------------------------------------------------------------------
     def _weights(self, group: str, dtype: torch.dtype, device: torch.device):
         """``(w1, b1, w2, b2, w3, b3)`` stacked over layers in nn.Linear layout ``[L, out, in]``, in
-        the KV dtype.  Rebuilt when a parameter changed (version counters) or moved."""
+        the KV dtype.  Rebuilt when a parameter changed (version counters), moved or was replaced: the host module
+        looks at every one of them on each call (about 4 us for 32 layers, 180 us walked in Python)."""
         mods: nn.ModuleList = getattr(self, group)
-        params = [p for m in mods for p in (m[0].weight, m[0].bias, m[3].weight, m[3].bias, m[6].weight, m[6].bias)]
-        key = (dtype, device, tuple(p._version for p in params), tuple(p.data_ptr() for p in params))
+        host = _lib.host()
         hit = self._stacked.get(group)
-        if hit is not None and hit[0] == key:
-            return hit[1]
+        if hit is not None and hit[0] == (dtype, device, len(mods)) and host.unchanged(hit[1]):
+            return hit[2]
         with torch.no_grad():
             packed = tuple(
                 torch.stack([getattr(m[i], name).detach() for m in mods]).to(device=device, dtype=dtype).contiguous()
                 for i in (0, 3, 6) for name in ("weight", "bias"))
-        self._stacked[group] = (key, packed)
+        steps = [(self._modules, group)]
+        for i, m in mods._modules.items():
+            steps.append((mods._modules, i))
+            for j in ("0", "3", "6"):
+                steps.append((m._modules, j))
+                steps += [(m._modules[j]._parameters, name) for name in ("weight", "bias")]
+        watch = host.watch(steps)
+        if watch is None:              # a parametrized Linear computes its weight on each access: nothing to hold on to
+            self._stacked.pop(group, None)
+        else:
+            self._stacked[group] = ((dtype, device, len(mods)), watch, packed)
         return packed
+
+    def _layer_weights(self, group: str, l0: int, l1: int, dtype: torch.dtype, device: torch.device):
+        w = self._weights(group, dtype, device)
+        return w if (l0, l1) == (0, w[0].shape[0]) else tuple(t[l0:l1] for t in w)
 
     def _apply(self, fn, *a, **kw):  # .cuda() / .half() invalidate the stacked copies
         self._stacked = {}
@@ -179,7 +193,7 @@ class _CCMBase(nn.Module):
                     if out is not None or dst != s0:
                         ops.copy_tokens(view, dview, s0, n, dst)
                 else:
-                    w = tuple(t[l0:l1] for t in self._weights(g, kv_cache.dtype, kv_cache.device))
+                    w = self._layer_weights(g, l0, l1, kv_cache.dtype, kv_cache.device)
                     ops.ccm_mlp(view, dview, w, cf, s0, n, dst)
             dst += self._segment_len(n)
         return dst
@@ -202,12 +216,39 @@ class _CCMBase(nn.Module):
             mk = lambda xs: torch.tensor(xs, dtype=torch.int32, device=dev)
             starts, counts, dsts = mk([g[2] for g in segs]), mk([g[3] for g in segs]), mk(dst)
             for view, dview, g in ((views[0], dviews[0], gk), (views[1], dviews[1], gv)):
-                w = tuple(t[l0:l1] for t in self._weights(g, kv_cache.dtype, dev))
+                w = self._layer_weights(g, l0, l1, kv_cache.dtype, dev)
                 ops.ccm_mlp_ragged(view, dview, w, cf, starts, counts, dsts, n_max, self.min_seq_len)
             dst = [d + self._segment_len(g[3]) for d, g in zip(dst, segs)]
         return dst
 
+    def _forward_layers(self, kv_cache: Sequence[LayerKV], segments) -> Optional[List[LayerKV]]:
+        """The whole list in one launch: ``segments`` = ``[(k group, v group, start, length)]`` in token order.  None
+        when the list cannot take that path (tensors of different geometry, more than 64 layers)."""
+        if len(kv_cache) == 0 or len(kv_cache) > len(getattr(self, segments[0][0])):
+            return None
+        k = kv_cache[0][0]
+        _lib.require_gpu(k, "kv_cache")
+        if k.dtype not in (torch.float16, torch.bfloat16):
+            return None
+        segs, weights, dst = [], [], 0
+        for gk, gv, start, n in segments:
+            segs.append((start, n, dst))
+            weights += [self._weights(gk, k.dtype, k.device), self._weights(gv, k.dtype, k.device)]
+            dst += self._segment_len(n)
+        out = _lib.host().ccm_layers(kv_cache, tuple(weights), tuple(segs), dst, self.compression_factor, self.min_seq_len)
+        if out is not None:
+            _lib.note_enqueued()
+        return out
+
     def _forward_split(self, kv_cache: Sequence[LayerKV], it_len: Sequence[int], split: bool) -> List[LayerKV]:
+        if len(kv_cache):
+            S = kv_cache[0][0].shape[2]
+            img = min(int(it_len[0]), S) if split else 0
+            segments = [("compress_ik", "compress_iv", 0, img)] if img else []
+            segments.append(("compress_tk", "compress_tv", img, S - img))
+            out = self._forward_layers(kv_cache, segments)
+            if out is not None:
+                return out
         out: List[LayerKV] = []
         for layer, (k, v) in enumerate(kv_cache):
             _lib.require_gpu(k, "kv_cache")

@@ -282,6 +282,20 @@ int fc_ccm_mlp_ragged(const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp
                       int32_t max_seg_len, int32_t min_rows, void* stream);
 
 /*
+ * The same MLPs over a cache that is a list of per-layer tensors (what `forward(kv_cache, it_len)` of the compressor
+ * modules gets, utils_ccm/module_ccm_v11.py:697-729), both planes and every segment in ONE launch.
+ * k_layers / v_layers: HOST arrays of num_layers device pointers, one dense tensor each, all of the geometry of k_src /
+ * v_src (whose base is not read); k_dst / v_dst: dense, all layers in one allocation each, not overlapping any source.
+ * weights[segment * 2 + plane] (plane 0 = K); segment s compresses source tokens [seg_start[s], + seg_len[s]) to
+ * destination tokens from dst_start[s] on and copies its seg_len % cf remainder behind them; a segment of fewer than
+ * min_rows * cf tokens is copied whole.  At most 64 layers and 2 segments.
+ */
+int fc_ccm_mlp_layers(const void* const* k_layers, const void* const* v_layers, const fc_kv_view* k_src,
+                      const fc_kv_view* v_src, const fc_kv_view* k_dst, const fc_kv_view* v_dst,
+                      const fc_mlp_weights* weights, int32_t num_segments, const int32_t* seg_start,
+                      const int32_t* seg_len, const int32_t* dst_start, int32_t cf, int32_t min_rows, void* stream);
+
+/*
  * Expected-attention scores: attention each key can expect from future queries whose distribution is
  * Gaussian with mean mean_query[layer][b][hq][128] and covariance cov_query[layer][b][hq][128][128]
  * (fp32, contiguous; cov_query may be NULL = mean only).  For the keys past the first n_sink of a sequence

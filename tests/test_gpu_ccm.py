@@ -210,3 +210,38 @@ def test_ccm_mlp_ragged_clamps_device_side_numbers(dev):
     assert bool((got[:, :, spare] == 9.0).all())
     assert torch.equal(got[1], case.kv_cache[1])                 # the V plane was not part of the call
     assert torch.equal(got[0, :, case.block_tables[1]], case.kv_cache[0, :, case.block_tables[1]])   # start past the view: nothing
+
+
+@pytest.mark.parametrize("dtype,cf,S,img,B,min_seq_len", [
+    (torch.float16, 2, 623, 576, 1, 1),     # remainder behind both segments' rows, image and text
+    (torch.bfloat16, 5, 4, 0, 3, 1),        # shorter than the factor: copied whole
+    (torch.bfloat16, 2, 64, 63, 2, 2),      # text of one token passed through, one full 32-row tile
+    (torch.float16, 5, 1285, 0, 1, 1),      # streamed W1, several wavefronts per column, last tile ragged
+    (torch.float16, 1, 33, 1, 5, 1),        # factor 1: one row past a tile
+])
+def test_ccm_forward_over_a_list_is_one_launch(dev, dtype, cf, S, img, B, min_seq_len):
+    """The compressor module on a list of per-layer tensors (permuted views, as a runner's extraction hands out):
+    one entry-point call for all layers, planes and segments, equal to the oracle's forward; a list whose tensors do
+    not share a geometry goes layer by layer and gives the same bits."""
+    from types import SimpleNamespace
+    from fastcache_amd.utils_ccm import KVCacheLinearDecoupleCompressor
+    L, H = 3, 3
+    cfg = SimpleNamespace(text_config=SimpleNamespace(num_hidden_layers=L, num_key_value_heads=H, hidden_size=H * 128))
+    torch.manual_seed(11)
+    module = KVCacheLinearDecoupleCompressor(cfg, compression_factor=cf, min_seq_len=min_seq_len)
+    sd = {k: v.clone() for k, v in module.state_dict().items()}
+    module = module.to(dev).to(dtype).eval()
+    g = torch.Generator().manual_seed(2)
+    hf = [tuple(torch.randn(B, S, H, 128, generator=g).to(dtype).transpose(1, 2) for _ in range(2)) for _ in range(L)]
+    ref = occm.linear_decouple_forward(hf, [img, S - img], sd, cf, min_seq_len)
+    on_gpu = [tuple(t.to(dev) for t in kv) for kv in hf]
+    before = _lib.enqueue_count()
+    out = module(on_gpu, [img, S - img])
+    assert _lib.enqueue_count() == before + 1
+    mixed = [(on_gpu[0][0].contiguous(), on_gpu[0][1])] + on_gpu[1:]
+    one_by_one = module(mixed, [img, S - img])
+    for (gk, gv), (rk, rv), (sk, sv) in zip(out, ref, one_by_one):
+        assert gk.is_contiguous() and gk.shape == rk.shape
+        assert torch.equal(gk, sk) and torch.equal(gv, sv)
+        assert_mlp_close(gk.cpu(), rk, dtype)
+        assert_mlp_close(gv.cpu(), rv, dtype)
