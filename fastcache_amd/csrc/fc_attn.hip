@@ -417,6 +417,296 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
   *o = da_pack<DTYPE>(acc / L);
 }
 
+// ---- few columns: one short chain per workgroup ----------------------------------------------------------------------
+// A step of a few sequences is latency, not bandwidth: three users of 300 to 900 tokens move 3.4 MB a layer, and the
+// split kernel spent 11.3 us on it, the merge 3.3 and the append 1.9, each behind the one before (bf16, 28 query heads on
+// 4).  Here a workgroup of eight wavefronts owns a range of a (sequence, kv head) column, the whole context where that is
+// short: the wavefronts take the 32-token tiles in turn, K and V of the first tile (and K of the second) are requested
+// at once instead of K before V, every wavefront carries its own running softmax and no phase waits for the workgroup,
+// and the eight are merged through LDS.  The step's new K and V rows may be appended by the same workgroups (k_new).
+//   S^T[key][head] = K Q^T  on v_mfma_f32_16x16x32: the A operand (16 keys x 64 contiguous bytes per instruction)
+//                           comes straight from memory; the lane then owns ONE head and 8 keys of the tile, so maxima
+//                           and sums run over its registers and two lane exchanges;
+//   O^T[dim][head] = V^T P^T: the probabilities are already the B operand (keys in the order the accumulator gives
+//                           them); V goes through the wavefront's 8 KB of LDS and is read transposed, 2 bytes at a time.
+// Probabilities enter as a sum of 16-bit operands in the cache dtype: two (as the split kernel does for 5 to 8 heads), or
+// three for bf16 groups of up to 4 heads, where the split kernel multiplies in fp32.
+#define DC_WAVES 8
+#define DC_THREADS (DC_WAVES * 64)
+#define DC_HEADS 16
+#define DC_PSTRIDE 132                                             // floats per partial output row (padded against bank conflicts)
+#define DC_VROW 272                                                // LDS bytes per V row: 4 rows apart = 64 bytes apart in banks
+#define DC_STAGE (DA_TILE * DC_VROW)
+#define DC_PART (DC_WAVES * DC_STAGE)                              // V stages, then the partial outputs
+#define DC_LDS (DC_PART + DC_WAVES * DC_HEADS * 8)
+static_assert(DC_PART >= DC_WAVES * DC_HEADS * DC_PSTRIDE * 4, "the partial outputs share the V stages' memory");
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned da_u32x4 __attribute__((ext_vector_type(4)));   // native vector: arrays of it stay in registers
+
+// C[16][16] += A[16][32] * B[32][16]: lane (row or column l % 16, quarter l / 16) holds k = quarter * 8 .. + 7; result:
+// column l % 16, rows quarter * 4 + i
+template <int DTYPE>
+__device__ __forceinline__ f32x4 da_mfma16(const uint4& a, const uint4& b, f32x4 c) {
+  if constexpr (DTYPE == FC_BF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+// two floats -> packed storage dtype, round to nearest even, in one conversion instruction
+template <int DTYPE>
+__device__ __forceinline__ unsigned da_pack2(float x, float y) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  const f32x2 v = {x, y};
+  if constexpr (DTYPE == FC_BF16) return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+  else return __builtin_bit_cast(unsigned, __builtin_convertvector(v, f16x2));
+}
+
+// 8 floats -> 8 values of the storage dtype; the floats keep what the rounding left
+template <int DTYPE>
+__device__ __forceinline__ uint4 da_split8(float (&p)[8]) {
+  unsigned w[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    w[e] = da_pack2<DTYPE>(p[2 * e], p[2 * e + 1]);
+    p[2 * e] -= DTYPE == FC_BF16 ? __uint_as_float(w[e] << 16) : fc_half_to_float((unsigned short)(w[e] & 0xffff));
+    p[2 * e + 1] -= DTYPE == FC_BF16 ? __uint_as_float(w[e] & 0xffff0000u) : fc_half_to_float((unsigned short)(w[e] >> 16));
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+struct DaAppend {                 // the step's new rows, one per sequence (k_new null: nothing to append)
+  const char *k_new, *v_new;
+  long long k_stride, v_stride;   // bytes between sequences; heads are adjacent
+  const int* slots;               // flat cache slot per sequence, negative = skip
+};
+
+template <int DTYPE, int TERMS, bool PAGED>
+__global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc, KvView vc, int layer,
+                                                                      const char* __restrict__ q, int Hq,
+                                                                      const int* __restrict__ lens, float c,
+                                                                      char* __restrict__ out, DaAppend ap, int chunk,
+                                                                      float* __restrict__ part_o,
+                                                                      float* __restrict__ part_ml, int max_splits) {
+  extern __shared__ __align__(16) char smem[];
+  const int b = blockIdx.y;
+  const int G = Hq / kc.num_kv_heads, gtiles = (G + DC_HEADS - 1) / DC_HEADS;
+  const int h = blockIdx.x / gtiles, g0 = (blockIdx.x - h * gtiles) * DC_HEADS;
+  const int ng = min(G - g0, DC_HEADS);
+  const int tid = threadIdx.x, lane = tid & 63, l15 = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // PAGED: both views are, and a sequence's table fits one entry per lane; otherwise both are dense
+  int ktbl = 0, vtbl = 0;
+  if constexpr (PAGED) {
+    ktbl = kc.block_tables[(long long)b * kc.table_stride + min(lane, kc.table_stride - 1)];
+    vtbl = vc.block_tables[(long long)b * vc.table_stride + min(lane, vc.table_stride - 1)];
+  }
+  int len = __builtin_amdgcn_readfirstlane(lens[b]);
+  len = max(min(len, kc.max_seq_len), 0);
+  const int slot = ap.k_new ? __builtin_amdgcn_readfirstlane(ap.slots[b]) : -1;
+  const int t0 = (int)blockIdx.z * chunk;
+  if (t0 >= len && blockIdx.z != 0) return;
+  const int end = min(len, t0 + chunk);
+  // the query heads as B operand; columns past the group are zero
+  uint4 qf[4];
+  {
+    const bool ok = l15 < ng;
+    const char* qp = q + (((long long)b * Hq + (h * G + g0 + (ok ? l15 : 0))) * FC_HEAD_DIM + qd * 8) * 2;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qf[ks] = ok ? *reinterpret_cast<const uint4*>(qp + ks * 64) : make_uint4(0, 0, 0, 0);
+  }
+  const char* kbase = kc.base + ((long long)layer * kc.stride_layer + (long long)h * kc.stride_head) * 2;
+  const char* vbase = vc.base + ((long long)layer * vc.stride_layer + (long long)h * vc.stride_head) * 2;
+  if (PAGED && slot >= 0) {
+    // The new row is written by the workgroup whose range it lies in, which then has to see it land before it reads
+    // it back, and by the last one of the sequence (it usually lies right behind the range; writing it twice is harmless).
+    const int page = slot >> kc.block_shift, at = slot & (kc.block_size - 1);
+    const int pos = (lane << kc.block_shift) + at;
+    const bool inside = __ballot(ktbl == page && pos >= t0 && pos < end && lane < kc.table_stride) != 0ull;
+    if ((inside || end == len) && tid < 32) {
+      const bool is_v = tid >= 16;
+      const long long koff = (long long)page * kc.stride_block + (long long)at * kc.stride_token;
+      const long long voff = (long long)page * vc.stride_block + (long long)at * vc.stride_token;
+      char* dst = is_v ? const_cast<char*>(vbase) + voff * 2 : const_cast<char*>(kbase) + koff * 2;
+      const char* src = is_v ? ap.v_new + (long long)b * ap.v_stride : ap.k_new + (long long)b * ap.k_stride;
+      *reinterpret_cast<uint4*>(dst + l15 * 16) = *reinterpret_cast<const uint4*>(src + (long long)h * FC_HEAD_DIM * 2 + l15 * 16);
+    }
+    if (inside) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
+  }
+  unsigned short* orow = reinterpret_cast<unsigned short*>(out) + ((long long)b * Hq + h * G + g0) * FC_HEAD_DIM;
+  if (len <= 0) {       // with several workgroups per column the merge writes the zeros
+    if (max_splits == 1)
+      for (int i = tid; i < ng * FC_HEAD_DIM; i += DC_THREADS) orow[i] = 0;
+    return;
+  }
+
+  const unsigned ktok = (unsigned)kc.stride_token * 2, vtok = (unsigned)vc.stride_token * 2;
+  auto tile_base = [&](const KvView& v, const char* base, int s0, int tbl) {
+    if constexpr (!PAGED) return base + ((long long)b * v.stride_batch + (long long)s0 * v.stride_token) * 2;
+    const int blk = max(__builtin_amdgcn_readlane(tbl, s0 >> v.block_shift), 0);
+    return base + ((long long)blk * v.stride_block + (long long)(s0 & (v.block_size - 1)) * v.stride_token) * 2;
+  };
+  // Rows past the end of the sequence re-read its last row; their logits are masked.  The scheduling barriers keep
+  // the loads from moving up before the tile their registers held has been used up.
+  auto load_k = [&](da_u32x4 (&kf)[8], int tile) {
+    const int s0 = t0 + tile * DA_TILE, rmax = end - 1 - s0;
+    const char* kg = tile_base(kc, kbase, s0, ktbl);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      const unsigned o = (unsigned)min(kb * 16 + l15, rmax) * ktok + qd * 16;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) kf[kb * 4 + ks] = *reinterpret_cast<const da_u32x4*>(kg + o + ks * 64);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto load_v = [&](da_u32x4 (&vf)[8], int tile) {
+    const int s0 = t0 + tile * DA_TILE, rmax = end - 1 - s0;
+    const char* vg = tile_base(vc, vbase, s0, vtbl) + l15 * 16;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const unsigned o = (unsigned)min(4 * u + qd, rmax) * vtok;
+      vf[u] = *reinterpret_cast<const da_u32x4*>(vg + o);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  float m = -INFINITY, l = 0.f;      // of head l15: the maximum is the tile group's, the sum this lane's keys'
+  f32x4 o[8];
+#pragma unroll
+  for (int db = 0; db < 8; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  char* vst = smem + wave * DC_STAGE;
+  char* v_put = vst + qd * DC_VROW + l15 * 16;                    // row 4 u + qd: u * 4 * DC_VROW further
+  const char* v_get = vst + 4 * qd * DC_VROW + l15 * 2;           // key 4 qd + j (and 16 further), dimension db * 16 + l15
+  const int tiles = (end - t0 + DA_TILE - 1) / DA_TILE, last = tiles - 1;
+  // One tile: its logits, its V rows into LDS; then the next V tile and the K tile after the next start loading into
+  // the registers that became free (past the last tile they re-read it: unconditional loads keep the tiles in registers).
+  auto use_tile = [&](da_u32x4 (&kf)[8], da_u32x4 (&vf)[8], int tile) {
+    f32x4 s[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) s[kb] = da_mfma16<DTYPE>(__builtin_bit_cast(uint4, kf[kb * 4 + ks]), qf[ks], s[kb]);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) *reinterpret_cast<da_u32x4*>(v_put + u * 4 * DC_VROW) = vf[u];
+    if (tile + DC_WAVES < tiles) {
+      load_v(vf, tile + DC_WAVES);
+      load_k(kf, min(tile + 2 * DC_WAVES, last));
+    }
+    float p[8];
+    const int live = end - t0 - tile * DA_TILE;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int key = (e >> 2) * 16 + qd * 4 + (e & 3);
+      p[e] = key < live ? s[e >> 2][e & 3] * c : -INFINITY;
+    }
+    float mx = p[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) mx = fmaxf(mx, p[e]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mn = fmaxf(m, mx);              // finite: a tile that is walked holds at least one live key
+    const float alpha = __builtin_amdgcn_exp2f(m - mn);
+    m = mn;
+    float sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      p[e] = __builtin_amdgcn_exp2f(p[e] - mn);
+      sum += p[e];
+    }
+    l = fmaf(l, alpha, sum);
+    uint4 pt[TERMS];
+#pragma unroll
+    for (int t = 0; t < TERMS; ++t) pt[t] = da_split8<DTYPE>(p);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // this wavefront's V rows before its transposed reads of them
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+      unsigned w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const char* r = v_get + ((e >> 1) * 16 + (2 * e & 3)) * DC_VROW + db * 32;
+        w[e] = (unsigned)*reinterpret_cast<const unsigned short*>(r) |
+               ((unsigned)*reinterpret_cast<const unsigned short*>(r + DC_VROW) << 16);
+      }
+      const uint4 vt = make_uint4(w[0], w[1], w[2], w[3]);
+      o[db] *= alpha;
+#pragma unroll
+      for (int t = 0; t < TERMS; ++t) o[db] = da_mfma16<DTYPE>(vt, pt[t], o[db]);
+      // not more transposed reads in flight than registers beside the tiles hold
+      if ((db & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the reads before the next tile's rows
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+
+  {
+    da_u32x4 ka[8], kb[8], va[8];
+    load_k(ka, min(wave, last));
+    load_v(va, min(wave, last));
+    if (wave + DC_WAVES < tiles) load_k(kb, wave + DC_WAVES);
+    for (int t = wave; t < tiles; t += 2 * DC_WAVES) {
+      use_tile(ka, va, t);
+      if (t + DC_WAVES >= tiles) break;
+      use_tile(kb, va, t + DC_WAVES);
+    }
+  }
+
+  // ---- the eight wavefronts' results into one ---------------------------------------------------------------------
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  float2* ml = reinterpret_cast<float2*>(smem + DC_PART);   // [wavefront][head]: maximum, sum
+  if (qd == 0) ml[wave * DC_HEADS + l15] = make_float2(m, l);
+  __syncthreads();                                         // also: every wavefront is done with its V rows
+  float M = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < DC_WAVES; ++w) M = fmaxf(M, ml[w * DC_HEADS + l15].x);
+  float* part = reinterpret_cast<float*>(smem);
+  {
+    const float wgt = __builtin_amdgcn_exp2f(m - M);        // 0 for a wavefront without tiles
+    if (l15 < ng) {
+#pragma unroll
+      for (int db = 0; db < 8; ++db)
+        *reinterpret_cast<f32x4*>(part + (wave * DC_HEADS + l15) * DC_PSTRIDE + db * 16 + qd * 4) = o[db] * wgt;
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < ng * FC_HEAD_DIM; i += DC_THREADS) {
+    const int g = i / FC_HEAD_DIM, d = i - g * FC_HEAD_DIM;
+    float mg = -INFINITY, lg = 0.f, acc = 0.f;
+#pragma unroll
+    for (int w = 0; w < DC_WAVES; ++w) mg = fmaxf(mg, ml[w * DC_HEADS + g].x);
+#pragma unroll
+    for (int w = 0; w < DC_WAVES; ++w) {
+      const float2 x = ml[w * DC_HEADS + g];
+      lg = fmaf(__builtin_amdgcn_exp2f(x.x - mg), x.y, lg);
+      acc += part[(w * DC_HEADS + g) * DC_PSTRIDE + d];
+    }
+    if (max_splits == 1) {
+      orow[i] = da_pack<DTYPE>(acc / lg);
+    } else {
+      const long long at = ((long long)b * Hq + h * G + g0 + g) * max_splits + blockIdx.z;
+      part_o[at * FC_HEAD_DIM + d] = acc;
+      if (d == 0) {
+        part_ml[at * 2] = mg;
+        part_ml[at * 2 + 1] = lg;
+      }
+    }
+  }
+}
+
 // ---- append / advance ----------------------------------------------------------------------------------
 template <int EB>
 __global__ __launch_bounds__(256) void store_kv_kernel(KvView kc, KvView vc, const char* __restrict__ k_new,
@@ -457,6 +747,79 @@ __global__ __launch_bounds__(256) void store_slots_kernel(const char* __restrict
 __global__ void advance_lens_kernel(int* lens, int n, int delta) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n && lens[i] >= 0) lens[i] += delta;
+}
+
+// A step's inputs into the static buffers of a captured graph, whole: rows [layer][sequence] of q, k and v into buffers
+// of max_batch sequences per layer, and slots, lengths and tables with the padding rows reset (slot -1, length 0, table
+// 0).  One launch instead of the nine fills and copies of a few microseconds each that stood before every replay.
+struct StageRows {
+  const uint4* src;
+  uint4* dst;
+  long long src_layer, src_row, dst_layer;   // in 16-byte pieces; destination rows are adjacent
+  int pieces;                                // per row
+};
+__global__ __launch_bounds__(256) void stage_decode_kernel(StageRows q, StageRows k, StageRows v, int layers, int bs,
+                                                           const int* __restrict__ slots, const int* __restrict__ lens,
+                                                           const int* __restrict__ tables, int width,
+                                                           int* __restrict__ g_slots, int* __restrict__ g_lens,
+                                                           int* __restrict__ g_tables, int max_bs, int g_width) {
+  const long long step = (long long)gridDim.x * 256;
+  const int per_row = q.pieces + k.pieces + v.pieces;
+  const long long n = (long long)layers * bs * per_row;
+  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n; i += step) {
+    const long long row = i / per_row;
+    int p = (int)(i - row * per_row);
+    const int l = (int)(row / bs), b = (int)(row - (long long)l * bs);
+    if (p < q.pieces) {
+      q.dst[l * q.dst_layer + (long long)b * q.pieces + p] = q.src[l * q.src_layer + b * q.src_row + p];
+    } else if ((p -= q.pieces) < k.pieces) {
+      k.dst[l * k.dst_layer + (long long)b * k.pieces + p] = k.src[l * k.src_layer + b * k.src_row + p];
+    } else {
+      p -= k.pieces;
+      v.dst[l * v.dst_layer + (long long)b * v.pieces + p] = v.src[l * v.src_layer + b * v.src_row + p];
+    }
+  }
+  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < (long long)max_bs * g_width; i += step) {
+    const int b = (int)(i / g_width), j = (int)(i - (long long)b * g_width);
+    g_tables[i] = b < bs && j < width ? tables[(long long)b * width + j] : 0;
+    if (j == 0) {
+      g_slots[b] = b < bs ? slots[b] : -1;
+      g_lens[b] = b < bs ? lens[b] : 0;
+    }
+  }
+}
+
+extern "C" int fc_stage_decode(const void* q, int64_t q_layer, int64_t q_row, const void* k, int64_t k_layer, int64_t k_row,
+                               const void* v, int64_t v_layer, int64_t v_row, int32_t num_layers, int32_t batch,
+                               int32_t q_elems, int32_t kv_elems, int32_t dtype, const int32_t* slots,
+                               const int32_t* context_lens, const int32_t* tables, int32_t table_width, void* q_static,
+                               void* k_static, void* v_static, int32_t* slots_static, int32_t* lens_static,
+                               int32_t* tables_static, int32_t max_batch, int32_t max_width, void* stream) {
+  const char* who = "fc_stage_decode";
+  FC_REQUIRE(q && k && v && slots && context_lens && tables && q_static && k_static && v_static && slots_static &&
+                 lens_static && tables_static,
+             FC_EINVAL, "%s: null pointer", who);
+  FC_REQUIRE(dtype == FC_F32 || dtype == FC_F16 || dtype == FC_BF16, FC_EINVAL, "%s: unknown dtype %d", who, dtype);
+  FC_REQUIRE(num_layers > 0 && batch > 0 && batch <= max_batch && table_width > 0 && table_width <= max_width && q_elems > 0 &&
+                 kv_elems > 0,
+             FC_EINVAL, "%s: bad sizes", who);
+  const int eb = fc_elem_bytes(dtype);
+  const int64_t all = (q_layer | q_row | k_layer | k_row | v_layer | v_row | q_elems | kv_elems) * eb;
+  FC_REQUIRE((all & 15) == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)q_static | (uintptr_t)k_static |
+                                  (uintptr_t)v_static) & 15) == 0,
+             FC_EINVAL, "%s: rows, strides and pointers must be multiples of 16 bytes", who);
+  const auto rows = [&](const void* src, int64_t layer, int64_t row, void* dst, int elems) {
+    return StageRows{(const uint4*)src, (uint4*)dst, layer * eb / 16, row * eb / 16, (long long)max_batch * elems * eb / 16,
+                     elems * eb / 16};
+  };
+  const long long n = (long long)num_layers * batch * (q_elems + 2 * kv_elems) * eb / 16;
+  const unsigned grid = (unsigned)(n / 256 + 1 < 1024 ? n / 256 + 1 : 1024);
+  hipLaunchKernelGGL(stage_decode_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream,
+                     rows(q, q_layer, q_row, q_static, q_elems), rows(k, k_layer, k_row, k_static, kv_elems),
+                     rows(v, v_layer, v_row, v_static, kv_elems), num_layers, batch, slots, context_lens, tables, table_width,
+                     slots_static, lens_static, tables_static, max_batch, max_width);
+  FC_CHECK_LAUNCH(who);
+  return FC_OK;
 }
 
 extern "C" int fc_store_kv(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* k_new,
@@ -529,10 +892,52 @@ static int da_compute_units() {
   return n;
 }
 
+// A 32-token tile never straddles two pages and its byte offsets fit 32 bits.
+static bool da_tile_in_page(const fc_kv_view* v) {
+  return v->stride_token >= 0 && v->stride_token < (1 << 24) &&
+         (v->block_tables == nullptr || (v->block_size >= DA_TILE && (v->block_size & (v->block_size - 1)) == 0));
+}
+
+// Tokens per workgroup of the column kernel, 0 = the launch does not take it.  Only launches whose workgroups are all
+// resident at once (one per compute unit: registers) do: beyond that bandwidth counts and the split kernel streams
+// better (128 columns of 1024 tokens: 19.4 us a layer against 19.6 to 23).  One 32-token tile per wavefront, 256 tokens, is
+// the shortest chain (a second tile costs about 3 us, a merge 3.5): 12 columns of 1024 tokens 13.2 -> 10.1 us, of 256
+// tokens without a merge 7.1, 48 columns of 1024 tokens 16.9 -> 13.0.  Where 256 would be too many workgroups, columns
+// short enough for one workgroup each still gain by not being merged: 192 columns of 512 tokens 16.7 -> 15.4 us, 256 of
+// 768 tokens 23.6 -> 22.5.
+#define DC_ONE 768
+static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
+  const int G = num_q_heads / k->num_kv_heads;
+  const long long cols = (long long)k->num_kv_heads * ((G + DC_HEADS - 1) / DC_HEADS) * k->batch;
+  const long long slots = da_compute_units() > 0 ? da_compute_units() : 256;
+  const auto pages_ok = [](const fc_kv_view* x) {       // one block-table entry per lane
+    return x->block_tables == nullptr || (x->max_seq_len - 1) / x->block_size < FC_WAVE;
+  };
+  if ((k->block_tables == nullptr) != (v->block_tables == nullptr) || k->max_seq_len <= 0 || !da_tile_in_page(k) ||
+      !da_tile_in_page(v) || !pages_ok(k) || !pages_ok(v))
+    return 0;
+  const int chunk = DC_WAVES * DA_TILE;
+  if (cols * ((k->max_seq_len + chunk - 1) / chunk) <= slots) return chunk;
+  return cols <= slots && k->max_seq_len <= DC_ONE ? DC_ONE : 0;
+}
+
+static int da_merge(const char* who, const fc_kv_view* k_cache, const float* part_o, const float* part_ml,
+                    const int32_t* context_lens, int num_q_heads, int splits, int chunk, void* out, void* stream) {
+  dim3 grid(num_q_heads, k_cache->batch);
+  if (k_cache->dtype == FC_BF16)
+    hipLaunchKernelGGL((decode_merge_kernel<FC_BF16>), grid, dim3(FC_HEAD_DIM), 0, (hipStream_t)stream, part_o, part_ml,
+                       context_lens, k_cache->max_seq_len, num_q_heads, splits, chunk, (char*)out);
+  else
+    hipLaunchKernelGGL((decode_merge_kernel<FC_F16>), grid, dim3(FC_HEAD_DIM), 0, (hipStream_t)stream, part_o, part_ml,
+                       context_lens, k_cache->max_seq_len, num_q_heads, splits, chunk, (char*)out);
+  FC_CHECK_LAUNCH(who);
+  return FC_OK;
+}
+
 // Checks and launches shared by the entry points; `workspace` is a device address.
 static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t layer,
                       const void* q, void* out, int32_t num_q_heads, const int32_t* context_lens, float scale,
-                      void* workspace, int64_t workspace_bytes, void* stream) {
+                      void* workspace, int64_t workspace_bytes, void* stream, const DaAppend* append = nullptr) {
   int rc;
   if ((rc = fc_check_view(k_cache, who)) || (rc = fc_check_view(v_cache, who))) return rc;
   FC_REQUIRE(k_cache->dtype == v_cache->dtype && k_cache->num_layers == v_cache->num_layers &&
@@ -541,10 +946,47 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
              FC_EINVAL, "%s: K and V views disagree", who);
   FC_REQUIRE(k_cache->dtype == FC_F16 || k_cache->dtype == FC_BF16, FC_EUNSUPPORTED, "%s: fp16/bf16 caches only", who);
   FC_REQUIRE(layer >= 0 && layer < k_cache->num_layers, FC_EINVAL, "%s: layer %d out of range", who, layer);
-  FC_REQUIRE(q && out && context_lens && workspace, FC_EINVAL, "%s: null pointer", who);
-  FC_REQUIRE((((uintptr_t)q | (uintptr_t)workspace) & 15) == 0, FC_EINVAL, "%s: q/workspace not 16-byte aligned", who);
   FC_REQUIRE(num_q_heads > 0 && num_q_heads % k_cache->num_kv_heads == 0, FC_EINVAL,
              "%s: num_q_heads %d not a multiple of num_kv_heads %d", who, num_q_heads, k_cache->num_kv_heads);
+  FC_REQUIRE(q && out && context_lens, FC_EINVAL, "%s: null pointer", who);
+  const int column = da_column_chunk(k_cache, v_cache, num_q_heads);
+  const int csplits = column ? (k_cache->max_seq_len + column - 1) / column : 0;
+  // one workgroup per column needs no workspace; a caller that appends in the same call has asked whether one is needed
+  FC_REQUIRE(workspace || (csplits == 1 && append), FC_EINVAL, "%s: null workspace", who);
+  FC_REQUIRE((((uintptr_t)q | (uintptr_t)workspace) & 15) == 0, FC_EINVAL, "%s: q/workspace not 16-byte aligned", who);
+  if (column) {
+    // (for a range of 256 tokens or more per workgroup the splits fit what the smallest chunk of 256 needs)
+    FC_REQUIRE((csplits == 1 && append) ||
+                   workspace_bytes >= fc_decode_attn_workspace_bytes(k_cache->batch, num_q_heads, k_cache->max_seq_len),
+               FC_EINVAL, "%s: workspace of %lld bytes is too small", who, (long long)workspace_bytes);
+    const int G = num_q_heads / k_cache->num_kv_heads;
+    dim3 grid(k_cache->num_kv_heads * ((G + DC_HEADS - 1) / DC_HEADS), k_cache->batch, csplits);
+    float* part_o = (float*)workspace;
+    float* part_ml = part_o ? part_o + (int64_t)k_cache->batch * num_q_heads * csplits * FC_HEAD_DIM : nullptr;
+    const DaAppend ap = append ? *append : DaAppend{nullptr, nullptr, 0, 0, nullptr};
+    const KvView k = fc_make_view(k_cache), v = fc_make_view(v_cache);
+#define DC_LAUNCH2(DT, TERMS, PG)                                                                                  \
+  do {                                                                                                             \
+    FC_ALLOW_LDS((decode_column_kernel<DT, TERMS, PG>), DC_LDS);                                                    \
+    hipLaunchKernelGGL((decode_column_kernel<DT, TERMS, PG>), grid, dim3(DC_THREADS), DC_LDS, (hipStream_t)stream, k, \
+                       v, layer, (const char*)q, num_q_heads, context_lens, scale * DA_LOG2E, (char*)out, ap,       \
+                       column, part_o, part_ml, csplits);                                                           \
+  } while (0)
+#define DC_LAUNCH(DT, TERMS) \
+  if (k_cache->block_tables) DC_LAUNCH2(DT, TERMS, true); else DC_LAUNCH2(DT, TERMS, false)
+    if (k_cache->dtype == FC_F16) {
+      DC_LAUNCH(FC_F16, 2);
+    } else if (G > 4) {
+      DC_LAUNCH(FC_BF16, 2);
+    } else {
+      DC_LAUNCH(FC_BF16, 3);
+    }
+#undef DC_LAUNCH2
+#undef DC_LAUNCH
+    FC_CHECK_LAUNCH(who);
+    if (csplits > 1) return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, csplits, column, out, stream);
+    return FC_OK;
+  }
   const int64_t need = fc_decode_attn_workspace_bytes(k_cache->batch, num_q_heads, k_cache->max_seq_len);
   FC_REQUIRE(workspace_bytes >= need, FC_EINVAL, "%s: workspace of %lld bytes, %lld needed", who,
              (long long)workspace_bytes, (long long)need);
@@ -586,11 +1028,7 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
   if (splits > 0) {
     FC_REQUIRE(Hkv * gtiles <= 65535 && B <= 65535, FC_EUNSUPPORTED, "%s: grid too large", who);
     dim3 grid(splits, Hkv * gtiles, B);
-    const auto tile_in_page = [](const fc_kv_view* v, const KvView& d) {
-      return v->stride_token >= 0 && v->stride_token < (1 << 24) &&   // a tile's byte offsets fit 32 bits
-             (v->block_tables == nullptr || (d.block_shift >= 5));
-    };
-    const bool fast = tile_in_page(k_cache, k) && tile_in_page(v_cache, v);
+    const bool fast = da_tile_in_page(k_cache) && da_tile_in_page(v_cache);
 #define DA_LAUNCH(DT, GTV, FA)                                                                                   \
   do {                                                                                                          \
     FC_ALLOW_LDS((decode_attn_kernel<DT, GTV, FA>), DaCfg<GTV>::lds(DA_CHUNK_MAX));                             \
@@ -612,15 +1050,7 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
 #undef DA_LAUNCH
     FC_CHECK_LAUNCH(who);
   }
-  dim3 mgrid(num_q_heads, B);
-  if (bf)
-    hipLaunchKernelGGL((decode_merge_kernel<FC_BF16>), mgrid, dim3(FC_HEAD_DIM), 0, st, part_o, part_ml, context_lens,
-                       k_cache->max_seq_len, num_q_heads, splits, chunk, (char*)out);
-  else
-    hipLaunchKernelGGL((decode_merge_kernel<FC_F16>), mgrid, dim3(FC_HEAD_DIM), 0, st, part_o, part_ml, context_lens,
-                       k_cache->max_seq_len, num_q_heads, splits, chunk, (char*)out);
-  FC_CHECK_LAUNCH(who);
-  return FC_OK;
+  return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, splits, chunk, out, stream);
 }
 
 extern "C" int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t layer, const void* q,
@@ -628,6 +1058,60 @@ extern "C" int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cac
                               void* workspace, int64_t workspace_bytes, void* stream) {
   return da_enqueue("fc_decode_attn", k_cache, v_cache, layer, q, out, num_q_heads, context_lens, scale, workspace,
                     workspace_bytes, stream);
+}
+
+// Append and attention of one layer.  The workgroup of a column appends its own head's row, so the fused form needs
+// one workgroup per kv head (groups of up to 16 query heads) and both caches on one block table; otherwise the rows
+// go in first, in a launch of their own.
+static bool da_appends_inside(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
+  return num_q_heads / k->num_kv_heads <= DC_HEADS && k->block_tables && k->block_tables == v->block_tables &&
+         k->table_stride == v->table_stride && k->block_size == v->block_size && da_column_chunk(k, v, num_q_heads) > 0;
+}
+
+extern "C" int64_t fc_decode_layer_workspace_bytes(const fc_kv_view* k_cache, const fc_kv_view* v_cache,
+                                                   int32_t num_q_heads) {
+  if (!k_cache || !v_cache || num_q_heads <= 0 || k_cache->num_kv_heads <= 0 || k_cache->batch <= 0 ||
+      num_q_heads % k_cache->num_kv_heads || k_cache->block_size <= 0 || v_cache->block_size <= 0)
+    return -1;
+  if (da_appends_inside(k_cache, v_cache, num_q_heads) &&
+      da_column_chunk(k_cache, v_cache, num_q_heads) >= k_cache->max_seq_len)
+    return 0;
+  return fc_decode_attn_workspace_bytes(k_cache->batch, num_q_heads, k_cache->max_seq_len);
+}
+
+extern "C" int fc_decode_layer(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
+                               int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping,
+                               void* out, int32_t num_q_heads, const int32_t* context_lens, float scale, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+  const char* who = "fc_decode_layer";
+  int rc;
+  if ((rc = fc_check_view(k_cache, who)) || (rc = fc_check_view(v_cache, who))) return rc;
+  FC_REQUIRE(k_new && v_new && slot_mapping, FC_EINVAL, "%s: null pointer", who);
+  FC_REQUIRE(k_cache->block_tables && v_cache->block_tables && k_cache->num_layers == 1 && v_cache->num_layers == 1, FC_EINVAL,
+             "%s: paged caches of one layer expected", who);
+  const int64_t row = (int64_t)k_cache->num_kv_heads * FC_HEAD_DIM;
+  for (const fc_kv_view* v : {k_cache, v_cache})
+    FC_REQUIRE((v->stride_token == row || v->block_size == 1) && (v->stride_head == FC_HEAD_DIM || v->num_kv_heads == 1) &&
+                   (v->stride_block == 0 || v->stride_block == row * v->block_size),
+               FC_EINVAL, "%s: a slot counts tokens of a contiguous cache", who);
+  FC_REQUIRE(num_q_heads > 0 && num_q_heads % k_cache->num_kv_heads == 0, FC_EINVAL,
+             "%s: num_q_heads %d not a multiple of num_kv_heads %d", who, num_q_heads, k_cache->num_kv_heads);
+  const int eb = fc_elem_bytes(k_cache->dtype);
+  FC_REQUIRE((((uintptr_t)k_new | (uintptr_t)v_new | (uint64_t)(k_stride * eb) | (uint64_t)(v_stride * eb)) & 15) == 0, FC_EINVAL,
+             "%s: new rows not 16-byte aligned", who);
+  if (da_appends_inside(k_cache, v_cache, num_q_heads)) {
+    const DaAppend ap = {(const char*)k_new, (const char*)v_new, k_stride * eb, v_stride * eb, slot_mapping};
+    return da_enqueue(who, k_cache, v_cache, 0, q, out, num_q_heads, context_lens, scale, workspace, workspace_bytes,
+                      stream, &ap);
+  }
+  // what the attention would refuse is refused before the rows are written
+  FC_REQUIRE(q && out && context_lens && workspace, FC_EINVAL, "%s: null pointer", who);
+  FC_REQUIRE(workspace_bytes >= fc_decode_attn_workspace_bytes(k_cache->batch, num_q_heads, k_cache->max_seq_len), FC_EINVAL,
+             "%s: workspace too small", who);
+  if ((rc = fc_store_kv_slots(k_new, k_stride, v_new, v_stride, k_cache->base, v_cache->base, slot_mapping, k_cache->batch,
+                              (int32_t)row, k_cache->dtype, stream)))
+    return rc;
+  return da_enqueue(who, k_cache, v_cache, 0, q, out, num_q_heads, context_lens, scale, workspace, workspace_bytes, stream);
 }
 
 // ---- the same attention for callers that cannot allocate -------------------------------------------------

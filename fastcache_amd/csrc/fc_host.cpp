@@ -9,10 +9,11 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
-#include <c10/core/InferenceMode.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -257,6 +258,235 @@ PyObject* py_ccm_layers(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   });
 }
 
+// ---- one attention layer of a decode step ---------------------------------------------------------------------------------
+// decode_layer(q, k, v, k_cache, v_cache, slot_mapping, context_lens, block_tables, scale, q_heads, kv_heads, head_dim,
+//              workspace or None) -> out [n, q_heads * head_dim], or None when the arguments are not the plain decode
+// step (the caller's general path then serves or refuses them).
+PyObject* py_decode_layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    need_args(nargs, 13, "decode_layer");
+    for (int i = 0; i < 8; ++i)
+      if (!is_tensor(args[i])) Py_RETURN_NONE;
+    const at::Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
+    const at::Tensor &kc = THPVariable_Unpack(args[3]), &vc = THPVariable_Unpack(args[4]);
+    const at::Tensor &slots = THPVariable_Unpack(args[5]), &lens = THPVariable_Unpack(args[6]), &tables = THPVariable_Unpack(args[7]);
+    const double scale = PyFloat_AsDouble(args[8]);
+    if (scale == -1.0 && PyErr_Occurred()) throw PyFailed();
+    const int64_t hq = as_int(args[9]), hkv = as_int(args[10]), d = as_int(args[11]);
+    const at::ScalarType dt = kc.scalar_type();
+    if (!q.is_cuda() || (dt != at::kHalf && dt != at::kBFloat16) || kc.dim() != 4 || tables.dim() != 2 || d <= 0) Py_RETURN_NONE;
+    const auto dev = q.device();
+    const int64_t n = tables.size(0), row = hkv * d;
+    for (const at::Tensor* t : {&k, &v, &kc, &vc, &slots, &lens, &tables})
+      if (t->device() != dev) Py_RETURN_NONE;
+    for (const at::Tensor* t : {&q, &k, &v, &vc})
+      if (t->scalar_type() != dt) Py_RETURN_NONE;
+    for (const at::Tensor* t : {&slots, &lens, &tables})
+      if (t->scalar_type() != at::kInt || !t->is_contiguous()) Py_RETURN_NONE;
+    if (n == 0 || slots.numel() != n || lens.numel() != n || q.numel() != n * hq * d || !q.is_contiguous()) Py_RETURN_NONE;
+    // new rows: [n, ...] with the row's elements adjacent
+    int64_t stride[2];
+    int i = 0;
+    for (const at::Tensor* t : {&k, &v}) {
+      if (t->numel() != n * row) Py_RETURN_NONE;
+      if (t->is_contiguous()) stride[i] = row;
+      else if (t->dim() == 2 && t->size(0) == n && t->stride(1) == 1) stride[i] = t->stride(0);
+      else Py_RETURN_NONE;
+      ++i;
+    }
+    if (kc.sizes() != vc.sizes() || kc.size(2) != hkv || kc.size(3) != d || !kc.is_contiguous() || !vc.is_contiguous())
+      Py_RETURN_NONE;
+    fc_kv_view kv{};
+    kv.base = kc.data_ptr();
+    kv.stride_token = row;
+    kv.stride_head = hkv > 1 ? d : 0;
+    kv.stride_block = kc.size(0) > 1 ? kc.size(1) * row : 0;
+    kv.block_tables = (const int32_t*)tables.const_data_ptr();
+    kv.table_stride = (int32_t)tables.size(1);
+    kv.block_size = (int32_t)kc.size(1);
+    kv.dtype = dtype_code(dt);
+    kv.num_layers = 1;
+    kv.batch = (int32_t)n;
+    kv.num_kv_heads = (int32_t)hkv;
+    kv.head_dim = (int32_t)d;
+    kv.max_seq_len = (int32_t)(tables.size(1) * kc.size(1));
+    fc_kv_view vv = kv;
+    vv.base = vc.data_ptr();
+    const int64_t need = fc_decode_layer_workspace_bytes(&kv, &vv, (int32_t)hq);
+    if (need < 0) Py_RETURN_NONE;
+    at::Tensor ws;
+    void* wsp = nullptr;
+    int64_t ws_bytes = 0;
+    if (need > 0) {
+      if (args[12] != Py_None) ws = tensor(args[12], "workspace");
+      // the allocator hands blocks out per stream, so a workspace of this call is safe with any number of them
+      if (!ws.defined() || ws.device() != dev || ws.scalar_type() != at::kByte || !ws.is_contiguous() || ws.numel() < need)
+        ws = at::empty({need}, q.options().dtype(at::kByte));
+      wsp = ws.data_ptr();
+      ws_bytes = ws.numel();
+    }
+    at::Tensor out = at::empty({n, hq * d}, q.options());
+    check(fc_decode_layer(&kv, &vv, q.const_data_ptr(), k.const_data_ptr(), stride[0], v.const_data_ptr(), stride[1],
+                          (const int32_t*)slots.const_data_ptr(), out.data_ptr(), (int32_t)hq,
+                          (const int32_t*)lens.const_data_ptr(), (float)scale, wsp, ws_bytes, stream_of(q)),
+          "fc_decode_layer");
+    return wrap(std::move(out));
+  });
+}
+
+// stage_decode(q, k, v, slots, lens, tables, q_static, k_static, v_static, slots_static, lens_static, tables_static) ->
+// True, or False when a tensor is not of the plain form (the caller then copies piece by piece)
+PyObject* py_stage_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    need_args(nargs, 12, "stage_decode");
+    const at::Tensor* t[12];
+    for (int i = 0; i < 12; ++i) {
+      if (!is_tensor(args[i])) Py_RETURN_FALSE;
+      t[i] = &THPVariable_Unpack(args[i]);
+      if (!t[i]->is_cuda() || t[i]->device() != t[0]->device()) Py_RETURN_FALSE;
+    }
+    const at::Tensor& gq = *t[6];
+    const int64_t L = gq.size(0), bs = t[0]->dim() == 3 ? t[0]->size(1) : 0;
+    for (int i = 0; i < 3; ++i) {
+      const at::Tensor &x = *t[i], &g = *t[6 + i];
+      if (x.dim() != 3 || g.dim() != 3 || x.scalar_type() != gq.scalar_type() || g.scalar_type() != gq.scalar_type() ||
+          x.size(0) != L || g.size(0) != L || x.size(1) != bs || g.size(1) != gq.size(1) || x.size(2) != g.size(2) ||
+          x.stride(2) != 1 || !g.is_contiguous())
+        Py_RETURN_FALSE;
+      const int64_t eb = x.element_size();
+      if ((x.stride(0) * eb) % 16 || (x.stride(1) * eb) % 16 || (x.size(2) * eb) % 16 || ((uintptr_t)x.const_data_ptr() & 15))
+        Py_RETURN_FALSE;
+    }
+    if (t[1]->size(2) != t[2]->size(2)) Py_RETURN_FALSE;
+    for (int i = 3; i < 6; ++i)
+      for (const at::Tensor* x : {t[i], t[6 + i]})
+        if (x->scalar_type() != at::kInt || !x->is_contiguous()) Py_RETURN_FALSE;
+    const at::Tensor &tab = *t[5], &gtab = *t[11];
+    if (bs < 1 || bs > gq.size(1) || t[3]->numel() != bs || t[4]->numel() != bs || tab.dim() != 2 || tab.size(0) != bs ||
+        gtab.dim() != 2 || gtab.size(0) != gq.size(1) || tab.size(1) < 1 || tab.size(1) > gtab.size(1) ||
+        t[9]->numel() != gq.size(1) || t[10]->numel() != gq.size(1))
+      Py_RETURN_FALSE;
+    const auto ints = [](const at::Tensor& x) { return (int32_t*)x.data_ptr(); };
+    check(fc_stage_decode(t[0]->const_data_ptr(), t[0]->stride(0), t[0]->stride(1), t[1]->const_data_ptr(), t[1]->stride(0),
+                          t[1]->stride(1), t[2]->const_data_ptr(), t[2]->stride(0), t[2]->stride(1), (int32_t)L, (int32_t)bs,
+                          (int32_t)t[0]->size(2), (int32_t)t[1]->size(2), dtype_code(gq.scalar_type()), ints(*t[3]),
+                          ints(*t[4]), ints(tab), (int32_t)tab.size(1), t[6]->data_ptr(), t[7]->data_ptr(), t[8]->data_ptr(),
+                          ints(*t[9]), ints(*t[10]), ints(gtab), (int32_t)gq.size(1), (int32_t)gtab.size(1), stream_of(gq)),
+          "fc_stage_decode");
+    Py_RETURN_TRUE;
+  });
+}
+
+// ---- a step's numbers to the device -----------------------------------------------------------------------------------------
+struct Packed {
+  at::Tensor host, dev;
+  int64_t at = 0;
+  Packed(int64_t bytes, const c10::Device& device)
+      : host(at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true))),
+        dev(at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(device))) {}
+  template <typename T>
+  T* take(int64_t n) {
+    T* p = (T*)((char*)host.data_ptr() + at);
+    at += n * (int64_t)sizeof(T);
+    return p;
+  }
+  at::Tensor part(int64_t byte, int64_t n, at::ScalarType t) { return dev.narrow(0, byte, n * (int64_t)c10::elementSize(t)).view(t); }
+};
+
+c10::Device device_arg(PyObject* o) { return tensor(o, "device reference").device(); }
+
+// rows of Python ints, right-padded with -1
+int64_t table_width(PyObject* tables, Py_ssize_t n) {
+  int64_t width = 0;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* row = PyList_GET_ITEM(tables, i);
+    if (!PyList_Check(row)) fail("a block table is a list of page numbers");
+    width = std::max<int64_t>(width, PyList_GET_SIZE(row));
+  }
+  return width;
+}
+
+void fill_tables(PyObject* tables, Py_ssize_t n, int64_t width, int32_t* out) {
+  for (Py_ssize_t i = 0; i < n; ++i, out += width) {
+    PyObject* row = PyList_GET_ITEM(tables, i);
+    const Py_ssize_t len = PyList_GET_SIZE(row);
+    for (Py_ssize_t j = 0; j < len; ++j) out[j] = (int32_t)as_int(PyList_GET_ITEM(row, j));
+    for (int64_t j = len; j < width; ++j) out[j] = -1;
+  }
+}
+
+// decode_inputs(ids, lens, tables, block_size, ref) -> (input_ids, positions, slots, context_lens, block_tables) on the
+// device of `ref`: one pinned buffer and one copy instead of five of each
+PyObject* py_decode_inputs(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    need_args(nargs, 5, "decode_inputs");
+    for (int i = 0; i < 3; ++i)
+      if (!PyList_Check(args[i])) fail("decode_inputs: lists expected");
+    const Py_ssize_t n = PyList_GET_SIZE(args[0]);
+    if (n == 0 || PyList_GET_SIZE(args[1]) != n || PyList_GET_SIZE(args[2]) != n) fail("decode_inputs: lists of one length expected");
+    const int64_t bs = as_int(args[3]), width = table_width(args[2], n);
+    Packed pk(n * 16 + n * 8 + n * width * 4, device_arg(args[4]));
+    int64_t *ids = pk.take<int64_t>(n), *pos = pk.take<int64_t>(n);
+    int32_t *slots = pk.take<int32_t>(n), *lens = pk.take<int32_t>(n), *tab = pk.take<int32_t>(n * width);
+    for (Py_ssize_t i = 0; i < n; ++i) {
+      ids[i] = as_int(PyList_GET_ITEM(args[0], i));
+      const int64_t len = as_int(PyList_GET_ITEM(args[1], i));
+      pos[i] = len;
+      lens[i] = (int32_t)len;
+      PyObject* row = PyList_GET_ITEM(args[2], i);
+      const Py_ssize_t pages = PyList_GET_SIZE(row);
+      if (pages == 0) {
+        PyErr_SetString(PyExc_IndexError, "sequence without pages");
+        throw PyFailed();
+      }
+      const int64_t page = as_int(PyList_GET_ITEM(row, std::min<int64_t>(len / bs, pages - 1)));
+      slots[i] = (int32_t)(page * bs + len % bs);
+    }
+    fill_tables(args[2], n, width, tab);
+    pk.dev.copy_(pk.host, true);
+    PyObject* out = PyTuple_New(5);
+    PyTuple_SET_ITEM(out, 0, wrap(pk.part(0, n, at::kLong)));
+    PyTuple_SET_ITEM(out, 1, wrap(pk.part(n * 8, n, at::kLong)));
+    PyTuple_SET_ITEM(out, 2, wrap(pk.part(n * 16, n, at::kInt)));
+    PyTuple_SET_ITEM(out, 3, wrap(pk.part(n * 20, n, at::kInt)));
+    PyTuple_SET_ITEM(out, 4, wrap(pk.part(n * 24, n * width, at::kInt).view({n, width})));
+    return out;
+  });
+}
+
+// upload_tables(tables, rows, ref) -> (block_tables [n, width], then one int32 tensor per list of `rows`)
+PyObject* py_upload_tables(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    need_args(nargs, 3, "upload_tables");
+    if (!PyList_Check(args[0]) || !PyTuple_Check(args[1])) fail("upload_tables: a list of tables and a tuple of lists expected");
+    const Py_ssize_t n = PyList_GET_SIZE(args[0]), extra = PyTuple_GET_SIZE(args[1]);
+    const int64_t width = table_width(args[0], n);
+    int64_t total = n * width;
+    for (Py_ssize_t i = 0; i < extra; ++i) {
+      if (!PyList_Check(PyTuple_GET_ITEM(args[1], i))) fail("upload_tables: lists of ints expected");
+      total += PyList_GET_SIZE(PyTuple_GET_ITEM(args[1], i));
+    }
+    Packed pk(total * 4, device_arg(args[2]));
+    fill_tables(args[0], n, width, pk.take<int32_t>(n * width));
+    for (Py_ssize_t i = 0; i < extra; ++i) {
+      PyObject* row = PyTuple_GET_ITEM(args[1], i);
+      const Py_ssize_t len = PyList_GET_SIZE(row);
+      int32_t* p = pk.take<int32_t>(len);
+      for (Py_ssize_t j = 0; j < len; ++j) p[j] = (int32_t)as_int(PyList_GET_ITEM(row, j));
+    }
+    pk.dev.copy_(pk.host, true);
+    PyObject* out = PyTuple_New(1 + extra);
+    PyTuple_SET_ITEM(out, 0, wrap(pk.part(0, n * width, at::kInt).view({n, width})));
+    int64_t byte = n * width * 4;
+    for (Py_ssize_t i = 0; i < extra; ++i) {
+      const int64_t len = PyList_GET_SIZE(PyTuple_GET_ITEM(args[1], i));
+      PyTuple_SET_ITEM(out, 1 + i, wrap(pk.part(byte, len, at::kInt)));
+      byte += len * 4;
+    }
+    return out;
+  });
+}
+
 PyObject* py_init(PyObject*, PyObject* error) {
   Py_XDECREF(g_error);
   Py_INCREF(error);
@@ -270,6 +500,14 @@ PyMethodDef kMethods[] = {
     {"unchanged", py_unchanged, METH_O, "unchanged(capsule) -> bool"},
     {"ccm_layers", (PyCFunction)(void (*)(void))py_ccm_layers, METH_FASTCALL,
      "ccm_layers(pairs, weights, segments, out_len, factor, min_rows) -> list of pairs, or None"},
+    {"decode_layer", (PyCFunction)(void (*)(void))py_decode_layer, METH_FASTCALL,
+     "decode_layer(q, k, v, k_cache, v_cache, slots, lens, tables, scale, q_heads, kv_heads, head_dim, workspace) -> out or None"},
+    {"stage_decode", (PyCFunction)(void (*)(void))py_stage_decode, METH_FASTCALL,
+     "stage_decode(q, k, v, slots, lens, tables, and the six static buffers) -> bool"},
+    {"decode_inputs", (PyCFunction)(void (*)(void))py_decode_inputs, METH_FASTCALL,
+     "decode_inputs(ids, lens, tables, block_size, ref) -> five device tensors"},
+    {"upload_tables", (PyCFunction)(void (*)(void))py_upload_tables, METH_FASTCALL,
+     "upload_tables(tables, (list, ...), ref) -> device tensors"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "host path of fastcache_amd", -1, kMethods, nullptr, nullptr, nullptr, nullptr};

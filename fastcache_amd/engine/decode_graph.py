@@ -142,9 +142,14 @@ class BucketedDecodeGraphs:
         """Replay the graph of the smallest bucket that holds the batch, with the current decode context."""
         bs = q.shape[1]
         context = get_context()
-        self.reset_graph_vars()
         graph = self.graphs[next(x for x in self.graph_bs if x >= bs)]
         gv = self.graph_vars
+        if _lib.host().stage_decode(q, k, v, context.slot_mapping, context.context_lens, context.block_tables, gv["q"],
+                                    gv["k"], gv["v"], gv["slot_mapping"], gv["context_lens"], gv["block_tables"]):
+            _lib.note_enqueued()
+            graph.replay()
+            return gv["outputs"][:, :bs]
+        self.reset_graph_vars()
         gv["q"][:, :bs] = q
         gv["k"][:, :bs] = k
         gv["v"][:, :bs] = v

@@ -82,14 +82,10 @@ class PagedKVRunner:
     def preare_block_tables(self, seqs: Seq[Sequence]) -> torch.Tensor:
         """int32 ``[B, max blocks]`` right-padded with -1 (llava_model_runner.py:541-549; the
         reference spells it this way)."""
-        width = max(len(s.block_table) for s in seqs)
-        rows = [s.block_table + [-1] * (width - len(s.block_table)) for s in seqs]
-        return torch.tensor(rows, dtype=torch.int32, pin_memory=True).to(self.device, non_blocking=True)
+        return _lib.host().upload_tables([s.block_table for s in seqs], (), self.kv_cache)[0]
 
     def _table_and_lens(self, tables: Seq[Seq[int]], lens: Seq[int]):
-        width = max(len(t) for t in tables)
-        tt = torch.tensor([list(t) + [-1] * (width - len(t)) for t in tables], dtype=torch.int32, device=self.device)
-        return tt, torch.tensor(list(lens), dtype=torch.int32, device=self.device)
+        return _lib.host().upload_tables([list(t) for t in tables], (list(lens),), self.kv_cache)
 
     # -- paged <-> HuggingFace layout ----------------------------------------------------------------
     def _extract_kv_cache_fast(self, block_table: List[int], seq_len: int) -> List[LayerKV]:
@@ -306,17 +302,8 @@ class PagedKVRunner:
     def prepare_decode(self, seqs: List[Sequence]):
         """``positions = context_lens = kv_cache_len``; the new token's slot is position ``kv_cache_len``
         of the sequence (llava_model_runner.py:637-674)."""
-        input_ids, positions, slots, lens = [], [], [], []
-        for s in seqs:
-            n = s.kv_cache_len
-            input_ids.append(s.last_token)
-            positions.append(n)
-            lens.append(n)
-            bi, pos = divmod(n, self.block_size)
-            blk = s.block_table[bi] if bi < len(s.block_table) else s.block_table[-1]
-            slots.append(blk * self.block_size + pos)
-        mk = lambda x, dt: torch.tensor(x, dtype=dt, pin_memory=True).to(self.device, non_blocking=True)
-        input_ids, positions = mk(input_ids, torch.int64), mk(positions, torch.int64)
-        set_context(False, slot_mapping=mk(slots, torch.int32), context_lens=mk(lens, torch.int32),
-                    block_tables=self.preare_block_tables(seqs))
+        input_ids, positions, slots, lens, tables = _lib.host().decode_inputs(
+            [s.last_token for s in seqs], [s.kv_cache_len for s in seqs], [s.block_table for s in seqs], self.block_size,
+            self.kv_cache)
+        set_context(False, slot_mapping=slots, context_lens=lens, block_tables=tables)
         return input_ids, positions

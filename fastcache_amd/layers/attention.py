@@ -69,10 +69,18 @@ class Attention(nn.Module):
         self.workspace: Optional[torch.Tensor] = None   # set by a graph runner that owns the scratch memory
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+        ctx = get_context()
+        if not ctx.is_prefill and ctx.block_tables is not None:
+            # the plain decode step: append and attention through one native call (and one launch where that is faster)
+            out = _lib.host().decode_layer(q, k, v, self.k_cache, self.v_cache, ctx.slot_mapping, ctx.context_lens,
+                                           ctx.block_tables, self.scale, self.num_heads, self.num_kv_heads, self.head_dim,
+                                           self.workspace)
+            if out is not None:
+                _lib.note_enqueued()
+                return out
         q = q.view(-1, self.num_heads, self.head_dim)
         k = k.view(-1, self.num_kv_heads, self.head_dim)
         v = v.view(-1, self.num_kv_heads, self.head_dim)
-        ctx = get_context()
         store_kvcache(k, v, self.k_cache, self.v_cache, ctx.slot_mapping)
         if ctx.is_prefill:
             raise NotImplementedError("prefill attention is outside the KV-cache compression path built here")

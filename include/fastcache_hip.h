@@ -478,6 +478,34 @@ int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t
                    float scale, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * Append and attention of one layer of a decode step (nanovllm/layers/attention.py:62-79): row i of k_new / v_new
+ * ([batch][num_kv_heads][head_dim], `*_stride` elements between sequences) goes to cache slot slot_mapping[i]
+ * (negative: skipped), then query i attends the first context_lens[i] tokens of sequence i.  The caches are one layer,
+ * paged, with contiguous tokens; slot_mapping[i] is a token of sequence i.  `workspace` may be NULL when
+ * fc_decode_layer_workspace_bytes returns 0 (the appending is then part of the attention's launch), otherwise it
+ * holds that many bytes.
+ */
+int64_t fc_decode_layer_workspace_bytes(const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t num_q_heads);
+int fc_decode_layer(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
+                    int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping, void* out,
+                    int32_t num_q_heads, const int32_t* context_lens, float scale, void* workspace,
+                    int64_t workspace_bytes, void* stream);
+
+/*
+ * A decode step's inputs into the static buffers of a captured graph (what the decode branch of `run_model` patches
+ * before a replay, nanovllm/engine/llava_model_runner.py:697-710): q [num_layers][batch][q_elems] and k, v
+ * [num_layers][batch][kv_elems] (strides in elements) into contiguous buffers of max_batch sequences per layer; slots,
+ * lengths and tables [batch][table_width] into buffers of max_batch rows of max_width entries, the rows past `batch`
+ * reset to slot -1, length 0, table 0.
+ */
+int fc_stage_decode(const void* q, int64_t q_layer, int64_t q_row, const void* k, int64_t k_layer, int64_t k_row,
+                    const void* v, int64_t v_layer, int64_t v_row, int32_t num_layers, int32_t batch, int32_t q_elems,
+                    int32_t kv_elems, int32_t dtype, const int32_t* slots, const int32_t* context_lens,
+                    const int32_t* tables, int32_t table_width, void* q_static, void* k_static, void* v_static,
+                    int32_t* slots_static, int32_t* lens_static, int32_t* tables_static, int32_t max_batch,
+                    int32_t max_width, void* stream);
+
+/*
  * fc_decode_attn for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): the chunk partials go to a buffer built into the library, a
  * file-scope device array of fc_decode_attn_static_capacity() bytes (16 MiB) that every GPU the library runs on

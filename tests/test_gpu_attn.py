@@ -258,3 +258,42 @@ def test_decode_attention_empty_rows(dev):
     assert torch.equal(some[0], full[0]) and bool((some[1:] == 0).all())
     none = ops.decode_attn(kview, vview, 0, q, torch.zeros(3, dtype=torch.int32, device=dev), 128 ** -0.5, ws).cpu()
     assert bool((none == 0).all())
+
+
+@pytest.mark.parametrize("dtype,Hq,Hkv,lens,slot_at", [
+    (torch.bfloat16, 28, 4, [300, 900, 1, 0, 31, 32, 33, 255, 256, 257, 511, 513], 0),   # the new row right behind the context
+    (torch.bfloat16, 8, 2, [1, 2, 32, 33, 256, 257, 512, 900], -1),                      # the new row is the last attended one
+    (torch.float16, 4, 4, [2047, 5, 1024], -1),
+    (torch.float16, 32, 2, [700, 130], -2),                                              # 16 heads a group; a row inside the context
+    (torch.bfloat16, 40, 2, [300, 77], -1),                                              # 20 heads a group: rows go in first
+    (torch.bfloat16, 8, 2, [2500, 40], -1),                                              # too long for one workgroup a column
+])
+def test_attention_layer_appends_and_attends(dev, dtype, Hq, Hkv, lens, slot_at):
+    """``Attention.forward`` of a decode step against the oracle on a cache the oracle appended to: every launch form the
+    layer picks (append inside the attention's launch or before it), rows behind, at and inside the attended range, a
+    sequence without context and a padded one (slot -1)."""
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    B = len(lens)
+    case = synth.make_paged_case(seed=31, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=[n + 1 for n in lens], dtype=dtype)
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(B, h * 128, generator=g).to(dtype) for h in (Hq, Hkv, Hkv))
+    tables, lens_t = case.table_tensor("cpu"), torch.tensor(lens, dtype=torch.int32)
+    pos = [max(0, n + slot_at) for n in lens]
+    slots = torch.tensor([case.block_tables[b][p // 256] * 256 + p % 256 for b, p in enumerate(pos)], dtype=torch.int32)
+    slots[-1] = -1
+    pool = case.kv_cache[:, 0].clone()
+    for p, new in ((0, k), (1, v)):
+        for b in range(B - 1):
+            pool[p].view(-1, Hkv, 128)[int(slots[b])] = new[b].view(Hkv, 128)
+    ref = oattn.decode_attention(q.view(B, Hq, 128), pool[0], pool[1], lens_t, tables, 128 ** -0.5)
+    layer = Attention(Hq, 128, 128 ** -0.5, Hkv)
+    on_gpu = case.kv_cache[:, 0].to(dev)
+    layer.k_cache, layer.v_cache = on_gpu[0], on_gpu[1]
+    set_context(False, slot_mapping=slots.to(dev), context_lens=lens_t.to(dev), block_tables=tables.to(dev))
+    try:
+        got = layer(q.to(dev), k.to(dev), v.to(dev)).cpu().view(B, Hq, 128)
+    finally:
+        reset_context()
+    assert torch.equal(on_gpu.cpu(), pool)
+    assert float((got.float() - ref.float()).abs().max()) < 4e-3
