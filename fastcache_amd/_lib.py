@@ -159,6 +159,21 @@ def host():
     return _host
 
 
+_cus = {}
+
+
+def compute_units(device: torch.device) -> int:
+    n = _cus.get(device)
+    if n is None:
+        n = _cus[device] = torch.cuda.get_device_properties(device).multi_processor_count
+    return n
+
+
+def upload_ints(values, ref: torch.Tensor) -> torch.Tensor:
+    """A list of Python ints as an int32 tensor on the device of ``ref``, through pinned memory and without waiting."""
+    return host().upload_tables([], (list(values),), ref)[1]
+
+
 _enqueued = 0
 
 

@@ -179,9 +179,10 @@ class BlockManager:
         from the prefix cache, so that no later request is handed them."""
         for block_id in block_ids:
             page = self.blocks[block_id]
-            if page.hash != NO_KEY and self._prefix_index.get(page.hash) == block_id:
-                del self._prefix_index[page.hash]
-            page.forget()
+            if page.hash != NO_KEY:
+                if self._prefix_index.get(page.hash) == block_id:
+                    del self._prefix_index[page.hash]
+                page.forget()
 
     # -- release after compression ------------------------------------------------------------------------
     def free_blocks_after_compression(self, seq: Sequence, blocks_to_keep: int) -> None:

@@ -157,16 +157,18 @@ class PagedKVRunner:
                             f"page {b} belongs to several sequences of the batch and sequence {s.seq_id} would "
                             "rewrite it in place; attach the page manager (block_manager=) so that it gets its own copy")
             return 0
-        # a page shared only inside the batch stays with the last sequence that names it
-        owners = {b: bm.blocks[b].ref_count for s in seqs for b in s.block_table if b >= 0}
+        blocks = bm.blocks
         plan = []
-        for s, w in zip(seqs, writes):
-            mine = []
-            for i, b in enumerate(s.block_table[:w]):
-                if owners[b] > 1:
-                    owners[b] -= 1
-                    mine.append(i)
-            plan.append((s, mine))
+        if any(blocks[b].ref_count > 1 for s, w in zip(seqs, writes) for b in s.block_table[:w] if b >= 0):
+            # a page shared only inside the batch stays with the last sequence that names it
+            owners = {b: blocks[b].ref_count for s in seqs for b in s.block_table if b >= 0}
+            for s, w in zip(seqs, writes):
+                mine = []
+                for i, b in enumerate(s.block_table[:w]):
+                    if owners[b] > 1:
+                        owners[b] -= 1
+                        mine.append(i)
+                plan.append((s, mine))
         need = sum(len(p) for _, p in plan)
         if need > len(bm.free_block_ids):
             raise _lib.FastcacheError(f"the batch would rewrite {need} pages it shares with other sequences and only "

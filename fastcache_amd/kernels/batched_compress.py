@@ -126,7 +126,7 @@ class BatchedGEMMCompressor(nn.Module):
         dviews = views if out is None else [_lib.dense_view(out[p][l0:l1]) for p in range(2)]
         if host_lens is not None and len(set(host_lens)) > 1:
             dev = kv_cache.device
-            mk = lambda xs: torch.tensor(xs, dtype=torch.int32, device=dev)
+            mk = lambda xs: _lib.upload_ints(xs, kv_cache)
             imgs = [min(int(it_len[0]), n) if it_len[0] > 0 else 0 for n in host_lens]
             dsts = [0] * len(imgs)
             for starts, counts, seg in (([0] * len(imgs), imgs, "i"), (imgs, [n - i for n, i in zip(host_lens, imgs)], "t")):

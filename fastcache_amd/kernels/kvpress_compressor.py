@@ -158,7 +158,7 @@ class KVPressCompressor(nn.Module):
         vview = _lib.paged_view(kv_cache[1][l0:l1], block_tables, seq_lens, max_len)
         kept = [self.paged_compressed_len(n) for n in lens]
         width = max(kept)
-        n_kept = torch.tensor(kept, dtype=torch.int32, device=dev)
+        n_kept = _lib.upload_ints(kept, kv_cache)
         if self.method_name == "knorm" and any(k < n for k, n in zip(kept, lens)):
             score = ops.knorm_mean_score(kview, dev)                                  # [L, B, S], -inf past each length
             idx = ops.topk_select(score, width, row_lens=seq_lens, n_kept=n_kept).view(L, B, 1, width)

@@ -26,6 +26,13 @@ def _i32(t: Optional[torch.Tensor], name: str, device) -> Optional[torch.Tensor]
     return t
 
 
+def _index_rows(shape, padded: bool, device) -> torch.Tensor:
+    """int32 index rows; ``padded``: rows that may be filled only in part end in -1."""
+    if padded:
+        return torch.full(shape, -1, dtype=torch.int32, device=device)
+    return torch.empty(shape, dtype=torch.int32, device=device)
+
+
 # ---------------------------------------------------------------------------------------------
 # scoring
 # ---------------------------------------------------------------------------------------------
@@ -180,7 +187,7 @@ def snapkv_press_preferred(keys: FcKvView, num_q_heads: int, window: int, comput
 def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window: int, kernel_size: int, k: int,
                  causal_window: bool = True, reduction: str = "mean", scale: Optional[float] = None,
                  seq_lens: Optional[torch.Tensor] = None, lse: Optional[torch.Tensor] = None,
-                 n_kept=None, ragged: bool = False, host_lens=None):
+                 n_kept=None, ragged: bool = False, host_lens=None, rows_only: bool = False):
     """SnapKV scores, selection (the window always kept; ``k`` or ``n_kept[b]`` positions per row, window included,
     more than the window) and in-place compaction of both planes, each (layer, sequence, kv head) column by one
     workgroup in one launch; then the window fill of the scores.  Returns ``(scores, indices)`` equal to
@@ -189,7 +196,10 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     ``n_kept``: the kept counts per sequence as Python ints (checked here: the kernel leaves a sequence longer than the
     window untouched when its count does not exceed the window, which a caller that then shortens the sequence
     would not notice; ``host_lens`` names the sequences no longer than the window, which are exempt).  A device
-    tensor is passed through unchecked for callers that have validated the counts themselves."""
+    tensor is passed through unchecked for callers that have validated the counts themselves.
+
+    ``rows_only``: for callers that want the moved rows alone; scores and indices stay scratch (no window fill, no
+    padding of the index rows) and None is returned."""
     if n_kept is not None and not isinstance(n_kept, torch.Tensor):
         counts = [int(c) for c in n_kept]
         lens_h = list(host_lens) if host_lens is not None else [keys.max_seq_len] * len(counts)
@@ -197,7 +207,7 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
         if len(counts) != keys.batch or bad:
             raise FastcacheError(f"snapkv_press: kept counts must exceed the window ({window}) and fit the index row "
                                  f"({k}) for every sequence longer than the window; offending sequences: {bad}")
-        n_kept = torch.tensor(counts, dtype=torch.int32, device=queries.device)
+        n_kept = _lib.upload_ints(counts, queries)
     if queries.dim() == 4:
         queries = queries.unsqueeze(0)
         if lse is not None and lse.dim() == 3:
@@ -222,10 +232,7 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     scores = torch.empty((L, B, H, stride), dtype=torch.float32, device=dev)
     row_max = torch.empty((L, B, H), dtype=torch.float32, device=dev)
     n_kept = _i32(n_kept, "n_kept", dev)
-    if n_kept is not None or ragged:
-        idx = torch.full((L, B, H, k), -1, dtype=torch.int32, device=dev)
-    else:
-        idx = torch.empty((L, B, H, k), dtype=torch.int32, device=dev)
+    idx = _index_rows((L, B, H, k), (n_kept is not None or ragged) and not rows_only, dev)
     if lse is not None:
         _lib.require_gpu(lse, "lse")
         if lse.dtype != torch.float32 or tuple(lse.shape) != (L, B, Hq, W):
@@ -235,6 +242,8 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     check(fn("fc_snapkv_press")(C.byref(keys), C.byref(values), queries.data_ptr(), ptr(lse), Hq, window, kernel_size,
                                 int(causal_window), scale, out_scale, scores.data_ptr(), stride, row_max.data_ptr(), k,
                                 ptr(n_kept), idx.data_ptr(), k, st), "fc_snapkv_press")
+    if rows_only:
+        return None
     check(fn("fc_snapkv_fill_window")(scores.data_ptr(), stride, L, B, H, ptr(seq_lens), keys.max_seq_len, window,
                                       row_max.data_ptr(), st), "fc_snapkv_fill_window")
     return scores, idx
@@ -271,10 +280,7 @@ def topk_select(scores: torch.Tensor, k: int, row_lens: Optional[torch.Tensor] =
     n_kept = _i32(n_kept, "n_kept", dev)
     per_row = row_lens is not None or n_kept is not None
     mod = (row_lens if row_lens is not None else n_kept).numel() if per_row else 1
-    if per_row:
-        out = torch.full((*scores.shape[:-1], k), -1, dtype=torch.int32, device=dev)
-    else:
-        out = torch.empty((*scores.shape[:-1], k), dtype=torch.int32, device=dev)
+    out = _index_rows((*scores.shape[:-1], k), per_row, dev)
     check(fn("fc_topk_select")(scores.data_ptr(), score_stride, rows, S, ptr(row_lens), rows_per_len, mod, k,
                                ptr(n_kept), out.data_ptr(), k, current_stream()), "fc_topk_select")
     return out
@@ -302,38 +308,34 @@ def press_column_fits(max_seq_len: int, k: int) -> bool:
 
 
 def knorm_press(keys: FcKvView, values: FcKvView, k: int, device, n_kept: Optional[torch.Tensor] = None,
-                ragged: bool = False):
+                ragged: bool = False, rows_only: bool = False):
     """Knorm scores, top-``k`` (or ``n_kept[b]``) per (layer, sequence, kv head) row and in-place compaction of
     both planes in one launch; returns ``(scores [L, B, Hkv, max_seq_len] fp32, indices [L, B, Hkv, k] int32)`` equal
     to ``knorm_score`` + ``topk_select`` + ``compact``.  With ``n_kept`` or ``ragged`` (sequences that may hold fewer
-    than ``k`` tokens) index entries past a row's kept count are -1."""
+    than ``k`` tokens) index entries past a row's kept count are -1 (not with ``rows_only``, for callers that want the
+    moved rows alone)."""
     L, B, H, S = keys.num_layers, keys.batch, keys.num_kv_heads, keys.max_seq_len
     scores = torch.empty((L, B, H, S), dtype=torch.float32, device=device)
     n_kept = _i32(n_kept, "n_kept", device)
-    if n_kept is not None or ragged:
-        idx = torch.full((L, B, H, k), -1, dtype=torch.int32, device=device)
-    else:
-        idx = torch.empty((L, B, H, k), dtype=torch.int32, device=device)
+    idx = _index_rows((L, B, H, k), (n_kept is not None or ragged) and not rows_only, device)
     check(fn("fc_knorm_press")(C.byref(keys), C.byref(values), scores.data_ptr(), S, k, ptr(n_kept), idx.data_ptr(), k,
                                current_stream()), "fc_knorm_press")
     return scores, idx
 
 
 def select_compact(keys: FcKvView, values: FcKvView, scores: torch.Tensor, k: int,
-                   n_kept: Optional[torch.Tensor] = None, ragged: bool = False) -> torch.Tensor:
+                   n_kept: Optional[torch.Tensor] = None, ragged: bool = False,
+                   rows_only: bool = False) -> torch.Tensor:
     """``topk_select`` over each sequence's own length and ``compact`` of both planes onto themselves in one launch;
     ``scores`` fp32 ``[L, B, Hkv, stride]`` contiguous.  Returns the indices ``[L, B, Hkv, k]`` (-1 past a row's kept
-    count with ``n_kept`` or ``ragged``)."""
+    count with ``n_kept`` or ``ragged``, unless ``rows_only``)."""
     _lib.require_gpu(scores, "scores")
     L, B, H = keys.num_layers, keys.batch, keys.num_kv_heads
     if scores.dtype != torch.float32 or scores.dim() != 4 or tuple(scores.shape[:3]) != (L, B, H) or \
             not scores.is_contiguous():
         raise FastcacheError("scores must be a contiguous fp32 [L, B, Hkv, stride] tensor matching the views")
     n_kept = _i32(n_kept, "n_kept", scores.device)
-    if n_kept is not None or ragged:
-        idx = torch.full((L, B, H, k), -1, dtype=torch.int32, device=scores.device)
-    else:
-        idx = torch.empty((L, B, H, k), dtype=torch.int32, device=scores.device)
+    idx = _index_rows((L, B, H, k), (n_kept is not None or ragged) and not rows_only, scores.device)
     check(fn("fc_select_compact")(C.byref(keys), C.byref(values), scores.data_ptr(), scores.shape[3], k, ptr(n_kept),
                                   idx.data_ptr(), k, current_stream()), "fc_select_compact")
     return idx

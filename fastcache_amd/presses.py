@@ -131,7 +131,7 @@ class ScorerPress:
         kview, vview = paged_press._views(pool, block_tables, seq_lens, seq_len)
         scores = self.paged_scores(kview, vview, lens, seq_lens, layers, seq_ids, pool.device)
         if out is None:
-            paged_press._select_and_compact(kview, vview, scores, seq_lens, kept, True, pool.shape[4])
+            paged_press._select_and_compact(kview, vview, scores, seq_lens, kept, True, pool.shape[4], rows_only=True)
             return
         self._compact_into(kview, vview, scores, seq_lens, kept, pool.shape[4], out, layers)
 
@@ -143,7 +143,7 @@ class ScorerPress:
         if len(set(kept)) == 1 and seq_lens is None:
             ops.compact(kview, vview, dk, dv, ops.topk_select(scores, width))
             return
-        n_kept = torch.tensor(kept, dtype=torch.int32, device=scores.device)
+        n_kept = _lib.upload_ints(kept, scores)
         idx = ops.topk_select(scores, width, row_lens=seq_lens, n_kept=n_kept, rows_per_len=heads)
         ops.compact(kview, vview, dk, dv, idx, n_kept=n_kept)
 
@@ -185,14 +185,14 @@ class _PerSequenceInputs:
 
     def __init__(self):
         self._batch = None            # (ids or None, {name: tensor [L, B, ...]})
-        self._by_seq = {}             # seq_id -> {name: tensor [L, ...]}
+        self._by_seq = {}             # seq_id -> ({name: tensor [L, B, ...]}, position in the batch)
 
     def put(self, tensors: dict, seq_ids=None) -> None:
         tensors = {k: v for k, v in tensors.items() if v is not None}
         self._batch = (None if seq_ids is None else list(seq_ids), tensors)
         if seq_ids is not None:
             for b, i in enumerate(seq_ids):
-                self._by_seq[i] = {k: v[:, b] for k, v in tensors.items()}
+                self._by_seq[i] = (tensors, b)
 
     def take(self, batch: int, seq_ids=None) -> dict:
         ids, tensors = self._batch if self._batch is not None else (None, None)
@@ -209,7 +209,7 @@ class _PerSequenceInputs:
             raise FastcacheError(f"the press holds no inputs for sequences {missing}")
         rows = [self._by_seq.pop(i) for i in seq_ids]
         self._batch = None
-        return {k: torch.stack([r[k] for r in rows], dim=1) for k in rows[0]}
+        return {k: torch.stack([held[k][:, b] for held, b in rows], dim=1) for k in rows[0][0]}
 
     def __bool__(self):
         return self._batch is not None or bool(self._by_seq)
@@ -231,7 +231,7 @@ class KnormPress(ScorerPress):
         from . import paged_press
         # scoring, selection and compaction of a column by one workgroup, one launch for the batch
         paged_press.knorm_compress_paged(pool, block_tables, seq_lens, seq_len, self.compression_ratio,
-                                         host_lens=lens if len(set(lens)) > 1 else None)
+                                         host_lens=lens if len(set(lens)) > 1 else None, rows_only=True)
 
 
 @dataclass
@@ -294,11 +294,12 @@ class SnapKVPress(ScorerPress):
             kview, vview = paged_press._views(pool, block_tables, seq_lens, seq_len)
             scores = ops.snapkv_score(kview, q, self.window_size, self.kernel_size, self.causal_window,
                                       self.reduction, seq_lens=seq_lens, lse=lse)
-            paged_press._select_and_compact(kview, vview, scores, seq_lens, kept, True, pool.shape[4])
+            paged_press._select_and_compact(kview, vview, scores, seq_lens, kept, True, pool.shape[4], rows_only=True)
             return
         paged_press.snapkv_compress_paged(pool, block_tables, seq_lens, seq_len, q, self.compression_ratio,
                                           self.window_size, self.kernel_size, self.causal_window, self.reduction,
-                                          self.window_in_budget, host_lens=lens if len(set(lens)) > 1 else None)
+                                          self.window_in_budget, host_lens=lens if len(set(lens)) > 1 else None,
+                                          rows_only=True)
 
     def window_queries(self, module, hidden_states, kwargs) -> torch.Tensor:
         """Rotated queries of the last ``window_size`` positions, ``[B, Hq, W, D]``: given directly as

@@ -213,7 +213,7 @@ class _CCMBase(nn.Module):
             n_max = max(g[3] for g in segs)
             if n_max == 0:
                 continue
-            mk = lambda xs: torch.tensor(xs, dtype=torch.int32, device=dev)
+            mk = lambda xs: _lib.upload_ints(xs, kv_cache)
             starts, counts, dsts = mk([g[2] for g in segs]), mk([g[3] for g in segs]), mk(dst)
             for view, dview, g in ((views[0], dviews[0], gk), (views[1], dviews[1], gv)):
                 w = self._layer_weights(g, l0, l1, kv_cache.dtype, dev)
