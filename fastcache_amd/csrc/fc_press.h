@@ -37,7 +37,7 @@ __device__ __forceinline__ void kp_select_and_move(const KvView& kv, const KvVie
     sel[pos] = i;
   };
   if (LEAN && n <= THREADS * KP_KPT)
-    tk_select_row_regs<THREADS, KP_KPT>(sh.reg_keys, key_at, n, want, emit);
+    tk_select_row_regs<THREADS, KP_KPT>(sh.reg_keys, nullptr, key_at, n, want, emit);
   else
     tk_select_row<THREADS>(sh.lds_keys, key_at, n, want, emit);
   for (int i = tid; i < tail_kept; i += THREADS) emit(want + i, n + i);

@@ -126,6 +126,22 @@ __device__ __forceinline__ void tk_select_row(TkShared<THREADS>& sh, KeyAt key_a
   }
 }
 
+// orders a wavefront's LDS writes before its following LDS reads of other lanes' data, and the other way round
+__device__ __forceinline__ void tk_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Smallest and largest of an unsigned value over the wavefront, wave-uniform.
+__device__ __forceinline__ void tk_wave_range(unsigned& lo, unsigned& hi) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, (unsigned)__shfl_xor((int)lo, o, 64));
+    hi = max(hi, (unsigned)__shfl_xor((int)hi, o, 64));
+  }
+}
+
 // The same selection with the row's keys held in registers: every wavefront owns a contiguous segment of the row and
 // its lane l the keys segment + e * 64 + l, e < KPT, read and converted ONCE (key_at is called once per key), so the
 // digit passes and the ordered pass cost a handful of vector instructions per key instead of an LDS read and a
@@ -134,44 +150,112 @@ __device__ __forceinline__ void tk_select_row(TkShared<THREADS>& sh, KeyAt key_a
 // workgroups keep the compute unit busy every barrier costs about a microsecond, so the passes are arranged for few
 // of them: one per digit pass (every wavefront scans the 256 bins for itself instead of sharing a scan through LDS;
 // three histograms in rotation, so that clearing the next one needs no barrier of its own) and one before the
-// ordered pass.  The digit passes stop as soon as every key left in the threshold bin is kept (then no tie has to
-// be ranked): rows of distinct scores end after two or three passes.
-// Keys never produced by tk_key (0) stand for "no key here"; they rank below every real key.
+// ordered pass.  The digits are those of the key's distance from the row's smallest key, counted from the highest bit
+// that differs within the row: the scores of a row share their leading bits, and digits cut at fixed places would put
+// most keys of the first passes into one or two bins, where their LDS atomics queue up.  The digit passes stop as
+// soon as every key left in the threshold bin is kept (then no tie has to be ranked): rows of distinct scores end
+// after two passes.
+// Keys never produced by tk_key (0) stand for "no key here".
 template <int THREADS>
 struct TkSharedRegs {
   unsigned hist[3][TK_BINS];
   unsigned w_eq[THREADS / FC_WAVE], w_gt[THREADS / FC_WAVE];
+  unsigned w_lo[THREADS / FC_WAVE], w_hi[THREADS / FC_WAVE];
 };
 
-template <int THREADS, int KPT, typename KeyAt, typename Emit>
-__device__ __forceinline__ void tk_select_row_regs(TkSharedRegs<THREADS>& sh, KeyAt key_at, int n, int kk, Emit emit) {
+// Where the keys of a row lie: key e of this lane is row position pos(e), if e < live and pos(e) < end.
+template <int THREADS>
+struct TkSegment {
+  int beg, end, live;
+  __device__ __forceinline__ explicit TkSegment(int n) {
+    constexpr int WAVES = THREADS / FC_WAVE;
+    const int seg = (((n + WAVES - 1) / WAVES) + 63) & ~63;   // <= KPT * 64 by the caller's bound
+    beg = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) * seg;
+    end = min(n, beg + seg);
+    live = end > beg ? (end - beg + 63) >> 6 : 0;             // wave-uniform: 64-key groups of this wavefront
+  }
+  __device__ __forceinline__ int pos(int e) const { return beg + e * 64 + ((int)threadIdx.x & 63); }
+};
+
+// A lane's keys: REGS in registers and, of more, the rest in LDS (`rest`, TK_LDS_KEYS(THREADS, KPT) words).  Loops over
+// the keys are unrolled, so which of the two a key is in is decided at compile time.
+#define TK_REGS(KPT) ((KPT) <= 40 ? (KPT) : 40)
+#define TK_LDS_KEYS(THREADS, KPT) (((KPT) - TK_REGS(KPT)) * (THREADS))
+template <int THREADS, int KPT>
+struct TkKeys {
+  unsigned reg[TK_REGS(KPT)];
+  unsigned* mine;
+  __device__ __forceinline__ explicit TkKeys(unsigned* rest) {
+    mine = rest + ((int)threadIdx.x >> 6) * (KPT - TK_REGS(KPT)) * 64 + ((int)threadIdx.x & 63);
+  }
+  __device__ __forceinline__ unsigned get(int e) const { return e < TK_REGS(KPT) ? reg[e < TK_REGS(KPT) ? e : 0] : mine[(e - TK_REGS(KPT)) * 64]; }
+  __device__ __forceinline__ void set(int e, unsigned v) {
+    if (e < TK_REGS(KPT)) reg[e < TK_REGS(KPT) ? e : 0] = v;
+    else mine[(e - TK_REGS(KPT)) * 64] = v;
+  }
+};
+
+// The number of live key groups as a value of its own, for one unrolled loop: taken from the common variable, the compiler
+// would keep a lane mask for each of the comparisons from loop to loop, in spilled registers.
+__device__ __forceinline__ int tk_live_here(int live) {
+  asm volatile("" : "+s"(live));
+  return live;
+}
+
+// Ends every eighth key of an unrolled loop of a long row: loads of more keys at once than that would be kept in registers
+// that the keys need.
+#define TK_EIGHT(KPT, e) do { if ((KPT) > TK_REGS(KPT) && ((e) & 7) == 7) __builtin_amdgcn_sched_barrier(0); } while (0)
+
+// ... with the keys already there (0 where there is none)
+template <int THREADS, int KPT, typename Emit>
+__device__ __forceinline__ void tk_select_loaded(TkSharedRegs<THREADS>& sh, const TkSegment<THREADS>& sg, TkKeys<THREADS, KPT>& key,
+                                                 int kk, Emit emit) {
   constexpr int WAVES = THREADS / FC_WAVE;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int seg = (((n + WAVES - 1) / WAVES) + 63) & ~63;   // <= KPT * 64 by the caller's bound
-  const int beg = wave * seg;
-  const int end = min(n, beg + seg);
-  const int live_e = end > beg ? (end - beg + 63) >> 6 : 0;   // wave-uniform: 64-key groups of this wavefront
-  unsigned key[KPT];
+  unsigned lo = 0xffffffffu, hi = 0;
 #pragma unroll
   for (int e = 0; e < KPT; ++e) {
-    const int i = beg + e * 64 + lane;
-    key[e] = (e < live_e && i < end) ? key_at(i) : 0u;
+    const unsigned u = key.get(e);
+    if (u != 0u) lo = min(lo, u);
+    hi = max(hi, u);
+    TK_EIGHT(KPT, e);
   }
+  tk_wave_range(lo, hi);
   for (int i = tid; i < 2 * TK_BINS; i += THREADS) (&sh.hist[0][0])[i] = 0;   // histograms of the first two passes
+  if (lane == 0) { sh.w_lo[wave] = lo; sh.w_hi[wave] = hi; }
   __syncthreads();
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    lo = min(lo, sh.w_lo[w]);
+    hi = max(hi, sh.w_hi[w]);
+  }
+  // from here on a key stands as its distance from the smallest one, plus one (0 stays "no key"); the largest key is
+  // below 2^32 - 1 above the smallest, whose own distance is at least tk_key(-inf), so nothing wraps
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    const unsigned u = key.get(e);
+    key.set(e, u != 0u ? u - lo + 1u : 0u);
+    TK_EIGHT(KPT, e);
+  }
+  const unsigned span = hi - lo + 1u;
   unsigned prefix = 0, mask = 0, remaining = (unsigned)kk;
   bool whole_bin = false;   // every key that matches the prefix so far is kept
-  int pass = 0;
-  for (int shift = 24; shift >= 0 && !whole_bin; shift -= 8, ++pass) {
+  int top = 32 - __clz((int)span);   // bits not yet looked at
+  for (int pass = 0; top > 0 && !whole_bin; ++pass) {
+    const int shift = max(top - 8, 0);
+    const unsigned dmask = (1u << (top - shift)) - 1u;
+    top = shift;
     unsigned* hist = sh.hist[pass % 3];
     if (pass >= 1)   // the histogram of the pass after this one; its last readers are two barriers back
       for (int i = tid; i < TK_BINS; i += THREADS) sh.hist[(pass + 1) % 3][i] = 0;
+    const int live_e = tk_live_here(sg.live);
 #pragma unroll
     for (int e = 0; e < KPT; ++e) {
       if (e < live_e) {
-        const unsigned u = key[e];
-        if (u != 0u && (u & mask) == prefix) atomicAdd(&hist[(u >> shift) & 255u], 1u);
+        const unsigned u = key.get(e);
+        if (u != 0u && (u & mask) == prefix) atomicAdd(&hist[(u >> shift) & dmask], 1u);
       }
+      TK_EIGHT(KPT, e);
     }
     __syncthreads();
     // every wavefront for itself: lane t holds bins 255 - 4t .. 252 - 4t (descending), suffix sums over the 256 bins
@@ -205,20 +289,22 @@ __device__ __forceinline__ void tk_select_row_regs(TkSharedRegs<THREADS>& sh, Ke
     remaining = __shfl(left, src, 64);
     whole_bin = __shfl(size, src, 64) == remaining;
     prefix |= bin << shift;
-    mask |= 255u << shift;
+    mask |= dmask << shift;
   }
   // kept: keys whose masked bits exceed the prefix, and of those that equal it the first `remaining` by index
-  // (all of them when whole_bin; after four passes the masked bits are the whole key)
+  // (all of them when whole_bin; after the last pass the masked bits are the whole key)
   const unsigned T = prefix;
   const unsigned need = remaining;
   unsigned eq_cnt = 0, gt_cnt = 0;
+  const int live_c = tk_live_here(sg.live);
 #pragma unroll
   for (int e = 0; e < KPT; ++e) {
-    if (e < live_e) {
-      const unsigned u = key[e], m = u & mask;
+    if (e < live_c) {
+      const unsigned u = key.get(e), m = u & mask;
       eq_cnt += __popcll(__ballot(u != 0u && m == T));
       gt_cnt += __popcll(__ballot(u != 0u && m > T));
     }
+    TK_EIGHT(KPT, e);
   }
   if (lane == 0) { sh.w_eq[wave] = eq_cnt; sh.w_gt[wave] = gt_cnt; }
   __syncthreads();
@@ -233,20 +319,42 @@ __device__ __forceinline__ void tk_select_row_regs(TkSharedRegs<THREADS>& sh, Ke
     eq_seen = eq_run;
   }
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const int live_o = tk_live_here(sg.live);
+  int first = sg.pos(0);
+  asm volatile("" : "+v"(first));   // likewise: the positions are computed again, not kept from when the keys were read
 #pragma unroll
   for (int e = 0; e < KPT; ++e) {
-    if (e < live_e) {
-      const unsigned u = key[e], m = u & mask;
+    if (e < live_o) {
+      const unsigned u = key.get(e), m = u & mask;
       const bool is_eq = u != 0u && m == T;
       const unsigned long long eqb = __ballot(is_eq);
       const unsigned my_rank = eq_seen + __popcll(eqb & lt_mask);
       const bool sel = u != 0u && (m > T || (is_eq && my_rank < need));
       const unsigned long long sb = __ballot(sel);
-      if (sel) emit((int)(out_pos + __popcll(sb & lt_mask)), beg + e * 64 + lane);
+      if (sel) emit((int)(out_pos + __popcll(sb & lt_mask)), first + e * 64);
       eq_seen += __popcll(eqb);
       out_pos += __popcll(sb);
     }
+    TK_EIGHT(KPT, e);
   }
+}
+
+template <int THREADS, int KPT, typename KeyAt, typename Emit>
+__device__ __forceinline__ void tk_select_row_regs(TkSharedRegs<THREADS>& sh, unsigned* rest, KeyAt key_at, int n, int kk, Emit emit) {
+  const TkSegment<THREADS> sg(n);
+  TkKeys<THREADS, KPT> key(rest);
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    const int i = sg.pos(e);
+    if constexpr (KPT > TK_REGS(KPT)) {   // always a load, of an existing key: 72 lane masks would not fit the registers
+      const unsigned u = key_at(min(i, n - 1));
+      key.set(e, e < sg.live && i < sg.end ? u : 0u);
+    } else {
+      key.set(e, (e < sg.live && i < sg.end) ? key_at(i) : 0u);
+    }
+    TK_EIGHT(KPT, e);
+  }
+  tk_select_loaded<THREADS, KPT>(sh, sg, key, kk, emit);
 }
 
 // LDS of whichever form of the selection a kernel ends up calling

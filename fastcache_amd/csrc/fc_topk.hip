@@ -1,27 +1,25 @@
 // Row-wise top-k selection with lowest-index tie-break and ascending-index output.
 //
-// One workgroup per score row: 4 wavefronts, or 16 for rows of more than 8192 scores (few such rows make a
-// launch, so each has to be walked by more lanes).  The row is mapped to order-preserving 32-bit
-// keys and staged in LDS; an MSB-first radix select (4 passes of 8 bits, LDS histogram) finds
-// the exact key T of the k-th largest element and how many elements equal to T are still
-// needed.  A final ordered pass keeps every key > T plus the first `need` keys == T in index
-// order, using wavefront ballots for the running ranks, so the output is ascending and
-// deterministic.  Rows too long for LDS are re-read from global memory (L2-resident).
+// One workgroup per score row, the row's order-preserving 32-bit keys in registers (tk_select_row_regs): 256 threads for
+// rows of up to 512 scores, 512 up to 4096, 1024 up to 16 384, where few such rows make a launch and each has to be
+// walked by more lanes, 512 again up to 36 864 with part of the keys in LDS, so that two rows share a compute unit (288
+// rows of 30 000: 47 us; 71 us with 1024 threads and one row at a time).  Longer
+// rows are selected with the keys re-read from global memory (L2-resident), four passes of 8 bits over an LDS histogram
+// and an ordered pass.  Bound by the chain of short steps of a row, not by its bytes.
 #include "fc_select.h"
 
-#define TK_LDS_MAX_KEYS 15360        // 60 KiB of keys: several workgroups of 256 threads per CU
-#define TK_LONG_ROW 8192             // rows longer than this take 1024 threads
-#define TK_LDS_MAX_KEYS_LONG 36864   // 144 KiB of keys: one workgroup of 1024 threads per CU
+#define TK_MAX_REG_KEYS (512 * 72)
 
-template <bool LDS_KEYS, int TK_THREADS>
-__global__ __launch_bounds__(TK_THREADS) void topk_kernel(const float* __restrict__ scores,
+// KPT = keys per thread in registers; 0 = re-read from memory
+template <int TK_THREADS, int KPT>
+__global__ __launch_bounds__(TK_THREADS, KPT > 16 ? 4 : 1) void topk_kernel(const float* __restrict__ scores,
                                                           int score_stride, int len,
                                                           const int* __restrict__ row_lens,
                                                           int rows_per_len, int row_lens_mod, int k,
                                                           const int* __restrict__ n_kept,
                                                           int* __restrict__ indices, int index_stride) {
-  extern __shared__ __align__(16) unsigned lds_keys[];
-  __shared__ TkShared<TK_THREADS> sh;
+  __shared__ TkArea<TK_THREADS> sh;
+  __shared__ unsigned rest[TK_LDS_KEYS(TK_THREADS, KPT) + 1];
 
   const int r = blockIdx.x;
   const int tid = threadIdx.x;
@@ -39,31 +37,12 @@ __global__ __launch_bounds__(TK_THREADS) void topk_kernel(const float* __restric
     for (int i = tid; i < n; i += TK_THREADS) out[i] = i;
     return;
   }
-
-  if (LDS_KEYS) {
-    // 16-byte loads, four per thread in flight, when the row starts on a 16-byte boundary
-    int done = 0;
-    if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {
-      const float4* row4 = reinterpret_cast<const float4*>(row);
-      uint4* keys4 = reinterpret_cast<uint4*>(lds_keys);
-      const int n4 = n >> 2;
-      for (int i0 = 0; i0 < n4; i0 += 4 * TK_THREADS) {
-        float4 v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = row4[min(i0 + u * TK_THREADS + tid, n4 - 1)];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int i = i0 + u * TK_THREADS + tid;
-          if (i < n4) keys4[i] = make_uint4(tk_key(v[u].x), tk_key(v[u].y), tk_key(v[u].z), tk_key(v[u].w));
-        }
-      }
-      done = n4 << 2;
-    }
-    for (int i = done + tid; i < n; i += TK_THREADS) lds_keys[i] = tk_key(row[i]);
-  }
-  auto key_at = [&](int i) -> unsigned { return LDS_KEYS ? lds_keys[i] : tk_key(row[i]); };
-
-  tk_select_row<TK_THREADS>(sh, key_at, n, kk, [&](int pos, int i) { out[pos] = i; });
+  auto key_at = [&](int i) -> unsigned { return tk_key(row[i]); };
+  auto emit = [&](int pos, int i) { out[pos] = i; };
+  if constexpr (KPT > 0)
+    tk_select_row_regs<TK_THREADS, KPT>(sh.reg_keys, rest, key_at, n, kk, emit);
+  else
+    tk_select_row<TK_THREADS>(sh.lds_keys, key_at, n, kk, emit);
 }
 
 extern "C" int fc_topk_select(const float* scores, int32_t score_stride, int32_t rows, int32_t len,
@@ -81,17 +60,14 @@ extern "C" int fc_topk_select(const float* scores, int32_t score_stride, int32_t
              FC_EINVAL, "fc_topk_select: rows_per_len and row_lens_mod must be positive when per-row sizes are given");
   if (rows == 0 || len == 0) return FC_OK;
   hipStream_t st = (hipStream_t)stream;
-#define TK_LAUNCH(LK, TH, LDSB)                                                                                    \
-  hipLaunchKernelGGL((topk_kernel<LK, TH>), dim3(rows), dim3(TH), (size_t)(LDSB), st, scores, score_stride, len,  \
-                     row_lens, rows_per_len, row_lens_mod, k, n_kept, indices, index_stride)
-  if (len <= TK_LONG_ROW) {
-    TK_LAUNCH(true, 256, (size_t)len * 4);
-  } else if (len <= TK_LDS_MAX_KEYS_LONG) {
-    FC_ALLOW_LDS((topk_kernel<true, 1024>), TK_LDS_MAX_KEYS_LONG * 4);
-    TK_LAUNCH(true, 1024, (size_t)len * 4);
-  } else {
-    TK_LAUNCH(false, 1024, 0);
-  }
+#define TK_LAUNCH(TH, KPT)                                                                                         \
+  hipLaunchKernelGGL((topk_kernel<TH, KPT>), dim3(rows), dim3(TH), 0, st, scores, score_stride, len, row_lens,     \
+                     rows_per_len, row_lens_mod, k, n_kept, indices, index_stride)
+  if (len <= 512) TK_LAUNCH(256, 2);
+  else if (len <= 4096) TK_LAUNCH(512, 8);
+  else if (len <= 16384) TK_LAUNCH(1024, 16);
+  else if (len <= TK_MAX_REG_KEYS) TK_LAUNCH(512, 72);
+  else TK_LAUNCH(1024, 0);
 #undef TK_LAUNCH
   FC_CHECK_LAUNCH("fc_topk_select");
   return FC_OK;

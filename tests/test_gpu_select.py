@@ -27,6 +27,26 @@ def test_topk_random_and_tied_rows(dev, S, k):
         assert bool((got[..., 1:] > got[..., :-1]).all()) if k > 1 else True
 
 
+@pytest.mark.parametrize("S", [512, 513, 4096, 4097, 16384, 16385, 36864, 36865])
+def test_topk_row_length_limits(dev, S):
+    """Row lengths on both sides of every change of launch shape, continuous and heavily tied (negative, equal and
+    near-equal scores: the digits are cut within the row's own range), with shorter rows in the same launch."""
+    g = torch.Generator().manual_seed(S)
+    base = torch.randn(6, S, generator=g)
+    base[1] = torch.randint(0, 3, (S,), generator=g).float() - 4.0
+    base[2] = -7.25
+    base[3] = 1000.0 + base[3] * 1e-3
+    base[4, ::2] = -float("inf")
+    for k in (1, S // 3, S - 1):
+        assert torch.equal(ops.topk_select(base.to(dev), k).cpu().long(), opress.topk_lowest_index(base, k)), k
+    lens = [S, S - 63, S // 2 + 1, 65, 3, 1]
+    kept = [S // 4, S // 4, S // 2, 64, 2, 1]
+    got = ops.topk_select(base.to(dev), max(kept), row_lens=torch.tensor(lens, dtype=torch.int32, device=dev),
+                          n_kept=torch.tensor(kept, dtype=torch.int32, device=dev)).cpu().long()
+    for r, (n, kk) in enumerate(zip(lens, kept)):
+        assert torch.equal(got[r, :kk], opress.topk_lowest_index(base[r, :n], kk))
+
+
 def test_topk_special_values(dev):
     """NaN ranks above +inf, -0 equals +0 (the lower index wins), -inf is taken last."""
     row = torch.tensor([0.0, -0.0, float("inf"), float("nan"), -float("inf"), 1.0, float("nan"), -1.0, 0.0, 1.0])
