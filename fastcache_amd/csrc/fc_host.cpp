@@ -258,6 +258,80 @@ PyObject* py_ccm_layers(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   });
 }
 
+// ---- presses on one layer's dense tensors -------------------------------------------------------------------------------------
+// [B, H, S, D] K and V of one geometry on one GPU, and a kept count the out-of-place kernels take
+bool press_takes(const at::Tensor& k, const at::Tensor& v, int64_t n) {
+  return k.is_cuda() && v.device() == k.device() && k.dim() == 4 && k.sizes() == v.sizes() &&
+         k.scalar_type() == v.scalar_type() && k.stride(3) == 1 && v.stride(3) == 1 && n > 0 && n <= k.size(2) &&
+         k.numel() > 0 && k.size(2) <= 36864;
+}
+
+PyObject* pair(at::Tensor a, at::Tensor b) {
+  PyObject* out = PyTuple_New(2);
+  if (!out) throw PyFailed();
+  PyTuple_SET_ITEM(out, 0, wrap(std::move(a)));
+  PyTuple_SET_ITEM(out, 1, wrap(std::move(b)));
+  return out;
+}
+
+// knorm_into(keys, values, n) -> (k, v) [B, H, n, D], or None
+PyObject* py_knorm_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    need_args(nargs, 3, "knorm_into");
+    if (!is_tensor(args[0]) || !is_tensor(args[1])) Py_RETURN_NONE;
+    const at::Tensor &k = THPVariable_Unpack(args[0]), &v = THPVariable_Unpack(args[1]);
+    const int64_t n = as_int(args[2]);
+    if (!press_takes(k, v, n)) Py_RETURN_NONE;
+    const int64_t B = k.size(0), H = k.size(1), S = k.size(2), D = k.size(3);
+    at::Tensor ok = at::empty({B, H, n, D}, k.options()), ov = at::empty({B, H, n, D}, k.options()), scores;
+    const fc_kv_view kv = dense_view(k, 1, 0), vv = dense_view(v, 1, 0), dk = dense_view(ok, 1, 0), dv = dense_view(ov, 1, 0);
+    // short columns are scored by the workgroups that gather them, each for itself; longer ones by the whole chip first
+    float* sp = nullptr;
+    if (S > 1024) {
+      scores = at::empty({B, H, S}, k.options().dtype(at::kFloat));
+      sp = scores.data_ptr<float>();
+    }
+    check(fc_knorm_press_into(&kv, &vv, &dk, &dv, (int32_t)n, sp, (int32_t)S, stream_of(k)), "fc_knorm_press_into");
+    return pair(std::move(ok), std::move(ov));
+  });
+}
+
+// snapkv_into(keys, values, queries, lse or None, n, window, kernel_size, causal, scale, out_scale) -> (k, v), or None
+PyObject* py_snapkv_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    need_args(nargs, 10, "snapkv_into");
+    for (int i = 0; i < 3; ++i)
+      if (!is_tensor(args[i])) Py_RETURN_NONE;
+    const at::Tensor &k = THPVariable_Unpack(args[0]), &v = THPVariable_Unpack(args[1]), &q = THPVariable_Unpack(args[2]);
+    const int64_t n = as_int(args[4]), W = as_int(args[5]), ksz = as_int(args[6]), causal = as_int(args[7]);
+    const double scale = PyFloat_AsDouble(args[8]), out_scale = PyFloat_AsDouble(args[9]);
+    if (PyErr_Occurred()) throw PyFailed();
+    if (!press_takes(k, v, n) || q.dim() != 4 || q.device() != k.device() || q.scalar_type() != k.scalar_type() ||
+        !q.is_contiguous() || (k.scalar_type() != at::kHalf && k.scalar_type() != at::kBFloat16))
+      Py_RETURN_NONE;
+    const int64_t B = k.size(0), H = k.size(1), S = k.size(2), D = k.size(3), hq = q.size(1);
+    if (q.size(0) != B || q.size(2) != W || q.size(3) != D || hq % H || (hq / H) * ((W + 31) / 32) > 16 || n <= W ||
+        S - W <= ksz || ksz < 1 || !(ksz & 1) || ksz > 63)
+      Py_RETURN_NONE;
+    const float* lse = nullptr;
+    if (args[3] != Py_None) {
+      const at::Tensor& t = tensor(args[3], "lse");
+      if (t.device() != k.device() || t.scalar_type() != at::kFloat || !t.is_contiguous() || t.numel() != B * hq * W) Py_RETURN_NONE;
+      lse = t.const_data_ptr<float>();
+    }
+    at::Tensor ok = at::empty({B, H, n, D}, k.options()), ov = at::empty({B, H, n, D}, k.options());
+    const fc_kv_view kv = dense_view(k, 1, 0), vv = dense_view(v, 1, 0), dk = dense_view(ok, 1, 0), dv = dense_view(ov, 1, 0);
+    const int32_t nsplit = fc_snapkv_select_splits(&kv, (int32_t)hq, (int32_t)W);
+    const int64_t bytes = fc_snapkv_select_workspace_bytes(1, (int32_t)B, (int32_t)hq, (int32_t)H, (int32_t)W, (int32_t)S, nsplit);
+    at::Tensor ws = at::empty({bytes}, k.options().dtype(at::kByte));
+    check(fc_snapkv_press_into(&kv, &vv, &dk, &dv, q.const_data_ptr(), lse, (int32_t)hq, (int32_t)W, (int32_t)ksz,
+                               (int32_t)causal, (float)scale, (float)out_scale, (int32_t)n, nsplit, ws.data_ptr(), bytes,
+                               stream_of(k)),
+          "fc_snapkv_press_into");
+    return pair(std::move(ok), std::move(ov));
+  });
+}
+
 // ---- one attention layer of a decode step ---------------------------------------------------------------------------------
 // decode_layer(q, k, v, k_cache, v_cache, slot_mapping, context_lens, block_tables, scale, q_heads, kv_heads, head_dim,
 //              workspace or None) -> out [n, q_heads * head_dim], or None when the arguments are not the plain decode
@@ -508,6 +582,9 @@ PyMethodDef kMethods[] = {
      "decode_inputs(ids, lens, tables, block_size, ref) -> five device tensors"},
     {"upload_tables", (PyCFunction)(void (*)(void))py_upload_tables, METH_FASTCALL,
      "upload_tables(tables, (list, ...), ref) -> device tensors"},
+    {"knorm_into", (PyCFunction)(void (*)(void))py_knorm_into, METH_FASTCALL, "knorm_into(keys, values, n) -> (k, v) or None"},
+    {"snapkv_into", (PyCFunction)(void (*)(void))py_snapkv_into, METH_FASTCALL,
+     "snapkv_into(keys, values, queries, lse, n, window, kernel_size, causal, scale, out_scale) -> (k, v) or None"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "host path of fastcache_amd", -1, kMethods, nullptr, nullptr, nullptr, nullptr};

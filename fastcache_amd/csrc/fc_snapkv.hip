@@ -31,6 +31,7 @@
 // Table entries of a live sequence must be allocated blocks: a negative entry inside the sequence
 // reads block 0 instead of faulting.
 #include "fc_press.h"
+#include "fc_tail.h"
 
 #define SK_KT 64           // keys per tile
 #define SK_TILEB (SK_KT * 256)  // LDS bytes per key tile (rows unpadded, 16-byte chunks XOR-swizzled)
@@ -420,6 +421,18 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
     if (lse && ok)   // natural-log sum of exp(scale * q.k) over the keys the query sees
       nmfin = -1.4426950408889634f *
               lse[((((long long)l * kv.batch + b) * Hq + (h * G + qg)) * W + qi + lrow)];
+    if constexpr (MODE == 2) {
+      if (!lse && ok) {   // the pieces' (max, sum) into the log-sum-exp, by every workgroup for its own queries
+        const float* pp = part + ((((long long)l * kv.batch + b) * Hq + (h * G + qg)) * W + qi + lrow) * nsplit * 2;
+        const int used = (T + (T + nsplit - 1) / nsplit - 1) / ((T + nsplit - 1) / nsplit);   // pieces that had tiles
+        float M = SK_NEG;
+        for (int s = 0; s < used; ++s) M = fmaxf(M, pp[2 * s]);
+        float L = 0.f;
+        for (int s = 0; s < used; ++s) L += pp[2 * s + 1] * sk_exp2(pp[2 * s] - M);
+        nmfin = -1.4426950408889634f * ((M + __builtin_amdgcn_logf(L)) * 0.6931471805599453f);
+      }
+      if (row_max && split == 0 && tid == 0) row_max[((long long)l * kv.batch + b) * Hkv + h] = -INFINITY;
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) nm[i] = __shfl(nmfin, (i >> 2) * 8 + lhalf * 4 + (i & 3), 64);
   }
@@ -558,49 +571,31 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
   }
 }
 
-// Split columns: the pieces' (max, sum) per window query -> natural-log sum of exponentials.
-__global__ __launch_bounds__(256) void snapkv_merge_stats_kernel(const float* __restrict__ part, long long queries_total,
-                                                                 int queries_per_seq, int batch,
-                                                                 const int* __restrict__ seq_lens, int max_seq_len,
-                                                                 int nsplit, float* __restrict__ lse) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;   // (layer, b, hq, w) flattened
-  if (i >= queries_total) return;
-  const int b = (int)((i / queries_per_seq) % batch);
-  int S = seq_lens ? seq_lens[b] : max_seq_len;
-  S = S < max_seq_len ? (S < 0 ? 0 : S) : max_seq_len;
-  const int T = (S + SK_KT - 1) / SK_KT;
-  if (T == 0) return;
-  const int tps = (T + nsplit - 1) / nsplit;
-  const int used = (T + tps - 1) / tps;                            // pieces that had tiles
-  const float* pp = part + i * nsplit * 2;
-  float M = SK_NEG;
-  for (int s = 0; s < used; ++s) M = fmaxf(M, pp[2 * s]);
-  float L = 0.f;
-  for (int s = 0; s < used; ++s) L += pp[2 * s + 1] * sk_exp2(pp[2 * s] - M);
-  lse[i] = (M + __builtin_amdgcn_logf(L)) * 0.6931471805599453f;   // log2 units -> natural log
-}
-
-// Split columns: zero-padded moving average of the raw per-key sums, the tail past the sequence, the row maximum.
+// Split columns: zero-padded moving average of the raw per-key sums, the tail past the sequence, the row maximum (which
+// the summing kernel has set to -inf; scores are not negative, so their bits are ordered like integers).  A workgroup
+// takes SP_KEYS keys of a row: one per row left 30 000 keys to 256 threads (146 us on 288 rows, 20 now).
+#define SP_KEYS 1024
 __global__ __launch_bounds__(256) void snapkv_pool_kernel(const float* __restrict__ raw, float* __restrict__ scores,
-                                                          int score_stride, const int* __restrict__ seq_lens,
+                                                          int score_stride, int Hkv, const int* __restrict__ seq_lens,
                                                           int max_seq_len, int W, int ksz, float out_mul,
                                                           float* __restrict__ row_max) {
-  __shared__ float red[4];
-  const int h = blockIdx.x, b = blockIdx.y, l = blockIdx.z;
-  const long long row = ((long long)l * gridDim.y + b) * gridDim.x + h;
+  const int pieces = gridDim.x / Hkv;
+  const int h = blockIdx.x / pieces, b = blockIdx.y, l = blockIdx.z;
+  const int s0 = (blockIdx.x - h * pieces) * SP_KEYS, s1 = min(s0 + SP_KEYS, score_stride);
+  const long long row = ((long long)l * gridDim.y + b) * Hkv + h;
   int S = seq_lens ? seq_lens[b] : max_seq_len;
   S = S < max_seq_len ? (S < 0 ? 0 : S) : max_seq_len;
   const float* in = raw + row * score_stride;
   float* out = scores + row * score_stride;
   const int tid = threadIdx.x;
   if (S <= W) {
-    for (int s = tid; s < score_stride; s += 256) out[s] = s < S ? 0.f : -INFINITY;
-    if (row_max && tid == 0) row_max[row] = -INFINITY;
+    for (int s = s0 + tid; s < s1; s += 256) out[s] = s < S ? 0.f : -INFINITY;
+    if (row_max && s0 == 0 && tid == 0) row_max[row] = -INFINITY;
     return;
   }
   const int SW = S - W, hw = ksz >> 1;
   float mx = -INFINITY;
-  for (int s = tid; s < score_stride; s += 256) {
+  for (int s = s0 + tid; s < s1; s += 256) {
     if (s < SW) {
       float a = 0.f;
       for (int x = max(s - hw, 0); x <= min(s + hw, SW - 1); ++x) a += in[x];
@@ -613,9 +608,7 @@ __global__ __launch_bounds__(256) void snapkv_pool_kernel(const float* __restric
   }
   if (row_max) {
     mx = fc_wave_max(mx);
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    if (tid == 0) row_max[row] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if ((tid & 63) == 0 && mx >= 0.f) atomicMax(reinterpret_cast<int*>(row_max + row), __float_as_int(mx));
   }
 }
 
@@ -799,6 +792,40 @@ extern "C" int fc_snapkv_press(const fc_kv_view* keys, const fc_kv_view* values,
 }
 
 // ---- split columns ------------------------------------------------------------------------------------
+// Key ranges per column (nsplit workgroups each, 1 = whole columns in one launch).  One workgroup per column leaves most
+// of the chip idle below a thousand columns; too many pay a workgroup's start (queries, table, first tiles: f) for a
+// handful of tiles.  A compute unit works its workgroups off one after the other (two at a time share its matrix pipes
+// and gain nothing, except with four wavefronts, of which one or two multiply), so a sweep takes
+//   ceil(columns * n / slots) * (tiles per range * a + f)
+// with a microseconds per 64-key tile and f per start, and n with the smallest sum is taken (whole columns do both
+// sweeps in one start).  Fitted to and checked against measurements (us for scoring + selection by n, window 64 unless
+// said): 8 columns x 1024 keys 46 / 32 / 26 / 23 for n = 1 / 2 / 4 / 8; 32 x 4096 154 / 90 / 60 / 48, 62 with 16;
+// 288 x 4096 254 / 228 / 220 / 248; 288 x 30011 1897 / 1572 / 1421 / 1387, 1466 with 16; 4 x 12000 (7 heads a group)
+// 667 / 342 / 194 / 123, 83 with 24; 448 x 3000 431 / 460 / 471; 256 x 2000 (window 32) 75 / 57 / 68.
+// 1 also when the split kernels do not apply (more than 16 query row blocks per kv head, pages that are no multiple of
+// 64 tokens).
+extern "C" int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) {
+  if (!keys || keys->num_kv_heads <= 0 || window <= 0) return 1;
+  const long long columns = (long long)keys->num_layers * keys->batch * keys->num_kv_heads;
+  const int blocks = (num_q_heads / keys->num_kv_heads) * ((window + 31) / 32);
+  const int tiles = (keys->max_seq_len + SK_KT - 1) / SK_KT;
+  const bool paged_ok = !keys->block_tables || (keys->block_size >= SK_KT && (keys->block_size & (keys->block_size - 1)) == 0 &&
+                                                (keys->max_seq_len - 1) / keys->block_size < SK_TBL);
+  if (columns <= 0 || columns >= 1000 || blocks > 16 || !paged_ok) return 1;
+  const double a = blocks > 8 ? 1.7 : blocks > 4 ? 0.83 : 0.7, f = blocks > 8 ? 9.0 : 7.0;
+  const long long slots = blocks > 4 ? 256 : 512;
+  int best_n = 1;
+  double best = (double)((columns + slots - 1) / slots) * (2.0 * tiles * a + f);
+  for (int n = 2; n <= 32 && n * 2 <= tiles; ++n) {
+    const double cost = 2.0 * (double)((columns * n + slots - 1) / slots) * ((tiles + n - 1) / n * a + f);
+    if (cost < best) {
+      best = cost;
+      best_n = n;
+    }
+  }
+  return best_n;
+}
+
 extern "C" int64_t fc_snapkv_split_workspace_bytes(int32_t num_layers, int32_t batch, int32_t num_q_heads,
                                                    int32_t num_kv_heads, int32_t window, int32_t score_stride,
                                                    int32_t nsplit) {
@@ -809,14 +836,14 @@ extern "C" int64_t fc_snapkv_split_workspace_bytes(int32_t num_layers, int32_t b
   return (nq * nsplit * 2 + nq + (int64_t)num_layers * batch * num_kv_heads * score_stride + 64) * (int64_t)sizeof(float);
 }
 
-extern "C" int fc_snapkv_score_split(const fc_kv_view* keys, const void* queries, const float* lse, int32_t num_q_heads,
-                                     int32_t window, int32_t kernel_size, int32_t causal_window, float scale,
-                                     float out_scale, float* scores, int32_t score_stride, float* row_max,
-                                     int32_t nsplit, void* workspace, int64_t workspace_bytes, void* stream) {
-  const char* who = "fc_snapkv_score_split";
+// The two sweeps of split columns: per-key sums (not yet pooled) in the workspace, whose address goes to *raw_out.
+static int snapkv_split_sums(const char* who, const fc_kv_view* keys, const void* queries, const float* lse,
+                             int32_t num_q_heads, int32_t window, int32_t kernel_size, int32_t causal_window, float scale,
+                             int32_t score_stride, float* row_max, int32_t nsplit, void* workspace, int64_t workspace_bytes,
+                             void* stream, const float** raw_out) {
   int rc = fc_check_view(keys, who);
   if (rc) return rc;
-  FC_REQUIRE(queries && scores && workspace, FC_EINVAL, "%s: null pointer", who);
+  FC_REQUIRE(queries && workspace, FC_EINVAL, "%s: null pointer", who);
   FC_REQUIRE(((uintptr_t)queries & 15) == 0 && ((uintptr_t)workspace & 15) == 0, FC_EINVAL,
              "%s: queries / workspace not 16-byte aligned", who);
   FC_REQUIRE(keys->dtype == FC_F16 || keys->dtype == FC_BF16, FC_EUNSUPPORTED,
@@ -844,42 +871,132 @@ extern "C" int fc_snapkv_score_split(const fc_kv_view* keys, const void* queries
              (long long)workspace_bytes, (long long)need);
   FC_REQUIRE((long long)Hkv * nsplit <= 2147483647LL && B <= 65535 && L <= 65535, FC_EUNSUPPORTED, "%s: grid too large",
              who);
-  if (keys->max_seq_len == 0) return FC_OK;
   const long long nq = (long long)L * B * num_q_heads * window;
   float* part = (float*)workspace;
-  float* lse_ws = part + nq * nsplit * 2;
-  float* raw = lse_ws + nq;
+  float* raw = part + nq * nsplit * 2;
+  *raw_out = raw;
+  if (keys->max_seq_len == 0) return FC_OK;
   hipStream_t st = (hipStream_t)stream;
   const float c = scale * 1.4426950408889634f;
-  const float out_mul = out_scale / (float)kernel_size;
   const char* q = (const char*)queries;
   dim3 grid(Hkv * nsplit, B, L);
-  const float* lse_use = lse;
 #define SK_SPLIT(DT, NWV, MD)                                                                                      \
   do {                                                                                                           \
     FC_ALLOW_LDS((snapkv_kernel<DT, NWV, true, MD>), SkCfg<NWV>::LDS);                                            \
     hipLaunchKernelGGL((snapkv_kernel<DT, NWV, true, MD>), grid, dim3(NWV * 64), SkCfg<NWV>::LDS, st, kv, q,     \
-                       num_q_heads, window, kernel_size, causal_window, c, out_mul, scores, score_stride,        \
-                       row_max, lse_use, nsplit, part, raw, SkPress{});                                          \
+                       num_q_heads, window, kernel_size, causal_window, c, 1.0f, (float*)nullptr, score_stride,  \
+                       row_max, lse, nsplit, part, raw, SkPress{});                                              \
   } while (0)
 #define SK_SPLIT_NW(DT, MD)                     \
   if (waves <= 4) SK_SPLIT(DT, 4, MD);          \
   else if (waves <= 8) SK_SPLIT(DT, 8, MD);     \
   else SK_SPLIT(DT, 16, MD)
-  if (!lse) {   // pieces' statistics, then their merge into the log-sum-exp
+  if (!lse) {   // pieces' statistics; the summing workgroups merge them for their own queries
     if (keys->dtype == FC_BF16) { SK_SPLIT_NW(FC_BF16, 1); } else { SK_SPLIT_NW(FC_F16, 1); }
-    hipLaunchKernelGGL(snapkv_merge_stats_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, st,
-                       (const float*)part, nq, num_q_heads * window, B, keys->seq_lens, keys->max_seq_len, nsplit,
-                       lse_ws);
-    lse_use = lse_ws;
   }
   if (keys->dtype == FC_BF16) { SK_SPLIT_NW(FC_BF16, 2); } else { SK_SPLIT_NW(FC_F16, 2); }
 #undef SK_SPLIT_NW
 #undef SK_SPLIT
-  hipLaunchKernelGGL(snapkv_pool_kernel, dim3(Hkv, B, L), dim3(256), 0, st, (const float*)raw, scores, score_stride,
-                     keys->seq_lens, keys->max_seq_len, window, kernel_size, out_mul, row_max);
   FC_CHECK_LAUNCH(who);
   return FC_OK;
+}
+
+extern "C" int fc_snapkv_score_split(const fc_kv_view* keys, const void* queries, const float* lse, int32_t num_q_heads,
+                                     int32_t window, int32_t kernel_size, int32_t causal_window, float scale,
+                                     float out_scale, float* scores, int32_t score_stride, float* row_max,
+                                     int32_t nsplit, void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* who = "fc_snapkv_score_split";
+  FC_REQUIRE(scores, FC_EINVAL, "%s: null pointer", who);
+  const float* raw = nullptr;
+  const int rc = snapkv_split_sums(who, keys, queries, lse, num_q_heads, window, kernel_size, causal_window, scale,
+                                   score_stride, row_max, nsplit, workspace, workspace_bytes, stream, &raw);
+  if (rc || keys->max_seq_len == 0) return rc;
+  const int pieces = (score_stride + SP_KEYS - 1) / SP_KEYS;
+  FC_REQUIRE((long long)keys->num_kv_heads * pieces <= 2147483647LL, FC_EUNSUPPORTED, "%s: grid too large", who);
+  hipLaunchKernelGGL(snapkv_pool_kernel, dim3(keys->num_kv_heads * pieces, keys->batch, keys->num_layers), dim3(256), 0,
+                     (hipStream_t)stream, raw, scores, score_stride, keys->num_kv_heads, keys->seq_lens, keys->max_seq_len,
+                     window, kernel_size, out_scale / (float)kernel_size, row_max);
+  FC_CHECK_LAUNCH(who);
+  return FC_OK;
+}
+
+// ---- scoring and selection without a score tensor -------------------------------------------------------------------
+extern "C" int64_t fc_snapkv_select_workspace_bytes(int32_t num_layers, int32_t batch, int32_t num_q_heads,
+                                                    int32_t num_kv_heads, int32_t window, int32_t max_seq_len,
+                                                    int32_t nsplit) {
+  return fc_snapkv_split_workspace_bytes(num_layers, batch, num_q_heads, num_kv_heads, window, max_seq_len, nsplit);
+}
+
+// Scores every column (split over nsplit workgroups, or whole with nsplit 1) into the workspace, then selects: the
+// window and the k - window best of the other keys.
+static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                              const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
+                              int32_t window, int32_t kernel_size, int32_t causal_window, float scale, float out_scale,
+                              int32_t k, const int32_t* n_kept, int32_t* indices, int32_t index_stride, int32_t nsplit,
+                              void* workspace, int64_t workspace_bytes, void* stream) {
+  int rc = fc_check_view(keys, who);
+  if (rc) return rc;
+  const int stride = keys->max_seq_len;
+  FC_REQUIRE(n_kept || (k > window && k <= index_stride), FC_EINVAL, "%s: k=%d must exceed the window (%d) and fit %d", who, k,
+             window, index_stride);
+  FC_REQUIRE(index_stride <= stride && stride <= CS_MAX_KEYS, FC_EUNSUPPORTED, "%s: index_stride %d, max_seq_len %d (at most %d)",
+             who, index_stride, stride, CS_MAX_KEYS);
+  ColumnSelect a{};
+  a.stride = stride;
+  a.k = k;
+  a.n_kept = n_kept;
+  a.window = window;
+  a.ksz = kernel_size;
+  a.out_mul = out_scale / (float)kernel_size;
+  a.indices = indices;
+  a.index_stride = index_stride;
+  a.parts = out_k ? fc_gather_parts(keys, k) : 0;
+  if (nsplit > 1) {
+    const float* raw = nullptr;
+    if ((rc = snapkv_split_sums(who, keys, queries, lse, num_q_heads, window, kernel_size, causal_window, scale, stride,
+                                nullptr, nsplit, workspace, workspace_bytes, stream, &raw)))
+      return rc;
+    a.in = raw;
+    return fc_column_select(who, CS_SUMS, keys, values, out_k, out_v, a, (hipStream_t)stream);
+  }
+  FC_REQUIRE(workspace && workspace_bytes >= (int64_t)keys->num_layers * keys->batch * keys->num_kv_heads * stride * 4, FC_EINVAL,
+             "%s: workspace too small", who);
+  float* scores = (float*)workspace;
+  if ((rc = snapkv_score_impl(who, keys, queries, num_q_heads, window, kernel_size, causal_window, scale, out_scale, scores,
+                              stride, nullptr, lse, stream)))
+    return rc;
+  a.in = scores;
+  return fc_column_select(who, CS_SCORES, keys, values, out_k, out_v, a, (hipStream_t)stream);
+}
+
+extern "C" int fc_snapkv_select(const fc_kv_view* keys, const void* queries, const float* lse, int32_t num_q_heads,
+                                int32_t window, int32_t kernel_size, int32_t causal_window, float scale, float out_scale,
+                                int32_t k, const int32_t* n_kept, int32_t* indices, int32_t index_stride, int32_t nsplit,
+                                void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* who = "fc_snapkv_select";
+  FC_REQUIRE(indices && index_stride >= 0, FC_EINVAL, "%s: null indices", who);
+  return snapkv_select_impl(who, keys, keys, nullptr, nullptr, queries, lse, num_q_heads, window, kernel_size, causal_window,
+                            scale, out_scale, k, n_kept, indices, index_stride, nsplit, workspace, workspace_bytes, stream);
+}
+
+extern "C" int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                                    const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
+                                    int32_t window, int32_t kernel_size, int32_t causal_window, float scale,
+                                    float out_scale, int32_t k, int32_t nsplit, void* workspace, int64_t workspace_bytes,
+                                    void* stream) {
+  const char* who = "fc_snapkv_press_into";
+  int rc;
+  for (const fc_kv_view* v : {keys, values, out_k, out_v})
+    if ((rc = fc_check_view(v, who))) return rc;
+  for (const fc_kv_view* v : {values, out_k, out_v})
+    FC_REQUIRE(keys->dtype == v->dtype && keys->num_layers == v->num_layers && keys->batch == v->batch &&
+                   keys->num_kv_heads == v->num_kv_heads,
+               FC_EINVAL, "%s: views disagree on dtype/layers/batch/heads", who);
+  FC_REQUIRE(keys->max_seq_len == values->max_seq_len && k <= keys->max_seq_len && k <= out_k->max_seq_len &&
+                 k <= out_v->max_seq_len,
+             FC_EINVAL, "%s: k=%d exceeds a view's max_seq_len", who, k);
+  return snapkv_select_impl(who, keys, values, out_k, out_v, queries, lse, num_q_heads, window, kernel_size, causal_window,
+                            scale, out_scale, k, nullptr, nullptr, k, nsplit, workspace, workspace_bytes, stream);
 }
 
 extern "C" int fc_snapkv_fill_window(float* scores, int32_t score_stride, int32_t num_layers, int32_t batch,

@@ -1,0 +1,244 @@
+// What follows the scoring of a press when the kept rows do not move inside their own column by the workgroup that
+// scored it: selection of every column's kept positions, and the gather of its K and V rows into other tensors.
+//
+// column_select_kernel: one workgroup per column and part.  The column's keys are held in registers (of the longest rows, 72
+// keys per thread of 512, 40 in registers and the rest in LDS), scored on the way in: given scores, per-key sums of the
+// SnapKV sweep still to be pooled, or the norms of the key rows themselves.  It either writes the kept positions (a
+// compaction launch follows) or, with `parts` workgroups per column that all make the same selection, copies its share of
+// the kept rows: a HuggingFace hook has a handful of columns, and eight workgroups that each select are faster than one that
+// selects for a second launch.
+// Bound by latency: a column's selection is about 8 us of short steps (4096 keys; 24 us with the keys in LDS and digits
+// at fixed places), the rows of one layer are then in flight over the whole chip.  288 rows of 30 000 pooled sums: 63 us
+// (147 us with 1024 threads and one workgroup to a compute unit, the terms of the pooling read one by one).
+#include "fc_norm.h"
+#include "fc_rows.h"
+#include "fc_select.h"
+#include "fc_tail.h"
+
+// Pooling: 64-key groups a wavefront stages at a time, and its floats for them (a kernel of at most 63 reaches 62 keys past
+// the groups).  The longest rows stage fewer, so that with their keys in LDS two workgroups fit a compute unit's 160 KB.
+#define CS_GROUPS(KPT) ((KPT) > 16 ? 4 : (KPT) < 8 ? (KPT) : 8)
+#define CS_STAGE(KPT) (CS_GROUPS(KPT) * 64 + 64)
+
+template <int SRC, int DTYPE, int THREADS, int KPT>
+__global__ __launch_bounds__(THREADS, KPT > 16 ? 4 : 1) void column_select_kernel(KvView kv, KvView vv, KvView dk, KvView dv, ColumnSelect a) {
+  constexpr int EB = DTYPE == FC_F32 ? 4 : 2;
+  constexpr int LPR = FC_HEAD_DIM * EB / 16, RPP = THREADS / LPR;
+  extern __shared__ __align__(16) int cs_lds[];   // [part_rows] kept positions, the keys that registers do not hold, then what SRC stages
+  __shared__ TkSharedRegs<THREADS> sh;
+  unsigned* rest = reinterpret_cast<unsigned*>(cs_lds + a.part_rows);
+  const int tid = threadIdx.x;
+  const int parts = a.parts > 0 ? a.parts : 1;
+  const int h = (int)blockIdx.x / parts, part = (int)blockIdx.x - h * parts;
+  const int b = blockIdx.y, l = blockIdx.z;
+  const int S = fc_seq_len(kv, b);
+  int kk = a.n_kept ? a.n_kept[b] : a.k;
+  kk = min(min(kk, S), a.index_stride);
+  if (kk <= 0) return;
+  const long long row = ((long long)l * kv.batch + b) * kv.num_kv_heads + h;
+  const int tail = min(a.window, S);
+  const int n = S - tail, want = kk - tail;
+  const int per = a.parts > 0 ? (kk + parts - 1) / parts : 0;
+  const int p0 = part * per, p1 = min(kk, p0 + per);
+  int* idx_row = a.indices + row * a.index_stride;
+  auto emit = [&](int pos, int i) {
+    if (a.parts == 0) idx_row[pos] = i;
+    else if (pos >= p0 && pos < p1) cs_lds[pos - p0] = i;
+  };
+  if (n <= 0) {              // every position is a window position: the first kept-count of them
+    for (int i = tid; i < kk; i += THREADS) emit(i, i);
+  } else if (want < 0) {     // not a selection that keeps the window; the host does not ask for it
+    return;
+  } else if (want >= n) {    // everything (want == n) stays
+    for (int i = tid; i < kk; i += THREADS) emit(i, i);
+  } else if (want == 0) {    // the window alone
+    for (int i = tid; i < tail; i += THREADS) emit(i, n + i);
+  } else {
+    const float* in = a.in + row * a.stride;
+    if constexpr (SRC == CS_NORMS) {
+      // the arithmetic of knorm_kernel, four rows per lane in flight
+      float* sc = reinterpret_cast<float*>(cs_lds + a.part_rows + TK_LDS_KEYS(THREADS, KPT));
+      const int sub = tid % LPR, rg = tid / LPR;
+      const char* kbase = kv.base + ((long long)l * kv.stride_layer + (long long)h * kv.stride_head) * EB + sub * 16;
+      for (int r0 = 0; r0 < n; r0 += RPP * 4) {
+        uint4 x[4];
+        unsigned live = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          long long off = fc_token_offset(kv, b, min(r0 + u * RPP + rg, n - 1));
+          live |= off >= 0 ? (1u << u) : 0u;
+          off = off < 0 ? 0 : off;
+          x[u] = *reinterpret_cast<const uint4*>(kbase + off * EB);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          float part_sum = fc_group_sum<16>(row_sumsq_part<DTYPE>(x[u]));
+          if (LPR == 32) part_sum += __shfl_xor(part_sum, 16, 64);
+          const int r = r0 + u * RPP + rg;
+          if (r < n && sub == 0) sc[r] = (live >> u) & 1u ? -sqrtf(part_sum) : -INFINITY;
+        }
+      }
+      __syncthreads();
+      tk_select_row_regs<THREADS, KPT>(sh, rest, [&](int i) { return tk_key(sc[i]); }, n, want, emit);
+    } else if constexpr (SRC == CS_SUMS) {
+      // Zero-padded moving average of the per-key sums, each key's terms in ascending order like the pooling kernel's.
+      // A wavefront stages its own segment, CS_GROUPS keys a lane and the neighbours at both ends at a time, in LDS of its own
+      // (terms read from memory one by one made the launch above 40 us longer).
+      const TkSegment<THREADS> sg(n);
+      const int hw = a.ksz >> 1, lane = tid & 63;
+      float* st = reinterpret_cast<float*>(rest + TK_LDS_KEYS(THREADS, KPT)) + (tid >> 6) * CS_STAGE(KPT);
+      TkKeys<THREADS, KPT> key(rest);
+      constexpr int G = CS_GROUPS(KPT);
+      float v[G + 1];                       // what the wavefront stages next, on its way while the keys before it are pooled
+      auto fetch = [&](int e0) {
+#pragma unroll
+        for (int g = 0; g <= G; ++g) v[g] = in[min(max(sg.beg + (e0 + g) * 64 - hw + lane, 0), n - 1)];
+      };
+      fetch(0);
+#pragma unroll
+      for (int e0 = 0; e0 < KPT; e0 += G) {
+#pragma unroll
+        for (int g = 0; g <= G; ++g) {
+          const int x = sg.beg + (e0 + g) * 64 - hw + lane;
+          st[g * 64 + lane] = x >= 0 && x < n ? v[g] : 0.f;
+        }
+        if (e0 + G < KPT) fetch(e0 + G);
+        tk_wave_sync();
+        float s[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) s[g] = 0.f;
+        for (int j = 0; j < a.ksz; ++j) {
+#pragma unroll
+          for (int g = 0; g < G; ++g) s[g] += st[g * 64 + lane + j];
+        }
+        tk_wave_sync();
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const int e = e0 + g;
+          key.set(e, e < sg.live && sg.pos(e) < sg.end ? tk_key(s[g] * a.out_mul) : 0u);
+        }
+        if constexpr (KPT > G) __builtin_amdgcn_sched_barrier(0);
+      }
+      tk_select_loaded<THREADS, KPT>(sh, sg, key, want, emit);
+    } else {
+      tk_select_row_regs<THREADS, KPT>(sh, rest, [&](int i) { return tk_key(in[i]); }, n, want, emit);
+    }
+    for (int i = tid; i < tail; i += THREADS) emit(want + i, n + i);
+  }
+  if (a.parts == 0) return;
+  __syncthreads();
+  // this workgroup's rows of both planes: source and destination are different tensors, any order will do
+  const int sub = tid % LPR, rg = tid / LPR;
+  const long long kcol = ((long long)l * kv.stride_layer + (long long)h * kv.stride_head) * EB + sub * 16;
+  const long long vcol = ((long long)l * vv.stride_layer + (long long)h * vv.stride_head) * EB + sub * 16;
+  const long long dkcol = ((long long)l * dk.stride_layer + (long long)h * dk.stride_head) * EB + sub * 16;
+  const long long dvcol = ((long long)l * dv.stride_layer + (long long)h * dv.stride_head) * EB + sub * 16;
+  constexpr int U = 4;
+  for (int j0 = p0; j0 < p1; j0 += RPP * U) {
+    cp_u32x4 kb[U], vb[U];
+    unsigned kok = 0, vok = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {      // every lane always loads; rows past the end re-read the last one
+      const int s = cs_lds[min(j0 + u * RPP + rg, p1 - 1) - p0];
+      const long long ko = fc_token_offset(kv, b, s), vo = fc_token_offset(vv, b, s);
+      kok |= ko >= 0 ? (1u << u) : 0u;
+      vok |= vo >= 0 ? (1u << u) : 0u;
+      kb[u] = *reinterpret_cast<const cp_u32x4*>(kv.base + kcol + max(ko, 0ll) * EB);
+      vb[u] = *reinterpret_cast<const cp_u32x4*>(vv.base + vcol + max(vo, 0ll) * EB);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = j0 + u * RPP + rg;
+      if (j >= p1) continue;
+      const long long ko = fc_token_offset(dk, b, j), vo = fc_token_offset(dv, b, j);
+      if (ko >= 0 && ((kok >> u) & 1u)) *reinterpret_cast<cp_u32x4*>(dk.base + dkcol + ko * EB) = kb[u];
+      if (vo >= 0 && ((vok >> u) & 1u)) *reinterpret_cast<cp_u32x4*>(dv.base + dvcol + vo * EB) = vb[u];
+    }
+  }
+}
+
+int fc_column_select(const char* who, int src, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                     const fc_kv_view* out_v, ColumnSelect a, hipStream_t st) {
+  const int n = keys->max_seq_len;
+  FC_REQUIRE(n <= CS_MAX_KEYS, FC_EUNSUPPORTED, "%s: %d keys in a column (at most %d)", who, n, CS_MAX_KEYS);
+  const int parts = a.parts > 0 ? a.parts : 1;
+  a.part_rows = a.parts > 0 ? (a.index_stride + parts - 1) / parts : 0;
+  const KvView kv = fc_make_view(keys), vv = fc_make_view(values);
+  const KvView dk = fc_make_view(out_k ? out_k : keys), dv = fc_make_view(out_v ? out_v : values);
+  FC_REQUIRE((long long)keys->num_kv_heads * parts <= 0x7fffffffLL, FC_EUNSUPPORTED, "%s: grid too large", who);
+  dim3 grid(keys->num_kv_heads * parts, keys->batch, keys->num_layers);
+  FC_REQUIRE(src != CS_SUMS || (a.ksz >= 1 && a.ksz <= 63), FC_EINVAL, "%s: kernel_size %d", who, a.ksz);
+#define CS_LAUNCH(SRC, DT, TH, KPT)                                                                               \
+  do {                                                                                                            \
+    const size_t lds = 4 * ((size_t)a.part_rows + TK_LDS_KEYS(TH, KPT) +                                          \
+                            (SRC == CS_NORMS ? n : SRC == CS_SUMS ? TH / 64 * CS_STAGE(KPT) : 0));                \
+    FC_REQUIRE(lds <= 120 * 1024, FC_EUNSUPPORTED, "%s: %zu bytes of LDS per workgroup", who, lds);                \
+    FC_ALLOW_LDS((column_select_kernel<SRC, DT, TH, KPT>), 120 * 1024);                                            \
+    hipLaunchKernelGGL((column_select_kernel<SRC, DT, TH, KPT>), grid, dim3(TH), lds, st, kv, vv, dk, dv, a);       \
+  } while (0)
+  // 1024 threads for the long rows, where lanes shorten the chain; 256 for short ones, where fewer wavefronts meet at the
+  // barriers; the longest rows with 512 again, two workgroups to a compute unit (288 rows are then one round, not two)
+#define CS_SIZE(SRC, DT)                               \
+  if (n <= 512) CS_LAUNCH(SRC, DT, 256, 2);            \
+  else if (n <= 4096) CS_LAUNCH(SRC, DT, 512, 8);      \
+  else if (n <= 16384) CS_LAUNCH(SRC, DT, 1024, 16);   \
+  else CS_LAUNCH(SRC, DT, 512, 72)
+#define CS_SIZE_SHORT(SRC, DT)                         \
+  if (n <= 512) CS_LAUNCH(SRC, DT, 256, 2);            \
+  else CS_LAUNCH(SRC, DT, 512, 8)
+#define CS_DTYPE(SRC)                                                                                 \
+  if (keys->dtype == FC_F32) { CS_SIZE(SRC, FC_F32); }                                                \
+  else { CS_SIZE(SRC, FC_F16); }          /* rows of two-byte elements are moved, not computed with */
+  if (src == CS_SCORES) {
+    CS_DTYPE(CS_SCORES);
+  } else if (src == CS_SUMS) {
+    CS_SIZE(CS_SUMS, FC_F16);             // SnapKV scores fp16 / bf16 caches only
+  } else if (keys->dtype == FC_F32) {
+    CS_SIZE_SHORT(CS_NORMS, FC_F32);
+  } else if (keys->dtype == FC_BF16) {
+    CS_SIZE_SHORT(CS_NORMS, FC_BF16);
+  } else {
+    CS_SIZE_SHORT(CS_NORMS, FC_F16);
+  }
+#undef CS_DTYPE
+#undef CS_SIZE_SHORT
+#undef CS_SIZE
+#undef CS_LAUNCH
+  FC_CHECK_LAUNCH(who);
+  return FC_OK;
+}
+
+static int cs_check(const char* who, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                    const fc_kv_view* out_v, int k) {
+  int rc;
+  for (const fc_kv_view* v : {keys, values, out_k, out_v})
+    if ((rc = fc_check_view(v, who))) return rc;
+  for (const fc_kv_view* v : {values, out_k, out_v})
+    FC_REQUIRE(keys->dtype == v->dtype && keys->num_layers == v->num_layers && keys->batch == v->batch &&
+                   keys->num_kv_heads == v->num_kv_heads,
+               FC_EINVAL, "%s: views disagree on dtype/layers/batch/heads", who);
+  FC_REQUIRE(keys->max_seq_len == values->max_seq_len, FC_EINVAL, "%s: key and value views disagree on length", who);
+  FC_REQUIRE(k >= 0 && k <= keys->max_seq_len && k <= out_k->max_seq_len && k <= out_v->max_seq_len, FC_EINVAL,
+             "%s: k=%d exceeds a view's max_seq_len", who, k);
+  return FC_OK;
+}
+
+extern "C" int fc_knorm_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                                   const fc_kv_view* out_v, int32_t k, float* scores, int32_t score_stride, void* stream) {
+  const char* who = "fc_knorm_press_into";
+  int rc = cs_check(who, keys, values, out_k, out_v, k);
+  if (rc) return rc;
+  if (k == 0 || keys->max_seq_len == 0) return FC_OK;
+  ColumnSelect a{};
+  a.k = a.index_stride = k;
+  a.parts = fc_gather_parts(keys, k);
+  if (!scores) {   // the workgroups that gather a column score it as well
+    FC_REQUIRE(keys->max_seq_len <= CS_NORMS_MAX, FC_EUNSUPPORTED, "%s: columns of more than %d keys need a score buffer", who,
+               CS_NORMS_MAX);
+    return fc_column_select(who, CS_NORMS, keys, values, out_k, out_v, a, (hipStream_t)stream);
+  }
+  if ((rc = fc_knorm_score(keys, scores, score_stride, stream))) return rc;
+  a.in = scores;
+  a.stride = score_stride;
+  return fc_column_select(who, CS_SCORES, keys, values, out_k, out_v, a, (hipStream_t)stream);
+}

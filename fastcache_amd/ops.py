@@ -249,6 +249,45 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     return scores, idx
 
 
+def snapkv_select_splits(keys: FcKvView, num_q_heads: int, window: int) -> int:
+    """Key ranges per column for :func:`snapkv_select` (the rule and its measurements stand at
+    ``fc_snapkv_select_splits``)."""
+    return int(fn("fc_snapkv_select_splits")(C.byref(keys), num_q_heads, window))
+
+
+def snapkv_select(keys: FcKvView, queries: torch.Tensor, window: int, kernel_size: int, k: int,
+                  causal_window: bool = True, reduction: str = "mean", scale: Optional[float] = None,
+                  lse: Optional[torch.Tensor] = None, n_kept: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The indices ``snapkv_score`` + ``topk_select`` give for counts above the window, without a score tensor:
+    int32 ``[L, B, Hkv, k]`` (entries past a row's count ``n_kept[b]`` are left as they are)."""
+    queries = queries.contiguous()
+    _lib.require_gpu(queries, "queries")
+    L, B, Hq, W, D = queries.shape
+    H, S, dev = keys.num_kv_heads, keys.max_seq_len, queries.device
+    if (L, B) != (keys.num_layers, keys.batch) or W != window or D != keys.head_dim:
+        raise FastcacheError(f"queries {tuple(queries.shape)} do not match the key view "
+                             f"(L={keys.num_layers}, B={keys.batch}, W={window}, D={keys.head_dim})")
+    if _lib.dtype_code(queries.dtype) != keys.dtype:
+        raise FastcacheError("queries and keys must share a dtype")
+    if reduction not in ("mean", "sum"):
+        raise ValueError("reduction must be 'mean' or 'sum'")
+    if lse is not None:
+        _lib.require_gpu(lse, "lse")
+        if lse.dtype != torch.float32 or tuple(lse.shape) != (L, B, Hq, W):
+            raise FastcacheError(f"lse must be fp32 [L={L}, B={B}, Hq={Hq}, W={W}], got {lse.dtype} {tuple(lse.shape)}")
+        lse = lse.contiguous()
+    n_kept = _i32(n_kept, "n_kept", dev)
+    nsplit = snapkv_select_splits(keys, Hq, W)
+    nbytes = int(fn("fc_snapkv_select_workspace_bytes")(L, B, Hq, H, W, S, nsplit))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    idx = torch.empty((L, B, H, k), dtype=torch.int32, device=dev)
+    check(fn("fc_snapkv_select")(C.byref(keys), queries.data_ptr(), ptr(lse), Hq, window, kernel_size, int(causal_window),
+                                 1.0 / math.sqrt(D) if scale is None else scale,
+                                 1.0 / (W * (Hq // H)) if reduction == "mean" else 1.0, k, ptr(n_kept), idx.data_ptr(), k,
+                                 nsplit, ws.data_ptr(), nbytes, current_stream()), "fc_snapkv_select")
+    return idx
+
+
 # ---------------------------------------------------------------------------------------------
 # selection and compaction
 # ---------------------------------------------------------------------------------------------

@@ -36,19 +36,12 @@ def _views(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.T
             _lib.paged_view(kv_cache[1], block_tables, seq_lens, max_seq_len))
 
 
-def _select_and_compact(kview, vview, scores, seq_lens, kept: List[int], compact: bool, heads: int,
-                        rows_only: bool = False) -> PressResult:
+def _select_and_compact(kview, vview, scores, seq_lens, kept: List[int], compact: bool, heads: int) -> PressResult:
     """Top-k per (layer, sequence, head) row and in-place compaction; one launch each whether or not the
-    sequences keep the same number of tokens.  ``rows_only``: the caller drops the result."""
+    sequences keep the same number of tokens.  (Both in one launch, ``ops.select_compact``, has half the workgroups for
+    the compaction: 288 columns of 12000 keys 294 us against 237, 576 of 16384 1228 against 1181, 2304 of 4096 536 against
+    525.)"""
     width = max(kept)
-    one_launch = (compact and width > 0 and ops.press_column_fits(kview.max_seq_len, width) and scores.dim() == 4 and
-                  scores.shape[2] == kview.num_kv_heads and scores.is_contiguous())
-    if one_launch:       # selection and compaction of a column by one workgroup
-        if len(set(kept)) == 1:
-            return PressResult(ops.select_compact(kview, vview, scores, width), width, scores)
-        n_kept = _lib.upload_ints(kept, scores)
-        return PressResult(ops.select_compact(kview, vview, scores, width, n_kept=n_kept, rows_only=rows_only), width,
-                           scores, list(kept))
     if len(set(kept)) == 1:
         idx = ops.topk_select(scores, width)
         if compact and width > 0:
@@ -72,8 +65,14 @@ def knorm_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq
     lens = list(host_lens) if host_lens is not None else [seq_len] * block_tables.shape[0]
     kept = [n_kept_for(n, compression_ratio) for n in lens]
     width = max(kept)
-    if compact and 0 < width and ops.press_column_fits(seq_len, width):
-        # one launch: every (layer, sequence, head) column is scored, selected and compacted by one workgroup
+    # One launch (every (layer, sequence, head) column is scored, selected and compacted by one workgroup) or norms,
+    # selection and compaction each over the whole chip: below about one and a half columns per compute unit the single
+    # workgroups leave it half idle (us per pass, half kept: 112 columns of 1000 bf16 keys 46 -> 31, of 12000 309 -> 251, 288 of
+    # 2000 106 -> 96, of 18000 1073 -> 935; from there on one launch wins: 576 of 2000 fp32 379 against 412, 1152 of 2000
+    # 354 against 406).
+    columns = kview.num_layers * kview.batch * kview.num_kv_heads
+    if (compact and 0 < width and ops.press_column_fits(seq_len, width) and
+            2 * columns > 3 * _lib.compute_units(kv_cache.device)):
         if len(set(kept)) == 1:
             scores, idx = ops.knorm_press(kview, vview, width, kv_cache.device)
             return PressResult(idx, width, scores)
@@ -81,7 +80,7 @@ def knorm_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq
         scores, idx = ops.knorm_press(kview, vview, width, kv_cache.device, n_kept=n_kept, rows_only=rows_only)
         return PressResult(idx, width, scores, list(kept))
     scores = ops.knorm_score(kview, kv_cache.device)
-    return _select_and_compact(kview, vview, scores, seq_lens, kept, compact, kv_cache.shape[4], rows_only)
+    return _select_and_compact(kview, vview, scores, seq_lens, kept, compact, kv_cache.shape[4])
 
 
 def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.Tensor,
@@ -99,16 +98,26 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
     if not window_in_budget:
         kept = [min(n, k + window_size) for n, k in zip(lens, kept)]
     width = max(kept)
-    # The workgroup that scored a column also selects and compacts it when every row keeps more than the window
-    # (sequences no longer than the window keep their first positions either way).  In that launch the window positions
-    # rank above every scored key, while after the window fill they TIE with scored keys that equal the layer's largest
-    # score; the two selections differ only when more such keys than a row has places outside the window tie exactly,
-    # which needs equal scores at the very top: rows with fewer scored keys than the pooling kernel is wide (every pooled
-    # score the same) take the separate launches.
-    if (compact and all(k > window_size or n <= window_size for n, k in zip(lens, kept)) and width > window_size and
-            all(n <= window_size or n - window_size > kernel_size for n in lens) and
-            ops.snapkv_press_fits(kview, queries.shape[-3], window_size, width) and
-            ops.snapkv_press_preferred(kview, queries.shape[-3], window_size, _lib.compute_units(kv_cache.device))):
+    # Without the filled scores: every row keeps more than the window (sequences no longer than the window keep their
+    # first positions either way), the window positions rank above every scored key and only the others are ranked.
+    # After the window fill they TIE with scored keys that equal the layer's largest score; the two selections differ
+    # only when more such keys than a row has places outside the window tie exactly, which needs equal scores at the
+    # very top: rows with fewer scored keys than the pooling kernel is wide (every pooled score the same) take the
+    # filled scores.
+    window_apart = (compact and all(k > window_size or n <= window_size for n, k in zip(lens, kept)) and
+                    width > window_size and all(n <= window_size or n - window_size > kernel_size for n in lens))
+    # One launch (the workgroup that scored a column also selects and compacts it) or key ranges: with the scores wanted
+    # by the rule of snapkv_press_preferred; without them the selection needs no pooled scores in memory and the
+    # compaction has a workgroup per plane, and ranges win wherever cutting the columns does (us per pass, a third kept:
+    # 112 columns of 4096 keys 295 -> 193, of 1000 94 -> 73, 320 of 12000 1721 -> 1341, 288 of 8192 623 -> 583; whole columns
+    # 576 of 2000 281 against 306, 896 of 4096 736 against 812).
+    hq = queries.shape[-3]
+    fits = window_apart and ops.snapkv_press_fits(kview, hq, window_size, width)
+    if rows_only:
+        one_launch = fits and ops.snapkv_select_splits(kview, hq, window_size) == 1
+    else:
+        one_launch = fits and ops.snapkv_press_preferred(kview, hq, window_size, _lib.compute_units(kv_cache.device))
+    if one_launch:
         same = len(set(kept)) == 1 and len(set(lens)) == 1
         res = ops.snapkv_press(kview, vview, queries, window_size, kernel_size, width, causal_window, reduction,
                                seq_lens=seq_lens, n_kept=None if same else kept, host_lens=lens, rows_only=rows_only)
@@ -116,6 +125,11 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
             return None
         scores, idx = res
         return PressResult(idx, width, scores, None if same else list(kept))
+    if rows_only and window_apart and kview.max_seq_len <= 36864 and (hq // kview.num_kv_heads) * ((window_size + 31) // 32) <= 16:
+        n_kept = None if len(set(kept)) == 1 and len(set(lens)) == 1 else _lib.upload_ints(kept, kv_cache)
+        idx = ops.snapkv_select(kview, queries, window_size, kernel_size, width, causal_window, reduction, n_kept=n_kept)
+        ops.compact(kview, vview, kview, vview, idx, n_kept=n_kept)
+        return None
     scores = ops.snapkv_score(kview, queries, window_size, kernel_size, causal_window, reduction,
                               seq_lens=seq_lens)
-    return _select_and_compact(kview, vview, scores, seq_lens, kept, compact, kv_cache.shape[4], rows_only)
+    return _select_and_compact(kview, vview, scores, seq_lens, kept, compact, kv_cache.shape[4])

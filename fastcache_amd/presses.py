@@ -74,12 +74,21 @@ class ScorerPress:
         """int32 ``[B, Hkv, n_kept]`` ascending positions of the ``n_kept`` best scores per row."""
         return ops.topk_select(scores.contiguous(), n_kept)
 
+    def _press_into(self, module, hidden_states, keys, values, kwargs, n):
+        """Scores, selection and gather of one layer as one native call, for the presses that have one: ``(k, v)``, or
+        None when the shape does not take it."""
+        return None
+
     def compress(self, module, hidden_states, keys, values, attentions, kwargs):
         if self.compression_ratio == 0:
             return keys, values
-        scores = self.score(module, hidden_states, keys, values, attentions, kwargs)
         q_len = hidden_states.shape[1] if hidden_states is not None else keys.shape[2]
         n = self.n_kept(q_len)
+        out = self._press_into(module, hidden_states, keys, values, kwargs, n)
+        if out is not None:
+            _lib.note_enqueued()
+            return out
+        scores = self.score(module, hidden_states, keys, values, attentions, kwargs)
         B, H, S, D = keys.shape
         idx = self.select(scores, n).view(1, B, H, n)
         out_k = torch.empty((B, H, n, D), dtype=keys.dtype, device=keys.device)
@@ -131,7 +140,7 @@ class ScorerPress:
         kview, vview = paged_press._views(pool, block_tables, seq_lens, seq_len)
         scores = self.paged_scores(kview, vview, lens, seq_lens, layers, seq_ids, pool.device)
         if out is None:
-            paged_press._select_and_compact(kview, vview, scores, seq_lens, kept, True, pool.shape[4], rows_only=True)
+            paged_press._select_and_compact(kview, vview, scores, seq_lens, kept, True, pool.shape[4])
             return
         self._compact_into(kview, vview, scores, seq_lens, kept, pool.shape[4], out, layers)
 
@@ -222,6 +231,11 @@ class KnormPress(ScorerPress):
     def score(self, module, hidden_states, keys, values, attentions, kwargs) -> torch.Tensor:
         return ops.knorm_score(_lib.dense_view(keys), keys.device)[0]
 
+    def _press_into(self, module, hidden_states, keys, values, kwargs, n):
+        if type(self).score is not KnormPress.score or type(self).select is not ScorerPress.select:
+            return None                               # a subclass scores or selects in its own way
+        return _lib.host().knorm_into(keys, values, n)
+
     def paged_scores(self, kview, vview, lens, seq_lens, layers, seq_ids, device) -> torch.Tensor:
         return ops.knorm_score(kview, device)
 
@@ -294,7 +308,7 @@ class SnapKVPress(ScorerPress):
             kview, vview = paged_press._views(pool, block_tables, seq_lens, seq_len)
             scores = ops.snapkv_score(kview, q, self.window_size, self.kernel_size, self.causal_window,
                                       self.reduction, seq_lens=seq_lens, lse=lse)
-            paged_press._select_and_compact(kview, vview, scores, seq_lens, kept, True, pool.shape[4], rows_only=True)
+            paged_press._select_and_compact(kview, vview, scores, seq_lens, kept, True, pool.shape[4])
             return
         paged_press.snapkv_compress_paged(pool, block_tables, seq_lens, seq_len, q, self.compression_ratio,
                                           self.window_size, self.kernel_size, self.causal_window, self.reduction,
@@ -319,6 +333,23 @@ class SnapKVPress(ScorerPress):
         half = q.shape[-1] // 2
         rot = torch.cat((-q[..., half:], q[..., :half]), dim=-1)
         return (q * cos + rot * sin).contiguous()
+
+    def _press_into(self, module, hidden_states, keys, values, kwargs, n):
+        if type(self).score is not SnapKVPress.score or type(self).select is not ScorerPress.select:
+            return None                               # a subclass scores or selects in its own way
+        B, H, S, D = keys.shape
+        assert S > self.window_size, "Query length should be greater than the window size"
+        W, ksz = self.window_size, self.kernel_size
+        # as on the runner hook: the window is always kept and only the other keys are ranked, which is the selection
+        # over the filled scores when more is kept than the window and a row's scores are not all one pooled value
+        if n <= W or S - W <= ksz or self.reduction not in ("mean", "sum"):
+            return None
+        q = self.window_queries(module, hidden_states, kwargs)
+        lse = kwargs.get("lse") if kwargs is not None else None
+        if q.dtype != keys.dtype:
+            q = q.to(keys.dtype)
+        out_scale = 1.0 / (W * (q.shape[1] // H)) if self.reduction == "mean" else 1.0
+        return _lib.host().snapkv_into(keys, values, q, lse, n, W, ksz, self.causal_window, 1.0 / math.sqrt(D), out_scale)
 
     def score(self, module, hidden_states, keys, values, attentions, kwargs) -> torch.Tensor:
         S = keys.shape[2]

@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from fastcache_amd import _lib, ops, paged_press, synth
-from fastcache_amd.presses import SimLayerKVPress, ThinKPress
+from fastcache_amd.presses import KnormPress, SimLayerKVPress, SnapKVPress, ThinKPress
 from oracle import paged as opaged
 from oracle import presses as opress
 
@@ -779,3 +779,63 @@ def test_paged_press_ragged_batch_in_one_launch_set(dev, press):
                 assert torch.equal(rows[:, :, :k_keep], opress.gather_tokens(dense, idx))
                 old = torch.cat([case.kv_cache[p, l, blk] for blk in blocks])[:n].permute(1, 0, 2).unsqueeze(0)
                 assert torch.equal(rows[:, :, k_keep:], old[:, :, k_keep:])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,S", [(1, 3, 96), (2, 2, 512), (1, 2, 513), (1, 2, 1024), (1, 9, 1025), (1, 2, 4097), (1, 1, 16385),
+                                   (1, 1, 36864), (1, 1, 36865)])
+def test_layer_hooks_in_one_call(dev, dtype, B, H, S):
+    """KnormPress and SnapKVPress on one layer's K and V (score, selection and gather as one native call) on both sides of
+    every change of launch shape: the kept rows are those of the stable selection over the scores, in ascending order,
+    and every byte is the source row's.  V rows carry their position, which gives the selection back."""
+    g = torch.Generator().manual_seed(S)
+    W, ksz = 32, 7
+    k = torch.randn(B, H, S, 128, generator=g).to(dtype)
+    v = torch.randn(B, H, S, 128, generator=g).to(dtype)
+    pos = torch.arange(S)
+    v[..., 0], v[..., 1] = (pos % 256).to(dtype), (pos // 256).to(dtype)
+    q = torch.randn(B, 2 * H, W, 128, generator=g).to(dtype)
+    kd, vd, qd = k.to(dev), v.to(dev), q.to(dev)
+    hidden = torch.zeros(B, S, 1)
+    for keep in sorted({W + 1, S // 2, S - 1}):
+        ratio = 1.0 - (keep + 0.5) / S
+        for press in [KnormPress(ratio)] + ([] if dtype == torch.float32 else [SnapKVPress(ratio, window_size=W, kernel_size=ksz)]):
+            ok, ov = (t.cpu() for t in press.compress(None, hidden, kd, vd, None, {"queries": qd}))
+            assert ok.shape == ov.shape == (B, H, keep, 128)
+            idx = ov[..., 0].long() + 256 * ov[..., 1].long()
+            assert torch.equal(ok, opress.gather_tokens(k, idx)) and torch.equal(ov, opress.gather_tokens(v, idx))
+            assert bool((idx[..., 1:] > idx[..., :-1]).all())
+            scores = press.score(None, hidden, kd, vd, None, {"queries": qd}).cpu()
+            want = opress.topk_lowest_index(scores, keep)
+            if isinstance(press, KnormPress):
+                assert torch.equal(idx, want)
+            else:                       # other partial sums than the score tensor's: only near-threshold keys may differ
+                assert bool((idx[..., -W:] == pos[-W:]).all())
+                kth = scores.gather(-1, want).min(-1, keepdim=True).values
+                got = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, idx, True)
+                ref = torch.zeros_like(got).scatter_(-1, want, True)
+                assert not bool(((got ^ ref) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+
+
+@pytest.mark.parametrize("S", [600, 5000, 17000])
+def test_snapkv_select_ragged(dev, S):
+    """Selection straight from the sweeps' sums for sequences of different lengths, one of them no longer than the
+    window, one just above it: the positions the score tensor's selection keeps, up to keys at the threshold."""
+    L, Hq, H, W, ksz = 2, 4, 2, 32, 5
+    lens, keep = [S, S // 2 + 3, 20, W + ksz + 1], [S // 4, S // 5, 20, W + 2]
+    case = synth.make_paged_case(seed=S, num_layers=L, batch=4, num_kv_heads=H, seq_lens=lens, dtype=torch.bfloat16,
+                                 num_q_heads=Hq, window=W)
+    pool, tab, lens_d, q = case.kv_cache.to(dev), case.table_tensor(dev), case.lens_tensor(dev), case.queries.to(dev)
+    kview = _lib.paged_view(pool[0], tab, lens_d, S)
+    n_kept = torch.tensor(keep, dtype=torch.int32, device=dev)
+    idx = ops.snapkv_select(kview, q, W, ksz, max(keep), True, "sum", n_kept=n_kept).cpu().long()
+    scores = ops.snapkv_score(kview, q, W, ksz, True, "sum", seq_lens=lens_d).cpu()
+    for b, (n, kk) in enumerate(zip(lens, keep)):
+        sc, got = scores[:, b, :, :n], idx[:, b, :, :kk]
+        assert bool((got[..., 1:] > got[..., :-1]).all())
+        tail = min(W, n)
+        assert bool((got[..., -tail:] == torch.arange(n - tail, n)).all())
+        want = opress.topk_lowest_index(sc, kk)
+        kth = sc.gather(-1, want).min(-1, keepdim=True).values
+        diff = torch.zeros_like(sc, dtype=torch.bool).scatter_(-1, got, True) ^ torch.zeros_like(sc, dtype=torch.bool).scatter_(-1, want, True)
+        assert not bool((diff & ((sc - kth).abs() > 2e-4 * kth.abs())).any())
