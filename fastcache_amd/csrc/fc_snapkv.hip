@@ -64,6 +64,7 @@ struct SkPress {
   const int* n_kept;    // [batch] in device memory, or null
   int* indices;         // [layers][batch][kv heads][index_stride]
   int index_stride;
+  const int* order;     // [batch] sequences in the order their columns are to start, or null (as they come)
 };
 
 // LDS the press tail carves out of the key tiles and the per-key sum area behind them: the score row, the kept
@@ -93,8 +94,20 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
   int* tbl = reinterpret_cast<int*>(smem + ST * SK_TILEB + (4 * NW + 4) * SK_KT * 4);
 
   const int Hkv = kv.num_kv_heads;
-  const int b = blockIdx.y, l = blockIdx.z;
-  const int h = MODE == 0 ? (int)blockIdx.x : (int)blockIdx.x % Hkv;
+  int b = blockIdx.y, l = blockIdx.z;
+  int h = MODE == 0 ? (int)blockIdx.x : (int)blockIdx.x % Hkv;
+  if constexpr (PRESS) {
+    // Sequences of different lengths: all columns of the longest start first and those of the shortest last, so that the
+    // last workgroups to start are the ones that end soonest (28 layers x 4 heads of 13 sequences of 200 to 2300 tokens:
+    // 494 us, 534 us with the columns as they came).
+    if (press.order) {
+      const unsigned id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), cols = gridDim.x * gridDim.z;
+      const unsigned r = id / cols, c = id - r * cols;
+      b = min(max(__builtin_amdgcn_readfirstlane(press.order[r]), 0), kv.batch - 1);
+      l = (int)(c / gridDim.x);
+      h = (int)(c - (unsigned)l * gridDim.x);
+    }
+  }
   const int split = MODE == 0 ? 0 : (int)blockIdx.x / Hkv;
   const int G = Hq / Hkv;
   const int WB = (W + 31) / 32;        // 32-row blocks per query head
@@ -665,7 +678,7 @@ static int snapkv_score_impl(const char* who, const fc_kv_view* keys, const void
                              float* scores, int32_t score_stride, float* row_max, const float* lse, void* stream,
                              const fc_kv_view* press_values = nullptr, int32_t press_k = 0,
                              const int32_t* press_n_kept = nullptr, int32_t* press_indices = nullptr,
-                             int32_t press_index_stride = 0) {
+                             int32_t press_index_stride = 0, const int32_t* press_order = nullptr) {
   int rc = fc_check_view(keys, who);
   if (rc) return rc;
   FC_REQUIRE(queries && scores, FC_EINVAL, "%s: null pointer", who);
@@ -720,6 +733,7 @@ static int snapkv_score_impl(const char* who, const fc_kv_view* keys, const void
     press.n_kept = press_n_kept;
     press.indices = press_indices;
     press.index_stride = press_index_stride;
+    press.order = press_order;
 #define SK_PRESS(DT, NWV)                                                                                        \
   do {                                                                                                         \
     FC_ALLOW_LDS((snapkv_kernel<DT, NWV, true, 0, true>), SkCfg<NWV>::LDS);                                     \
@@ -789,6 +803,17 @@ extern "C" int fc_snapkv_press(const fc_kv_view* keys, const fc_kv_view* values,
   FC_REQUIRE(values && row_max, FC_EINVAL, "%s: null value view or row_max", who);
   return snapkv_score_impl(who, keys, queries, num_q_heads, window, kernel_size, causal_window, scale, out_scale,
                            scores, score_stride, row_max, lse, stream, values, k, n_kept, indices, index_stride);
+}
+
+extern "C" int fc_snapkv_press_ordered(const fc_kv_view* keys, const fc_kv_view* values, const void* queries,
+                                       const float* lse, int32_t num_q_heads, int32_t window, int32_t kernel_size,
+                                       int32_t causal_window, float scale, float out_scale, float* scores,
+                                       int32_t score_stride, float* row_max, int32_t k, const int32_t* n_kept,
+                                       int32_t* indices, int32_t index_stride, const int32_t* order, void* stream) {
+  const char* who = "fc_snapkv_press_ordered";
+  FC_REQUIRE(values && row_max && order, FC_EINVAL, "%s: null value view, row_max or order", who);
+  return snapkv_score_impl(who, keys, queries, num_q_heads, window, kernel_size, causal_window, scale, out_scale,
+                           scores, score_stride, row_max, lse, stream, values, k, n_kept, indices, index_stride, order);
 }
 
 // ---- split columns ------------------------------------------------------------------------------------

@@ -200,6 +200,7 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
 
     ``rows_only``: for callers that want the moved rows alone; scores and indices stay scratch (no window fill, no
     padding of the index rows) and None is returned."""
+    order = None
     if n_kept is not None and not isinstance(n_kept, torch.Tensor):
         counts = [int(c) for c in n_kept]
         lens_h = list(host_lens) if host_lens is not None else [keys.max_seq_len] * len(counts)
@@ -207,7 +208,11 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
         if len(counts) != keys.batch or bad:
             raise FastcacheError(f"snapkv_press: kept counts must exceed the window ({window}) and fit the index row "
                                  f"({k}) for every sequence longer than the window; offending sequences: {bad}")
-        n_kept = _lib.upload_ints(counts, queries)
+        if len(set(lens_h)) > 1:            # the longest sequences' columns start first
+            n_kept, order = _lib.host().upload_tables(
+                [], (counts, sorted(range(len(lens_h)), key=lambda b: -lens_h[b])), queries)[1:]
+        else:
+            n_kept = _lib.upload_ints(counts, queries)
     if queries.dim() == 4:
         queries = queries.unsqueeze(0)
         if lse is not None and lse.dim() == 3:
@@ -239,9 +244,12 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
             raise FastcacheError(f"lse must be fp32 [L={L}, B={B}, Hq={Hq}, W={W}], got {lse.dtype} {tuple(lse.shape)}")
         lse = lse.contiguous()
     st = current_stream()
-    check(fn("fc_snapkv_press")(C.byref(keys), C.byref(values), queries.data_ptr(), ptr(lse), Hq, window, kernel_size,
-                                int(causal_window), scale, out_scale, scores.data_ptr(), stride, row_max.data_ptr(), k,
-                                ptr(n_kept), idx.data_ptr(), k, st), "fc_snapkv_press")
+    args = (C.byref(keys), C.byref(values), queries.data_ptr(), ptr(lse), Hq, window, kernel_size, int(causal_window),
+            scale, out_scale, scores.data_ptr(), stride, row_max.data_ptr(), k, ptr(n_kept), idx.data_ptr(), k)
+    if order is None:
+        check(fn("fc_snapkv_press")(*args, st), "fc_snapkv_press")
+    else:
+        check(fn("fc_snapkv_press_ordered")(*args, order.data_ptr(), st), "fc_snapkv_press_ordered")
     if rows_only:
         return None
     check(fn("fc_snapkv_fill_window")(scores.data_ptr(), stride, L, B, H, ptr(seq_lens), keys.max_seq_len, window,

@@ -171,6 +171,13 @@ int fc_snapkv_press(const fc_kv_view* keys, const fc_kv_view* values, const void
                     int32_t num_q_heads, int32_t window, int32_t kernel_size, int32_t causal_window, float scale,
                     float out_scale, float* scores, int32_t score_stride, float* row_max, int32_t k,
                     const int32_t* n_kept, int32_t* indices, int32_t index_stride, void* stream);
+/* The same with the sequences' columns started in the order of `order` ([batch], a permutation): longest first keeps the
+ * launch's end short when the lengths differ. */
+int fc_snapkv_press_ordered(const fc_kv_view* keys, const fc_kv_view* values, const void* queries, const float* lse,
+                            int32_t num_q_heads, int32_t window, int32_t kernel_size, int32_t causal_window,
+                            float scale, float out_scale, float* scores, int32_t score_stride, float* row_max,
+                            int32_t k, const int32_t* n_kept, int32_t* indices, int32_t index_stride,
+                            const int32_t* order, void* stream);
 
 /*
  * The same scores with every (layer, sequence, kv head) column cut into `nsplit` key ranges, one workgroup each:

@@ -839,3 +839,20 @@ def test_snapkv_select_ragged(dev, S):
         kth = sc.gather(-1, want).min(-1, keepdim=True).values
         diff = torch.zeros_like(sc, dtype=torch.bool).scatter_(-1, got, True) ^ torch.zeros_like(sc, dtype=torch.bool).scatter_(-1, want, True)
         assert not bool((diff & ((sc - kth).abs() > 2e-4 * kth.abs())).any())
+
+
+@pytest.mark.parametrize("lens", [[300, 1500, 64, 900, 900], [40, 2000]])
+def test_snapkv_press_longest_columns_first(dev, lens):
+    """Sequence lengths known on the host order the launch's columns; the results are those of the launch as it comes."""
+    L, Hq, H, W, ksz, keep = 3, 8, 2, 32, 5, [max(n // 4, 33) for n in lens]
+    case = synth.make_paged_case(seed=4, num_layers=L, batch=len(lens), num_kv_heads=H, seq_lens=lens, dtype=torch.bfloat16,
+                                 num_q_heads=Hq, window=W)
+    tab, lens_d, q = case.table_tensor(dev), case.lens_tensor(dev), case.queries.to(dev)
+    out = []
+    for counts in (keep, torch.tensor(keep, dtype=torch.int32, device=dev)):
+        pool = case.kv_cache.to(dev)
+        kv = [_lib.paged_view(pool[p], tab, lens_d, max(lens)) for p in range(2)]
+        scores, idx = ops.snapkv_press(*kv, q, W, ksz, max(keep), True, "sum", seq_lens=lens_d, n_kept=counts, host_lens=lens)
+        out.append((scores, idx, pool))
+    for a, b in zip(*out):
+        assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
