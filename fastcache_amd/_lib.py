@@ -91,6 +91,8 @@ SIGNATURES = {
     "fc_quantize_fp8": (C.c_int, [_VP, C.c_int64, _I, _I, _VP, _VP, _VP, C.c_int64, _VP]),
     "fc_dequantize_fp8": (C.c_int, [_VP, _VP, C.c_int64, _I, _I, _I, _VP, _VP]),
     "fc_quantize_rows_asym": (C.c_int, [_VP, C.c_int64, _I, _I, _VP, _VP, _VP]),
+    "fc_quantize_pair_workspace_bytes": (C.c_int64, [_I]),
+    "fc_quantize_pair": (C.c_int, [_I, _VP, _VP, C.c_int64, _I, _I, _VP, _VP, _VP, _VP, _VP, C.c_int64, _VP]),
     "fc_quantize_group4": (C.c_int, [_VP, C.c_int64, _I, _I, _I, _VP, _VP, _VP]),
     "fc_dequantize_group4": (C.c_int, [_VP, _VP, C.c_int64, _I, _I, _I, _I, _VP, _VP]),
     "fc_expected_attention_workspace_bytes": (C.c_int64, [_I, _I, _I, _I]),

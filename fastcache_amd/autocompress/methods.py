@@ -20,7 +20,7 @@ from typing import Dict, List, Tuple
 
 import torch
 
-from .. import ops
+from .. import _lib, ops
 from .._lib import FastcacheError
 
 
@@ -36,6 +36,7 @@ class QuantizationMethod:
         self._quant_type = self._parse_quant_type(quant_type)
         self._group_size = group_size
         self._symmetric = symmetric
+        self._native_kind = ("INT8", "INT4", "NF4", "FP8_E4M3", "FP8_E5M2").index(self._quant_type.name)   # FC_QUANT_*
 
     def _parse_quant_type(self, quant_type: str) -> "QuantizationMethod.QuantType":
         mapping = {"int8": self.QuantType.INT8, "int4": self.QuantType.INT4, "fp8": self.QuantType.FP8_E4M3,
@@ -52,6 +53,11 @@ class QuantizationMethod:
 
     def compress(self, keys: torch.Tensor, values: torch.Tensor, **kwargs):
         """``((quantised keys, key scales), (quantised values, value scales))`` (methods.py:604-620)."""
+        if type(self) is QuantizationMethod and self._symmetric:      # both tensors by one native call
+            out = _lib.host().quantize_pair(self._native_kind, keys, values, self._group_size)
+            if out is not None:
+                _lib.note_enqueued()
+                return out
         return self._quantize(keys), self._quantize(values)
 
     def _quantize(self, tensor: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -82,6 +88,10 @@ class QuantizationMethod:
 
     def dequantize(self, quantized: torch.Tensor, scale: torch.Tensor, dtype: torch.dtype = torch.float16) -> torch.Tensor:
         t = self._quant_type
+        out = _lib.host().dequantize(self._native_kind, quantized, scale, dtype, self._group_size)
+        if out is not None:
+            _lib.note_enqueued()
+            return out
         if t == self.QuantType.INT8:
             if quantized.dtype == torch.uint8:
                 raise FastcacheError("asymmetric int8 codes cannot be de-quantised: the reference's expression "

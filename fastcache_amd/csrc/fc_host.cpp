@@ -10,6 +10,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
@@ -332,6 +333,80 @@ PyObject* py_snapkv_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   });
 }
 
+// ---- quantisers ----------------------------------------------------------------------------------------------------------
+at::ScalarType fp8_type(int64_t kind) { return kind == FC_QUANT_E5M2 ? at::kFloat8_e5m2 : at::kFloat8_e4m3fn; }
+
+// quantize_pair(kind, keys, values, group_size) -> ((codes, scale), (codes, scale)) with one launch for both tensors (two for
+// float8), or None (the caller's general path then serves or refuses the arguments)
+PyObject* py_quantize_pair(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    need_args(nargs, 4, "quantize_pair");
+    if (!is_tensor(args[1]) || !is_tensor(args[2])) Py_RETURN_NONE;
+    const int64_t kind = as_int(args[0]), group = as_int(args[3]);
+    at::Tensor x[2] = {THPVariable_Unpack(args[1]), THPVariable_Unpack(args[2])};
+    const at::ScalarType dt = x[0].scalar_type();
+    if (!x[0].is_cuda() || x[1].device() != x[0].device() || x[1].scalar_type() != dt || x[0].sizes() != x[1].sizes() ||
+        x[0].dim() < 1 || x[0].numel() == 0 || (dt != at::kFloat && dt != at::kHalf && dt != at::kBFloat16))
+      Py_RETURN_NONE;
+    const bool fp8 = kind == FC_QUANT_E4M3 || kind == FC_QUANT_E5M2, bits4 = kind == FC_QUANT_INT4 || kind == FC_QUANT_NF4;
+    const int64_t last = x[0].size(-1), d = bits4 ? group : last, n = x[0].numel();
+    if (bits4 && (group < 2 || group % 2 || last % group)) Py_RETURN_NONE;
+    for (at::Tensor& t : x) t = t.contiguous();
+    std::vector<int64_t> shape = x[0].sizes().vec(), lead = shape;
+    if (bits4) shape.back() = last / 2;
+    lead.back() = bits4 ? last / group : 1;
+    at::Tensor codes[2], scale[2];
+    for (int i = 0; i < 2; ++i) {
+      codes[i] = at::empty(shape, x[0].options().dtype(kind == FC_QUANT_INT8 ? at::kChar : fp8 ? fp8_type(kind) : at::kByte));
+      scale[i] = fp8 ? at::empty({}, x[0].options()) : at::empty(lead, x[0].options());
+    }
+    const int64_t bytes = fc_quantize_pair_workspace_bytes((int32_t)kind);
+    at::Tensor ws;
+    if (bytes) ws = at::empty({bytes}, x[0].options().dtype(at::kByte));
+    check(fc_quantize_pair((int32_t)kind, x[0].const_data_ptr(), x[1].const_data_ptr(), n / d, (int32_t)d, dtype_code(dt),
+                           codes[0].data_ptr(), codes[1].data_ptr(), scale[0].data_ptr(), scale[1].data_ptr(),
+                           bytes ? ws.data_ptr() : nullptr, bytes, stream_of(x[0])),
+          "fc_quantize_pair");
+    PyObject* out[2];
+    for (int i = 0; i < 2; ++i) out[i] = pair(std::move(codes[i]), fp8 ? scale[i].expand(lead) : std::move(scale[i]));
+    return Py_BuildValue("(NN)", out[0], out[1]);
+  });
+}
+
+// dequantize(kind, codes, scale, dtype, group_size) -> tensor, or None (likewise)
+PyObject* py_dequantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    need_args(nargs, 5, "dequantize");
+    if (!is_tensor(args[1]) || !is_tensor(args[2]) || !THPDtype_Check(args[3])) Py_RETURN_NONE;
+    const int64_t kind = as_int(args[0]), group = as_int(args[4]);
+    const at::Tensor &q = THPVariable_Unpack(args[1]), &s = THPVariable_Unpack(args[2]);
+    const at::ScalarType dt = reinterpret_cast<THPDtype*>(args[3])->scalar_type;
+    const bool fp8 = kind == FC_QUANT_E4M3 || kind == FC_QUANT_E5M2, bits4 = kind == FC_QUANT_INT4 || kind == FC_QUANT_NF4;
+    if (!q.is_cuda() || s.device() != q.device() || s.scalar_type() != dt || !q.is_contiguous() || q.dim() < 1 || q.numel() == 0 ||
+        s.numel() == 0 || (dt != at::kFloat && dt != at::kHalf && dt != at::kBFloat16))
+      Py_RETURN_NONE;
+    if (q.scalar_type() != (kind == FC_QUANT_INT8 ? at::kChar : bits4 ? at::kByte : fp8_type(kind))) Py_RETURN_NONE;
+    const int64_t n = bits4 ? 2 * q.numel() : q.numel(), d = bits4 ? group : q.size(-1);
+    if (!fp8 && (d < 1 || n % d || s.numel() != n / d || !s.is_contiguous())) Py_RETURN_NONE;
+    std::vector<int64_t> shape = q.sizes().vec();
+    if (bits4) shape.back() *= 2;
+    at::Tensor out = at::empty(shape, q.options().dtype(dt));
+    const int32_t code = dtype_code(dt);
+    void* st = stream_of(q);
+    if (fp8)
+      check(fc_dequantize_fp8((const uint8_t*)q.const_data_ptr(), s.const_data_ptr(), n, kind == FC_QUANT_E5M2, code, code, out.data_ptr(), st),
+            "fc_dequantize_fp8");
+    else if (bits4)
+      check(fc_dequantize_group4((const uint8_t*)q.const_data_ptr(), s.const_data_ptr(), n / d, (int32_t)d, code, code,
+                                 kind == FC_QUANT_NF4, out.data_ptr(), st),
+            "fc_dequantize_group4");
+    else
+      check(fc_dequantize_rows((const int8_t*)q.const_data_ptr(), s.const_data_ptr(), n / d, (int32_t)d, code, code, out.data_ptr(), st),
+            "fc_dequantize_rows");
+    return wrap(std::move(out));
+  });
+}
+
 // ---- one attention layer of a decode step ---------------------------------------------------------------------------------
 // decode_layer(q, k, v, k_cache, v_cache, slot_mapping, context_lens, block_tables, scale, q_heads, kv_heads, head_dim,
 //              workspace or None) -> out [n, q_heads * head_dim], or None when the arguments are not the plain decode
@@ -582,6 +657,10 @@ PyMethodDef kMethods[] = {
      "decode_inputs(ids, lens, tables, block_size, ref) -> five device tensors"},
     {"upload_tables", (PyCFunction)(void (*)(void))py_upload_tables, METH_FASTCALL,
      "upload_tables(tables, (list, ...), ref) -> device tensors"},
+    {"quantize_pair", (PyCFunction)(void (*)(void))py_quantize_pair, METH_FASTCALL,
+     "quantize_pair(kind, keys, values, group_size) -> ((codes, scale), (codes, scale)) or None"},
+    {"dequantize", (PyCFunction)(void (*)(void))py_dequantize, METH_FASTCALL,
+     "dequantize(kind, codes, scale, dtype, group_size) -> tensor or None"},
     {"knorm_into", (PyCFunction)(void (*)(void))py_knorm_into, METH_FASTCALL, "knorm_into(keys, values, n) -> (k, v) or None"},
     {"snapkv_into", (PyCFunction)(void (*)(void))py_snapkv_into, METH_FASTCALL,
      "snapkv_into(keys, values, queries, lse, n, window, kernel_size, causal, scale, out_scale) -> (k, v) or None"},

@@ -74,11 +74,11 @@ __global__ __launch_bounds__(256) void dequantize_rows_kernel(const signed char*
 // MODE 0: integer codes, scale = clamp(max|x| / 7, 1e-8), code = clamp(round(x / scale), -8, 7) + 8.
 // MODE 1: NF4, scale = clamp(max|x|, 1e-8), code = index of the table entry nearest to x / scale
 //         (table rounded to the tensor dtype, differences rounded to it as well, first minimum wins).
-__constant__ float kNf4Table[16] = {-1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.39491748809814453f,
-                                    -0.28444138169288635f, -0.18477343022823334f, -0.09105003625154495f, 0.0f,
-                                    0.07958029955625534f, 0.16093020141124725f, 0.24611230194568634f,
-                                    0.33791524171829224f, 0.44070982933044434f, 0.5626170039176941f,
-                                    0.7229568362236023f, 1.0f};
+#define QZ_NF4_LEVELS                                                                                                  \
+  -1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.39491748809814453f, -0.28444138169288635f, -0.18477343022823334f, \
+      -0.09105003625154495f, 0.0f, 0.07958029955625534f, 0.16093020141124725f, 0.24611230194568634f,                   \
+      0.33791524171829224f, 0.44070982933044434f, 0.5626170039176941f, 0.7229568362236023f, 1.0f
+__constant__ float kNf4Table[16] = {QZ_NF4_LEVELS};
 
 // the NF4 levels rounded to the tensor dtype, once per workgroup (the caller synchronises)
 template <int DTYPE>
@@ -289,6 +289,13 @@ __device__ __forceinline__ unsigned char qz_to_fp8(float f) {
   return (unsigned char)(r | sign);
 }
 
+// four finite values by the conversion instructions, which round the same way
+template <int E5M2>
+__device__ __forceinline__ unsigned qz_to_fp8x4(float a, float b, float c, float d) {
+  if constexpr (E5M2) return (unsigned)__builtin_amdgcn_cvt_pk_bf8_f32(c, d, __builtin_amdgcn_cvt_pk_bf8_f32(a, b, 0, false), true);
+  return (unsigned)__builtin_amdgcn_cvt_pk_fp8_f32(c, d, __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false), true);
+}
+
 template <int E5M2>
 __device__ __forceinline__ float qz_from_fp8(unsigned char c) {
   const unsigned sign = ((unsigned)c & 0x80u) << 24;
@@ -379,6 +386,10 @@ __global__ __launch_bounds__(256) void quantize_rows_asym_kernel(const char* __r
 // A row is covered by LPR = row bytes / 16 lanes with one 16-byte load each and stays in registers between the
 // reduction and the second step; a thread handles QZ_U rows so that several loads are in flight.  The arithmetic is
 // the same, step for step, as in the kernels above, which remain the path for every other row length.
+// Bound by memory since the quotients are products with a reciprocal (qz_quot), the maxima are taken on bit patterns, two
+// elements per instruction, and integers are rounded and packed by additions and byte permutes.  Two bf16 tensors of 33.5M
+// elements (33 us at the rate of a large copy), before -> now: int8 76 -> 32.5 us, 4 bits 70 -> 30, NF4 114 -> 35, float8
+// (which reads its input twice) 89 -> 58; back to bf16: 36 -> 33.5, 34 -> 28.5, 35 -> 31, 44 -> 33.
 // largest grids of the flat passes (their workgroups loop beyond that)
 #ifndef QZ_GRID_CAP
 #define QZ_GRID_CAP 8192
@@ -432,19 +443,120 @@ __device__ __forceinline__ float qz_row_max(float v) {
   return v;
 }
 
+// The quotient v / sc of two values of the storage dtype, as far as its rounding TO that dtype goes: rs = rcp(sc).  A
+// 16-bit quotient's rounding is decided at the midpoints of two neighbouring values, which have one significant bit more
+// than a value has: p + 1 where sc has p, so m * sc = v is impossible for an odd p + 1 bit m, and no quotient is nearer to
+// a midpoint than 2^-(2p + 1) of itself.  bf16 (p = 8): v * rs, off by 2^-22, is near enough.  fp16 (p = 11): one
+// correction step leaves half a last place of fp32, 2^-24 (below the smallest normal number, where midpoints have fewer
+// bits and can be met, the step makes such a quotient exact).  Both for finite sc > 0 and |v| <= the row's largest.
+// The division instruction sequence costs ten operations per element, more than reading and storing it.
+template <int DTYPE>
+__device__ __forceinline__ float qz_quot(float v, float sc, float rs) {
+  if constexpr (DTYPE == FC_F32) return v / sc;
+  const float y = v * rs;
+  if constexpr (DTYPE == FC_BF16) return y;
+  return __builtin_fmaf(__builtin_fmaf(-y, sc, v), rs, y);
+}
+// EPL finite values to the storage dtype and back, two per instruction where the hardware has it
+template <int DTYPE, int N>
+__device__ __forceinline__ void qz_round_finite(float (&v)[N]) {
+  if constexpr (DTYPE == FC_BF16) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int j = 0; j < N; j += 2) {
+      const unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector((f2){v[j], v[j + 1]}, b2));
+      v[j] = __uint_as_float(w << 16);
+      v[j + 1] = __uint_as_float(w & 0xffff0000u);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] = qz_round<DTYPE>(v[j]);
+  }
+}
+// Largest |x| of 16 bytes of 16-bit elements as its bit pattern (above the pattern of infinity: a NaN is among them)
+__device__ __forceinline__ unsigned qz_abs_bits(const uint4& x) {
+  typedef unsigned short u2 __attribute__((ext_vector_type(2)));
+  const auto mag = [](unsigned w) { return __builtin_bit_cast(u2, w & 0x7fff7fffu); };
+  const u2 m = __builtin_elementwise_max(__builtin_elementwise_max(mag(x.x), mag(x.y)), __builtin_elementwise_max(mag(x.z), mag(x.w)));
+  return max((unsigned)m.x, (unsigned)m.y);
+}
+template <int DTYPE>
+__device__ __forceinline__ float qz_from_abs_bits(unsigned b) {
+  constexpr unsigned inf = DTYPE == FC_BF16 ? 0x7f80u : 0x7c00u;
+  if (b > inf) return __builtin_nanf("");
+  return DTYPE == FC_BF16 ? fc_bf16_to_float((unsigned short)b) : fc_half_to_float((unsigned short)b);
+}
+
+// NF4 codes without a search per element.  The code is a step function of the quotient t, with 15 thresholds th[i]: the
+// smallest value of the dtype whose difference to level i + 1, rounded, is the smaller one (qz_code4).  t in [-1, 1] falls
+// into one of 129 buckets of 1/64; no bucket holds more than one threshold (levels are 0.079 apart), so a bucket's entry
+// is the code below its threshold and the threshold.
+struct Nf4Steps { float th[15]; };
+template <int DTYPE>
+constexpr float qz_const_round(float f) {
+  if (DTYPE == FC_F32) return f;
+  if (DTYPE == FC_F16) return (float)(_Float16)f;
+  unsigned u = __builtin_bit_cast(unsigned, f);
+  u += 0x7fffu + ((u >> 16) & 1u);
+  return __builtin_bit_cast(float, u & 0xffff0000u);
+}
+template <int DTYPE>
+constexpr Nf4Steps qz_nf4_steps() {
+  const float levels[16] = {QZ_NF4_LEVELS};
+  Nf4Steps s{};
+  for (int i = 0; i < 15; ++i) {
+    const float lo = qz_const_round<DTYPE>(levels[i]), hi = qz_const_round<DTYPE>(levels[i + 1]);
+    float below = lo, at = hi;   // the code of `below` is i, that of `at` i + 1: halve until they are neighbours
+    while (true) {
+      const float mid = qz_const_round<DTYPE>(below + (at - below) * 0.5f);
+      if (mid <= below || mid >= at) break;
+      const float d_lo = qz_const_round<DTYPE>(mid - lo), d_hi = qz_const_round<DTYPE>(hi - mid);
+      if (d_hi < d_lo) at = mid;
+      else below = mid;
+    }
+    s.th[i] = at;
+  }
+  return s;
+}
+struct Nf4Bucket { float th; float below; };
+#define QZ_BUCKETS 130
+__device__ __forceinline__ int qz_bucket(float t) { return min(max((int)__builtin_fmaf(t, 64.f, 64.f), 0), QZ_BUCKETS - 1); }
+template <int DTYPE>
+__device__ __forceinline__ void qz_fill_buckets(Nf4Bucket* tab) {
+  constexpr Nf4Steps s = qz_nf4_steps<DTYPE>();
+  for (int b = threadIdx.x; b < QZ_BUCKETS; b += 256) {
+    Nf4Bucket e{INFINITY, 0.f};
+#pragma unroll
+    for (int i = 0; i < 15; ++i) {
+      const int at = qz_bucket(s.th[i]);
+      if (at < b) e.below += 1.f;
+      if (at == b) e.th = s.th[i];
+    }
+    tab[b] = e;
+  }
+}
+
+// one or two tensors of one shape in a launch, by blockIdx.y (a cache's keys and values are quantised together)
+struct QzPair {
+  const char* x[2];
+  char* out[2];
+  char* scale[2];
+  char* absmax;      // KIND 2, one tensor
+};
+
 // KIND 0: symmetric codes (int8 store), 1: asymmetric codes + (scale, zero), 2: quantise -> dequantise,
 // 3 / 4: packed 4-bit integer / NF4 codes of a group
 template <int DTYPE, int LPR, int KIND>
-__global__ __launch_bounds__(256) void quant_rows_fast_kernel(const char* __restrict__ x, long long rows, float qmax,
-                                                              char* __restrict__ out, char* __restrict__ scale,
-                                                              char* __restrict__ absmax) {
+__global__ __launch_bounds__(256) void quant_rows_fast_kernel(QzPair io, long long rows, float qmax) {
   constexpr int EPL = QzV<DTYPE>::EPL;
   constexpr int RPB = 256 / LPR;   // rows per block and step
   __shared__ float levels[16];
-  if (KIND == 4) {
-    qz_fill_levels<DTYPE>(levels);
-    __syncthreads();
-  }
+  __shared__ Nf4Bucket buckets[KIND == 4 ? QZ_BUCKETS : 1];
+  const char* __restrict__ x = io.x[blockIdx.y];
+  char* __restrict__ out = io.out[blockIdx.y];
+  char* __restrict__ scale = io.scale[blockIdx.y];
+  char* __restrict__ absmax = io.absmax;
   const int sub = threadIdx.x % LPR, rg = threadIdx.x / LPR;
   uint4 xin[QZ_U];
   long long row[QZ_U];
@@ -454,6 +566,11 @@ __global__ __launch_bounds__(256) void quant_rows_fast_kernel(const char* __rest
     const long long rc = row[u] < rows ? row[u] : rows - 1;
     xin[u] = *reinterpret_cast<const uint4*>(x + (rc * LPR + sub) * 16);
   }
+  if (KIND == 4) {
+    qz_fill_levels<DTYPE>(levels);
+    qz_fill_buckets<DTYPE>(buckets);
+    __syncthreads();
+  }
 #pragma unroll
   for (int u = 0; u < QZ_U; ++u) {
     const bool live = row[u] < rows;
@@ -461,28 +578,52 @@ __global__ __launch_bounds__(256) void quant_rows_fast_kernel(const char* __rest
     float v[EPL];
     qz_unpack<DTYPE>(xin[u], v);
     float mx = KIND == 1 ? -INFINITY : 0.f, mn = INFINITY, nanf = 0.f;
+    if constexpr (DTYPE != FC_F32 && KIND != 1) {
+      mx = qz_from_abs_bits<DTYPE>((unsigned)qz_row_max<LPR>((float)qz_abs_bits(xin[u])));
+    } else {
 #pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-      if (v[j] != v[j]) nanf = 1.f;
-      mx = fmaxf(mx, KIND == 1 ? v[j] : fabsf(v[j]));
-      if (KIND == 1) mn = fminf(mn, v[j]);
+      for (int j = 0; j < EPL; ++j) {
+        if (v[j] != v[j]) nanf = 1.f;
+        mx = fmaxf(mx, KIND == 1 ? v[j] : fabsf(v[j]));
+        if (KIND == 1) mn = fminf(mn, v[j]);
+      }
+      mx = qz_row_max<LPR>(mx);
+      if (KIND == 1) mn = -qz_row_max<LPR>(-mn);
+      if (qz_row_max<LPR>(nanf) > 0.f) mx = mn = __builtin_nanf("");
     }
-    mx = qz_row_max<LPR>(mx);
-    if (KIND == 1) mn = -qz_row_max<LPR>(-mn);
-    if (qz_row_max<LPR>(nanf) > 0.f) mx = mn = __builtin_nanf("");
     if constexpr (KIND == 0 || KIND == 3 || KIND == 4) {
-      float sc = KIND == 4 ? mx : qz_round<DTYPE>(mx / qmax);
+      float sc = KIND == 4 ? mx : qz_round<DTYPE>(DTYPE == FC_BF16 ? mx * __builtin_amdgcn_rcpf(qmax) : mx / qmax);
       sc = qz_round<DTYPE>(sc != sc ? sc : fmaxf(sc, 1e-8f));
       if (live && sub == 0) qz_store<DTYPE>(scale, r, sc);
+      const float rs = __builtin_amdgcn_rcpf(sc);
+      const bool plain = sc > 0.f && sc < INFINITY;   // else: a NaN or an infinity in the row, or an fp16 scale that is 0
+      float t[EPL];
+      if (__all(plain)) {
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) t[j] = qz_quot<DTYPE>(v[j], sc, rs);
+        qz_round_finite<DTYPE>(t);
+      }
       if constexpr (KIND == 0) {
         unsigned w[EPL / 4] = {};
+        if (__all(plain)) {
+          // 1.5 * 2^23 + t rounds t half to even to an integer and holds it, in two's complement, in its low byte
 #pragma unroll
-        for (int j = 0; j < EPL; ++j) {
-          float t = rintf(qz_round<DTYPE>(v[j] / sc));
-          const bool is_nan = t != t;
-          t = fminf(fmaxf(t, -qmax - 1.f), qmax);
-          const int c = is_nan ? 0 : (int)t;
-          w[j / 4] |= ((unsigned)c & 0xffu) << (8 * (j & 3));
+          for (int j = 0; j < EPL; ++j) t[j] = __builtin_amdgcn_fmed3f(t[j], -qmax - 1.f, qmax) + 12582912.f;
+#pragma unroll
+          for (int j = 0; j < EPL; j += 4) {
+            const unsigned lo = __builtin_amdgcn_perm(__float_as_uint(t[j + 1]), __float_as_uint(t[j]), 0x0c0c0400u);
+            const unsigned hi = __builtin_amdgcn_perm(__float_as_uint(t[j + 3]), __float_as_uint(t[j + 2]), 0x04000c0cu);
+            w[j / 4] = lo | hi;
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < EPL; ++j) {
+            float y = rintf(qz_round<DTYPE>(v[j] / sc));
+            const bool is_nan = y != y;
+            y = fminf(fmaxf(y, -qmax - 1.f), qmax);
+            const int c = is_nan ? 0 : (int)y;
+            w[j / 4] |= ((unsigned)c & 0xffu) << (8 * (j & 3));
+          }
         }
         if (live) {
           if constexpr (EPL == 8) *reinterpret_cast<uint2*>(out + (r * LPR + sub) * 8) = make_uint2(w[0], w[1]);
@@ -490,8 +631,28 @@ __global__ __launch_bounds__(256) void quant_rows_fast_kernel(const char* __rest
         }
       } else {
         unsigned w = 0;
+        if (__all(plain)) {
+          if constexpr (KIND == 3) {
 #pragma unroll
-        for (int j = 0; j < EPL; ++j) w |= (unsigned)qz_code4<DTYPE, KIND == 4 ? 1 : 0>(v[j], sc, levels) << (4 * j);
+            for (int j = 0; j < EPL; ++j) t[j] = rintf(__builtin_amdgcn_fmed3f(t[j], -8.f, 7.f));
+          } else {
+#pragma unroll
+            for (int j = 0; j < EPL; ++j) {
+              const Nf4Bucket e = buckets[qz_bucket(t[j])];
+              t[j] = e.below + (t[j] >= e.th ? 1.f : 0.f);
+            }
+          }
+          // four codes as the digits of one number (0 .. 65535, exact)
+#pragma unroll
+          for (int j = 0; j < EPL; j += 4) {
+            float f = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(t[j + 3], 16.f, t[j + 2]), 16.f, t[j + 1]), 16.f, t[j]);
+            if (KIND == 3) f += (float)0x8888;
+            w |= (unsigned)f << (4 * j);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < EPL; ++j) w |= (unsigned)qz_code4<DTYPE, KIND == 4 ? 1 : 0>(v[j], sc, levels) << (4 * j);
+        }
         if (live) {
           if constexpr (EPL == 8) *reinterpret_cast<unsigned*>(out + (r * LPR + sub) * 4) = w;
           else *reinterpret_cast<unsigned short*>(out + (r * LPR + sub) * 2) = (unsigned short)w;
@@ -545,30 +706,79 @@ __device__ __forceinline__ void qz_store8(char* out, long long i8, const float (
   }
 }
 
+// ... of values whose sum `any` is not NaN (so none of them is): bf16 two per instruction
+template <int ODT>
+__device__ __forceinline__ void qz_store8(char* out, long long i8, const float (&y)[8], float any) {
+  if constexpr (ODT == FC_BF16) {
+    if (any == any) {
+      typedef float f2 __attribute__((ext_vector_type(2)));
+      typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+      const auto two = [&](int j) { return __builtin_bit_cast(unsigned, __builtin_convertvector((f2){y[j], y[j + 1]}, b2)); };
+      reinterpret_cast<uint4*>(out)[i8] = make_uint4(two(0), two(2), two(4), two(6));
+      return;
+    }
+  }
+  qz_store8<ODT>(out, i8, y);
+}
+// NaN if one of the values is
+__device__ __forceinline__ float qz_sum8(const float (&y)[8]) {
+  return ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
+}
+// eight float8 codes by the conversion instructions; NaN codes, whose sign those change, by the integer rule
+template <int E5M2>
+__device__ __forceinline__ void qz_from_fp8x8(const uint2& c, float (&v)[8]) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int j = 0; j < 8; j += 4) {
+    const unsigned w = j ? c.y : c.x;
+    const f2 a = E5M2 ? __builtin_amdgcn_cvt_pk_f32_bf8(w, false) : __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
+    const f2 b = E5M2 ? __builtin_amdgcn_cvt_pk_f32_bf8(w, true) : __builtin_amdgcn_cvt_pk_f32_fp8(w, true);
+    v[j] = a.x; v[j + 1] = a.y; v[j + 2] = b.x; v[j + 3] = b.y;
+  }
+  const float any = qz_sum8(v);
+  if (any != any) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = qz_from_fp8<E5M2>((unsigned char)((j < 4 ? c.x : c.y) >> (8 * (j & 3))));
+  }
+}
+
+// row (or group) of the i-th eight elements: a shift where the row length is a power of two, since a 64-bit division costs
+// a thread more than its eight elements do
+struct QzRowOf {
+  int d8, shift;
+  explicit QzRowOf(int d) : d8(d / 8), shift(-1) {
+    for (int s = 0; s < 28; ++s)
+      if ((1 << s) == d8) shift = s;
+  }
+  __device__ __forceinline__ long long operator()(long long i) const { return shift >= 0 ? i >> shift : i / d8; }
+};
+
 // out = float(code) * scale: int8 rows (KIND 0, one scale per d codes), fp8 (KIND 1 / 2 = E4M3 / E5M2, one scale)
 template <int SDT, int ODT, int KIND>
 __global__ __launch_bounds__(256) void dequantize_vec_kernel(const unsigned char* __restrict__ q,
-                                                             const char* __restrict__ scale, long long n8, int d,
+                                                             const char* __restrict__ scale, long long n8, QzRowOf row_of,
                                                              char* __restrict__ out) {
   const float sc1 = KIND == 0 ? 0.f : qz_load<SDT>(scale, 0);
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256) {
     const uint2 c = reinterpret_cast<const uint2*>(q)[i];
-    const float sc = KIND == 0 ? qz_load<SDT>(scale, (i * 8) / d) : sc1;
+    const float sc = KIND == 0 ? qz_load<SDT>(scale, row_of(i)) : sc1;
     float y[8];
+    if constexpr (KIND == 0) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const unsigned b = ((j < 4 ? c.x : c.y) >> (8 * (j & 3))) & 0xffu;
-      const float v = KIND == 0 ? (float)(signed char)b : KIND == 1 ? qz_from_fp8<0>((unsigned char)b) : qz_from_fp8<1>((unsigned char)b);
-      y[j] = v * sc;
+      for (int j = 0; j < 8; ++j) y[j] = (float)(signed char)(((j < 4 ? c.x : c.y) >> (8 * (j & 3))) & 0xffu);
+    } else {
+      qz_from_fp8x8<KIND == 2>(c, y);
     }
-    qz_store8<ODT>(out, i, y);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) y[j] *= sc;
+    qz_store8<ODT>(out, i, y, qz_sum8(y));
   }
 }
 
 // 4-bit codes, 8 elements = 4 bytes per thread; one scale per g elements
 template <int TDT, int SDT, int ODT, int MODE>
 __global__ __launch_bounds__(256) void dequantize_group4_vec_kernel(const unsigned char* __restrict__ packed,
-                                                                    const char* __restrict__ scale, long long n8, int g,
+                                                                    const char* __restrict__ scale, long long n8, QzRowOf row_of,
                                                                     char* __restrict__ out) {
   __shared__ float levels[16];
   if (MODE == 1) {
@@ -577,32 +787,43 @@ __global__ __launch_bounds__(256) void dequantize_group4_vec_kernel(const unsign
   }
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256) {
     const unsigned c = reinterpret_cast<const unsigned*>(packed)[i];
-    const float sc = qz_load<SDT>(scale, (i * 8) / g);
+    const float sc = qz_load<SDT>(scale, row_of(i));
     float y[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const unsigned code = (c >> (4 * j)) & 15u;
       y[j] = (MODE == 0 ? (float)(int)code - 8.f : levels[code]) * sc;
     }
-    qz_store8<ODT>(out, i, y);
+    qz_store8<ODT>(out, i, y, qz_sum8(y));
   }
 }
 
 // whole-tensor passes over 16-byte pieces: the largest |x| of a block's share, fp8 codes, quantise -> dequantise
 template <int DTYPE>
-__global__ __launch_bounds__(256) void absmax_partial_vec_kernel(const char* __restrict__ x, long long nv, long long n,
-                                                                 float* __restrict__ partial) {
+__global__ __launch_bounds__(256) void absmax_partial_vec_kernel(QzPair io, long long nv, long long n,
+                                                                 float* __restrict__ partials) {
+  const char* __restrict__ x = io.x[blockIdx.y];
+  float* __restrict__ partial = partials + blockIdx.y * QZ_PARTS;
   constexpr int EPL = QzV<DTYPE>::EPL;
   __shared__ float wm[4];
   float mx = 0.f;
   bool has_nan = false;
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nv; i += (long long)gridDim.x * 256) {
-    float v[EPL];
-    qz_unpack<DTYPE>(reinterpret_cast<const uint4*>(x)[i], v);
+  if constexpr (DTYPE != FC_F32) {
+    unsigned bits = 0;
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nv; i += (long long)gridDim.x * 256)
+      bits = max(bits, qz_abs_bits(reinterpret_cast<const uint4*>(x)[i]));
+    mx = qz_from_abs_bits<DTYPE>(bits);
+    has_nan = mx != mx;
+    mx = has_nan ? 0.f : mx;
+  } else {
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nv; i += (long long)gridDim.x * 256) {
+      float v[EPL];
+      qz_unpack<DTYPE>(reinterpret_cast<const uint4*>(x)[i], v);
 #pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-      has_nan |= v[j] != v[j];
-      mx = fmaxf(mx, fabsf(v[j]));
+      for (int j = 0; j < EPL; ++j) {
+        has_nan |= v[j] != v[j];
+        mx = fmaxf(mx, fabsf(v[j]));
+      }
     }
   }
   for (long long i = nv * EPL + (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
@@ -641,13 +862,15 @@ __device__ __forceinline__ float qz_reduce_partials(const float* __restrict__ pa
 
 // MODE 0: y = quantise -> dequantise with the whole-tensor scale; MODE 1 / 2: fp8 codes (E4M3 / E5M2)
 template <int DTYPE, int MODE>
-__global__ __launch_bounds__(256) void tensor_apply_vec_kernel(const char* __restrict__ x, long long nv, long long n,
-                                                               const float* __restrict__ partial, int nparts,
-                                                               float qmax, char* __restrict__ y,
-                                                               char* __restrict__ scale, char* __restrict__ absmax) {
+__global__ __launch_bounds__(256) void tensor_apply_vec_kernel(QzPair io, long long nv, long long n,
+                                                               const float* __restrict__ partials, int nparts, float qmax) {
   constexpr int EPL = QzV<DTYPE>::EPL;
   __shared__ float wm[4];
-  const float mx = qz_reduce_partials(partial, nparts, wm);
+  const char* __restrict__ x = io.x[blockIdx.y];
+  char* __restrict__ y = io.out[blockIdx.y];
+  char* __restrict__ scale = io.scale[blockIdx.y];
+  char* __restrict__ absmax = io.absmax;
+  const float mx = qz_reduce_partials(partials + blockIdx.y * QZ_PARTS, nparts, wm);
   float sc;
   if (MODE == 0) {
     sc = qz_round<DTYPE>(mx / qmax);
@@ -659,6 +882,8 @@ __global__ __launch_bounds__(256) void tensor_apply_vec_kernel(const char* __res
     if (scale) qz_store<DTYPE>(scale, 0, sc);
     if (absmax) qz_store<DTYPE>(absmax, 0, mx);
   }
+  const float rs = __builtin_amdgcn_rcpf(sc);
+  const bool plain = sc > 0.f && sc < INFINITY;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nv; i += (long long)gridDim.x * 256) {
     float v[EPL];
     qz_unpack<DTYPE>(reinterpret_cast<const uint4*>(x)[i], v);
@@ -669,9 +894,18 @@ __global__ __launch_bounds__(256) void tensor_apply_vec_kernel(const char* __res
       reinterpret_cast<uint4*>(y)[i] = qz_pack<DTYPE>(o);
     } else {
       unsigned w[EPL / 4] = {};
+      if (plain) {   // the same for the whole tensor
 #pragma unroll
-      for (int j = 0; j < EPL; ++j)
-        w[j / 4] |= (unsigned)qz_to_fp8<MODE == 2>(qz_round<DTYPE>(v[j] / sc)) << (8 * (j & 3));
+        for (int j = 0; j < EPL; ++j)   // the correction step turns -0 into +0
+          v[j] = DTYPE == FC_F16 ? copysignf(qz_quot<DTYPE>(v[j], sc, rs), v[j]) : qz_quot<DTYPE>(v[j], sc, rs);
+        qz_round_finite<DTYPE>(v);
+#pragma unroll
+        for (int j = 0; j < EPL; j += 4) w[j / 4] = qz_to_fp8x4<MODE == 2>(v[j], v[j + 1], v[j + 2], v[j + 3]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < EPL; ++j)
+          w[j / 4] |= (unsigned)qz_to_fp8<MODE == 2>(qz_round<DTYPE>(v[j] / sc)) << (8 * (j & 3));
+      }
       if constexpr (EPL == 8) reinterpret_cast<uint2*>(y)[i] = make_uint2(w[0], w[1]);
       else reinterpret_cast<unsigned*>(y)[i] = w[0];
     }
@@ -690,25 +924,25 @@ static inline int qz_fast_lpr(const void* x, long long row_elems, int dtype) {
   return bytes == 128 ? 8 : bytes == 256 ? 16 : bytes == 512 ? 32 : 0;
 }
 
-#define QZ_FAST_LAUNCH(DT, LPRV, KIND, ...)                                                                        \
-  do {                                                                                                             \
-    const long long per_block = (256 / (LPRV)) * QZ_U;                                                             \
-    const long long nb = (rows_ + per_block - 1) / per_block;                                                      \
-    if (nb > 2147483647LL) { fc_set_error("%s: too many rows", who); return FC_EUNSUPPORTED; }                     \
-    hipLaunchKernelGGL((quant_rows_fast_kernel<DT, LPRV, KIND>), dim3((unsigned)nb), dim3(256), 0, st, __VA_ARGS__); \
-  } while (0)
-#define QZ_FAST_LPR(DT, KIND, ...)                                   \
-  do {                                                               \
-    if (lpr == 8) QZ_FAST_LAUNCH(DT, 8, KIND, __VA_ARGS__);          \
-    else if (lpr == 16) QZ_FAST_LAUNCH(DT, 16, KIND, __VA_ARGS__);   \
-    else QZ_FAST_LAUNCH(DT, 32, KIND, __VA_ARGS__);                  \
-  } while (0)
-#define QZ_FAST(KIND, ...)                                           \
-  do {                                                               \
-    if (dtype == FC_F32) QZ_FAST_LPR(FC_F32, KIND, __VA_ARGS__);     \
-    else if (dtype == FC_F16) QZ_FAST_LPR(FC_F16, KIND, __VA_ARGS__); \
-    else QZ_FAST_LPR(FC_BF16, KIND, __VA_ARGS__);                    \
-  } while (0)
+template <int DTYPE, int KIND>
+static int qz_launch_rows(const char* who, const QzPair& io, int tensors, int lpr, long long rows, float qmax, hipStream_t st) {
+  const long long per_block = (256 / lpr) * QZ_U, nb = (rows + per_block - 1) / per_block;
+  FC_REQUIRE(nb <= 2147483647LL, FC_EUNSUPPORTED, "%s: too many rows", who);
+  const dim3 grid((unsigned)nb, tensors), block(256);
+  if (lpr == 8) hipLaunchKernelGGL((quant_rows_fast_kernel<DTYPE, 8, KIND>), grid, block, 0, st, io, rows, qmax);
+  else if (lpr == 16) hipLaunchKernelGGL((quant_rows_fast_kernel<DTYPE, 16, KIND>), grid, block, 0, st, io, rows, qmax);
+  else hipLaunchKernelGGL((quant_rows_fast_kernel<DTYPE, 32, KIND>), grid, block, 0, st, io, rows, qmax);
+  return FC_OK;
+}
+template <int KIND>
+static int qz_fast(const char* who, const QzPair& io, int tensors, int lpr, long long rows, int dtype, float qmax, hipStream_t st) {
+  if (dtype == FC_F32) return qz_launch_rows<FC_F32, KIND>(who, io, tensors, lpr, rows, qmax, st);
+  if (dtype == FC_F16) return qz_launch_rows<FC_F16, KIND>(who, io, tensors, lpr, rows, qmax, st);
+  return qz_launch_rows<FC_BF16, KIND>(who, io, tensors, lpr, rows, qmax, st);
+}
+static inline QzPair qz_one(const void* x, void* out, void* scale, void* absmax = nullptr) {
+  return QzPair{{(const char*)x, nullptr}, {(char*)out, nullptr}, {(char*)scale, nullptr}, (char*)absmax};
+}
 
 extern "C" int64_t fc_fake_quantize_workspace_bytes(void) { return QZ_PARTS * (int64_t)sizeof(float); }
 
@@ -724,9 +958,8 @@ extern "C" int fc_fake_quantize(const void* x, void* y, int64_t rows, int32_t d,
   const float qmax = (float)((1 << (bits - 1)) - 1);
   hipStream_t st = (hipStream_t)stream;
   if (!per_tensor && qz_fast_lpr(x, d, dtype) && ((uintptr_t)y & 15) == 0) {
-    const int lpr = qz_fast_lpr(x, d, dtype);
-    const long long rows_ = rows;
-    QZ_FAST(2, (const char*)x, (long long)rows, qmax, (char*)y, (char*)scale, (char*)absmax);
+    const int rc = qz_fast<2>(who, qz_one(x, y, scale, absmax), 1, qz_fast_lpr(x, d, dtype), rows, dtype, qmax, st);
+    if (rc) return rc;
   } else if (!per_tensor) {
     const long long blocks = (rows + 3) / 4;
     FC_REQUIRE(blocks <= 2147483647LL, FC_EUNSUPPORTED, "%s: too many rows", who);
@@ -747,10 +980,10 @@ extern "C" int fc_fake_quantize(const void* x, void* y, int64_t rows, int32_t d,
   do {                                                                                                               \
     if (vec) {                                                                                                       \
       const long long nv = n / QzV<DT>::EPL;                                                                         \
-      hipLaunchKernelGGL((absmax_partial_vec_kernel<DT>), dim3(nparts), dim3(256), 0, st, (const char*)x, nv, n,     \
-                         (float*)workspace);                                                                         \
-      hipLaunchKernelGGL((tensor_apply_vec_kernel<DT, 0>), dim3(blocks), dim3(256), 0, st, (const char*)x, nv, n,    \
-                         (const float*)workspace, nparts, qmax, (char*)y, (char*)scale, (char*)absmax);              \
+      const QzPair io = qz_one(x, y, scale, absmax);                                                                 \
+      hipLaunchKernelGGL((absmax_partial_vec_kernel<DT>), dim3(nparts), dim3(256), 0, st, io, nv, n, (float*)workspace); \
+      hipLaunchKernelGGL((tensor_apply_vec_kernel<DT, 0>), dim3(blocks), dim3(256), 0, st, io, nv, n,                \
+                         (const float*)workspace, nparts, qmax);                                                     \
     } else {                                                                                                         \
       hipLaunchKernelGGL((absmax_partial_kernel<DT>), dim3(nparts), dim3(256), 0, st, (const char*)x, n,             \
                          (float*)workspace);                                                                         \
@@ -778,8 +1011,8 @@ extern "C" int fc_quantize_rows(const void* x, int64_t rows, int32_t d, int32_t 
   const float qmax = (float)((1 << (bits - 1)) - 1);
   hipStream_t st = (hipStream_t)stream;
   if (const int lpr = qz_fast_lpr(x, d, dtype); lpr && ((uintptr_t)q & 7) == 0) {
-    const long long rows_ = rows;
-    QZ_FAST(0, (const char*)x, (long long)rows, qmax, (char*)q, (char*)scale, (char*)nullptr);
+    const int rc = qz_fast<0>(who, qz_one(x, q, scale), 1, lpr, rows, dtype, qmax, st);
+    if (rc) return rc;
     FC_CHECK_LAUNCH(who);
     return FC_OK;
   }
@@ -809,7 +1042,7 @@ extern "C" int fc_dequantize_rows(const int8_t* q, const void* scale, int64_t ro
   do {                                                                                                               \
     if (vec)                                                                                                         \
       hipLaunchKernelGGL((dequantize_vec_kernel<S, O, 0>), dim3(blocks8), dim3(256), 0, st, (const unsigned char*)q, \
-                         (const char*)scale, n8, d, (char*)out);                                                     \
+                         (const char*)scale, n8, QzRowOf(d), (char*)out);                                                     \
     else                                                                                                             \
       hipLaunchKernelGGL((dequantize_rows_kernel<S, O>), dim3((unsigned)blocks), dim3(256), 0, st,                   \
                          (const signed char*)q, (const char*)scale, (long long)rows, d, (char*)out);                 \
@@ -828,6 +1061,20 @@ extern "C" int fc_dequantize_rows(const int8_t* q, const void* scale, int64_t ro
   return FC_OK;
 }
 
+static int qz_fp8_parts(long long n) { return (int)((n + 255) / 256 < QZ_PARTS ? (n + 255) / 256 : QZ_PARTS); }
+static unsigned qz_fp8_blocks(long long n) { return (unsigned)((n + 1023) / 1024 < QZ_GRID_CAP ? (n + 1023) / 1024 : QZ_GRID_CAP); }
+
+// 16-byte aligned inputs: one absmax and one conversion launch for one or two tensors of n elements
+template <int DTYPE>
+static void qz_fp8_vec(const QzPair& io, int tensors, long long n, int e5m2, float* partials, hipStream_t st) {
+  const long long nv = n / QzV<DTYPE>::EPL;
+  const int nparts = qz_fp8_parts(n);
+  const dim3 grid(qz_fp8_blocks(n), tensors), block(256);
+  hipLaunchKernelGGL((absmax_partial_vec_kernel<DTYPE>), dim3(nparts, tensors), block, 0, st, io, nv, n, partials);
+  if (e5m2) hipLaunchKernelGGL((tensor_apply_vec_kernel<DTYPE, 2>), grid, block, 0, st, io, nv, n, (const float*)partials, nparts, 0.f);
+  else hipLaunchKernelGGL((tensor_apply_vec_kernel<DTYPE, 1>), grid, block, 0, st, io, nv, n, (const float*)partials, nparts, 0.f);
+}
+
 extern "C" int fc_quantize_fp8(const void* x, int64_t n, int32_t dtype, int32_t e5m2, uint8_t* q, void* scale,
                                void* workspace, int64_t workspace_bytes, void* stream) {
   const char* who = "fc_quantize_fp8";
@@ -838,24 +1085,13 @@ extern "C" int fc_quantize_fp8(const void* x, int64_t n, int32_t dtype, int32_t 
              "%s: needs a workspace of %lld bytes", who, (long long)fc_fake_quantize_workspace_bytes());
   if (n == 0) return FC_OK;
   hipStream_t st = (hipStream_t)stream;
-  const int nparts = (int)((n + 255) / 256 < QZ_PARTS ? (n + 255) / 256 : QZ_PARTS);
-  const long long want = (n + 1023) / 1024;
-  const unsigned blocks = (unsigned)(want < QZ_GRID_CAP ? want : QZ_GRID_CAP);
+  const int nparts = qz_fp8_parts(n);
+  const unsigned blocks = qz_fp8_blocks(n);
   const bool vec = ((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 7) == 0;
 #define F8(DT)                                                                                                       \
   do {                                                                                                               \
     if (vec) {                                                                                                       \
-      const long long nv = n / QzV<DT>::EPL;                                                                         \
-      hipLaunchKernelGGL((absmax_partial_vec_kernel<DT>), dim3(nparts), dim3(256), 0, st, (const char*)x, nv,        \
-                         (long long)n, (float*)workspace);                                                           \
-      if (e5m2)                                                                                                      \
-        hipLaunchKernelGGL((tensor_apply_vec_kernel<DT, 2>), dim3(blocks), dim3(256), 0, st, (const char*)x, nv,     \
-                           (long long)n, (const float*)workspace, nparts, 0.f, (char*)q, (char*)scale,               \
-                           (char*)nullptr);                                                                          \
-      else                                                                                                           \
-        hipLaunchKernelGGL((tensor_apply_vec_kernel<DT, 1>), dim3(blocks), dim3(256), 0, st, (const char*)x, nv,     \
-                           (long long)n, (const float*)workspace, nparts, 0.f, (char*)q, (char*)scale,               \
-                           (char*)nullptr);                                                                          \
+      qz_fp8_vec<DT>(qz_one(x, q, scale), 1, n, e5m2, (float*)workspace, st);                                        \
       break;                                                                                                         \
     }                                                                                                                \
     hipLaunchKernelGGL((absmax_partial_kernel<DT>), dim3(nparts), dim3(256), 0, st, (const char*)x, (long long)n,   \
@@ -890,10 +1126,10 @@ extern "C" int fc_dequantize_fp8(const uint8_t* q, const void* scale, int64_t n,
     if (vec) {                                                                                                       \
       if (e5m2)                                                                                                      \
         hipLaunchKernelGGL((dequantize_vec_kernel<S, O, 2>), dim3(blocks8), dim3(256), 0, st,                        \
-                           (const unsigned char*)q, (const char*)scale, (long long)(n / 8), 1, (char*)out);          \
+                           (const unsigned char*)q, (const char*)scale, (long long)(n / 8), QzRowOf(8), (char*)out);          \
       else                                                                                                           \
         hipLaunchKernelGGL((dequantize_vec_kernel<S, O, 1>), dim3(blocks8), dim3(256), 0, st,                        \
-                           (const unsigned char*)q, (const char*)scale, (long long)(n / 8), 1, (char*)out);          \
+                           (const unsigned char*)q, (const char*)scale, (long long)(n / 8), QzRowOf(8), (char*)out);          \
       break;                                                                                                         \
     }                                                                                                                \
     if (e5m2)                                                                                                        \
@@ -928,8 +1164,8 @@ extern "C" int fc_quantize_rows_asym(const void* x, int64_t rows, int32_t d, int
   FC_REQUIRE(blocks <= 2147483647LL, FC_EUNSUPPORTED, "%s: too many rows", who);
   hipStream_t st = (hipStream_t)stream;
   if (const int lpr = qz_fast_lpr(x, d, dtype); lpr && ((uintptr_t)q & 7) == 0) {
-    const long long rows_ = rows;
-    QZ_FAST(1, (const char*)x, (long long)rows, 0.f, (char*)q, (char*)params, (char*)nullptr);
+    const int rc = qz_fast<1>(who, qz_one(x, q, params), 1, lpr, rows, dtype, 0.f, st);
+    if (rc) return rc;
     FC_CHECK_LAUNCH(who);
     return FC_OK;
   }
@@ -953,9 +1189,9 @@ extern "C" int fc_quantize_group4(const void* x, int64_t groups, int32_t group_s
   FC_REQUIRE(blocks <= 2147483647LL, FC_EUNSUPPORTED, "%s: too many groups", who);
   hipStream_t st = (hipStream_t)stream;
   if (const int lpr = qz_fast_lpr(x, group_size, dtype); lpr && ((uintptr_t)packed & 3) == 0) {
-    const long long rows_ = groups;
-    if (nf4) QZ_FAST(4, (const char*)x, (long long)groups, 1.f, (char*)packed, (char*)scale, (char*)nullptr);
-    else QZ_FAST(3, (const char*)x, (long long)groups, 7.f, (char*)packed, (char*)scale, (char*)nullptr);
+    const QzPair io = qz_one(x, packed, scale);
+    const int rc = nf4 ? qz_fast<4>(who, io, 1, lpr, groups, dtype, 1.f, st) : qz_fast<3>(who, io, 1, lpr, groups, dtype, 7.f, st);
+    if (rc) return rc;
     FC_CHECK_LAUNCH(who);
     return FC_OK;
   }
@@ -986,7 +1222,7 @@ extern "C" int fc_dequantize_group4(const uint8_t* packed, const void* scale, in
   do {                                                                                                               \
     if (vec)                                                                                                         \
       hipLaunchKernelGGL((dequantize_group4_vec_kernel<T, S, O, MD>), dim3(blocks8), dim3(256), 0, st,               \
-                         (const unsigned char*)packed, (const char*)scale, n8, group_size, (char*)out);              \
+                         (const unsigned char*)packed, (const char*)scale, n8, QzRowOf(group_size), (char*)out);              \
     else                                                                                                             \
       hipLaunchKernelGGL((dequantize_group4_kernel<T, S, O, MD>), dim3((unsigned)blocks), dim3(256), 0, st,          \
                          (const unsigned char*)packed, (const char*)scale, (long long)groups, group_size,            \
@@ -1005,6 +1241,52 @@ extern "C" int fc_dequantize_group4(const uint8_t* packed, const void* scale, in
   else { fc_set_error("%s: table dtype %d with scale dtype %d", who, t, sd); return FC_EUNSUPPORTED; }
 #undef DGD
 #undef DG
+  FC_CHECK_LAUNCH(who);
+  return FC_OK;
+}
+
+extern "C" int64_t fc_quantize_pair_workspace_bytes(int32_t kind) {
+  return kind == FC_QUANT_E4M3 || kind == FC_QUANT_E5M2 ? 2 * fc_fake_quantize_workspace_bytes() : 0;
+}
+
+extern "C" int fc_quantize_pair(int32_t kind, const void* x0, const void* x1, int64_t rows, int32_t d, int32_t dtype,
+                                void* codes0, void* codes1, void* scale0, void* scale1, void* workspace,
+                                int64_t workspace_bytes, void* stream) {
+  const char* who = "fc_quantize_pair";
+  FC_REQUIRE(kind >= FC_QUANT_INT8 && kind <= FC_QUANT_E5M2, FC_EINVAL, "%s: kind %d", who, kind);
+  FC_REQUIRE(x0 && x1 && codes0 && codes1 && scale0 && scale1, FC_EINVAL, "%s: null pointer", who);
+  FC_REQUIRE(rows >= 0 && d > 0, FC_EINVAL, "%s: bad sizes rows=%lld d=%d", who, (long long)rows, d);
+  FC_REQUIRE(dtype == FC_F32 || dtype == FC_F16 || dtype == FC_BF16, FC_EUNSUPPORTED, "%s: dtype %d", who, dtype);
+  if (rows == 0) return FC_OK;
+  hipStream_t st = (hipStream_t)stream;
+  const QzPair io{{(const char*)x0, (const char*)x1}, {(char*)codes0, (char*)codes1}, {(char*)scale0, (char*)scale1}, nullptr};
+  const bool fp8 = kind == FC_QUANT_E4M3 || kind == FC_QUANT_E5M2;
+  const bool aligned = ((((uintptr_t)x0 | (uintptr_t)x1) & 15) | (((uintptr_t)codes0 | (uintptr_t)codes1) & 7)) == 0;
+  const int lpr = qz_fast_lpr(x0, d, dtype);
+  int rc = FC_OK;
+  if (aligned && fp8) {
+    FC_REQUIRE(workspace && workspace_bytes >= fc_quantize_pair_workspace_bytes(kind), FC_EINVAL, "%s: workspace too small", who);
+    const long long n = rows * (long long)d;
+    const int e5m2 = kind == FC_QUANT_E5M2;
+    if (dtype == FC_F32) qz_fp8_vec<FC_F32>(io, 2, n, e5m2, (float*)workspace, st);
+    else if (dtype == FC_F16) qz_fp8_vec<FC_F16>(io, 2, n, e5m2, (float*)workspace, st);
+    else qz_fp8_vec<FC_BF16>(io, 2, n, e5m2, (float*)workspace, st);
+  } else if (aligned && lpr) {
+    if (kind == FC_QUANT_INT8) rc = qz_fast<0>(who, io, 2, lpr, rows, dtype, 127.f, st);
+    else if (kind == FC_QUANT_INT4) rc = qz_fast<3>(who, io, 2, lpr, rows, dtype, 7.f, st);
+    else rc = qz_fast<4>(who, io, 2, lpr, rows, dtype, 1.f, st);
+  } else {   // other row lengths and alignments: one tensor after the other
+    for (int i = 0; i < 2 && !rc; ++i) {
+      if (fp8)
+        rc = fc_quantize_fp8(io.x[i], rows * (int64_t)d, dtype, kind == FC_QUANT_E5M2, (uint8_t*)io.out[i], io.scale[i], workspace,
+                             workspace_bytes, stream);
+      else if (kind == FC_QUANT_INT8)
+        rc = fc_quantize_rows(io.x[i], rows, d, dtype, 8, (int8_t*)io.out[i], io.scale[i], stream);
+      else
+        rc = fc_quantize_group4(io.x[i], rows, d, dtype, kind == FC_QUANT_NF4, (uint8_t*)io.out[i], io.scale[i], stream);
+    }
+  }
+  if (rc) return rc;
   FC_CHECK_LAUNCH(who);
   return FC_OK;
 }

@@ -438,6 +438,13 @@ int fc_dequantize_fp8(const uint8_t* q, const void* scale, int64_t n, int32_t e5
 int fc_quantize_rows_asym(const void* x, int64_t rows, int32_t d, int32_t dtype, uint8_t* q, void* params,
                           void* stream);
 
+/* Two tensors of one shape (a cache's keys and values) in the launches of one; results as by the single entry points:
+ * int8 rows of d (8 bits), groups of d in 4 bits, or float8 over rows * d elements. */
+enum { FC_QUANT_INT8 = 0, FC_QUANT_INT4 = 1, FC_QUANT_NF4 = 2, FC_QUANT_E4M3 = 3, FC_QUANT_E5M2 = 4 };
+int64_t fc_quantize_pair_workspace_bytes(int32_t kind);
+int fc_quantize_pair(int32_t kind, const void* x0, const void* x1, int64_t rows, int32_t d, int32_t dtype, void* codes0,
+                     void* codes1, void* scale0, void* scale1, void* workspace, int64_t workspace_bytes, void* stream);
+
 /*
  * 4-bit quantisation of groups of `group_size` consecutive elements, two codes per byte (element 2j in
  * the low nibble), one scale per group in the dtype of x.

@@ -441,3 +441,52 @@ def test_quantisers_special_rows_all_row_lengths(dev, dtype, d):
         same(mx, rmx)
         same(sc, rsc)
         same(y, ry)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["int8", "int4", "nf4", "fp8_e4m3", "fp8_e5m2"])
+def test_quantised_pair_every_significand(dev, dtype, kind):
+    """Keys and values quantised together and back against the eager expressions, bit for bit: rows whose largest
+    magnitude and elements run over the dtype's bit patterns (each quotient's rounding is decided by its last bits), rows
+    with a NaN, an infinity, only zeros and only tiny values, a row count that leaves the last block partly empty, and a
+    row length and an alignment that take the generic kernels."""
+    g = torch.Generator().manual_seed(7)
+    itype, mant, top = {torch.float32: (torch.int32, 23, 0x42000000), torch.float16: (torch.int16, 10, 0x4400),
+                        torch.bfloat16: (torch.int16, 7, 0x4200)}[dtype]
+    quant = {"int8": lambda t: oa.quantize_int8(t), "int4": lambda t: oa.quantize_int4(t, 128), "nf4": lambda t: oa.quantize_nf4(t, 128),
+             "fp8_e4m3": lambda t: oa.quantize_fp8(t, False), "fp8_e5m2": lambda t: oa.quantize_fp8(t, True)}[kind]
+
+    def rows(n):
+        largest = torch.randint(top - (4 << mant), top, (n, 1), generator=g)
+        bits = (largest - torch.randint(0, 12 << mant, (n, 128), generator=g)).clamp_min(0)
+        bits[:, 0] = largest[:, 0]
+        x = bits.to(itype).view(dtype)
+        return torch.where(torch.rand(n, 128, generator=g) < 0.5, -x, x)
+
+    def bits_of(t):
+        return t.cpu().contiguous().view(torch.uint8)
+
+    method = ac.QuantizationMethod(kind)
+    x = [rows(2051), rows(2051)]
+    special = [t.clone() for t in x]
+    for t in special:
+        t[3], t[4], t[5, 9], t[6, 11] = 0, t[4] * 1e-4, float("nan"), float("inf")
+    for k, v in (x, special):
+        if kind.startswith("fp8") and k is special[0]:
+            continue                                   # one scale for the tensor: a NaN makes every code NaN
+        got = method.compress(k.to(dev), v.to(dev))
+        for (q, s), t in zip(got, (k, v)):
+            rq, rs = quant(t)
+            assert torch.equal(bits_of(q), bits_of(rq)) and s.dtype == t.dtype
+            assert torch.equal(s.cpu().reshape(-1).nan_to_num(7.0), rs.reshape(-1).expand(s.numel()).nan_to_num(7.0))
+            back = method.dequantize(q, s, dtype).cpu()
+            if kind in ("int4", "nf4"):
+                ref = oa.dequantize_4bit(q.cpu(), s.cpu(), 128, kind == "nf4", dtype)
+            else:
+                ref = (q.cpu().float() * s.cpu().float().reshape(-1, 1)).to(dtype)
+            assert torch.equal(back.nan_to_num(7.0), ref.nan_to_num(7.0)) and torch.equal(back.isnan(), ref.isnan())
+    if not kind.startswith("fp8") and kind != "int8":
+        return
+    k, v = x[0][:40, :40].contiguous().to(dev), torch.cat([x[0].reshape(-1)[:1601]]).to(dev)[1:].view(40, 40)
+    for (q, s), t in zip(method.compress(k, v), (k, v)):
+        assert torch.equal(bits_of(q), bits_of(quant(t.cpu())[0]))
