@@ -448,7 +448,7 @@ __device__ __forceinline__ float qz_row_max(float v) {
 // than a value has: p + 1 where sc has p, so m * sc = v is impossible for an odd p + 1 bit m, and no quotient is nearer to
 // a midpoint than 2^-(2p + 1) of itself.  bf16 (p = 8): v * rs, off by 2^-22, is near enough.  fp16 (p = 11): one
 // correction step leaves half a last place of fp32, 2^-24 (below the smallest normal number, where midpoints have fewer
-// bits and can be met, the step makes such a quotient exact).  Both for finite sc > 0 and |v| <= the row's largest.
+// bits and can be met, the step makes such a quotient exact).  Both for 0 < sc < 2^126 and |v| <= the row's largest.
 // The division instruction sequence costs ten operations per element, more than reading and storing it.
 template <int DTYPE>
 __device__ __forceinline__ float qz_quot(float v, float sc, float rs) {
@@ -596,7 +596,9 @@ __global__ __launch_bounds__(256) void quant_rows_fast_kernel(QzPair io, long lo
       sc = qz_round<DTYPE>(sc != sc ? sc : fmaxf(sc, 1e-8f));
       if (live && sub == 0) qz_store<DTYPE>(scale, r, sc);
       const float rs = __builtin_amdgcn_rcpf(sc);
-      const bool plain = sc > 0.f && sc < INFINITY;   // else: a NaN or an infinity in the row, or an fp16 scale that is 0
+      // else: a NaN or an infinity in the row, an fp16 scale that is 0, or a reciprocal below the normal numbers, which the
+      // instruction gives as 0 (the largest bf16 values as an NF4 scale)
+      const bool plain = sc > 0.f && sc < 0x1p126f;
       float t[EPL];
       if (__all(plain)) {
 #pragma unroll
@@ -883,7 +885,7 @@ __global__ __launch_bounds__(256) void tensor_apply_vec_kernel(QzPair io, long l
     if (absmax) qz_store<DTYPE>(absmax, 0, mx);
   }
   const float rs = __builtin_amdgcn_rcpf(sc);
-  const bool plain = sc > 0.f && sc < INFINITY;
+  const bool plain = sc > 0.f && sc < 0x1p126f;   // as in the row kernel
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nv; i += (long long)gridDim.x * 256) {
     float v[EPL];
     qz_unpack<DTYPE>(reinterpret_cast<const uint4*>(x)[i], v);
