@@ -614,13 +614,14 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     for (int e = 1; e < 8; ++e) mx = fmaxf(mx, p[e]);
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m, mx);              // finite: a tile that is walked holds at least one live key
-    const float alpha = __builtin_amdgcn_exp2f(m - mn);
-    m = mn;
+    const float mo = m;
+    m = fmaxf(m, mx);
+    const float ref = m == -INFINITY ? 0.f : m;   // so far only logits of -inf: they weigh nothing, and -inf - -inf is NaN
+    const float alpha = __builtin_amdgcn_exp2f(mo - ref);
     float sum = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      p[e] = __builtin_amdgcn_exp2f(p[e] - mn);
+      p[e] = __builtin_amdgcn_exp2f(p[e] - ref);
       sum += p[e];
     }
     l = fmaf(l, alpha, sum);
@@ -675,7 +676,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   for (int w = 0; w < DC_WAVES; ++w) M = fmaxf(M, ml[w * DC_HEADS + l15].x);
   float* part = reinterpret_cast<float*>(smem);
   {
-    const float wgt = __builtin_amdgcn_exp2f(m - M);        // 0 for a wavefront without tiles
+    const float wgt = __builtin_amdgcn_exp2f(m - (M == -INFINITY ? 0.f : M));   // 0 for a wavefront without tiles
     if (l15 < ng) {
 #pragma unroll
       for (int db = 0; db < 8; ++db)
@@ -691,7 +692,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
 #pragma unroll
     for (int w = 0; w < DC_WAVES; ++w) {
       const float2 x = ml[w * DC_HEADS + g];
-      lg = fmaf(__builtin_amdgcn_exp2f(x.x - mg), x.y, lg);
+      lg = fmaf(__builtin_amdgcn_exp2f(x.x - (mg == -INFINITY ? 0.f : mg)), x.y, lg);
       acc += part[(w * DC_HEADS + g) * DC_PSTRIDE + d];
     }
     if (max_splits == 1) {

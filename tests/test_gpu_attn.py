@@ -297,3 +297,26 @@ def test_attention_layer_appends_and_attends(dev, dtype, Hq, Hkv, lens, slot_at)
         reset_context()
     assert torch.equal(on_gpu.cpu(), pool)
     assert float((got.float() - ref.float()).abs().max()) < 4e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lens,max_pages", [([200, 33, 64], 1), ([700, 300], 3)])     # one workgroup a column; several
+def test_keys_of_infinite_distance_weigh_nothing(dev, dtype, lens, max_pages):
+    """Keys whose logit is -inf (here the first ones of every context, whole 32-key tiles and, in the longer contexts, a
+    whole workgroup's range) take no weight, as in a softmax over the whole row."""
+    from fastcache_amd.layers.attention import decode_attention
+    Hq, Hkv, B = 8, 2, len(lens)
+    case = synth.make_paged_case(seed=5, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=lens, dtype=dtype)
+    pool = case.kv_cache[:, 0].clone()
+    for b, n in enumerate(lens):
+        for p in range(n // 2):
+            pool[0, case.block_tables[b][p // 256], p % 256, :, 0] = -float("inf")
+    q = torch.randn(B, Hq, 128, generator=torch.Generator().manual_seed(1)).to(dtype)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    tables, lens_t = case.table_tensor("cpu"), torch.tensor(lens, dtype=torch.int32)
+    assert tables.shape[1] == max_pages
+    ref = oattn.decode_attention(q, pool[0], pool[1], lens_t, tables, 128 ** -0.5)
+    assert bool(torch.isfinite(ref).all())
+    on_gpu = pool.to(dev)
+    got = decode_attention(q.to(dev), on_gpu[0], on_gpu[1], lens_t.to(dev), tables.to(dev), 128 ** -0.5).cpu()
+    assert float((got.float() - ref.float()).abs().max()) < 4e-3      # as for finite keys above
