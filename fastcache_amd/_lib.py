@@ -177,8 +177,16 @@ def compute_units(device: torch.device) -> int:
     return n
 
 
+def refuse_capture() -> None:
+    """Raise while the current stream is being captured: a copy from this call's staging memory would be read again by
+    every replay, after the memory has gone to somebody else."""
+    if torch.cuda.is_current_stream_capturing():
+        raise FastcacheError("numbers held by the host cannot be uploaded while a graph is being captured")
+
+
 def upload_ints(values, ref: torch.Tensor) -> torch.Tensor:
     """A list of Python ints as an int32 tensor on the device of ``ref``, through pinned memory and without waiting."""
+    refuse_capture()
     return host().upload_tables([], (list(values),), ref)[1]
 
 

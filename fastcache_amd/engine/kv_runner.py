@@ -85,6 +85,7 @@ class PagedKVRunner:
         return _lib.host().upload_tables([s.block_table for s in seqs], (), self.kv_cache)[0]
 
     def _table_and_lens(self, tables: Seq[Seq[int]], lens: Seq[int]):
+        _lib.refuse_capture()
         return _lib.host().upload_tables([list(t) for t in tables], (list(lens),), self.kv_cache)
 
     # -- paged <-> HuggingFace layout ----------------------------------------------------------------

@@ -209,6 +209,7 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
             raise FastcacheError(f"snapkv_press: kept counts must exceed the window ({window}) and fit the index row "
                                  f"({k}) for every sequence longer than the window; offending sequences: {bad}")
         if len(set(lens_h)) > 1:            # the longest sequences' columns start first
+            _lib.refuse_capture()
             n_kept, order = _lib.host().upload_tables(
                 [], (counts, sorted(range(len(lens_h)), key=lambda b: -lens_h[b])), queries)[1:]
         else:

@@ -350,3 +350,19 @@ def test_snapkv_press_object_with_the_prefill_log_sum_exp(dev):
         for (ak, av), (bk, bv) in zip(opaged.extract_kv(pools[0][0], pools[0][1][b], 350),
                                       opaged.extract_kv(pools[1][0], pools[1][1][b], 350)):
             assert torch.equal(ak, bk) and torch.equal(av, bv)
+
+
+def test_host_numbers_are_not_uploaded_under_capture(dev):
+    """A replay would read the staging memory of the captured call again: refused, and the capture stays usable."""
+    from fastcache_amd import _lib
+    x = torch.zeros(4, device=dev)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.add_(1)
+        with pytest.raises(_lib.FastcacheError, match="captured"):
+            _lib.upload_ints([1, 2], x)
+    for _ in range(3):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert bool((x == 3).all())
+    assert _lib.upload_ints([1, 2], x).tolist() == [1, 2]
