@@ -124,7 +124,8 @@ struct Watch {
 
 const char* const kWatch = "fastcache_amd.Watch";
 
-int64_t version_of(const at::Tensor& t) { return t.is_inference() ? 0 : (int64_t)t._version(); }
+// inference tensors keep no version, so a write to one would not be seen: _version() raises for them
+int64_t version_of(const at::Tensor& t) { return (int64_t)t._version(); }
 
 // watch([(dict, key), ...]) -> capsule, or None when a key is missing
 PyObject* py_watch(PyObject*, PyObject* list) {

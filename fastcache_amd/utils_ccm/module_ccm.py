@@ -110,6 +110,9 @@ class _CCMBase(nn.Module):
             self._stacked[group] = ((dtype, device, len(mods)), watch, packed)
         return packed
 
+    def __getstate__(self):          # a copied or pickled module packs its weights anew; a watch belongs to its process
+        return {**self.__dict__, "_stacked": {}}
+
     def _layer_weights(self, group: str, l0: int, l1: int, dtype: torch.dtype, device: torch.device):
         w = self._weights(group, dtype, device)
         return w if (l0, l1) == (0, w[0].shape[0]) else tuple(t[l0:l1] for t in w)

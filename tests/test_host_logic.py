@@ -481,3 +481,27 @@ def test_bench_refuses_graph_workloads_under_the_profiler():
     res = subprocess.run([sys.executable, str(root / "bench.py"), "--workload", "decode-eager"], capture_output=True,
                          text=True, env=env)
     assert res.returncode == 1 and "no GPU" in res.stderr          # passed the fence, stopped at the missing GPU
+
+
+def test_packed_weights_leave_the_module_copyable_and_follow_replaced_parameters():
+    """A compressor that has packed its weights is copied and pickled like one that has not, sees parameters that were
+    written to or replaced, and refuses parameters whose writes cannot be seen (inference tensors)."""
+    import copy
+    import pickle
+    cfg = SimpleNamespace(text_config=SimpleNamespace(num_hidden_layers=2, num_key_value_heads=2, hidden_size=256))
+    module = KVCacheLinearDecoupleCompressor(cfg, compression_factor=2)
+    cpu = torch.device("cpu")
+    pack = lambda m: m._weights("compress_tk", torch.float32, cpu)
+    first = pack(module)
+    assert pack(module) is first
+    for twin in (copy.deepcopy(module), pickle.loads(pickle.dumps(module))):
+        assert torch.equal(pack(twin)[0], first[0]) and pack(twin)[0].data_ptr() != first[0].data_ptr()
+    with torch.no_grad():
+        module.compress_tk[1][0].weight.add_(1)
+    assert torch.equal(pack(module)[0][1], module.compress_tk[1][0].weight)
+    module.compress_tk[0][6].bias = torch.nn.Parameter(torch.full((128,), 3.0))
+    assert bool((pack(module)[5][0] == 3).all())
+    with torch.inference_mode():
+        module.compress_tk[0][6].bias = torch.nn.Parameter(torch.zeros(128))
+    with pytest.raises(RuntimeError, match="version"):
+        pack(module)
