@@ -247,7 +247,13 @@ PyObject* py_ccm_layers(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                               (int32_t)as_int(args[5]), stream_of(k0)),
             "fc_ccm_mlp_layers");
     }
-    std::vector<at::Tensor> parts = all.unbind(0);
+    // plain tensors that share the allocation and nothing else: as autograd's views of one base they could not be written
+    // to with values that require a gradient, and a write to one would count as a write to all
+    std::vector<at::Tensor> parts;
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      parts = all.unbind(0);
+    }
     PyObject* out = PyList_New(L);
     if (!out) throw PyFailed();
     for (Py_ssize_t l = 0; l < L; ++l) {
