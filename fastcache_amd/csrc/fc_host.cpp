@@ -282,6 +282,12 @@ PyObject* pair(at::Tensor a, at::Tensor b) {
   return out;
 }
 
+// Scratch for the kept positions when selection and gather are to be launches of their own, else undefined.
+at::Tensor gather_apart(const at::Tensor& k, int64_t n) {
+  if (!fc_press_gather_apart((int32_t)(k.size(0) * k.size(1)), (int32_t)k.size(2), (int32_t)n)) return at::Tensor();
+  return at::empty({k.size(0), k.size(1), n}, k.options().dtype(at::kInt));
+}
+
 // knorm_into(keys, values, n) -> (k, v) [B, H, n, D], or None
 PyObject* py_knorm_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return guarded([&]() -> PyObject* {
@@ -299,7 +305,10 @@ PyObject* py_knorm_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       scores = at::empty({B, H, S}, k.options().dtype(at::kFloat));
       sp = scores.data_ptr<float>();
     }
-    check(fc_knorm_press_into(&kv, &vv, &dk, &dv, (int32_t)n, sp, (int32_t)S, stream_of(k)), "fc_knorm_press_into");
+    const at::Tensor idx = gather_apart(k, n);
+    check(fc_knorm_press_into(&kv, &vv, &dk, &dv, (int32_t)n, sp, (int32_t)S, idx.defined() ? idx.data_ptr<int32_t>() : nullptr,
+                              stream_of(k)),
+          "fc_knorm_press_into");
     return pair(std::move(ok), std::move(ov));
   });
 }
@@ -332,8 +341,10 @@ PyObject* py_snapkv_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int32_t nsplit = fc_snapkv_select_splits(&kv, (int32_t)hq, (int32_t)W);
     const int64_t bytes = fc_snapkv_select_workspace_bytes(1, (int32_t)B, (int32_t)hq, (int32_t)H, (int32_t)W, (int32_t)S, nsplit);
     at::Tensor ws = at::empty({bytes}, k.options().dtype(at::kByte));
+    const at::Tensor idx = gather_apart(k, n);
     check(fc_snapkv_press_into(&kv, &vv, &dk, &dv, q.const_data_ptr(), lse, (int32_t)hq, (int32_t)W, (int32_t)ksz,
-                               (int32_t)causal, (float)scale, (float)out_scale, (int32_t)n, nsplit, ws.data_ptr(), bytes,
+                               (int32_t)causal, (float)scale, (float)out_scale, (int32_t)n,
+                               idx.defined() ? idx.data_ptr<int32_t>() : nullptr, nsplit, ws.data_ptr(), bytes,
                                stream_of(k)),
           "fc_snapkv_press_into");
     return pair(std::move(ok), std::move(ov));

@@ -975,7 +975,7 @@ static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_
   a.out_mul = out_scale / (float)kernel_size;
   a.indices = indices;
   a.index_stride = index_stride;
-  a.parts = out_k ? fc_gather_parts(keys, k) : 0;
+  a.parts = out_k && !indices ? fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, k) : 0;
   if (nsplit > 1) {
     const float* raw = nullptr;
     if ((rc = snapkv_split_sums(who, keys, queries, lse, num_q_heads, window, kernel_size, causal_window, scale, stride,
@@ -1007,8 +1007,8 @@ extern "C" int fc_snapkv_select(const fc_kv_view* keys, const void* queries, con
 extern "C" int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
                                     const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
                                     int32_t window, int32_t kernel_size, int32_t causal_window, float scale,
-                                    float out_scale, int32_t k, int32_t nsplit, void* workspace, int64_t workspace_bytes,
-                                    void* stream) {
+                                    float out_scale, int32_t k, int32_t* indices, int32_t nsplit, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
   const char* who = "fc_snapkv_press_into";
   int rc;
   for (const fc_kv_view* v : {keys, values, out_k, out_v})
@@ -1020,8 +1020,9 @@ extern "C" int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* va
   FC_REQUIRE(keys->max_seq_len == values->max_seq_len && k <= keys->max_seq_len && k <= out_k->max_seq_len &&
                  k <= out_v->max_seq_len,
              FC_EINVAL, "%s: k=%d exceeds a view's max_seq_len", who, k);
-  return snapkv_select_impl(who, keys, values, out_k, out_v, queries, lse, num_q_heads, window, kernel_size, causal_window,
-                            scale, out_scale, k, nullptr, nullptr, k, nsplit, workspace, workspace_bytes, stream);
+  rc = snapkv_select_impl(who, keys, values, out_k, out_v, queries, lse, num_q_heads, window, kernel_size, causal_window,
+                          scale, out_scale, k, nullptr, indices, k, nsplit, workspace, workspace_bytes, stream);
+  return rc || !indices ? rc : fc_compact(keys, values, out_k, out_v, indices, k, keys->num_kv_heads, k, nullptr, stream);
 }
 
 extern "C" int fc_snapkv_fill_window(float* scores, int32_t score_stride, int32_t num_layers, int32_t batch,

@@ -26,8 +26,7 @@ int fc_column_select(const char* who, int src, const fc_kv_view* keys, const fc_
                      const fc_kv_view* out_v, ColumnSelect a, hipStream_t st);
 
 // workgroups per column for a gather: about two per compute unit in all, no share below 64 rows
-static inline int fc_gather_parts(const fc_kv_view* keys, int k) {
-  const long long cols = (long long)keys->num_layers * keys->batch * keys->num_kv_heads;
+static inline int fc_gather_parts(long long cols, int k) {
   long long p = (512 + cols - 1) / cols;
   if (p > (k + 63) / 64) p = (k + 63) / 64;
   p = p < 1 ? 1 : p > 16 ? 16 : p;

@@ -223,22 +223,36 @@ static int cs_check(const char* who, const fc_kv_view* keys, const fc_kv_view* v
   return FC_OK;
 }
 
+// Whether a press into other tensors should select and gather in launches of their own.  The workgroups that gather a
+// column each select it as well; above 4096 keys that takes 1024 threads, one workgroup to a compute unit, and costs a
+// round for every compute units' worth of them.  us per hook, gather inside -> apart, 30 % dropped: 24 columns of 6000 keys
+// 48 -> 43, 96 of 6000 133 -> 118, of 12000 282 -> 241, 256 of 8000 419 -> 394; 8 of 12000 35 -> 40, 12 of 6000 27 -> 33 (one
+// round); at 4096 keys and less, where two and more share a compute unit, 96 of 4000 76 -> 77, 64 of 2000 29 -> 34.
+extern "C" int fc_press_gather_apart(int32_t columns, int32_t max_seq_len, int32_t k) {
+  if (columns <= 0 || k <= 0) return 0;
+  return max_seq_len > 4096 && (long long)columns * fc_gather_parts(columns, k) > 256;
+}
+
 extern "C" int fc_knorm_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
-                                   const fc_kv_view* out_v, int32_t k, float* scores, int32_t score_stride, void* stream) {
+                                   const fc_kv_view* out_v, int32_t k, float* scores, int32_t score_stride, int32_t* indices,
+                                   void* stream) {
   const char* who = "fc_knorm_press_into";
   int rc = cs_check(who, keys, values, out_k, out_v, k);
   if (rc) return rc;
   if (k == 0 || keys->max_seq_len == 0) return FC_OK;
   ColumnSelect a{};
   a.k = a.index_stride = k;
-  a.parts = fc_gather_parts(keys, k);
+  a.parts = indices ? 0 : fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, k);
+  a.indices = indices;
   if (!scores) {   // the workgroups that gather a column score it as well
     FC_REQUIRE(keys->max_seq_len <= CS_NORMS_MAX, FC_EUNSUPPORTED, "%s: columns of more than %d keys need a score buffer", who,
                CS_NORMS_MAX);
-    return fc_column_select(who, CS_NORMS, keys, values, out_k, out_v, a, (hipStream_t)stream);
+    rc = fc_column_select(who, CS_NORMS, keys, values, out_k, out_v, a, (hipStream_t)stream);
+    return rc || !indices ? rc : fc_compact(keys, values, out_k, out_v, indices, k, keys->num_kv_heads, k, nullptr, stream);
   }
   if ((rc = fc_knorm_score(keys, scores, score_stride, stream))) return rc;
   a.in = scores;
   a.stride = score_stride;
-  return fc_column_select(who, CS_SCORES, keys, values, out_k, out_v, a, (hipStream_t)stream);
+  rc = fc_column_select(who, CS_SCORES, keys, values, out_k, out_v, a, (hipStream_t)stream);
+  return rc || !indices ? rc : fc_compact(keys, values, out_k, out_v, indices, k, keys->num_kv_heads, k, nullptr, stream);
 }

@@ -107,10 +107,14 @@ int fc_knorm_score(const fc_kv_view* keys, float* scores, int32_t score_stride, 
  * tokens of smallest norm per (layer, b, kv head) row, as fc_knorm_score + fc_topk_select + fc_compact give (what
  * kvpress.ScorerPress.compress does per layer inside the attention hook, utils_ccm/utils_compress.py:209-270).  The out
  * views must not overlap the sources.  scores: scratch float[num_layers][batch][num_kv_heads][score_stride], or NULL
- * for max_seq_len <= 4096 (then one launch does all of it).
+ * for max_seq_len <= 4096 (then one launch does all of it).  indices: NULL, or scratch int32[num_layers][batch]
+ * [num_kv_heads][k]; with it the selection is a launch of one workgroup per row and the gather launches of their own.
  */
+/* 1 where fc_knorm_press_into / fc_snapkv_press_into are faster with `indices` */
+int fc_press_gather_apart(int32_t columns, int32_t max_seq_len, int32_t k);
 int fc_knorm_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
-                        const fc_kv_view* out_v, int32_t k, float* scores, int32_t score_stride, void* stream);
+                        const fc_kv_view* out_v, int32_t k, float* scores, int32_t score_stride, int32_t* indices,
+                        void* stream);
 
 /*
  * Head-averaged key norms of the in-tree adapter: mean_norm[l][b][s] = mean_h ||K[l][b][h][s]||_2
@@ -202,7 +206,8 @@ int fc_snapkv_score_split(const fc_kv_view* keys, const void* queries, const flo
  * fc_topk_select give for k > window (up to scored keys that tie exactly with the layer's largest score).  A sequence no
  * longer than the window keeps its first k positions.  At most 36864 tokens per sequence.  nsplit: workgroups per column
  * (fc_snapkv_select_splits picks one); workspace: fc_snapkv_select_workspace_bytes.
- * fc_snapkv_press_into also gathers the kept K and V rows into out_k / out_v, which must not overlap the sources.
+ * fc_snapkv_press_into also gathers the kept K and V rows into out_k / out_v, which must not overlap the sources
+ * (indices: as for fc_knorm_press_into).
  */
 int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q_heads, int32_t window);
 int64_t fc_snapkv_select_workspace_bytes(int32_t num_layers, int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
@@ -214,7 +219,8 @@ int fc_snapkv_select(const fc_kv_view* keys, const void* queries, const float* l
 int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
                          const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
                          int32_t window, int32_t kernel_size, int32_t causal_window, float scale, float out_scale,
-                         int32_t k, int32_t nsplit, void* workspace, int64_t workspace_bytes, void* stream);
+                         int32_t k, int32_t* indices, int32_t nsplit, void* workspace, int64_t workspace_bytes,
+                         void* stream);
 
 /*
  * Sets the window entries scores[l][b][h][S_b-W .. S_b) to the maximum over
