@@ -553,6 +553,32 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
   const int ncols = src->batch * src->num_kv_heads;
   int wpc = 1;
   while (wpc < ML_WAVES && (int64_t)ncols * wpc / ML_WAVES * src->num_layers < 1024 && ML_ROWS * wpc * 2 <= c) wpc *= 2;
+  if (cf > 2 && !rag && ml_compute_units() > 0) {
+    // With streamed W1 a workgroup takes one column group, and what counts is rounds of workgroups times iterations of
+    // each (and about 0.4 of one to start).  The launch is bound by memory: four fifths of the compute units keep it
+    // as busy as all of them, so a last round that is not full costs what it holds, but no less than 0.8.  Of equal
+    // splits the one with fewer wavefronts per column, which wait for each other at every store.  us per pass on 28
+    // layers of 4 heads, as many wavefronts as make 1024 workgroups -> this rule: 16 sequences of 700 tokens 424 -> 320, of
+    // 3000 1051 -> 940, of 16384 4331 -> 4271, 8 of 8000 1330 -> 1205, 3 of 3000 313 -> 268.  Sequences of different
+    // lengths stay with the many small workgroups: the longest one would decide (5 of 2666 to 8000 794 -> 961).
+    const int64_t ncu = ml_compute_units();
+    const auto tables_fit = [&](const fc_kv_view* v, int64_t last, int cpw) {     // in LDS, else every row waits for its entry
+      return !v->block_tables || v->block_size <= 0 || last / v->block_size < ML_TBLTOT / cpw;
+    };
+    double best = -1.0;
+    for (int w = 1; w <= ML_WAVES && (w == 1 || ML_ROWS * w < 2 * c); w *= 2) {
+      const int cpw = ML_WAVES / w;
+      if (!tables_fit(src, (int64_t)seg_start + (int64_t)c * cf - 1, cpw) || !tables_fit(dst, (int64_t)dst_start + c - 1, cpw)) continue;
+      const int64_t wgs = (int64_t)((ncols + cpw - 1) / cpw) * src->num_layers, left = wgs % ncu;
+      const double part = (double)left / (double)ncu;
+      const double rounds = (double)(wgs / ncu) + (left == 0 ? 0.0 : part > 0.8 ? part : 0.8);
+      const double cost = rounds * ((c + ML_ROWS * w - 1) / (ML_ROWS * w) + 0.4);
+      if (best < 0 || cost < best) {
+        best = cost;
+        wpc = w;
+      }
+    }
+  }
   const int cols_per_wg = ML_WAVES / wpc;
   // One workgroup occupies a compute unit (its LDS), and loading the weights costs it a few microseconds.
   // When a column group is short work, let each workgroup walk several groups of its layer; pick the number

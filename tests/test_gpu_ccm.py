@@ -262,3 +262,28 @@ def test_ccm_forward_results_are_separate_tensors(dev):
     k0.mul_(scale)
     assert k0.requires_grad and (v0._version, k1._version) == versions
     assert all(torch.equal(a, b) for a, b in zip(before, (v0, k1)))
+
+
+@pytest.mark.parametrize("L,B,S,block_size", [
+    (28, 16, 700, 256),      # a wavefront per column
+    (28, 8, 703, 256),       # two
+    (28, 4, 700, 256),       # four
+    (28, 16, 3200, 32),      # block tables of 100 pages: not for a wavefront per column
+    (29, 9, 26, 256),        # last column group partly empty, five rows a column
+])
+def test_ccm_mlp_is_the_same_however_columns_are_split(dev, L, B, S, block_size):
+    """A batch through the MLP in place, and each of its sequences alone (whose columns are split over more wavefronts):
+    the same bytes everywhere, since a row's arithmetic does not depend on the split."""
+    H, cf = 4, 5
+    per = -(-S // block_size)
+    pool = torch.empty((L, B * per + 1, block_size, H, 128), dtype=torch.bfloat16, device=dev).normal_()
+    tables = torch.randperm(B * per + 1, device=dev)[:B * per].view(B, per).int().contiguous()
+    w = tuple((torch.randn(shape, device=dev) * 0.05).bfloat16()
+              for shape in ((L, 128, 128 * cf), (L, 128), (L, 128, 128), (L, 128), (L, 128, 128), (L, 128)))
+    alone = pool.clone()
+    view = _lib.paged_view(pool, tables, None, S)
+    ops.ccm_mlp(view, view, w, cf, 0, S, 0)
+    for b in range(B):
+        one = _lib.paged_view(alone, tables[b:b + 1], None, S)
+        ops.ccm_mlp(one, one, w, cf, 0, S, 0)
+    assert torch.equal(pool.view(torch.int16), alone.view(torch.int16))
