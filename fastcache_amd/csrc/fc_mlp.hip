@@ -546,60 +546,75 @@ static int ml_check(const char* who, const fc_kv_view* src, const fc_kv_view* ds
 
 // The MLP launch for c > 0 rows per column: c rows for every sequence from (seg_start, dst_start), or, with the
 // three arrays, every sequence's own segment with at most c rows.
+// How many wavefronts share a column, and how many workgroups of a (layer, plane) walk its column groups.  One workgroup
+// fills a compute unit (its LDS), so what counts is rounds of workgroups times iterations of each, plus the start: loading
+// the weights, about 0.4 of an iteration, 0.7 with resident W1 (whose workgroups may walk several groups for one start).  The
+// launch is bound by memory: with streamed W1 four fifths of the compute units keep it as busy as all of them, so a last
+// round that is not full costs what it holds, but no less than 0.8 (with resident W1, whose workgroups do not wait for each
+// other's chunks, a whole round: 45 sequences of 640 tokens in 15 walks a layer instead of 8 took 2 % longer).  Of equal splits the one with fewer wavefronts per column, which wait for
+// each other at every store.  us per pass, as many wavefronts as make 1024 workgroups -> this split: 28 layers of 4
+// heads, factor 5, 16 sequences of 700 tokens 424 -> 323, of 3000 1051 -> 935, of 16384 4331 -> 4223, 8 of 8000
+// 1326 -> 1191, 3 of 3000 313 -> 266; factor 2, 16 of 700 428 -> 314, 8 of 700 246 -> 205; 32 layers of 32 heads,
+// factor 2, 1 of 1100 442 -> 319, 2 of 640 416 -> 325, 4 of 1500 1299 -> 1210, 12 and more the same.
+struct MlSplit { int wpc, gx; };
+template <typename Fits>
+static MlSplit ml_split(int ncols, int jobs, int c, int cf, Fits fits) {
+  const int64_t ncu = ml_compute_units() > 0 ? ml_compute_units() : 256;
+  const double least = cf <= 2 ? 1.0 : 0.8;
+  MlSplit best{ML_WAVES, ncols};      // what is left when no split fits
+  double best_cost = -1.0;
+  for (int wpc = 1; wpc <= ML_WAVES && (wpc == 1 || ML_ROWS * wpc < 2 * c); wpc *= 2) {
+    if (!fits(wpc)) continue;
+    const int cpw = ML_WAVES / wpc, groups = (ncols + cpw - 1) / cpw, iters = (c + ML_ROWS * wpc - 1) / (ML_ROWS * wpc);
+    for (int per = 1; per <= groups && per <= (cf <= 2 ? 64 : 1); ++per) {
+      const int g = (groups + per - 1) / per;
+      const int64_t wgs = (int64_t)g * jobs, left = wgs % ncu;
+      const double part = (double)left / (double)ncu;
+      const double rounds = (double)(wgs / ncu) + (left == 0 ? 0.0 : part > least ? part : least);
+      const double cost = rounds * ((double)((groups + g - 1) / g) * iters + (cf <= 2 ? 0.7 : 0.4));
+      if (best_cost < 0 || cost < best_cost) {
+        best_cost = cost;
+        best = {wpc, g};
+      }
+    }
+  }
+  return best;
+}
+
 static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weights* w, int cf,
                      int seg_start, int c, int dst_start, const int32_t* seg_start_v, const int32_t* seg_len_v,
                      const int32_t* dst_start_v, int min_rows, hipStream_t st) {
   const bool rag = seg_len_v != nullptr;
   const int ncols = src->batch * src->num_kv_heads;
-  int wpc = 1;
-  while (wpc < ML_WAVES && (int64_t)ncols * wpc / ML_WAVES * src->num_layers < 1024 && ML_ROWS * wpc * 2 <= c) wpc *= 2;
-  if (cf > 2 && !rag && ml_compute_units() > 0) {
-    // With streamed W1 a workgroup takes one column group, and what counts is rounds of workgroups times iterations of
-    // each (and about 0.4 of one to start).  The launch is bound by memory: four fifths of the compute units keep it
-    // as busy as all of them, so a last round that is not full costs what it holds, but no less than 0.8.  Of equal
-    // splits the one with fewer wavefronts per column, which wait for each other at every store.  us per pass on 28
-    // layers of 4 heads, as many wavefronts as make 1024 workgroups -> this rule: 16 sequences of 700 tokens 424 -> 320, of
-    // 3000 1051 -> 940, of 16384 4331 -> 4271, 8 of 8000 1330 -> 1205, 3 of 3000 313 -> 268.  Sequences of different
-    // lengths stay with the many small workgroups: the longest one would decide (5 of 2666 to 8000 794 -> 961).
-    const int64_t ncu = ml_compute_units();
-    const auto tables_fit = [&](const fc_kv_view* v, int64_t last, int cpw) {     // in LDS, else every row waits for its entry
-      return !v->block_tables || v->block_size <= 0 || last / v->block_size < ML_TBLTOT / cpw;
+  int wpc = 1, gx = 0;
+  if (!rag) {
+    const auto tables_fit = [&](int wpc_) {     // in LDS, else every row waits for its entry
+      const int cap = ML_TBLTOT / (ML_WAVES / wpc_);
+      const auto fit = [&](const fc_kv_view* v, int64_t last) { return !v->block_tables || v->block_size <= 0 || last / v->block_size < cap; };
+      return fit(src, (int64_t)seg_start + (int64_t)c * cf - 1) && fit(dst, (int64_t)dst_start + c - 1);
     };
+    const MlSplit sp = ml_split(ncols, src->num_layers, c, cf, tables_fit);
+    wpc = sp.wpc;
+    gx = sp.gx;
+  } else {
+    // Sequences of different lengths: many small workgroups, or the longest sequence would decide (5 of 2666 to 8000
+    // tokens: 794 us per pass, 961 with the split by the largest row count).
+    while (wpc < ML_WAVES && (int64_t)ncols * wpc / ML_WAVES * src->num_layers < 1024 && ML_ROWS * wpc * 2 <= c) wpc *= 2;
+    const int groups = (ncols * wpc + ML_WAVES - 1) / ML_WAVES, ncu = ml_compute_units();
+    const double t_group = 1.5 * ((c + ML_ROWS * wpc - 1) / (ML_ROWS * wpc)) * (cf + 2), t_start = 4.0;   // microseconds, roughly
+    gx = groups;
     double best = -1.0;
-    for (int w = 1; w <= ML_WAVES && (w == 1 || ML_ROWS * w < 2 * c); w *= 2) {
-      const int cpw = ML_WAVES / w;
-      if (!tables_fit(src, (int64_t)seg_start + (int64_t)c * cf - 1, cpw) || !tables_fit(dst, (int64_t)dst_start + c - 1, cpw)) continue;
-      const int64_t wgs = (int64_t)((ncols + cpw - 1) / cpw) * src->num_layers, left = wgs % ncu;
-      const double part = (double)left / (double)ncu;
-      const double rounds = (double)(wgs / ncu) + (left == 0 ? 0.0 : part > 0.8 ? part : 0.8);
-      const double cost = rounds * ((c + ML_ROWS * w - 1) / (ML_ROWS * w) + 0.4);
-      if (best < 0 || cost < best) {
-        best = cost;
-        wpc = w;
-      }
-    }
-  }
-  const int cols_per_wg = ML_WAVES / wpc;
-  // One workgroup occupies a compute unit (its LDS), and loading the weights costs it a few microseconds.
-  // When a column group is short work, let each workgroup walk several groups of its layer; pick the number
-  // per workgroup that minimises rounds * (groups * time per group + start-up) in a coarse model.
-  const int ncg = (ncols + cols_per_wg - 1) / cols_per_wg;
-  int gx = ncg;
-  {
-    const int ncu = ml_compute_units();
-    const int n_iter = (c + ML_ROWS * wpc - 1) / (ML_ROWS * wpc);
-    const double t_group = 1.5 * n_iter * (cf + 2), t_start = 4.0;   // microseconds, roughly
-    double best = -1.0;
-    for (int per = 1; cf <= 2 && ncu > 0 && per <= ncg && per <= 64; ++per) {
-      const int g = (ncg + per - 1) / per;
+    for (int per = 1; cf <= 2 && ncu > 0 && per <= groups && per <= 64; ++per) {
+      const int g = (groups + per - 1) / per;
       const long long rounds = ((long long)g * src->num_layers + ncu - 1) / ncu;
-      const double cost = (double)rounds * (((ncg + g - 1) / g) * t_group + t_start);
+      const double cost = (double)rounds * (((groups + g - 1) / g) * t_group + t_start);
       if (best < 0 || cost < best) {
         best = cost;
         gx = g;
       }
     }
   }
+  const int cols_per_wg = ML_WAVES / wpc, ncg = (ncols + cols_per_wg - 1) / cols_per_wg;
   dim3 grid(gx, src->num_layers);
   const size_t lds = ML_LDS;
   KvView s = fc_make_view(src), d = fc_make_view(dst);
@@ -739,7 +754,8 @@ extern "C" int fc_ccm_mlp_layers(const void* const* k_layers, const void* const*
       for (int i = 0; i < 6; ++i) a.w[s][p][i] = (const char*)ws[i];
     }
     // How many wavefronts share a column and how many column groups a workgroup walks: the pair with the fewest
-    // rounds * (groups * time per group + start-up), the same coarse model as the single launch's.
+    // rounds * (groups * time per group + start-up).  (With the last round counted as in ml_split: 0.92 to 1.03 times as
+    // fast, on the whole slower; the two segments share the launch, so a round of one is filled up by the other.)
     const int ncu = ml_compute_units() > 0 ? ml_compute_units() : 256;
     double best = -1.0;
     a.wpc[s] = 1;

@@ -264,17 +264,21 @@ def test_ccm_forward_results_are_separate_tensors(dev):
     assert all(torch.equal(a, b) for a, b in zip(before, (v0, k1)))
 
 
-@pytest.mark.parametrize("L,B,S,block_size", [
-    (28, 16, 700, 256),      # a wavefront per column
-    (28, 8, 703, 256),       # two
-    (28, 4, 700, 256),       # four
-    (28, 16, 3200, 32),      # block tables of 100 pages: not for a wavefront per column
-    (29, 9, 26, 256),        # last column group partly empty, five rows a column
+@pytest.mark.parametrize("L,B,S,block_size,cf", [
+    (28, 16, 700, 256, 5),      # a wavefront per column
+    (28, 8, 703, 256, 5),       # two
+    (28, 4, 700, 256, 5),       # four
+    (28, 16, 3200, 32, 5),      # block tables of 100 pages: not for a wavefront per column
+    (1, 2, 25000, 32, 5),       # of 782 pages: for no split
+    (29, 9, 26, 256, 5),        # last column group partly empty, five rows a column
+    (28, 21, 703, 256, 2),      # resident W1, several column groups to a workgroup
+    (28, 3, 700, 256, 2),
+    (28, 5, 90, 256, 1),
 ])
-def test_ccm_mlp_is_the_same_however_columns_are_split(dev, L, B, S, block_size):
+def test_ccm_mlp_is_the_same_however_columns_are_split(dev, L, B, S, block_size, cf):
     """A batch through the MLP in place, and each of its sequences alone (whose columns are split over more wavefronts):
     the same bytes everywhere, since a row's arithmetic does not depend on the split."""
-    H, cf = 4, 5
+    H = 4
     per = -(-S // block_size)
     pool = torch.empty((L, B * per + 1, block_size, H, 128), dtype=torch.bfloat16, device=dev).normal_()
     tables = torch.randperm(B * per + 1, device=dev)[:B * per].view(B, per).int().contiguous()
