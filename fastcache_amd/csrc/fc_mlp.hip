@@ -544,18 +544,17 @@ static int ml_check(const char* who, const fc_kv_view* src, const fc_kv_view* ds
   return FC_OK;
 }
 
-// The MLP launch for c > 0 rows per column: c rows for every sequence from (seg_start, dst_start), or, with the
-// three arrays, every sequence's own segment with at most c rows.
-// How many wavefronts share a column, and how many workgroups of a (layer, plane) walk its column groups.  One workgroup
-// fills a compute unit (its LDS), so what counts is rounds of workgroups times iterations of each, plus the start: loading
-// the weights, about 0.4 of an iteration, 0.7 with resident W1 (whose workgroups may walk several groups for one start).  The
-// launch is bound by memory: with streamed W1 four fifths of the compute units keep it as busy as all of them, so a last
-// round that is not full costs what it holds, but no less than 0.8 (with resident W1, whose workgroups do not wait for each
-// other's chunks, a whole round: 45 sequences of 640 tokens in 15 walks a layer instead of 8 took 2 % longer).  Of equal splits the one with fewer wavefronts per column, which wait for
-// each other at every store.  us per pass, as many wavefronts as make 1024 workgroups -> this split: 28 layers of 4
-// heads, factor 5, 16 sequences of 700 tokens 424 -> 323, of 3000 1051 -> 935, of 16384 4331 -> 4223, 8 of 8000
-// 1326 -> 1191, 3 of 3000 313 -> 266; factor 2, 16 of 700 428 -> 314, 8 of 700 246 -> 205; 32 layers of 32 heads,
-// factor 2, 1 of 1100 442 -> 319, 2 of 640 416 -> 325, 4 of 1500 1299 -> 1210, 12 and more the same.
+// How many wavefronts share a column, and how many workgroups of a (layer, plane) walk its column groups.  One
+// workgroup fills a compute unit (its LDS), so what counts is rounds of workgroups times iterations of each, plus the
+// start: loading the weights, about 0.4 of an iteration, 0.7 with resident W1 (whose workgroups may walk several groups
+// for one start).  The launch is bound by memory: with streamed W1 four fifths of the compute units keep it as busy as
+// all of them, so a last round that is not full costs what it holds, but no less than 0.8 (with resident W1, whose
+// workgroups do not wait for each other's chunks, a whole round: 45 sequences of 640 tokens in 15 walks a layer instead
+// of 8 took 2 % longer).  Of equal splits the one with fewer wavefronts per column, which wait for each other at every
+// store.  us per pass, as many wavefronts as make 1024 workgroups -> this split: 28 layers of 4 heads, factor 5,
+// 16 sequences of 700 tokens 424 -> 323, of 3000 1051 -> 935, of 16384 4331 -> 4223, 8 of 8000 1326 -> 1191, 3 of 3000
+// 313 -> 266; factor 2, 16 of 700 428 -> 314, 8 of 700 246 -> 205; 32 layers of 32 heads, factor 2, 1 of 1100
+// 442 -> 319, 2 of 640 416 -> 325, 4 of 1500 1299 -> 1210, 12 and more the same.
 struct MlSplit { int wpc, gx; };
 template <typename Fits>
 static MlSplit ml_split(int ncols, int jobs, int c, int cf, Fits fits) {
@@ -581,6 +580,8 @@ static MlSplit ml_split(int ncols, int jobs, int c, int cf, Fits fits) {
   return best;
 }
 
+// The MLP launch for c > 0 rows per column: c rows for every sequence from (seg_start, dst_start), or, with the
+// three arrays, every sequence's own segment with at most c rows.
 static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weights* w, int cf,
                      int seg_start, int c, int dst_start, const int32_t* seg_start_v, const int32_t* seg_len_v,
                      const int32_t* dst_start_v, int min_rows, hipStream_t st) {
