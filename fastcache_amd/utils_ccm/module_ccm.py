@@ -94,15 +94,17 @@ class _CCMBase(nn.Module):
         if hit is not None and hit[0] == (dtype, device, len(mods)) and host.unchanged(hit[1]):
             return hit[2]
         with torch.no_grad():
+            linear = [(m[0], m[3], m[6]) for m in mods]
             packed = tuple(
-                torch.stack([getattr(m[i], name).detach() for m in mods]).to(device=device, dtype=dtype).contiguous()
-                for i in (0, 3, 6) for name in ("weight", "bias"))
+                torch.stack([getattr(three[i], name) for three in linear]).to(device=device, dtype=dtype).contiguous()
+                for i in range(3) for name in ("weight", "bias"))
         steps = [(self._modules, group)]
         for i, m in mods._modules.items():
             steps.append((mods._modules, i))
+            inner = m._modules
             for j in ("0", "3", "6"):
-                steps.append((m._modules, j))
-                steps += [(m._modules[j]._parameters, name) for name in ("weight", "bias")]
+                params = inner[j]._parameters
+                steps += [(inner, j), (params, "weight"), (params, "bias")]
         watch = host.watch(steps)
         if watch is None:              # a parametrized Linear computes its weight on each access: nothing to hold on to
             self._stacked.pop(group, None)
