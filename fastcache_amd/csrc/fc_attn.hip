@@ -506,7 +506,8 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   }
   int len = __builtin_amdgcn_readfirstlane(lens[b]);
   len = max(min(len, kc.max_seq_len), 0);
-  const int slot = ap.k_new ? __builtin_amdgcn_readfirstlane(ap.slots[b]) : -1;
+  const int nb = (int)gridDim.y;
+  int slot = PAGED && ap.k_new && lane < nb ? ap.slots[lane] : -1;   // the new rows' slots, 64 sequences at a time
   const int t0 = (int)blockIdx.z * chunk;
   if (t0 >= len && blockIdx.z != 0) return;
   const int end = min(len, t0 + chunk);
@@ -520,19 +521,37 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   }
   const char* kbase = kc.base + ((long long)layer * kc.stride_layer + (long long)h * kc.stride_head) * 2;
   const char* vbase = vc.base + ((long long)layer * vc.stride_layer + (long long)h * vc.stride_head) * 2;
-  if (PAGED && slot >= 0) {
-    // The new row is written by the workgroup whose range it lies in, which then has to see it land before it reads
-    // it back, and by the last one of the sequence (it usually lies right behind the range; writing it twice is harmless).
-    const int page = slot >> kc.block_shift, at = slot & (kc.block_size - 1);
-    const int pos = (lane << kc.block_shift) + at;
-    const bool inside = __ballot(ktbl == page && pos >= t0 && pos < end && lane < kc.table_stride) != 0ull;
-    if ((inside || end == len) && tid < 32) {
-      const bool is_v = tid >= 16;
-      const long long koff = (long long)page * kc.stride_block + (long long)at * kc.stride_token;
-      const long long voff = (long long)page * vc.stride_block + (long long)at * vc.stride_token;
-      char* dst = is_v ? const_cast<char*>(vbase) + voff * 2 : const_cast<char*>(kbase) + koff * 2;
-      const char* src = is_v ? ap.v_new + (long long)b * ap.v_stride : ap.k_new + (long long)b * ap.k_stride;
-      *reinterpret_cast<uint4*>(dst + l15 * 16) = *reinterpret_cast<const uint4*>(src + (long long)h * FC_HEAD_DIM * 2 + l15 * 16);
+  if (PAGED && ap.k_new) {
+    // A new row inside this workgroup's range is written by this workgroup, which then has to see it land before it reads
+    // it back, whichever sequence of the batch it belongs to (a table may be listed twice with lengths one apart, or a page
+    // be shared): nobody depends on another workgroup's write.  The sequence's own row is also written by its last
+    // workgroup, since it usually lies right behind the range.  Workgroups that write one row write the same bytes.
+    const int e0 = t0 >> kc.block_shift, e1 = (end - 1) >> kc.block_shift;      // pages of the range (none: e1 < e0)
+    bool inside = false;
+    for (int j0 = 0; j0 < nb; j0 += FC_WAVE) {
+      if (j0 > 0) slot = j0 + lane < nb ? ap.slots[j0 + lane] : -1;
+      const int page = slot >> kc.block_shift, at = slot & (kc.block_size - 1);
+      bool hit = false;
+      for (int e = e0; e <= e1; ++e) {
+        const int pos = (e << kc.block_shift) + at;
+        hit |= slot >= 0 && page == __builtin_amdgcn_readlane(ktbl, e) && pos >= t0 && pos < end;
+      }
+      unsigned long long todo = __ballot(hit);
+      inside |= todo != 0ull;
+      if (end == len) todo |= __ballot(slot >= 0 && j0 + lane == b);
+      while (todo) {                                                            // wave-uniform
+        const int j = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const int row = __builtin_amdgcn_readlane(slot, j);
+        const long long rpage = row >> kc.block_shift, rat = row & (kc.block_size - 1);
+        if (tid < 32) {
+          const bool is_v = tid >= 16;
+          const long long koff = rpage * kc.stride_block + rat * kc.stride_token, voff = rpage * vc.stride_block + rat * vc.stride_token;
+          char* dst = is_v ? const_cast<char*>(vbase) + voff * 2 : const_cast<char*>(kbase) + koff * 2;
+          const char* src = is_v ? ap.v_new + (j0 + j) * ap.v_stride : ap.k_new + (j0 + j) * ap.k_stride;
+          *reinterpret_cast<uint4*>(dst + l15 * 16) = *reinterpret_cast<const uint4*>(src + (long long)h * FC_HEAD_DIM * 2 + l15 * 16);
+        }
+      }
     }
     if (inside) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

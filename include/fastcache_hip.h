@@ -530,10 +530,10 @@ int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t
 /*
  * Append and attention of one layer of a decode step (nanovllm/layers/attention.py:62-79): row i of k_new / v_new
  * ([batch][num_kv_heads][head_dim], `*_stride` elements between sequences) goes to cache slot slot_mapping[i]
- * (negative: skipped), then query i attends the first context_lens[i] tokens of sequence i.  The caches are one layer,
- * paged, with contiguous tokens; slot_mapping[i] is a token of sequence i.  `workspace` may be NULL when
- * fc_decode_layer_workspace_bytes returns 0 (the appending is then part of the attention's launch), otherwise it
- * holds that many bytes.
+ * (negative: skipped), then query i attends the first context_lens[i] tokens of sequence i.  Every new row is in the
+ * cache before any query reads it, also a row in a page that several sequences of the batch read.  The caches are one
+ * layer, paged, with contiguous tokens.  `workspace` may be NULL when fc_decode_layer_workspace_bytes returns 0 (the
+ * appending is then part of the attention's launch), otherwise it holds that many bytes.
  */
 int64_t fc_decode_layer_workspace_bytes(const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t num_q_heads);
 int fc_decode_layer(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,

@@ -320,3 +320,43 @@ def test_keys_of_infinite_distance_weigh_nothing(dev, dtype, lens, max_pages):
     on_gpu = pool.to(dev)
     got = decode_attention(q.to(dev), on_gpu[0], on_gpu[1], lens_t.to(dev), tables.to(dev), 128 ** -0.5).cpu()
     assert float((got.float() - ref.float()).abs().max()) < 4e-3      # as for finite keys above
+
+
+@pytest.mark.parametrize("copies,lens,block_size", [
+    (3, [300, 40], 256),            # one workgroup a column
+    (2, [254, 700], 256),           # several; the second copy's row is the first of a page
+    (5, [30, 64, 255], 32),
+    (35, [260, 90], 64),            # more sequences than a wavefront has lanes
+])
+def test_new_rows_are_seen_by_every_sequence_that_reads_their_page(dev, copies, lens, block_size):
+    """The same table listed several times with lengths one apart: several tokens of one sequence in one step, each
+    attending the rows of those before it, which other rows of the batch append (attention.py:62-79 stores all rows
+    before any sequence is attended)."""
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    dtype, Hq, Hkv = torch.bfloat16, 2, 1
+    case = synth.make_paged_case(seed=41, num_layers=1, batch=len(lens), num_kv_heads=Hkv, seq_lens=[n + copies for n in lens],
+                                 dtype=dtype, block_size=block_size)
+    rows = [(s, j) for j in range(copies) for s in range(len(lens))]        # copies of a sequence far apart in the batch
+    B = len(rows)
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(B, h * 128, generator=g).to(dtype) for h in (Hq, Hkv, Hkv))
+    tables = case.table_tensor("cpu")[[s for s, _ in rows]].contiguous()
+    lens_t = torch.tensor([lens[s] + j + 1 for s, j in rows], dtype=torch.int32)
+    pos = [lens[s] + j for s, j in rows]
+    slots = torch.tensor([case.block_tables[s][p // block_size] * block_size + p % block_size for (s, _), p in zip(rows, pos)],
+                         dtype=torch.int32)
+    pool = case.kv_cache[:, 0].clone()
+    for p, new in ((0, k), (1, v)):
+        pool[p].view(-1, Hkv, 128)[slots.long()] = new.view(B, Hkv, 128)
+    ref = oattn.decode_attention(q.view(B, Hq, 128), pool[0], pool[1], lens_t, tables, 128 ** -0.5)
+    layer = Attention(Hq, 128, 128 ** -0.5, Hkv)
+    on_gpu = case.kv_cache[:, 0].to(dev)
+    layer.k_cache, layer.v_cache = on_gpu[0], on_gpu[1]
+    set_context(False, slot_mapping=slots.to(dev), context_lens=lens_t.to(dev), block_tables=tables.to(dev))
+    try:
+        got = layer(q.to(dev), k.to(dev), v.to(dev)).cpu().view(B, Hq, 128)
+    finally:
+        reset_context()
+    assert torch.equal(on_gpu.cpu(), pool)
+    assert float((got.float() - ref.float()).abs().max()) < 4e-3      # as above
