@@ -430,7 +430,13 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 //   O^T[dim][head] = V^T P^T: the probabilities are already the B operand (keys in the order the accumulator gives
 //                           them); V goes through the wavefront's 8 KB of LDS and is read transposed, 2 bytes at a time.
 // Probabilities enter as a sum of 16-bit operands in the cache dtype: two (as the split kernel does for 5 to 8 heads), or
-// three for bf16 groups of up to 4 heads, where the split kernel multiplies in fp32.
+// three for bf16 groups of up to 4 heads, where the split kernel multiplies in fp32.  Two fp16 operands hold 22 bits, but
+// only down to 2^-3: below, the second one runs into fp16's subnormal step (2^-24), and a probability under 2^-25 would
+// count in the sum and not in the output.  fp16 probabilities are therefore scaled by 2^14 (exactly; 1 stays below the
+// largest fp16 value) and the partial output back: what the operands drop is below 2^-39 of the tile's largest weight.
+// Error of the unrounded output against 64 bits, 3 contexts of up to 2040 keys, 1 / 2 / 4 fp16 heads a group, this kernel
+// and the split kernel in fp32: flat 1.08 / 1.09 / 1.08e-7 and 1.12 / 1.09 / 1.12e-7, peaked 8.5 / 9.4 / 9.8e-8 and
+// 8.3 / 8.9 / 9.1e-8 (a third operand leaves the latter as they are); per layer 8.34 us before and after.
 #define DC_WAVES 8
 #define DC_THREADS (DC_WAVES * 64)
 #define DC_HEADS 16
@@ -439,6 +445,7 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 #define DC_STAGE (DA_TILE * DC_VROW)
 #define DC_PART (DC_WAVES * DC_STAGE)                              // V stages, then the partial outputs
 #define DC_LDS (DC_PART + DC_WAVES * DC_HEADS * 8)
+#define DC_P_SCALE(DT) ((DT) == FC_F16 ? 16384.f : 1.f)
 static_assert(DC_PART >= DC_WAVES * DC_HEADS * DC_PSTRIDE * 4, "the partial outputs share the V stages' memory");
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -642,6 +649,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     for (int e = 0; e < 8; ++e) {
       p[e] = __builtin_amdgcn_exp2f(p[e] - ref);
       sum += p[e];
+      p[e] *= DC_P_SCALE(DTYPE);
     }
     l = fmaf(l, alpha, sum);
     uint4 pt[TERMS];
@@ -695,7 +703,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   for (int w = 0; w < DC_WAVES; ++w) M = fmaxf(M, ml[w * DC_HEADS + l15].x);
   float* part = reinterpret_cast<float*>(smem);
   {
-    const float wgt = __builtin_amdgcn_exp2f(m - (M == -INFINITY ? 0.f : M));   // 0 for a wavefront without tiles
+    const float wgt = __builtin_amdgcn_exp2f(m - (M == -INFINITY ? 0.f : M)) * (1.f / DC_P_SCALE(DTYPE));   // 0 for a wavefront without tiles
     if (l15 < ng) {
 #pragma unroll
       for (int db = 0; db < 8; ++db)

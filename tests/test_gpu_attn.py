@@ -360,3 +360,34 @@ def test_new_rows_are_seen_by_every_sequence_that_reads_their_page(dev, copies, 
         reset_context()
     assert torch.equal(on_gpu.cpu(), pool)
     assert float((got.float() - ref.float()).abs().max()) < 4e-3      # as above
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(2, 2), (4, 2), (8, 2), (14, 2)])
+@pytest.mark.parametrize("lens", [[64, 250], [700, 300]])                    # one workgroup a column; several
+@pytest.mark.parametrize("below", [12, 20, 26])
+def test_small_fp16_probabilities_keep_their_bits(dev, Hq, Hkv, lens, below):
+    """Of every 32 keys one has the largest logit and a value of zero, the others 2^-below of its weight: the output is what
+    those add, and its error stays within the output's own rounding (2^-11 of an element) and 2^-13 for the logits in
+    fp32 (26 times 2^-24 and an exponential: below 2^-18 of a weight; the sum over equal weights adds no more).  An fp16
+    operand with its subnormal step of 2^-24 has no bits left for such weights."""
+    from fastcache_amd.layers.attention import decode_attention
+    dtype, B, scale = torch.float16, len(lens), 128 ** -0.5
+    case = synth.make_paged_case(seed=6, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=lens, dtype=dtype)
+    pool, tables = case.kv_cache[:, 0].clone(), case.table_tensor("cpu")
+    g = torch.Generator().manual_seed(8)
+    pool[0] = 0
+    pool[0, ..., 0] = -below * 0.6931471805599453 / scale / 16                # the query's first element is 16
+    pool[1] = (512 + 512 * torch.rand(pool[1].shape, generator=g)).to(dtype)
+    for at in range(0, 256, 32):
+        pool[:, :, at] = 0
+    q = torch.zeros(B, Hq, 128, dtype=dtype)
+    q[..., 0] = 16
+    on_gpu, lens_t = pool.to(dev), torch.tensor(lens, dtype=torch.int32)
+    got = decode_attention(q.to(dev), on_gpu[0], on_gpu[1], lens_t.to(dev), tables.to(dev), scale).cpu().double()
+    for b, n in enumerate(lens):
+        pages = tables[b, :(n + 255) // 256].long()
+        k, v = (pool[p, pages].reshape(-1, Hkv, 128)[:n].double().repeat_interleave(Hq // Hkv, 1) for p in range(2))
+        w = torch.softmax(torch.einsum("hd,nhd->hn", q[b].double(), k) * scale, dim=-1)
+        ref = torch.einsum("hn,nhd->hd", w, v)
+        # 2^-25: half of fp16's smallest step, for outputs below its normal range
+        assert bool(((got[b] - ref).abs() <= (2.0 ** -11 + 2.0 ** -13) * ref.abs() + 2.0 ** -25).all())
