@@ -45,6 +45,10 @@ __device__ __forceinline__ unsigned short da_pack(float f) {
 
 
 #define DA_PV_MFMA_MIN 8               // heads per workgroup from which p * V runs on the matrix pipe (measured: no gain below)
+// What probabilities are multiplied with before they become 16-bit operands, and outputs divided by: fp16's exponent ends at
+// 2^-14 (subnormal step 2^-24), so of a probability p <= 1 as hi + lo the second half would lose bits from 2^-3 down, and
+// all of p below 2^-25, which still counts in the sum.  A power of two: exact, and 1 stays below fp16's largest value.
+#define DA_P_SCALE(DT) ((DT) == FC_F16 ? 16384.f : 1.f)
 #define DA_TILE 32                     // keys per tile: one MFMA block, 8 KB of K or V rows
 // The chunk's block-table entries are prefetched one per lane of a wavefront: the largest chunk in the smallest
 // page the fast path takes (32 tokens, block_shift >= 5), starting anywhere in a page, must span at most 64 entries.
@@ -235,9 +239,10 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
       const float p = __builtin_amdgcn_exp2f(x[j] - m);   // exp2(-inf) = 0 for the padded slots
       if (lane + 64 * j < live_tiles * DA_TILE) {         // every slot of a live tile is read by phase 3
         if constexpr (PV_MFMA) {
-          const unsigned short hi = da_pack<DTYPE>(p);
+          const float ps = p * DA_P_SCALE(DTYPE);
+          const unsigned short hi = da_pack<DTYPE>(ps);
           const float hf = DTYPE == FC_BF16 ? fc_bf16_to_float(hi) : fc_half_to_float(hi);
-          p2[g * chunk + lane + 64 * j] = (unsigned)hi | ((unsigned)da_pack<DTYPE>(p - hf) << 16);
+          p2[g * chunk + lane + 64 * j] = (unsigned)hi | ((unsigned)da_pack<DTYPE>(ps - hf) << 16);
         } else {
           sc[g * chunk + lane + 64 * j] = p;
         }
@@ -317,7 +322,7 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
     for (int i = tid; i < GT * FC_HEAD_DIM; i += DA_THREADS) {
       const int g = i / FC_HEAD_DIM, d = i - g * FC_HEAD_DIM;
       if (g0 + g < G) {
-        const float o = (red[0][g][d] + red[1][g][d]) + (red[2][g][d] + red[3][g][d]);
+        const float o = ((red[0][g][d] + red[1][g][d]) + (red[2][g][d] + red[3][g][d])) * (1.f / DA_P_SCALE(DTYPE));
         part_o[(((long long)b * Hq + (h * G + g0 + g)) * max_splits + split) * FC_HEAD_DIM + d] = o;
       }
     }
@@ -430,10 +435,8 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 //   O^T[dim][head] = V^T P^T: the probabilities are already the B operand (keys in the order the accumulator gives
 //                           them); V goes through the wavefront's 8 KB of LDS and is read transposed, 2 bytes at a time.
 // Probabilities enter as a sum of 16-bit operands in the cache dtype: two (as the split kernel does for 5 to 8 heads), or
-// three for bf16 groups of up to 4 heads, where the split kernel multiplies in fp32.  Two fp16 operands hold 22 bits, but
-// only down to 2^-3: below, the second one runs into fp16's subnormal step (2^-24), and a probability under 2^-25 would
-// count in the sum and not in the output.  fp16 probabilities are therefore scaled by 2^14 (exactly; 1 stays below the
-// largest fp16 value) and the partial output back: what the operands drop is below 2^-39 of the tile's largest weight.
+// three for bf16 groups of up to 4 heads, where the split kernel multiplies in fp32.  Two fp16 operands hold 22 bits of
+// a probability down to 2^-17 and what they drop is below 2^-39 of the tile's largest (DA_P_SCALE).
 // Error of the unrounded output against 64 bits, 3 contexts of up to 2040 keys, 1 / 2 / 4 fp16 heads a group, this kernel
 // and the split kernel in fp32: flat 1.08 / 1.09 / 1.08e-7 and 1.12 / 1.09 / 1.12e-7, peaked 8.5 / 9.4 / 9.8e-8 and
 // 8.3 / 8.9 / 9.1e-8 (a third operand leaves the latter as they are); per layer 8.34 us before and after.
@@ -445,7 +448,6 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 #define DC_STAGE (DA_TILE * DC_VROW)
 #define DC_PART (DC_WAVES * DC_STAGE)                              // V stages, then the partial outputs
 #define DC_LDS (DC_PART + DC_WAVES * DC_HEADS * 8)
-#define DC_P_SCALE(DT) ((DT) == FC_F16 ? 16384.f : 1.f)
 static_assert(DC_PART >= DC_WAVES * DC_HEADS * DC_PSTRIDE * 4, "the partial outputs share the V stages' memory");
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -649,7 +651,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     for (int e = 0; e < 8; ++e) {
       p[e] = __builtin_amdgcn_exp2f(p[e] - ref);
       sum += p[e];
-      p[e] *= DC_P_SCALE(DTYPE);
+      p[e] *= DA_P_SCALE(DTYPE);
     }
     l = fmaf(l, alpha, sum);
     uint4 pt[TERMS];
@@ -703,7 +705,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   for (int w = 0; w < DC_WAVES; ++w) M = fmaxf(M, ml[w * DC_HEADS + l15].x);
   float* part = reinterpret_cast<float*>(smem);
   {
-    const float wgt = __builtin_amdgcn_exp2f(m - (M == -INFINITY ? 0.f : M)) * (1.f / DC_P_SCALE(DTYPE));   // 0 for a wavefront without tiles
+    const float wgt = __builtin_amdgcn_exp2f(m - (M == -INFINITY ? 0.f : M)) * (1.f / DA_P_SCALE(DTYPE));   // 0 for a wavefront without tiles
     if (l15 < ng) {
 #pragma unroll
       for (int db = 0; db < 8; ++db)

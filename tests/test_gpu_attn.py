@@ -363,9 +363,10 @@ def test_new_rows_are_seen_by_every_sequence_that_reads_their_page(dev, copies, 
 
 
 @pytest.mark.parametrize("Hq,Hkv", [(2, 2), (4, 2), (8, 2), (14, 2)])
-@pytest.mark.parametrize("lens", [[64, 250], [700, 300]])                    # one workgroup a column; several
+@pytest.mark.parametrize("lens,table", [([64, 250], 1), ([700, 300], 3),     # one workgroup a column; several
+                                        ([64, 250, 700], 70)])                # a table too wide for that kernel
 @pytest.mark.parametrize("below", [12, 20, 26])
-def test_small_fp16_probabilities_keep_their_bits(dev, Hq, Hkv, lens, below):
+def test_small_fp16_probabilities_keep_their_bits(dev, Hq, Hkv, lens, table, below):
     """Of every 32 keys one has the largest logit and a value of zero, the others 2^-below of its weight: the output is what
     those add, and its error stays within the output's own rounding (2^-11 of an element) and 2^-13 for the logits in
     fp32 (26 times 2^-24 and an exponential: below 2^-18 of a weight; the sum over equal weights adds no more).  An fp16
@@ -373,7 +374,7 @@ def test_small_fp16_probabilities_keep_their_bits(dev, Hq, Hkv, lens, below):
     from fastcache_amd.layers.attention import decode_attention
     dtype, B, scale = torch.float16, len(lens), 128 ** -0.5
     case = synth.make_paged_case(seed=6, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=lens, dtype=dtype)
-    pool, tables = case.kv_cache[:, 0].clone(), case.table_tensor("cpu")
+    pool, tables = case.kv_cache[:, 0].clone(), case.table_tensor("cpu", table)
     g = torch.Generator().manual_seed(8)
     pool[0] = 0
     pool[0, ..., 0] = -below * 0.6931471805599453 / scale / 16                # the query's first element is 16
