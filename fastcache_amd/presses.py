@@ -79,6 +79,11 @@ class ScorerPress:
         None when the shape does not take it."""
         return None
 
+    def _scores_and_selects_as(self, press) -> bool:
+        """Whether ``score`` is that class's and ``select`` the plain one: neither overridden nor set on this object."""
+        return (getattr(self.score, "__func__", None) is press.score and
+                getattr(self.select, "__func__", None) is ScorerPress.select)
+
     def compress(self, module, hidden_states, keys, values, attentions, kwargs):
         if self.compression_ratio == 0:
             return keys, values
@@ -232,8 +237,8 @@ class KnormPress(ScorerPress):
         return ops.knorm_score(_lib.dense_view(keys), keys.device)[0]
 
     def _press_into(self, module, hidden_states, keys, values, kwargs, n):
-        if type(self).score is not KnormPress.score or type(self).select is not ScorerPress.select:
-            return None                               # a subclass scores or selects in its own way
+        if not self._scores_and_selects_as(KnormPress):
+            return None
         return _lib.host().knorm_into(keys, values, n)
 
     def paged_scores(self, kview, vview, lens, seq_lens, layers, seq_ids, device) -> torch.Tensor:
@@ -335,8 +340,8 @@ class SnapKVPress(ScorerPress):
         return (q * cos + rot * sin).contiguous()
 
     def _press_into(self, module, hidden_states, keys, values, kwargs, n):
-        if type(self).score is not SnapKVPress.score or type(self).select is not ScorerPress.select:
-            return None                               # a subclass scores or selects in its own way
+        if not self._scores_and_selects_as(SnapKVPress):
+            return None
         B, H, S, D = keys.shape
         assert S > self.window_size, "Query length should be greater than the window size"
         W, ksz = self.window_size, self.kernel_size

@@ -817,6 +817,26 @@ def test_layer_hooks_in_one_call(dev, dtype, B, H, S):
                 assert not bool(((got ^ ref) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
 
 
+@pytest.mark.parametrize("name", ["knorm", "snapkv"])
+def test_a_score_or_selection_set_on_the_press_is_used(dev, name):
+    """``score`` and ``select`` given to one object count as those of a subclass do."""
+    B, H, S, W, keep = 1, 2, 400, 32, 200
+    g = torch.Generator().manual_seed(3)
+    k, v, q = (torch.randn(B, h, n, 128, generator=g).to(torch.bfloat16).to(dev) for h, n in ((H, S), (H, S), (2 * H, W)))
+    given = torch.rand(B, H, S, generator=g)
+    make = lambda: KnormPress(0.5) if name == "knorm" else SnapKVPress(0.5, window_size=W)
+    press = make()
+    press.score = lambda *a, **kw: given.to(dev)
+    ok, ov = press.compress(None, torch.zeros(B, S, 1), k, v, None, {"queries": q})
+    idx = opress.topk_lowest_index(given, keep)
+    assert torch.equal(ok.cpu(), opress.gather_tokens(k.cpu(), idx)) and torch.equal(ov.cpu(), opress.gather_tokens(v.cpu(), idx))
+    press = make()
+    first = torch.arange(keep, dtype=torch.int32, device=dev).expand(B, H, keep).contiguous()
+    press.select = lambda scores, n: first
+    ok, ov = press.compress(None, torch.zeros(B, S, 1), k, v, None, {"queries": q})
+    assert torch.equal(ok, k[:, :, :keep]) and torch.equal(ov, v[:, :, :keep])
+
+
 @pytest.mark.parametrize("S", [600, 5000, 17000])
 def test_snapkv_select_ragged(dev, S):
     """Selection straight from the sweeps' sums for sequences of different lengths, one of them no longer than the
