@@ -93,7 +93,9 @@ class ScorerPress:
         if out is not None:
             _lib.note_enqueued()
             return out
-        scores = self.score(module, hidden_states, keys, values, attentions, kwargs)
+        return self._gather(keys, values, self.score(module, hidden_states, keys, values, attentions, kwargs), n)
+
+    def _gather(self, keys, values, scores, n):
         B, H, S, D = keys.shape
         idx = self.select(scores, n).view(1, B, H, n)
         out_k = torch.empty((B, H, n, D), dtype=keys.dtype, device=keys.device)
@@ -354,16 +356,19 @@ class SnapKVPress(ScorerPress):
         if q.dtype != keys.dtype:
             q = q.to(keys.dtype)
         out_scale = 1.0 / (W * (q.shape[1] // H)) if self.reduction == "mean" else 1.0
-        return _lib.host().snapkv_into(keys, values, q, lse, n, W, ksz, self.causal_window, 1.0 / math.sqrt(D), out_scale)
+        out = _lib.host().snapkv_into(keys, values, q, lse, n, W, ksz, self.causal_window, 1.0 / math.sqrt(D), out_scale)
+        return out if out is not None else self._gather(keys, values, self._window_scores(keys, q, lse), n)
 
     def score(self, module, hidden_states, keys, values, attentions, kwargs) -> torch.Tensor:
         S = keys.shape[2]
         assert S > self.window_size, "Query length should be greater than the window size"
         q = self.window_queries(module, hidden_states, kwargs)
-        head_dim = keys.shape[-1]
         lse = kwargs.get("lse") if kwargs is not None else None      # [B, Hq, W] from the prefill's attention kernel
+        return self._window_scores(keys, q, lse)
+
+    def _window_scores(self, keys, q, lse) -> torch.Tensor:
         return ops.snapkv_score(_lib.dense_view(keys), q.to(keys.dtype), self.window_size, self.kernel_size,
-                                self.causal_window, self.reduction, 1.0 / math.sqrt(head_dim), lse=lse)[0]
+                                self.causal_window, self.reduction, 1.0 / math.sqrt(keys.shape[-1]), lse=lse)[0]
 
 
 @dataclass

@@ -837,6 +837,32 @@ def test_a_score_or_selection_set_on_the_press_is_used(dev, name):
     assert torch.equal(ok, k[:, :, :keep]) and torch.equal(ov, v[:, :, :keep])
 
 
+@pytest.mark.parametrize("S,keep,contiguous", [(500, 150, True), (500, 20, True),      # the native call; no more kept than the window
+                                               (500, 150, False), (36865, 900, True)])  # what the native call leaves to the others
+def test_window_queries_are_made_once(dev, S, keep, contiguous):
+    """The projection of the window queries runs once per layer, whichever path serves the layer."""
+    B, H, Hq, W = 1, 1, 2, 64
+    g = torch.Generator().manual_seed(5)
+    k, v, q = (torch.randn(B, h, n, 128, generator=g).to(torch.float16).to(dev) for h, n in ((H, S), (H, S), (Hq, W)))
+    if not contiguous:
+        q = q.transpose(1, 2).contiguous().transpose(1, 2)
+    calls = []
+
+    class Counted(SnapKVPress):
+        def window_queries(self, module, hidden_states, kwargs):
+            calls.append(1)
+            return q
+
+    press = Counted(1.0 - (keep + 0.5) / S, window_size=W)
+    ok, ov = press.compress(None, torch.zeros(B, S, 1), k, v, None, {})
+    assert len(calls) == 1
+    if keep > W and S == 500 and contiguous:      # other partial sums than the score tensor's: as many rows, the window among them
+        assert ok.shape == (B, H, keep, 128) and torch.equal(ok[:, :, -W:], k[:, :, -W:])
+    else:
+        idx = press.select(press.score(None, None, k, v, None, {}), keep).cpu().long()
+        assert torch.equal(ok.cpu(), opress.gather_tokens(k.cpu(), idx)) and torch.equal(ov.cpu(), opress.gather_tokens(v.cpu(), idx))
+
+
 @pytest.mark.parametrize("S", [600, 5000, 17000])
 def test_snapkv_select_ragged(dev, S):
     """Selection straight from the sweeps' sums for sequences of different lengths, one of them no longer than the
