@@ -36,7 +36,10 @@ class QuantizationMethod:
         self._quant_type = self._parse_quant_type(quant_type)
         self._group_size = group_size
         self._symmetric = symmetric
-        self._native_kind = ("INT8", "INT4", "NF4", "FP8_E4M3", "FP8_E5M2").index(self._quant_type.name)   # FC_QUANT_*
+
+    @property
+    def _native_kind(self) -> int:                      # FC_QUANT_*
+        return _NATIVE_KINDS[self._quant_type]
 
     def _parse_quant_type(self, quant_type: str) -> "QuantizationMethod.QuantType":
         mapping = {"int8": self.QuantType.INT8, "int4": self.QuantType.INT4, "fp8": self.QuantType.FP8_E4M3,
@@ -53,7 +56,8 @@ class QuantizationMethod:
 
     def compress(self, keys: torch.Tensor, values: torch.Tensor, **kwargs):
         """``((quantised keys, key scales), (quantised values, value scales))`` (methods.py:604-620)."""
-        if type(self) is QuantizationMethod and self._symmetric:      # both tensors by one native call
+        if self._symmetric and type(self) is QuantizationMethod and _QUANTIZERS.isdisjoint(self.__dict__):
+            # both tensors by one native call (a subclass, or a quantiser set on this object, goes its own way)
             out = _lib.host().quantize_pair(self._native_kind, keys, values, self._group_size)
             if out is not None:
                 _lib.note_enqueued()
@@ -100,6 +104,11 @@ class QuantizationMethod:
         if t in (self.QuantType.INT4, self.QuantType.NF4):
             return ops.dequantize_group4(quantized, scale, self._group_size, t == self.QuantType.NF4, dtype)
         return ops.dequantize_fp8(quantized, scale, dtype)
+
+
+_NATIVE_KINDS = {QuantizationMethod.QuantType[name]: kind for kind, name in
+                 enumerate(("INT8", "INT4", "NF4", "FP8_E4M3", "FP8_E5M2"))}
+_QUANTIZERS = frozenset(name for name in vars(QuantizationMethod) if name.startswith("_quantize"))
 
 
 class MLPCompressionMethod:

@@ -492,3 +492,19 @@ def test_quantised_pair_every_significand(dev, dtype, kind):
     k, v = x[0][:40, :40].contiguous().to(dev), torch.cat([x[0].reshape(-1)[:1601]]).to(dev)[1:].view(40, 40)
     for (q, s), t in zip(method.compress(k, v), (k, v)):
         assert torch.equal(bits_of(q), bits_of(quant(t.cpu())[0]))
+
+
+def test_a_quantiser_set_on_the_method_is_used(dev):
+    """A ``_quantize*`` given to one object counts as a subclass's does, and so does another quantiser type."""
+    from fastcache_amd.autocompress.methods import QuantizationMethod
+    k, v = (torch.randn(2, 3, 40, 128, generator=torch.Generator().manual_seed(i)).half().to(dev) for i in range(2))
+    for name in ("_quantize", "_quantize_int8"):
+        method = QuantizationMethod("int8")
+        setattr(method, name, lambda t: (t + 1, t + 2))
+        for (codes, scale), t in zip(method.compress(k, v), (k, v)):
+            assert torch.equal(codes, t + 1) and torch.equal(scale, t + 2)
+    method = QuantizationMethod("int8")
+    method._quant_type = QuantizationMethod.QuantType.INT4
+    for (codes, scale), (want, want_scale) in zip(method.compress(k, v), QuantizationMethod("int4").compress(k, v)):
+        assert torch.equal(codes, want) and torch.equal(scale, want_scale)
+        assert torch.equal(method.dequantize(codes, scale), QuantizationMethod("int4").dequantize(codes, scale))
