@@ -25,6 +25,15 @@ def _mlp(head_dim: int, cf: int) -> nn.Sequential:
         nn.Linear(head_dim, head_dim))
 
 
+def _linears(mlp: nn.Module):
+    """``(name in the container, module)`` of ``mlp[0]``, ``mlp[3]`` and ``mlp[6]``, whatever their names are."""
+    inner = mlp._modules
+    if type(mlp) is nn.Sequential:
+        items = list(inner.items())
+        return items[0], items[3], items[6]
+    return tuple((next((name for name, m in inner.items() if m is mlp[i]), None), mlp[i]) for i in (0, 3, 6))
+
+
 def _mlp_list(n_layer: int, head_dim: int, cf: int) -> nn.ModuleList:
     return nn.ModuleList([_mlp(head_dim, cf) for _ in range(n_layer)])
 
@@ -94,17 +103,17 @@ class _CCMBase(nn.Module):
         if hit is not None and hit[0] == (dtype, device, len(mods)) and host.unchanged(hit[1]):
             return hit[2]
         with torch.no_grad():
-            linear = [(m[0], m[3], m[6]) for m in mods]
+            linear = [_linears(m) for m in mods]
             packed = tuple(
-                torch.stack([getattr(three[i], name) for three in linear]).to(device=device, dtype=dtype).contiguous()
+                torch.stack([getattr(three[i][1], name) for three in linear]).to(device=device, dtype=dtype).contiguous()
                 for i in range(3) for name in ("weight", "bias"))
         steps = [(self._modules, group)]
-        for i, m in mods._modules.items():
+        for (i, m), three in zip(mods._modules.items(), linear):
             steps.append((mods._modules, i))
             inner = m._modules
-            for j in ("0", "3", "6"):
-                params = inner[j]._parameters
-                steps += [(inner, j), (params, "weight"), (params, "bias")]
+            for name, layer in three:
+                params = layer._parameters
+                steps += [(inner, name), (params, "weight"), (params, "bias")]
         watch = host.watch(steps)
         if watch is None:              # a parametrized Linear computes its weight on each access: nothing to hold on to
             self._stacked.pop(group, None)

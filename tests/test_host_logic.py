@@ -505,3 +505,34 @@ def test_packed_weights_leave_the_module_copyable_and_follow_replaced_parameters
         module.compress_tk[0][6].bias = torch.nn.Parameter(torch.zeros(128))
     with pytest.raises(RuntimeError, match="version"):
         pack(module)
+
+
+def test_weights_of_sequentials_with_named_children():
+    """The three Linears are found by position, whatever their names, and followed like the numbered ones."""
+    from collections import OrderedDict
+    cfg = SimpleNamespace(text_config=SimpleNamespace(num_hidden_layers=2, num_key_value_heads=2, hidden_size=256))
+    module = KVCacheLinearDecoupleCompressor(cfg, compression_factor=2)
+    cpu = torch.device("cpu")
+    pack = lambda: module._weights("compress_tk", torch.float32, cpu)
+    plain = pack()
+    names = ["w1", "relu1", "drop1", "w2", "relu2", "drop2", "w3"]
+    module.compress_tk[1] = torch.nn.Sequential(OrderedDict(zip(names, module.compress_tk[1])))
+    named = pack()
+    assert pack() is named and all(torch.equal(a, b) for a, b in zip(named, plain))
+    with torch.no_grad():
+        module.compress_tk[1].w3.bias.add_(1)
+    assert torch.equal(pack()[5][1], plain[5][1] + 1)
+    module.compress_tk[1].w2 = torch.nn.Linear(128, 128)
+    assert torch.equal(pack()[2][1], module.compress_tk[1][3].weight)
+
+    class Own(torch.nn.Module):                       # indexable, in an order of its own
+        def __init__(self, mlp):
+            super().__init__()
+            self.third, self.second, self.first = mlp[6], mlp[3], mlp[0]
+
+        def __getitem__(self, i):
+            return {0: self.first, 3: self.second, 6: self.third}[i]
+
+    module.compress_tk[0] = Own(module.compress_tk[0])
+    again = pack()
+    assert pack() is again and torch.equal(again[0][0], plain[0][0]) and torch.equal(again[4][0], plain[4][0])
