@@ -237,22 +237,20 @@ PyObject* py_ccm_layers(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       dst[s] = (int32_t)as_int(PyTuple_GET_ITEM(seg, 2));
     }
     const int64_t C = as_int(args[3]), B = k0.size(0), H = k0.size(1), D = k0.size(3);
-    // one allocation for all layers: what the caller gets are contiguous tensors inside it
-    at::Tensor all = at::empty({2 * (int64_t)L, B, H, C, D}, k0.options());
-    if (all.numel() > 0) {
-      fc_kv_view ks = dense_view(k0, L, 0), vs = dense_view(v0, L, 0);
-      fc_kv_view kd = dense_view(all.select(0, 0), L, B * H * C * D), vd = kd;
-      vd.base = (char*)all.data_ptr() + (int64_t)L * B * H * C * D * all.element_size();
-      check(fc_ccm_mlp_layers(ptr[0], ptr[1], &ks, &vs, &kd, &vd, w, nseg, start, len, dst, (int32_t)as_int(args[4]),
-                              (int32_t)as_int(args[5]), stream_of(k0)),
-            "fc_ccm_mlp_layers");
-    }
-    // plain tensors that share the allocation and nothing else: as autograd's views of one base they could not be written
-    // to with values that require a gradient, and a write to one would count as a write to all
-    std::vector<at::Tensor> parts;
-    {
-      at::AutoDispatchBelowADInplaceOrView below;
-      parts = all.unbind(0);
+    // a tensor per layer and plane, as the layers one by one would give: each can be saved, resized or dropped by itself
+    std::vector<at::Tensor> parts(2 * L);
+    void* to[2][64];
+    for (int p = 0; p < 2; ++p)
+      for (Py_ssize_t l = 0; l < L; ++l) {
+        at::Tensor& t = parts[p * L + l];
+        t = at::empty({B, H, C, D}, k0.options());
+        to[p][l] = t.data_ptr();
+      }
+    if (parts[0].numel() > 0) {
+      const fc_kv_view ks = dense_view(k0, L, 0), vs = dense_view(v0, L, 0), kd = dense_view(parts[0], L, 0);
+      check(fc_ccm_mlp_layers_into(ptr[0], ptr[1], to[0], to[1], &ks, &vs, &kd, &kd, w, nseg, start, len, dst,
+                                   (int32_t)as_int(args[4]), (int32_t)as_int(args[5]), stream_of(k0)),
+            "fc_ccm_mlp_layers_into");
     }
     PyObject* out = PyList_New(L);
     if (!out) throw PyFailed();

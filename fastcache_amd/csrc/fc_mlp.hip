@@ -433,7 +433,7 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
 // ---- a list of per-layer tensors, both planes and every segment in ONE launch ---------------------------------
 // A HuggingFace cache is a list of (K, V) tensors, one pair per layer; one prompt of it is little work per tensor (32
 // columns of 288 rows: 12 us of kernel), so what a launch per (layer, plane, segment) costs is the launches.  The
-// source addresses travel in the kernel's arguments (no table upload).  blockIdx.y = (segment, plane, layer); each
+// addresses travel in the kernel's arguments (no table upload).  blockIdx.y = (segment, plane, layer); each
 // segment has its own split of the columns, and a segment's remainder rows (or all rows of one too short to compress)
 // are copied behind its compressed rows by the same workgroup: source and destination are different tensors, so
 // nothing has to be ordered.
@@ -441,6 +441,7 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
 #define ML_LIST_SEGS 2
 struct MlpList {
   const char* src[2][ML_LIST_LAYERS];           // [plane][layer]
+  char* dst[2][ML_LIST_LAYERS];
   const char* w[ML_LIST_SEGS][2][6];            // [segment][plane]: w1, b1, w2, b2, w3, b3, all layers stacked
   int seg_start[ML_LIST_SEGS], c_rows[ML_LIST_SEGS], rem[ML_LIST_SEGS], dst_start[ML_LIST_SEGS];
   int wpc[ML_LIST_SEGS], ncg[ML_LIST_SEGS], gx[ML_LIST_SEGS];
@@ -458,7 +459,7 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_list_kernel(KvVi
   const KvView& src = p ? vsrc : ksrc;
   const KvView& dst = p ? vdst : kdst;
   const char* slayer = a.src[p][l];
-  char* dlayer = dst.base + (long long)l * dst.stride_layer * 2;
+  char* dlayer = a.dst[p][l];
   const int c = a.c_rows[seg], wpc = a.wpc[seg], ncg = a.ncg[seg];
   const long long ll = l;
   if (c > 0)
@@ -705,12 +706,11 @@ extern "C" int fc_ccm_mlp_ragged(const fc_kv_view* src, const fc_kv_view* dst, c
   return FC_OK;
 }
 
-extern "C" int fc_ccm_mlp_layers(const void* const* k_layers, const void* const* v_layers, const fc_kv_view* k_src,
-                                 const fc_kv_view* v_src, const fc_kv_view* k_dst, const fc_kv_view* v_dst,
-                                 const fc_mlp_weights* weights, int32_t num_segments, const int32_t* seg_start,
-                                 const int32_t* seg_len, const int32_t* dst_start, int32_t cf, int32_t min_rows,
-                                 void* stream) {
-  const char* who = "fc_ccm_mlp_layers";
+// k_out / v_out null: all layers of a plane in one allocation, a layer stride apart
+static int ml_list(const char* who, const void* const* k_layers, const void* const* v_layers, void* const* k_out, void* const* v_out,
+                   const fc_kv_view* k_src, const fc_kv_view* v_src, const fc_kv_view* k_dst, const fc_kv_view* v_dst,
+                   const fc_mlp_weights* weights, int32_t num_segments, const int32_t* seg_start, const int32_t* seg_len,
+                   const int32_t* dst_start, int32_t cf, int32_t min_rows, void* stream) {
   FC_REQUIRE(k_layers && v_layers && k_src && v_src && k_dst && v_dst && weights && seg_start && seg_len && dst_start,
              FC_EINVAL, "%s: null pointer", who);
   FC_REQUIRE(num_segments >= 1 && num_segments <= ML_LIST_SEGS, FC_EINVAL, "%s: %d segments (1 or 2)", who, num_segments);
@@ -730,8 +730,12 @@ extern "C" int fc_ccm_mlp_layers(const void* const* k_layers, const void* const*
   MlpList a;
   for (int p = 0; p < 2; ++p)
     for (int l = 0; l < k_src->num_layers; ++l) {
+      const fc_kv_view* dv = views[p][1];
+      void* const* out = p ? v_out : k_out;
       a.src[p][l] = (const char*)(p ? v_layers : k_layers)[l];
-      FC_REQUIRE(a.src[p][l] && ((uintptr_t)a.src[p][l] & 15) == 0, FC_EINVAL, "%s: layer %d not 16-byte aligned", who, l);
+      a.dst[p][l] = out ? (char*)out[l] : (char*)dv->base + (int64_t)l * dv->stride_layer * 2;
+      FC_REQUIRE(a.src[p][l] && a.dst[p][l] && (((uintptr_t)a.src[p][l] | (uintptr_t)a.dst[p][l]) & 15) == 0, FC_EINVAL,
+                 "%s: layer %d not 16-byte aligned", who, l);
     }
   const int ncols = k_src->batch * k_src->num_kv_heads;
   const int lp = 2 * k_src->num_layers;     // (plane, layer) pairs per segment
@@ -798,4 +802,24 @@ extern "C" int fc_ccm_mlp_layers(const void* const* k_layers, const void* const*
 #undef ML_LIST
   FC_CHECK_LAUNCH(who);
   return FC_OK;
+}
+
+extern "C" int fc_ccm_mlp_layers(const void* const* k_layers, const void* const* v_layers, const fc_kv_view* k_src,
+                                 const fc_kv_view* v_src, const fc_kv_view* k_dst, const fc_kv_view* v_dst,
+                                 const fc_mlp_weights* weights, int32_t num_segments, const int32_t* seg_start,
+                                 const int32_t* seg_len, const int32_t* dst_start, int32_t cf, int32_t min_rows,
+                                 void* stream) {
+  return ml_list("fc_ccm_mlp_layers", k_layers, v_layers, nullptr, nullptr, k_src, v_src, k_dst, v_dst, weights, num_segments,
+                 seg_start, seg_len, dst_start, cf, min_rows, stream);
+}
+
+extern "C" int fc_ccm_mlp_layers_into(const void* const* k_layers, const void* const* v_layers, void* const* k_out,
+                                      void* const* v_out, const fc_kv_view* k_src, const fc_kv_view* v_src,
+                                      const fc_kv_view* k_dst, const fc_kv_view* v_dst, const fc_mlp_weights* weights,
+                                      int32_t num_segments, const int32_t* seg_start, const int32_t* seg_len,
+                                      const int32_t* dst_start, int32_t cf, int32_t min_rows, void* stream) {
+  const char* who = "fc_ccm_mlp_layers_into";
+  FC_REQUIRE(k_out && v_out, FC_EINVAL, "%s: null pointer", who);
+  return ml_list(who, k_layers, v_layers, k_out, v_out, k_src, v_src, k_dst, v_dst, weights, num_segments, seg_start, seg_len,
+                 dst_start, cf, min_rows, stream);
 }

@@ -337,6 +337,13 @@ int fc_ccm_mlp_layers(const void* const* k_layers, const void* const* v_layers, 
                       const fc_kv_view* v_src, const fc_kv_view* k_dst, const fc_kv_view* v_dst,
                       const fc_mlp_weights* weights, int32_t num_segments, const int32_t* seg_start,
                       const int32_t* seg_len, const int32_t* dst_start, int32_t cf, int32_t min_rows, void* stream);
+/* The same with destinations of their own: k_out / v_out are HOST arrays of num_layers device pointers, one tensor each of the
+ * geometry of k_dst / v_dst (whose base is not read). */
+int fc_ccm_mlp_layers_into(const void* const* k_layers, const void* const* v_layers, void* const* k_out, void* const* v_out,
+                           const fc_kv_view* k_src, const fc_kv_view* v_src, const fc_kv_view* k_dst,
+                           const fc_kv_view* v_dst, const fc_mlp_weights* weights, int32_t num_segments,
+                           const int32_t* seg_start, const int32_t* seg_len, const int32_t* dst_start, int32_t cf,
+                           int32_t min_rows, void* stream);
 
 /*
  * Expected-attention scores: attention each key can expect from future queries whose distribution is

@@ -248,13 +248,15 @@ def test_ccm_forward_over_a_list_is_one_launch(dev, dtype, cf, S, img, B, min_se
 
 
 def test_ccm_forward_results_are_separate_tensors(dev):
-    """The results of one launch share an allocation and nothing else: each can be written to with values that require a
+    """The results of one launch share nothing: each has memory of its own, can be written to with values that require a
     gradient, and a write to one does not count as a write to another."""
     from types import SimpleNamespace
     from fastcache_amd.utils_ccm import KVCacheLinearDecoupleCompressor
     cfg = SimpleNamespace(text_config=SimpleNamespace(num_hidden_layers=2, num_key_value_heads=2, hidden_size=256))
     module = KVCacheLinearDecoupleCompressor(cfg, compression_factor=2).to(dev).to(torch.float16).eval()
     out = module([tuple(torch.randn(1, 2, 40, 128, device=dev).half() for _ in range(2)) for _ in range(2)], [0, 40])
+    for t in (t for kv in out for t in kv):
+        assert t.untyped_storage().nbytes() == t.numel() * t.element_size() and t.storage_offset() == 0
     (k0, v0), (k1, _) = out
     before = [t.clone() for t in (v0, k1)]
     versions = v0._version, k1._version
