@@ -9,7 +9,8 @@
 * ``select``: ``fc_select_compact`` the same way (``KP_WIDE_BYTES_SELECT``);
 * ``splits``: ``fc_snapkv_score`` / ``fc_snapkv_score_split`` with 1, 2, 4 and 8 key ranges per column (the rule is
   ``ops.snapkv_splits``);
-* ``press``:  the one-launch SnapKV press against split scoring + ``fc_select_compact`` (``ops.snapkv_press_preferred``).
+* ``press``:  the one-launch SnapKV press against split scoring, selection and compaction in launches of their own
+  (``ops.snapkv_press_preferred``).
 
 Every figure is the mean of 20 launches after 5, HIP events on the current stream.
 """
@@ -80,9 +81,12 @@ def splits(dev):
 
 
 def press(dev):
-    print("SnapKV press, a quarter kept, ms per pass: one launch / split scoring + fc_select_compact:")
+    print("SnapKV press, a quarter kept, ms per pass: one launch / split scoring + selection + compaction:")
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    for L, B, Hq, Hkv, S in ((28, 4, 28, 4, 4096), (28, 6, 28, 4, 4096), (36, 8, 32, 8, 4096), (20, 4, 28, 4, 12000)):
+    for L, B, Hq, Hkv, S in ((28, 1, 28, 4, 1000), (28, 2, 28, 4, 2000), (28, 1, 28, 4, 4096), (28, 2, 28, 4, 4096),
+                             (36, 1, 32, 8, 4096), (28, 4, 28, 4, 1000), (28, 4, 28, 4, 4096), (28, 6, 28, 4, 4096),
+                             (36, 3, 32, 8, 4096), (36, 1, 32, 8, 8192), (28, 4, 28, 4, 8192), (28, 6, 28, 4, 8192),
+                             (28, 8, 28, 4, 8192), (20, 4, 28, 4, 12000), (28, 4, 28, 4, 12000), (36, 8, 32, 8, 4096)):
         k, v, q = _snap_case(L, B, Hq, Hkv, S, dev)
         kv, vv = _lib.dense_view(k), _lib.dense_view(v)
         n = S // 4
@@ -94,7 +98,7 @@ def press(dev):
 
         def two():
             sc = ops.snapkv_score(kv, q, 64, 7, True, "sum", splits=ns)
-            ops.select_compact(kv, vv, sc, n)
+            ops.compact(kv, vv, kv, vv, ops.topk_select(sc, n))
         print(f"  {L * B * Hkv:5d} columns x {S:6d} keys: {one:.3f} / {_time(two):.3f} ({ns} ranges)   "
               f"(ops.snapkv_press_preferred: {ops.snapkv_press_preferred(kv, Hq, 64, cus)})")
         del k, v, q

@@ -347,8 +347,9 @@ class SnapKVPress(ScorerPress):
         B, H, S, D = keys.shape
         assert S > self.window_size, "Query length should be greater than the window size"
         W, ksz = self.window_size, self.kernel_size
-        # as on the runner hook: the window is always kept and only the other keys are ranked, which is the selection
-        # over the filled scores when more is kept than the window and a row's scores are not all one pooled value
+        # As on the runner hook: the window is always kept and only the other keys are ranked.  Over the filled scores (the
+        # path of the shapes refused below) the window ties with the keys of the layer's largest score and ranks behind
+        # them; the two selections differ when a row has more such keys than places outside the window.
         if n <= W or S - W <= ksz or self.reduction not in ("mean", "sum"):
             return None
         q = self.window_queries(module, hidden_states, kwargs)

@@ -863,6 +863,24 @@ def test_window_queries_are_made_once(dev, S, keep, contiguous):
         assert torch.equal(ok.cpu(), opress.gather_tokens(k.cpu(), idx)) and torch.equal(ov.cpu(), opress.gather_tokens(v.cpu(), idx))
 
 
+@pytest.mark.parametrize("S,keep", [(400, 40), (1500, 700), (5000, 100)])
+@pytest.mark.parametrize("with_lse", [False, True])
+def test_snapkv_hook_keeps_the_window_in_rows_of_equal_scores(dev, S, keep, with_lse):
+    """Zero queries weigh every key alike: all scores are equal except at the ends of the zero-padded pooling.  The window
+    is kept whole, ahead of the keys that tie with the largest score, and of those the first ones are."""
+    B, H, W, ksz = 2, 2, 32, 5
+    g = torch.Generator().manual_seed(S)
+    k, v = (torch.randn(B, H, S, 128, generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
+    kw = {"queries": torch.zeros(B, 2 * H, W, 128, dtype=torch.bfloat16, device=dev)}
+    if with_lse:
+        seen = torch.arange(S - W + 1, S + 1, dtype=torch.float32, device=dev)       # keys that window query i sees
+        kw["lse"] = seen.log().expand(B, 2 * H, W).contiguous()
+    press = SnapKVPress(1.0 - (keep + 0.5) / S, window_size=W, kernel_size=ksz)
+    ok, ov = press.compress(None, torch.zeros(B, S, 1), k, v, None, kw)
+    idx = torch.cat([torch.arange(ksz // 2, ksz // 2 + keep - W), torch.arange(S - W, S)]).to(dev)
+    assert torch.equal(ok, k[:, :, idx]) and torch.equal(ov, v[:, :, idx])
+
+
 @pytest.mark.parametrize("S", [600, 5000, 17000])
 def test_snapkv_select_ragged(dev, S):
     """Selection straight from the sweeps' sums for sequences of different lengths, one of them no longer than the
