@@ -909,19 +909,6 @@ extern "C" int64_t fc_decode_attn_workspace_bytes(int32_t batch, int32_t num_q_h
   return (int64_t)batch * num_q_heads * (splits > 0 ? splits : 1) * (FC_HEAD_DIM + 2) * (int64_t)sizeof(float);
 }
 
-// compute units of the current device (0 if the query fails), cached per device
-static int da_compute_units() {
-  static std::atomic<int> cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 0) n = 0;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 // A 32-token tile never straddles two pages and its byte offsets fit 32 bits.
 static bool da_tile_in_page(const fc_kv_view* v) {
   return v->stride_token >= 0 && v->stride_token < (1 << 24) &&
@@ -939,7 +926,7 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
   const int G = num_q_heads / k->num_kv_heads;
   const long long cols = (long long)k->num_kv_heads * ((G + DC_HEADS - 1) / DC_HEADS) * k->batch;
-  const long long slots = da_compute_units() > 0 ? da_compute_units() : 256;
+  const long long slots = fc_compute_units();
   const auto pages_ok = [](const fc_kv_view* x) {       // one block-table entry per lane
     return x->block_tables == nullptr || (x->max_seq_len - 1) / x->block_size < FC_WAVE;
   };
@@ -1035,10 +1022,10 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
   // device, so the choice is the same at capture and at every replay.
   int chunk = DA_CHUNK;
   {
-    const int slots = 2 * da_compute_units();
+    const int slots = 2 * fc_compute_units();
     const long long cols = (long long)Hkv * gtiles * B;
     double best = -1.0;
-    for (int cand = DA_CHUNK; slots > 0 && cand <= DA_CHUNK_MAX; cand += DA_TILE) {
+    for (int cand = DA_CHUNK; cand <= DA_CHUNK_MAX; cand += DA_TILE) {
       if ((DA_RING + gt * cand * 4) * 2 > 158 * 1024) break;
       const long long wgs = cols * ((k_cache->max_seq_len + cand - 1) / cand);
       const double cost = (double)((wgs + slots - 1) / slots) * (cand + 96.0);

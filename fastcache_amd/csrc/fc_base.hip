@@ -1,5 +1,6 @@
 // Library-wide pieces of libfastcache_hip: ABI version, per-thread error text, view validation.
 #include "fc_common.h"
+#include <atomic>
 
 static thread_local char g_err[512] = "";
 
@@ -12,6 +13,16 @@ void fc_set_error(const char* fmt, ...) {
 
 extern "C" int fc_abi_version(void) { return FC_ABI_VERSION; }
 extern "C" const char* fc_last_error(void) { return g_err; }
+
+int fc_compute_units() {
+  static std::atomic<int> cus[64];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if ((n = cus[dev].load(std::memory_order_relaxed)) > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+  cus[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
 
 int fc_check_view(const fc_kv_view* v, const char* who) {
   FC_REQUIRE(v != nullptr, FC_EINVAL, "%s: null view", who);

@@ -44,6 +44,9 @@ void fc_set_error(const char* fmt, ...);
 
 int fc_check_view(const fc_kv_view* v, const char* who);
 
+// compute units of the current device (an MI355X's 256 where there is none to ask)
+int fc_compute_units();
+
 static inline int fc_elem_bytes(int dtype) { return dtype == FC_F32 ? 4 : 2; }
 
 // ---- device-side copy of a view ---------------------------------------------------------------

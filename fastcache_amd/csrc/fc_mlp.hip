@@ -484,18 +484,6 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_list_kernel(KvVi
   }
 }
 
-// compute units of the current device (0 if the query fails)
-static int ml_compute_units() {
-  static int cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus[dev] = n;
-  }
-  return cus[dev];
-}
-
 // What the MLP leaves of a ragged segment: the seg_len % cf remainder tokens, or the whole segment of a sequence
 // too short to compress, copied to their place behind the compressed rows.  One workgroup per (head, sequence,
 // layer); 16 tokens per pass, all loaded before any is stored (destination token <= source token, ascending).
@@ -559,7 +547,7 @@ static int ml_check(const char* who, const fc_kv_view* src, const fc_kv_view* ds
 struct MlSplit { int wpc, gx; };
 template <typename Fits>
 static MlSplit ml_split(int ncols, int jobs, int c, int cf, Fits fits) {
-  const int64_t ncu = ml_compute_units() > 0 ? ml_compute_units() : 256;
+  const int64_t ncu = fc_compute_units();
   const double least = cf <= 2 ? 1.0 : 0.8;
   MlSplit best{ML_WAVES, ncols};      // what is left when no split fits
   double best_cost = -1.0;
@@ -602,11 +590,11 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
     // Sequences of different lengths: many small workgroups, or the longest sequence would decide (5 of 2666 to 8000
     // tokens: 794 us per pass, 961 with the split by the largest row count).
     while (wpc < ML_WAVES && (int64_t)ncols * wpc / ML_WAVES * src->num_layers < 1024 && ML_ROWS * wpc * 2 <= c) wpc *= 2;
-    const int groups = (ncols * wpc + ML_WAVES - 1) / ML_WAVES, ncu = ml_compute_units();
+    const int groups = (ncols * wpc + ML_WAVES - 1) / ML_WAVES, ncu = fc_compute_units();
     const double t_group = 1.5 * ((c + ML_ROWS * wpc - 1) / (ML_ROWS * wpc)) * (cf + 2), t_start = 4.0;   // microseconds, roughly
     gx = groups;
     double best = -1.0;
-    for (int per = 1; cf <= 2 && ncu > 0 && per <= groups && per <= 64; ++per) {
+    for (int per = 1; cf <= 2 && per <= groups && per <= 64; ++per) {
       const int g = (groups + per - 1) / per;
       const long long rounds = ((long long)g * src->num_layers + ncu - 1) / ncu;
       const double cost = (double)rounds * (((groups + g - 1) / g) * t_group + t_start);
@@ -761,7 +749,7 @@ static int ml_list(const char* who, const void* const* k_layers, const void* con
     // How many wavefronts share a column and how many column groups a workgroup walks: the pair with the fewest
     // rounds * (groups * time per group + start-up).  (With the last round counted as in ml_split: 0.92 to 1.03 times as
     // fast, on the whole slower; the two segments share the launch, so a round of one is filled up by the other.)
-    const int ncu = ml_compute_units() > 0 ? ml_compute_units() : 256;
+    const int ncu = fc_compute_units();
     double best = -1.0;
     a.wpc[s] = 1;
     a.ncg[s] = (ncols + ML_WAVES - 1) / ML_WAVES;

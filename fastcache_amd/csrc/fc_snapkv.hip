@@ -838,7 +838,7 @@ extern "C" int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q
                                                 (keys->max_seq_len - 1) / keys->block_size < SK_TBL);
   if (columns <= 0 || columns >= 1000 || blocks > 16 || !paged_ok) return 1;
   const double a = blocks > 8 ? 1.7 : blocks > 4 ? 0.83 : 0.7, f = blocks > 8 ? 9.0 : 7.0;
-  const long long slots = blocks > 4 ? 256 : 512;
+  const long long slots = (long long)fc_compute_units() * (blocks > 4 ? 1 : 2);
   int best_n = 1;
   double best = (double)((columns + slots - 1) / slots) * (2.0 * tiles * a + f);
   for (int n = 2; n <= 32 && n * 2 <= tiles; ++n) {

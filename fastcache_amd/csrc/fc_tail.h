@@ -27,7 +27,7 @@ int fc_column_select(const char* who, int src, const fc_kv_view* keys, const fc_
 
 // workgroups per column for a gather: about two per compute unit in all, no share below 64 rows
 static inline int fc_gather_parts(long long cols, int k) {
-  long long p = (512 + cols - 1) / cols;
+  long long p = (2 * fc_compute_units() + cols - 1) / cols;
   if (p > (k + 63) / 64) p = (k + 63) / 64;
   p = p < 1 ? 1 : p > 16 ? 16 : p;
   const int lds = (k + 8191) / 8192;      // a share's positions are in LDS, at most 32 KB of them

@@ -230,7 +230,7 @@ static int cs_check(const char* who, const fc_kv_view* keys, const fc_kv_view* v
 // round); at 4096 keys and less, where two and more share a compute unit, 96 of 4000 76 -> 77, 64 of 2000 29 -> 34.
 extern "C" int fc_press_gather_apart(int32_t columns, int32_t max_seq_len, int32_t k) {
   if (columns <= 0 || k <= 0) return 0;
-  return max_seq_len > 4096 && (long long)columns * fc_gather_parts(columns, k) > 256;
+  return max_seq_len > 4096 && (long long)columns * fc_gather_parts(columns, k) > fc_compute_units();
 }
 
 extern "C" int fc_knorm_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
