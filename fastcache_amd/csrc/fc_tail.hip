@@ -244,15 +244,14 @@ extern "C" int fc_knorm_press_into(const fc_kv_view* keys, const fc_kv_view* val
   a.k = a.index_stride = k;
   a.parts = indices ? 0 : fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, k);
   a.indices = indices;
-  if (!scores) {   // the workgroups that gather a column score it as well
+  if (!scores) {   // the workgroups that select a column score it as well
     FC_REQUIRE(keys->max_seq_len <= CS_NORMS_MAX, FC_EUNSUPPORTED, "%s: columns of more than %d keys need a score buffer", who,
                CS_NORMS_MAX);
-    rc = fc_column_select(who, CS_NORMS, keys, values, out_k, out_v, a, (hipStream_t)stream);
-    return rc || !indices ? rc : fc_compact(keys, values, out_k, out_v, indices, k, keys->num_kv_heads, k, nullptr, stream);
+  } else if ((rc = fc_knorm_score(keys, scores, score_stride, stream))) {
+    return rc;
   }
-  if ((rc = fc_knorm_score(keys, scores, score_stride, stream))) return rc;
   a.in = scores;
   a.stride = score_stride;
-  rc = fc_column_select(who, CS_SCORES, keys, values, out_k, out_v, a, (hipStream_t)stream);
+  rc = fc_column_select(who, scores ? CS_SCORES : CS_NORMS, keys, values, out_k, out_v, a, (hipStream_t)stream);
   return rc || !indices ? rc : fc_compact(keys, values, out_k, out_v, indices, k, keys->num_kv_heads, k, nullptr, stream);
 }

@@ -149,7 +149,7 @@ def snapkv_score(keys: FcKvView, queries: torch.Tensor, window: int, kernel_size
 
 
 def snapkv_press_fits(keys: FcKvView, num_q_heads: int, window: int, index_stride: int) -> bool:
-    """Whether :func:`snapkv_press` takes this shape (otherwise: ``snapkv_score`` + ``select_compact``): at most 16
+    """Whether :func:`snapkv_press` takes this shape (otherwise: ``snapkv_score``, selection and compaction): at most 16
     blocks of 32 window queries per kv head, pages of 64*2^n tokens or a dense view, and
     the score row plus the kept positions inside the LDS of the key tiles."""
     if num_q_heads % keys.num_kv_heads:
@@ -168,13 +168,14 @@ def snapkv_press_fits(keys: FcKvView, num_q_heads: int, window: int, index_strid
 
 def snapkv_press_preferred(keys: FcKvView, num_q_heads: int, window: int, compute_units: int = 256) -> bool:
     """Whether the one-launch press (whole columns) or split scoring (:func:`snapkv_splits` key ranges per column, then
-    ``select_compact``) is the faster form for a shape both take.  Whole columns cost ``rounds x column time`` with
-    ``rounds = ceil(columns / workgroups the GPU holds)`` (two per compute unit, one with 16 wavefronts), split scoring
-    grows linearly with the columns but pays a merge, a pooling and a compaction launch.  Measured on MI355X (28 x B x 4
-    and 36 x B x 8 columns of 4096 to 12000 keys; ``python -m fastcache_amd.crossovers press``, figures in
-    profiles/launch_shape_crossovers.txt): whole columns win or tie when the last round is at least 80 % full
-    or the columns are short (up to 4096 keys: 0.64 against 0.72 ms at 448 columns, 0.92 against 1.01 at 672, at worst
-    2.5 % behind); long columns in poorly filled rounds lose (320 x 12000: 1.64 against 1.37 ms)."""
+    ``topk_select`` and ``compact``) is the faster form for a shape both take, where scores and indices are wanted.  Whole
+    columns cost ``rounds x column time`` with ``rounds = ceil(columns / workgroups the GPU holds)`` (two per compute unit,
+    one with 16 wavefronts), split scoring grows linearly with the columns but pays a merge, a pooling, a selection and a
+    compaction launch.  Measured on MI355X (28 x B x 4 and 36 x B x 8 columns; ``python -m fastcache_amd.crossovers press``,
+    figures in profiles/launch_shape_crossovers.txt): whole columns win or tie when the last round is at least 80 % full
+    or the columns are short (up to 4096 keys: 0.62 against 0.71 ms at 448 columns, 0.91 against 1.00 at 672, 0.32 against
+    0.40 at 224; 112 columns, less than a quarter of a round, are behind with 0.27 against 0.24); long columns in poorly
+    filled rounds lose (288 x 8192: 0.57 against 0.53 ms, 320 x 12000: 1.63 against 1.35)."""
     if snapkv_splits(keys, num_q_heads, window) == 1:
         return True
     columns = keys.num_layers * keys.batch * keys.num_kv_heads
@@ -191,7 +192,7 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     """SnapKV scores, selection (the window always kept; ``k`` or ``n_kept[b]`` positions per row, window included,
     more than the window) and in-place compaction of both planes, each (layer, sequence, kv head) column by one
     workgroup in one launch; then the window fill of the scores.  Returns ``(scores, indices)`` equal to
-    ``snapkv_score`` + ``select_compact``.  Shapes must satisfy :func:`snapkv_press_fits`.
+    ``snapkv_score`` + ``topk_select`` + ``compact`` (up to keys that tie exactly with the layer's largest score).  Shapes must satisfy :func:`snapkv_press_fits`.
 
     ``n_kept``: the kept counts per sequence as Python ints (checked here: the kernel leaves a sequence longer than the
     window untouched when its count does not exceed the window, which a caller that then shortens the sequence
@@ -376,7 +377,8 @@ def select_compact(keys: FcKvView, values: FcKvView, scores: torch.Tensor, k: in
                    rows_only: bool = False) -> torch.Tensor:
     """``topk_select`` over each sequence's own length and ``compact`` of both planes onto themselves in one launch;
     ``scores`` fp32 ``[L, B, Hkv, stride]`` contiguous.  Returns the indices ``[L, B, Hkv, k]`` (-1 past a row's kept
-    count with ``n_kept`` or ``ragged``, unless ``rows_only``)."""
+    count with ``n_kept`` or ``ragged``, unless ``rows_only``).  For callers that want one launch: the paged presses
+    issue the two apart, which gives the compaction a workgroup per plane."""
     _lib.require_gpu(scores, "scores")
     L, B, H = keys.num_layers, keys.batch, keys.num_kv_heads
     if scores.dtype != torch.float32 or scores.dim() != 4 or tuple(scores.shape[:3]) != (L, B, H) or \

@@ -817,6 +817,34 @@ def test_layer_hooks_in_one_call(dev, dtype, B, H, S):
                 assert not bool(((got ^ ref) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,k", [(1, 1), (512, 100), (513, 513), (1025, 300), (4096, 4000)])
+def test_knorm_press_into_forms(dev, dtype, S, k):
+    """The entry point's four forms (scores in a buffer or in the selecting workgroups' LDS, gather inside or apart) give the
+    same bytes, up to the largest column without a score buffer; a longer one is refused."""
+    import ctypes
+    B, H = 2, 3
+    g = torch.Generator().manual_seed(S)
+    kd, vd = (torch.randn(B, H, S, 128, generator=g).to(dtype).to(dev) for _ in range(2))
+    call = _lib.fn("fc_knorm_press_into")
+    results = []
+    for buffer in (True, False):
+        for apart in (False, True):
+            ok, ov = (torch.empty(B, H, k, 128, dtype=dtype, device=dev) for _ in range(2))
+            scores = torch.empty(B, H, S, device=dev)
+            idx = torch.empty(B, H, k, dtype=torch.int32, device=dev)
+            views = [_lib.dense_view(t) for t in (kd, vd, ok, ov)]
+            _lib.check(call(*(ctypes.byref(v) for v in views), k, scores.data_ptr() if buffer else None, S,
+                            idx.data_ptr() if apart else None, _lib.current_stream()), "fc_knorm_press_into")
+            results.append((ok, ov))
+    want = opress.topk_lowest_index(ops.knorm_score(_lib.dense_view(kd), dev)[0].cpu(), k)
+    for ok, ov in results:
+        assert torch.equal(ok.cpu(), opress.gather_tokens(kd.cpu(), want)) and torch.equal(ov.cpu(), opress.gather_tokens(vd.cpu(), want))
+    long = torch.empty(1, 1, 4097, 128, dtype=dtype, device=dev)
+    views = [_lib.dense_view(long)] * 4
+    assert call(*(ctypes.byref(v) for v in views), 1, None, 4097, None, _lib.current_stream()) == -2
+
+
 @pytest.mark.parametrize("name", ["knorm", "snapkv"])
 def test_a_score_or_selection_set_on_the_press_is_used(dev, name):
     """``score`` and ``select`` given to one object count as those of a subclass do."""
