@@ -437,6 +437,7 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 // Probabilities enter as a sum of 16-bit operands in the cache dtype: two (as the split kernel does for 5 to 8 heads), or
 // three for bf16 groups of up to 4 heads, where the split kernel multiplies in fp32.  Two fp16 operands hold 22 bits of
 // a probability down to 2^-17 and what they drop is below 2^-39 of the tile's largest (DA_P_SCALE).
+// (An infinite value in V gives NaN: a term of its probability is zero or negative.  In fp32 it gave an infinity.)
 // Error of the unrounded output against 64 bits, 3 contexts of up to 2040 keys, 1 / 2 / 4 fp16 heads a group, this kernel
 // and the split kernel in fp32: flat 1.08 / 1.09 / 1.08e-7 and 1.12 / 1.09 / 1.12e-7, peaked 8.5 / 9.4 / 9.8e-8 and
 // 8.3 / 8.9 / 9.1e-8 (a third operand leaves the latter as they are); per layer 8.34 us before and after.
