@@ -3,8 +3,9 @@
 // each Linear's output rounded to the storage dtype.  Reads and writes the caches in place.
 //
 // Shape of the work: one workgroup of 8 wavefronts (two per SIMD, so that one multiplies while
-// the other converts, loads or stores) per group of (sequence, head) columns of one
-// layer; a wavefront owns 32 rows of one column per iteration.  The three GEMMs are transposed
+// the other converts, loads or stores) per group of columns of one layer; a column is one sequence's rows of
+// 1 << hsh heads that lie side by side, row r being output token r >> hsh of head r % (1 << hsh); a wavefront owns 32
+// rows of one column per iteration.  The three GEMMs are transposed
 // (features along the accumulator registers, one token per lane) and chained through registers:
 //   layer 1  H1^T = W1 * X^T   A = W1 rows from LDS, B = X token rows;
 //   layer 2  H2^T = W2 * H1^T  B = layer 1's accumulators, converted in place;
@@ -23,9 +24,10 @@
 // W2 and W3 (permuted) stay in LDS for the life of the workgroup; W1 streams through a double
 // buffer one 128-column chunk (one source token) at a time, shared by the wavefronts; each
 // wavefront prefetches the X rows of the next chunk into registers while it multiplies the current one.
-// In-place safety: output row j lands on token dst_start + j <= seg_start + cf*j; all rows of an
+// In-place safety: output token j lands on token dst_start + j <= seg_start + cf*j; all rows of an
 // iteration are read before the workgroup barrier that precedes its stores, and later iterations
 // read tokens no earlier iteration writes.
+#include <math.h>
 #include "fc_common.h"
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -93,6 +95,28 @@ __device__ __forceinline__ void ml_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The sequence whose segment is the rank-th longest (of equal ones the first); more than 256 sequences are taken as they
+// come.  Every wavefront works it out for itself: lane i counts the segments ahead of its own.
+__device__ __forceinline__ int ml_ranked_sequence(const int* __restrict__ seg_len_v, int batch, int rank) {
+  if (batch <= 1 || batch > 256) return rank;
+  const int lane = threadIdx.x & 63;
+  int found = rank;
+  for (int i0 = 0; i0 < batch; i0 += 64) {
+    const int i = i0 + lane, own = seg_len_v[min(i, batch - 1)];
+    int ahead = 0;
+    for (int j0 = 0; j0 < batch; j0 += 64) {
+      const int other = seg_len_v[min(j0 + lane, batch - 1)], m = min(64, batch - j0);
+      for (int j = 0; j < m; ++j) {
+        const int len = __builtin_amdgcn_readlane(other, j);
+        ahead += (len > own || (len == own && j0 + j < i)) ? 1 : 0;
+      }
+    }
+    const unsigned long long who = __ballot(i < batch && ahead == rank);
+    if (who) found = i0 + __ffsll((long long)who) - 1;
+  }
+  return __builtin_amdgcn_readfirstlane(found);
+}
+
 // SRC_T / DST_T: 0 = dense view (no table), 1 = paged view whose table row fits the LDS cache,
 // 2 = paged view read through global memory.
 // W1R: all of W1 fits the two LDS chunk buffers (cf <= 2) and is loaded once; otherwise W1 streams
@@ -107,7 +131,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
                                          const char* __restrict__ w1l, const char* __restrict__ b1l,
                                          const char* __restrict__ w2l, const char* __restrict__ b2l,
                                          const char* __restrict__ w3l, const char* __restrict__ b3l, int cf,
-                                         int seg_start, int c_rows, int dst_start, int wpc, int ncols, int ncg, int cg0,
+                                         int seg_start, int c_rows, int dst_start, int hsh, int wpc, int ncols, int ncg, int cg0,
                                          int cg_step, const int* __restrict__ seg_start_v,
                                          const int* __restrict__ seg_len_v, const int* __restrict__ dst_start_v,
                                          int min_rows) {
@@ -124,7 +148,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
   const int lq = lane >> 2, lp = lane & 3;   // memory-side layout: row lq (and 16 + lq), 16-byte piece lp of 64 bytes
   const int cols_per_wg = ML_WAVES / wpc;
   const int sub = wave % wpc;
-  const int H = src.num_kv_heads;
+  const int hg_per_seq = src.num_kv_heads >> hsh;   // columns of a sequence
   const int K1 = cf * 128;
   // the column this wavefront works on; set per column group
   int col = 0, b = 0, h = 0;
@@ -202,10 +226,14 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
   };
 
   const int rows_per_iter = ML_ROWS * wpc;
-  int n_iter = (c_rows + rows_per_iter - 1) / rows_per_iter;
+  int n_iter = ((c_rows << hsh) + rows_per_iter - 1) / rows_per_iter;
   int q_total = n_iter * cf;      // W1 chunk q = (iteration q / cf, token kc = q % cf) sits in buffer q & 1
-  const char* sbase = nullptr;   // this lane's piece of token 0 of the column's head, per column group
+  const char* sbase = nullptr;   // this lane's piece of token 0 of the column's first head, per column group
   char* dbase = nullptr;
+  // the heads of this lane's two rows on the memory side: rows advance by multiples of 32, so they stay the same
+  const int hmask = (1 << hsh) - 1;
+  const int sho[2] = {(lq & hmask) * (int)src.stride_head * 2, ((16 + lq) & hmask) * (int)src.stride_head * 2};
+  const int dho[2] = {(lq & hmask) * (int)dst.stride_head * 2, ((16 + lq) & hmask) * (int)dst.stride_head * 2};
 
   // X rows of chunk q: xf[2*c4 + rh] holds bytes [64*c4 + 16*lp, +16) of the token row of output row 16*rh + lq
   auto x_load = [&](uint4 (&xf)[8], int q) {
@@ -217,7 +245,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
     // computed from them is never stored.
 #pragma unroll
     for (int rh = 0; rh < 2; ++rh) {
-      int r = min(row0 + rh * 16 + lq, cr - 1);
+      int r = min((row0 + rh * 16 + lq) >> hsh, cr - 1);
       int tok = ss + cf * r + kc;
       if constexpr (RAG) {   // a column with no rows, or fewer than the launch's bound, reads some valid token
         r = max(r, 0);
@@ -226,7 +254,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
       long long off = src_off(tok);
       off = off < 0 ? 0 : off;
 #pragma unroll
-      for (int c4 = 0; c4 < 4; ++c4) xf[c4 * 2 + rh] = *reinterpret_cast<const uint4*>(sbase + off * 2 + c4 * 64);
+      for (int c4 = 0; c4 < 4; ++c4) xf[c4 * 2 + rh] = *reinterpret_cast<const uint4*>(sbase + off * 2 + sho[rh] + c4 * 64);
     }
   };
   // Re-laying through this wavefront's 2 KB of LDS: rows of 64 bytes, the four 16-byte pieces of a row XOR-ed
@@ -328,10 +356,10 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
       char* rowp[2];
 #pragma unroll
       for (int rh = 0; rh < 2; ++rh) {
-        const int r = row0 + rh * 16 + lq;
+        const int r = (row0 + rh * 16 + lq) >> hsh;
         long long off = -1;
         if (col_ok && r < cr) off = dst_off(ds + r);
-        rowp[rh] = off >= 0 ? dbase + off * 2 : nullptr;
+        rowp[rh] = off >= 0 ? dbase + off * 2 + dho[rh] : nullptr;
       }
       // (a half-wave writes one 8-byte half per row, so rows that share a piece position in a bank window keep
       // their halves swapped: bit 3 xor bit 4 of the row number)
@@ -372,8 +400,9 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
     if (cg != cg0) __syncthreads();   // every wavefront is done with the previous group's tables and W1 buffers
     col = cg * cols_per_wg + wave / wpc;
     col_ok = col < ncols;
-    b = col_ok ? col / H : 0;
-    h = col_ok ? col - (col / H) * H : 0;
+    b = col_ok ? col / hg_per_seq : 0;
+    h = col_ok ? (col - b * hg_per_seq) << hsh : 0;
+    if constexpr (RAG) b = ml_ranked_sequence(seg_len_v, src.batch, b);
     sbase = slayer + (long long)h * src.stride_head * 2 + lp * 16;
     dbase = dlayer + (long long)h * dst.stride_head * 2 + lp * 16;
     if constexpr (RAG) {
@@ -397,7 +426,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
       int most = 0;
 #pragma unroll
       for (int w = 0; w < ML_WAVES; ++w) most = max(most, wave_rows[w]);
-      n_iter = (most + rows_per_iter - 1) / rows_per_iter;
+      n_iter = ((most << hsh) + rows_per_iter - 1) / rows_per_iter;
       q_total = n_iter * cf;
     }
 #pragma unroll
@@ -418,16 +447,22 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
                                                             const char* __restrict__ b1, const char* __restrict__ w2,
                                                             const char* __restrict__ b2, const char* __restrict__ w3,
                                                             const char* __restrict__ b3, int cf, int seg_start,
-                                                            int c_rows, int dst_start, int wpc, int ncols, int ncg,
+                                                            int c_rows, int dst_start, int hsh, int wpc, int ncols, int ncg,
                                                             const int* __restrict__ seg_start_v,
                                                             const int* __restrict__ seg_len_v,
                                                             const int* __restrict__ dst_start_v, int min_rows) {
   extern __shared__ __align__(16) char lds[];
-  const long long l = blockIdx.y;
+  long long l = blockIdx.y;
+  int group = blockIdx.x;
+  if constexpr (RAG) {   // one workgroup per group of columns, the longest sequences' groups of all layers first
+    const unsigned id = blockIdx.x + gridDim.x * blockIdx.y;
+    group = (int)(id / gridDim.y);
+    l = id - (unsigned)group * gridDim.y;
+  }
   mlp_body<DTYPE, SRC_T, DST_T, W1R, RAG>(
       lds, src, dst, src.base + l * src.stride_layer * 2, dst.base + l * dst.stride_layer * 2, w1 + l * 128 * cf * 256,
       b1 + l * 256, w2 + l * 128 * 256, b2 + l * 256, w3 + l * 128 * 256, b3 + l * 256, cf, seg_start, c_rows, dst_start,
-      wpc, ncols, ncg, blockIdx.x, gridDim.x, seg_start_v, seg_len_v, dst_start_v, min_rows);
+      hsh, wpc, ncols, ncg, group, gridDim.x, seg_start_v, seg_len_v, dst_start_v, min_rows);
 }
 
 // ---- a list of per-layer tensors, both planes and every segment in ONE launch ---------------------------------
@@ -466,7 +501,7 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_list_kernel(KvVi
     mlp_body<DTYPE, 0, 0, W1R, false>(lds, src, dst, slayer, dlayer, a.w[seg][p][0] + ll * 128 * cf * 256,
                                       a.w[seg][p][1] + ll * 256, a.w[seg][p][2] + ll * 128 * 256, a.w[seg][p][3] + ll * 256,
                                       a.w[seg][p][4] + ll * 128 * 256, a.w[seg][p][5] + ll * 256, cf, a.seg_start[seg], c,
-                                      a.dst_start[seg], wpc, ncols, ncg, blockIdx.x, gx, nullptr, nullptr, nullptr, 0);
+                                      a.dst_start[seg], 0, wpc, ncols, ncg, blockIdx.x, gx, nullptr, nullptr, nullptr, 0);
   const int rem = a.rem[seg];
   if (rem > 0) {   // 16 lanes per row
     const int cols_per_wg = ML_WAVES / wpc, sub = threadIdx.x & 15;
@@ -533,36 +568,50 @@ static int ml_check(const char* who, const fc_kv_view* src, const fc_kv_view* ds
   return FC_OK;
 }
 
-// How many wavefronts share a column, and how many workgroups of a (layer, plane) walk its column groups.  One
-// workgroup fills a compute unit (its LDS), so what counts is rounds of workgroups times iterations of each, plus the
-// start: loading the weights, about 0.4 of an iteration, 0.7 with resident W1 (whose workgroups may walk several groups
-// for one start).  The launch is bound by memory: with streamed W1 four fifths of the compute units keep it as busy as
-// all of them, so a last round that is not full costs what it holds, but no less than 0.8 (with resident W1, whose
-// workgroups do not wait for each other's chunks, a whole round: 45 sequences of 640 tokens in 15 walks a layer instead
-// of 8 took 2 % longer).  Of equal splits the one with fewer wavefronts per column, which wait for each other at every
-// store.  us per pass, as many wavefronts as make 1024 workgroups -> this split: 28 layers of 4 heads, factor 5,
-// 16 sequences of 700 tokens 424 -> 323, of 3000 1051 -> 935, of 16384 4331 -> 4223, 8 of 8000 1326 -> 1191, 3 of 3000
-// 313 -> 266; factor 2, 16 of 700 428 -> 314, 8 of 700 246 -> 205; 32 layers of 32 heads, factor 2, 1 of 1100
-// 442 -> 319, 2 of 640 416 -> 325, 4 of 1500 1299 -> 1210, 12 and more the same.
-struct MlSplit { int wpc, gx; };
+// How many heads make a column (1 << hsh), how many wavefronts share one, and how many workgroups of a (layer, plane) walk
+// its column groups.  One workgroup fills a compute unit (its LDS), so what counts is rounds of workgroups times iterations
+// of each, plus the start: loading the weights, about 0.4 of an iteration, 0.7 with resident W1, whose workgroups may walk
+// several groups for one start and lose 0.25 between two of them (tables, first rows).  The launch is bound by memory: seven
+// eighths of the compute units keep it as busy as all of them, so a last round that is not full costs what it holds, but no
+// less than 0.85.  Of equal splits the one with fewer wavefronts per column, which wait for each other at every store.
+// Heads in one column make columns of more rows, so that fewer rows of the last iteration are idle and fewer groups are
+// walked; what a wavefront reads and writes is a contiguous piece of the page whichever way.  us per launch, one head
+// per column -> this split: 32 layers of 32 heads, factor 2, 45 sequences of 576 tokens 2080 -> 2017, of 64 322 -> 287;
+// 3 of 576 178 -> 158, of 64 36 -> 30; factor 5, 20 of 576 886 -> 863, of 524 855 -> 769; 28 layers of 4 heads, factor 5,
+// 16 of 16384 2090 -> 2050, of 700 114 -> 113; factor 2, 16 of 8000 1271 -> 1153.
+//
+// Sequences of different lengths (`rag`): a workgroup takes one group, the longest sequences' groups start first, and the
+// compute units are busy until about half a group's time before the end; no split ends before its longest column does.
+// Lengths are on the device: columns are taken to be two thirds of the longest on average (a third to the whole of it).
+// Of equal splits the one with more heads per column.  us per launch, as many wavefronts as make 1024 workgroups in the
+// order of the batch -> this: 28 layers of 4 heads, factor 5, 16 sequences of 5461 to 16384 tokens 1680 -> 1455, 5 of 2666
+// to 8000 331 -> 284, 9 of 700 to 2100 163 -> 131, 16 of 300 to 900 164 -> 125; factor 2, 16 of 3000 to 9000 1342 -> 920, 16 of
+// 300 to 900 158 -> 120; 32 layers of 32 heads, factor 5, 20 of 14 to 824 870 -> 658, factor 2 854 -> 793.
+struct MlSplit { int hsh, wpc, gx; };
 template <typename Fits>
-static MlSplit ml_split(int ncols, int jobs, int c, int cf, Fits fits) {
-  const int64_t ncu = fc_compute_units();
-  const double least = cf <= 2 ? 1.0 : 0.8;
-  MlSplit best{ML_WAVES, ncols};      // what is left when no split fits
+static MlSplit ml_split(int batch, int heads, int max_hsh, int jobs, int c, int cf, bool rag, Fits fits) {
+  const double ncu = fc_compute_units();
+  MlSplit best{0, ML_WAVES, batch * heads};      // what is left when no split fits
   double best_cost = -1.0;
-  for (int wpc = 1; wpc <= ML_WAVES && (wpc == 1 || ML_ROWS * wpc < 2 * c); wpc *= 2) {
-    if (!fits(wpc)) continue;
-    const int cpw = ML_WAVES / wpc, groups = (ncols + cpw - 1) / cpw, iters = (c + ML_ROWS * wpc - 1) / (ML_ROWS * wpc);
-    for (int per = 1; per <= groups && per <= (cf <= 2 ? 64 : 1); ++per) {
-      const int g = (groups + per - 1) / per;
-      const int64_t wgs = (int64_t)g * jobs, left = wgs % ncu;
-      const double part = (double)left / (double)ncu;
-      const double rounds = (double)(wgs / ncu) + (left == 0 ? 0.0 : part > least ? part : least);
-      const double cost = rounds * ((double)((groups + g - 1) / g) * iters + (cf <= 2 ? 0.7 : 0.4));
-      if (best_cost < 0 || cost < best_cost) {
-        best_cost = cost;
-        best = {wpc, g};
+  for (int i = 0; i <= max_hsh; ++i) {
+    const int hsh = rag ? max_hsh - i : i;
+    const int per_seq = heads >> hsh, ncols = batch * per_seq;
+    const int64_t rows = (int64_t)c << hsh;
+    for (int wpc = 1; wpc <= ML_WAVES && (wpc == 1 || ML_ROWS * wpc < 2 * rows); wpc *= 2) {
+      if (!fits(wpc)) continue;
+      const int cpw = ML_WAVES / wpc, groups = (ncols + cpw - 1) / cpw;
+      const double most = (double)((rows + ML_ROWS * wpc - 1) / (ML_ROWS * wpc));
+      const double iters = rag ? 0.67 * (double)rows / (ML_ROWS * wpc) + 0.5 : most;
+      for (int per = 1; per <= groups && per <= (cf <= 2 && !rag ? 64 : 1); ++per) {   // groups a workgroup walks
+        const int g = (groups + per - 1) / per;
+        const double wgs = (double)g * jobs / ncu, whole = floor(wgs), part = wgs - whole;
+        const double one = cf <= 2 ? (double)((groups + g - 1) / g) * (iters + 0.25) + 0.7 : iters + 0.4;
+        const double rounds = whole + (part <= 0.0 ? 0.0 : part > 0.85 ? part : 0.85);
+        const double cost = !rag ? rounds * one : fmax(one - iters + most, wgs * one + 0.5 * iters);
+        if (best_cost < 0 || cost < best_cost) {
+          best_cost = cost;
+          best = {hsh, wpc, g};
+        }
       }
     }
   }
@@ -575,35 +624,20 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
                      int seg_start, int c, int dst_start, const int32_t* seg_start_v, const int32_t* seg_len_v,
                      const int32_t* dst_start_v, int min_rows, hipStream_t st) {
   const bool rag = seg_len_v != nullptr;
-  const int ncols = src->batch * src->num_kv_heads;
-  int wpc = 1, gx = 0;
-  if (!rag) {
-    const auto tables_fit = [&](int wpc_) {     // in LDS, else every row waits for its entry
-      const int cap = ML_TBLTOT / (ML_WAVES / wpc_);
-      const auto fit = [&](const fc_kv_view* v, int64_t last) { return !v->block_tables || v->block_size <= 0 || last / v->block_size < cap; };
-      return fit(src, (int64_t)seg_start + (int64_t)c * cf - 1) && fit(dst, (int64_t)dst_start + c - 1);
-    };
-    const MlSplit sp = ml_split(ncols, src->num_layers, c, cf, tables_fit);
-    wpc = sp.wpc;
-    gx = sp.gx;
-  } else {
-    // Sequences of different lengths: many small workgroups, or the longest sequence would decide (5 of 2666 to 8000
-    // tokens: 794 us per pass, 961 with the split by the largest row count).
-    while (wpc < ML_WAVES && (int64_t)ncols * wpc / ML_WAVES * src->num_layers < 1024 && ML_ROWS * wpc * 2 <= c) wpc *= 2;
-    const int groups = (ncols * wpc + ML_WAVES - 1) / ML_WAVES, ncu = fc_compute_units();
-    const double t_group = 1.5 * ((c + ML_ROWS * wpc - 1) / (ML_ROWS * wpc)) * (cf + 2), t_start = 4.0;   // microseconds, roughly
-    gx = groups;
-    double best = -1.0;
-    for (int per = 1; cf <= 2 && per <= groups && per <= 64; ++per) {
-      const int g = (groups + per - 1) / per;
-      const long long rounds = ((long long)g * src->num_layers + ncu - 1) / ncu;
-      const double cost = (double)rounds * (((groups + g - 1) / g) * t_group + t_start);
-      if (best < 0 || cost < best) {
-        best = cost;
-        gx = g;
-      }
-    }
-  }
+  // heads whose rows of a token lie side by side, in both views, may share a column
+  int max_hsh = 0;
+  if (src->stride_head < src->stride_token && dst->stride_head < dst->stride_token && src->stride_token < (1 << 24) &&
+      dst->stride_token < (1 << 24))
+    while (max_hsh < 5 && src->num_kv_heads % (2 << max_hsh) == 0 && c < (1 << 29) >> max_hsh) ++max_hsh;
+  const auto tables_fit = [&](int wpc_) {     // in LDS, else every row waits for its entry
+    const int cap = ML_TBLTOT / (ML_WAVES / wpc_);
+    const auto fit = [&](const fc_kv_view* v, int64_t last) { return !v->block_tables || v->block_size <= 0 || last / v->block_size < cap; };
+    return rag ? fit(src, src->max_seq_len - 1) && fit(dst, dst->max_seq_len - 1)
+               : fit(src, (int64_t)seg_start + (int64_t)c * cf - 1) && fit(dst, (int64_t)dst_start + c - 1);
+  };
+  const MlSplit sp = ml_split(src->batch, src->num_kv_heads, max_hsh, src->num_layers, c, cf, rag, tables_fit);
+  const int hsh = sp.hsh, wpc = sp.wpc, gx = sp.gx;
+  const int ncols = src->batch * (src->num_kv_heads >> hsh);
   const int cols_per_wg = ML_WAVES / wpc, ncg = (ncols + cols_per_wg - 1) / cols_per_wg;
   dim3 grid(gx, src->num_layers);
   const size_t lds = ML_LDS;
@@ -623,7 +657,7 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
     FC_ALLOW_LDS((mlp_kernel<DT, ST, DTT, WR, RG>), (int)lds);                                                    \
     hipLaunchKernelGGL((mlp_kernel<DT, ST, DTT, WR, RG>), grid, dim3(ML_THREADS), lds, st, s, d, (const char*)w->w1, \
                        (const char*)w->b1, (const char*)w->w2, (const char*)w->b2, (const char*)w->w3,             \
-                       (const char*)w->b3, cf, seg_start, c, dst_start, wpc, ncols, ncg, seg_start_v, seg_len_v,   \
+                       (const char*)w->b3, cf, seg_start, c, dst_start, hsh, wpc, ncols, ncg, seg_start_v, seg_len_v,   \
                        dst_start_v, min_rows);                                                                     \
   } while (0)
 #define ML_DISPATCH(DT, WR)                                                         \

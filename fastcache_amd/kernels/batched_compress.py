@@ -129,14 +129,22 @@ class BatchedGEMMCompressor(nn.Module):
             mk = lambda xs: _lib.upload_ints(xs, kv_cache)
             imgs = [min(int(it_len[0]), n) if it_len[0] > 0 else 0 for n in host_lens]
             dsts = [0] * len(imgs)
+            plan = []      # all uploads before the first launch: one that is refused leaves the cache as it was
             for starts, counts, seg in (([0] * len(imgs), imgs, "i"), (imgs, [n - i for n, i in zip(host_lens, imgs)], "t")):
                 if max(counts) == 0:
                     continue
-                st, ct, dt = mk(starts), mk(counts), mk(dsts)
-                for view, dview, kind in ((views[0], dviews[0], "k"), (views[1], dviews[1], "v")):
-                    ops.ccm_mlp_ragged(view, dview, self._weights(seg + kind, kv_cache.dtype, dev, (l0, l1)), cf, st, ct,
-                                       dt, max(counts), self.min_seq_len)
+                where = (starts, counts, dsts)
+                # a segment that is the same for all sequences (the image) is the uniform call
+                same = all(len(set(xs)) == 1 for xs in where) and counts[0] // cf >= self.min_seq_len
+                plan.append((seg, max(counts), [xs[0] for xs in where] if same else [mk(xs) for xs in where], same))
                 dsts = [d + self._seg_len(n) for d, n in zip(dsts, counts)]
+            for seg, n_max, (st, ct, dt), same in plan:
+                for view, dview, kind in ((views[0], dviews[0], "k"), (views[1], dviews[1], "v")):
+                    w = self._weights(seg + kind, kv_cache.dtype, dev, (l0, l1))
+                    if same:
+                        ops.ccm_mlp(view, dview, w, cf, st, ct, dt)
+                    else:
+                        ops.ccm_mlp_ragged(view, dview, w, cf, st, ct, dt, n_max, self.min_seq_len)
             return dsts
         for s0, n, seg in ((0, img, "i"), (img, seq_len - img, "t")):
             if n == 0:

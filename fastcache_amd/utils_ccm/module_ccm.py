@@ -214,11 +214,14 @@ class _CCMBase(nn.Module):
 
     def _paged_forward_ragged(self, views, dviews, lens: List[int], it_len, layer_range, kv_cache) -> List[int]:
         """One launch set for sequences of different lengths: per segment of the class's split rule, the
-        sequences' (start, length, destination) go to the device as three small int32 tensors."""
+        sequences' (start, length, destination) go to the device as three small int32 tensors.  A segment that is the
+        same for all of them (the image in front of texts of different lengths) is the uniform call, whose launch need
+        not provide for different lengths (20 sequences of 32 layers x 32 heads x 576 tokens, factor 2: 880 us, 950)."""
         cf, (l0, l1) = self.compression_factor, layer_range
         dev = kv_cache.device
         per_seq = [self._paged_segments(n, it_len) for n in lens]
         dst = [0] * len(lens)
+        plan = []      # all uploads before the first launch: one that is refused leaves the cache as it was
         for j in range(max(len(p) for p in per_seq)):
             segs = [p[j] if j < len(p) else (p[-1][0], p[-1][1], 0, 0) for p in per_seq]
             gk, gv = segs[0][0], segs[0][1]
@@ -228,11 +231,17 @@ class _CCMBase(nn.Module):
             if n_max == 0:
                 continue
             mk = lambda xs: _lib.upload_ints(xs, kv_cache)
-            starts, counts, dsts = mk([g[2] for g in segs]), mk([g[3] for g in segs]), mk(dst)
+            where = [[g[2] for g in segs], [g[3] for g in segs], dst]
+            same = all(len(set(xs)) == 1 for xs in where) and n_max // cf >= self.min_seq_len
+            plan.append((gk, gv, n_max, [xs[0] for xs in where] if same else [mk(xs) for xs in where], same))
+            dst = [d + self._segment_len(g[3]) for d, g in zip(dst, segs)]
+        for gk, gv, n_max, (starts, counts, dsts), same in plan:
             for view, dview, g in ((views[0], dviews[0], gk), (views[1], dviews[1], gv)):
                 w = self._layer_weights(g, l0, l1, kv_cache.dtype, dev)
-                ops.ccm_mlp_ragged(view, dview, w, cf, starts, counts, dsts, n_max, self.min_seq_len)
-            dst = [d + self._segment_len(g[3]) for d, g in zip(dst, segs)]
+                if same:
+                    ops.ccm_mlp(view, dview, w, cf, starts, counts, dsts)
+                else:
+                    ops.ccm_mlp_ragged(view, dview, w, cf, starts, counts, dsts, n_max, self.min_seq_len)
         return dst
 
     def _forward_layers(self, kv_cache: Sequence[LayerKV], segments) -> Optional[List[LayerKV]]:

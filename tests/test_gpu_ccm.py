@@ -293,3 +293,37 @@ def test_ccm_mlp_is_the_same_however_columns_are_split(dev, L, B, S, block_size,
         one = _lib.paged_view(alone, tables[b:b + 1], None, S)
         ops.ccm_mlp(one, one, w, cf, 0, S, 0)
     assert torch.equal(pool.view(torch.int16), alone.view(torch.int16))
+
+
+@pytest.mark.parametrize("L,H,lens,block_size,cf", [
+    (2, 6, [333, 70, 333, 2, 211], 256, 2),                       # two heads a column (6 = 2 x 3), equal lengths, one row
+    (2, 3, [333, 70, 5, 64], 256, 5),                             # an odd number of heads; a sequence of one row
+    (28, 4, [900, 300, 611, 4, 899, 45, 702], 256, 5),            # four heads a column, eight wavefronts share it
+    (28, 4, [5000, 1700, 3001], 256, 5),                          # a head a column, eight wavefronts share it
+    (8, 32, [640, 590, 1100, 777], 256, 2),                       # heads by the dozen, resident W1
+    (1, 4, [64 + 7 * i % 131 for i in range(70)], 32, 3),         # more sequences than a wavefront has lanes
+    (1, 2, [20 + i % 37 for i in range(260)], 32, 2),             # more than are put in order
+    (1, 2, [25000, 300], 32, 5),                                  # block tables that do not fit
+])
+def test_ccm_mlp_ragged_is_each_sequence_alone(dev, L, H, lens, block_size, cf):
+    """Sequences of different lengths in one launch, longest first, heads sharing columns: the same bytes as every
+    sequence by a uniform call of its own."""
+    B, per = len(lens), -(-max(lens) // block_size)
+    pool = torch.empty((L, B * per + 1, block_size, H, 128), dtype=torch.float16, device=dev).normal_()
+    tables = torch.randperm(B * per + 1, device=dev)[:B * per].view(B, per).int().contiguous()
+    w = tuple((torch.randn(shape, device=dev) * 0.05).half()
+              for shape in ((L, 128, 128 * cf), (L, 128), (L, 128, 128), (L, 128), (L, 128, 128), (L, 128)))
+    alone = pool.clone()
+    mk = lambda xs: torch.tensor(xs, dtype=torch.int32, device=dev)
+    starts = [n // 3 for n in lens]
+    counts = [n - s for n, s in zip(lens, starts)]
+    dsts = [s // 2 for s in starts]
+    view = _lib.paged_view(pool, tables, mk(lens), max(lens))
+    ops.ccm_mlp_ragged(view, view, w, cf, mk(starts), mk(counts), mk(dsts), max(counts), 1)
+    for b in range(B):
+        one = _lib.paged_view(alone, tables[b:b + 1], None, max(lens))
+        if counts[b] >= cf:
+            ops.ccm_mlp(one, one, w, cf, starts[b], counts[b], dsts[b])
+        else:
+            ops.copy_tokens(one, one, starts[b], counts[b], dsts[b])
+    assert torch.equal(pool.view(torch.int16), alone.view(torch.int16))
