@@ -187,10 +187,15 @@ def refuse_capture() -> None:
         raise FastcacheError("numbers held by the host cannot be uploaded while a graph is being captured")
 
 
-def upload_ints(values, ref: torch.Tensor) -> torch.Tensor:
-    """A list of Python ints as an int32 tensor on the device of ``ref``, through pinned memory and without waiting."""
+def upload_rows(rows, ref: torch.Tensor):
+    """Lists of Python ints as int32 tensors on the device of ``ref``: one copy, through pinned memory and without waiting."""
     refuse_capture()
-    return host().upload_tables([], (list(values),), ref)[1]
+    return host().upload_tables([], tuple([r if type(r) is list else list(r) for r in rows]), ref)[1:]
+
+
+def upload_ints(values, ref: torch.Tensor) -> torch.Tensor:
+    """... of one list"""
+    return upload_rows((values,), ref)[0]
 
 
 _enqueued = 0

@@ -86,7 +86,7 @@ class PagedKVRunner:
 
     def _table_and_lens(self, tables: Seq[Seq[int]], lens: Seq[int]):
         _lib.refuse_capture()
-        return _lib.host().upload_tables([list(t) for t in tables], (list(lens),), self.kv_cache)
+        return _lib.host().upload_tables([t if type(t) is list else list(t) for t in tables], (list(lens),), self.kv_cache)
 
     # -- paged <-> HuggingFace layout ----------------------------------------------------------------
     def _extract_kv_cache_fast(self, block_table: List[int], seq_len: int) -> List[LayerKV]:
@@ -145,7 +145,14 @@ class PagedKVRunner:
         such pages); without one, a batch whose tables name a page twice where it would be rewritten is refused.
         Runs before any row is rewritten; returns the number of pages copied."""
         bm = self.block_manager
-        writes = [self._pages_rewritten(comp, len(s), [image_len, max(1, len(s) - image_len)]) for s in seqs]
+        by_len: Dict[int, int] = {}        # sequences of one length rewrite the same number of pages
+        writes = []
+        for s in seqs:
+            n = len(s)
+            w = by_len.get(n)
+            if w is None:
+                w = by_len[n] = self._pages_rewritten(comp, n, [image_len, max(1, n - image_len)])
+            writes.append(w)
         if bm is None:
             owners: Dict[int, int] = {}
             for s in seqs:

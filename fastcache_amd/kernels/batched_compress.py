@@ -126,7 +126,6 @@ class BatchedGEMMCompressor(nn.Module):
         dviews = views if out is None else [_lib.dense_view(out[p][l0:l1]) for p in range(2)]
         if host_lens is not None and len(set(host_lens)) > 1:
             dev = kv_cache.device
-            mk = lambda xs: _lib.upload_ints(xs, kv_cache)
             imgs = [min(int(it_len[0]), n) if it_len[0] > 0 else 0 for n in host_lens]
             dsts = [0] * len(imgs)
             plan = []      # all uploads before the first launch: one that is refused leaves the cache as it was
@@ -136,7 +135,7 @@ class BatchedGEMMCompressor(nn.Module):
                 where = (starts, counts, dsts)
                 # a segment that is the same for all sequences (the image) is the uniform call
                 same = all(len(set(xs)) == 1 for xs in where) and counts[0] // cf >= self.min_seq_len
-                plan.append((seg, max(counts), [xs[0] for xs in where] if same else [mk(xs) for xs in where], same))
+                plan.append((seg, max(counts), [xs[0] for xs in where] if same else _lib.upload_rows(where, kv_cache), same))
                 dsts = [d + self._seg_len(n) for d, n in zip(dsts, counts)]
             for seg, n_max, (st, ct, dt), same in plan:
                 for view, dview, kind in ((views[0], dviews[0], "k"), (views[1], dviews[1], "v")):

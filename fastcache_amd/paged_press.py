@@ -8,6 +8,8 @@ of the same pages in place.  Three launches per pass, nothing leaves the device.
 """
 from __future__ import annotations
 
+import math
+from collections import namedtuple
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
 
@@ -36,6 +38,20 @@ def _views(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.T
             _lib.paged_view(kv_cache[1], block_tables, seq_lens, max_seq_len))
 
 
+# what ops.snapkv_press_fits reads of a key view
+_Geometry = namedtuple("_Geometry", "block_tables block_size max_seq_len stride_token num_kv_heads")
+
+
+def _press_rows(kv_cache, block_tables, seq_lens, seq_len, width, counts=None, order=None, snapkv=None) -> bool:
+    """The host module's call for callers that want the moved rows alone; False: not of the plain form, nothing done."""
+    if counts is not None:
+        _lib.refuse_capture()
+    if _lib.host().press_rows(kv_cache, block_tables, seq_lens, seq_len, width, counts, order, snapkv) is None:
+        return False
+    _lib.note_enqueued()
+    return True
+
+
 def _select_and_compact(kview, vview, scores, seq_lens, kept: List[int], compact: bool, heads: int) -> PressResult:
     """Top-k per (layer, sequence, head) row and in-place compaction; one launch each whether or not the
     sequences keep the same number of tokens.  (Both in one launch, ``ops.select_compact``, has half the workgroups for
@@ -61,7 +77,6 @@ def knorm_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq
     Python ints, ``seq_len`` their maximum), over sequences of different lengths in the same launches: each keeps
     ``int(its length * (1 - compression_ratio))`` tokens.  ``rows_only``: the caller wants the pages compacted and
     nothing else (scores and indices stay scratch)."""
-    kview, vview = _views(kv_cache, block_tables, seq_lens, seq_len)
     lens = list(host_lens) if host_lens is not None else [seq_len] * block_tables.shape[0]
     kept = [n_kept_for(n, compression_ratio) for n in lens]
     width = max(kept)
@@ -70,9 +85,14 @@ def knorm_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq
     # workgroups leave it half idle (us per pass, half kept: 112 columns of 1000 bf16 keys 46 -> 31, of 12000 309 -> 251, 288 of
     # 2000 106 -> 96, of 18000 1073 -> 935; from there on one launch wins: 576 of 2000 fp32 379 against 412, 1152 of 2000
     # 354 against 406).
-    columns = kview.num_layers * kview.batch * kview.num_kv_heads
-    if (compact and 0 < width and ops.press_column_fits(seq_len, width) and
-            2 * columns > 3 * _lib.compute_units(kv_cache.device)):
+    columns = kv_cache.shape[1] * block_tables.shape[0] * kv_cache.shape[-2] if kv_cache.is_cuda else 0
+    one_launch = (compact and 0 < width and ops.press_column_fits(seq_len, width) and
+                  2 * columns > 3 * _lib.compute_units(kv_cache.device))
+    if one_launch and rows_only and _press_rows(kv_cache, block_tables, seq_lens, seq_len, width,
+                                                None if len(set(kept)) == 1 else kept):
+        return None
+    kview, vview = _views(kv_cache, block_tables, seq_lens, seq_len)
+    if one_launch:
         if len(set(kept)) == 1:
             scores, idx = ops.knorm_press(kview, vview, width, kv_cache.device)
             return PressResult(idx, width, scores)
@@ -92,7 +112,6 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
     the same launches.  ``queries`` are the rotated window queries ``[L, B, Hq, W, D]`` (the last W positions of
     every sequence).  With ``window_in_budget`` (kvpress) the observation window counts towards ``n_kept``;
     otherwise it is kept on top of it.  ``rows_only``: the caller wants the pages compacted and nothing else."""
-    kview, vview = _views(kv_cache, block_tables, seq_lens, seq_len)
     lens = list(host_lens) if host_lens is not None else [seq_len] * block_tables.shape[0]
     kept = [n_kept_for(n, compression_ratio) for n in lens]
     if not window_in_budget:
@@ -112,6 +131,18 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
     # 112 columns of 4096 keys 295 -> 193, of 1000 94 -> 73, 320 of 12000 1721 -> 1341, 288 of 8192 623 -> 583; whole columns
     # 576 of 2000 281 against 306, 896 of 4096 736 against 812).
     hq = queries.shape[-3]
+    H = kv_cache.shape[-2]
+    if (rows_only and window_apart and queries.dim() == 5 and kv_cache.dim() == 6 and reduction in ("mean", "sum") and
+            window_size > 0 and H > 0 and hq % H == 0 and hq > 0):
+        shape = _Geometry(True, kv_cache.shape[3], seq_len, kv_cache.stride(3), H)
+        same = len(set(kept)) == 1 and len(set(lens)) == 1
+        order = sorted(range(len(lens)), key=lambda b: -lens[b]) if len(set(lens)) > 1 else None   # longest first
+        if _press_rows(kv_cache, block_tables, seq_lens, seq_len, width, None if same else kept, order,
+                       (queries, window_size, kernel_size, int(causal_window), 1.0 / math.sqrt(kv_cache.shape[5]),
+                        1.0 / (window_size * (hq // H)) if reduction == "mean" else 1.0,
+                        int(ops.snapkv_press_fits(shape, hq, window_size, width)))):
+            return None
+    kview, vview = _views(kv_cache, block_tables, seq_lens, seq_len)
     fits = window_apart and ops.snapkv_press_fits(kview, hq, window_size, width)
     if rows_only:
         one_launch = fits and ops.snapkv_select_splits(kview, hq, window_size) == 1

@@ -219,7 +219,8 @@ class _CCMBase(nn.Module):
         not provide for different lengths (20 sequences of 32 layers x 32 heads x 576 tokens, factor 2: 880 us, 950)."""
         cf, (l0, l1) = self.compression_factor, layer_range
         dev = kv_cache.device
-        per_seq = [self._paged_segments(n, it_len) for n in lens]
+        by_len = {n: self._paged_segments(n, it_len) for n in set(lens)}
+        per_seq = [by_len[n] for n in lens]
         dst = [0] * len(lens)
         plan = []      # all uploads before the first launch: one that is refused leaves the cache as it was
         for j in range(max(len(p) for p in per_seq)):
@@ -230,10 +231,9 @@ class _CCMBase(nn.Module):
             n_max = max(g[3] for g in segs)
             if n_max == 0:
                 continue
-            mk = lambda xs: _lib.upload_ints(xs, kv_cache)
-            where = [[g[2] for g in segs], [g[3] for g in segs], dst]
+            where = ([g[2] for g in segs], [g[3] for g in segs], dst)
             same = all(len(set(xs)) == 1 for xs in where) and n_max // cf >= self.min_seq_len
-            plan.append((gk, gv, n_max, [xs[0] for xs in where] if same else [mk(xs) for xs in where], same))
+            plan.append((gk, gv, n_max, [xs[0] for xs in where] if same else _lib.upload_rows(where, kv_cache), same))
             dst = [d + self._segment_len(g[3]) for d, g in zip(dst, segs)]
         for gk, gv, n_max, (starts, counts, dsts), same in plan:
             for view, dview, g in ((views[0], dviews[0], gk), (views[1], dviews[1], gv)):

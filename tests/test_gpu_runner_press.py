@@ -366,3 +366,37 @@ def test_host_numbers_are_not_uploaded_under_capture(dev):
     torch.cuda.synchronize()
     assert bool((x == 3).all())
     assert _lib.upload_ints([1, 2], x).tolist() == [1, 2]
+
+
+@pytest.mark.parametrize("press", ["knorm", "snapkv"])
+@pytest.mark.parametrize("L,H,hq,lens,planes", [
+    (3, 4, 8, [700], "whole"),                      # few columns: norms / key ranges, selection, compaction
+    (16, 4, 28, [333, 1200, 64, 901, 33, 500, 77, 1024], "whole"),     # ragged, one launch, sequences no longer than the window
+    (16, 4, 28, [600] * 8, "layers"),               # equal lengths; a slice of the pool's layers
+    (12, 8, 16, [900] * 5 + [899], "copied"),       # queries whose rows do not lie side by side: the general path
+])
+def test_rows_only_moves_the_rows_of_the_general_path(dev, press, L, H, hq, lens, planes):
+    """The host module's call against scores, indices and compaction as calls of their own: the same pool."""
+    torch.manual_seed(3)
+    B, W, per = len(lens), 32, -(-max(lens) // 256)
+    pool = torch.randn((2, L + 2, B * per + 1, 256, H, 128), device=dev).to(torch.bfloat16)
+    tables = torch.randperm(B * per + 1, device=dev)[:B * per].view(B, per).int().contiguous()
+    lens_d = torch.tensor(lens, dtype=torch.int32, device=dev)
+    queries = torch.randn((L, B, hq, W, 128), device=dev).to(torch.bfloat16)
+    if planes == "copied":
+        queries = queries.transpose(2, 3).contiguous().transpose(2, 3)
+    part = slice(1, L + 1) if planes == "layers" else slice(0, L)
+    got, want = pool.clone(), pool.clone()
+    for p, rows_only in ((got, True), (want, False)):
+        args = (p[:, part], tables, lens_d, max(lens))
+        host = lens if len(set(lens)) > 1 else None
+        if press == "knorm":
+            paged_press.knorm_compress_paged(*args, 0.4, host_lens=host, rows_only=rows_only)
+        else:
+            paged_press.snapkv_compress_paged(*args, queries, 0.4, window_size=W, host_lens=host, rows_only=rows_only)
+    for b, n in enumerate(lens):
+        rows = paged_press.n_kept_for(n, 0.4)
+        for i in range(-(-rows // 256)):
+            m = min(256, rows - i * 256)
+            page = int(tables[b, i])
+            assert torch.equal(got[:, :, page, :m].view(torch.int16), want[:, :, page, :m].view(torch.int16)), (b, i)
