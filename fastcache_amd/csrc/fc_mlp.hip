@@ -228,13 +228,8 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
   const int rows_per_iter = ML_ROWS * wpc;
   int n_iter = ((c_rows << hsh) + rows_per_iter - 1) / rows_per_iter;
   int q_total = n_iter * cf;      // W1 chunk q = (iteration q / cf, token kc = q % cf) sits in buffer q & 1
-  const char* sbase = nullptr;   // this lane's piece of token 0 of the column's first head, per column group
+  const char* sbase = nullptr;   // this lane's piece of token 0 of its head, per column group
   char* dbase = nullptr;
-  // the heads of this lane's two rows on the memory side: rows advance by multiples of 32, so they stay the same
-  const int hmask = (1 << hsh) - 1;
-  const int sho[2] = {(lq & hmask) * (int)src.stride_head * 2, ((16 + lq) & hmask) * (int)src.stride_head * 2};
-  const int dho[2] = {(lq & hmask) * (int)dst.stride_head * 2, ((16 + lq) & hmask) * (int)dst.stride_head * 2};
-
   // X rows of chunk q: xf[2*c4 + rh] holds bytes [64*c4 + 16*lp, +16) of the token row of output row 16*rh + lq
   auto x_load = [&](uint4 (&xf)[8], int q) {
     const int it = q / cf, kc = q - it * cf;
@@ -254,7 +249,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
       long long off = src_off(tok);
       off = off < 0 ? 0 : off;
 #pragma unroll
-      for (int c4 = 0; c4 < 4; ++c4) xf[c4 * 2 + rh] = *reinterpret_cast<const uint4*>(sbase + off * 2 + sho[rh] + c4 * 64);
+      for (int c4 = 0; c4 < 4; ++c4) xf[c4 * 2 + rh] = *reinterpret_cast<const uint4*>(sbase + off * 2 + c4 * 64);
     }
   };
   // Re-laying through this wavefront's 2 KB of LDS: rows of 64 bytes, the four 16-byte pieces of a row XOR-ed
@@ -359,7 +354,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
         const int r = (row0 + rh * 16 + lq) >> hsh;
         long long off = -1;
         if (col_ok && r < cr) off = dst_off(ds + r);
-        rowp[rh] = off >= 0 ? dbase + off * 2 + dho[rh] : nullptr;
+        rowp[rh] = off >= 0 ? dbase + off * 2 : nullptr;
       }
       // (a half-wave writes one 8-byte half per row, so rows that share a piece position in a bank window keep
       // their halves swapped: bit 3 xor bit 4 of the row number)
@@ -403,8 +398,9 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
     b = col_ok ? col / hg_per_seq : 0;
     h = col_ok ? (col - b * hg_per_seq) << hsh : 0;
     if constexpr (RAG) b = ml_ranked_sequence(seg_len_v, src.batch, b);
-    sbase = slayer + (long long)h * src.stride_head * 2 + lp * 16;
-    dbase = dlayer + (long long)h * dst.stride_head * 2 + lp * 16;
+    // a lane's two rows on the memory side are rows lq and 16 + lq of every 32, of one and the same head
+    sbase = slayer + (long long)(h + (lq & ((1 << hsh) - 1))) * src.stride_head * 2 + lp * 16;
+    dbase = dlayer + (long long)(h + (lq & ((1 << hsh) - 1))) * dst.stride_head * 2 + lp * 16;
     if constexpr (RAG) {
       // The sequence's own segment.  Numbers from device memory are cut to what the host validated: the views'
       // max_seq_len (which their block tables cover) and the launch's row bound.
@@ -624,11 +620,11 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
                      int seg_start, int c, int dst_start, const int32_t* seg_start_v, const int32_t* seg_len_v,
                      const int32_t* dst_start_v, int min_rows, hipStream_t st) {
   const bool rag = seg_len_v != nullptr;
-  // heads whose rows of a token lie side by side, in both views, may share a column
+  // heads whose rows of a token lie side by side, in both views, may share a column, up to 16 (a lane's two rows of every
+  // 32 are then of one head; 32 heads to a column were never the faster split)
   int max_hsh = 0;
-  if (src->stride_head < src->stride_token && dst->stride_head < dst->stride_token && src->stride_token < (1 << 24) &&
-      dst->stride_token < (1 << 24))
-    while (max_hsh < 5 && src->num_kv_heads % (2 << max_hsh) == 0 && c < (1 << 29) >> max_hsh) ++max_hsh;
+  if (src->stride_head < src->stride_token && dst->stride_head < dst->stride_token)
+    while (max_hsh < 4 && src->num_kv_heads % (2 << max_hsh) == 0 && c < (1 << 29) >> max_hsh) ++max_hsh;
   const auto tables_fit = [&](int wpc_) {     // in LDS, else every row waits for its entry
     const int cap = ML_TBLTOT / (ML_WAVES / wpc_);
     const auto fit = [&](const fc_kv_view* v, int64_t last) { return !v->block_tables || v->block_size <= 0 || last / v->block_size < cap; };
