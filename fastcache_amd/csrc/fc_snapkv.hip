@@ -37,6 +37,7 @@
 #define SK_TILEB (SK_KT * 256)  // LDS bytes per key tile (rows unpadded, 16-byte chunks XOR-swizzled)
 #define SK_NEG (-1.0e30f)  // "minus infinity" that stays finite under subtraction
 #define SK_TBL 1024        // block-table entries of one sequence cached in LDS
+#define SK_PIECES 16       // statistics of key ranges in registers at a time
 
 __device__ __forceinline__ float sk_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -424,9 +425,9 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
     const bool ok = rb_valid && qi + lrow < W;
     if constexpr (MODE == 1) {   // this piece's statistics of the query, in log2 units; done
       if (ok && lhalf == 0) {
-        float* pp = part + (((((long long)l * kv.batch + b) * Hq + (h * G + qg)) * W + qi + lrow) * nsplit + split) * 2;
-        pp[0] = mnew * c;
-        pp[1] = ll;
+        float2* pp = reinterpret_cast<float2*>(part) +
+                     ((((long long)l * kv.batch + b) * Hkv + h) * nsplit + split) * (G * W) + qg * W + qi + lrow;
+        *pp = make_float2(mnew * c, ll);
       }
       return;
     }
@@ -436,12 +437,29 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
               lse[((((long long)l * kv.batch + b) * Hq + (h * G + qg)) * W + qi + lrow)];
     if constexpr (MODE == 2) {
       if (!lse && ok) {   // the pieces' (max, sum) into the log-sum-exp, by every workgroup for its own queries
-        const float* pp = part + ((((long long)l * kv.batch + b) * Hq + (h * G + qg)) * W + qi + lrow) * nsplit * 2;
+        // (one piece after the other for all of a column's queries, so a wavefront reads 256 bytes at a time, and up to
+        // SK_PIECES pieces asked for at once: pairs of one query side by side, read one by one, were 13 of the launch's
+        // 20.6 us on 8 columns of 4096 keys in 32 pieces; the launch now takes 11.6)
+        const float2* pp = reinterpret_cast<const float2*>(part) +
+                           (((long long)l * kv.batch + b) * Hkv + h) * nsplit * (G * W) + qg * W + qi + lrow;
         const int used = (T + (T + nsplit - 1) / nsplit - 1) / ((T + nsplit - 1) / nsplit);   // pieces that had tiles
-        float M = SK_NEG;
-        for (int s = 0; s < used; ++s) M = fmaxf(M, pp[2 * s]);
-        float L = 0.f;
-        for (int s = 0; s < used; ++s) L += pp[2 * s + 1] * sk_exp2(pp[2 * s] - M);
+        float2 st[SK_PIECES];
+        auto fetch = [&](int s0) {
+#pragma unroll
+          for (int i = 0; i < SK_PIECES; ++i) st[i] = pp[(long long)min(s0 + i, used - 1) * (G * W)];
+        };
+        float M = SK_NEG, L = 0.f;
+        for (int s0 = 0; s0 < used; s0 += SK_PIECES) {
+          fetch(s0);
+#pragma unroll
+          for (int i = 0; i < SK_PIECES; ++i) M = fmaxf(M, st[i].x);     // past the last piece that one again
+        }
+        for (int s0 = 0; s0 < used; s0 += SK_PIECES) {
+          if (used > SK_PIECES) fetch(s0);
+#pragma unroll
+          for (int i = 0; i < SK_PIECES; ++i)
+            if (s0 + i < used) L += st[i].y * sk_exp2(st[i].x - M);
+        }
         nmfin = -1.4426950408889634f * ((M + __builtin_amdgcn_logf(L)) * 0.6931471805599453f);
       }
       if (row_max && split == 0 && tid == 0) row_max[((long long)l * kv.batch + b) * Hkv + h] = -INFINITY;
@@ -824,9 +842,10 @@ extern "C" int fc_snapkv_press_ordered(const fc_kv_view* keys, const fc_kv_view*
 //   ceil(columns * n / slots) * (tiles per range * a + f)
 // with a microseconds per 64-key tile and f per start, and n with the smallest sum is taken (whole columns do both
 // sweeps in one start).  Fitted to and checked against measurements (us for scoring + selection by n, window 64 unless
-// said): 8 columns x 1024 keys 46 / 32 / 26 / 23 for n = 1 / 2 / 4 / 8; 32 x 4096 154 / 90 / 60 / 48, 62 with 16;
-// 288 x 4096 254 / 228 / 220 / 248; 288 x 30011 1897 / 1572 / 1421 / 1387, 1466 with 16; 4 x 12000 (7 heads a group)
-// 667 / 342 / 194 / 123, 83 with 24; 448 x 3000 431 / 460 / 471; 256 x 2000 (window 32) 75 / 57 / 68.
+// said): 8 columns x 1000 keys 48 / 35 / 28 / 23 for n = 1 / 2 / 4 / 8; 8 x 4096 29 with 16, 28 with 32; 32 x 4096
+// 155 / 85 / 54 / 41, 44 with 16; 288 x 4096 253 / 223 / 220 / 234; 288 x 30011 1998 / 1521 / 1396 / 1368, 1408 with 16;
+// 4 x 12000 (7 heads a group) 671 / 334 / 185 / 111, 64 with 24, 58 with 32; 448 x 3000 (7 heads a group, window 32)
+// 228 / 242 / 244; 256 x 2000 75 / 57 / 67.
 // 1 also when the split kernels do not apply (more than 16 query row blocks per kv head, pages that are no multiple of
 // 64 tokens).
 extern "C" int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) {

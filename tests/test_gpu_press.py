@@ -605,6 +605,7 @@ def test_snapkv_scores_from_given_log_sum_exp(dev, dtype, Hq, Hkv, S, W, ksz, ca
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("Hq,Hkv,S,W,ksz,causal,splits", [(8, 2, 2000, 64, 7, True, 3), (8, 2, 2000, 64, 7, True, 31),
+                                                           (8, 2, 2000, 64, 7, True, 16), (4, 2, 2175, 64, 7, True, 17),
                                                            (14, 2, 1500, 48, 15, False, 4), (4, 1, 700, 64, 5, True, 2),
                                                            (16, 4, 1100, 32, 63, True, 5)])
 def test_snapkv_split_columns(dev, dtype, Hq, Hkv, S, W, ksz, causal, splits):
