@@ -298,13 +298,11 @@ PyObject* py_knorm_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::Tensor ok = at::empty({B, H, n, D}, k.options()), ov = at::empty({B, H, n, D}, k.options()), scores;
     const fc_kv_view kv = dense_view(k, 1, 0), vv = dense_view(v, 1, 0), dk = dense_view(ok, 1, 0), dv = dense_view(ov, 1, 0);
     // Short columns are scored by the workgroups that gather them, each for itself; longer ones by the whole chip first, in a
-    // launch and a tensor more.  us per hook, half kept, one launch against norms first, bf16 columns of 333 / 700 / 1000 keys
-    // (333: also fp32): 8 columns 11.2 11.0, 13.0 12.6, 15.3 12.9 (16.6 14.1); 32 of one prompt 11.2 17.4, 14.6 19.9,
-    // 18.9 20.6 (16.9 26.6); 32 of four 11.1 11.4, 14.6 13.1, 18.4 14.5; 256 16.9 21.4, 30.8 31.1, 41.7 38.5 (28.3 35.7); at
-    // 1500 to 4096 keys one launch takes 1.0 to 2.5 times as long.  What one launch spares is the norms' launch, which has a
-    // workgroup for every 16 tokens of all heads of a prompt: few for one prompt of many heads.
+    // launch and a tensor more.  us per hook, half kept, one launch against norms first, bf16 columns of 333 / 500 / 600 /
+    // 1000 keys: 8 columns 9.2 11.0, 10.4 11.1, 11.4 10.4, 14.4 11.0; 32 of one prompt 9.5 11.3, 10.8 10.9, 11.9 11.2, 17.7
+    // 12.1; 32 of four 9.5 11.3, 10.8 11.3, 12.3 11.9, 17.8 12.6; 256 16.3 17.0, 21.9 21.5, 26.2 25.3, 40.6 37.9.
     float* sp = nullptr;
-    if (S > 1024) {
+    if (S > 512) {
       scores = at::empty({B, H, S}, k.options().dtype(at::kFloat));
       sp = scores.data_ptr<float>();
     }

@@ -176,15 +176,23 @@ int fc_column_select(const char* who, int src, const fc_kv_view* keys, const fc_
     FC_ALLOW_LDS((column_select_kernel<SRC, DT, TH, KPT>), 120 * 1024);                                            \
     hipLaunchKernelGGL((column_select_kernel<SRC, DT, TH, KPT>), grid, dim3(TH), lds, st, kv, vv, dk, dv, a);       \
   } while (0)
-  // 1024 threads for the long rows, where lanes shorten the chain; 256 for short ones, where fewer wavefronts meet at the
-  // barriers; the longest rows with 512 again, two workgroups to a compute unit (288 rows are then one round, not two)
+  // Keys per thread as few as hold the row: the passes over them are unrolled, and keys that are not there still cost their
+  // share.  512 threads up to 4096 keys, 1024 for longer rows, where lanes shorten the chain, and 512 again for the longest,
+  // two workgroups to a compute unit (288 rows are then one round, not two).  us per hook, half kept, 256 threads of 2 keys
+  // up to 512, 512 of 8 up to 4096, 1024 of 16 up to 16384 -> this: Knorm, 8 columns of 333 keys 10.7 -> 9.2, of 500
+  // 12.5 -> 10.4, of 1000 (norms first) 11.9 -> 11.0, of 5000 22.3 -> 19.7, of 9000 28.1 -> 27.0; SnapKV, 8 of 1000
+  // 25.0 -> 23.6, 32 of 2000 35.2 -> 33.9, of 7000 81.8 -> 79.3.
 #define CS_SIZE(SRC, DT)                               \
-  if (n <= 512) CS_LAUNCH(SRC, DT, 256, 2);            \
+  if (n <= 512) CS_LAUNCH(SRC, DT, 512, 1);            \
+  else if (n <= 1024) CS_LAUNCH(SRC, DT, 512, 2);      \
+  else if (n <= 2048) CS_LAUNCH(SRC, DT, 512, 4);      \
   else if (n <= 4096) CS_LAUNCH(SRC, DT, 512, 8);      \
+  else if (n <= 8192) CS_LAUNCH(SRC, DT, 1024, 8);     \
+  else if (n <= 12288) CS_LAUNCH(SRC, DT, 1024, 12);   \
   else if (n <= 16384) CS_LAUNCH(SRC, DT, 1024, 16);   \
   else CS_LAUNCH(SRC, DT, 512, 72)
 #define CS_SIZE_SHORT(SRC, DT)                         \
-  if (n <= 512) CS_LAUNCH(SRC, DT, 256, 2);            \
+  if (n <= 512) CS_LAUNCH(SRC, DT, 512, 1);            \
   else CS_LAUNCH(SRC, DT, 512, 8)
 #define CS_DTYPE(SRC)                                                                                 \
   if (keys->dtype == FC_F32) { CS_SIZE(SRC, FC_F32); }                                                \
@@ -192,7 +200,7 @@ int fc_column_select(const char* who, int src, const fc_kv_view* keys, const fc_
   if (src == CS_SCORES) {
     CS_DTYPE(CS_SCORES);
   } else if (src == CS_SUMS) {
-    CS_SIZE(CS_SUMS, FC_F16);             // SnapKV scores fp16 / bf16 caches only
+    CS_SIZE(CS_SUMS, FC_F16);
   } else if (keys->dtype == FC_F32) {
     CS_SIZE_SHORT(CS_NORMS, FC_F32);
   } else if (keys->dtype == FC_BF16) {

@@ -783,7 +783,7 @@ def test_paged_press_ragged_batch_in_one_launch_set(dev, press):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("B,H,S", [(1, 3, 96), (2, 2, 512), (1, 2, 513), (1, 2, 1024), (1, 9, 1025), (1, 2, 4097), (1, 1, 16385),
+@pytest.mark.parametrize("B,H,S", [(1, 3, 96), (2, 2, 512), (1, 2, 513), (1, 2, 1024), (1, 9, 1025), (1, 2, 2048), (2, 2, 2049), (1, 2, 4097), (1, 1, 8193), (1, 1, 12289), (1, 1, 16385),
                                    (1, 1, 36864), (1, 1, 36865), (2, 9, 4097)])
 def test_layer_hooks_in_one_call(dev, dtype, B, H, S):
     """KnormPress and SnapKVPress on one layer's K and V (score, selection and gather as one native call) on both sides of
