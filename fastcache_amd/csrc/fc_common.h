@@ -266,3 +266,15 @@ __device__ __forceinline__ void fc_lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 #endif  // __HIPCC__
+
+// Division of 32-bit numbers below 2^31 by a number known at launch: a multiplication and a shift (Granlund and
+// Montgomery 1994, round-up method).
+struct FcDivisor {
+  unsigned d, mul, shift;
+  __device__ __forceinline__ unsigned quotient(unsigned n) const { return (__umulhi(n, mul) + n) >> shift; }
+};
+static inline FcDivisor fc_divisor(unsigned d) {
+  unsigned s = 0;
+  while ((1ull << s) < d) ++s;
+  return {d, (unsigned)((((1ull << s) - d) << 32) / d + 1), s};
+}

@@ -28,6 +28,7 @@
 // iteration are read before the workgroup barrier that precedes its stores, and later iterations
 // read tokens no earlier iteration writes.
 #include <math.h>
+#include <algorithm>
 #include "fc_common.h"
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -124,9 +125,13 @@ __device__ __forceinline__ int ml_ranked_sequence(const int* __restrict__ seg_le
 // RAG: every sequence has its own segment: seg_start_v / seg_len_v / dst_start_v [batch] in device memory; c_rows is
 // then the largest row count any sequence can have (it bounds the loops), and a sequence whose segment gives fewer
 // than min_rows rows is left to the copy kernel below.
+// FLAT (dense views that do not overlap, nothing to keep in order): there are no columns; the c_rows rows of all
+// (sequence, head) pairs are one list of `frows` rows, and the workgroups of a (layer, plane) take 256 of them in turn.
 // The body works on ONE layer of one plane: `slayer` / `dlayer` and the weight pointers carry the layer already; a
 // workgroup takes the column groups cg0, cg0 + cg_step, ... below ncg.
-template <int DTYPE, int SRC_T, int DST_T, bool W1R, bool RAG>
+struct MlFlat { unsigned rows; FcDivisor per_pair, heads; };
+
+template <int DTYPE, int SRC_T, int DST_T, bool W1R, bool RAG, bool FLAT = false>
 __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvView& dst, const char* slayer, char* dlayer,
                                          const char* __restrict__ w1l, const char* __restrict__ b1l,
                                          const char* __restrict__ w2l, const char* __restrict__ b2l,
@@ -134,7 +139,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
                                          int seg_start, int c_rows, int dst_start, int hsh, int wpc, int ncols, int ncg, int cg0,
                                          int cg_step, const int* __restrict__ seg_start_v,
                                          const int* __restrict__ seg_len_v, const int* __restrict__ dst_start_v,
-                                         int min_rows) {
+                                         int min_rows, MlFlat flat = MlFlat{}) {
   char* w1buf = lds;                       // 2 x ML_WBYTES
   char* w2buf = lds + 2 * ML_WBYTES;       // permuted
   char* w3buf = lds + 3 * ML_WBYTES;       // permuted
@@ -226,7 +231,15 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
   };
 
   const int rows_per_iter = ML_ROWS * wpc;
-  int n_iter = ((c_rows << hsh) + rows_per_iter - 1) / rows_per_iter;
+  // FLAT: this workgroup's share of the rows, 256 per iteration, the workgroups' turns interleaved
+  const int n_flat = FLAT ? ((int)((flat.rows + ML_ROWS * ML_WAVES - 1) / (ML_ROWS * ML_WAVES)) - cg0 + cg_step - 1) / cg_step : 0;
+  auto flat_row = [&](int it) { return (unsigned)(it * cg_step + cg0) * (ML_ROWS * ML_WAVES) + wave * ML_ROWS; };
+  auto flat_off = [&](const KvView& v, unsigned r, int start, int per, int kc) -> long long {
+    const unsigned pr = flat.per_pair.quotient(r), j = r - pr * flat.per_pair.d;
+    const unsigned bb = flat.heads.quotient(pr), hh = pr - bb * flat.heads.d;
+    return (long long)bb * v.stride_batch + (long long)hh * v.stride_head + (long long)(start + (int)j * per + kc) * v.stride_token;
+  };
+  int n_iter = FLAT ? n_flat : ((c_rows << hsh) + rows_per_iter - 1) / rows_per_iter;
   int q_total = n_iter * cf;      // W1 chunk q = (iteration q / cf, token kc = q % cf) sits in buffer q & 1
   const char* sbase = nullptr;   // this lane's piece of token 0 of its head, per column group
   char* dbase = nullptr;
@@ -240,6 +253,12 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
     // computed from them is never stored.
 #pragma unroll
     for (int rh = 0; rh < 2; ++rh) {
+      if constexpr (FLAT) {
+        const long long off = flat_off(src, min(flat_row(it) + rh * 16 + lq, flat.rows - 1), seg_start, cf, kc);
+#pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4) xf[c4 * 2 + rh] = *reinterpret_cast<const uint4*>(sbase + off * 2 + c4 * 64);
+        continue;
+      }
       int r = min((row0 + rh * 16 + lq) >> hsh, cr - 1);
       int tok = ss + cf * r + kc;
       if constexpr (RAG) {   // a column with no rows, or fewer than the launch's bound, reads some valid token
@@ -342,7 +361,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
     }
     // every wavefront of the column has consumed this iteration's source rows: stores may alias them
     // (a wavefront that owns its column alone is ordered by its own data dependences)
-    if (wpc > 1) __syncthreads();
+    if (!FLAT && wpc > 1) __syncthreads();
     {
       // The lane owns output row lrow and, per 32-feature block, features (i/4)*8 + lhalf*4 + i%4: four 8-byte
       // pieces go to the wavefront's LDS rows (64 bytes = one feature block of a row); read back in the
@@ -353,7 +372,12 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
       for (int rh = 0; rh < 2; ++rh) {
         const int r = (row0 + rh * 16 + lq) >> hsh;
         long long off = -1;
-        if (col_ok && r < cr) off = dst_off(ds + r);
+        if constexpr (FLAT) {
+          const unsigned fr = flat_row(it) + rh * 16 + lq;
+          if (fr < flat.rows) off = flat_off(dst, fr, dst_start, 1, 0);
+        } else if (col_ok && r < cr) {
+          off = dst_off(ds + r);
+        }
         rowp[rh] = off >= 0 ? dbase + off * 2 : nullptr;
       }
       // (a half-wave writes one 8-byte half per row, so rows that share a piece position in a bank window keep
@@ -394,11 +418,12 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
   for (int cg = cg0; cg < ncg; cg += cg_step) {
     if (cg != cg0) __syncthreads();   // every wavefront is done with the previous group's tables and W1 buffers
     col = cg * cols_per_wg + wave / wpc;
-    col_ok = col < ncols;
+    col_ok = FLAT || col < ncols;
     b = col_ok ? col / hg_per_seq : 0;
     h = col_ok ? (col - b * hg_per_seq) << hsh : 0;
     if constexpr (RAG) b = ml_ranked_sequence(seg_len_v, src.batch, b);
     // a lane's two rows on the memory side are rows lq and 16 + lq of every 32, of one and the same head
+    if constexpr (FLAT) b = h = 0;
     sbase = slayer + (long long)(h + (lq & ((1 << hsh) - 1))) * src.stride_head * 2 + lp * 16;
     dbase = dlayer + (long long)(h + (lq & ((1 << hsh) - 1))) * dst.stride_head * 2 + lp * 16;
     if constexpr (RAG) {
@@ -412,7 +437,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
       cr = min(min(cr, c_rows), dst.max_seq_len - ds);
       if (lane == 0) wave_rows[wave] = cr;
     }
-    fill_tables();
+    if (!FLAT) fill_tables();
     if (!W1R) {
       w1_load(0);
       w1_store(0);
@@ -434,7 +459,7 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
     }
     // the streaming variant is launched with one column group per workgroup (its groups are long, and the
     // loop would cost it registers it does not have)
-    if (!W1R) break;
+    if (!W1R || FLAT) break;
   }
 }
 
@@ -464,10 +489,14 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView sr
 // ---- a list of per-layer tensors, both planes and every segment in ONE launch ---------------------------------
 // A HuggingFace cache is a list of (K, V) tensors, one pair per layer; one prompt of it is little work per tensor (32
 // columns of 288 rows: 12 us of kernel), so what a launch per (layer, plane, segment) costs is the launches.  The
-// addresses travel in the kernel's arguments (no table upload).  blockIdx.y = (segment, plane, layer); each
-// segment has its own split of the columns, and a segment's remainder rows (or all rows of one too short to compress)
-// are copied behind its compressed rows by the same workgroup: source and destination are different tensors, so
-// nothing has to be ordered.
+// addresses travel in the kernel's arguments (no table upload).  blockIdx.y = (segment, plane, layer).  Source and destination
+// are different tensors, so nothing has to be ordered: the rows of all columns are one list (FLAT), which leaves no
+// wavefront without rows but in the last turn, needs no barrier at the stores and has neighbouring workgroups at
+// neighbouring rows; the remainder rows of a segment (or all rows of one too short to compress) are copied behind its
+// compressed rows by the same workgroups.  Bound by memory, at 4.4 to 5.1 TB/s.  us per forward, columns of a head each, split
+// over wavefronts and walked in groups -> this: 32 layers of 32 heads, factor 2, 2 prompts of 576 + 100 tokens 257 -> 249, 4 of
+// 576 + 47 453 -> 439, 8 of 576 + 1500 2836 -> 2808, one of 576 + 47 127 both; factor 5, 3 of 576 + 1000 753 -> 704; 28 layers of
+// 4 heads, factor 2, 2 of 3000 129 -> 124, 8 of 6000 920 -> 900; factor 5 the same.
 #define ML_LIST_LAYERS 64
 #define ML_LIST_SEGS 2
 struct MlpList {
@@ -475,7 +504,8 @@ struct MlpList {
   char* dst[2][ML_LIST_LAYERS];
   const char* w[ML_LIST_SEGS][2][6];            // [segment][plane]: w1, b1, w2, b2, w3, b3, all layers stacked
   int seg_start[ML_LIST_SEGS], c_rows[ML_LIST_SEGS], rem[ML_LIST_SEGS], dst_start[ML_LIST_SEGS];
-  int wpc[ML_LIST_SEGS], ncg[ML_LIST_SEGS], gx[ML_LIST_SEGS];
+  int gx[ML_LIST_SEGS];
+  MlFlat flat[ML_LIST_SEGS];
 };
 
 template <int DTYPE, bool W1R>
@@ -491,26 +521,23 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_list_kernel(KvVi
   const KvView& dst = p ? vdst : kdst;
   const char* slayer = a.src[p][l];
   char* dlayer = a.dst[p][l];
-  const int c = a.c_rows[seg], wpc = a.wpc[seg], ncg = a.ncg[seg];
+  const int c = a.c_rows[seg];
   const long long ll = l;
   if (c > 0)
-    mlp_body<DTYPE, 0, 0, W1R, false>(lds, src, dst, slayer, dlayer, a.w[seg][p][0] + ll * 128 * cf * 256,
-                                      a.w[seg][p][1] + ll * 256, a.w[seg][p][2] + ll * 128 * 256, a.w[seg][p][3] + ll * 256,
-                                      a.w[seg][p][4] + ll * 128 * 256, a.w[seg][p][5] + ll * 256, cf, a.seg_start[seg], c,
-                                      a.dst_start[seg], 0, wpc, ncols, ncg, blockIdx.x, gx, nullptr, nullptr, nullptr, 0);
+    mlp_body<DTYPE, 0, 0, W1R, false, true>(lds, src, dst, slayer, dlayer, a.w[seg][p][0] + ll * 128 * cf * 256,
+                                            a.w[seg][p][1] + ll * 256, a.w[seg][p][2] + ll * 128 * 256, a.w[seg][p][3] + ll * 256,
+                                            a.w[seg][p][4] + ll * 128 * 256, a.w[seg][p][5] + ll * 256, cf, a.seg_start[seg], c,
+                                            a.dst_start[seg], 0, 1, ncols, 0x7fffffff, blockIdx.x, gx, nullptr, nullptr, nullptr, 0,
+                                            a.flat[seg]);
   const int rem = a.rem[seg];
   if (rem > 0) {   // 16 lanes per row
-    const int cols_per_wg = ML_WAVES / wpc, sub = threadIdx.x & 15;
-    const int s0 = a.seg_start[seg] + c * cf, d0 = a.dst_start[seg] + c;
-    for (int cg = blockIdx.x; cg < ncg; cg += gx) {
-      const int c0 = cg * cols_per_wg, rows = min(cols_per_wg, ncols - c0) * rem;
-      for (int i = threadIdx.x >> 4; i < rows; i += ML_THREADS / 16) {
-        const int col = c0 + i / rem, t = i - (i / rem) * rem;
-        const int b = col / src.num_kv_heads, h = col - b * src.num_kv_heads;
-        const long long so = (long long)b * src.stride_batch + (long long)h * src.stride_head + (long long)(s0 + t) * src.stride_token;
-        const long long dof = (long long)b * dst.stride_batch + (long long)h * dst.stride_head + (long long)(d0 + t) * dst.stride_token;
-        *reinterpret_cast<uint4*>(dlayer + dof * 2 + sub * 16) = *reinterpret_cast<const uint4*>(slayer + so * 2 + sub * 16);
-      }
+    const int sub = threadIdx.x & 15, s0 = a.seg_start[seg] + c * cf, d0 = a.dst_start[seg] + c;
+    for (int i = (int)blockIdx.x * (ML_THREADS / 16) + (threadIdx.x >> 4); i < ncols * rem; i += gx * (ML_THREADS / 16)) {
+      const int col = i / rem, t = i - col * rem;
+      const int b = col / src.num_kv_heads, h = col - b * src.num_kv_heads;
+      const long long so = (long long)b * src.stride_batch + (long long)h * src.stride_head + (long long)(s0 + t) * src.stride_token;
+      const long long dof = (long long)b * dst.stride_batch + (long long)h * dst.stride_head + (long long)(d0 + t) * dst.stride_token;
+      *reinterpret_cast<uint4*>(dlayer + dof * 2 + sub * 16) = *reinterpret_cast<const uint4*>(slayer + so * 2 + sub * 16);
     }
   }
 }
@@ -776,28 +803,20 @@ static int ml_list(const char* who, const void* const* k_layers, const void* con
       const void* ws[6] = {w.w1, w.b1, w.w2, w.b2, w.w3, w.b3};
       for (int i = 0; i < 6; ++i) a.w[s][p][i] = (const char*)ws[i];
     }
-    // How many wavefronts share a column and how many column groups a workgroup walks: the pair with the fewest
-    // rounds * (groups * time per group + start-up).  (With the last round counted as in ml_split: 0.92 to 1.03 times as
-    // fast, on the whole slower; the two segments share the launch, so a round of one is filled up by the other.)
-    const int ncu = fc_compute_units();
+    // Workgroups per (layer, plane): the fewest rounds times (iterations and the start, as in ml_split).
+    const double ncu = fc_compute_units();
+    const int64_t rows = (int64_t)ncols * c, turns = (rows + ML_ROWS * ML_WAVES - 1) / (ML_ROWS * ML_WAVES);
+    FC_REQUIRE(rows < (1LL << 31) && (int64_t)ncols * a.rem[s] < (1LL << 31), FC_EUNSUPPORTED, "%s: too many rows", who);
+    a.flat[s] = MlFlat{(unsigned)rows, fc_divisor(c > 0 ? c : 1), fc_divisor(k_src->num_kv_heads)};
     double best = -1.0;
-    a.wpc[s] = 1;
-    a.ncg[s] = (ncols + ML_WAVES - 1) / ML_WAVES;
-    a.gx[s] = a.ncg[s];
-    for (int wpc = 1; wpc <= ML_WAVES && (wpc == 1 || ML_ROWS * wpc < 2 * c); wpc *= 2) {
-      const int cpw = ML_WAVES / wpc, ncg = (ncols + cpw - 1) / cpw;
-      const int n_iter = (c + ML_ROWS * wpc - 1) / (ML_ROWS * wpc);
-      const double t_group = 1.5 * n_iter * (cf + 2), t_start = 4.0;
-      for (int per = 1; per <= ncg && per <= (cf <= 2 ? 64 : 1); ++per) {
-        const int g = (ncg + per - 1) / per;
-        const long long rounds = ((long long)g * lp + ncu - 1) / ncu;
-        const double cost = (double)rounds * (((ncg + g - 1) / g) * t_group + t_start);
-        if (best < 0 || cost < best) {
-          best = cost;
-          a.wpc[s] = wpc;
-          a.ncg[s] = ncg;
-          a.gx[s] = g;
-        }
+    a.gx[s] = (int)std::min<int64_t>(8, ((int64_t)ncols * a.rem[s] + 31) / 32);     // a segment that is copied whole
+    for (int64_t g = 1; g <= turns && (g == 1 || (double)(g * lp) <= 8.0 * ncu); ++g) {
+      const double wgs = (double)g * lp / ncu, whole = floor(wgs), part = wgs - whole;
+      const double rounds = whole + (part <= 0.0 ? 0.0 : part > 0.85 ? part : 0.85);
+      const double cost = rounds * ((double)((turns + g - 1) / g) + (cf <= 2 ? 0.7 : 0.4));
+      if (best < 0 || cost < best) {
+        best = cost;
+        a.gx[s] = (int)g;
       }
     }
     if (c + a.rem[s] > 0 && a.gx[s] > gmax) gmax = a.gx[s];

@@ -218,6 +218,8 @@ def test_ccm_mlp_ragged_clamps_device_side_numbers(dev):
     (torch.bfloat16, 2, 64, 63, 2, 2),      # text of one token passed through, one full 32-row tile
     (torch.float16, 5, 1285, 0, 1, 1),      # streamed W1, several wavefronts per column, last tile ragged
     (torch.float16, 1, 33, 1, 5, 1),        # factor 1: one row past a tile
+    (torch.float16, 2, 515, 0, 3, 1),       # 257 rows a head: turns of 256 rows cross heads and sequences
+    (torch.bfloat16, 3, 2 * 127 * 3, 127 * 3, 2, 1),   # two segments of 127 rows a head
 ])
 def test_ccm_forward_over_a_list_is_one_launch(dev, dtype, cf, S, img, B, min_seq_len):
     """The compressor module on a list of per-layer tensors (permuted views, as a runner's extraction hands out):
