@@ -994,7 +994,7 @@ static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_
   a.out_mul = out_scale / (float)kernel_size;
   a.indices = indices;
   a.index_stride = index_stride;
-  a.parts = out_k && !indices ? fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, k) : 0;
+  a.parts = out_k && !indices ? fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, keys->max_seq_len, k) : 0;
   if (nsplit > 1) {
     const float* raw = nullptr;
     if ((rc = snapkv_split_sums(who, keys, queries, lse, num_q_heads, window, kernel_size, causal_window, scale, stride,

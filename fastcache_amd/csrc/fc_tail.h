@@ -19,15 +19,19 @@ struct ColumnSelect {
 
 enum { CS_SCORES = 0, CS_SUMS = 1, CS_NORMS = 2 };
 #define CS_MAX_KEYS (512 * 72)   // keys of a column, held in registers
+#define CS_WIDE 4096               // longer columns are selected by 1024 threads
 #define CS_NORMS_MAX 4096         // columns that the gathering workgroups score themselves: their scores lie in LDS
 
 // Launches the selection for columns of at most keys->max_seq_len keys; the out views are read only when a.parts > 0.
 int fc_column_select(const char* who, int src, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
                      const fc_kv_view* out_v, ColumnSelect a, hipStream_t st);
 
-// workgroups per column for a gather: about two per compute unit in all, no share below 64 rows
-static inline int fc_gather_parts(long long cols, int k) {
-  long long p = (2 * fc_compute_units() + cols - 1) / cols;
+// Workgroups per column for a gather, no share below 64 rows: about two per compute unit in all; one where columns are long
+// enough to be selected by 1024 threads each (CS_WIDE), of which a compute unit holds one workgroup: what does not fit the
+// first round would select its column behind it.
+static inline int fc_gather_parts(long long cols, int n, int k) {
+  const long long ncu = fc_compute_units();
+  long long p = n > CS_WIDE ? ncu / cols : (2 * ncu + cols - 1) / cols;
   if (p > (k + 63) / 64) p = (k + 63) / 64;
   p = p < 1 ? 1 : p > 16 ? 16 : p;
   const int lds = (k + 8191) / 8192;      // a share's positions are in LDS, at most 32 KB of them

@@ -232,13 +232,17 @@ static int cs_check(const char* who, const fc_kv_view* keys, const fc_kv_view* v
 }
 
 // Whether a press into other tensors should select and gather in launches of their own.  The workgroups that gather a
-// column each select it as well; above 4096 keys that takes 1024 threads, one workgroup to a compute unit, and costs a
-// round for every compute units' worth of them.  us per hook, gather inside -> apart, 30 % dropped: 24 columns of 6000 keys
-// 48 -> 43, 96 of 6000 133 -> 118, of 12000 282 -> 241, 256 of 8000 419 -> 394; 8 of 12000 35 -> 40, 12 of 6000 27 -> 33 (one
-// round); at 4096 keys and less, where two and more share a compute unit, 96 of 4000 76 -> 77, 64 of 2000 29 -> 34.
+// column each select it as well; of columns of more than 4096 keys there is one round of them (fc_gather_parts), and what
+// they lose against a gather over the whole chip is the time the selection takes, with fewer rows in flight after it: apart
+// where a workgroup's share is large.  us per hook, gather inside -> apart: Knorm, 24 columns of 5000 keys, 350 rows a share
+// 30.7, 37.4; 64 of 8000, 1400 a share 91.8, 101.6; 128 of 8000, 2800 a share 210, 210; of 12000, 4200 a share 317, 309, 1200 a
+// share 160, 169; 192 of 5000, 3500 a share 200, 199; 256 of 8000, 1600 a share 205, 214, 5600 a share 417, 396; SnapKV, 24 of 7000
+// 60.5, 66.5, 128 of 7000 177, 187.  Shorter columns, two and more workgroups to a compute unit: 96 of 4000 76, 77, 64 of 2000
+// 29, 34.
 extern "C" int fc_press_gather_apart(int32_t columns, int32_t max_seq_len, int32_t k) {
-  if (columns <= 0 || k <= 0) return 0;
-  return max_seq_len > 4096 && (long long)columns * fc_gather_parts(columns, k) > fc_compute_units();
+  if (columns <= 0 || k <= 0 || max_seq_len <= CS_WIDE) return 0;
+  const int parts = fc_gather_parts(columns, max_seq_len, k);
+  return (long long)columns * parts > fc_compute_units() || (k + parts - 1) / parts > 2600;
 }
 
 extern "C" int fc_knorm_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
@@ -250,7 +254,7 @@ extern "C" int fc_knorm_press_into(const fc_kv_view* keys, const fc_kv_view* val
   if (k == 0 || keys->max_seq_len == 0) return FC_OK;
   ColumnSelect a{};
   a.k = a.index_stride = k;
-  a.parts = indices ? 0 : fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, k);
+  a.parts = indices ? 0 : fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, keys->max_seq_len, k);
   a.indices = indices;
   if (!scores) {   // the workgroups that select a column score it as well
     FC_REQUIRE(keys->max_seq_len <= CS_NORMS_MAX, FC_EUNSUPPORTED, "%s: columns of more than %d keys need a score buffer", who,

@@ -783,11 +783,12 @@ def test_paged_press_ragged_batch_in_one_launch_set(dev, press):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("B,H,S", [(1, 3, 96), (2, 2, 512), (1, 2, 513), (1, 2, 1024), (1, 9, 1025), (1, 2, 2048), (2, 2, 2049), (1, 2, 4097), (1, 1, 8193), (1, 1, 12289), (1, 1, 16385),
-                                   (1, 1, 36864), (1, 1, 36865), (2, 9, 4097)])
+@pytest.mark.parametrize("B,H,S", [(1, 3, 96), (2, 2, 512), (1, 2, 513), (1, 2, 1024), (1, 9, 1025), (1, 2, 2048), (2, 2, 2049),
+                                   (1, 2, 4097), (1, 1, 8193), (1, 1, 12289), (1, 1, 16385), (1, 1, 36864), (1, 1, 36865),
+                                   (2, 9, 4097), (3, 43, 4097)])
 def test_layer_hooks_in_one_call(dev, dtype, B, H, S):
     """KnormPress and SnapKVPress on one layer's K and V (score, selection and gather as one native call) on both sides of
-    every change of launch shape, the last one with selection and gather apart: the kept rows are those of the stable selection over the scores, in ascending order,
+    every change of launch shape, the last one also with selection and gather apart (4096 rows kept): the kept rows are those of the stable selection over the scores, in ascending order,
     and every byte is the source row's.  V rows carry their position, which gives the selection back."""
     g = torch.Generator().manual_seed(S)
     W, ksz = 32, 7
