@@ -694,7 +694,7 @@ struct Scratch {
 // press_rows(pool, tables, lens, max_len, width, counts or None, order or None, snapkv or None) -> True, or None (the
 // caller's general path then serves or refuses the arguments).  The kept rows of every column move to the front of its pages;
 // scores and indices are scratch.  counts: kept rows per sequence where they differ; order: the sequences, longest first.
-// snapkv = (queries, window, kernel_size, causal, scale, out_scale, fits): one launch where the shape fits one and cutting
+// snapkv = (queries, window, kernel_size, causal, scale, out_scale, fits, mean length): one launch where the shape fits one and cutting
 // the columns does not pay, else key ranges, selection and compaction; None: the Knorm press in one launch.  Views, scratch and uploads in Python cost 25 to 45 us before the launch,
 // with the GPU idle behind the last pass's synchronisation: 13 sequences of 200 to 2300 tokens (SnapKV, 28 layers) 500 -> 475 us.
 PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -718,7 +718,7 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     bool one = true;
     double scale = 0, out_scale = 0;
     if (args[7] != Py_None) {
-      if (!PyTuple_Check(args[7]) || PyTuple_GET_SIZE(args[7]) != 7) fail("press_rows: the SnapKV arguments are a tuple of seven");
+      if (!PyTuple_Check(args[7]) || PyTuple_GET_SIZE(args[7]) != 8) fail("press_rows: the SnapKV arguments are a tuple of eight");
       const auto item = [&](int i) { return PyTuple_GET_ITEM(args[7], i); };
       q = tensor(item(0), "queries");
       W = as_int(item(1));
@@ -732,7 +732,8 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
           q.size(0) != L || q.size(1) != B || q.size(3) != W || q.size(4) != D || W <= 0 || q.size(2) % H)
         Py_RETURN_NONE;
       hq = q.size(2);
-      nsplit = fc_snapkv_select_splits(&kv, (int32_t)hq, (int32_t)W);
+      nsplit = fits ? fc_snapkv_select_splits_ragged(&kv, (int32_t)hq, (int32_t)W, (int32_t)as_int(item(7)))
+                    : fc_snapkv_select_splits(&kv, (int32_t)hq, (int32_t)W);
       one = fits && nsplit == 1;
       if (!one && (S > 36864 || (hq / H) * ((W + 31) / 32) > 16)) Py_RETURN_NONE;
     }

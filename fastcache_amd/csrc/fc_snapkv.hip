@@ -848,16 +848,27 @@ extern "C" int fc_snapkv_press_ordered(const fc_kv_view* keys, const fc_kv_view*
 // 228 / 242 / 244; 256 x 2000 75 / 57 / 67.
 // 1 also when the split kernels do not apply (more than 16 query row blocks per kv head, pages that are no multiple of
 // 64 tokens).
-extern "C" int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) {
-  if (!keys || keys->num_kv_heads <= 0 || window <= 0) return 1;
-  const long long columns = (long long)keys->num_layers * keys->batch * keys->num_kv_heads;
-  const int blocks = (num_q_heads / keys->num_kv_heads) * ((window + 31) / 32);
-  const int tiles = (keys->max_seq_len + SK_KT - 1) / SK_KT;
+struct SkSplitShape { long long columns, slots; int tiles, blocks; double a, f; };
+static bool sk_split_shape(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, SkSplitShape& s) {
+  if (!keys || keys->num_kv_heads <= 0 || window <= 0) return false;
+  s.columns = (long long)keys->num_layers * keys->batch * keys->num_kv_heads;
+  s.blocks = (num_q_heads / keys->num_kv_heads) * ((window + 31) / 32);
+  s.tiles = (keys->max_seq_len + SK_KT - 1) / SK_KT;
   const bool paged_ok = !keys->block_tables || (keys->block_size >= SK_KT && (keys->block_size & (keys->block_size - 1)) == 0 &&
                                                 (keys->max_seq_len - 1) / keys->block_size < SK_TBL);
-  if (columns <= 0 || columns >= 1000 || blocks > 16 || !paged_ok) return 1;
-  const double a = blocks > 8 ? 1.7 : blocks > 4 ? 0.83 : 0.7, f = blocks > 8 ? 9.0 : 7.0;
-  const long long slots = (long long)fc_compute_units() * (blocks > 4 ? 1 : 2);
+  if (s.columns <= 0 || s.columns >= 1000 || s.blocks > 16 || !paged_ok) return false;
+  s.a = s.blocks > 8 ? 1.7 : s.blocks > 4 ? 0.83 : 0.7;
+  s.f = s.blocks > 8 ? 9.0 : 7.0;
+  s.slots = (long long)fc_compute_units() * (s.blocks > 4 ? 1 : 2);
+  return true;
+}
+
+extern "C" int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) {
+  SkSplitShape s;
+  if (!sk_split_shape(keys, num_q_heads, window, s)) return 1;
+  const long long columns = s.columns, slots = s.slots;
+  const int tiles = s.tiles;
+  const double a = s.a, f = s.f;
   int best_n = 1;
   double best = (double)((columns + slots - 1) / slots) * (2.0 * tiles * a + f);
   for (int n = 2; n <= 32 && n * 2 <= tiles; ++n) {
@@ -868,6 +879,27 @@ extern "C" int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q
     }
   }
   return best_n;
+}
+
+// Sequences of different lengths, where the rule above cuts columns of the longest length: whole columns end when the longest
+// does or, longest first, when all of the work is done; key ranges are cut from every column alike, so their launches are
+// as long as the mean, but selection and compaction become launches of their own (27 us).  Of lengths within a sixteenth of
+// the longest on average, and of long columns of four wavefronts, which move a column's rows slowly, the rule above stands.
+// us per pass, 60 % dropped, ranges -> whole columns: 28 layers of 4 heads (7 query heads, window 32), 5 sequences of 1125 to
+// 9000 keys 865 -> 705, 8 of 3000 to 9000 1615 -> 1365, 3 of 500 to 4000 344 -> 316, window 64, 7 of 1500 to 12000 2294 -> 2072;
+// 36 layers of 8 heads, 2 of 500 to 4000 466 -> 348, window 64, 2 of 625 to 5000 684 -> 502.
+extern "C" int32_t fc_snapkv_select_splits_ragged(const fc_kv_view* keys, int32_t num_q_heads, int32_t window,
+                                                  int32_t mean_len) {
+  const int32_t equal = fc_snapkv_select_splits(keys, num_q_heads, window);
+  SkSplitShape s;
+  if (equal == 1 || !sk_split_shape(keys, num_q_heads, window, s) || mean_len <= 0 ||
+      16LL * mean_len >= 15LL * keys->max_seq_len || (s.blocks <= 4 && s.tiles > 96))
+    return equal;
+  const double share = (double)s.columns / (double)s.slots, mean = (double)mean_len / SK_KT;
+  const double whole = fmax(2.0 * s.tiles * s.a + s.f, share * (2.0 * mean * s.a + s.f));
+  for (int n = 2; n <= 32 && n * 2 <= s.tiles; ++n)
+    if (2.0 * fmax(1.0, share * n) * (mean / n * s.a + s.f) + 27.0 < whole) return equal;
+  return 1;
 }
 
 extern "C" int64_t fc_snapkv_split_workspace_bytes(int32_t num_layers, int32_t batch, int32_t num_q_heads,

@@ -140,7 +140,7 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
         if _press_rows(kv_cache, block_tables, seq_lens, seq_len, width, None if same else kept, order,
                        (queries, window_size, kernel_size, int(causal_window), 1.0 / math.sqrt(kv_cache.shape[5]),
                         1.0 / (window_size * (hq // H)) if reduction == "mean" else 1.0,
-                        int(ops.snapkv_press_fits(shape, hq, window_size, width)))):
+                        int(ops.snapkv_press_fits(shape, hq, window_size, width)), sum(lens) // len(lens))):
             return None
     kview, vview = _views(kv_cache, block_tables, seq_lens, seq_len)
     fits = window_apart and ops.snapkv_press_fits(kview, hq, window_size, width)

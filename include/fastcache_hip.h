@@ -210,6 +210,9 @@ int fc_snapkv_score_split(const fc_kv_view* keys, const void* queries, const flo
  * (indices: as for fc_knorm_press_into).
  */
 int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q_heads, int32_t window);
+/* The same for a batch of sequences of different lengths whose columns, whole, start longest first
+ * (fc_snapkv_press_ordered): mean_len is the sequences' mean length, the view's max_seq_len their largest. */
+int32_t fc_snapkv_select_splits_ragged(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len);
 int64_t fc_snapkv_select_workspace_bytes(int32_t num_layers, int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
                                          int32_t window, int32_t max_seq_len, int32_t nsplit);
 int fc_snapkv_select(const fc_kv_view* keys, const void* queries, const float* lse, int32_t num_q_heads,

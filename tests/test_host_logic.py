@@ -536,3 +536,25 @@ def test_weights_of_sequentials_with_named_children():
     module.compress_tk[0] = Own(module.compress_tk[0])
     again = pack()
     assert pack() is again and torch.equal(again[0][0], plain[0][0]) and torch.equal(again[4][0], plain[4][0])
+
+
+def test_snapkv_splits_of_sequences_of_different_lengths():
+    """The ragged rule only ever takes back a cut that the rule for equal lengths makes: where the longest length is the
+    exception, whole columns; where lengths are nearly equal, or columns long and of four wavefronts, that rule stands."""
+    import ctypes
+    from fastcache_amd import _lib
+
+    def both(L, B, H, hq, S, W, mean):
+        v = _lib.FcKvView(num_layers=L, batch=B, num_kv_heads=H, max_seq_len=S, block_size=256, block_tables=1, stride_token=H * 128)
+        return (_lib.fn("fc_snapkv_select_splits")(ctypes.byref(v), hq, W),
+                _lib.fn("fc_snapkv_select_splits_ragged")(ctypes.byref(v), hq, W, mean))
+
+    assert both(28, 5, 4, 28, 9000, 32, 5100) == (3, 1)
+    assert both(28, 5, 4, 28, 9000, 32, 8900) == (3, 3)        # nearly equal
+    assert both(36, 2, 8, 32, 4000, 32, 2700) == (3, 1)
+    assert both(36, 2, 8, 32, 9000, 32, 6000)[1] > 1           # four wavefronts, long columns
+    for L, B, H, hq, W in ((28, 1, 4, 28, 32), (28, 8, 4, 28, 64), (36, 3, 8, 32, 64), (32, 1, 32, 32, 32)):
+        for S in (100, 600, 2500, 9000, 30000):
+            for mean in (0, 1, S // 2, S - 1, S, S + 5):
+                equal, ragged = both(L, B, H, hq, S, W, mean)
+                assert ragged in (1, equal), (L, B, H, S, mean)
