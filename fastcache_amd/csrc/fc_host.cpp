@@ -695,7 +695,7 @@ struct Scratch {
 // caller's general path then serves or refuses the arguments).  The kept rows of every column move to the front of its pages;
 // scores and indices are scratch.  counts: kept rows per sequence where they differ; order: the sequences, longest first.
 // snapkv = (queries, window, kernel_size, causal, scale, out_scale, fits, mean length): one launch where the shape fits one and cutting
-// the columns does not pay, else key ranges, selection and compaction; None: the Knorm press in one launch.  Views, scratch and uploads in Python cost 25 to 45 us before the launch,
+// the columns does not pay, else key ranges, selection and compaction; None: the Knorm press in one launch; False: its norms, selection and compaction.  Views, scratch and uploads in Python cost 25 to 45 us before the launch,
 // with the GPU idle behind the last pass's synchronisation: 13 sequences of 200 to 2300 tokens (SnapKV, 28 layers) 500 -> 475 us.
 PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return guarded([&]() -> PyObject* {
@@ -717,7 +717,8 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     int32_t nsplit = 1;
     bool one = true;
     double scale = 0, out_scale = 0;
-    if (args[7] != Py_None) {
+    const bool norms_apart = args[7] == Py_False;
+    if (args[7] != Py_None && !norms_apart) {
       if (!PyTuple_Check(args[7]) || PyTuple_GET_SIZE(args[7]) != 8) fail("press_rows: the SnapKV arguments are a tuple of eight");
       const auto item = [&](int i) { return PyTuple_GET_ITEM(args[7], i); };
       q = tensor(item(0), "queries");
@@ -770,7 +771,13 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Scratch mem(Scratch::room(idx_bytes) + Scratch::room(cols * S * 4) + cols * 4, pool);
     int32_t* idx = (int32_t*)mem.take(idx_bytes);
     float* scores = (float*)mem.take(cols * S * 4);
-    if (!q.defined()) {
+    if (norms_apart) {
+      check(fc_knorm_score(&kv, scores, (int32_t)S, stream), "fc_knorm_score");
+      check(fc_topk_select(scores, (int32_t)S, (int32_t)cols, (int32_t)S, counts ? lens.data_ptr<int32_t>() : nullptr, (int32_t)H,
+                           counts ? (int32_t)B : 1, (int32_t)width, counts, idx, (int32_t)width, stream),
+            "fc_topk_select");
+      check(fc_compact(&kv, &vv, &kv, &vv, idx, (int32_t)width, (int32_t)H, (int32_t)width, counts, stream), "fc_compact");
+    } else if (!q.defined()) {
       check(fc_knorm_press(&kv, &vv, scores, (int32_t)S, (int32_t)width, counts, idx, (int32_t)width, stream), "fc_knorm_press");
     } else if (order) {
       check(fc_snapkv_press_ordered(&kv, &vv, q.const_data_ptr(), nullptr, (int32_t)hq, (int32_t)W, (int32_t)ksz, (int32_t)causal,

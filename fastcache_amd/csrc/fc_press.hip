@@ -171,7 +171,10 @@ extern "C" int fc_knorm_press(const fc_kv_view* keys, const fc_kv_view* values, 
     hipLaunchKernelGGL((knorm_press_kernel<DT, TH>), grid, dim3(TH), lds, st, kv, vv, scores, score_stride, k,   \
                        n_kept, indices, index_stride, smax);                                                     \
   } while (0)
-  const bool wide = (long long)smax * FC_HEAD_DIM * fc_elem_bytes(keys->dtype) >= KP_WIDE_BYTES_PRESS;
+  // Columns no more than compute units are wide whatever their length, since nothing else fills the chip (us per pass, 256
+  // -> 1024 threads: 112 columns of 300 bf16 keys 50 -> 47, of 1000 74 -> 55, 224 of 1000 78 -> 64; 336 of 1000 85 -> 87).
+  const bool wide = (long long)smax * FC_HEAD_DIM * fc_elem_bytes(keys->dtype) >= KP_WIDE_BYTES_PRESS ||
+                    (long long)keys->num_kv_heads * keys->batch * keys->num_layers <= fc_compute_units();
 #define KP_DISPATCH(DT) \
   if (wide) KP_LAUNCH(DT, 1024); else KP_LAUNCH(DT, 256)
   switch (keys->dtype) {

@@ -81,15 +81,18 @@ def knorm_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq
     kept = [n_kept_for(n, compression_ratio) for n in lens]
     width = max(kept)
     # One launch (every (layer, sequence, head) column is scored, selected and compacted by one workgroup) or norms,
-    # selection and compaction each over the whole chip: below about one and a half columns per compute unit the single
-    # workgroups leave it half idle (us per pass, half kept: 112 columns of 1000 bf16 keys 46 -> 31, of 12000 309 -> 251, 288 of
-    # 2000 106 -> 96, of 18000 1073 -> 935; from there on one launch wins: 576 of 2000 fp32 379 against 412, 1152 of 2000
-    # 354 against 406).
+    # selection and compaction each over the whole chip.  One workgroup per column leaves part of the chip idle below about
+    # one and a half columns per compute unit, which long columns feel and short ones do not (us per pass, 60 % dropped, one
+    # launch against three, bf16: 112 columns of 300 keys 47 48, of 1000 55 62, of 3000 87 91, of 9000 219 202; 224 of 1000 64
+    # 73, of 3000 112 124, of 9000 343 332; 288 of 300 52 53, of 1000 81 80, of 3000 175 160, of 9000 516 446; from there on
+    # one launch wins: 448 of 3000 227 229, 576 of 1000 102 116, 1024 of 3000 443 492).
     columns = kv_cache.shape[1] * block_tables.shape[0] * kv_cache.shape[-2] if kv_cache.is_cuda else 0
+    cus = _lib.compute_units(kv_cache.device) if columns else 1
     one_launch = (compact and 0 < width and ops.press_column_fits(seq_len, width) and
-                  2 * columns > 3 * _lib.compute_units(kv_cache.device))
-    if one_launch and rows_only and _press_rows(kv_cache, block_tables, seq_lens, seq_len, width,
-                                                None if len(set(kept)) == 1 else kept):
+                  seq_len <= (5000 if columns <= cus else 1000 if 2 * columns <= 3 * cus else seq_len))
+    if (rows_only and compact and 0 < width and columns and
+            _press_rows(kv_cache, block_tables, seq_lens, seq_len, width, None if len(set(kept)) == 1 else kept,
+                        snapkv=None if one_launch else False)):
         return None
     kview, vview = _views(kv_cache, block_tables, seq_lens, seq_len)
     if one_launch:

@@ -370,7 +370,9 @@ def test_host_numbers_are_not_uploaded_under_capture(dev):
 
 @pytest.mark.parametrize("press", ["knorm", "snapkv"])
 @pytest.mark.parametrize("L,H,hq,lens,planes", [
-    (3, 4, 8, [700], "whole"),                      # few columns: norms / key ranges, selection, compaction
+    (3, 4, 8, [700], "whole"),                      # few columns: one launch / key ranges, selection, compaction
+    (3, 4, 8, [5200, 1300, 40], "whole"),           # long ones: norms / key ranges, selection, compaction, ragged
+    (16, 4, 28, [1100, 333, 64, 901, 700], "whole"),           # some more columns than compute units: likewise
     (16, 4, 28, [333, 1200, 64, 901, 33, 500, 77, 1024], "whole"),     # ragged, one launch, sequences no longer than the window
     (16, 4, 28, [600] * 8, "layers"),               # equal lengths; a slice of the pool's layers
     (12, 8, 16, [900] * 5 + [899], "copied"),       # queries whose rows do not lie side by side: the general path
