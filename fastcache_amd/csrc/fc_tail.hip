@@ -17,11 +17,13 @@
 
 // Pooling: 64-key groups a wavefront stages at a time, and its floats for them (a kernel of at most 63 reaches 62 keys past
 // the groups).  The longest rows stage fewer, so that with their keys in LDS two workgroups fit a compute unit's 160 KB.
-#define CS_GROUPS(KPT) ((KPT) > 16 ? 4 : (KPT) < 8 ? (KPT) : 8)
+// A lane's keys are a whole number of them: a key past the lane's last would be put where the wavefronts stage.
+#define CS_GROUPS(KPT) ((KPT) > 16 ? 4 : (KPT) < 8 ? (KPT) : (KPT) % 8 == 0 ? 8 : 6)
 #define CS_STAGE(KPT) (CS_GROUPS(KPT) * 64 + 64)
 
 template <int SRC, int DTYPE, int THREADS, int KPT>
 __global__ __launch_bounds__(THREADS, KPT > 16 ? 4 : 1) void column_select_kernel(KvView kv, KvView vv, KvView dk, KvView dv, ColumnSelect a) {
+  static_assert(KPT % CS_GROUPS(KPT) == 0, "the pooling fills every key of a lane and no other");
   constexpr int EB = DTYPE == FC_F32 ? 4 : 2;
   constexpr int LPR = FC_HEAD_DIM * EB / 16, RPP = THREADS / LPR;
   extern __shared__ __align__(16) int cs_lds[];   // [part_rows] kept positions, the keys that registers do not hold, then what SRC stages

@@ -819,6 +819,33 @@ def test_layer_hooks_in_one_call(dev, dtype, B, H, S):
                 assert not bool(((got ^ ref) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
 
 
+@pytest.mark.parametrize("S", [500, 1000, 2000, 4096, 8000, 8681, 12320, 16000, 20000])     # one of each selection size
+def test_selection_of_pooled_sums_is_the_same_every_time(dev, S):
+    """A SnapKV hook whose columns are each selected by many workgroups, again and again: one selection, and no key kept or
+    dropped that the scores do not allow."""
+    H, W, keep = 32, 32, S // 5
+    g = torch.Generator(device=dev).manual_seed(S)
+    k = torch.randn(1, H, S, 128, generator=g, device=dev).to(torch.float16)
+    v = torch.zeros_like(k)
+    pos = torch.arange(S, device=dev)
+    v[..., 0], v[..., 1] = (pos % 256).to(v.dtype), (pos // 256).to(v.dtype)
+    q = torch.randn(1, H, W, 128, generator=g, device=dev).to(torch.float16)
+    press = SnapKVPress(1.0 - (keep + 0.5) / S, window_size=W, kernel_size=7)
+    hidden = torch.zeros(1, S, 1)
+    scores = press.score(None, hidden, k, v, None, {"queries": q})
+    kth = scores.topk(keep, -1).values[..., -1:]
+    first = None
+    for _ in range(12):
+        ov = press.compress(None, hidden, k, v, None, {"queries": q})[1]
+        idx = ov[..., 0].long() + 256 * ov[..., 1].long()
+        first = idx if first is None else first
+        assert torch.equal(idx, first)
+    got = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, first, True)
+    assert bool((got.sum(-1) == keep).all())
+    # other partial sums than the score tensor's: only keys near the threshold may differ, as above
+    assert not bool(((got ^ (scores >= kth)) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("S,k", [(1, 1), (512, 100), (513, 513), (1025, 300), (4096, 4000)])
 def test_knorm_press_into_forms(dev, dtype, S, k):
