@@ -429,6 +429,7 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 // short: the wavefronts take the 32-token tiles in turn, K and V of the first tile (and K of the second) are requested
 // at once instead of K before V, every wavefront carries its own running softmax and no phase waits for the workgroup,
 // and the eight are merged through LDS.  The step's new K and V rows may be appended by the same workgroups (k_new).
+// The ranges of a column are merged by a launch of their own or (TURN) by the workgroup of the column that arrives last.
 //   S^T[key][head] = K Q^T  on v_mfma_f32_16x16x32: the A operand (16 keys x 64 contiguous bytes per instruction)
 //                           comes straight from memory; the lane then owns ONE head and 8 keys of the tile, so maxima
 //                           and sums run over its registers and two lane exchanges;
@@ -447,6 +448,7 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 #define DC_PSTRIDE 132                                             // floats per partial output row (padded against bank conflicts)
 #define DC_VROW 272                                                // LDS bytes per V row: 4 rows apart = 64 bytes apart in banks
 #define DC_STAGE (DA_TILE * DC_VROW)
+#define DC_MERGE 8                                                // partial rows in flight per thread of the merge
 #define DC_PART (DC_WAVES * DC_STAGE)                              // V stages, then the partial outputs
 #define DC_LDS (DC_PART + DC_WAVES * DC_HEADS * 8)
 static_assert(DC_PART >= DC_WAVES * DC_HEADS * DC_PSTRIDE * 4, "the partial outputs share the V stages' memory");
@@ -494,13 +496,29 @@ struct DaAppend {                 // the step's new rows, one per sequence (k_ne
   const int* slots;               // flat cache slot per sequence, negative = skip
 };
 
-template <int DTYPE, int TERMS, bool PAGED>
+// Arrivals per column of a launch whose last workgroup merges, a row of counters per turn (fc_decode_layer_turn).  Zero
+// between launches: whoever merges puts the zero back.
+#define DC_COLUMNS 512
+static __device__ unsigned dc_arrived[FC_DECODE_TURNS][DC_COLUMNS];
+
+// Partial results that another workgroup of the same launch reads go past the caches of this XCD.
+template <bool TURN>
+__device__ __forceinline__ void dc_put(float* p, float x) {
+  if constexpr (TURN) __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = x;
+}
+__device__ __forceinline__ float2 dc_get2(const float* p) {      // 8-byte aligned
+  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT));
+}
+
+template <int DTYPE, int TERMS, bool PAGED, bool TURN>
 __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc, KvView vc, int layer,
                                                                       const char* __restrict__ q, int Hq,
                                                                       const int* __restrict__ lens, float c,
                                                                       char* __restrict__ out, DaAppend ap, int chunk,
-                                                                      float* __restrict__ part_o,
-                                                                      float* __restrict__ part_ml, int max_splits) {
+                                                                      float* part_o, float* part_ml, int max_splits,
+                                                                      int turn) {
   extern __shared__ __align__(16) char smem[];
   const int b = blockIdx.y;
   const int G = Hq / kc.num_kv_heads, gtiles = (G + DC_HEADS - 1) / DC_HEADS;
@@ -569,8 +587,9 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     }
   }
   unsigned short* orow = reinterpret_cast<unsigned short*>(out) + ((long long)b * Hq + h * G + g0) * FC_HEAD_DIM;
+  const bool whole = max_splits == 1 || (TURN && len <= chunk);
   if (len <= 0) {       // with several workgroups per column the merge writes the zeros
-    if (max_splits == 1)
+    if (whole)
       for (int i = tid; i < ng * FC_HEAD_DIM; i += DC_THREADS) orow[i] = 0;
     return;
   }
@@ -725,16 +744,64 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
       lg = fmaf(__builtin_amdgcn_exp2f(x.x - (mg == -INFINITY ? 0.f : mg)), x.y, lg);
       acc += part[(w * DC_HEADS + g) * DC_PSTRIDE + d];
     }
-    if (max_splits == 1) {
+    if (whole) {
       orow[i] = da_pack<DTYPE>(acc / lg);
     } else {
       const long long at = ((long long)b * Hq + h * G + g0 + g) * max_splits + blockIdx.z;
-      part_o[at * FC_HEAD_DIM + d] = acc;
+      dc_put<TURN>(part_o + at * FC_HEAD_DIM + d, acc);
       if (d == 0) {
-        part_ml[at * 2] = mg;
-        part_ml[at * 2 + 1] = lg;
+        dc_put<TURN>(part_ml + at * 2, mg);
+        dc_put<TURN>(part_ml + at * 2 + 1, lg);
       }
     }
+  }
+  if (!TURN || whole) return;
+
+  // ---- the column's workgroups into one: whoever arrives last ------------------------------------------------------
+  // Every workgroup whose range holds a token gets here, ns of them; nobody waits.  The partial results have reached the
+  // device's point of coherence before the workgroup counts itself, so the last one reads all of them there.  (Ordinary
+  // stores with a release and an acquire, which write back and drop caches, instead: 341 us for the 28 layers that take
+  // 296 this way and 374 with the merge's own launch, host bound.)
+  const int ns = (len + chunk - 1) / chunk;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  unsigned* arrived = &dc_arrived[turn][blockIdx.y * gridDim.x + blockIdx.x];
+  unsigned* before = reinterpret_cast<unsigned*>(smem);
+  if (tid == 0) *before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (*before != (unsigned)(ns - 1)) return;
+  if (tid == 0) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const long long col = ((long long)b * Hq + h * G + g0) * max_splits;
+  float2* all = reinterpret_cast<float2*>(smem + 16);       // [head][range]: maximum, sum
+  constexpr int PAIRS = FC_HEAD_DIM / 2;
+  float2 x[DC_MERGE];
+  const auto load_o = [&](int i, int s0) {                  // two dimensions of a head, ranges s0 ..
+    const float* po = part_o + (col + (long long)(i / PAIRS) * max_splits) * FC_HEAD_DIM + i % PAIRS * 2;
+#pragma unroll
+    for (int j = 0; j < DC_MERGE; ++j)
+      x[j] = s0 + j < ns ? dc_get2(po + (long long)(s0 + j) * FC_HEAD_DIM) : make_float2(0.f, 0.f);
+  };
+  if (tid < ng * PAIRS) load_o(tid, 0);
+  for (int i = tid; i < ng * ns; i += DC_THREADS) all[i] = dc_get2(part_ml + (col + (long long)(i / ns) * max_splits + i % ns) * 2);
+  __syncthreads();
+  // the arithmetic and the order of decode_merge_kernel
+  for (int i = tid; i < ng * PAIRS; i += DC_THREADS) {
+    const float2* ml = all + i / PAIRS * ns;
+    float M = -INFINITY, L = 0.f;
+    float2 acc = make_float2(0.f, 0.f);
+    for (int s = 0; s < ns; ++s) M = fmaxf(M, ml[s].x);
+    for (int s0 = 0; s0 < ns; s0 += DC_MERGE) {
+      if (i != tid || s0) load_o(i, s0);
+#pragma unroll
+      for (int j = 0; j < DC_MERGE; ++j) {
+        const float2 e = s0 + j < ns ? ml[s0 + j] : make_float2(-INFINITY, 0.f);
+        const float w = __builtin_amdgcn_exp2f(e.x - M);
+        L = fmaf(w, e.y, L);
+        acc.x = fmaf(w, x[j].x, acc.x);
+        acc.y = fmaf(w, x[j].y, acc.y);
+      }
+    }
+    reinterpret_cast<unsigned*>(orow)[i] = (unsigned)da_pack<DTYPE>(acc.x / L) | ((unsigned)da_pack<DTYPE>(acc.y / L) << 16);
   }
 }
 
@@ -924,6 +991,12 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 // short enough for one workgroup each still gain by not being merged: 192 columns of 512 tokens 16.7 -> 15.4 us, 256 of
 // 768 tokens 23.6 -> 22.5.
 #define DC_ONE 768
+// Eager layers, launched one by one, gain where the last workgroup of a column merges it: a launch less for the host
+// (12 to 13 us a layer before) and 0 to 1 us of waiting for the device.  28 layers, merge launch -> last workgroup: 2 ranges
+// 379 -> 284 us, 4 of 12 to 48 columns 372 -> 296 to 346, 10 of 8 columns 380 -> 318, 14 of 4 columns 379 -> 327, 15 of 16
+// columns 375 -> 381, 16 of 8 columns 379 -> 364, 24 to 31 of 8 columns 1 to 2 % slower (28 of 4 columns 6 % faster): the
+// ranges of a column are read eight at a time by one workgroup, past the caches.
+#define DC_SPLITS 14
 static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
   const int G = num_q_heads / k->num_kv_heads;
   const long long cols = (long long)k->num_kv_heads * ((G + DC_HEADS - 1) / DC_HEADS) * k->batch;
@@ -955,7 +1028,8 @@ static int da_merge(const char* who, const fc_kv_view* k_cache, const float* par
 // Checks and launches shared by the entry points; `workspace` is a device address.
 static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t layer,
                       const void* q, void* out, int32_t num_q_heads, const int32_t* context_lens, float scale,
-                      void* workspace, int64_t workspace_bytes, void* stream, const DaAppend* append = nullptr) {
+                      void* workspace, int64_t workspace_bytes, void* stream, const DaAppend* append = nullptr,
+                      int turn = -1) {
   int rc;
   if ((rc = fc_check_view(k_cache, who)) || (rc = fc_check_view(v_cache, who))) return rc;
   FC_REQUIRE(k_cache->dtype == v_cache->dtype && k_cache->num_layers == v_cache->num_layers &&
@@ -982,16 +1056,20 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
     float* part_o = (float*)workspace;
     float* part_ml = part_o ? part_o + (int64_t)k_cache->batch * num_q_heads * csplits * FC_HEAD_DIM : nullptr;
     const DaAppend ap = append ? *append : DaAppend{nullptr, nullptr, 0, 0, nullptr};
+    if ((int64_t)grid.x * grid.y > DC_COLUMNS || csplits > DC_SPLITS || !k_cache->block_tables) turn = -1;
     const KvView k = fc_make_view(k_cache), v = fc_make_view(v_cache);
-#define DC_LAUNCH2(DT, TERMS, PG)                                                                                  \
+#define DC_LAUNCH3(DT, TERMS, PG, TURN)                                                                            \
   do {                                                                                                             \
-    FC_ALLOW_LDS((decode_column_kernel<DT, TERMS, PG>), DC_LDS);                                                    \
-    hipLaunchKernelGGL((decode_column_kernel<DT, TERMS, PG>), grid, dim3(DC_THREADS), DC_LDS, (hipStream_t)stream, k, \
-                       v, layer, (const char*)q, num_q_heads, context_lens, scale * DA_LOG2E, (char*)out, ap,       \
-                       column, part_o, part_ml, csplits);                                                           \
+    FC_ALLOW_LDS((decode_column_kernel<DT, TERMS, PG, TURN>), DC_LDS);                                              \
+    hipLaunchKernelGGL((decode_column_kernel<DT, TERMS, PG, TURN>), grid, dim3(DC_THREADS), DC_LDS, (hipStream_t)stream, \
+                       k, v, layer, (const char*)q, num_q_heads, context_lens, scale * DA_LOG2E, (char*)out, ap,    \
+                       column, part_o, part_ml, csplits, turn);                                                    \
   } while (0)
-#define DC_LAUNCH(DT, TERMS) \
-  if (k_cache->block_tables) DC_LAUNCH2(DT, TERMS, true); else DC_LAUNCH2(DT, TERMS, false)
+// (a turn comes with paged caches)
+#define DC_LAUNCH(DT, TERMS)                                      \
+  if (!k_cache->block_tables) DC_LAUNCH3(DT, TERMS, false, false); \
+  else if (turn < 0 || csplits == 1) DC_LAUNCH3(DT, TERMS, true, false); \
+  else DC_LAUNCH3(DT, TERMS, true, true)
     if (k_cache->dtype == FC_F16) {
       DC_LAUNCH(FC_F16, 2);
     } else if (G > 4) {
@@ -999,10 +1077,11 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
     } else {
       DC_LAUNCH(FC_BF16, 3);
     }
-#undef DC_LAUNCH2
+#undef DC_LAUNCH3
 #undef DC_LAUNCH
     FC_CHECK_LAUNCH(who);
-    if (csplits > 1) return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, csplits, column, out, stream);
+    if (csplits > 1 && turn < 0)
+      return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, csplits, column, out, stream);
     return FC_OK;
   }
   const int64_t need = fc_decode_attn_workspace_bytes(k_cache->batch, num_q_heads, k_cache->max_seq_len);
@@ -1101,8 +1180,17 @@ extern "C" int fc_decode_layer(const fc_kv_view* k_cache, const fc_kv_view* v_ca
                                int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping,
                                void* out, int32_t num_q_heads, const int32_t* context_lens, float scale, void* workspace,
                                int64_t workspace_bytes, void* stream) {
+  return fc_decode_layer_turn(k_cache, v_cache, q, k_new, k_stride, v_new, v_stride, slot_mapping, out, num_q_heads,
+                              context_lens, scale, workspace, workspace_bytes, -1, stream);
+}
+
+extern "C" int fc_decode_layer_turn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
+                                    int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping,
+                                    void* out, int32_t num_q_heads, const int32_t* context_lens, float scale,
+                                    void* workspace, int64_t workspace_bytes, int32_t turn, void* stream) {
   const char* who = "fc_decode_layer";
   int rc;
+  FC_REQUIRE(turn >= -1 && turn < FC_DECODE_TURNS, FC_EINVAL, "%s: turn %d", who, turn);
   if ((rc = fc_check_view(k_cache, who)) || (rc = fc_check_view(v_cache, who))) return rc;
   FC_REQUIRE(k_new && v_new && slot_mapping, FC_EINVAL, "%s: null pointer", who);
   FC_REQUIRE(k_cache->block_tables && v_cache->block_tables && k_cache->num_layers == 1 && v_cache->num_layers == 1, FC_EINVAL,
@@ -1120,7 +1208,7 @@ extern "C" int fc_decode_layer(const fc_kv_view* k_cache, const fc_kv_view* v_ca
   if (da_appends_inside(k_cache, v_cache, num_q_heads)) {
     const DaAppend ap = {(const char*)k_new, (const char*)v_new, k_stride * eb, v_stride * eb, slot_mapping};
     return da_enqueue(who, k_cache, v_cache, 0, q, out, num_q_heads, context_lens, scale, workspace, workspace_bytes,
-                      stream, &ap);
+                      stream, &ap, turn);
   }
   // what the attention would refuse is refused before the rows are written
   FC_REQUIRE(q && out && context_lens && workspace, FC_EINVAL, "%s: null pointer", who);

@@ -426,6 +426,29 @@ PyObject* py_dequantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   });
 }
 
+// The counters of a stream's decode launches: the index of the stream among those seen on its device, or -1 where a
+// launch of its own must merge.  A graph under capture may be replayed on another stream; a stream that is not torch's
+// own may be destroyed and its handle given to the next one while it still runs.
+int decode_turn(const at::Tensor& t, const c10::hip::HIPStream& stream) {
+  constexpr int kDevices = 64;
+  static std::vector<c10::StreamId> seen[kDevices];     // under the interpreter's lock
+  const int dev = t.get_device();
+  const c10::StreamId id = stream.id();
+  if (dev < 0 || dev >= kDevices || (id != 0 && !(id & 1))) return -1;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream.stream(), &capture) != hipSuccess) {
+    (void)hipGetLastError();
+    return -1;
+  }
+  if (capture != hipStreamCaptureStatusNone) return -1;
+  auto& ids = seen[dev];
+  const auto at = std::find(ids.begin(), ids.end(), id);
+  if (at != ids.end()) return (int)(at - ids.begin());
+  if (ids.size() >= FC_DECODE_TURNS) return -1;
+  ids.push_back(id);
+  return (int)ids.size() - 1;
+}
+
 // ---- one attention layer of a decode step ---------------------------------------------------------------------------------
 // decode_layer(q, k, v, k_cache, v_cache, slot_mapping, context_lens, block_tables, scale, q_heads, kv_heads, head_dim,
 //              workspace or None) -> out [n, q_heads * head_dim], or None when the arguments are not the plain decode
@@ -494,9 +517,11 @@ PyObject* py_decode_layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       ws_bytes = ws.numel();
     }
     at::Tensor out = at::empty({n, hq * d}, q.options());
-    check(fc_decode_layer(&kv, &vv, q.const_data_ptr(), k.const_data_ptr(), stride[0], v.const_data_ptr(), stride[1],
+    const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(q.get_device());
+    check(fc_decode_layer_turn(&kv, &vv, q.const_data_ptr(), k.const_data_ptr(), stride[0], v.const_data_ptr(), stride[1],
                           (const int32_t*)slots.const_data_ptr(), out.data_ptr(), (int32_t)hq,
-                          (const int32_t*)lens.const_data_ptr(), (float)scale, wsp, ws_bytes, stream_of(q)),
+                          (const int32_t*)lens.const_data_ptr(), (float)scale, wsp, ws_bytes, ws_bytes ? decode_turn(q, stream) : -1,
+                          (void*)stream.stream()),
           "fc_decode_layer");
     return wrap(std::move(out));
   });

@@ -550,6 +550,17 @@ int fc_decode_layer(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const 
                     int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping, void* out,
                     int32_t num_q_heads, const int32_t* context_lens, float scale, void* workspace,
                     int64_t workspace_bytes, void* stream);
+/*
+ * The same with one launch less where a column is cut into ranges: the workgroup that finishes last merges them.  It is
+ * told by counters of the device; `turn`, 0 .. FC_DECODE_TURNS - 1, says which, -1 asks for the launch of its own.  Two
+ * calls of one turn must not run on a device at the same time: a turn belongs to one stream, and is not for a captured
+ * graph, which may be replayed on any.  The counters are back at zero when the launch has ended.
+ */
+#define FC_DECODE_TURNS 64
+int fc_decode_layer_turn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
+                         int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping, void* out,
+                         int32_t num_q_heads, const int32_t* context_lens, float scale, void* workspace,
+                         int64_t workspace_bytes, int32_t turn, void* stream);
 
 /*
  * A decode step's inputs into the static buffers of a captured graph (what the decode branch of `run_model` patches

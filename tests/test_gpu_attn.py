@@ -322,6 +322,63 @@ def test_keys_of_infinite_distance_weigh_nothing(dev, dtype, lens, max_pages):
     assert float((got.float() - ref.float()).abs().max()) < 4e-3      # as for finite keys above
 
 
+@pytest.mark.parametrize("dtype,Hq,Hkv,lens,pages", [
+    (torch.bfloat16, 28, 4, [300, 0, 1, 255, 256, 257, 511], 2),
+    (torch.float16, 8, 8, [2048, 2047, 700], 8),                # ranges read eight at a time: one group of them, one more
+    (torch.bfloat16, 8, 2, [2049, 1], 9),
+    (torch.float16, 32, 2, [3584, 513], 14),                    # 16 heads a group; the most ranges the last workgroup merges
+    (torch.bfloat16, 7, 1, [3600], 15),                         # one more: a launch merges
+])
+def test_last_workgroup_merges_as_the_merge_launch(dev, dtype, Hq, Hkv, lens, pages):
+    """A column's ranges merged by its last workgroup (streams of torch, outside capture) against the launch that merges
+    (inside a captured graph, and on streams whose handle torch does not own): the same bits, launch after launch, with two
+    streams at work at once, and the oracle's values."""
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    B = len(lens)
+    case = synth.make_paged_case(seed=51, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=[n + 1 for n in lens], dtype=dtype)
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(B, h * 128, generator=g).to(dtype) for h in (Hq, Hkv, Hkv))
+    tables = case.table_tensor("cpu")
+    tables = torch.cat([tables, tables[:, :1].expand(-1, max(0, pages - tables.shape[1]))], 1)[:, :pages].contiguous()
+    lens_t = torch.tensor(lens, dtype=torch.int32)
+    slots = torch.full((B,), -1, dtype=torch.int32)
+    pool = case.kv_cache[:, 0]
+    ref = oattn.decode_attention(q.view(B, Hq, 128), pool[0], pool[1], lens_t, tables, 128 ** -0.5)
+    layer = Attention(Hq, 128, 128 ** -0.5, Hkv)
+    on_gpu = pool.to(dev)
+    layer.k_cache, layer.v_cache = on_gpu[0], on_gpu[1]
+    q, k, v = q.to(dev), k.to(dev), v.to(dev)
+    set_context(False, slot_mapping=slots.to(dev), context_lens=lens_t.to(dev), block_tables=tables.to(dev))
+    try:
+        side = [torch.cuda.Stream(), torch.cuda.Stream()]
+        foreign = torch.cuda.ExternalStream(torch.cuda.Stream().cuda_stream)
+        torch.cuda.synchronize()
+        outs = [layer(q, k, v) for _ in range(3)]
+        for _ in range(4):                                       # two streams at once
+            for s in side:
+                with torch.cuda.stream(s):
+                    outs.append(layer(q, k, v))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(foreign):
+            merged = layer(q, k, v)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            held = layer(q, k, v)
+        for _ in range(3):
+            held.zero_()
+            graph.replay()
+            outs.append(layer(q, k, v))
+            torch.cuda.synchronize()
+            assert torch.equal(held.view(torch.int16), merged.view(torch.int16))
+    finally:
+        reset_context()
+    for o in outs:
+        assert torch.equal(o.view(torch.int16), merged.view(torch.int16))
+    assert float((merged.cpu().view(B, Hq, 128).float() - ref.float()).abs().max()) < 4e-3
+
+
 @pytest.mark.parametrize("copies,lens,block_size", [
     (3, [300, 40], 256),            # one workgroup a column
     (2, [254, 700], 256),           # several; the second copy's row is the first of a page
