@@ -984,13 +984,24 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 }
 
 // Tokens per workgroup of the column kernel, 0 = the launch does not take it.  Only launches whose workgroups are all
-// resident at once (one per compute unit: registers) do: beyond that bandwidth counts and the split kernel streams
+// resident at once (one per compute unit: registers) do, and a few more: beyond that bandwidth counts and the split kernel streams
 // better (128 columns of 1024 tokens: 19.4 us a layer against 19.6 to 23).  One 32-token tile per wavefront, 256 tokens, is
 // the shortest chain (a second tile costs about 3 us, a merge 3.5): 12 columns of 1024 tokens 13.2 -> 10.1 us, of 256
 // tokens without a merge 7.1, 48 columns of 1024 tokens 16.9 -> 13.0.  Where 256 would be too many workgroups, columns
 // short enough for one workgroup each still gain by not being merged: 192 columns of 512 tokens 16.7 -> 15.4 us, 256 of
 // 768 tokens 23.6 -> 22.5.
+// Longer ranges, several tiles a wavefront, as long as one round of workgroups holds them, against the split kernel (us a
+// pass: eager layers, 28 or 16 of them, append and merge launches included; captured layers gain the same shares).  Groups of
+// 5 and more heads, where a K and V read once feeds the matrix pipe for all of them: 2 tiles, 48 columns of 1500 tokens
+// 569 -> 464, 24 of 5000 639 -> 489; 4, 64 of 4000 in groups of 8 1012 -> 752; 8, 200 of 1700 1073 -> 929; 8, 64 of 8000
+// 784 -> 697; and two rounds of whole columns, 360 of 600 621 -> 451, 400 of 300 529 -> 330, but not of longer ones (360 of
+// 2000 1030 -> 1054).  Groups of 3 and 4: 2 tiles 572 -> 487 (96 of 1000), 3 635 -> 587, 4 748 -> 715, 802 -> 743, one
+// 693 -> 697; 5 730 -> 799, 921 -> 1027.  Smaller groups: 2 tiles 588 -> 551 (64 of 2000), 675 -> 533; 3 and 4 between
+// 789 -> 707 and 541 -> 571, 653 -> 678.
 #define DC_ONE 768
+#define DC_TILES_FEW 2
+#define DC_TILES_SOME 4
+#define DC_TILES_MANY 16
 // Eager layers, launched one by one, gain where the last workgroup of a column merges it: a launch less for the host
 // (12 to 13 us a layer before) and 0 to 1 us of waiting for the device.  28 layers, merge launch -> last workgroup: 2 ranges
 // 379 -> 284 us, 4 of 12 to 48 columns 372 -> 296 to 346, 10 of 8 columns 380 -> 318, 14 of 4 columns 379 -> 327, 15 of 16
@@ -1009,7 +1020,11 @@ static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_h
     return 0;
   const int chunk = DC_WAVES * DA_TILE;
   if (cols * ((k->max_seq_len + chunk - 1) / chunk) <= slots) return chunk;
-  return cols <= slots && k->max_seq_len <= DC_ONE ? DC_ONE : 0;
+  if (cols <= (G > 4 ? 2 : 1) * slots && k->max_seq_len <= DC_ONE) return DC_ONE;
+  const int most = G > 4 ? DC_TILES_MANY : G > 2 ? DC_TILES_SOME : DC_TILES_FEW;
+  for (int m = 2; m <= most; ++m)
+    if (cols * ((k->max_seq_len + m * chunk - 1) / (m * chunk)) <= slots) return m * chunk;
+  return 0;
 }
 
 static int da_merge(const char* who, const fc_kv_view* k_cache, const float* part_o, const float* part_ml,

@@ -267,6 +267,12 @@ def test_decode_attention_empty_rows(dev):
     (torch.float16, 32, 2, [700, 130], -2),                                              # 16 heads a group; a row inside the context
     (torch.bfloat16, 40, 2, [300, 77], -1),                                              # 20 heads a group: rows go in first
     (torch.bfloat16, 8, 2, [2500, 40], -1),                                              # too long for one workgroup a column
+    # many columns: ranges of 512 tokens and more, on both sides of their ends, and of a wavefront's second tile
+    (torch.bfloat16, 16, 2, ([1023, 511, 512, 513, 1, 256, 257, 767] * 5)[:33], -1),
+    (torch.float16, 2, 2, ([900, 511, 512, 1023, 40] * 7)[:33], 0),
+    (torch.bfloat16, 8, 2, ([1700, 767, 768, 769, 1535, 1536, 33] * 6)[:40], -1),        # 4 heads a group: 768
+    (torch.float16, 8, 1, ([3900, 1535, 1536, 1537, 100, 3072, 3073] * 10)[:65], -1),    # 8 heads a group: 1536
+    (torch.bfloat16, 32, 4, ([700, 511, 512, 1, 600] * 14)[:70], -1),                    # two rounds of whole columns
 ])
 def test_attention_layer_appends_and_attends(dev, dtype, Hq, Hkv, lens, slot_at):
     """``Attention.forward`` of a decode step against the oracle on a cache the oracle appended to: every launch form the
@@ -328,6 +334,7 @@ def test_keys_of_infinite_distance_weigh_nothing(dev, dtype, lens, max_pages):
     (torch.bfloat16, 8, 2, [2049, 1], 9),
     (torch.float16, 32, 2, [3584, 513], 14),                    # 16 heads a group; the most ranges the last workgroup merges
     (torch.bfloat16, 7, 1, [3600], 15),                         # one more: a launch merges
+    (torch.bfloat16, 14, 2, ([1000, 512, 513, 0, 80] * 7)[:33], 4),     # ranges of 512
 ])
 def test_last_workgroup_merges_as_the_merge_launch(dev, dtype, Hq, Hkv, lens, pages):
     """A column's ranges merged by its last workgroup (streams of torch, outside capture) against the launch that merges
