@@ -522,6 +522,7 @@ class DecodeWorkload(Workload):
         self.device = device
         if hybrid:   # the decode half of configuration 5: 16 caches compressed to 3280 tokens, 7 query heads per kv head
             self.name, self.dtype_name = "cfg5-decode-after-hybrid-minicpm-v-2.6", "bf16"
+            self.kernel_name = "decode_column_kernel"
             self.L, self.B, self.Hq, self.Hkv, self.T, dtype = 28, 16, 28, 4, graph_steps, torch.bfloat16
             self.lens_text = "3280 (16384 compressed to 20 %)"
             self.case = synth.decode_case(seed=seed, num_layers=self.L, batch=self.B, num_kv_heads=self.Hkv,
@@ -738,7 +739,8 @@ _COUNTER_RUN = {"commit": "76bf753", "date": "2026-11-25"}   # the tree whose ke
 #  cfg5's readings came out as at commit 3ee0b1a)
 _COUNTER_RUN_OF = {"cfg5-ccm-hybrid-minicpm-v-2.6": {"commit": "cbd5ec4", "date": "2026-11-25"},
                    "cfg1-knorm-llama-7b": {"commit": "cbd5ec4", "date": "2026-11-25"},
-                   "cfg2-snapkv-qwen3-8b": {"commit": "cbd5ec4", "date": "2026-11-25"}}
+                   "cfg2-snapkv-qwen3-8b": {"commit": "cbd5ec4", "date": "2026-11-25"},
+                   "cfg5-decode-after-hybrid-minicpm-v-2.6": {"commit": "0a758fa", "date": "2026-12-02"}}
 _FETCH_SCALE = 524288 / 2.623e5
 _WRITE_SCALE = 524288 / 5.284e5
 _COUNTER_KIB = {  # workload name -> (FETCH_SIZE, WRITE_SIZE) per dispatch of the dominant kernel
@@ -753,7 +755,7 @@ _COUNTER_KIB = {  # workload name -> (FETCH_SIZE, WRITE_SIZE) per dispatch of th
     # graphs).  A launch reads every cached token once and the caches grow by a token per step, so the reading
     # is scaled from that run's algorithmic bytes per launch (third entry) to those of the measured graph.
     "cfg4-decode-paged-attention-llava-1.5-7b": (8.059e5, 7414.0, 1648099328),
-    "cfg5-decode-after-hybrid-minicpm-v-2.6": (5.308e4, 1904.0, 107790336),
+    "cfg5-decode-after-hybrid-minicpm-v-2.6": (5.270e4, 924.0, 107790336),
 }
 
 
