@@ -435,13 +435,15 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 //                           and sums run over its registers and two lane exchanges;
 //   O^T[dim][head] = V^T P^T: the probabilities are already the B operand (keys in the order the accumulator gives
 //                           them); V goes through the wavefront's 8 KB of LDS and is read transposed, 2 bytes at a time.
-// Probabilities enter as a sum of 16-bit operands in the cache dtype: two (as the split kernel does for 5 to 8 heads), or
-// three for bf16 groups of up to 4 heads, where the split kernel multiplies in fp32.  Two fp16 operands hold 22 bits of
-// a probability down to 2^-17 and what they drop is below 2^-39 of the tile's largest (DA_P_SCALE).
+// Probabilities enter as a sum of 16-bit operands in the cache dtype: two for groups of 5 and more heads (as in the split
+// kernel), three for up to 4 heads, where the split kernel multiplies in fp32: three bf16 operands hold all 24 bits, three
+// fp16 operands all bits of a probability down to 2^-15, and what they drop is below 2^-39 of the tile's largest
+// (DA_P_SCALE).  A tile's products are summed by themselves, least operands first, and rounded into the output once.
+// Error of the unrounded output against 64 bits, geometric mean over 7 settings (1 / 2 / 4 heads a group, 2 to 64 contexts of
+// 500 to 3500 keys, 12 seeds), this kernel / the split kernel: logits of deviation 1, fp16 2.03 / 2.10e-7, bf16
+// 1.85 / 1.97e-7; of deviation 3, 1.003 and 1.002 of it; of deviation 6, 1.000 and 0.999 (two fp16 operands, and operands
+// added to the output one by one: 1.010 and 1.014, 1.012 and 1.016, 1.002 and 1.004 of the split kernel's).
 // (An infinite value in V gives NaN: a term of its probability is zero or negative.  In fp32 it gave an infinity.)
-// Error of the unrounded output against 64 bits, 3 contexts of up to 2040 keys, 1 / 2 / 4 fp16 heads a group, this kernel
-// and the split kernel in fp32: flat 1.08 / 1.09 / 1.08e-7 and 1.12 / 1.09 / 1.12e-7, peaked 8.5 / 9.4 / 9.8e-8 and
-// 8.3 / 8.9 / 9.1e-8 (a third operand leaves the latter as they are); per layer 8.34 us before and after.
 #define DC_WAVES 8
 #define DC_THREADS (DC_WAVES * 64)
 #define DC_HEADS 16
@@ -691,9 +693,10 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
                ((unsigned)*reinterpret_cast<const unsigned short*>(r + DC_VROW) << 16);
       }
       const uint4 vt = make_uint4(w[0], w[1], w[2], w[3]);
-      o[db] *= alpha;
+      f32x4 pv = f32x4{0.f, 0.f, 0.f, 0.f};        // the tile's own sum, least operands first: o is rounded once a tile
 #pragma unroll
-      for (int t = 0; t < TERMS; ++t) o[db] = da_mfma16<DTYPE>(vt, pt[t], o[db]);
+      for (int t = TERMS; t > 0; --t) pv = da_mfma16<DTYPE>(vt, pt[t - 1], pv);
+      o[db] = o[db] * alpha + pv;
       // not more transposed reads in flight than registers beside the tiles hold
       if ((db & 3) == 3) __builtin_amdgcn_sched_barrier(0);
     }
@@ -1086,11 +1089,9 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
   else if (turn < 0 || csplits == 1) DC_LAUNCH3(DT, TERMS, true, false); \
   else DC_LAUNCH3(DT, TERMS, true, true)
     if (k_cache->dtype == FC_F16) {
-      DC_LAUNCH(FC_F16, 2);
-    } else if (G > 4) {
-      DC_LAUNCH(FC_BF16, 2);
+      if (G > 4) { DC_LAUNCH(FC_F16, 2); } else { DC_LAUNCH(FC_F16, 3); }
     } else {
-      DC_LAUNCH(FC_BF16, 3);
+      if (G > 4) { DC_LAUNCH(FC_BF16, 2); } else { DC_LAUNCH(FC_BF16, 3); }
     }
 #undef DC_LAUNCH3
 #undef DC_LAUNCH

@@ -456,3 +456,34 @@ def test_small_fp16_probabilities_keep_their_bits(dev, Hq, Hkv, lens, table, bel
         ref = torch.einsum("hn,nhd->hd", w, v)
         # 2^-25: half of fp16's smallest step, for outputs below its normal range
         assert bool(((got[b] - ref).abs() <= (2.0 ** -11 + 2.0 ** -13) * ref.abs() + 2.0 ** -25).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,n", [(16, 16, 3), (16, 8, 32), (16, 4, 33), (12, 4, 250)])
+def test_probabilities_of_up_to_four_heads_keep_24_bits(dev, dtype, Hq, Hkv, n):
+    """One key of weight x = 2^-e, and two of weight 1 whose values are minus x's first 8 bits and minus the next 8: what the
+    output holds is the rest of x, at most 2^6 of its last places, so that dropping one place changes it by 2^-6.  Sums of
+    the three are multiples of that place below 2^24 of them, which fp32 holds in any order; the weights' sum and the
+    division may round differently, and then the output by one step, against the kernel that multiplies probabilities in
+    fp32 (taken for wide tables)."""
+    from fastcache_amd.layers.attention import decode_attention
+    B, scale, up = 16, 0.6931471805599453, 2.0 ** 15        # this scale times log2 e is 1 in fp32: exponents are exact
+    case = synth.make_paged_case(seed=6, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=[n] * B, dtype=dtype)
+    tables, wide = case.table_tensor("cpu"), case.table_tensor("cpu", 70)
+    e = torch.randint(1, 256, (B, Hkv), generator=torch.Generator().manual_seed(9)) / 64
+    pool, first = case.kv_cache[:, 0].clone(), tables[:, 0].long()
+    pool[0] = 0
+    pool[0, ..., 0] = -20                                   # the query's first element is 16: 2^-320 for the other keys
+    rest = torch.exp2(-e.double()).float().double()
+    for i, t in enumerate([0, n // 2, n - 1]):
+        pool[0, first, t, :, 0] = (-e / 16).to(dtype) if i == 0 else 0
+        part = torch.full_like(rest, -1.0) if i == 0 else rest.bfloat16().double()
+        pool[1, first, t] = (-part * up).to(dtype).unsqueeze(-1)
+        rest = rest if i == 0 else rest - part
+    q = torch.zeros(B, Hq, 128, dtype=dtype)
+    q[..., 0] = 16
+    on_gpu, lens_t = pool.to(dev), torch.full((B,), n, dtype=torch.int32)
+    got, fp32 = (decode_attention(q.to(dev), on_gpu[0], on_gpu[1], lens_t.to(dev), t.to(dev), scale).cpu().double()
+                 for t in (tables, wide))
+    assert float((fp32 != 0).double().mean()) > 0.9 and float(fp32.abs().max()) <= 2.0 ** -18 * up
+    assert bool(((got - fp32).abs() <= torch.finfo(dtype).eps * fp32.abs()).all())
