@@ -39,6 +39,11 @@ __device__ __forceinline__ void da_unpack8(const uint4& x, float (&f)[8]) {
 }
 
 template <int DTYPE>
+__device__ __forceinline__ float da_unpack(unsigned short x) {
+  return DTYPE == FC_BF16 ? fc_bf16_to_float(x) : fc_half_to_float(x);
+}
+
+template <int DTYPE>
 __device__ __forceinline__ unsigned short da_pack(float f) {
   return DTYPE == FC_BF16 ? fc_float_to_bf16(f) : fc_float_to_half(f);
 }
@@ -443,7 +448,8 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 // 500 to 3500 keys, 12 seeds), this kernel / the split kernel: logits of deviation 1, fp16 2.03 / 2.10e-7, bf16
 // 1.85 / 1.97e-7; of deviation 3, 1.003 and 1.002 of it; of deviation 6, 1.000 and 0.999 (two fp16 operands, and operands
 // added to the output one by one: 1.010 and 1.014, 1.012 and 1.016, 1.002 and 1.004 of the split kernel's).
-// (An infinite value in V gives NaN: a term of its probability is zero or negative.  In fp32 it gave an infinity.)
+// An infinite value in V meets operands that are zero or negative; what is no number after the last tile is formed again
+// with the probabilities in fp32.
 #define DC_WAVES 8
 #define DC_THREADS (DC_WAVES * 64)
 #define DC_HEADS 16
@@ -636,16 +642,19 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   char* v_put = vst + qd * DC_VROW + l15 * 16;                    // row 4 u + qd: u * 4 * DC_VROW further
   const char* v_get = vst + 4 * qd * DC_VROW + l15 * 2;           // key 4 qd + j (and 16 further), dimension db * 16 + l15
   const int tiles = (end - t0 + DA_TILE - 1) / DA_TILE, last = tiles - 1;
-  // One tile: its logits, its V rows into LDS; then the next V tile and the K tile after the next start loading into
-  // the registers that became free (past the last tile they re-read it: unconditional loads keep the tiles in registers).
-  auto use_tile = [&](da_u32x4 (&kf)[8], da_u32x4 (&vf)[8], int tile) {
-    f32x4 s[2];
+  auto dot = [&](const da_u32x4 (&kf)[8], f32x4 (&s)[2]) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) s[kb] = da_mfma16<DTYPE>(__builtin_bit_cast(uint4, kf[kb * 4 + ks]), qf[ks], s[kb]);
     }
+  };
+  // One tile: its logits, its V rows into LDS; then the next V tile and the K tile after the next start loading into
+  // the registers that became free (past the last tile they re-read it: unconditional loads keep the tiles in registers).
+  auto use_tile = [&](da_u32x4 (&kf)[8], da_u32x4 (&vf)[8], int tile) {
+    f32x4 s[2];
+    dot(kf, s);
 #pragma unroll
     for (int u = 0; u < 8; ++u) *reinterpret_cast<da_u32x4*>(v_put + u * 4 * DC_VROW) = vf[u];
     if (tile + DC_WAVES < tiles) {
@@ -717,9 +726,61 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     }
   }
 
-  // ---- the eight wavefronts' results into one ---------------------------------------------------------------------
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
+  // Results that are no number, formed again with the probabilities in fp32: an infinity in V gives an infinity then, unless
+  // its key weighs nothing.  Never taken with finite keys and values; the question costs 16 comparisons a lane.
+  bool redo = false;
+#pragma unroll
+  for (int db = 0; db < 8; ++db)
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) redo |= __builtin_isunordered(o[db][i], o[db][i + 1]);
+  if (__builtin_expect(__any(redo), 0)) {
+#pragma unroll
+    for (int db = 0; db < 8; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float ref = m == -INFINITY ? 0.f : m;
+    for (int t = wave; t < tiles; t += DC_WAVES) {
+      da_u32x4 kf[8], vf[8];
+      f32x4 s[2];
+      load_k(kf, t);
+      load_v(vf, t);
+      dot(kf, s);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) *reinterpret_cast<da_u32x4*>(v_put + u * 4 * DC_VROW) = vf[u];
+      float p[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = __builtin_amdgcn_exp2f(s[e >> 2][e & 3] * c - ref) * DA_P_SCALE(DTYPE);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const int live = end - t0 - t * DA_TILE;
+#pragma unroll 1
+      for (int e = 0; e < 8; ++e) {
+        const float own = p[0];
+#pragma unroll
+        for (int j = 0; j < 7; ++j) p[j] = p[j + 1];
+#pragma unroll 1
+        for (int k4 = 0; k4 < 4; ++k4) {
+          const int key = (e >> 2) * 16 + k4 * 4 + (e & 3);
+          const float pk = __shfl(own, k4 * 16 + l15, 64);
+          if (key >= live) continue;                           // wave-uniform
+          const char* r = vst + key * DC_VROW + qd * 8;
+#pragma unroll
+          for (int db = 0; db < 8; ++db) {
+            const uint2 x = *reinterpret_cast<const uint2*>(r + db * 32);
+            const unsigned w[2] = {x.x, x.y};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[db][i] = fmaf(pk, da_unpack<DTYPE>((unsigned short)(w[i >> 1] >> (i & 1) * 16)), o[db][i]);
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  }
+
+  // ---- the eight wavefronts' results into one ---------------------------------------------------------------------
   float2* ml = reinterpret_cast<float2*>(smem + DC_PART);   // [wavefront][head]: maximum, sum
   if (qd == 0) ml[wave * DC_HEADS + l15] = make_float2(m, l);
   __syncthreads();                                         // also: every wavefront is done with its V rows

@@ -487,3 +487,38 @@ def test_probabilities_of_up_to_four_heads_keep_24_bits(dev, dtype, Hq, Hkv, n):
                  for t in (tables, wide))
     assert float((fp32 != 0).double().mean()) > 0.9 and float(fp32.abs().max()) <= 2.0 ** -18 * up
     assert bool(((got - fp32).abs() <= torch.finfo(dtype).eps * fp32.abs()).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,wide", [(2, 2, 0), (4, 2, 0), (8, 2, 0), (14, 2, 0), (32, 2, 0),
+                                         (2, 2, 70), (8, 2, 70)])     # a table too wide for the column kernel
+@pytest.mark.parametrize("lens", [[64, 250], [700, 300], [1500, 40] * 15])      # one workgroup a column; several; tiles per wavefront
+def test_infinite_values_stay_infinite(dev, dtype, Hq, Hkv, wide, lens):
+    """An infinity in V reaches the outputs of its dimension, with its sign and as that, whatever its key weighs above
+    nothing: the largest weight, those of the other keys, 2^-60; two of different sign and NaN give NaN; the other dimensions
+    are those of a cache without."""
+    from fastcache_amd.layers.attention import decode_attention
+    B, scale = len(lens), 128 ** -0.5
+    case = synth.make_paged_case(seed=12, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=lens, dtype=dtype)
+    pool, tables = case.kv_cache[:, 0].clone(), case.table_tensor("cpu", wide or None)
+    q = torch.randn(B, Hq, 128, generator=torch.Generator().manual_seed(1)).to(dtype)
+    q[..., 0] = 16
+    pool[0, ..., 0] = 0
+    inf, at = float("inf"), lambda b, t: (case.block_tables[b][t // 256], t % 256)
+    for b, n in enumerate(lens):
+        pool[(0, *at(b, 9))][:, 0], pool[(0, *at(b, n // 2))][:, 0] = 8, -32       # about 2^16 and 2^-65 of the others' weight
+        v = [pool[(1, *at(b, t))] for t in (9, n // 2, 3, n - 2)]
+        v[0][:, 5], v[0][:, 6], v[1][:, 7], v[1][:, 8], v[2][:, 64], v[3][:, 127] = inf, -inf, inf, -inf, inf, -inf
+        v[0][:, 30], v[1][:, 30], v[2][:, 31] = inf, -inf, float("nan")
+    tables_d, lens_t = tables.to(dev), torch.tensor(lens, dtype=torch.int32)
+    got = decode_attention(q.to(dev), pool[0].to(dev), pool[1].to(dev), lens_t.to(dev), tables_d, scale).cpu().float()
+    special = [5, 6, 7, 8, 30, 31, 64, 127]
+    assert bool((got[..., [5, 7, 64]] == inf).all()) and bool((got[..., [6, 8, 127]] == -inf).all())
+    assert bool(got[..., [30, 31]].isnan().all())
+    finite = pool.clone()
+    finite[1, ..., special] = 0
+    ref = oattn.decode_attention(q, finite[0], finite[1], lens_t, tables, scale).float()
+    rest = [d for d in range(128) if d not in special]
+    # one key carries nearly all of the weight: outputs are as large as values, and both sides round theirs once (a step of
+    # the type apart where the fp32 results, 1e-5 apart at most, lie on two sides of a middle)
+    assert bool(((got - ref)[..., rest].abs() <= torch.finfo(dtype).eps * ref[..., rest].abs() + 1e-5).all())
