@@ -269,7 +269,7 @@ PyObject* py_ccm_layers(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 bool press_takes(const at::Tensor& k, const at::Tensor& v, int64_t n) {
   return k.is_cuda() && v.device() == k.device() && k.dim() == 4 && k.sizes() == v.sizes() &&
          k.scalar_type() == v.scalar_type() && k.stride(3) == 1 && v.stride(3) == 1 && n > 0 && n <= k.size(2) &&
-         k.numel() > 0 && k.size(2) <= 36864;
+         k.numel() > 0 && k.size(2) <= FC_SELECT_MAX_KEYS;
 }
 
 PyObject* pair(at::Tensor a, at::Tensor b) {
@@ -758,10 +758,9 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
           q.size(0) != L || q.size(1) != B || q.size(3) != W || q.size(4) != D || W <= 0 || q.size(2) % H)
         Py_RETURN_NONE;
       hq = q.size(2);
-      nsplit = fits ? fc_snapkv_select_splits_ragged(&kv, (int32_t)hq, (int32_t)W, (int32_t)as_int(item(7)))
-                    : fc_snapkv_select_splits(&kv, (int32_t)hq, (int32_t)W);
-      one = fits && nsplit == 1;
-      if (!one && (S > 36864 || (hq / H) * ((W + 31) / 32) > 16)) Py_RETURN_NONE;
+      nsplit = fc_snapkv_rows_route(&kv, (int32_t)hq, (int32_t)W, fits, (int32_t)as_int(item(7)));
+      if (nsplit < 0) Py_RETURN_NONE;
+      one = nsplit == 0;
     }
     const int32_t *counts = nullptr, *order = nullptr;
     at::Tensor numbers;      // kept until the launches are enqueued

@@ -902,6 +902,16 @@ extern "C" int32_t fc_snapkv_select_splits_ragged(const fc_kv_view* keys, int32_
   return 1;
 }
 
+extern "C" int32_t fc_snapkv_rows_route(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t fits,
+                                        int32_t mean_len) {
+  if (!keys || keys->num_kv_heads <= 0 || window <= 0) return -1;
+  const int32_t n = fits ? fc_snapkv_select_splits_ragged(keys, num_q_heads, window, mean_len)
+                         : fc_snapkv_select_splits(keys, num_q_heads, window);
+  if (fits && n == 1) return 0;
+  const int blocks = num_q_heads / keys->num_kv_heads * ((window + 31) / 32);
+  return keys->max_seq_len <= FC_SELECT_MAX_KEYS && blocks <= 16 ? n : -1;
+}
+
 extern "C" int64_t fc_snapkv_split_workspace_bytes(int32_t num_layers, int32_t batch, int32_t num_q_heads,
                                                    int32_t num_kv_heads, int32_t window, int32_t score_stride,
                                                    int32_t nsplit) {
@@ -1015,8 +1025,8 @@ static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_
   const int stride = keys->max_seq_len;
   FC_REQUIRE(n_kept || (k > window && k <= index_stride), FC_EINVAL, "%s: k=%d must exceed the window (%d) and fit %d", who, k,
              window, index_stride);
-  FC_REQUIRE(index_stride <= stride && stride <= CS_MAX_KEYS, FC_EUNSUPPORTED, "%s: index_stride %d, max_seq_len %d (at most %d)",
-             who, index_stride, stride, CS_MAX_KEYS);
+  FC_REQUIRE(index_stride <= stride && stride <= FC_SELECT_MAX_KEYS, FC_EUNSUPPORTED,
+             "%s: index_stride %d, max_seq_len %d (at most %d)", who, index_stride, stride, FC_SELECT_MAX_KEYS);
   ColumnSelect a{};
   a.stride = stride;
   a.k = k;

@@ -18,7 +18,6 @@ struct ColumnSelect {
 };
 
 enum { CS_SCORES = 0, CS_SUMS = 1, CS_NORMS = 2 };
-#define CS_MAX_KEYS (512 * 72)   // keys of a column, held in registers
 #define CS_WIDE 4096               // longer columns are selected by 1024 threads
 #define CS_NORMS_MAX 4096         // columns that the gathering workgroups score themselves: their scores lie in LDS
 

@@ -162,7 +162,8 @@ __global__ __launch_bounds__(THREADS, KPT > 16 ? 4 : 1) void column_select_kerne
 int fc_column_select(const char* who, int src, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
                      const fc_kv_view* out_v, ColumnSelect a, hipStream_t st) {
   const int n = keys->max_seq_len;
-  FC_REQUIRE(n <= CS_MAX_KEYS, FC_EUNSUPPORTED, "%s: %d keys in a column (at most %d)", who, n, CS_MAX_KEYS);
+  static_assert(512 * 72 >= FC_SELECT_MAX_KEYS, "the longest rows are held by 512 threads of 72 keys");
+  FC_REQUIRE(n <= FC_SELECT_MAX_KEYS, FC_EUNSUPPORTED, "%s: %d keys in a column (at most %d)", who, n, FC_SELECT_MAX_KEYS);
   const int parts = a.parts > 0 ? a.parts : 1;
   a.part_rows = a.parts > 0 ? (a.index_stride + parts - 1) / parts : 0;
   const KvView kv = fc_make_view(keys), vv = fc_make_view(values);

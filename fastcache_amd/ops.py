@@ -265,11 +265,19 @@ def snapkv_select_splits(keys: FcKvView, num_q_heads: int, window: int) -> int:
     return int(fn("fc_snapkv_select_splits")(C.byref(keys), num_q_heads, window))
 
 
+def snapkv_rows_route(keys: FcKvView, num_q_heads: int, window: int, fits: bool, mean_len: int) -> int:
+    """The launches of a press whose caller wants the moved rows alone: 0 = :func:`snapkv_press`, n > 0 =
+    :func:`snapkv_select` in n key ranges per column, then :func:`compact`, -1 = neither."""
+    return int(fn("fc_snapkv_rows_route")(C.byref(keys), num_q_heads, window, int(fits), mean_len))
+
+
 def snapkv_select(keys: FcKvView, queries: torch.Tensor, window: int, kernel_size: int, k: int,
                   causal_window: bool = True, reduction: str = "mean", scale: Optional[float] = None,
-                  lse: Optional[torch.Tensor] = None, n_kept: Optional[torch.Tensor] = None) -> torch.Tensor:
+                  lse: Optional[torch.Tensor] = None, n_kept: Optional[torch.Tensor] = None,
+                  splits: Optional[int] = None) -> torch.Tensor:
     """The indices ``snapkv_score`` + ``topk_select`` give for counts above the window, without a score tensor:
-    int32 ``[L, B, Hkv, k]`` (entries past a row's count ``n_kept[b]`` are left as they are)."""
+    int32 ``[L, B, Hkv, k]`` (entries past a row's count ``n_kept[b]`` are left as they are).  ``splits``: key ranges per
+    column; default :func:`snapkv_select_splits`."""
     queries = queries.contiguous()
     _lib.require_gpu(queries, "queries")
     L, B, Hq, W, D = queries.shape
@@ -287,7 +295,7 @@ def snapkv_select(keys: FcKvView, queries: torch.Tensor, window: int, kernel_siz
             raise FastcacheError(f"lse must be fp32 [L={L}, B={B}, Hq={Hq}, W={W}], got {lse.dtype} {tuple(lse.shape)}")
         lse = lse.contiguous()
     n_kept = _i32(n_kept, "n_kept", dev)
-    nsplit = snapkv_select_splits(keys, Hq, W)
+    nsplit = snapkv_select_splits(keys, Hq, W) if splits is None else splits
     nbytes = int(fn("fc_snapkv_select_workspace_bytes")(L, B, Hq, H, W, S, nsplit))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     idx = torch.empty((L, B, H, k), dtype=torch.int32, device=dev)

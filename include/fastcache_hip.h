@@ -200,11 +200,15 @@ int fc_snapkv_score_split(const fc_kv_view* keys, const void* queries, const flo
                           float* scores, int32_t score_stride, float* row_max, int32_t nsplit, void* workspace,
                           int64_t workspace_bytes, void* stream);
 
+/* The longest columns of the selections that hold a column's keys in registers and LDS (fc_snapkv_select,
+ * fc_snapkv_press_into, fc_knorm_press_into). */
+#define FC_SELECT_MAX_KEYS 36864
+
 /*
  * SnapKV scoring and selection without a score tensor: the window positions and the k - window (n_kept[b] - window) best of
  * the other keys of every (layer, b, kv head) row, ascending, as fc_snapkv_score + fc_snapkv_fill_window +
  * fc_topk_select give for k > window (up to scored keys that tie exactly with the layer's largest score).  A sequence no
- * longer than the window keeps its first k positions.  At most 36864 tokens per sequence.  nsplit: workgroups per column
+ * longer than the window keeps its first k positions.  At most FC_SELECT_MAX_KEYS tokens per sequence.  nsplit: workgroups per column
  * (fc_snapkv_select_splits picks one); workspace: fc_snapkv_select_workspace_bytes.
  * fc_snapkv_press_into also gathers the kept K and V rows into out_k / out_v, which must not overlap the sources
  * (indices: as for fc_knorm_press_into).
@@ -213,6 +217,10 @@ int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q_heads, int
 /* The same for a batch of sequences of different lengths whose columns, whole, start longest first
  * (fc_snapkv_press_ordered): mean_len is the sequences' mean length, the view's max_seq_len their largest. */
 int32_t fc_snapkv_select_splits_ragged(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len);
+/* The launches of a press whose caller wants the moved rows alone: 0 = whole columns in one launch (fc_snapkv_press or
+ * fc_snapkv_press_ordered), n > 0 = fc_snapkv_select with nsplit n, then fc_compact, -1 = neither takes the shape.  fits:
+ * whether the one launch takes it (it needs the score row and the kept positions in LDS); mean_len as above. */
+int32_t fc_snapkv_rows_route(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t fits, int32_t mean_len);
 int64_t fc_snapkv_select_workspace_bytes(int32_t num_layers, int32_t batch, int32_t num_q_heads, int32_t num_kv_heads,
                                          int32_t window, int32_t max_seq_len, int32_t nsplit);
 int fc_snapkv_select(const fc_kv_view* keys, const void* queries, const float* lse, int32_t num_q_heads,

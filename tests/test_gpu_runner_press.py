@@ -402,3 +402,35 @@ def test_rows_only_moves_the_rows_of_the_general_path(dev, press, L, H, hq, lens
             m = min(256, rows - i * 256)
             page = int(tables[b, i])
             assert torch.equal(got[:, :, page, :m].view(torch.int16), want[:, :, page, :m].view(torch.int16)), (b, i)
+
+
+@pytest.mark.parametrize("L,H,hq,lens", [
+    (4, 2, 8, [600, 64]),           # cut by the longest length alone, whole by the lengths of the batch
+    (4, 2, 8, [600, 590]),          # cut
+    (16, 4, 28, [1100, 333, 64, 901, 700]),
+])
+def test_rows_only_general_path_launches_what_the_host_module_does(dev, monkeypatch, L, H, hq, lens):
+    """Where the host module's call declines, the same rule decides between whole columns and key ranges: the calls it
+    makes instead are those of ``fc_snapkv_rows_route`` for the batch's lengths, and the pool is the same."""
+    import ctypes
+    from fastcache_amd import _lib, ops
+    torch.manual_seed(5)
+    B, W, per = len(lens), 32, -(-max(lens) // 256)
+    pool = torch.randn((2, L, B * per + 1, 256, H, 128), device=dev).to(torch.bfloat16)
+    tables = torch.randperm(B * per + 1, device=dev)[:B * per].view(B, per).int().contiguous()
+    lens_d = torch.tensor(lens, dtype=torch.int32, device=dev)
+    queries = torch.randn((L, B, hq, W, 128), device=dev).to(torch.bfloat16)
+    got, want = pool.clone(), pool.clone()
+    paged_press.snapkv_compress_paged(want, tables, lens_d, max(lens), queries, 0.2, window_size=W, host_lens=lens, rows_only=True)
+    called = []
+    for name in ("snapkv_press", "snapkv_select", "snapkv_score"):
+        def spy(*args, _call=getattr(ops, name), _name=name, **kwargs):
+            called.append((_name, kwargs.get("splits")))
+            return _call(*args, **kwargs)
+        monkeypatch.setattr(ops, name, spy)
+    monkeypatch.setattr(paged_press, "_press_rows", lambda *a, **k: False)
+    paged_press.snapkv_compress_paged(got, tables, lens_d, max(lens), queries, 0.2, window_size=W, host_lens=lens, rows_only=True)
+    kview = _lib.paged_view(got[0], tables, lens_d, max(lens))
+    route = _lib.fn("fc_snapkv_rows_route")(ctypes.byref(kview), hq, W, 1, sum(lens) // B)
+    assert called == [("snapkv_press", None) if route == 0 else ("snapkv_select", route)]
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

@@ -558,3 +558,27 @@ def test_snapkv_splits_of_sequences_of_different_lengths():
             for mean in (0, 1, S // 2, S - 1, S, S + 5):
                 equal, ragged = both(L, B, H, hq, S, W, mean)
                 assert ragged in (1, equal), (L, B, H, S, mean)
+
+
+def test_snapkv_rows_route_is_the_split_rules():
+    """0 where the one launch takes the shape and its rule leaves columns whole, else the ranges of the rule that applies,
+    and -1 past the selection's keys or with more than 16 blocks of window queries."""
+    import ctypes
+    from fastcache_amd import _lib
+
+    def route(L, B, H, hq, S, W, fits, mean):
+        v = _lib.FcKvView(num_layers=L, batch=B, num_kv_heads=H, max_seq_len=S, block_size=256, block_tables=1, stride_token=H * 128)
+        return (_lib.fn("fc_snapkv_rows_route")(ctypes.byref(v), hq, W, fits, mean),
+                _lib.fn("fc_snapkv_select_splits")(ctypes.byref(v), hq, W),
+                _lib.fn("fc_snapkv_select_splits_ragged")(ctypes.byref(v), hq, W, mean))
+
+    for L, B, H, hq, W in ((4, 2, 2, 8, 32), (28, 5, 4, 28, 32), (36, 8, 8, 32, 64), (28, 8, 4, 28, 64)):
+        for S in (100, 600, 4000, 9000, 36864):
+            for mean in (S // 3, S):
+                got, equal, ragged = route(L, B, H, hq, S, W, 1, mean)
+                assert got == (0 if ragged == 1 else ragged)
+                assert route(L, B, H, hq, S, W, 0, mean)[0] == equal
+    assert route(4, 2, 2, 8, 600, 32, 1, 180) == (0, 5, 1)
+    assert route(4, 2, 2, 8, 36865, 32, 0, 36865)[0] == -1
+    assert route(4, 2, 1, 17, 600, 32, 0, 600)[0] == -1          # 17 blocks
+    assert route(2000, 1, 1, 4, 36865, 32, 1, 36865)[0] == 0     # whole columns need no selection of their own
