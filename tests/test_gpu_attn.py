@@ -338,8 +338,9 @@ def test_keys_of_infinite_distance_weigh_nothing(dev, dtype, lens, max_pages):
 ])
 def test_last_workgroup_merges_as_the_merge_launch(dev, dtype, Hq, Hkv, lens, pages):
     """A column's ranges merged by its last workgroup (streams of torch, outside capture) against the launch that merges
-    (inside a captured graph, and on streams whose handle torch does not own): the same bits, launch after launch, with two
-    streams at work at once, and the oracle's values."""
+    (inside a captured graph, and on streams whose handle torch does not own): which kernels ran, and the same bits, launch
+    after launch, with two streams at work at once, and the oracle's values.  Outputs lie where NaN was: a launch that found
+    its counters not at zero would leave them."""
     from fastcache_amd.layers import Attention
     from fastcache_amd.utils.context import reset_context, set_context
     B = len(lens)
@@ -357,26 +358,48 @@ def test_last_workgroup_merges_as_the_merge_launch(dev, dtype, Hq, Hkv, lens, pa
     layer.k_cache, layer.v_cache = on_gpu[0], on_gpu[1]
     q, k, v = q.to(dev), k.to(dev), v.to(dev)
     set_context(False, slot_mapping=slots.to(dev), context_lens=lens_t.to(dev), block_tables=tables.to(dev))
+
+    def call():
+        torch.full((B, Hq * 128), float("nan"), dtype=dtype, device=dev)       # freed: the output's memory
+        return layer(q, k, v)
+
+    def kernels(fn):
+        """(whether its columns merge themselves, launches of decode_merge_kernel) of the one decode layer in ``fn``"""
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
+            fn()
+            torch.cuda.synchronize()
+        names = [e.name for e in prof.events()]
+        column = [n for n in names if "decode_column_kernel<" in n]
+        assert len(column) == 1, names
+        return column[0].split(">")[0].endswith("true"), sum("decode_merge_kernel" in n for n in names)
+
+    last, launch = (True, 0), (False, 1)
+    eager = last if pages <= 14 else launch
     try:
         side = [torch.cuda.Stream(), torch.cuda.Stream()]
         foreign = torch.cuda.ExternalStream(torch.cuda.Stream().cuda_stream)
         torch.cuda.synchronize()
-        outs = [layer(q, k, v) for _ in range(3)]
+        outs = [call() for _ in range(3)]
+        assert kernels(lambda: outs.append(call())) == eager
         for _ in range(4):                                       # two streams at once
             for s in side:
                 with torch.cuda.stream(s):
-                    outs.append(layer(q, k, v))
+                    outs.append(call())
         torch.cuda.synchronize()
+        with torch.cuda.stream(side[1]):
+            assert kernels(lambda: outs.append(call())) == eager
         with torch.cuda.stream(foreign):
-            merged = layer(q, k, v)
+            merged = call()
+            assert kernels(lambda: outs.append(call())) == launch
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             held = layer(q, k, v)
+        assert kernels(graph.replay) == launch
         for _ in range(3):
             held.zero_()
             graph.replay()
-            outs.append(layer(q, k, v))
+            outs.append(call())
             torch.cuda.synchronize()
             assert torch.equal(held.view(torch.int16), merged.view(torch.int16))
     finally:
