@@ -10,7 +10,8 @@
 //   phase 1  logits: one v_mfma_f32_32x32x16 block per tile, query heads as (zero-padded) rows;
 //   phase 2  chunk softmax statistics (max, sum of exp2), one wavefront per query head;
 //   phase 3  sum of p * V rows from LDS: on the VALU, 8 output dims per lane, 16 partial sums folded through
-//            LDS; for 8 heads per workgroup on the matrix pipe with V read transposed from LDS;
+//            LDS; for 8 heads per workgroup on the matrix pipe with V read transposed from LDS (there an infinity in V
+//            gives NaN: the second half of its probability is zero or negative);
 // Each chunk writes (max, sum, unnormalised output) to the workspace; a second kernel merges the
 // chunks of a sequence.  Grid sizes depend only on the view's max_seq_len, never on the lengths on
 // the device, so both launches can be replayed from a graph while the lengths grow.
@@ -1047,9 +1048,9 @@ static bool da_tile_in_page(const fc_kv_view* v) {
          (v->block_tables == nullptr || (v->block_size >= DA_TILE && (v->block_size & (v->block_size - 1)) == 0));
 }
 
-// Tokens per workgroup of the column kernel, 0 = the launch does not take it.  Only launches whose workgroups are all
-// resident at once (one per compute unit: registers) do, and a few more: beyond that bandwidth counts and the split kernel streams
-// better (128 columns of 1024 tokens: 19.4 us a layer against 19.6 to 23).  One 32-token tile per wavefront, 256 tokens, is
+// Tokens per workgroup of the column kernel, 0 = the launch does not take it.  It takes launches whose workgroups are all
+// resident at once (one per compute unit: registers) and, of groups of 5 and more heads, twice as many short columns: beyond
+// that bandwidth counts and the split kernel streams better (128 columns of 1024 tokens: 19.4 us a layer against 19.6 to 23).  One 32-token tile per wavefront, 256 tokens, is
 // the shortest chain (a second tile costs about 3 us, a merge 3.5): 12 columns of 1024 tokens 13.2 -> 10.1 us, of 256
 // tokens without a merge 7.1, 48 columns of 1024 tokens 16.9 -> 13.0.  Where 256 would be too many workgroups, columns
 // short enough for one workgroup each still gain by not being merged: 192 columns of 512 tokens 16.7 -> 15.4 us, 256 of

@@ -126,7 +126,7 @@ __device__ __forceinline__ int ml_ranked_sequence(const int* __restrict__ seg_le
 // then the largest row count any sequence can have (it bounds the loops), and a sequence whose segment gives fewer
 // than min_rows rows is left to the copy kernel below.
 // FLAT (dense views that do not overlap, nothing to keep in order): there are no columns; the c_rows rows of all
-// (sequence, head) pairs are one list of `frows` rows, and the workgroups of a (layer, plane) take 256 of them in turn.
+// (sequence, head) pairs are one list of `flat.rows` rows, and the workgroups of a (layer, plane) take 256 of them in turn.
 // The body works on ONE layer of one plane: `slayer` / `dlayer` and the weight pointers carry the layer already; a
 // workgroup takes the column groups cg0, cg0 + cg_step, ... below ncg.
 struct MlFlat { unsigned rows; FcDivisor per_pair, heads; };

@@ -777,8 +777,8 @@ static int snapkv_score_impl(const char* who, const fc_kv_view* keys, const void
                        row_max, lse, 1, (float*)nullptr, (float*)nullptr, SkPress{});                        \
   } while (0)
   // One wavefront per 32-row block of window queries, but never fewer than four: a lone wavefront has to fetch a whole
-  // key tile by itself between two barriers (one block of queries: 7.2 ms with one wavefront, 0.87 ms with four of
-  // which three only fetch, 2048 columns of 4096 keys); two blocks score 2-7 % slower with four wavefronts than with
+  // key tile by itself between two barriers (one block of queries: 7.2 ms with one wavefront, 0.87 ms with four, 2048 columns
+  // of 4096 keys; the other three multiply rows of zeros, as every wavefront past the last block does); two blocks score 2-7 % slower with four wavefronts than with
   // two, but four is what the press tail needs, and scoring and press must sum in the same order to agree bit for bit
   // (whole pass, 2048 columns of 4096 keys and 8192 of 1024: 1.37 -> 1.34 ms and 1.41 -> 1.27 ms in one launch).
 #define SK_DISPATCH2(DT, FA)                 \

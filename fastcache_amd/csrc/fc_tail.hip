@@ -240,8 +240,10 @@ static int cs_check(const char* who, const fc_kv_view* keys, const fc_kv_view* v
 // where a workgroup's share is large.  us per hook, gather inside -> apart: Knorm, 24 columns of 5000 keys, 350 rows a share
 // 30.7, 37.4; 64 of 8000, 1400 a share 91.8, 101.6; 128 of 8000, 2800 a share 210, 210; of 12000, 4200 a share 317, 309, 1200 a
 // share 160, 169; 192 of 5000, 3500 a share 200, 199; 256 of 8000, 1600 a share 205, 214, 5600 a share 417, 396; SnapKV, 24 of 7000
-// 60.5, 66.5, 128 of 7000 177, 187.  Shorter columns, two and more workgroups to a compute unit: 96 of 4000 76, 77, 64 of 2000
-// 29, 34.
+// 60.5, 66.5, 128 of 7000 177, 187.  Above 16 384 keys likewise: Knorm, 32 of 20 000, 1250 a share 113, 119, 64 of 20 000,
+// 2500 a share 227, 230, of 30 000, 3750 a share 336, 331, 128 of 20 000, 2000 a share 269, 268, 5000 a share 424, 407; SnapKV,
+// 64 of 30 000, 1500 a share 403, 406, 3750 a share 512, 506.  Shorter columns, two and more workgroups to a compute unit: 96 of
+// 4000 76, 77, 64 of 2000 29, 34.
 extern "C" int fc_press_gather_apart(int32_t columns, int32_t max_seq_len, int32_t k) {
   if (columns <= 0 || k <= 0 || max_seq_len <= CS_WIDE) return 0;
   const int parts = fc_gather_parts(columns, max_seq_len, k);
