@@ -371,14 +371,20 @@ def test_host_numbers_are_not_uploaded_under_capture(dev):
 @pytest.mark.parametrize("press", ["knorm", "snapkv"])
 @pytest.mark.parametrize("L,H,hq,lens,planes", [
     (3, 4, 8, [700], "whole"),                      # few columns: one launch / key ranges, selection, compaction
-    (3, 4, 8, [5200, 1300, 40], "whole"),           # long ones: norms / key ranges, selection, compaction, ragged
+    (3, 4, 8, [5200, 1300, 40], "whole"),           # long ones: norms, selection, compaction, ragged
+    (3, 4, 8, [5200, 1300, 60], "whole"),           # the same and key ranges: 40 keep fewer than SnapKV's window, 60 more
     (16, 4, 28, [1100, 333, 64, 901, 700], "whole"),           # some more columns than compute units: likewise
-    (16, 4, 28, [333, 1200, 64, 901, 33, 500, 77, 1024], "whole"),     # ragged, one launch, sequences no longer than the window
+    (16, 4, 28, [333, 1200, 64, 901, 33, 500, 77, 1024], "whole"),     # ragged, one launch
+    (16, 4, 28, [333, 1200, 64, 901, 32, 500, 77, 1024], "whole"),     # a sequence no longer than the window
     (16, 4, 28, [600] * 8, "layers"),               # equal lengths; a slice of the pool's layers
     (12, 8, 16, [900] * 5 + [899], "copied"),       # queries whose rows do not lie side by side: the general path
 ])
-def test_rows_only_moves_the_rows_of_the_general_path(dev, press, L, H, hq, lens, planes):
-    """The host module's call against scores, indices and compaction as calls of their own: the same pool."""
+def test_rows_only_moves_the_rows_of_the_general_path(dev, monkeypatch, press, L, H, hq, lens, planes):
+    """The host module's call (which SnapKV asks where every sequence longer than the window keeps more than it, and which
+    declines queries that do not lie side by side) against scores, indices and compaction as calls of their own: the same
+    pool."""
+    served, plain = [], paged_press._press_rows
+    monkeypatch.setattr(paged_press, "_press_rows", lambda *a, **k: served.append(plain(*a, **k)) or served[-1])
     torch.manual_seed(3)
     B, W, per = len(lens), 32, -(-max(lens) // 256)
     pool = torch.randn((2, L + 2, B * per + 1, 256, H, 128), device=dev).to(torch.bfloat16)
@@ -396,6 +402,8 @@ def test_rows_only_moves_the_rows_of_the_general_path(dev, press, L, H, hq, lens
             paged_press.knorm_compress_paged(*args, 0.4, host_lens=host, rows_only=rows_only)
         else:
             paged_press.snapkv_compress_paged(*args, queries, 0.4, window_size=W, host_lens=host, rows_only=rows_only)
+    asked = press == "knorm" or all(n <= W or paged_press.n_kept_for(n, 0.4) > W for n in lens)
+    assert served == ([not (press == "snapkv" and planes == "copied")] if asked else [])
     for b, n in enumerate(lens):
         rows = paged_press.n_kept_for(n, 0.4)
         for i in range(-(-rows // 256)):
