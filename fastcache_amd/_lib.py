@@ -82,6 +82,8 @@ SIGNATURES = {
     "fc_select_compact": (C.c_int, [_V, _V, _VP, _I, _I, _VP, _VP, _I, _VP]),
     "fc_ccm_mlp": (C.c_int, [_V, _V, C.POINTER(FcMlpWeights), _I, _I, _I, _I, _VP]),
     "fc_ccm_mlp_ragged": (C.c_int, [_V, _V, C.POINTER(FcMlpWeights), _I, _VP, _VP, _VP, _I, _I, _VP]),
+    "fc_ccm_mlp_kv": (C.c_int, [_V, _V, _V, _V, C.POINTER(FcMlpWeights), _I, _I, _I, _I, _VP]),
+    "fc_ccm_mlp_kv_ragged": (C.c_int, [_V, _V, _V, _V, C.POINTER(FcMlpWeights), _I, _VP, _VP, _VP, _I, _I, _VP]),
     "fc_ccm_mlp_layers": (C.c_int, [_VP, _VP, _V, _V, _V, _V, C.POINTER(FcMlpWeights), _I, c_i32p, c_i32p, c_i32p, _I, _I,
                                     _VP]),
     "fc_ccm_mlp_layers_into": (C.c_int, [_VP, _VP, _VP, _VP, _V, _V, _V, _V, C.POINTER(FcMlpWeights), _I, c_i32p, c_i32p, c_i32p,

@@ -463,27 +463,38 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
   }
 }
 
+// K and V of a cache: the same geometry at two places, each with weights of its own (one plane: the first of each).  Both in
+// one launch: of few columns a plane alone leaves compute units idle, and every launch ends with some idle.  us per pass of a
+// runner, a launch per plane -> one, 28 layers of 4 heads: factor 5, one sequence of 2705 tokens 148 -> 122, 4 of 5840
+// 490 -> 463, 14 of 3875 to 11626 2342 -> 2189; factor 2, 14 of 3685 to 11056 2257 -> 2193; 32 layers of 32 heads, image of
+// 576: factor 5, 8 of 607 940 -> 823, factor 2, 9 of 590 to 657 1129 -> 1034, 45 of 640 and 24 of 590 to 1158 the same.
+struct MlPlanes {
+  char* src[2];
+  char* dst[2];
+  const char* w[2][6];     // w1, b1, w2, b2, w3, b3, all layers stacked
+};
+
+// blockIdx.y = plane x layers + layer
 template <int DTYPE, int SRC_T, int DST_T, bool W1R, bool RAG>
-__global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView src, KvView dst, const char* __restrict__ w1,
-                                                            const char* __restrict__ b1, const char* __restrict__ w2,
-                                                            const char* __restrict__ b2, const char* __restrict__ w3,
-                                                            const char* __restrict__ b3, int cf, int seg_start,
+__global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_kernel(KvView src, KvView dst, MlPlanes a, int cf, int seg_start,
                                                             int c_rows, int dst_start, int hsh, int wpc, int ncols, int ncg,
                                                             const int* __restrict__ seg_start_v,
                                                             const int* __restrict__ seg_len_v,
                                                             const int* __restrict__ dst_start_v, int min_rows) {
   extern __shared__ __align__(16) char lds[];
-  long long l = blockIdx.y;
+  int pl = blockIdx.y;
   int group = blockIdx.x;
   if constexpr (RAG) {   // one workgroup per group of columns, the longest sequences' groups of all layers first
     const unsigned id = blockIdx.x + gridDim.x * blockIdx.y;
     group = (int)(id / gridDim.y);
-    l = id - (unsigned)group * gridDim.y;
+    pl = (int)(id - (unsigned)group * gridDim.y);
   }
+  const int p = pl >= src.num_layers;
+  const long long l = pl - (p ? src.num_layers : 0);
   mlp_body<DTYPE, SRC_T, DST_T, W1R, RAG>(
-      lds, src, dst, src.base + l * src.stride_layer * 2, dst.base + l * dst.stride_layer * 2, w1 + l * 128 * cf * 256,
-      b1 + l * 256, w2 + l * 128 * 256, b2 + l * 256, w3 + l * 128 * 256, b3 + l * 256, cf, seg_start, c_rows, dst_start,
-      hsh, wpc, ncols, ncg, group, gridDim.x, seg_start_v, seg_len_v, dst_start_v, min_rows);
+      lds, src, dst, a.src[p] + l * src.stride_layer * 2, a.dst[p] + l * dst.stride_layer * 2, a.w[p][0] + l * 128 * cf * 256,
+      a.w[p][1] + l * 256, a.w[p][2] + l * 128 * 256, a.w[p][3] + l * 256, a.w[p][4] + l * 128 * 256, a.w[p][5] + l * 256, cf,
+      seg_start, c_rows, dst_start, hsh, wpc, ncols, ncg, group, gridDim.x, seg_start_v, seg_len_v, dst_start_v, min_rows);
 }
 
 // ---- a list of per-layer tensors, both planes and every segment in ONE launch ---------------------------------
@@ -542,17 +553,18 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_list_kernel(KvVi
   }
 }
 
-// What the MLP leaves of a ragged segment: the seg_len % cf remainder tokens, or the whole segment of a sequence
+// What the MLP leaves of a segment (the launch's, or with the arrays each sequence's own): the seg_len % cf remainder tokens, or the whole segment of a sequence
 // too short to compress, copied to their place behind the compressed rows.  One workgroup per (head, sequence,
-// layer); 16 tokens per pass, all loaded before any is stored (destination token <= source token, ascending).
-__global__ __launch_bounds__(256) void mlp_tail_copy_kernel(KvView src, KvView dst, int cf, int min_rows, int c_max,
+// plane and layer); 16 tokens per pass, all loaded before any is stored (destination token <= source token, ascending).
+__global__ __launch_bounds__(256) void mlp_tail_copy_kernel(KvView src, KvView dst, MlPlanes a, int cf, int min_rows, int c_max,
                                                             const int* __restrict__ seg_start_v,
                                                             const int* __restrict__ seg_len_v,
-                                                            const int* __restrict__ dst_start_v, int same_place) {
-  const int h = blockIdx.x, b = blockIdx.y, l = blockIdx.z;
-  const int ss = min(max(seg_start_v[b], 0), src.max_seq_len);
-  const int sl = min(max(seg_len_v[b], 0), src.max_seq_len - ss);
-  const int ds = min(max(dst_start_v[b], 0), dst.max_seq_len);
+                                                            const int* __restrict__ dst_start_v, int seg_start, int seg_len,
+                                                            int dst_start, int same_place) {
+  const int h = blockIdx.x, b = blockIdx.y, p = (int)blockIdx.z >= src.num_layers, l = (int)blockIdx.z - (p ? src.num_layers : 0);
+  const int ss = min(max(seg_start_v ? seg_start_v[b] : seg_start, 0), src.max_seq_len);
+  const int sl = min(max(seg_len_v ? seg_len_v[b] : seg_len, 0), src.max_seq_len - ss);
+  const int ds = min(max(dst_start_v ? dst_start_v[b] : dst_start, 0), dst.max_seq_len);
   int c = sl / cf;
   if (c < min_rows) c = 0;
   c = min(min(c, c_max), dst.max_seq_len - ds);
@@ -560,8 +572,8 @@ __global__ __launch_bounds__(256) void mlp_tail_copy_kernel(KvView src, KvView d
   const int cnt = min(sl - c * cf, dst.max_seq_len - d0);
   if (cnt <= 0 || (same_place && s0 == d0)) return;
   const int sub = threadIdx.x & 15, tr = threadIdx.x >> 4;
-  const char* sb = src.base + ((long long)l * src.stride_layer + (long long)h * src.stride_head) * 2 + sub * 16;
-  char* db = dst.base + ((long long)l * dst.stride_layer + (long long)h * dst.stride_head) * 2 + sub * 16;
+  const char* sb = a.src[p] + ((long long)l * src.stride_layer + (long long)h * src.stride_head) * 2 + sub * 16;
+  char* db = a.dst[p] + ((long long)l * dst.stride_layer + (long long)h * dst.stride_head) * 2 + sub * 16;
   for (int i0 = 0; i0 < cnt; i0 += 16) {
     const int i = i0 + tr;
     uint4 row = make_uint4(0, 0, 0, 0);
@@ -642,8 +654,8 @@ static MlSplit ml_split(int batch, int heads, int max_hsh, int jobs, int c, int 
 }
 
 // The MLP launch for c > 0 rows per column: c rows for every sequence from (seg_start, dst_start), or, with the
-// three arrays, every sequence's own segment with at most c rows.
-static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weights* w, int cf,
+// three arrays, every sequence's own segment with at most c rows.  `a`: the planes, in views of src's and dst's geometry.
+static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* dst, const MlPlanes& a, int planes, int cf,
                      int seg_start, int c, int dst_start, const int32_t* seg_start_v, const int32_t* seg_len_v,
                      const int32_t* dst_start_v, int min_rows, hipStream_t st) {
   const bool rag = seg_len_v != nullptr;
@@ -658,11 +670,11 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
     return rag ? fit(src, src->max_seq_len - 1) && fit(dst, dst->max_seq_len - 1)
                : fit(src, (int64_t)seg_start + (int64_t)c * cf - 1) && fit(dst, (int64_t)dst_start + c - 1);
   };
-  const MlSplit sp = ml_split(src->batch, src->num_kv_heads, max_hsh, src->num_layers, c, cf, rag, tables_fit);
+  const MlSplit sp = ml_split(src->batch, src->num_kv_heads, max_hsh, planes * src->num_layers, c, cf, rag, tables_fit);
   const int hsh = sp.hsh, wpc = sp.wpc, gx = sp.gx;
   const int ncols = src->batch * (src->num_kv_heads >> hsh);
   const int cols_per_wg = ML_WAVES / wpc, ncg = (ncols + cols_per_wg - 1) / cols_per_wg;
-  dim3 grid(gx, src->num_layers);
+  dim3 grid(gx, planes * src->num_layers);
   const size_t lds = ML_LDS;
   KvView s = fc_make_view(src), d = fc_make_view(dst);
   auto table_mode = [&](const KvView& v, int last_token) {
@@ -678,10 +690,8 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
 #define ML_LAUNCH(DT, ST, DTT, WR, RG)                                                                                 \
   do {                                                                                                             \
     FC_ALLOW_LDS((mlp_kernel<DT, ST, DTT, WR, RG>), (int)lds);                                                    \
-    hipLaunchKernelGGL((mlp_kernel<DT, ST, DTT, WR, RG>), grid, dim3(ML_THREADS), lds, st, s, d, (const char*)w->w1, \
-                       (const char*)w->b1, (const char*)w->w2, (const char*)w->b2, (const char*)w->w3,             \
-                       (const char*)w->b3, cf, seg_start, c, dst_start, hsh, wpc, ncols, ncg, seg_start_v, seg_len_v,   \
-                       dst_start_v, min_rows);                                                                     \
+    hipLaunchKernelGGL((mlp_kernel<DT, ST, DTT, WR, RG>), grid, dim3(ML_THREADS), lds, st, s, d, a, cf, seg_start, c, \
+                       dst_start, hsh, wpc, ncols, ncg, seg_start_v, seg_len_v, dst_start_v, min_rows);            \
   } while (0)
 #define ML_DISPATCH(DT, WR)                                                         \
   if (rag) {                                                                        \
@@ -704,51 +714,116 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
   return FC_OK;
 }
 
-extern "C" int fc_ccm_mlp(const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weights* w, int32_t cf,
-                          int32_t seg_start, int32_t seg_len, int32_t dst_start, void* stream) {
-  const char* who = "fc_ccm_mlp";
-  int rc = ml_check(who, src, dst, w, cf);
+// One or two planes of one geometry (strides, tables, lengths), each with weights of its own.
+static int ml_planes(const char* who, const fc_kv_view* const src[2], const fc_kv_view* const dst[2], const fc_mlp_weights* w,
+                     int planes, int cf, MlPlanes& a) {
+  int rc;
+  for (int p = 0; p < planes; ++p) {
+    if ((rc = ml_check(who, src[p], dst[p], w ? w + p : nullptr, cf))) return rc;
+    for (const fc_kv_view* const* v : {src, dst}) {
+      const fc_kv_view& moved = *v[p];
+      FC_REQUIRE(moved.block_tables == v[0]->block_tables && moved.dtype == v[0]->dtype &&
+                     moved.num_layers == v[0]->num_layers && moved.batch == v[0]->batch &&
+                     moved.num_kv_heads == v[0]->num_kv_heads && moved.max_seq_len == v[0]->max_seq_len &&
+                     moved.stride_layer == v[0]->stride_layer && moved.stride_block == v[0]->stride_block &&
+                     moved.stride_batch == v[0]->stride_batch && moved.stride_token == v[0]->stride_token &&
+                     moved.stride_head == v[0]->stride_head && moved.block_size == v[0]->block_size &&
+                     moved.table_stride == v[0]->table_stride,
+                 FC_EINVAL, "%s: the planes' views differ in more than their place", who);
+    }
+    a.src[p] = (char*)src[p]->base;
+    a.dst[p] = (char*)dst[p]->base;
+    const void* ws[6] = {w[p].w1, w[p].b1, w[p].w2, w[p].b2, w[p].w3, w[p].b3};
+    for (int i = 0; i < 6; ++i) a.w[p][i] = (const char*)ws[i];
+  }
+  FC_REQUIRE(planes * src[0]->num_layers <= 65535, FC_EUNSUPPORTED, "%s: too many layers", who);
+  return FC_OK;
+}
+
+// remainders and pass-through segments; nothing to move when a pass-through segment already lies at its place
+static void ml_tails(const fc_kv_view* const src[2], const fc_kv_view* const dst[2], const MlPlanes& a, int planes, int cf,
+                     int min_rows, int c, const int32_t* seg_start_v, const int32_t* seg_len_v, const int32_t* dst_start_v,
+                     int seg_start, int seg_len, int dst_start, hipStream_t st) {
+  int same = 1;
+  for (int p = 0; p < planes; ++p)
+    same = same && src[p]->base == dst[p]->base && src[p]->block_tables == dst[p]->block_tables &&
+           src[p]->stride_layer == dst[p]->stride_layer && src[p]->stride_batch == dst[p]->stride_batch;
+  hipLaunchKernelGGL(mlp_tail_copy_kernel, dim3(src[0]->num_kv_heads, src[0]->batch, planes * src[0]->num_layers), dim3(256), 0, st,
+                     fc_make_view(src[0]), fc_make_view(dst[0]), a, cf, min_rows, c, seg_start_v, seg_len_v, dst_start_v,
+                     seg_start, seg_len, dst_start, same);
+}
+
+static int ml_uniform(const char* who, const fc_kv_view* const src[2], const fc_kv_view* const dst[2], const fc_mlp_weights* w,
+                      int planes, int cf, int seg_start, int seg_len, int dst_start, void* stream) {
+  MlPlanes a{};
+  int rc = ml_planes(who, src, dst, w, planes, cf, a);
   if (rc) return rc;
   FC_REQUIRE(seg_start >= 0 && seg_len >= 0 && dst_start >= 0, FC_EINVAL, "%s: negative range", who);
-  FC_REQUIRE((int64_t)seg_start + seg_len <= src->max_seq_len, FC_EINVAL,
+  FC_REQUIRE((int64_t)seg_start + seg_len <= src[0]->max_seq_len, FC_EINVAL,
              "%s: segment [%d, %d) exceeds the source view's max_seq_len %d", who, seg_start, seg_start + seg_len,
-             src->max_seq_len);
+             src[0]->max_seq_len);
   const int c = seg_len / cf;
   const int rem = seg_len - c * cf;
-  FC_REQUIRE((int64_t)dst_start + c + rem <= dst->max_seq_len, FC_EINVAL,
+  FC_REQUIRE((int64_t)dst_start + c + rem <= dst[0]->max_seq_len, FC_EINVAL,
              "%s: output [%d, %d) exceeds the destination view's max_seq_len %d", who, dst_start,
-             dst_start + c + rem, dst->max_seq_len);
-  if (c > 0 && (rc = ml_launch(who, src, dst, w, cf, seg_start, c, dst_start, nullptr, nullptr, nullptr, 0,
+             dst_start + c + rem, dst[0]->max_seq_len);
+  if (c > 0 && (rc = ml_launch(who, src[0], dst[0], a, planes, cf, seg_start, c, dst_start, nullptr, nullptr, nullptr, 0,
                                (hipStream_t)stream)))
     return rc;
-  if (rem > 0) return fc_copy_tokens(src, dst, seg_start + c * cf, rem, dst_start + c, stream);
+  if (rem > 0 && planes == 1) return fc_copy_tokens(src[0], dst[0], seg_start + c * cf, rem, dst_start + c, stream);
+  if (rem > 0) ml_tails(src, dst, a, planes, cf, 0, c, nullptr, nullptr, nullptr, seg_start, seg_len, dst_start, (hipStream_t)stream);
+  FC_CHECK_LAUNCH(who);
   return FC_OK;
+}
+
+static int ml_ragged(const char* who, const fc_kv_view* const src[2], const fc_kv_view* const dst[2], const fc_mlp_weights* w,
+                     int planes, int cf, const int32_t* seg_start, const int32_t* seg_len, const int32_t* dst_start,
+                     int max_seg_len, int min_rows, void* stream) {
+  MlPlanes a{};
+  int rc = ml_planes(who, src, dst, w, planes, cf, a);
+  if (rc) return rc;
+  FC_REQUIRE(seg_start && seg_len && dst_start, FC_EINVAL, "%s: null segment arrays", who);
+  FC_REQUIRE(max_seg_len >= 0 && max_seg_len <= src[0]->max_seq_len, FC_EINVAL,
+             "%s: max_seg_len %d outside [0, max_seq_len %d]", who, max_seg_len, src[0]->max_seq_len);
+  FC_REQUIRE(min_rows >= 0, FC_EINVAL, "%s: negative min_rows", who);
+  FC_REQUIRE(src[0]->num_kv_heads <= 65535, FC_EUNSUPPORTED, "%s: too many heads", who);
+  if (max_seg_len == 0) return FC_OK;
+  hipStream_t st = (hipStream_t)stream;
+  const int c = max_seg_len / cf;
+  if (c > 0 && c >= min_rows &&
+      (rc = ml_launch(who, src[0], dst[0], a, planes, cf, 0, c, 0, seg_start, seg_len, dst_start, min_rows, st)))
+    return rc;
+  ml_tails(src, dst, a, planes, cf, min_rows, c, seg_start, seg_len, dst_start, 0, 0, 0, st);
+  FC_CHECK_LAUNCH(who);
+  return FC_OK;
+}
+
+extern "C" int fc_ccm_mlp(const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weights* w, int32_t cf,
+                          int32_t seg_start, int32_t seg_len, int32_t dst_start, void* stream) {
+  const fc_kv_view *s[2] = {src, src}, *d[2] = {dst, dst};
+  return ml_uniform("fc_ccm_mlp", s, d, w, 1, cf, seg_start, seg_len, dst_start, stream);
+}
+
+extern "C" int fc_ccm_mlp_kv(const fc_kv_view* k_src, const fc_kv_view* k_dst, const fc_kv_view* v_src, const fc_kv_view* v_dst,
+                             const fc_mlp_weights* weights, int32_t cf, int32_t seg_start, int32_t seg_len, int32_t dst_start,
+                             void* stream) {
+  const fc_kv_view *s[2] = {k_src, v_src}, *d[2] = {k_dst, v_dst};
+  return ml_uniform("fc_ccm_mlp_kv", s, d, weights, 2, cf, seg_start, seg_len, dst_start, stream);
 }
 
 extern "C" int fc_ccm_mlp_ragged(const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weights* w, int32_t cf,
                                  const int32_t* seg_start, const int32_t* seg_len, const int32_t* dst_start,
                                  int32_t max_seg_len, int32_t min_rows, void* stream) {
-  const char* who = "fc_ccm_mlp_ragged";
-  int rc = ml_check(who, src, dst, w, cf);
-  if (rc) return rc;
-  FC_REQUIRE(seg_start && seg_len && dst_start, FC_EINVAL, "%s: null segment arrays", who);
-  FC_REQUIRE(max_seg_len >= 0 && max_seg_len <= src->max_seq_len, FC_EINVAL,
-             "%s: max_seg_len %d outside [0, max_seq_len %d]", who, max_seg_len, src->max_seq_len);
-  FC_REQUIRE(min_rows >= 0, FC_EINVAL, "%s: negative min_rows", who);
-  FC_REQUIRE(src->num_kv_heads <= 65535, FC_EUNSUPPORTED, "%s: too many heads", who);
-  if (max_seg_len == 0) return FC_OK;
-  hipStream_t st = (hipStream_t)stream;
-  const int c = max_seg_len / cf;
-  if (c > 0 && c >= min_rows &&
-      (rc = ml_launch(who, src, dst, w, cf, 0, c, 0, seg_start, seg_len, dst_start, min_rows, st)))
-    return rc;
-  // remainders and pass-through segments; nothing to move when a pass-through segment already lies at its place
-  const int same = src->base == dst->base && src->block_tables == dst->block_tables &&
-                   src->stride_layer == dst->stride_layer && src->stride_batch == dst->stride_batch;
-  hipLaunchKernelGGL(mlp_tail_copy_kernel, dim3(src->num_kv_heads, src->batch, src->num_layers), dim3(256), 0, st,
-                     fc_make_view(src), fc_make_view(dst), cf, min_rows, c, seg_start, seg_len, dst_start, same);
-  FC_CHECK_LAUNCH(who);
-  return FC_OK;
+  const fc_kv_view *s[2] = {src, src}, *d[2] = {dst, dst};
+  return ml_ragged("fc_ccm_mlp_ragged", s, d, w, 1, cf, seg_start, seg_len, dst_start, max_seg_len, min_rows, stream);
+}
+
+extern "C" int fc_ccm_mlp_kv_ragged(const fc_kv_view* k_src, const fc_kv_view* k_dst, const fc_kv_view* v_src,
+                                    const fc_kv_view* v_dst, const fc_mlp_weights* weights, int32_t cf,
+                                    const int32_t* seg_start, const int32_t* seg_len, const int32_t* dst_start,
+                                    int32_t max_seg_len, int32_t min_rows, void* stream) {
+  const fc_kv_view *s[2] = {k_src, v_src}, *d[2] = {k_dst, v_dst};
+  return ml_ragged("fc_ccm_mlp_kv_ragged", s, d, weights, 2, cf, seg_start, seg_len, dst_start, max_seg_len, min_rows, stream);
 }
 
 // k_out / v_out null: all layers of a plane in one allocation, a layer stride apart

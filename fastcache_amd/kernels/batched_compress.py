@@ -92,17 +92,18 @@ class BatchedGEMMCompressor(nn.Module):
         # one stacked copy of the layer list (the reference stacks as well, batched_compress.py:394-395)
         src = [torch.stack([kv[p] for kv in kv_cache]) for p in range(2)]
         out = [torch.empty((L, B, H, C, D), dtype=k0.dtype, device=k0.device) for _ in range(2)]
-        for p, kind in ((0, "k"), (1, "v")):
-            sv, dv = _lib.dense_view(src[p]), _lib.dense_view(out[p])
-            dst = 0
-            for seg_start, n, g in ((0, img, "i" + kind), (img, S - img, "t" + kind)):
-                if n == 0:
-                    continue
-                if n // cf < self.min_seq_len:
-                    ops.copy_tokens(sv, dv, seg_start, n, dst)
-                else:
-                    ops.ccm_mlp(sv, dv, self._weights(g, k0.dtype, k0.device, (l0, l1)), cf, seg_start, n, dst)
-                dst += self._seg_len(n)
+        sv, dv = [_lib.dense_view(t) for t in src], [_lib.dense_view(t) for t in out]
+        dst = 0
+        for seg_start, n, seg in ((0, img, "i"), (img, S - img, "t")):
+            if n == 0:
+                continue
+            if n // cf < self.min_seq_len:
+                for p in range(2):
+                    ops.copy_tokens(sv[p], dv[p], seg_start, n, dst)
+            else:
+                w = [self._weights(seg + kind, k0.dtype, k0.device, (l0, l1)) for kind in "kv"]
+                ops.ccm_mlp_kv(sv, dv, w, cf, seg_start, n, dst)
+            dst += self._seg_len(n)
         return [(out[0][i], out[1][i]) for i in range(L)]
 
     def paged_compressed_len(self, seq_len: int, it_len: Sequence[int]) -> int:
@@ -138,23 +139,22 @@ class BatchedGEMMCompressor(nn.Module):
                 plan.append((seg, max(counts), [xs[0] for xs in where] if same else _lib.upload_rows(where, kv_cache), same))
                 dsts = [d + self._seg_len(n) for d, n in zip(dsts, counts)]
             for seg, n_max, (st, ct, dt), same in plan:
-                for view, dview, kind in ((views[0], dviews[0], "k"), (views[1], dviews[1], "v")):
-                    w = self._weights(seg + kind, kv_cache.dtype, dev, (l0, l1))
-                    if same:
-                        ops.ccm_mlp(view, dview, w, cf, st, ct, dt)
-                    else:
-                        ops.ccm_mlp_ragged(view, dview, w, cf, st, ct, dt, n_max, self.min_seq_len)
+                w = [self._weights(seg + kind, kv_cache.dtype, dev, (l0, l1)) for kind in "kv"]
+                if same:
+                    ops.ccm_mlp_kv(views, dviews, w, cf, st, ct, dt)
+                else:
+                    ops.ccm_mlp_kv_ragged(views, dviews, w, cf, st, ct, dt, n_max, self.min_seq_len)
             return dsts
         for s0, n, seg in ((0, img, "i"), (img, seq_len - img, "t")):
             if n == 0:
                 continue
-            for view, dview, kind in ((views[0], dviews[0], "k"), (views[1], dviews[1], "v")):
-                if n // cf < self.min_seq_len:
-                    if out is not None or dst != s0:
+            if n // cf < self.min_seq_len:
+                if out is not None or dst != s0:
+                    for view, dview in zip(views, dviews):
                         ops.copy_tokens(view, dview, s0, n, dst)
-                else:
-                    ops.ccm_mlp(view, dview, self._weights(seg + kind, kv_cache.dtype, kv_cache.device, (l0, l1)), cf,
-                                s0, n, dst)
+            else:
+                w = [self._weights(seg + kind, kv_cache.dtype, kv_cache.device, (l0, l1)) for kind in "kv"]
+                ops.ccm_mlp_kv(views, dviews, w, cf, s0, n, dst)
             dst += self._seg_len(n)
         return dst
 

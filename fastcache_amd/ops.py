@@ -425,20 +425,39 @@ def copy_tokens_from_layers(layers, dst: FcKvView, count: int, dst_start: int = 
 # ---------------------------------------------------------------------------------------------
 # CCM MLP
 # ---------------------------------------------------------------------------------------------
-def ccm_mlp(src: FcKvView, dst: FcKvView, weights: Tuple[torch.Tensor, ...], cf: int, seg_start: int,
-            seg_len: int, dst_start: int) -> None:
-    """weights = (w1 [L,128,cf*128], b1 [L,128], w2 [L,128,128], b2, w3, b3) in the KV dtype."""
-    w1, b1, w2, b2, w3, b3 = weights
-    L = src.num_layers
-    D = src.head_dim
+def _mlp_weights(view: FcKvView, weights: Tuple[torch.Tensor, ...], cf: int) -> FcMlpWeights:
+    L, D = view.num_layers, view.head_dim
     shapes = [(L, D, cf * D), (L, D), (L, D, D), (L, D), (L, D, D), (L, D)]
     for t, shp, name in zip(weights, shapes, ("w1", "b1", "w2", "b2", "w3", "b3")):
         _lib.require_gpu(t, name)
-        if tuple(t.shape) != shp or not t.is_contiguous() or _lib.dtype_code(t.dtype) != src.dtype:
+        if tuple(t.shape) != shp or not t.is_contiguous() or _lib.dtype_code(t.dtype) != view.dtype:
             raise FastcacheError(f"{name} must be contiguous {shp} in the KV dtype, got {tuple(t.shape)} {t.dtype}")
-    w = FcMlpWeights(*(t.data_ptr() for t in weights))
+    return FcMlpWeights(*(t.data_ptr() for t in weights))
+
+
+def ccm_mlp(src: FcKvView, dst: FcKvView, weights: Tuple[torch.Tensor, ...], cf: int, seg_start: int,
+            seg_len: int, dst_start: int) -> None:
+    """weights = (w1 [L,128,cf*128], b1 [L,128], w2 [L,128,128], b2, w3, b3) in the KV dtype."""
+    w = _mlp_weights(src, weights, cf)
     check(fn("fc_ccm_mlp")(C.byref(src), C.byref(dst), C.byref(w), cf, seg_start, seg_len, dst_start,
                            current_stream()), "fc_ccm_mlp")
+
+
+def ccm_mlp_kv(srcs, dsts, weights, cf: int, seg_start: int, seg_len: int, dst_start: int) -> None:
+    """``ccm_mlp`` of both planes in one launch: pairs (K, V) of views that differ in their place only, and of weights."""
+    w = (FcMlpWeights * 2)(*(_mlp_weights(s, x, cf) for s, x in zip(srcs, weights)))
+    check(fn("fc_ccm_mlp_kv")(C.byref(srcs[0]), C.byref(dsts[0]), C.byref(srcs[1]), C.byref(dsts[1]), w, cf, seg_start,
+                              seg_len, dst_start, current_stream()), "fc_ccm_mlp_kv")
+
+
+def _segment_arrays(view: FcKvView, dev, seg_start: torch.Tensor, seg_len: torch.Tensor, dst_start: torch.Tensor):
+    arrays = []
+    for t, name in ((seg_start, "seg_start"), (seg_len, "seg_len"), (dst_start, "dst_start")):
+        t = _i32(t, name, dev)
+        if t.numel() != view.batch:
+            raise FastcacheError(f"{name} must hold one entry per sequence ({view.batch}), got {t.numel()}")
+        arrays.append(t)
+    return arrays
 
 
 def ccm_mlp_ragged(src: FcKvView, dst: FcKvView, weights: Tuple[torch.Tensor, ...], cf: int,
@@ -446,23 +465,20 @@ def ccm_mlp_ragged(src: FcKvView, dst: FcKvView, weights: Tuple[torch.Tensor, ..
                    min_rows: int) -> None:
     """``ccm_mlp`` with one segment per sequence: int32 device tensors ``[B]``; a sequence whose segment has fewer
     than ``min_rows * cf`` tokens is copied through; ``max_seg_len`` bounds ``seg_len``."""
-    L, D = src.num_layers, src.head_dim
-    shapes = [(L, D, cf * D), (L, D), (L, D, D), (L, D), (L, D, D), (L, D)]
-    for t, shp, name in zip(weights, shapes, ("w1", "b1", "w2", "b2", "w3", "b3")):
-        _lib.require_gpu(t, name)
-        if tuple(t.shape) != shp or not t.is_contiguous() or _lib.dtype_code(t.dtype) != src.dtype:
-            raise FastcacheError(f"{name} must be contiguous {shp} in the KV dtype, got {tuple(t.shape)} {t.dtype}")
-    dev = weights[0].device
-    arrays = []
-    for t, name in ((seg_start, "seg_start"), (seg_len, "seg_len"), (dst_start, "dst_start")):
-        t = _i32(t, name, dev)
-        if t.numel() != src.batch:
-            raise FastcacheError(f"{name} must hold one entry per sequence ({src.batch}), got {t.numel()}")
-        arrays.append(t)
-    w = FcMlpWeights(*(t.data_ptr() for t in weights))
-    check(fn("fc_ccm_mlp_ragged")(C.byref(src), C.byref(dst), C.byref(w), cf, arrays[0].data_ptr(),
-                                  arrays[1].data_ptr(), arrays[2].data_ptr(), max_seg_len, min_rows,
-                                  current_stream()), "fc_ccm_mlp_ragged")
+    w = _mlp_weights(src, weights, cf)
+    arrays = _segment_arrays(src, weights[0].device, seg_start, seg_len, dst_start)
+    check(fn("fc_ccm_mlp_ragged")(C.byref(src), C.byref(dst), C.byref(w), cf, *(t.data_ptr() for t in arrays),
+                                  max_seg_len, min_rows, current_stream()), "fc_ccm_mlp_ragged")
+
+
+def ccm_mlp_kv_ragged(srcs, dsts, weights, cf: int, seg_start: torch.Tensor, seg_len: torch.Tensor,
+                      dst_start: torch.Tensor, max_seg_len: int, min_rows: int) -> None:
+    """``ccm_mlp_ragged`` of both planes in one launch, pairs as for ``ccm_mlp_kv``."""
+    w = (FcMlpWeights * 2)(*(_mlp_weights(s, x, cf) for s, x in zip(srcs, weights)))
+    arrays = _segment_arrays(srcs[0], weights[0][0].device, seg_start, seg_len, dst_start)
+    check(fn("fc_ccm_mlp_kv_ragged")(C.byref(srcs[0]), C.byref(dsts[0]), C.byref(srcs[1]), C.byref(dsts[1]), w, cf,
+                                     *(t.data_ptr() for t in arrays), max_seg_len, min_rows, current_stream()),
+          "fc_ccm_mlp_kv_ragged")
 
 
 def expected_attention_score(keys: FcKvView, values: FcKvView, mean_query: torch.Tensor,

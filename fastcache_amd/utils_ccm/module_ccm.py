@@ -202,13 +202,13 @@ class _CCMBase(nn.Module):
         for gk, gv, s0, n in self._paged_segments(seq_len, it_len):
             if n == 0:
                 continue
-            for view, dview, g in ((views[0], dviews[0], gk), (views[1], dviews[1], gv)):
-                if n // cf < self.min_seq_len:
-                    if out is not None or dst != s0:
+            if n // cf < self.min_seq_len:
+                if out is not None or dst != s0:
+                    for view, dview in zip(views, dviews):
                         ops.copy_tokens(view, dview, s0, n, dst)
-                else:
-                    w = self._layer_weights(g, l0, l1, kv_cache.dtype, kv_cache.device)
-                    ops.ccm_mlp(view, dview, w, cf, s0, n, dst)
+            else:
+                w = [self._layer_weights(g, l0, l1, kv_cache.dtype, kv_cache.device) for g in (gk, gv)]
+                ops.ccm_mlp_kv(views, dviews, w, cf, s0, n, dst)
             dst += self._segment_len(n)
         return dst
 
@@ -236,12 +236,11 @@ class _CCMBase(nn.Module):
             plan.append((gk, gv, n_max, [xs[0] for xs in where] if same else _lib.upload_rows(where, kv_cache), same))
             dst = [d + self._segment_len(g[3]) for d, g in zip(dst, segs)]
         for gk, gv, n_max, (starts, counts, dsts), same in plan:
-            for view, dview, g in ((views[0], dviews[0], gk), (views[1], dviews[1], gv)):
-                w = self._layer_weights(g, l0, l1, kv_cache.dtype, dev)
-                if same:
-                    ops.ccm_mlp(view, dview, w, cf, starts, counts, dsts)
-                else:
-                    ops.ccm_mlp_ragged(view, dview, w, cf, starts, counts, dsts, n_max, self.min_seq_len)
+            w = [self._layer_weights(g, l0, l1, kv_cache.dtype, dev) for g in (gk, gv)]
+            if same:
+                ops.ccm_mlp_kv(views, dviews, w, cf, starts, counts, dsts)
+            else:
+                ops.ccm_mlp_kv_ragged(views, dviews, w, cf, starts, counts, dsts, n_max, self.min_seq_len)
         return dst
 
     def _forward_layers(self, kv_cache: Sequence[LayerKV], segments) -> Optional[List[LayerKV]]:

@@ -322,6 +322,11 @@ typedef struct fc_mlp_weights {
 int fc_ccm_mlp(const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weights* w,
                int32_t cf, int32_t seg_start, int32_t seg_len, int32_t dst_start, void* stream);
 
+/* Both planes of a cache at once: weights[0] for K, weights[1] for V; the views of the two planes differ in `base` only. */
+int fc_ccm_mlp_kv(const fc_kv_view* k_src, const fc_kv_view* k_dst, const fc_kv_view* v_src, const fc_kv_view* v_dst,
+                  const fc_mlp_weights* weights, int32_t cf, int32_t seg_start, int32_t seg_len, int32_t dst_start,
+                  void* stream);
+
 /*
  * The same compressor when every sequence has its own segment (a batch of prompts of different lengths compressed in
  * one pass instead of the reference's per-sequence loop, nanovllm/engine/llava_model_runner.py:745-786):
@@ -334,6 +339,11 @@ int fc_ccm_mlp(const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weight
 int fc_ccm_mlp_ragged(const fc_kv_view* src, const fc_kv_view* dst, const fc_mlp_weights* w, int32_t cf,
                       const int32_t* seg_start, const int32_t* seg_len, const int32_t* dst_start,
                       int32_t max_seg_len, int32_t min_rows, void* stream);
+
+/* Both planes of a cache at once, as fc_ccm_mlp_kv. */
+int fc_ccm_mlp_kv_ragged(const fc_kv_view* k_src, const fc_kv_view* k_dst, const fc_kv_view* v_src, const fc_kv_view* v_dst,
+                         const fc_mlp_weights* weights, int32_t cf, const int32_t* seg_start, const int32_t* seg_len,
+                         const int32_t* dst_start, int32_t max_seg_len, int32_t min_rows, void* stream);
 
 /*
  * The same MLPs over a cache that is a list of per-layer tensors (what `forward(kv_cache, it_len)` of the compressor

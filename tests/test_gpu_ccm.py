@@ -329,3 +329,45 @@ def test_ccm_mlp_ragged_is_each_sequence_alone(dev, L, H, lens, block_size, cf):
         else:
             ops.copy_tokens(one, one, starts[b], counts[b], dsts[b])
     assert torch.equal(pool.view(torch.int16), alone.view(torch.int16))
+
+
+@pytest.mark.parametrize("lens,block_size,cf,dense", [
+    ([700], 256, 5, False),                     # one sequence: fewer columns than compute units
+    ([333, 333, 333], 256, 2, True),            # a remainder token, into tensors of its own
+    ([333, 70, 2, 211], 256, 2, False),         # lengths, among them one of a single row
+    ([90, 41, 64], 16, 3, True),
+])
+def test_ccm_mlp_both_planes_in_one_call(dev, lens, block_size, cf, dense):
+    """K and V by one call, each with its own weights: the same bytes as a call per plane."""
+    L, H, B, S = 3, 4, len(lens), max(lens)
+    per = -(-S // block_size)
+    pool = torch.empty((2, L, B * per + 1, block_size, H, 128), dtype=torch.bfloat16, device=dev).normal_()
+    tables = torch.randperm(B * per + 1, device=dev)[:B * per].view(B, per).int().contiguous()
+    w = [tuple((torch.randn(shape, device=dev) * 0.05).bfloat16()
+               for shape in ((L, 128, 128 * cf), (L, 128), (L, 128, 128), (L, 128), (L, 128, 128), (L, 128))) for _ in range(2)]
+    mk = lambda xs: torch.tensor(xs, dtype=torch.int32, device=dev)
+    got = []
+    for together in (True, False):
+        planes, out = pool.clone(), torch.zeros((2, L, B, H, S, 128), dtype=pool.dtype, device=dev)
+        src = [_lib.paged_view(planes[p], tables, mk(lens), S) for p in range(2)]
+        dst = [_lib.dense_view(out[p]) for p in range(2)] if dense else src
+        segs = [[n // 4 for n in lens], [n - n // 4 for n in lens], [n // 8 for n in lens]]
+        if len(set(lens)) == 1:
+            s, c, d = (x[0] for x in segs)
+            if together:
+                ops.ccm_mlp_kv(src, dst, w, cf, s, c, d)
+            else:
+                for p in range(2):
+                    ops.ccm_mlp(src[p], dst[p], w[p], cf, s, c, d)
+        elif together:
+            ops.ccm_mlp_kv_ragged(src, dst, w, cf, *map(mk, segs), max(segs[1]), 1)
+        else:
+            for p in range(2):
+                ops.ccm_mlp_ragged(src[p], dst[p], w[p], cf, *map(mk, segs), max(segs[1]), 1)
+        got.append((planes, out))
+    for a, b in zip(*got):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    assert torch.equal(got[0][0], pool) == dense          # in place, or the pages left alone
+    v = _lib.paged_view(planes[1], tables, mk(lens), S - 1)
+    with pytest.raises(_lib.FastcacheError, match="differ in more than their place"):
+        ops.ccm_mlp_kv([src[0], v], dst, w, cf, 0, S - 1, 0)
