@@ -553,15 +553,20 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_list_kernel(KvVi
   }
 }
 
-// What the MLP leaves of a segment (the launch's, or with the arrays each sequence's own): the seg_len % cf remainder tokens, or the whole segment of a sequence
-// too short to compress, copied to their place behind the compressed rows.  One workgroup per (head, sequence,
-// plane and layer); 16 tokens per pass, all loaded before any is stored (destination token <= source token, ascending).
-__global__ __launch_bounds__(256) void mlp_tail_copy_kernel(KvView src, KvView dst, MlPlanes a, int cf, int min_rows, int c_max,
+// What the MLP leaves of a segment (the launch's, or with the arrays each sequence's own): the seg_len % cf remainder tokens, or
+// the whole segment of a sequence too short to compress, copied to their place behind the compressed rows.  One workgroup per
+// (sequence, plane and layer) and heads_per_wg heads, whose rows are one list, tokens ascending; ML_TAIL rows per pass, all
+// loaded before any is stored (destination token <= source token).  A workgroup per head was mostly the starting of workgroups,
+// a row or two each: 24 sequences x 32 heads x 64 layers and planes 60 us, 12 like this, 8 sequences 27, 6; 4 heads the same.
+// (Several rows per thread lose: the table reads of a thread's rows wait for each other, 10 to 20 us.)
+#define ML_TAIL 32
+__global__ __launch_bounds__(16 * ML_TAIL) void mlp_tail_copy_kernel(KvView src, KvView dst, MlPlanes a, int cf, int min_rows, int c_max,
                                                             const int* __restrict__ seg_start_v,
                                                             const int* __restrict__ seg_len_v,
                                                             const int* __restrict__ dst_start_v, int seg_start, int seg_len,
-                                                            int dst_start, int same_place) {
-  const int h = blockIdx.x, b = blockIdx.y, p = (int)blockIdx.z >= src.num_layers, l = (int)blockIdx.z - (p ? src.num_layers : 0);
+                                                            int dst_start, int same_place, int heads_per_wg) {
+  const int h0 = blockIdx.x * heads_per_wg, heads = min(heads_per_wg, src.num_kv_heads - h0);
+  const int b = blockIdx.y, p = (int)blockIdx.z >= src.num_layers, l = (int)blockIdx.z - (p ? src.num_layers : 0);
   const int ss = min(max(seg_start_v ? seg_start_v[b] : seg_start, 0), src.max_seq_len);
   const int sl = min(max(seg_len_v ? seg_len_v[b] : seg_len, 0), src.max_seq_len - ss);
   const int ds = min(max(dst_start_v ? dst_start_v[b] : dst_start, 0), dst.max_seq_len);
@@ -572,19 +577,20 @@ __global__ __launch_bounds__(256) void mlp_tail_copy_kernel(KvView src, KvView d
   const int cnt = min(sl - c * cf, dst.max_seq_len - d0);
   if (cnt <= 0 || (same_place && s0 == d0)) return;
   const int sub = threadIdx.x & 15, tr = threadIdx.x >> 4;
-  const char* sb = a.src[p] + ((long long)l * src.stride_layer + (long long)h * src.stride_head) * 2 + sub * 16;
-  char* db = a.dst[p] + ((long long)l * dst.stride_layer + (long long)h * dst.stride_head) * 2 + sub * 16;
-  for (int i0 = 0; i0 < cnt; i0 += 16) {
-    const int i = i0 + tr;
+  const char* sb = a.src[p] + (long long)l * src.stride_layer * 2 + sub * 16;
+  char* db = a.dst[p] + (long long)l * dst.stride_layer * 2 + sub * 16;
+  const unsigned rows = (unsigned)cnt * heads;
+  for (unsigned i0 = 0; i0 < rows; i0 += ML_TAIL) {
+    const unsigned i = i0 + tr, t = i / heads;
     uint4 row = make_uint4(0, 0, 0, 0);
-    long long so = -1, dof = -1;
-    if (i < cnt) {
-      so = fc_token_offset(src, b, s0 + i);
-      dof = fc_token_offset(dst, b, d0 + i);
+    long long so = -1, dof = -1, h = h0 + (int)(i - t * heads);
+    if (i < rows) {
+      so = fc_token_offset(src, b, s0 + (int)t);
+      dof = fc_token_offset(dst, b, d0 + (int)t);
     }
-    if (so >= 0) row = *reinterpret_cast<const uint4*>(sb + so * 2);
+    if (so >= 0) row = *reinterpret_cast<const uint4*>(sb + (so + h * src.stride_head) * 2);
     __syncthreads();
-    if (so >= 0 && dof >= 0) *reinterpret_cast<uint4*>(db + dof * 2) = row;
+    if (so >= 0 && dof >= 0) *reinterpret_cast<uint4*>(db + (dof + h * dst.stride_head) * 2) = row;
   }
 }
 
@@ -622,11 +628,11 @@ static int ml_check(const char* who, const fc_kv_view* src, const fc_kv_view* ds
 // order of the batch -> this: 28 layers of 4 heads, factor 5, 16 sequences of 5461 to 16384 tokens 1680 -> 1455, 5 of 2666
 // to 8000 331 -> 284, 9 of 700 to 2100 163 -> 131, 16 of 300 to 900 164 -> 125; factor 2, 16 of 3000 to 9000 1342 -> 920, 16 of
 // 300 to 900 158 -> 120; 32 layers of 32 heads, factor 5, 20 of 14 to 824 870 -> 658, factor 2 854 -> 793.
-struct MlSplit { int hsh, wpc, gx; };
+struct MlSplit { int hsh, wpc, gx; double cost; };   // cost in iterations
 template <typename Fits>
 static MlSplit ml_split(int batch, int heads, int max_hsh, int jobs, int c, int cf, bool rag, Fits fits) {
   const double ncu = fc_compute_units();
-  MlSplit best{0, ML_WAVES, batch * heads};      // what is left when no split fits
+  MlSplit best{0, ML_WAVES, batch * heads, 0.0};      // what is left when no split fits
   double best_cost = -1.0;
   for (int i = 0; i <= max_hsh; ++i) {
     const int hsh = rag ? max_hsh - i : i;
@@ -637,15 +643,18 @@ static MlSplit ml_split(int batch, int heads, int max_hsh, int jobs, int c, int 
       const int cpw = ML_WAVES / wpc, groups = (ncols + cpw - 1) / cpw;
       const double most = (double)((rows + ML_ROWS * wpc - 1) / (ML_ROWS * wpc));
       const double iters = rag ? 0.67 * (double)rows / (ML_ROWS * wpc) + 0.5 : most;
+      int last = 0;
       for (int per = 1; per <= groups && per <= (cf <= 2 && !rag ? 64 : 1); ++per) {   // groups a workgroup walks
         const int g = (groups + per - 1) / per;
-        const double wgs = (double)g * jobs / ncu, whole = floor(wgs), part = wgs - whole;
+        if (g == last) continue;
+        last = g;
+        const double wgs = (double)g * jobs / ncu, whole = (double)(int64_t)wgs, part = wgs - whole;
         const double one = cf <= 2 ? (double)((groups + g - 1) / g) * (iters + 0.25) + 0.7 : iters + 0.4;
         const double rounds = whole + (part <= 0.0 ? 0.0 : part > 0.85 ? part : 0.85);
         const double cost = !rag ? rounds * one : fmax(one - iters + most, wgs * one + 0.5 * iters);
         if (best_cost < 0 || cost < best_cost) {
           best_cost = cost;
-          best = {hsh, wpc, g};
+          best = {hsh, wpc, g, cost};
         }
       }
     }
@@ -657,7 +666,7 @@ static MlSplit ml_split(int batch, int heads, int max_hsh, int jobs, int c, int 
 // three arrays, every sequence's own segment with at most c rows.  `a`: the planes, in views of src's and dst's geometry.
 static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* dst, const MlPlanes& a, int planes, int cf,
                      int seg_start, int c, int dst_start, const int32_t* seg_start_v, const int32_t* seg_len_v,
-                     const int32_t* dst_start_v, int min_rows, hipStream_t st) {
+                     const int32_t* dst_start_v, int min_rows, hipStream_t st, const MlSplit* given = nullptr) {
   const bool rag = seg_len_v != nullptr;
   // heads whose rows of a token lie side by side, in both views, may share a column, up to 16 (a lane's two rows of every
   // 32 are then of one head; 32 heads to a column were never the faster split)
@@ -670,7 +679,24 @@ static int ml_launch(const char* who, const fc_kv_view* src, const fc_kv_view* d
     return rag ? fit(src, src->max_seq_len - 1) && fit(dst, dst->max_seq_len - 1)
                : fit(src, (int64_t)seg_start + (int64_t)c * cf - 1) && fit(dst, (int64_t)dst_start + c - 1);
   };
-  const MlSplit sp = ml_split(src->batch, src->num_kv_heads, max_hsh, planes * src->num_layers, c, cf, rag, tables_fit);
+  const MlSplit sp = given ? *given : ml_split(src->batch, src->num_kv_heads, max_hsh, planes * src->num_layers, c, cf, rag, tables_fit);
+  // Workgroups with resident W1 walk many columns each, and both planes' at a time are up to 3 % slower than one plane's after
+  // the other: together only where that saves 1.6 % of the iterations.  us per pass, together / a launch per plane, factor 2,
+  // saving: 32 layers of 32 heads, 24 of 640 tokens (0.7 %) 2639 / 2619, 45 4970 / 4927, 9 (12 %) 1049 / 1113; 28 of 4, 8 of
+  // 8000 (1.5 %) 1301 / 1262, 16 of 16384 (0.2 %) 4872 / 4837, 2 of 8000 (2.9 %) 353 / 384.  Factor 5, 45 of 640 4269 / 4297,
+  // 16 of 16384 4197 / 4252, 9 of 640 991 / 1059; different lengths, factor 2, 8 of 2666 to 8000 972 / 1035, 16 of 5461 to
+  // 16384 3397 / 3399.
+  if (planes == 2 && !rag && cf <= 2) {
+    const MlSplit one = ml_split(src->batch, src->num_kv_heads, max_hsh, src->num_layers, c, cf, false, tables_fit);
+    if (2.0 * one.cost < 1.016 * sp.cost) {
+      MlPlanes v{};
+      v.src[0] = a.src[1];
+      v.dst[0] = a.dst[1];
+      for (int i = 0; i < 6; ++i) v.w[0][i] = a.w[1][i];
+      int rc = ml_launch(who, src, dst, a, 1, cf, seg_start, c, dst_start, nullptr, nullptr, nullptr, min_rows, st, &one);
+      return rc ? rc : ml_launch(who, src, dst, v, 1, cf, seg_start, c, dst_start, nullptr, nullptr, nullptr, min_rows, st, &one);
+    }
+  }
   const int hsh = sp.hsh, wpc = sp.wpc, gx = sp.gx;
   const int ncols = src->batch * (src->num_kv_heads >> hsh);
   const int cols_per_wg = ML_WAVES / wpc, ncg = (ncols + cols_per_wg - 1) / cols_per_wg;
@@ -748,9 +774,10 @@ static void ml_tails(const fc_kv_view* const src[2], const fc_kv_view* const dst
   for (int p = 0; p < planes; ++p)
     same = same && src[p]->base == dst[p]->base && src[p]->block_tables == dst[p]->block_tables &&
            src[p]->stride_layer == dst[p]->stride_layer && src[p]->stride_batch == dst[p]->stride_batch;
-  hipLaunchKernelGGL(mlp_tail_copy_kernel, dim3(src[0]->num_kv_heads, src[0]->batch, planes * src[0]->num_layers), dim3(256), 0, st,
-                     fc_make_view(src[0]), fc_make_view(dst[0]), a, cf, min_rows, c, seg_start_v, seg_len_v, dst_start_v,
-                     seg_start, seg_len, dst_start, same);
+  const int heads = src[0]->num_kv_heads, per = heads < 32 ? heads : 32;
+  hipLaunchKernelGGL(mlp_tail_copy_kernel, dim3((heads + per - 1) / per, src[0]->batch, planes * src[0]->num_layers),
+                     dim3(16 * ML_TAIL), 0, st, fc_make_view(src[0]), fc_make_view(dst[0]), a, cf, min_rows, c, seg_start_v, seg_len_v, dst_start_v,
+                     seg_start, seg_len, dst_start, same, per);
 }
 
 static int ml_uniform(const char* who, const fc_kv_view* const src[2], const fc_kv_view* const dst[2], const fc_mlp_weights* w,

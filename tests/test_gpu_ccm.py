@@ -306,6 +306,7 @@ def test_ccm_mlp_is_the_same_however_columns_are_split(dev, L, B, S, block_size,
     (1, 4, [64 + 7 * i % 131 for i in range(70)], 32, 3),         # more sequences than a wavefront has lanes
     (1, 2, [20 + i % 37 for i in range(260)], 32, 2),             # more than are put in order
     (1, 2, [25000, 300], 32, 5),                                  # block tables that do not fit
+    (2, 40, [334, 71, 9, 64], 256, 5),                            # remainders of 40 heads: two workgroups, several passes
 ])
 def test_ccm_mlp_ragged_is_each_sequence_alone(dev, L, H, lens, block_size, cf):
     """Sequences of different lengths in one launch, longest first, heads sharing columns: the same bytes as every
