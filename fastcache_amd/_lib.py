@@ -40,6 +40,9 @@ class FcKvView(C.Structure):
     ]
 
 
+DECODE_ARRIVALS = 512       # FC_DECODE_ARRIVALS of the header
+
+
 class FcMlpWeights(C.Structure):
     _fields_ = [(n, C.c_void_p) for n in ("w1", "b1", "w2", "b2", "w3", "b3")]
 
@@ -116,6 +119,8 @@ SIGNATURES = {
     "fc_decode_layer_workspace_bytes": (C.c_int64, [_V, _V, _I]),
     "fc_decode_layer": (C.c_int, [_V, _V, _VP, _VP, C.c_int64, _VP, C.c_int64, _VP, _VP, _I, _VP, _F, _VP, C.c_int64, _VP]),
     "fc_decode_layer_turn": (C.c_int, [_V, _V, _VP, _VP, C.c_int64, _VP, C.c_int64, _VP, _VP, _I, _VP, _F, _VP, C.c_int64, _I, _VP]),
+    "fc_decode_layer_arrivals": (C.c_int, [_V, _V, _VP, _VP, C.c_int64, _VP, C.c_int64, _VP, _VP, _I, _VP, _F, _VP, C.c_int64, _VP,
+                                           _VP]),
     "fc_stage_decode": (C.c_int, [*([_VP, C.c_int64, C.c_int64] * 3), _I, _I, _I, _I, _I, _VP, _VP, _VP, _I, *([_VP] * 6), _I, _I,
                                   _VP]),
     "fc_decode_attn_static_capacity": (C.c_int64, []),

@@ -505,9 +505,9 @@ struct DaAppend {                 // the step's new rows, one per sequence (k_ne
   const int* slots;               // flat cache slot per sequence, negative = skip
 };
 
-// Arrivals per column of a launch whose last workgroup merges, a row of counters per turn (fc_decode_layer_turn).  Zero
-// between launches: whoever merges puts the zero back.
-#define DC_COLUMNS 512
+// Arrivals per column of a launch whose last workgroup merges, a row of counters per turn (fc_decode_layer_turn) or the
+// caller's (fc_decode_layer_arrivals).  Zero between launches: whoever merges puts the zero back.
+#define DC_COLUMNS FC_DECODE_ARRIVALS
 static __device__ unsigned dc_arrived[FC_DECODE_TURNS][DC_COLUMNS];
 
 // Partial results that another workgroup of the same launch reads go past the caches of this XCD.
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
                                                                       const int* __restrict__ lens, float c,
                                                                       char* __restrict__ out, DaAppend ap, int chunk,
                                                                       float* part_o, float* part_ml, int max_splits,
-                                                                      int turn) {
+                                                                      int turn, unsigned* arrivals) {
   extern __shared__ __align__(16) char smem[];
   const int b = blockIdx.y;
   const int G = Hq / kc.num_kv_heads, gtiles = (G + DC_HEADS - 1) / DC_HEADS;
@@ -834,7 +834,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   const int ns = (len + chunk - 1) / chunk;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  unsigned* arrived = &dc_arrived[turn][blockIdx.y * gridDim.x + blockIdx.x];
+  unsigned* arrived = (arrivals ? arrivals : dc_arrived[turn]) + (blockIdx.y * gridDim.x + blockIdx.x);
   unsigned* before = reinterpret_cast<unsigned*>(smem);
   if (tid == 0) *before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
@@ -1113,7 +1113,7 @@ static int da_merge(const char* who, const fc_kv_view* k_cache, const float* par
 static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t layer,
                       const void* q, void* out, int32_t num_q_heads, const int32_t* context_lens, float scale,
                       void* workspace, int64_t workspace_bytes, void* stream, const DaAppend* append = nullptr,
-                      int turn = -1) {
+                      int turn = -1, uint32_t* arrivals = nullptr) {
   int rc;
   if ((rc = fc_check_view(k_cache, who)) || (rc = fc_check_view(v_cache, who))) return rc;
   FC_REQUIRE(k_cache->dtype == v_cache->dtype && k_cache->num_layers == v_cache->num_layers &&
@@ -1140,19 +1140,23 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
     float* part_o = (float*)workspace;
     float* part_ml = part_o ? part_o + (int64_t)k_cache->batch * num_q_heads * csplits * FC_HEAD_DIM : nullptr;
     const DaAppend ap = append ? *append : DaAppend{nullptr, nullptr, 0, 0, nullptr};
-    if ((int64_t)grid.x * grid.y > DC_COLUMNS || csplits > DC_SPLITS || !k_cache->block_tables) turn = -1;
+    if ((int64_t)grid.x * grid.y > DC_COLUMNS || csplits > DC_SPLITS || !k_cache->block_tables) {
+      turn = -1;
+      arrivals = nullptr;
+    }
+    const bool last_merges = turn >= 0 || arrivals;
     const KvView k = fc_make_view(k_cache), v = fc_make_view(v_cache);
 #define DC_LAUNCH3(DT, TERMS, PG, TURN)                                                                            \
   do {                                                                                                             \
     FC_ALLOW_LDS((decode_column_kernel<DT, TERMS, PG, TURN>), DC_LDS);                                              \
     hipLaunchKernelGGL((decode_column_kernel<DT, TERMS, PG, TURN>), grid, dim3(DC_THREADS), DC_LDS, (hipStream_t)stream, \
                        k, v, layer, (const char*)q, num_q_heads, context_lens, scale * DA_LOG2E, (char*)out, ap,    \
-                       column, part_o, part_ml, csplits, turn);                                                    \
+                       column, part_o, part_ml, csplits, turn, arrivals);                                                  \
   } while (0)
 // (a turn comes with paged caches)
 #define DC_LAUNCH(DT, TERMS)                                      \
   if (!k_cache->block_tables) DC_LAUNCH3(DT, TERMS, false, false); \
-  else if (turn < 0 || csplits == 1) DC_LAUNCH3(DT, TERMS, true, false); \
+  else if (!last_merges || csplits == 1) DC_LAUNCH3(DT, TERMS, true, false); \
   else DC_LAUNCH3(DT, TERMS, true, true)
     if (k_cache->dtype == FC_F16) {
       if (G > 4) { DC_LAUNCH(FC_F16, 2); } else { DC_LAUNCH(FC_F16, 3); }
@@ -1162,7 +1166,7 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
 #undef DC_LAUNCH3
 #undef DC_LAUNCH
     FC_CHECK_LAUNCH(who);
-    if (csplits > 1 && turn < 0)
+    if (csplits > 1 && !last_merges)
       return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, csplits, column, out, stream);
     return FC_OK;
   }
@@ -1266,10 +1270,10 @@ extern "C" int fc_decode_layer(const fc_kv_view* k_cache, const fc_kv_view* v_ca
                               context_lens, scale, workspace, workspace_bytes, -1, stream);
 }
 
-extern "C" int fc_decode_layer_turn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
-                                    int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping,
-                                    void* out, int32_t num_q_heads, const int32_t* context_lens, float scale,
-                                    void* workspace, int64_t workspace_bytes, int32_t turn, void* stream) {
+static int da_layer(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new, int64_t k_stride,
+                    const void* v_new, int64_t v_stride, const int32_t* slot_mapping, void* out, int32_t num_q_heads,
+                    const int32_t* context_lens, float scale, void* workspace, int64_t workspace_bytes, int32_t turn,
+                    uint32_t* arrivals, void* stream) {
   const char* who = "fc_decode_layer";
   int rc;
   FC_REQUIRE(turn >= -1 && turn < FC_DECODE_TURNS, FC_EINVAL, "%s: turn %d", who, turn);
@@ -1290,7 +1294,7 @@ extern "C" int fc_decode_layer_turn(const fc_kv_view* k_cache, const fc_kv_view*
   if (da_appends_inside(k_cache, v_cache, num_q_heads)) {
     const DaAppend ap = {(const char*)k_new, (const char*)v_new, k_stride * eb, v_stride * eb, slot_mapping};
     return da_enqueue(who, k_cache, v_cache, 0, q, out, num_q_heads, context_lens, scale, workspace, workspace_bytes,
-                      stream, &ap, turn);
+                      stream, &ap, turn, arrivals);
   }
   // what the attention would refuse is refused before the rows are written
   FC_REQUIRE(q && out && context_lens && workspace, FC_EINVAL, "%s: null pointer", who);
@@ -1300,6 +1304,22 @@ extern "C" int fc_decode_layer_turn(const fc_kv_view* k_cache, const fc_kv_view*
                               (int32_t)row, k_cache->dtype, stream)))
     return rc;
   return da_enqueue(who, k_cache, v_cache, 0, q, out, num_q_heads, context_lens, scale, workspace, workspace_bytes, stream);
+}
+
+extern "C" int fc_decode_layer_turn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
+                                    int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping,
+                                    void* out, int32_t num_q_heads, const int32_t* context_lens, float scale,
+                                    void* workspace, int64_t workspace_bytes, int32_t turn, void* stream) {
+  return da_layer(k_cache, v_cache, q, k_new, k_stride, v_new, v_stride, slot_mapping, out, num_q_heads, context_lens, scale,
+                  workspace, workspace_bytes, turn, nullptr, stream);
+}
+
+extern "C" int fc_decode_layer_arrivals(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
+                                        int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping,
+                                        void* out, int32_t num_q_heads, const int32_t* context_lens, float scale,
+                                        void* workspace, int64_t workspace_bytes, uint32_t* arrivals, void* stream) {
+  return da_layer(k_cache, v_cache, q, k_new, k_stride, v_new, v_stride, slot_mapping, out, num_q_heads, context_lens, scale,
+                  workspace, workspace_bytes, -1, arrivals, stream);
 }
 
 // ---- the same attention for callers that cannot allocate -------------------------------------------------

@@ -451,11 +451,11 @@ int decode_turn(const at::Tensor& t, const c10::hip::HIPStream& stream) {
 
 // ---- one attention layer of a decode step ---------------------------------------------------------------------------------
 // decode_layer(q, k, v, k_cache, v_cache, slot_mapping, context_lens, block_tables, scale, q_heads, kv_heads, head_dim,
-//              workspace or None) -> out [n, q_heads * head_dim], or None when the arguments are not the plain decode
-// step (the caller's general path then serves or refuses them).
+//              workspace or None, out or None, arrivals or None) -> out [n, q_heads * head_dim], or None when the arguments
+// are not the plain decode step (the caller's general path then serves or refuses them).  arrivals: FC_DECODE_ARRIVALS zeros.
 PyObject* py_decode_layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return guarded([&]() -> PyObject* {
-    need_args(nargs, 13, "decode_layer");
+    need_args(nargs, 15, "decode_layer");
     for (int i = 0; i < 8; ++i)
       if (!is_tensor(args[i])) Py_RETURN_NONE;
     const at::Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
@@ -516,13 +516,32 @@ PyObject* py_decode_layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       wsp = ws.data_ptr();
       ws_bytes = ws.numel();
     }
-    at::Tensor out = at::empty({n, hq * d}, q.options());
+    at::Tensor out;
+    if (args[13] != Py_None) {
+      if (!is_tensor(args[13])) Py_RETURN_NONE;
+      out = THPVariable_Unpack(args[13]);
+      if (out.device() != dev || out.scalar_type() != dt || out.dim() != 2 || out.size(0) != n || out.size(1) != hq * d ||
+          !out.is_contiguous() || ((uintptr_t)out.const_data_ptr() & 15) != 0)
+        Py_RETURN_NONE;
+    } else {
+      out = at::empty({n, hq * d}, q.options());
+    }
     const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(q.get_device());
-    check(fc_decode_layer_turn(&kv, &vv, q.const_data_ptr(), k.const_data_ptr(), stride[0], v.const_data_ptr(), stride[1],
-                          (const int32_t*)slots.const_data_ptr(), out.data_ptr(), (int32_t)hq,
-                          (const int32_t*)lens.const_data_ptr(), (float)scale, wsp, ws_bytes, ws_bytes ? decode_turn(q, stream) : -1,
-                          (void*)stream.stream()),
-          "fc_decode_layer");
+    const int32_t *sp = (const int32_t*)slots.const_data_ptr(), *lp = (const int32_t*)lens.const_data_ptr();
+    if (args[14] != Py_None) {
+      const at::Tensor& arr = tensor(args[14], "arrivals");
+      if (arr.device() != dev || arr.scalar_type() != at::kInt || !arr.is_contiguous() || arr.numel() < FC_DECODE_ARRIVALS)
+        fail("decode_layer: arrivals must be contiguous int32 words on the device of q");
+      check(fc_decode_layer_arrivals(&kv, &vv, q.const_data_ptr(), k.const_data_ptr(), stride[0], v.const_data_ptr(), stride[1], sp,
+                                     out.data_ptr(), (int32_t)hq, lp, (float)scale, wsp, ws_bytes,
+                                     ws_bytes ? (uint32_t*)arr.data_ptr() : nullptr, (void*)stream.stream()),
+            "fc_decode_layer");
+    } else {
+      check(fc_decode_layer_turn(&kv, &vv, q.const_data_ptr(), k.const_data_ptr(), stride[0], v.const_data_ptr(), stride[1], sp,
+                                 out.data_ptr(), (int32_t)hq, lp, (float)scale, wsp, ws_bytes,
+                                 ws_bytes ? decode_turn(q, stream) : -1, (void*)stream.stream()),
+            "fc_decode_layer");
+    }
     return wrap(std::move(out));
   });
 }

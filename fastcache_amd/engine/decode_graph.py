@@ -18,6 +18,7 @@ from typing import Dict, List, Optional, Sequence
 import torch
 
 from .. import _lib, ops
+from ..layers.attention import Attention
 from ..utils.context import get_context, reset_context, set_context
 
 
@@ -95,8 +96,13 @@ class BucketedDecodeGraphs:
         self.graph_pool = None
 
     def _model(self, q, k, v, out):
+        # a layer's own result is written where it belongs: a copy node behind every layer was 4.6 of its 12.2 us (28 query
+        # heads on 4, 9 sequences of 100 to 248 tokens)
         for i, layer in enumerate(self.layers):
-            out[i] = layer(q[i], k[i], v[i])
+            to = out[i]
+            o = layer(q[i], k[i], v[i], out=to) if type(layer).forward is Attention.forward else layer(q[i], k[i], v[i])
+            if o.data_ptr() != to.data_ptr():      # another module's, or a forward hook's
+                to.copy_(o)
 
     @torch.inference_mode()
     def capture_cudagraph(self):
@@ -111,8 +117,10 @@ class BucketedDecodeGraphs:
         v = torch.zeros_like(k)
         outputs = torch.zeros_like(q)
         workspace = ops.decode_attn_workspace(bsz, a.num_heads, self.max_num_blocks * block_size, dev)
+        # the columns' last workgroups merge their ranges, told by counters that belong to the graphs like the workspace does
+        arrivals = torch.zeros(_lib.DECODE_ARRIVALS, dtype=torch.int32, device=dev)
         for layer in self.layers:
-            layer.workspace = workspace
+            layer.workspace, layer.arrivals = workspace, arrivals
         self.graph_bs = [b for b in [1, 2, 4, 8] + list(range(16, bsz + 1, 16)) if b <= bsz]
         if self.graph_bs[-1] != bsz:
             self.graph_bs.append(bsz)

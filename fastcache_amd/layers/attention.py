@@ -67,17 +67,19 @@ class Attention(nn.Module):
         self.num_heads, self.head_dim, self.scale, self.num_kv_heads = num_heads, head_dim, scale, num_kv_heads
         self.k_cache = self.v_cache = torch.tensor([])
         self.workspace: Optional[torch.Tensor] = None   # set by a graph runner that owns the scratch memory
+        self.arrivals: Optional[torch.Tensor] = None    # with it, int32 zeros for the kernels that merge a column's ranges
 
-    def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+    def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """q ``[N, Hq*D]``, k and v ``[N, Hkv*D]`` -> ``[N, Hq*D]``, in ``out`` where one is given."""
         ctx = get_context()
         if not ctx.is_prefill and ctx.block_tables is not None:
             # the plain decode step: append and attention through one native call (and one launch where that is faster)
-            out = _lib.host().decode_layer(q, k, v, self.k_cache, self.v_cache, ctx.slot_mapping, ctx.context_lens,
-                                           ctx.block_tables, self.scale, self.num_heads, self.num_kv_heads, self.head_dim,
-                                           self.workspace)
-            if out is not None:
+            done = _lib.host().decode_layer(q, k, v, self.k_cache, self.v_cache, ctx.slot_mapping, ctx.context_lens,
+                                            ctx.block_tables, self.scale, self.num_heads, self.num_kv_heads, self.head_dim,
+                                            self.workspace, out, self.arrivals)
+            if done is not None:
                 _lib.note_enqueued()
-                return out
+                return done
         q = q.view(-1, self.num_heads, self.head_dim)
         k = k.view(-1, self.num_kv_heads, self.head_dim)
         v = v.view(-1, self.num_kv_heads, self.head_dim)
@@ -86,4 +88,5 @@ class Attention(nn.Module):
             raise NotImplementedError("prefill attention is outside the KV-cache compression path built here")
         o = decode_attention(q.unsqueeze(1), self.k_cache, self.v_cache, ctx.context_lens, ctx.block_tables, self.scale,
                              workspace=self.workspace)
-        return o.view(-1, self.num_heads * self.head_dim)
+        o = o.view(-1, self.num_heads * self.head_dim)
+        return o if out is None else out.copy_(o)

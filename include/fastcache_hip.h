@@ -581,6 +581,17 @@ int fc_decode_layer_turn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, c
                          int64_t workspace_bytes, int32_t turn, void* stream);
 
 /*
+ * The same with counters of the caller's: FC_DECODE_ARRIVALS zeros in device memory, which like the workspace no other
+ * launch uses at the same time and which are zeros again when the launch has ended; NULL asks for the launch of its own.  A
+ * captured graph may hold them.
+ */
+#define FC_DECODE_ARRIVALS 512
+int fc_decode_layer_arrivals(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
+                             int64_t k_stride, const void* v_new, int64_t v_stride, const int32_t* slot_mapping, void* out,
+                             int32_t num_q_heads, const int32_t* context_lens, float scale, void* workspace,
+                             int64_t workspace_bytes, uint32_t* arrivals, void* stream);
+
+/*
  * A decode step's inputs into the static buffers of a captured graph (what the decode branch of `run_model` patches
  * before a replay, nanovllm/engine/llava_model_runner.py:697-710): q [num_layers][batch][q_elems] and k, v
  * [num_layers][batch][kv_elems] (strides in elements) into contiguous buffers of max_batch sequences per layer; slots,

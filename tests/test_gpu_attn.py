@@ -545,3 +545,53 @@ def test_infinite_values_stay_infinite(dev, dtype, Hq, Hkv, wide, lens):
     # one key carries nearly all of the weight: outputs are as large as values, and both sides round theirs once (a step of
     # the type apart where the fp32 results, 1e-5 apart at most, lie on two sides of a middle)
     assert bool(((got - ref)[..., rest].abs() <= torch.finfo(dtype).eps * ref[..., rest].abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens,plain,merges", [
+    (14, 2, [700, 0, 255, 513], True, 0),         # columns of several ranges: their last workgroup merges
+    (4, 2, [100, 256, 31], True, 0),              # one range a column
+    (7, 1, [3600, 40], True, 2),                  # more ranges than the last workgroup takes
+    (14, 2, [700, 0, 255, 513], False, 0),        # a layer of its own class: what it returns is copied
+])
+def test_bucket_graphs_hold_one_launch_per_layer(dev, Hq, Hkv, lens, plain, merges):
+    """What a bucket's graph launches, and the layers' results in the static output, replay after replay with eager steps on
+    the same layers between (which share the workspace and the counters)."""
+    from fastcache_amd.engine.decode_graph import BucketedDecodeGraphs
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+
+    class Doubled(Attention):
+        def forward(self, q, k, v):
+            return super().forward(q, k, v) * 2
+
+    L, B, dtype = 2, len(lens), torch.bfloat16
+    case = synth.make_paged_case(seed=61, num_layers=L, batch=B, num_kv_heads=Hkv, seq_lens=[n + 1 for n in lens], dtype=dtype)
+    pool, tables = case.kv_cache.to(dev), case.table_tensor(dev)
+    layers = [(Attention if plain else Doubled)(Hq, 128, 128 ** -0.5, Hkv) for _ in range(L)]
+    for l, a in enumerate(layers):
+        a.k_cache, a.v_cache = pool[0, l], pool[1, l]
+    graphs = BucketedDecodeGraphs(layers, B, tables.shape[1], dtype, dev)
+    graphs.capture_cudagraph()
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn(L, B, h * 128, generator=g).to(dtype).to(dev) for h in (Hq, Hkv, Hkv))
+    set_context(False, slot_mapping=torch.full((B,), -1, dtype=torch.int32, device=dev),
+                context_lens=torch.tensor(lens, dtype=torch.int32, device=dev), block_tables=tables)
+    try:
+        got, names = [], []
+        for _ in range(3):        # a profile now and then holds nothing of what ran in it
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
+                got.append(graphs.run(q, k, v).clone())
+                torch.cuda.synchronize()
+            names = names or [e.name for e in prof.events() if "decode_" in e.name]
+        assert sum("decode_column_kernel<" in n for n in names) == L
+        assert sum("decode_merge_kernel" in n for n in names) == merges
+        for _ in range(3):
+            with torch.inference_mode():
+                graphs.graph_vars["outputs"].fill_(float("nan"))
+            eager = torch.stack([a(q[l], k[l], v[l]) for l, a in enumerate(layers)])
+            got.append(graphs.run(q, k, v).clone())
+            torch.cuda.synchronize()
+    finally:
+        reset_context()
+    for o in got:
+        assert torch.equal(o.view(torch.int16), eager.view(torch.int16))
