@@ -15,6 +15,7 @@
 // Each chunk writes (max, sum, unnormalised output) to the workspace; a second kernel merges the
 // chunks of a sequence.  Grid sizes depend only on the view's max_seq_len, never on the lengths on
 // the device, so both launches can be replayed from a graph while the lengths grow.
+#include <type_traits>
 #include "fc_common.h"
 #include <atomic>
 #include <stdlib.h>
@@ -455,10 +456,9 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 #define DC_THREADS (DC_WAVES * 64)
 #define DC_HEADS 16
 #define DC_PSTRIDE 132                                             // floats per partial output row (padded against bank conflicts)
-#define DC_VROW 272                                                // LDS bytes per V row: 4 rows apart = 64 bytes apart in banks
-#define DC_STAGE (DA_TILE * DC_VROW)
+#define DC_STAGES 2                                                // V tiles of a wavefront in LDS or on their way
 #define DC_MERGE 8                                                // partial rows in flight per thread of the merge
-#define DC_PART (DC_WAVES * DC_STAGE)                              // V stages, then the partial outputs
+#define DC_PART (DC_WAVES * DC_STAGES * DA_TILEB)                   // V stages, then the partial outputs
 #define DC_LDS (DC_PART + DC_WAVES * DC_HEADS * 8)
 static_assert(DC_PART >= DC_WAVES * DC_HEADS * DC_PSTRIDE * 4, "the partial outputs share the V stages' memory");
 
@@ -497,6 +497,14 @@ __device__ __forceinline__ uint4 da_split8(float (&p)[8]) {
     p[2 * e + 1] -= DTYPE == FC_BF16 ? __uint_as_float(w[e] & 0xffff0000u) : fc_half_to_float((unsigned short)(w[e] >> 16));
   }
   return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// 8 bytes a lane from an absolute LDS address, transposed among 16 lanes: lane i of them gets the i-th 2-byte value of what
+// lanes 0 .. 3, 4 .. 7, 8 .. 11 and 12 .. 15 read (ds_read_b64_tr_b16)
+__device__ __forceinline__ uint2 da_lds_transposed(unsigned addr) {
+  typedef short da_s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                       reinterpret_cast<__attribute__((address_space(3))) da_s16x4*>((size_t)addr)));
 }
 
 struct DaAppend {                 // the step's new rows, one per sequence (k_new null: nothing to append)
@@ -609,39 +617,53 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     const int blk = max(__builtin_amdgcn_readlane(tbl, s0 >> v.block_shift), 0);
     return base + ((long long)blk * v.stride_block + (long long)(s0 & (v.block_size - 1)) * v.stride_token) * 2;
   };
-  // Rows past the end of the sequence re-read its last row; their logits are masked.  The scheduling barriers keep
-  // the loads from moving up before the tile their registers held has been used up.
+  // Rows past the end of the sequence re-read its last row, except K rows of a paged tile, which lies inside its page: they
+  // are read as they are, their logits are masked.  The scheduling barriers keep the loads from moving up before the tile
+  // their registers held has been used up.
+  const unsigned klane = (unsigned)l15 * ktok + qd * 16;
   auto load_k = [&](da_u32x4 (&kf)[8], int tile) {
     const int s0 = t0 + tile * DA_TILE, rmax = end - 1 - s0;
     const char* kg = tile_base(kc, kbase, s0, ktbl);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
-      const unsigned o = (unsigned)min(kb * 16 + l15, rmax) * ktok + qd * 16;
+      const char* g = PAGED ? kg + kb * 16 * (unsigned long long)ktok : kg;
+      const unsigned o = PAGED ? klane : (unsigned)min(kb * 16 + l15, rmax) * ktok + qd * 16;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) kf[kb * 4 + ks] = *reinterpret_cast<const da_u32x4*>(kg + o + ks * 64);
+      for (int ks = 0; ks < 4; ++ks) kf[kb * 4 + ks] = *reinterpret_cast<const da_u32x4*>(g + o + ks * 64);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto load_v = [&](da_u32x4 (&vf)[8], int tile) {
-    const int s0 = t0 + tile * DA_TILE, rmax = end - 1 - s0;
-    const char* vg = tile_base(vc, vbase, s0, vtbl) + l15 * 16;
-    __builtin_amdgcn_sched_barrier(0);
+  // V rows go to LDS without registers between, 4 rows of 256 bytes an instruction; the 16-byte pieces of a row are XOR-ed
+  // with the row number, so that the transposed reads of 16 rows at one place meet all banks.
+  const unsigned v_lds = __builtin_amdgcn_readfirstlane(fc_lds_addr(smem) + wave * DC_STAGES * DA_TILEB);
+  unsigned vlane[4];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const unsigned o = (unsigned)min(4 * u + qd, rmax) * vtok;
-      vf[u] = *reinterpret_cast<const da_u32x4*>(vg + o);
+  for (int j = 0; j < 4; ++j) vlane[j] = (unsigned)qd * vtok + ((l15 ^ (4 * j + qd)) << 4);
+  auto load_v = [&](int stage, int tile) {
+    const int s0 = t0 + tile * DA_TILE, rmax = end - 1 - s0;
+    const char* vg = tile_base(vc, vbase, s0, vtbl);
+    if (rmax >= DA_TILE - 1) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) fc_load_lds(vg + u * 4 * (unsigned long long)vtok, vlane[u & 3], v_lds + stage * DA_TILEB + u * 1024);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        fc_load_lds(vg, (unsigned)min(4 * u + qd, rmax) * vtok + ((l15 ^ ((4 * u + qd) & 15)) << 4), v_lds + stage * DA_TILEB + u * 1024);
     }
-    __builtin_amdgcn_sched_barrier(0);
   };
 
   float m = -INFINITY, l = 0.f;      // of head l15: the maximum is the tile group's, the sum this lane's keys'
   f32x4 o[8];
+  // Transposed reads: 16 lanes take four rows, 32 bytes of each, 8 bytes a lane, and lane i gets column i of the four: here
+  // dimension db * 16 + l15 of keys 4 qd .. 4 qd + 3 (and of the 16 keys further).
+  unsigned v_get[8];
+  {
+    const int row = 4 * qd + (l15 >> 2);
+    const unsigned at = (((l15 & 3) >> 1) ^ row) << 4;
 #pragma unroll
-  for (int db = 0; db < 8; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-  char* vst = smem + wave * DC_STAGE;
-  char* v_put = vst + qd * DC_VROW + l15 * 16;                    // row 4 u + qd: u * 4 * DC_VROW further
-  const char* v_get = vst + 4 * qd * DC_VROW + l15 * 2;           // key 4 qd + j (and 16 further), dimension db * 16 + l15
+    for (int db = 0; db < 8; ++db) v_get[db] = v_lds + row * 256 + (at ^ (db * 32)) + (l15 & 1) * 8;
+  }
   const int tiles = (end - t0 + DA_TILE - 1) / DA_TILE, last = tiles - 1;
   auto dot = [&](const da_u32x4 (&kf)[8], f32x4 (&s)[2]) {
 #pragma unroll
@@ -651,23 +673,23 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
       for (int ks = 0; ks < 4; ++ks) s[kb] = da_mfma16<DTYPE>(__builtin_bit_cast(uint4, kf[kb * 4 + ks]), qf[ks], s[kb]);
     }
   };
-  // One tile: its logits, its V rows into LDS; then the next V tile and the K tile after the next start loading into
-  // the registers that became free (past the last tile they re-read it: unconditional loads keep the tiles in registers).
-  auto use_tile = [&](da_u32x4 (&kf)[8], da_u32x4 (&vf)[8], int tile) {
+  // One tile: its logits, its probabilities, its V rows; then the tile after the next starts loading into the registers and
+  // the stage that became free.  V is asked for before K: whoever waits for a tile's K has its V as well.
+  // NEWER: whether the next tile has been asked for already, LOAD: whether there is one after the next; compile-time, since a
+  // branch around loads has the compiler wait for all that might be under way.
+  auto use_tile = [&](da_u32x4 (&kf)[8], auto stage, auto first, auto newer, auto load, int tile) {
+    constexpr int ST = decltype(stage)::value;
+    constexpr bool FIRST = decltype(first)::value, NEWER = decltype(newer)::value, LOAD = decltype(load)::value;
+    const int live = end - t0 - tile * DA_TILE;
     f32x4 s[2];
     dot(kf, s);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) *reinterpret_cast<da_u32x4*>(v_put + u * 4 * DC_VROW) = vf[u];
-    if (tile + DC_WAVES < tiles) {
-      load_v(vf, tile + DC_WAVES);
-      load_k(kf, min(tile + 2 * DC_WAVES, last));
-    }
     float p[8];
-    const int live = end - t0 - tile * DA_TILE;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int key = (e >> 2) * 16 + qd * 4 + (e & 3);
-      p[e] = key < live ? s[e >> 2][e & 3] * c : -INFINITY;
+    for (int e = 0; e < 8; ++e) p[e] = s[e >> 2][e & 3] * c;
+    if (live < DA_TILE) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if ((e >> 2) * 16 + qd * 4 + (e & 3) >= live) p[e] = -INFINITY;
     }
     float mx = p[0];
 #pragma unroll
@@ -675,9 +697,9 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float mo = m;
-    m = fmaxf(m, mx);
+    m = FIRST ? mx : fmaxf(m, mx);
     const float ref = m == -INFINITY ? 0.f : m;   // so far only logits of -inf: they weigh nothing, and -inf - -inf is NaN
-    const float alpha = __builtin_amdgcn_exp2f(mo - ref);
+    const float alpha = FIRST ? 0.f : __builtin_amdgcn_exp2f(mo - ref);
     float sum = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -685,45 +707,61 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
       sum += p[e];
       p[e] *= DA_P_SCALE(DTYPE);
     }
-    l = fmaf(l, alpha, sum);
+    l = FIRST ? sum : fmaf(l, alpha, sum);
     uint4 pt[TERMS];
 #pragma unroll
     for (int t = 0; t < TERMS; ++t) pt[t] = da_split8<DTYPE>(p);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // this wavefront's V rows before its transposed reads of them
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    fc_wait_vm<NEWER ? 16 : 0>();      // this tile's V rows are in LDS
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int db = 0; db < 8; ++db) {
-      unsigned w[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const char* r = v_get + ((e >> 1) * 16 + (2 * e & 3)) * DC_VROW + db * 32;
-        w[e] = (unsigned)*reinterpret_cast<const unsigned short*>(r) |
-               ((unsigned)*reinterpret_cast<const unsigned short*>(r + DC_VROW) << 16);
-      }
-      const uint4 vt = make_uint4(w[0], w[1], w[2], w[3]);
+      const uint2 lo = da_lds_transposed(v_get[db] + ST * DA_TILEB), hi = da_lds_transposed(v_get[db] + ST * DA_TILEB + 4096);
+      const uint4 vt = make_uint4(lo.x, lo.y, hi.x, hi.y);
       f32x4 pv = f32x4{0.f, 0.f, 0.f, 0.f};        // the tile's own sum, least operands first: o is rounded once a tile
 #pragma unroll
       for (int t = TERMS; t > 0; --t) pv = da_mfma16<DTYPE>(vt, pt[t - 1], pv);
-      o[db] = o[db] * alpha + pv;
+      o[db] = FIRST ? pv : o[db] * alpha + pv;
       // not more transposed reads in flight than registers beside the tiles hold
       if ((db & 3) == 3) __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the reads before the next tile's rows
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if constexpr (LOAD) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the reads of the stage before what overwrites it
+      load_v(ST, tile + 2 * DC_WAVES);
+      load_k(kf, tile + 2 * DC_WAVES);
+    }
   };
 
+  const int own = (tiles - wave + DC_WAVES - 1) / DC_WAVES;    // this wavefront's tiles (none: 0 or less)
+#pragma unroll
+  for (int db = 0; db < 8; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
   {
-    da_u32x4 ka[8], kb[8], va[8];
-    load_k(ka, min(wave, last));
-    load_v(va, min(wave, last));
-    if (wave + DC_WAVES < tiles) load_k(kb, wave + DC_WAVES);
-    for (int t = wave; t < tiles; t += 2 * DC_WAVES) {
-      use_tile(ka, va, t);
-      if (t + DC_WAVES >= tiles) break;
-      use_tile(kb, va, t + DC_WAVES);
+    constexpr std::integral_constant<int, 0> s0{};
+    constexpr std::integral_constant<int, 1> s1{};
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    da_u32x4 ka[8], kb[8];
+    if (own == 1) {
+      load_v(0, wave);
+      load_k(ka, wave);
+      use_tile(ka, s0, yes, no, no, wave);
+    } else if (own > 1) {
+      load_v(0, wave);
+      load_k(ka, wave);
+      load_v(1, wave + DC_WAVES);
+      load_k(kb, wave + DC_WAVES);
+      int t = wave, left = own;
+      for (; left > 3; left -= 2, t += 2 * DC_WAVES) {
+        use_tile(ka, s0, no, yes, yes, t);
+        use_tile(kb, s1, no, yes, yes, t + DC_WAVES);
+      }
+      if (left == 3) {
+        use_tile(ka, s0, no, yes, yes, t);
+        use_tile(kb, s1, no, yes, no, t + DC_WAVES);
+        use_tile(ka, s0, no, no, no, t + 2 * DC_WAVES);
+      } else {
+        use_tile(ka, s0, no, yes, no, t);
+        use_tile(kb, s1, no, no, no, t + DC_WAVES);
+      }
     }
   }
 
@@ -745,19 +783,15 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     for (int db = 0; db < 8; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
     const float ref = m == -INFINITY ? 0.f : m;
     for (int t = wave; t < tiles; t += DC_WAVES) {
-      da_u32x4 kf[8], vf[8];
+      da_u32x4 kf[8];
       f32x4 s[2];
+      load_v(0, t);
       load_k(kf, t);
-      load_v(vf, t);
       dot(kf, s);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) *reinterpret_cast<da_u32x4*>(v_put + u * 4 * DC_VROW) = vf[u];
       float p[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) p[e] = __builtin_amdgcn_exp2f(s[e >> 2][e & 3] * c - ref) * DA_P_SCALE(DTYPE);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      fc_wait_vm<0>();
       const int live = end - t0 - t * DA_TILE;
 #pragma unroll 1
       for (int e = 0; e < 8; ++e) {
@@ -769,19 +803,17 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
           const int key = (e >> 2) * 16 + k4 * 4 + (e & 3);
           const float pk = __shfl(own, k4 * 16 + l15, 64);
           if (key >= live) continue;                           // wave-uniform
-          const char* r = vst + key * DC_VROW + qd * 8;
+          const char* r = smem + wave * DC_STAGES * DA_TILEB + key * 256 + (qd & 1) * 8;
 #pragma unroll
           for (int db = 0; db < 8; ++db) {
-            const uint2 x = *reinterpret_cast<const uint2*>(r + db * 32);
+            const uint2 x = *reinterpret_cast<const uint2*>(r + (((2 * db + (qd >> 1)) ^ (key & 15)) << 4));
             const unsigned w[2] = {x.x, x.y};
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[db][i] = fmaf(pk, da_unpack<DTYPE>((unsigned short)(w[i >> 1] >> (i & 1) * 16)), o[db][i]);
           }
         }
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   }
 
