@@ -1097,10 +1097,14 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 // 569 -> 464, 24 of 5000 639 -> 489; 4, 64 of 4000 in groups of 8 1012 -> 752; 8, 200 of 1700 1073 -> 929; 8, 64 of 8000
 // 784 -> 697; and two rounds of whole columns, 360 of 600 621 -> 451, 400 of 300 529 -> 330, but not of longer ones (360 of
 // 2000 1030 -> 1054).  Groups of 3 and 4: 2 tiles 572 -> 487 (96 of 1000), 3 635 -> 587, 4 748 -> 715, 802 -> 743, one
-// 693 -> 697; 5 730 -> 799, 921 -> 1027.  Smaller groups: 2 tiles 588 -> 551 (64 of 2000), 675 -> 533; 3 and 4 between
-// 789 -> 707 and 541 -> 571, 653 -> 678.
+// 693 -> 697; 5 730 -> 799, 921 -> 1027.  Smaller groups: 2 tiles 588 -> 551 (64 of 2000), 675 -> 533; 3 to 6 where the
+// workgroups are seven eighths of the compute units with ranges 85 % full, or three quarters and whole columns (32 heads, 12
+// captured layers, or 28 eager ones): 6 sequences of 800 288 -> 234, 1 of 8000 445 -> 374, 2 of 5000 413 -> 393, 8 of 1300
+// 383 -> 343, 7 of 120 to 1200 691 -> 701; 4 of 1400 707 -> 666, 2 of 3000 609 -> 561; else 4 of 170 to 1700 657 -> 672, 622 -> 645,
+// 5 of 900 245 -> 254, 3 of 2500 634 -> 722, 5 of 1400 616 -> 703; more tiles: 8 of 2000 462 -> 472, 4 of 4000 459 -> 479, 2 of 8000
+// 553 -> 535.
 #define DC_ONE 768
-#define DC_TILES_FEW 2
+#define DC_TILES_FEW 6
 #define DC_TILES_SOME 4
 #define DC_TILES_MANY 16
 // Eager layers, launched one by one, gain where the last workgroup of a column merges it: a launch less for the host
@@ -1123,8 +1127,12 @@ static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_h
   if (cols * ((k->max_seq_len + chunk - 1) / chunk) <= slots) return chunk;
   if (cols <= (G > 4 ? 2 : 1) * slots && k->max_seq_len <= DC_ONE) return DC_ONE;
   const int most = G > 4 ? DC_TILES_MANY : G > 2 ? DC_TILES_SOME : DC_TILES_FEW;
-  for (int m = 2; m <= most; ++m)
-    if (cols * ((k->max_seq_len + m * chunk - 1) / (m * chunk)) <= slots) return m * chunk;
+  for (int m = 2; m <= most; ++m) {
+    const long long ranges = (k->max_seq_len + m * chunk - 1) / (m * chunk), wgs = cols * ranges;
+    if (wgs > slots) continue;
+    const bool full = ranges == 1 ? 4 * wgs >= 3 * slots : 8 * wgs >= 7 * slots && 20ll * k->max_seq_len >= 17 * ranges * m * chunk;
+    return G > 2 || m == 2 || full ? m * chunk : 0;
+  }
   return 0;
 }
 
