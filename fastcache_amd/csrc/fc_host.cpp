@@ -590,17 +590,37 @@ PyObject* py_stage_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 // ---- a step's numbers to the device -----------------------------------------------------------------------------------------
+// Up to FC_UPLOAD_MAX bytes travel as a kernel's arguments, more (and what a stream under capture is given, which the
+// callers refuse or torch does) as a copy from pinned memory.
 struct Packed {
   at::Tensor host, dev;
+  std::vector<char> small;
   int64_t at = 0;
+  c10::hip::HIPStream stream;
   Packed(int64_t bytes, const c10::Device& device)
-      : host(at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true))),
-        dev(at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(device))) {}
+      : dev(at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(device))),
+        stream(c10::hip::getCurrentHIPStream(device.index())) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool known = hipStreamIsCapturing(stream.stream(), &capture) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    if (known && capture == hipStreamCaptureStatusNone && bytes <= FC_UPLOAD_MAX && bytes % 4 == 0)
+      small.resize(std::max<int64_t>(bytes, 1));
+    else
+      host = at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+  }
   template <typename T>
   T* take(int64_t n) {
-    T* p = (T*)((char*)host.data_ptr() + at);
+    T* p = (T*)((small.empty() ? (char*)host.data_ptr() : small.data()) + at);
     at += n * (int64_t)sizeof(T);
     return p;
+  }
+  void send() {
+    if (small.empty()) {
+      dev.copy_(host, true);
+    } else if (dev.numel() > 0) {
+      const c10::DeviceGuard guard(dev.device());
+      check(fc_upload(dev.data_ptr(), small.data(), (int32_t)dev.numel(), (void*)stream.stream()), "fc_upload");
+    }
   }
   at::Tensor part(int64_t byte, int64_t n, at::ScalarType t) { return dev.narrow(0, byte, n * (int64_t)c10::elementSize(t)).view(t); }
 };
@@ -628,7 +648,7 @@ void fill_tables(PyObject* tables, Py_ssize_t n, int64_t width, int32_t* out) {
 }
 
 // decode_inputs(ids, lens, tables, block_size, ref) -> (input_ids, positions, slots, context_lens, block_tables) on the
-// device of `ref`: one pinned buffer and one copy instead of five of each
+// device of `ref`: one upload instead of five
 PyObject* py_decode_inputs(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return guarded([&]() -> PyObject* {
     need_args(nargs, 5, "decode_inputs");
@@ -655,7 +675,7 @@ PyObject* py_decode_inputs(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       slots[i] = (int32_t)(page * bs + len % bs);
     }
     fill_tables(args[2], n, width, tab);
-    pk.dev.copy_(pk.host, true);
+    pk.send();
     PyObject* out = PyTuple_New(5);
     PyTuple_SET_ITEM(out, 0, wrap(pk.part(0, n, at::kLong)));
     PyTuple_SET_ITEM(out, 1, wrap(pk.part(n * 8, n, at::kLong)));
@@ -686,7 +706,7 @@ PyObject* py_upload_tables(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       int32_t* p = pk.take<int32_t>(len);
       for (Py_ssize_t j = 0; j < len; ++j) p[j] = (int32_t)as_int(PyList_GET_ITEM(row, j));
     }
-    pk.dev.copy_(pk.host, true);
+    pk.send();
     PyObject* out = PyTuple_New(1 + extra);
     PyTuple_SET_ITEM(out, 0, wrap(pk.part(0, n * width, at::kInt).view({n, width})));
     int64_t byte = n * width * 4;
@@ -793,7 +813,7 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         p[i] = (int32_t)as_int(PyList_GET_ITEM(args[5], i));
         if (ordered) p[B + i] = (int32_t)as_int(PyList_GET_ITEM(args[6], i));
       }
-      pk.dev.copy_(pk.host, true);
+      pk.send();
       numbers = pk.dev;
       counts = (const int32_t*)numbers.data_ptr();
       if (ordered) order = counts + B;

@@ -556,6 +556,13 @@ int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t
                    float scale, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * `bytes` of host memory (whole 4-byte words, at most FC_UPLOAD_MAX) to device memory, in stream order; `host` may be
+ * reused when the call returns.  In a captured graph every replay writes the numbers of the capture.
+ */
+#define FC_UPLOAD_MAX 3072
+int fc_upload(void* dst, const void* host, int32_t bytes, void* stream);
+
+/*
  * Append and attention of one layer of a decode step (nanovllm/layers/attention.py:62-79): row i of k_new / v_new
  * ([batch][num_kv_heads][head_dim], `*_stride` elements between sequences) goes to cache slot slot_mapping[i]
  * (negative: skipped), then query i attends the first context_lens[i] tokens of sequence i.  Every new row is in the

@@ -442,3 +442,26 @@ def test_rows_only_general_path_launches_what_the_host_module_does(dev, monkeypa
     route = _lib.fn("fc_snapkv_rows_route")(ctypes.byref(kview), hq, W, 1, sum(lens) // B)
     assert called == [("snapkv_press", None) if route == 0 else ("snapkv_select", route)]
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("rows,width", [(1, 1), (9, 7), (64, 1), (13, 5), (64, 4), (64, 12), (96, 8), (97, 8), (90, 40)])
+def test_uploaded_tables_and_lengths(dev, rows, width):
+    """Numbers that travel as a kernel's arguments (up to 3072 bytes, three sizes of them) and those that are copied: the
+    tables padded with -1 and the lists behind them; the staging memory may be written again at once."""
+    ref = torch.zeros(1, device=dev)
+    tables = [[(r * 131 + i) % 1000 for i in range(width - r % width)] for r in range(rows)]
+    lens = [r * 7 + 1 for r in range(rows)]
+    got = [_lib.host().upload_tables(tables, (lens,), ref) for _ in range(3)]
+    more = _lib.host().upload_tables([[5] * width] * rows, (lens[::-1],), ref)
+    want = torch.tensor([t + [-1] * (width - len(t)) for t in tables], dtype=torch.int32)
+    for t, n in got:
+        assert torch.equal(t.cpu(), want) and n.tolist() == lens
+    assert bool((more[0] == 5).all()) and more[1].tolist() == lens[::-1]
+    buf = torch.full((1024,), -1, dtype=torch.int32, device=dev)
+    src = torch.arange(769, dtype=torch.int32)
+    assert _lib.fn("fc_upload")(buf.data_ptr(), src.data_ptr(), 3076, _lib.current_stream()) == -2
+    assert _lib.fn("fc_upload")(buf.data_ptr(), src.data_ptr(), 6, _lib.current_stream()) == -1
+    _lib.check(_lib.fn("fc_upload")(buf.data_ptr(), src.data_ptr(), 4 * min(768, rows * width), _lib.current_stream()), "fc_upload")
+    torch.cuda.synchronize()
+    n = min(768, rows * width)
+    assert torch.equal(buf[:n].cpu(), src[:n]) and bool((buf[n:] == -1).all())
