@@ -58,22 +58,25 @@ __global__ __launch_bounds__(THREADS, KPT > 16 ? 4 : 1) void column_select_kerne
   } else {
     const float* in = a.in + row * a.stride;
     if constexpr (SRC == CS_NORMS) {
-      // the arithmetic of knorm_kernel, four rows per lane in flight
+      // the arithmetic of knorm_kernel; of a short column twice as many rows per lane in flight
+      constexpr int NR = KPT == 1 ? 8 : 4;
       float* sc = reinterpret_cast<float*>(cs_lds + a.part_rows + TK_LDS_KEYS(THREADS, KPT));
       const int sub = tid % LPR, rg = tid / LPR;
       const char* kbase = kv.base + ((long long)l * kv.stride_layer + (long long)h * kv.stride_head) * EB + sub * 16;
-      for (int r0 = 0; r0 < n; r0 += RPP * 4) {
-        uint4 x[4];
+      for (int r0 = 0; r0 < n; r0 += RPP * NR) {
+        uint4 x[NR];
         unsigned live = 0;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < NR; ++u) {
+          if (r0 + u * RPP >= n) continue;         // wave-uniform: no loads of rows that are not there
           long long off = fc_token_offset(kv, b, min(r0 + u * RPP + rg, n - 1));
           live |= off >= 0 ? (1u << u) : 0u;
           off = off < 0 ? 0 : off;
           x[u] = *reinterpret_cast<const uint4*>(kbase + off * EB);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < NR; ++u) {
+          if (r0 + u * RPP >= n) continue;
           float part_sum = fc_group_sum<16>(row_sumsq_part<DTYPE>(x[u]));
           if (LPR == 32) part_sum += __shfl_xor(part_sum, 16, 64);
           const int r = r0 + u * RPP + rg;

@@ -276,3 +276,17 @@ def _rows_of_table(plane, table, S, H):
     if rows.shape[0] < S:
         rows = torch.cat([rows, torch.zeros(S - rows.shape[0], *rows.shape[1:], dtype=rows.dtype)])
     return rows.permute(1, 0, 2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S", [2, 31, 33, 127, 129, 255, 257, 385, 511, 512])
+def test_short_columns_scored_by_their_gathering_workgroups(dev, dtype, S):
+    """The Knorm hook on columns whose workgroups score them themselves, rows of the last turn missing or not, against scores
+    and selection by launches of their own: the same rows."""
+    from fastcache_amd.presses import KnormPress
+    g = torch.Generator().manual_seed(S)
+    k, v = (torch.randn(2, 3, S, 128, generator=g).to(dtype).to(dev) for _ in range(2))
+    got = KnormPress(0.5).compress(None, torch.zeros(2, S, 1, device=dev), k, v, None, {})
+    idx = ops.topk_select(ops.knorm_score(_lib.dense_view(k), dev), int(S * 0.5))[0].long()[..., None].expand(-1, -1, -1, 128)
+    for a, b in zip(got, (k, v)):
+        assert torch.equal(a, b.gather(2, idx))
