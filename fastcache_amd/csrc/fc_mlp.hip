@@ -296,12 +296,23 @@ __device__ __forceinline__ void mlp_body(char* lds, const KvView& src, const KvV
     // The prefetches are unconditional (straight-line code keeps the staging registers out of
     // scratch memory): past the last chunk the X rows are clamped to valid ones, and the
     // extra W1 chunk lands in the buffer nobody reads again.
-    x_load(xnext, q + 1);
-    ML_PIN();   // the prefetch stays ahead of this stage's multiplications
+    // Of a streamed W1 the next chunk is asked for ahead of the rows: loads arrive in order, and what waits for it at the
+    // end of the stage would wait for the rows as well, which have until the next stage.  us per pass, rows first -> W1 first,
+    // factor 5: 28 layers of 4 heads, 16 sequences of 16384 tokens 4191 -> 4130, 14 of 3875 to 11626 2113 -> 2048, 4 of 5840
+    // 459 -> 449; 32 of 32, 45 of 640 4193 -> 4127.  A list, whose rows any wavefront may fetch at any time, loses (8 prompts
+    // of 6000 tokens 783 -> 815).  Rows two chunks ahead, asked for before layers 2 and 3: no more than this, and 1 % less
+    // with W1 resident.
+    if (FLAT || W1R) x_load(xnext, q + 1);
     if (!W1R) {
+      if (FLAT) ML_PIN();
       __syncthreads();  // chunk q is in w1buf[q & 1]; every wavefront is done with chunk q - 1
       w1_load((kc + 1 < cf) ? kc + 1 : 0);
+      if (!FLAT) {
+        ML_PIN();
+        x_load(xnext, q + 1);
+      }
     }
+    ML_PIN();   // the prefetch stays ahead of this stage's multiplications
     {
       const char* wa = w1buf + (W1R ? kc : (q & 1)) * ML_WBYTES + lrow * ML_ROWB + lhalf * 16;
       uint4 af[2][4];      // weight fragments of k-step ks+1 are read while k-step ks multiplies
