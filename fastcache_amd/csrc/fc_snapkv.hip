@@ -886,9 +886,35 @@ static bool sk_split_shape(const fc_kv_view* keys, int32_t num_q_heads, int32_t 
   return true;
 }
 
+// Dense keys are one layer of a hook: a few to a few hundred columns, mostly one round, whose time the constants above miss by
+// the start of the second sweep, which costs a launch about as much as a whole column's one start.  Fitted to 162 shapes of
+// 200 to 12 000 keys and 4 to 256 columns by every n, all but 8 of which are within 2 % of the best n (those within 5 %): whole columns
+// 2 tiles a1 + f1, ranges 2 (tiles a + f) a round, down to one tile, and past SK_PIECES ranges m more, as every workgroup
+// reads their statistics twice.  us per hook, the rule above -> this: window 64, 8 columns of 400 keys 27.7 -> 19.9, of 1000
+// 23.1 -> 20.8, of 4000 32.4 -> 30.4, 32 of 250 21.5 -> 19.9, 64 of 400 28.8 -> 23.2; window 32, 16 of 350 23.1 -> 16.8, 32 of
+// 350 22.5 -> 17.1, of 1800 30.0 -> 27.6; 7 heads a group, 4 of 400 33.3 -> 25.9, of 4000 43.4 -> 39.5, 16 of 1000 31.2 -> 27.6.
+static int32_t sk_hook_splits(const SkSplitShape& s) {
+  const double a = s.blocks > 8 ? 1.65 : s.blocks > 4 ? 1.0 : 0.75, f = s.blocks > 8 ? 7.9 : s.blocks > 4 ? 5.2 : 4.2;
+  const double a1 = s.blocks > 8 ? 1.73 : s.blocks > 4 ? 1.12 : 1.02, f1 = s.blocks > 8 ? 8.5 : s.blocks > 4 ? 3.9 : 2.2;
+  const double m = s.blocks > 8 ? 6.0 : 3.0;
+  int best_n = 1;
+  double best = (double)((s.columns + s.slots - 1) / s.slots) * (2.0 * s.tiles * a1 + f1);
+  for (int n = 2; n <= 32 && n <= s.tiles; ++n) {
+    const double cost = 2.0 * (double)((s.columns * n + s.slots - 1) / s.slots) * ((s.tiles + n - 1) / n * a + f) +
+                        (n > SK_PIECES ? m : 0.0);
+    if (cost < best) {
+      best = cost;
+      best_n = n;
+    }
+  }
+  return best_n;
+}
+
 extern "C" int32_t fc_snapkv_select_splits(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) {
   SkSplitShape s;
   if (!sk_split_shape(keys, num_q_heads, window, s)) return 1;
+  // (token strides beyond what the split kernels take are left to the rule that cuts less)
+  if (!keys->block_tables && keys->num_layers == 1 && keys->stride_token >= 0 && keys->stride_token < (1 << 24)) return sk_hook_splits(s);
   const long long columns = s.columns, slots = s.slots;
   const int tiles = s.tiles;
   const double a = s.a, f = s.f;

@@ -819,6 +819,32 @@ def test_layer_hooks_in_one_call(dev, dtype, B, H, S):
                 assert not bool(((got ^ ref) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
 
 
+@pytest.mark.parametrize("Hq,H,W", [(8, 2, 64), (14, 2, 64), (7, 1, 32), (4, 4, 32)])     # 8, 14, 7 and 1 blocks of queries
+@pytest.mark.parametrize("S", [129, 191, 192, 193, 320, 449, 1100])
+def test_snapkv_hook_of_one_tile_a_range(dev, Hq, H, W, S):
+    """Short columns cut down to single tiles of 64 keys, the last one of one key, of all, or of window keys only: the
+    selection is that of the scores of whole columns but for keys near the threshold (other partial sums), window kept."""
+    keep, ksz = W + (S - W) // 3, 5
+    g = torch.Generator().manual_seed(S + Hq)
+    k = torch.randn(1, H, S, 128, generator=g).to(torch.float16)
+    v = torch.zeros_like(k)
+    pos = torch.arange(S)
+    v[..., 0], v[..., 1] = (pos % 256).to(v.dtype), (pos // 256).to(v.dtype)
+    kd, vd, q = k.to(dev), v.to(dev), torch.randn(1, Hq, W, 128, generator=g).to(torch.float16).to(dev)
+    assert S < 200 or ops.snapkv_select_splits(_lib.dense_view(kd), Hq, W) > 1
+    press = SnapKVPress(1.0 - (keep + 0.5) / S, window_size=W, kernel_size=ksz)
+    ok, ov = (t.cpu() for t in press.compress(None, torch.zeros(1, S, 1), kd, vd, None, {"queries": q}))
+    idx = ov[..., 0].long() + 256 * ov[..., 1].long()
+    assert torch.equal(ok, opress.gather_tokens(k, idx)) and bool((idx[..., 1:] > idx[..., :-1]).all())
+    assert bool((idx[..., -W:] == pos[-W:]).all())
+    scores = ops.snapkv_score(_lib.dense_view(kd), q[None], W, ksz, splits=1)[0].cpu()
+    want = opress.topk_lowest_index(scores, keep)
+    kth = scores.gather(-1, want).min(-1, keepdim=True).values
+    got = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, idx, True)
+    ref = torch.zeros_like(got).scatter_(-1, want, True)
+    assert not bool(((got ^ ref) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+
+
 @pytest.mark.parametrize("S", [500, 1000, 2000, 4096, 8000, 8681, 12320, 16000, 20000])     # one of each selection size
 def test_selection_of_pooled_sums_is_the_same_every_time(dev, S):
     """A SnapKV hook whose columns are each selected by many workgroups, again and again: one selection, and no key kept or

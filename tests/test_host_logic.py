@@ -560,6 +560,26 @@ def test_snapkv_splits_of_sequences_of_different_lengths():
                 assert ragged in (1, equal), (L, B, H, S, mean)
 
 
+def test_snapkv_splits_of_one_dense_layer():
+    """A hook's columns are cut by a rule of their own, down to one tile of 64 keys a range and never into more than 32; paged
+    columns, several layers and token strides that the split kernels do not take keep the other rule."""
+    import ctypes
+    from fastcache_amd import _lib
+
+    def splits(L, B, H, hq, S, W, **kw):
+        v = _lib.FcKvView(**dict(dict(num_layers=L, batch=B, num_kv_heads=H, max_seq_len=S, stride_token=128), **kw))
+        return _lib.fn("fc_snapkv_select_splits")(ctypes.byref(v), hq, W)
+
+    assert splits(1, 1, 8, 32, 400, 64) == 7 and splits(1, 1, 8, 32, 64, 64) == 1
+    assert splits(1, 1, 8, 32, 400, 64, block_tables=1, block_size=256) == splits(2, 1, 8, 32, 400, 64) == 1
+    assert splits(1, 1, 8, 32, 400, 64, stride_token=1 << 24) == splits(1, 1, 8, 32, 400, 64, stride_token=-128) == 1
+    assert splits(1, 1, 1, 17, 400, 32) == 1                    # 17 blocks of queries
+    for B, H, hq, W in ((1, 8, 32, 64), (8, 32, 32, 64), (1, 4, 28, 64), (3, 4, 28, 32)):
+        for S in (65, 128, 129, 1000, 5000, 36000):
+            n, tiles = splits(1, B, H, hq, S, W), -(-S // 64)
+            assert 1 <= n <= min(32, tiles)
+
+
 def test_snapkv_rows_route_is_the_split_rules():
     """0 where the one launch takes the shape and its rule leaves columns whole, else the ranges of the rule that applies,
     and -1 past the selection's keys or with more than 16 blocks of window queries."""
