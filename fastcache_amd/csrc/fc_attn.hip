@@ -388,7 +388,7 @@ template <int DTYPE>
 __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* __restrict__ part_o,
                                                                    const float* __restrict__ part_ml,
                                                                    const int* __restrict__ lens, int max_seq_len,
-                                                                   int Hq, int max_splits, int chunk,
+                                                                   int Hq, int max_splits, int chunk, int alone,
                                                                    char* __restrict__ out) {
   const int hq = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
   int len = min(lens[b], max_seq_len);
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
     *o = 0;
     return;
   }
-  const int ns = (len + chunk - 1) / chunk;
+  const int ns = len <= chunk + alone ? 1 : (len + chunk - 1) / chunk;
   const float* ml = part_ml + ((long long)b * Hq + hq) * max_splits * 2;
   const float* po = part_o + ((long long)b * Hq + hq) * max_splits * FC_HEAD_DIM + d;
   // eight splits per step so that their loads are in flight together
@@ -456,6 +456,10 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 #define DC_THREADS (DC_WAVES * 64)
 #define DC_HEADS 16
 #define DC_PSTRIDE 132                                             // floats per partial output row (padded against bank conflicts)
+// A sequence that reaches at most this far into its column's second range is its first workgroup's alone: a second tile for half
+// of the wavefronts is shorter than a merge.  us a layer, 16 captured layers of columns of 270 to 375 tokens, merged -> alone:
+// 4 columns 9.5 -> 8.1 to 8.7, 48 10.9 -> 8.9 to 9.6; of 400 9.5 -> 9.4, of 500 10.0 -> 10.6.
+#define DC_ALONE 128
 #define DC_STAGES 2                                                // V tiles of a wavefront in LDS or on their way
 #define DC_MERGE 8                                                // partial rows in flight per thread of the merge
 #define DC_PART (DC_WAVES * DC_STAGES * DA_TILEB)                   // V stages, then the partial outputs
@@ -553,9 +557,10 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   len = max(min(len, kc.max_seq_len), 0);
   const int nb = (int)gridDim.y;
   int slot = PAGED && ap.k_new && lane < nb ? ap.slots[lane] : -1;   // the new rows' slots, 64 sequences at a time
-  const int t0 = (int)blockIdx.z * chunk;
+  const int span = max_splits > 1 && len <= chunk + DC_ALONE ? chunk + DC_ALONE : chunk;
+  const int t0 = (int)blockIdx.z * span;
   if (t0 >= len && blockIdx.z != 0) return;
-  const int end = min(len, t0 + chunk);
+  const int end = min(len, t0 + span);
   // the query heads as B operand; columns past the group are zero
   uint4 qf[4];
   {
@@ -604,7 +609,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
     }
   }
   unsigned short* orow = reinterpret_cast<unsigned short*>(out) + ((long long)b * Hq + h * G + g0) * FC_HEAD_DIM;
-  const bool whole = max_splits == 1 || (TURN && len <= chunk);
+  const bool whole = max_splits == 1 || (TURN && len <= span);
   if (len <= 0) {       // with several workgroups per column the merge writes the zeros
     if (whole)
       for (int i = tid; i < ng * FC_HEAD_DIM; i += DC_THREADS) orow[i] = 0;
@@ -863,7 +868,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   // device's point of coherence before the workgroup counts itself, so the last one reads all of them there.  (Ordinary
   // stores with a release and an acquire, which write back and drop caches, instead: 341 us for the 28 layers that take
   // 296 this way and 374 with the merge's own launch, host bound.)
-  const int ns = (len + chunk - 1) / chunk;
+  const int ns = (len + span - 1) / span;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   unsigned* arrived = (arrivals ? arrivals : dc_arrived[turn]) + (blockIdx.y * gridDim.x + blockIdx.x);
@@ -1137,14 +1142,14 @@ static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_h
 }
 
 static int da_merge(const char* who, const fc_kv_view* k_cache, const float* part_o, const float* part_ml,
-                    const int32_t* context_lens, int num_q_heads, int splits, int chunk, void* out, void* stream) {
+                    const int32_t* context_lens, int num_q_heads, int splits, int chunk, int alone, void* out, void* stream) {
   dim3 grid(num_q_heads, k_cache->batch);
   if (k_cache->dtype == FC_BF16)
     hipLaunchKernelGGL((decode_merge_kernel<FC_BF16>), grid, dim3(FC_HEAD_DIM), 0, (hipStream_t)stream, part_o, part_ml,
-                       context_lens, k_cache->max_seq_len, num_q_heads, splits, chunk, (char*)out);
+                       context_lens, k_cache->max_seq_len, num_q_heads, splits, chunk, alone, (char*)out);
   else
     hipLaunchKernelGGL((decode_merge_kernel<FC_F16>), grid, dim3(FC_HEAD_DIM), 0, (hipStream_t)stream, part_o, part_ml,
-                       context_lens, k_cache->max_seq_len, num_q_heads, splits, chunk, (char*)out);
+                       context_lens, k_cache->max_seq_len, num_q_heads, splits, chunk, alone, (char*)out);
   FC_CHECK_LAUNCH(who);
   return FC_OK;
 }
@@ -1207,7 +1212,7 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
 #undef DC_LAUNCH
     FC_CHECK_LAUNCH(who);
     if (csplits > 1 && !last_merges)
-      return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, csplits, column, out, stream);
+      return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, csplits, column, DC_ALONE, out, stream);
     return FC_OK;
   }
   const int64_t need = fc_decode_attn_workspace_bytes(k_cache->batch, num_q_heads, k_cache->max_seq_len);
@@ -1273,7 +1278,7 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
 #undef DA_LAUNCH
     FC_CHECK_LAUNCH(who);
   }
-  return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, splits, chunk, out, stream);
+  return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, splits, chunk, 0, out, stream);
 }
 
 extern "C" int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t layer, const void* q,

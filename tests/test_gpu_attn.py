@@ -599,3 +599,43 @@ def test_bucket_graphs_hold_one_launch_per_layer(dev, Hq, Hkv, lens, plain, merg
         reset_context()
     for o in got:
         assert torch.equal(o.view(torch.int16), eager.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,lens,pages", [
+    (14, 2, [384, 385, 257, 383, 0, 512], 2),           # the first workgroup's alone, or two ranges merged, either side of the border
+    (2, 2, [384, 385, 641, 700], 3),
+    (8, 2, ([640, 641, 513, 768] * 12)[:46], 3),        # ranges of 512
+])
+def test_sequences_that_reach_a_little_into_a_second_range(dev, dtype, Hq, Hkv, lens, pages):
+    """Merged by the last workgroup, by a launch, or one workgroup's alone: the oracle's values, and the same bits whoever
+    merges."""
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    B = len(lens)
+    case = synth.make_paged_case(seed=71, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=[n + 1 for n in lens], dtype=dtype)
+    g = torch.Generator().manual_seed(6)
+    q, k, v = (torch.randn(B, h * 128, generator=g).to(dtype) for h in (Hq, Hkv, Hkv))
+    tables, lens_t = case.table_tensor("cpu")[:, :pages].contiguous(), torch.tensor(lens, dtype=torch.int32)
+    pool = case.kv_cache[:, 0]
+    ref = oattn.decode_attention(q.view(B, Hq, 128), pool[0], pool[1], lens_t, tables, 128 ** -0.5)
+    layer, on_gpu = Attention(Hq, 128, 128 ** -0.5, Hkv), pool.to(dev)
+    layer.k_cache, layer.v_cache = on_gpu[0], on_gpu[1]
+    q, k, v = q.to(dev), k.to(dev), v.to(dev)
+    set_context(False, slot_mapping=torch.full((B,), -1, dtype=torch.int32, device=dev), context_lens=lens_t.to(dev),
+                block_tables=tables.to(dev))
+    try:
+        eager = layer(q, k, v)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            held = layer(q, k, v)
+        for _ in range(3):
+            held.zero_()
+            graph.replay()
+            again = layer(q, k, v)
+            torch.cuda.synchronize()
+            assert torch.equal(held.view(torch.int16), eager.view(torch.int16))
+            assert torch.equal(again.view(torch.int16), eager.view(torch.int16))
+    finally:
+        reset_context()
+    assert float((eager.cpu().view(B, Hq, 128).float() - ref.float()).abs().max()) < 4e-3      # as above
