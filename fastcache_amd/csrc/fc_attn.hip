@@ -1090,8 +1090,7 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 }
 
 // Tokens per workgroup of the column kernel, 0 = the launch does not take it.  It takes launches whose workgroups are all
-// resident at once (one per compute unit: registers) and, of groups of 5 and more heads, twice as many short columns: beyond
-// that bandwidth counts and the split kernel streams better (128 columns of 1024 tokens: 19.4 us a layer against 19.6 to 23).  One 32-token tile per wavefront, 256 tokens, is
+// resident at once (one per compute unit: registers) and twice as many short columns: beyond that bandwidth counts and the split kernel streams better (128 columns of 1024 tokens: 19.4 us a layer against 19.6 to 23).  One 32-token tile per wavefront, 256 tokens, is
 // the shortest chain (a second tile costs about 3 us, a merge 3.5): 12 columns of 1024 tokens 13.2 -> 10.1 us, of 256
 // tokens without a merge 7.1, 48 columns of 1024 tokens 16.9 -> 13.0.  Where 256 would be too many workgroups, columns
 // short enough for one workgroup each still gain by not being merged: 192 columns of 512 tokens 16.7 -> 15.4 us, 256 of
@@ -1101,7 +1100,10 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 // 5 and more heads, where a K and V read once feeds the matrix pipe for all of them: 2 tiles, 48 columns of 1500 tokens
 // 569 -> 464, 24 of 5000 639 -> 489; 4, 64 of 4000 in groups of 8 1012 -> 752; 8, 200 of 1700 1073 -> 929; 8, 64 of 8000
 // 784 -> 697; and two rounds of whole columns, 360 of 600 621 -> 451, 400 of 300 529 -> 330, but not of longer ones (360 of
-// 2000 1030 -> 1054).  Groups of 3 and 4: 2 tiles 572 -> 487 (96 of 1000), 3 635 -> 587, 4 748 -> 715, 802 -> 743, one
+// 2000 1030 -> 1054).  Two rounds of whole columns of groups of 3 and 4 as well (32 heads on 8, 12 captured layers, max_seq_len
+// 768 / 512: 40 sequences of 100 to 700 368 -> 308, 60 of 700 528 -> 508; 48 of 100 to 500 323 -> 286, 60 of 300 to 500
+// 384 -> 358), of smaller groups only up to 256 tokens (32 heads: 12 of 100 to 250 231 -> 201, 14 of 250 263 -> 242; of 512, 12 of
+// 100 to 500 281 -> 244 but of 500 340 -> 354).  Groups of 3 and 4: 2 tiles 572 -> 487 (96 of 1000), 3 635 -> 587, 4 748 -> 715, 802 -> 743, one
 // 693 -> 697; 5 730 -> 799, 921 -> 1027.  Smaller groups: 2 tiles 588 -> 551 (64 of 2000), 675 -> 533; 3 to 6 where the
 // workgroups are seven eighths of the compute units with ranges 85 % full, or three quarters and whole columns (32 heads, 12
 // captured layers, or 28 eager ones): 6 sequences of 800 288 -> 234, 1 of 8000 445 -> 374, 2 of 5000 413 -> 393, 8 of 1300
@@ -1130,7 +1132,8 @@ static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_h
     return 0;
   const int chunk = DC_WAVES * DA_TILE;
   if (cols * ((k->max_seq_len + chunk - 1) / chunk) <= slots) return chunk;
-  if (cols <= (G > 4 ? 2 : 1) * slots && k->max_seq_len <= DC_ONE) return DC_ONE;
+  if (cols <= (G > 2 ? 2 : 1) * slots && k->max_seq_len <= DC_ONE) return DC_ONE;
+  if (cols <= 2 * slots && k->max_seq_len <= chunk) return chunk;
   const int most = G > 4 ? DC_TILES_MANY : G > 2 ? DC_TILES_SOME : DC_TILES_FEW;
   for (int m = 2; m <= most; ++m) {
     const long long ranges = (k->max_seq_len + m * chunk - 1) / (m * chunk), wgs = cols * ranges;

@@ -639,3 +639,36 @@ def test_sequences_that_reach_a_little_into_a_second_range(dev, dtype, Hq, Hkv, 
     finally:
         reset_context()
     assert float((eager.cpu().view(B, Hq, 128).float() - ref.float()).abs().max()) < 4e-3      # as above
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,B,most,one", [(32, 32, 9, 256, True), (32, 32, 9, 257, False), (32, 16, 32, 256, True), (32, 16, 33, 256, False),
+                                               (32, 8, 64, 512, True), (24, 8, 33, 768, True), (32, 8, 33, 769, False)])
+def test_two_rounds_of_short_columns(dev, dtype, Hq, Hkv, B, most, one):
+    """More columns than compute units and at most twice as many: short ones whole in one launch, which appends, the others by the
+    split kernel; the oracle's values either way."""
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    lens = [(most * (i + 1)) // B - 1 for i in range(B)]
+    case = synth.make_paged_case(seed=81, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=[n + 1 for n in lens], dtype=dtype)
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(B, h * 128, generator=g).to(dtype) for h in (Hq, Hkv, Hkv))
+    tables, lens_t = case.table_tensor("cpu"), torch.tensor(lens, dtype=torch.int32)
+    slots = torch.tensor([t[n // 256] * 256 + n % 256 for t, n in zip(case.block_tables, lens)], dtype=torch.int32)
+    pool = case.kv_cache[:, 0].clone()
+    ref = oattn.decode_attention(q.view(B, Hq, 128), pool[0], pool[1], lens_t, tables, 128 ** -0.5)
+    for p, new in ((0, k), (1, v)):
+        pool[p].view(-1, Hkv, 128)[slots.long()] = new.view(B, Hkv, 128)
+    layer, on_gpu = Attention(Hq, 128, 128 ** -0.5, Hkv), case.kv_cache[:, 0].to(dev)
+    layer.k_cache, layer.v_cache = on_gpu[0], on_gpu[1]
+    set_context(False, slot_mapping=slots.to(dev), context_lens=lens_t.to(dev), block_tables=tables.to(dev))
+    try:
+        got = [layer(q.to(dev), k.to(dev), v.to(dev)).cpu()]
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
+            got.append(layer(q.to(dev), k.to(dev), v.to(dev)).cpu())
+        assert any("decode_column_kernel<" in e.name for e in prof.events()) == one
+    finally:
+        reset_context()
+    assert torch.equal(on_gpu.cpu(), pool)
+    for o in got:
+        assert float((o.view(B, Hq, 128).float() - ref.float()).abs().max()) < 4e-3      # as above
