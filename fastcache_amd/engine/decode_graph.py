@@ -94,13 +94,14 @@ class BucketedDecodeGraphs:
         self.graph_bs: List[int] = []
         self.graph_vars: Dict[str, torch.Tensor] = {}
         self.graph_pool = None
+        self._scratch = ()          # what the captured kernels write besides the static buffers
 
     def _model(self, q, k, v, out):
         # a layer's own result is written where it belongs: a copy node behind every layer was 4.6 of its 12.2 us (28 query
         # heads on 4, 9 sequences of 100 to 248 tokens)
         for i, layer in enumerate(self.layers):
             to = out[i]
-            o = layer(q[i], k[i], v[i], out=to) if type(layer).forward is Attention.forward else layer(q[i], k[i], v[i])
+            o = layer(q[i], k[i], v[i], out=to) if getattr(layer.forward, "__func__", None) is Attention.forward else layer(q[i], k[i], v[i])
             if o.data_ptr() != to.data_ptr():      # another module's, or a forward hook's
                 to.copy_(o)
 
@@ -119,6 +120,7 @@ class BucketedDecodeGraphs:
         workspace = ops.decode_attn_workspace(bsz, a.num_heads, self.max_num_blocks * block_size, dev)
         # the columns' last workgroups merge their ranges, told by counters that belong to the graphs like the workspace does
         arrivals = torch.zeros(_lib.DECODE_ARRIVALS, dtype=torch.int32, device=dev)
+        self._scratch = (workspace, arrivals)       # the layers' own references end with the next capture
         for layer in self.layers:
             layer.workspace, layer.arrivals = workspace, arrivals
         self.graph_bs = [b for b in [1, 2, 4, 8] + list(range(16, bsz + 1, 16)) if b <= bsz]

@@ -672,3 +672,36 @@ def test_two_rounds_of_short_columns(dev, dtype, Hq, Hkv, B, most, one):
     assert torch.equal(on_gpu.cpu(), pool)
     for o in got:
         assert float((o.view(B, Hq, 128).float() - ref.float()).abs().max()) < 4e-3      # as above
+
+
+def test_graphs_keep_their_scratch_when_the_layers_are_captured_again(dev):
+    """Two sets of bucketed graphs over the same layers, the second capture of which replaces the layers' scratch: the first
+    set still owns what its kernels write, and a ``forward`` set on one layer object is called as it was set."""
+    from fastcache_amd.engine.decode_graph import BucketedDecodeGraphs
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    L, Hq, Hkv, lens, dtype = 2, 7, 1, [700, 1000], torch.bfloat16
+    case = synth.make_paged_case(seed=62, num_layers=L, batch=2, num_kv_heads=Hkv, seq_lens=[n + 1 for n in lens], dtype=dtype)
+    pool, tables = case.kv_cache.to(dev), case.table_tensor(dev)
+    layers = [Attention(Hq, 128, 128 ** -0.5, Hkv) for _ in range(L)]
+    for l, a in enumerate(layers):
+        a.k_cache, a.v_cache = pool[0, l], pool[1, l]
+    plain = layers[1].forward
+    layers[1].forward = lambda q, k, v: plain(q, k, v)
+    sets = []
+    for _ in range(2):
+        sets.append(BucketedDecodeGraphs(layers, 2, tables.shape[1], dtype, dev))
+        sets[-1].capture_cudagraph()
+    a, b = (s._scratch for s in sets)
+    assert layers[0].workspace is b[0] and a[0].data_ptr() != b[0].data_ptr() and a[1].data_ptr() != b[1].data_ptr()
+    others = [torch.full_like(a[0], 255) for _ in range(8)]
+    g = torch.Generator().manual_seed(8)
+    q, k, v = (torch.randn(L, 2, h * 128, generator=g).to(dtype).to(dev) for h in (Hq, Hkv, Hkv))
+    set_context(False, slot_mapping=torch.full((2,), -1, dtype=torch.int32, device=dev),
+                context_lens=torch.tensor(lens, dtype=torch.int32, device=dev), block_tables=tables)
+    try:
+        outs = [s.run(q, k, v).clone() for s in sets for _ in range(3)]
+    finally:
+        reset_context()
+    assert all(torch.equal(o.view(torch.int16), outs[0].view(torch.int16)) for o in outs)
+    assert all(bool((t == 255).all()) for t in others)
