@@ -69,8 +69,54 @@ struct DaCfg {
   // ring | logits, then probabilities [GT][chunk]: fp32, or with eight heads (p * V on the matrix pipe) each
   // probability as two 16-bit halves hi + lo in the cache dtype
   static constexpr bool PV_MFMA = GT >= DA_PV_MFMA_MIN;
-  static constexpr int lds(int chunk) { return DA_RING + GT * chunk * 4; }
+  static constexpr int lds(int chunk) { return DA_RING + GT * chunk * 4 + GT * 4; }
 };
+
+struct DaAppend {                 // the step's new rows, one per sequence (k_new null: nothing to append)
+  const char *k_new, *v_new;
+  long long k_stride, v_stride;   // bytes between sequences; heads are adjacent
+  const int* slots;               // flat cache slot per sequence, negative = skip
+};
+
+
+// A new row inside a workgroup's range [t0, end) is written by this workgroup, which then has to see it land before it reads
+// it back (true is returned), whichever sequence of the batch it belongs to (a table may be listed twice with lengths one
+// apart, or a page be shared): nobody depends on another workgroup's write.  The sequence's own row is also written by its last
+// workgroup, since it usually lies right behind the range.  Workgroups that write one row write the same bytes.
+// slot: of sequence `lane` (negative: none), ktbl: table entry `lane` of sequence b; both planes use one table.
+__device__ __forceinline__ bool da_append_rows(const KvView& kc, const KvView& vc, const DaAppend& ap, const char* kbase,
+                                               const char* vbase, int slot, int ktbl, int b, int h, int nb, int t0, int end,
+                                               int len, int tid) {
+  const int lane = tid & 63, l15 = tid & 15;
+  const int e0 = t0 >> kc.block_shift, e1 = (end - 1) >> kc.block_shift;      // pages of the range (none: e1 < e0)
+  bool inside = false;
+  for (int j0 = 0; j0 < nb; j0 += FC_WAVE) {
+    if (j0 > 0) slot = j0 + lane < nb ? ap.slots[j0 + lane] : -1;
+    const int page = slot >> kc.block_shift, at = slot & (kc.block_size - 1);
+    bool hit = false;
+    for (int e = e0; e <= e1; ++e) {
+      const int pos = (e << kc.block_shift) + at;
+      hit |= slot >= 0 && page == __builtin_amdgcn_readlane(ktbl, e) && pos >= t0 && pos < end;
+    }
+    unsigned long long todo = __ballot(hit);
+    inside |= todo != 0ull;
+    if (end == len) todo |= __ballot(slot >= 0 && j0 + lane == b);
+    while (todo) {                                                            // wave-uniform
+      const int j = __builtin_ctzll(todo);
+      todo &= todo - 1;
+      const int row = __builtin_amdgcn_readlane(slot, j);
+      const long long rpage = row >> kc.block_shift, rat = row & (kc.block_size - 1);
+      if (tid < 32) {
+        const bool is_v = tid >= 16;
+        const long long koff = rpage * kc.stride_block + rat * kc.stride_token, voff = rpage * vc.stride_block + rat * vc.stride_token;
+        char* dst = is_v ? const_cast<char*>(vbase) + voff * 2 : const_cast<char*>(kbase) + koff * 2;
+        const char* src = is_v ? ap.v_new + (j0 + j) * ap.v_stride : ap.k_new + (j0 + j) * ap.k_stride;
+        *reinterpret_cast<uint4*>(dst + l15 * 16) = *reinterpret_cast<const uint4*>(src + (long long)h * FC_HEAD_DIM * 2 + l15 * 16);
+      }
+    }
+  }
+  return inside;
+}
 
 // GT = query heads served per workgroup (a tile of the group, at most 8).
 // FAST = a 32-token tile never straddles two pages (dense view, or pages of 32*2^n tokens), so a tile
@@ -82,16 +128,19 @@ struct DaCfg {
 // wavefront are in flight for most of the kernel and no load waits behind a workgroup barrier.
 // Logits are one v_mfma_f32_32x32x16 block per tile with the query heads as rows (padded with zero
 // rows to 32): whatever the group size, K is read from LDS once.
-template <int DTYPE, int GT, bool FAST>
+// WHOLE: the chunk holds every sequence: the workgroup writes the output (as the merge of one chunk would) and, asked to
+// (one kv head a workgroup, one table for both planes), appends the step's rows.
+template <int DTYPE, int GT, bool FAST, bool WHOLE>
 __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, KvView vc, int layer,
                                                                     const char* __restrict__ q, int Hq,
                                                                     const int* __restrict__ lens, float c,
                                                                     float* __restrict__ part_o,
                                                                     float* __restrict__ part_ml, int max_splits,
-                                                                    int chunk) {
+                                                                    int chunk, char* __restrict__ out, DaAppend ap) {
   extern __shared__ __align__(16) char smem[];
   float* sc = reinterpret_cast<float*>(smem + DA_RING);          // [GT][chunk]
   unsigned* p2 = reinterpret_cast<unsigned*>(smem + DA_RING);    // the same seen as (hi, lo) pairs
+  float* sums = reinterpret_cast<float*>(smem + DA_RING + GT * chunk * 4);   // WHOLE: [GT]
   constexpr bool PV_MFMA = DaCfg<GT>::PV_MFMA;
   float(*red)[GT][FC_HEAD_DIM] = reinterpret_cast<float(*)[GT][FC_HEAD_DIM]>(smem);  // [16] partial outputs, reuses the ring
   static_assert(16 * GT * FC_HEAD_DIM * 4 <= DA_RING, "partial outputs must fit in the ring");
@@ -124,7 +173,12 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   }
   int len = __builtin_amdgcn_readfirstlane(lens[b]);
   len = min(len, kc.max_seq_len);
-  if (t0 >= len) return;
+  const int nb = (int)gridDim.z;
+  int slot = -1;
+  if constexpr (WHOLE) {
+    if (ap.k_new && lane < nb) slot = ap.slots[lane];
+  }
+  if (!WHOLE && t0 >= len) return;
   const int ntok = min(chunk, len - t0);
 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -142,6 +196,18 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
 
   const char* kbase = kc.base + ((long long)layer * kc.stride_layer + (long long)h * kc.stride_head) * 2;
   const char* vbase = vc.base + ((long long)layer * vc.stride_layer + (long long)h * vc.stride_head) * 2;
+  if constexpr (WHOLE) {
+    len = max(len, 0);
+    if (ap.k_new && da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, b, h, nb, 0, len, len, tid)) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
+    if (len == 0) {
+      unsigned short* orow = reinterpret_cast<unsigned short*>(out) + ((long long)b * Hq + h * G + g0) * FC_HEAD_DIM;
+      for (int i = tid; i < min(GT, G - g0) * FC_HEAD_DIM; i += DA_THREADS) orow[i] = 0;
+      return;
+    }
+  }
   const unsigned ring_lds = __builtin_amdgcn_readfirstlane(fc_lds_addr(smem)) + wave * (2 * DA_TILEB);
   char* ring = smem + wave * (2 * DA_TILEB);
 
@@ -257,13 +323,21 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
       sum += p;
     }
     sum = fc_wave_sum_uniform(sum);
-    if (lane == 0 && g0 + g < G) {
+    if (WHOLE) {
+      if (lane == 0) sums[g] = sum;
+    } else if (lane == 0 && g0 + g < G) {
       float* ml = part_ml + (((long long)b * Hq + (h * G + g0 + g)) * max_splits + split) * 2;
       ml[0] = m;
       ml[1] = sum;
     }
   }
   fc_lds_barrier();
+
+  const auto put = [&](int g, int d, float o) {
+    const long long row = (long long)b * Hq + (h * G + g0 + g);
+    if constexpr (WHOLE) reinterpret_cast<unsigned short*>(out)[row * FC_HEAD_DIM + d] = da_pack<DTYPE>(o / sums[g]);
+    else part_o[(row * max_splits + split) * FC_HEAD_DIM + d] = o;
+  };
 
   // ---- phase 3: sum of p * V over this wavefront's tiles -------------------------------------------
   if constexpr (PV_MFMA) {
@@ -330,7 +404,7 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
       const int g = i / FC_HEAD_DIM, d = i - g * FC_HEAD_DIM;
       if (g0 + g < G) {
         const float o = ((red[0][g][d] + red[1][g][d]) + (red[2][g][d] + red[3][g][d])) * (1.f / DA_P_SCALE(DTYPE));
-        part_o[(((long long)b * Hq + (h * G + g0 + g)) * max_splits + split) * FC_HEAD_DIM + d] = o;
+        put(g, d, o);
       }
     }
   } else {
@@ -378,7 +452,7 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
         float o = 0.f;
 #pragma unroll
         for (int sl = 0; sl < 16; ++sl) o += red[sl][g][d];
-        part_o[(((long long)b * Hq + (h * G + g0 + g)) * max_splits + split) * FC_HEAD_DIM + d] = o;
+        put(g, d, o);
       }
     }
   }
@@ -511,12 +585,6 @@ __device__ __forceinline__ uint2 da_lds_transposed(unsigned addr) {
                                        reinterpret_cast<__attribute__((address_space(3))) da_s16x4*>((size_t)addr)));
 }
 
-struct DaAppend {                 // the step's new rows, one per sequence (k_new null: nothing to append)
-  const char *k_new, *v_new;
-  long long k_stride, v_stride;   // bytes between sequences; heads are adjacent
-  const int* slots;               // flat cache slot per sequence, negative = skip
-};
-
 // Arrivals per column of a launch whose last workgroup merges, a row of counters per turn (fc_decode_layer_turn) or the
 // caller's (fc_decode_layer_arrivals).  Zero between launches: whoever merges puts the zero back.
 #define DC_COLUMNS FC_DECODE_ARRIVALS
@@ -572,38 +640,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   const char* kbase = kc.base + ((long long)layer * kc.stride_layer + (long long)h * kc.stride_head) * 2;
   const char* vbase = vc.base + ((long long)layer * vc.stride_layer + (long long)h * vc.stride_head) * 2;
   if (PAGED && ap.k_new) {
-    // A new row inside this workgroup's range is written by this workgroup, which then has to see it land before it reads
-    // it back, whichever sequence of the batch it belongs to (a table may be listed twice with lengths one apart, or a page
-    // be shared): nobody depends on another workgroup's write.  The sequence's own row is also written by its last
-    // workgroup, since it usually lies right behind the range.  Workgroups that write one row write the same bytes.
-    const int e0 = t0 >> kc.block_shift, e1 = (end - 1) >> kc.block_shift;      // pages of the range (none: e1 < e0)
-    bool inside = false;
-    for (int j0 = 0; j0 < nb; j0 += FC_WAVE) {
-      if (j0 > 0) slot = j0 + lane < nb ? ap.slots[j0 + lane] : -1;
-      const int page = slot >> kc.block_shift, at = slot & (kc.block_size - 1);
-      bool hit = false;
-      for (int e = e0; e <= e1; ++e) {
-        const int pos = (e << kc.block_shift) + at;
-        hit |= slot >= 0 && page == __builtin_amdgcn_readlane(ktbl, e) && pos >= t0 && pos < end;
-      }
-      unsigned long long todo = __ballot(hit);
-      inside |= todo != 0ull;
-      if (end == len) todo |= __ballot(slot >= 0 && j0 + lane == b);
-      while (todo) {                                                            // wave-uniform
-        const int j = __builtin_ctzll(todo);
-        todo &= todo - 1;
-        const int row = __builtin_amdgcn_readlane(slot, j);
-        const long long rpage = row >> kc.block_shift, rat = row & (kc.block_size - 1);
-        if (tid < 32) {
-          const bool is_v = tid >= 16;
-          const long long koff = rpage * kc.stride_block + rat * kc.stride_token, voff = rpage * vc.stride_block + rat * vc.stride_token;
-          char* dst = is_v ? const_cast<char*>(vbase) + voff * 2 : const_cast<char*>(kbase) + koff * 2;
-          const char* src = is_v ? ap.v_new + (j0 + j) * ap.v_stride : ap.k_new + (j0 + j) * ap.k_stride;
-          *reinterpret_cast<uint4*>(dst + l15 * 16) = *reinterpret_cast<const uint4*>(src + (long long)h * FC_HEAD_DIM * 2 + l15 * 16);
-        }
-      }
-    }
-    if (inside) {
+    if (da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, b, h, nb, t0, end, len, tid)) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     }
@@ -1090,7 +1127,8 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 }
 
 // Tokens per workgroup of the column kernel, 0 = the launch does not take it.  It takes launches whose workgroups are all
-// resident at once (one per compute unit: registers) and twice as many short columns: beyond that bandwidth counts and the split kernel streams better (128 columns of 1024 tokens: 19.4 us a layer against 19.6 to 23).  One 32-token tile per wavefront, 256 tokens, is
+// resident at once (one per compute unit: registers) and, of groups of 5 and more heads, twice as many short columns: beyond
+// that bandwidth counts and the split kernel streams better (128 columns of 1024 tokens: 19.4 us a layer against 19.6 to 23).  One 32-token tile per wavefront, 256 tokens, is
 // the shortest chain (a second tile costs about 3 us, a merge 3.5): 12 columns of 1024 tokens 13.2 -> 10.1 us, of 256
 // tokens without a merge 7.1, 48 columns of 1024 tokens 16.9 -> 13.0.  Where 256 would be too many workgroups, columns
 // short enough for one workgroup each still gain by not being merged: 192 columns of 512 tokens 16.7 -> 15.4 us, 256 of
@@ -1100,10 +1138,10 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 // 5 and more heads, where a K and V read once feeds the matrix pipe for all of them: 2 tiles, 48 columns of 1500 tokens
 // 569 -> 464, 24 of 5000 639 -> 489; 4, 64 of 4000 in groups of 8 1012 -> 752; 8, 200 of 1700 1073 -> 929; 8, 64 of 8000
 // 784 -> 697; and two rounds of whole columns, 360 of 600 621 -> 451, 400 of 300 529 -> 330, but not of longer ones (360 of
-// 2000 1030 -> 1054).  Two rounds of whole columns of groups of 3 and 4 as well (32 heads on 8, 12 captured layers, max_seq_len
-// 768 / 512: 40 sequences of 100 to 700 368 -> 308, 60 of 700 528 -> 508; 48 of 100 to 500 323 -> 286, 60 of 300 to 500
-// 384 -> 358), of smaller groups only up to 256 tokens (32 heads: 12 of 100 to 250 231 -> 201, 14 of 250 263 -> 242; of 512, 12 of
-// 100 to 500 281 -> 244 but of 500 340 -> 354).  Groups of 3 and 4: 2 tiles 572 -> 487 (96 of 1000), 3 635 -> 587, 4 748 -> 715, 802 -> 743, one
+// 2000 1030 -> 1054).  Smaller groups leave those to the split kernel, which holds them whole as well (12 captured layers, this /
+// that: 32 heads, 10 of 100 to 250 186 / 165, 14 of 250 247 / 220, 16 of 500 342 / 333; 32 heads on 8, 48 of 100 to 500
+// 287 / 289, of 500 373 / 337, 40 of 700 445 / 394, 36 of 100 to 700 301 / 315).
+// Groups of 3 and 4: 2 tiles 572 -> 487 (96 of 1000), 3 635 -> 587, 4 748 -> 715, 802 -> 743, one
 // 693 -> 697; 5 730 -> 799, 921 -> 1027.  Smaller groups: 2 tiles 588 -> 551 (64 of 2000), 675 -> 533; 3 to 6 where the
 // workgroups are seven eighths of the compute units with ranges 85 % full, or three quarters and whole columns (32 heads, 12
 // captured layers, or 28 eager ones): 6 sequences of 800 288 -> 234, 1 of 8000 445 -> 374, 2 of 5000 413 -> 393, 8 of 1300
@@ -1132,8 +1170,7 @@ static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_h
     return 0;
   const int chunk = DC_WAVES * DA_TILE;
   if (cols * ((k->max_seq_len + chunk - 1) / chunk) <= slots) return chunk;
-  if (cols <= (G > 2 ? 2 : 1) * slots && k->max_seq_len <= DC_ONE) return DC_ONE;
-  if (cols <= 2 * slots && k->max_seq_len <= chunk) return chunk;
+  if (cols <= (G > 4 ? 2 : 1) * slots && k->max_seq_len <= DC_ONE) return DC_ONE;
   const int most = G > 4 ? DC_TILES_MANY : G > 2 ? DC_TILES_SOME : DC_TILES_FEW;
   for (int m = 2; m <= most; ++m) {
     const long long ranges = (k->max_seq_len + m * chunk - 1) / (m * chunk), wgs = cols * ranges;
@@ -1142,6 +1179,51 @@ static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_h
     return G > 2 || m == 2 || full ? m * chunk : 0;
   }
   return 0;
+}
+
+// the smallest tile that holds the whole group (padded head rows cost nothing; splitting a group would
+// read its K and V once per tile); groups of more than 8 heads are served 8 at a time
+static int da_group_tile(int G) { return G > 4 ? 8 : G > 2 ? 4 : G > 1 ? 2 : 1; }
+
+// Tokens per workgroup: the multiple of 32 between 256 and 1024 that minimises rounds * (chunk + fixed part),
+// rounds = workgroups / (two per compute unit), rounded up.  Longer chunks spend less of a workgroup's life on
+// its ramp (first tiles in flight, nothing to compute yet) and its tail (statistics, partial results, no loads
+// in flight); a launch of few workgroups wants the chunk that fills whole rounds.  Measured: cfg4 (2880
+// columns, up to 2304 tokens) 0.327 ms per layer with 256, 0.297 with 512, 0.294 with 768; cfg5's decode (64
+// columns, 3584 tokens) 33.3 us with 256, 30.4 with 448.  Two workgroups must still fit a compute unit's LDS, which
+// caps the chunk for groups of 8 query heads.  Only the view's max_seq_len enters, never the lengths on the
+// device, so the choice is the same at capture and at every replay.
+static int da_split_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
+  const int G = num_q_heads / k->num_kv_heads, gt = da_group_tile(G);
+  const int slots = 2 * fc_compute_units();
+  const long long cols = (long long)k->num_kv_heads * ((G + gt - 1) / gt) * k->batch;
+  const auto fits = [&](int cand) { return (DA_RING + gt * cand * 4) * 2 <= 158 * 1024; };
+  int chunk = DA_CHUNK;
+  double best = -1.0;
+  for (int cand = DA_CHUNK; cand <= DA_CHUNK_MAX && fits(cand); cand += DA_TILE) {
+    const long long wgs = cols * ((k->max_seq_len + cand - 1) / cand);
+    const double cost = (double)((wgs + slots - 1) / slots) * (cand + 96.0);
+    if (best < 0 || cost < best - 1e-9) {
+      best = cost;
+      chunk = cand;
+    }
+  }
+  // Whole columns need no merge and append by themselves, two launches and 4 us a layer less, and long workgroups of different
+  // lengths even out where chunks come in rounds: 300 tokens of a round; workgroups past the first round cost their share of one.
+  // us per step, 12 captured layers, chunks -> whole: 32 heads, 20 sequences of 100 to 300 tokens 319 -> 272, of 500 546 -> 494,
+  // of 100 to 700 480 -> 413, of 100 to 1000 555 -> 417, of 1000 870 -> 829, 10 of 750 422 -> 371, 9 of 1000 472 -> 451, 60 of 100 to
+  // 500 800 -> 742, 90 of 500 1729 -> 1686; 32 on 16, 20 of 100 to 700 341 -> 272, 40 499 -> 448; 32 on 8, 90 of 128 to 500
+  // 579 -> 471, of 700 807 -> 723.  Fewer columns: 7 of 1000 328 -> 329, 5 of 100 to 900 247 -> 256.
+  const int whole = (k->max_seq_len + DA_TILE - 1) / DA_TILE * DA_TILE;
+  if (whole >= DA_CHUNK && whole <= DA_CHUNK_MAX && fits(whole) && da_tile_in_page(k) && da_tile_in_page(v) &&
+      fmax(1.0, (double)cols / slots) * (whole + 96.0) - 300.0 < best)
+    return whole;
+  return chunk;
+}
+
+// One workgroup a column of the split kernel: no merge, and where it may append (its kv head's rows, one table) one launch a layer.
+static bool da_split_whole(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
+  return k->max_seq_len > 0 && k->max_seq_len <= da_split_chunk(k, v, num_q_heads) && da_tile_in_page(k) && da_tile_in_page(v);
 }
 
 static int da_merge(const char* who, const fc_kv_view* k_cache, const float* part_o, const float* part_ml,
@@ -1222,33 +1304,8 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
   FC_REQUIRE(workspace_bytes >= need, FC_EINVAL, "%s: workspace of %lld bytes, %lld needed", who,
              (long long)workspace_bytes, (long long)need);
   const int B = k_cache->batch, Hkv = k_cache->num_kv_heads, G = num_q_heads / Hkv;
-  // the smallest tile that holds the whole group (padded head rows cost nothing; splitting a group would
-  // read its K and V once per tile); groups of more than 8 heads are served 8 at a time
-  const int gt = G > 4 ? 8 : G > 2 ? 4 : G > 1 ? 2 : 1;
-  const int gtiles = (G + gt - 1) / gt;
-  // Tokens per workgroup: the multiple of 32 between 256 and 1024 that minimises rounds * (chunk + fixed part),
-  // rounds = workgroups / (two per compute unit), rounded up.  Longer chunks spend less of a workgroup's life on
-  // its ramp (first tiles in flight, nothing to compute yet) and its tail (statistics, partial results, no loads
-  // in flight); a launch of few workgroups wants the chunk that fills whole rounds.  Measured: cfg4 (2880
-  // columns, up to 2304 tokens) 0.327 ms per layer with 256, 0.297 with 512, 0.294 with 768; cfg5's decode (64
-  // columns, 3584 tokens) 33.3 us with 256, 30.4 with 448.  Two workgroups must still fit a compute unit's LDS, which
-  // caps the chunk for groups of 8 query heads.  Only the view's max_seq_len enters, never the lengths on the
-  // device, so the choice is the same at capture and at every replay.
-  int chunk = DA_CHUNK;
-  {
-    const int slots = 2 * fc_compute_units();
-    const long long cols = (long long)Hkv * gtiles * B;
-    double best = -1.0;
-    for (int cand = DA_CHUNK; cand <= DA_CHUNK_MAX; cand += DA_TILE) {
-      if ((DA_RING + gt * cand * 4) * 2 > 158 * 1024) break;
-      const long long wgs = cols * ((k_cache->max_seq_len + cand - 1) / cand);
-      const double cost = (double)((wgs + slots - 1) / slots) * (cand + 96.0);
-      if (best < 0 || cost < best - 1e-9) {
-        best = cost;
-        chunk = cand;
-      }
-    }
-  }
+  const int gt = da_group_tile(G), gtiles = (G + gt - 1) / gt;
+  const int chunk = da_split_chunk(k_cache, v_cache, num_q_heads);
   const int splits = (k_cache->max_seq_len + chunk - 1) / chunk;
   float* part_o = (float*)workspace;
   float* part_ml = part_o + (int64_t)B * num_q_heads * (splits > 0 ? splits : 1) * FC_HEAD_DIM;
@@ -1259,27 +1316,29 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
   if (splits > 0) {
     FC_REQUIRE(Hkv * gtiles <= 65535 && B <= 65535, FC_EUNSUPPORTED, "%s: grid too large", who);
     dim3 grid(splits, Hkv * gtiles, B);
-    const bool fast = da_tile_in_page(k_cache) && da_tile_in_page(v_cache);
-#define DA_LAUNCH(DT, GTV, FA)                                                                                   \
+    const bool fast = da_tile_in_page(k_cache) && da_tile_in_page(v_cache), whole = da_split_whole(k_cache, v_cache, num_q_heads);
+    const DaAppend ap = append ? *append : DaAppend{nullptr, nullptr, 0, 0, nullptr};
+#define DA_LAUNCH(DT, GTV, FA, WH)                                                                                   \
   do {                                                                                                          \
-    FC_ALLOW_LDS((decode_attn_kernel<DT, GTV, FA>), DaCfg<GTV>::lds(DA_CHUNK_MAX));                             \
-    hipLaunchKernelGGL((decode_attn_kernel<DT, GTV, FA>), grid, dim3(DA_THREADS), DaCfg<GTV>::lds(chunk), st, k, \
-                       v, layer, (const char*)q, num_q_heads, context_lens, c, part_o, part_ml, splits, chunk); \
+    FC_ALLOW_LDS((decode_attn_kernel<DT, GTV, FA, WH>), DaCfg<GTV>::lds(DA_CHUNK_MAX));                             \
+    hipLaunchKernelGGL((decode_attn_kernel<DT, GTV, FA, WH>), grid, dim3(DA_THREADS), DaCfg<GTV>::lds(chunk), st, k, \
+                       v, layer, (const char*)q, num_q_heads, context_lens, c, part_o, part_ml, splits, chunk, (char*)out, ap); \
   } while (0)
-#define DA_DISPATCH2(DT, FA)                        \
+#define DA_DISPATCH2(DT, FA, WH)                    \
   switch (gt) {                                     \
-    case 8: DA_LAUNCH(DT, 8, FA); break;            \
-    case 4: DA_LAUNCH(DT, 4, FA); break;            \
-    case 2: DA_LAUNCH(DT, 2, FA); break;            \
-    default: DA_LAUNCH(DT, 1, FA); break;           \
+    case 8: DA_LAUNCH(DT, 8, FA, WH); break;        \
+    case 4: DA_LAUNCH(DT, 4, FA, WH); break;        \
+    case 2: DA_LAUNCH(DT, 2, FA, WH); break;        \
+    default: DA_LAUNCH(DT, 1, FA, WH); break;       \
   }
 #define DA_DISPATCH(DT) \
-  if (fast) { DA_DISPATCH2(DT, true) } else { DA_DISPATCH2(DT, false) }
+  if (whole) { DA_DISPATCH2(DT, true, true) } else if (fast) { DA_DISPATCH2(DT, true, false) } else { DA_DISPATCH2(DT, false, false) }
     if (bf) { DA_DISPATCH(FC_BF16) } else { DA_DISPATCH(FC_F16) }
 #undef DA_DISPATCH
 #undef DA_DISPATCH2
 #undef DA_LAUNCH
     FC_CHECK_LAUNCH(who);
+    if (whole) return FC_OK;
   }
   return da_merge(who, k_cache, part_o, part_ml, context_lens, num_q_heads, splits, chunk, 0, out, stream);
 }
@@ -1292,11 +1351,12 @@ extern "C" int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cac
 }
 
 // Append and attention of one layer.  The workgroup of a column appends its own head's row, so the fused form needs
-// one workgroup per kv head (groups of up to 16 query heads) and both caches on one block table; otherwise the rows
+// one workgroup per kv head (groups of up to 16 query heads, 8 for whole columns of the split kernel) and both caches on one block table; otherwise the rows
 // go in first, in a launch of their own.
 static bool da_appends_inside(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
   return num_q_heads / k->num_kv_heads <= DC_HEADS && k->block_tables && k->block_tables == v->block_tables &&
-         k->table_stride == v->table_stride && k->block_size == v->block_size && da_column_chunk(k, v, num_q_heads) > 0;
+         k->table_stride == v->table_stride && k->block_size == v->block_size &&
+         (da_column_chunk(k, v, num_q_heads) > 0 || (num_q_heads / k->num_kv_heads <= 8 && da_split_whole(k, v, num_q_heads)));
 }
 
 extern "C" int64_t fc_decode_layer_workspace_bytes(const fc_kv_view* k_cache, const fc_kv_view* v_cache,
