@@ -83,9 +83,9 @@ struct DaAppend {                 // the step's new rows, one per sequence (k_ne
 // it back (true is returned), whichever sequence of the batch it belongs to (a table may be listed twice with lengths one
 // apart, or a page be shared): nobody depends on another workgroup's write.  The sequence's own row is also written by its last
 // workgroup, since it usually lies right behind the range.  Workgroups that write one row write the same bytes.
-// slot: of sequence `lane` (negative: none), ktbl: table entry `lane` of sequence b; both planes use one table.
+// slot: of sequence `lane` (negative: none), ktbl: table entry tbl0 + `lane` of sequence b; both planes use one table.
 __device__ __forceinline__ bool da_append_rows(const KvView& kc, const KvView& vc, const DaAppend& ap, const char* kbase,
-                                               const char* vbase, int slot, int ktbl, int b, int h, int nb, int t0, int end,
+                                               const char* vbase, int slot, int ktbl, int tbl0, int b, int h, int nb, int t0, int end,
                                                int len, int tid) {
   const int lane = tid & 63, l15 = tid & 15;
   const int e0 = t0 >> kc.block_shift, e1 = (end - 1) >> kc.block_shift;      // pages of the range (none: e1 < e0)
@@ -96,7 +96,7 @@ __device__ __forceinline__ bool da_append_rows(const KvView& kc, const KvView& v
     bool hit = false;
     for (int e = e0; e <= e1; ++e) {
       const int pos = (e << kc.block_shift) + at;
-      hit |= slot >= 0 && page == __builtin_amdgcn_readlane(ktbl, e) && pos >= t0 && pos < end;
+      hit |= slot >= 0 && page == __builtin_amdgcn_readlane(ktbl, e - tbl0) && pos >= t0 && pos < end;
     }
     unsigned long long todo = __ballot(hit);
     inside |= todo != 0ull;
@@ -129,8 +129,8 @@ __device__ __forceinline__ bool da_append_rows(const KvView& kc, const KvView& v
 // Logits are one v_mfma_f32_32x32x16 block per tile with the query heads as rows (padded with zero
 // rows to 32): whatever the group size, K is read from LDS once.
 // WHOLE: the chunk holds every sequence: the workgroup writes the output (as the merge of one chunk would) and, asked to
-// (one kv head a workgroup, one table for both planes), appends the step's rows.
-template <int DTYPE, int GT, bool FAST, bool WHOLE>
+// (one kv head a workgroup, one table for both planes), appends the step's rows.  APPEND: several chunks do as well, FAST.
+template <int DTYPE, int GT, bool FAST, bool WHOLE, bool APPEND>
 __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, KvView vc, int layer,
                                                                     const char* __restrict__ q, int Hq,
                                                                     const int* __restrict__ lens, float c,
@@ -178,7 +178,8 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   if constexpr (WHOLE) {
     if (ap.k_new && lane < nb) slot = ap.slots[lane];
   }
-  if (!WHOLE && t0 >= len) return;
+  if constexpr (APPEND) slot = lane < nb ? ap.slots[lane] : -1;
+  if (!WHOLE && t0 >= len && (!APPEND || split != 0)) return;
   const int ntok = min(chunk, len - t0);
 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   const char* vbase = vc.base + ((long long)layer * vc.stride_layer + (long long)h * vc.stride_head) * 2;
   if constexpr (WHOLE) {
     len = max(len, 0);
-    if (ap.k_new && da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, b, h, nb, 0, len, len, tid)) {
+    if (ap.k_new && da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, 0, b, h, nb, 0, len, len, tid)) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     }
@@ -207,6 +208,14 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
       for (int i = tid; i < min(GT, G - g0) * FC_HEAD_DIM; i += DA_THREADS) orow[i] = 0;
       return;
     }
+  }
+  if constexpr (APPEND) {
+    len = max(len, 0);
+    if (da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, t0 >> kc.block_shift, b, h, nb, t0, min(len, t0 + chunk), len, tid)) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
+    if (len == 0) return;                  // the merge writes the zeros
   }
   const unsigned ring_lds = __builtin_amdgcn_readfirstlane(fc_lds_addr(smem)) + wave * (2 * DA_TILEB);
   char* ring = smem + wave * (2 * DA_TILEB);
@@ -640,7 +649,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   const char* kbase = kc.base + ((long long)layer * kc.stride_layer + (long long)h * kc.stride_head) * 2;
   const char* vbase = vc.base + ((long long)layer * vc.stride_layer + (long long)h * vc.stride_head) * 2;
   if (PAGED && ap.k_new) {
-    if (da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, b, h, nb, t0, end, len, tid)) {
+    if (da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, 0, b, h, nb, t0, end, len, tid)) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     }
@@ -1318,21 +1327,25 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
     dim3 grid(splits, Hkv * gtiles, B);
     const bool fast = da_tile_in_page(k_cache) && da_tile_in_page(v_cache), whole = da_split_whole(k_cache, v_cache, num_q_heads);
     const DaAppend ap = append ? *append : DaAppend{nullptr, nullptr, 0, 0, nullptr};
-#define DA_LAUNCH(DT, GTV, FA, WH)                                                                                   \
+#define DA_LAUNCH(DT, GTV, FA, WH, AP)                                                                                   \
   do {                                                                                                          \
-    FC_ALLOW_LDS((decode_attn_kernel<DT, GTV, FA, WH>), DaCfg<GTV>::lds(DA_CHUNK_MAX));                             \
-    hipLaunchKernelGGL((decode_attn_kernel<DT, GTV, FA, WH>), grid, dim3(DA_THREADS), DaCfg<GTV>::lds(chunk), st, k, \
+    FC_ALLOW_LDS((decode_attn_kernel<DT, GTV, FA, WH, AP>), DaCfg<GTV>::lds(DA_CHUNK_MAX));                             \
+    hipLaunchKernelGGL((decode_attn_kernel<DT, GTV, FA, WH, AP>), grid, dim3(DA_THREADS), DaCfg<GTV>::lds(chunk), st, k, \
                        v, layer, (const char*)q, num_q_heads, context_lens, c, part_o, part_ml, splits, chunk, (char*)out, ap); \
   } while (0)
-#define DA_DISPATCH2(DT, FA, WH)                    \
-  switch (gt) {                                     \
-    case 8: DA_LAUNCH(DT, 8, FA, WH); break;        \
-    case 4: DA_LAUNCH(DT, 4, FA, WH); break;        \
-    case 2: DA_LAUNCH(DT, 2, FA, WH); break;        \
-    default: DA_LAUNCH(DT, 1, FA, WH); break;       \
+#define DA_DISPATCH2(DT, FA, WH)                     \
+  switch (gt) {                                      \
+    case 8: DA_LAUNCH(DT, 8, FA, WH, false); break;  \
+    case 4: DA_LAUNCH(DT, 4, FA, WH, false); break;  \
+    case 2: DA_LAUNCH(DT, 2, FA, WH, false); break;  \
+    default: DA_LAUNCH(DT, 1, FA, WH, false); break; \
   }
-#define DA_DISPATCH(DT) \
-  if (whole) { DA_DISPATCH2(DT, true, true) } else if (fast) { DA_DISPATCH2(DT, true, false) } else { DA_DISPATCH2(DT, false, false) }
+#define DA_DISPATCH(DT)                                                                                  \
+  if (whole) { DA_DISPATCH2(DT, true, true) } else if (!fast) { DA_DISPATCH2(DT, false, false) }         \
+  else if (!ap.k_new) { DA_DISPATCH2(DT, true, false) }                                                  \
+  else if (gt == 4) DA_LAUNCH(DT, 4, true, false, true);      /* (da_split_appends: up to 4 heads) */   \
+  else if (gt == 2) DA_LAUNCH(DT, 2, true, false, true);                                                 \
+  else DA_LAUNCH(DT, 1, true, false, true);
     if (bf) { DA_DISPATCH(FC_BF16) } else { DA_DISPATCH(FC_F16) }
 #undef DA_DISPATCH
 #undef DA_DISPATCH2
@@ -1350,13 +1363,22 @@ extern "C" int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cac
                     workspace_bytes, stream);
 }
 
+// The split kernel's workgroups append where one serves a kv head: whole columns, and chunks of groups of up to 4 heads.  us per
+// step, 12 captured layers, a launch of its own -> inside: 32 heads, 4 sequences of 600 to 6000 tokens 762 -> 750, 8 of 200 to
+// 2000 502 -> 482, 20 of 300 to 2500 1090 -> 1059; 32 on 8, 30 of 400 to 4000 734 -> 706, 60 of 300 to 3000 1105 -> 1076; 90
+// sequences, whose slots are two loads a workgroup, the same; chunks of 7 heads a group lose (90 of 100 to 1000 541 -> 550).
+static bool da_split_appends(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
+  const int G = num_q_heads / k->num_kv_heads;
+  return G <= 8 && da_tile_in_page(k) && da_tile_in_page(v) && (G <= 4 || da_split_whole(k, v, num_q_heads));
+}
+
 // Append and attention of one layer.  The workgroup of a column appends its own head's row, so the fused form needs
 // one workgroup per kv head (groups of up to 16 query heads, 8 for whole columns of the split kernel) and both caches on one block table; otherwise the rows
 // go in first, in a launch of their own.
 static bool da_appends_inside(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
   return num_q_heads / k->num_kv_heads <= DC_HEADS && k->block_tables && k->block_tables == v->block_tables &&
          k->table_stride == v->table_stride && k->block_size == v->block_size &&
-         (da_column_chunk(k, v, num_q_heads) > 0 || (num_q_heads / k->num_kv_heads <= 8 && da_split_whole(k, v, num_q_heads)));
+         k->max_seq_len > 0 && (da_column_chunk(k, v, num_q_heads) > 0 || da_split_appends(k, v, num_q_heads));
 }
 
 extern "C" int64_t fc_decode_layer_workspace_bytes(const fc_kv_view* k_cache, const fc_kv_view* v_cache,
