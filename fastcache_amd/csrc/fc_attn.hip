@@ -83,15 +83,17 @@ struct DaAppend {                 // the step's new rows, one per sequence (k_ne
 // it back (true is returned), whichever sequence of the batch it belongs to (a table may be listed twice with lengths one
 // apart, or a page be shared): nobody depends on another workgroup's write.  The sequence's own row is also written by its last
 // workgroup, since it usually lies right behind the range.  Workgroups that write one row write the same bytes.
-// slot: of sequence `lane` (negative: none), ktbl: table entry tbl0 + `lane` of sequence b; both planes use one table.
+// slot: of sequence `lane` (negative: none), TWO: slot2 of sequence 64 + `lane`, asked for with it, ktbl: table entry tbl0 + `lane` of sequence b; both planes use one table.
+template <bool TWO>
 __device__ __forceinline__ bool da_append_rows(const KvView& kc, const KvView& vc, const DaAppend& ap, const char* kbase,
-                                               const char* vbase, int slot, int ktbl, int tbl0, int b, int h, int nb, int t0, int end,
+                                               const char* vbase, int slot, int slot2, int ktbl, int tbl0, int b, int h, int nb, int t0, int end,
                                                int len, int tid) {
   const int lane = tid & 63, l15 = tid & 15;
   const int e0 = t0 >> kc.block_shift, e1 = (end - 1) >> kc.block_shift;      // pages of the range (none: e1 < e0)
   bool inside = false;
   for (int j0 = 0; j0 < nb; j0 += FC_WAVE) {
-    if (j0 > 0) slot = j0 + lane < nb ? ap.slots[j0 + lane] : -1;
+    if (TWO && j0 == FC_WAVE) slot = slot2;
+    else if (j0 > 0) slot = j0 + lane < nb ? ap.slots[j0 + lane] : -1;
     const int page = slot >> kc.block_shift, at = slot & (kc.block_size - 1);
     bool hit = false;
     for (int e = e0; e <= e1; ++e) {
@@ -178,7 +180,11 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   if constexpr (WHOLE) {
     if (ap.k_new && lane < nb) slot = ap.slots[lane];
   }
-  if constexpr (APPEND) slot = lane < nb ? ap.slots[lane] : -1;
+  int slot2 = -1;
+  if constexpr (APPEND) {
+    slot = lane < nb ? ap.slots[lane] : -1;
+    if (FC_WAVE + lane < nb) slot2 = ap.slots[FC_WAVE + lane];
+  }
   if (!WHOLE && t0 >= len && (!APPEND || split != 0)) return;
   const int ntok = min(chunk, len - t0);
 
@@ -199,7 +205,7 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   const char* vbase = vc.base + ((long long)layer * vc.stride_layer + (long long)h * vc.stride_head) * 2;
   if constexpr (WHOLE) {
     len = max(len, 0);
-    if (ap.k_new && da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, 0, b, h, nb, 0, len, len, tid)) {
+    if (ap.k_new && da_append_rows<false>(kc, vc, ap, kbase, vbase, slot, -1, ktbl, 0, b, h, nb, 0, len, len, tid)) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     }
@@ -211,7 +217,7 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   }
   if constexpr (APPEND) {
     len = max(len, 0);
-    if (da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, t0 >> kc.block_shift, b, h, nb, t0, min(len, t0 + chunk), len, tid)) {
+    if (da_append_rows<true>(kc, vc, ap, kbase, vbase, slot, slot2, ktbl, t0 >> kc.block_shift, b, h, nb, t0, min(len, t0 + chunk), len, tid)) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     }
@@ -649,7 +655,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   const char* kbase = kc.base + ((long long)layer * kc.stride_layer + (long long)h * kc.stride_head) * 2;
   const char* vbase = vc.base + ((long long)layer * vc.stride_layer + (long long)h * vc.stride_head) * 2;
   if (PAGED && ap.k_new) {
-    if (da_append_rows(kc, vc, ap, kbase, vbase, slot, ktbl, 0, b, h, nb, t0, end, len, tid)) {
+    if (da_append_rows<false>(kc, vc, ap, kbase, vbase, slot, -1, ktbl, 0, b, h, nb, t0, end, len, tid)) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     }
@@ -1365,8 +1371,9 @@ extern "C" int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cac
 
 // The split kernel's workgroups append where one serves a kv head: whole columns, and chunks of groups of up to 4 heads.  us per
 // step, 12 captured layers, a launch of its own -> inside: 32 heads, 4 sequences of 600 to 6000 tokens 762 -> 750, 8 of 200 to
-// 2000 502 -> 482, 20 of 300 to 2500 1090 -> 1059; 32 on 8, 30 of 400 to 4000 734 -> 706, 60 of 300 to 3000 1105 -> 1076; 90
-// sequences, whose slots are two loads a workgroup, the same; chunks of 7 heads a group lose (90 of 100 to 1000 541 -> 550).
+// 2000 502 -> 482, 20 of 300 to 2500 1090 -> 1059; 32 on 8, 30 of 400 to 4000 734 -> 706, 60 of 300 to 3000 1105 -> 1076, 90
+// of 100 to 1200 863 -> 842 (861 where the slots past the first 64 were asked for in their turn); chunks of 7 heads a group
+// lose (90 of 100 to 1000 541 -> 550).
 static bool da_split_appends(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
   const int G = num_q_heads / k->num_kv_heads;
   return G <= 8 && da_tile_in_page(k) && da_tile_in_page(v) && (G <= 4 || da_split_whole(k, v, num_q_heads));
