@@ -808,7 +808,10 @@ static int ml_uniform(const char* who, const fc_kv_view* const src[2], const fc_
   if (c > 0 && (rc = ml_launch(who, src[0], dst[0], a, planes, cf, seg_start, c, dst_start, nullptr, nullptr, nullptr, 0,
                                (hipStream_t)stream)))
     return rc;
-  if (rem > 0 && planes == 1) return fc_copy_tokens(src[0], dst[0], seg_start + c * cf, rem, dst_start + c, stream);
+  if (rem > 0 && (planes == 1 || src[0]->batch > 65535)) {     // (more sequences than the tails' grid takes)
+    for (int p = 0; p < planes && !rc; ++p) rc = fc_copy_tokens(src[p], dst[p], seg_start + c * cf, rem, dst_start + c, stream);
+    return rc;
+  }
   if (rem > 0) ml_tails(src, dst, a, planes, cf, 0, c, nullptr, nullptr, nullptr, seg_start, seg_len, dst_start, (hipStream_t)stream);
   FC_CHECK_LAUNCH(who);
   return FC_OK;
