@@ -1373,10 +1373,11 @@ extern "C" int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cac
 // step, 12 captured layers, a launch of its own -> inside: 32 heads, 4 sequences of 600 to 6000 tokens 762 -> 750, 8 of 200 to
 // 2000 502 -> 482, 20 of 300 to 2500 1090 -> 1059; 32 on 8, 30 of 400 to 4000 734 -> 706, 60 of 300 to 3000 1105 -> 1076, 90
 // of 100 to 1200 863 -> 842 (861 where the slots past the first 64 were asked for in their turn); chunks of 7 heads a group
-// lose (90 of 100 to 1000 541 -> 550).
+// lose (90 of 100 to 1000 541 -> 550).  Every workgroup looks at the slots of the whole batch: above 128 sequences that costs
+// more than the launch (6 layers: 256 of 60 to 250 inside 1044, apart 911; 200 of 100 to 250 880, 779; 128 of 60 to 120 405, 406).
 static bool da_split_appends(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
   const int G = num_q_heads / k->num_kv_heads;
-  return G <= 8 && da_tile_in_page(k) && da_tile_in_page(v) && (G <= 4 || da_split_whole(k, v, num_q_heads));
+  return k->batch <= 2 * FC_WAVE && G <= 8 && da_tile_in_page(k) && da_tile_in_page(v) && (G <= 4 || da_split_whole(k, v, num_q_heads));
 }
 
 // Append and attention of one layer.  The workgroup of a column appends its own head's row, so the fused form needs

@@ -643,10 +643,10 @@ def test_sequences_that_reach_a_little_into_a_second_range(dev, dtype, Hq, Hkv, 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("Hq,Hkv,B,most,launches", [
-    (32, 32, 9, 256, 1), (32, 32, 17, 512, 1), (32, 32, 10, 768, 1), (32, 32, 17, 1024, 1), (32, 32, 9, 1025, 2), (32, 16, 70, 1025, 2), (4, 2, 130, 1100, 2),
+    (32, 32, 9, 256, 1), (32, 32, 17, 512, 1), (32, 32, 10, 768, 1), (32, 32, 17, 1024, 1), (32, 32, 9, 1025, 2), (32, 16, 70, 1025, 2), (6, 3, 128, 1300, 2), (6, 3, 129, 1300, 3),
     (32, 16, 33, 256, 1), (32, 16, 40, 900, 1),
     (32, 8, 64, 512, 1), (24, 8, 65, 768, 1), (32, 8, 33, 1024, 2),             # of 1024 tokens two workgroups do not fit
-    (28, 4, 66, 768, 1), (32, 4, 129, 256, 1), (32, 4, 129, 512, 3), (40, 4, 129, 256, 2)])      # 10 heads a group: two workgroups, which do not append
+    (28, 4, 66, 768, 1), (32, 4, 129, 256, 2), (16, 8, 128, 256, 1), (32, 4, 129, 512, 3), (40, 4, 129, 256, 2)])      # 10 heads a group: two workgroups, which do not append
 def test_more_columns_than_compute_units(dev, dtype, Hq, Hkv, B, most, launches):
     """Columns held whole by one workgroup each, which append the step's rows and write the output, or chunks that append (of up
     to 4 heads a group) and a merge: the launches of a layer, the caches' bytes and the oracle's values, an empty sequence among them, a row that belongs to no
