@@ -591,22 +591,25 @@ PyObject* py_stage_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
 // ---- a step's numbers to the device -----------------------------------------------------------------------------------------
 // Up to FC_UPLOAD_MAX bytes travel as a kernel's arguments, more (and what a stream under capture is given, which the
-// callers refuse or torch does) as a copy from pinned memory.
+// callers refuse or torch does, and what is not for a GPU) as a copy from pinned memory.
 struct Packed {
   at::Tensor host, dev;
   std::vector<char> small;
   int64_t at = 0;
-  c10::hip::HIPStream stream;
+  void* stream = nullptr;      // of `small`
   Packed(int64_t bytes, const c10::Device& device)
-      : dev(at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(device))),
-        stream(c10::hip::getCurrentHIPStream(device.index())) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool known = hipStreamIsCapturing(stream.stream(), &capture) == hipSuccess;
-    if (!known) (void)hipGetLastError();
-    if (known && capture == hipStreamCaptureStatusNone && bytes <= FC_UPLOAD_MAX && bytes % 4 == 0)
-      small.resize(std::max<int64_t>(bytes, 1));
-    else
-      host = at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+      : dev(at::empty({bytes}, at::TensorOptions().dtype(at::kByte).device(device))) {
+    if (device.is_cuda() && bytes <= FC_UPLOAD_MAX && bytes % 4 == 0) {
+      const hipStream_t st = c10::hip::getCurrentHIPStream(device.index()).stream();
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(st, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+      } else if (capture == hipStreamCaptureStatusNone) {
+        small.resize(std::max<int64_t>(bytes, 1));
+        stream = (void*)st;
+      }
+    }
+    if (small.empty()) host = at::empty({bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
   }
   template <typename T>
   T* take(int64_t n) {
@@ -619,7 +622,7 @@ struct Packed {
       dev.copy_(host, true);
     } else if (dev.numel() > 0) {
       const c10::DeviceGuard guard(dev.device());
-      check(fc_upload(dev.data_ptr(), small.data(), (int32_t)dev.numel(), (void*)stream.stream()), "fc_upload");
+      check(fc_upload(dev.data_ptr(), small.data(), (int32_t)dev.numel(), stream), "fc_upload");
     }
   }
   at::Tensor part(int64_t byte, int64_t n, at::ScalarType t) { return dev.narrow(0, byte, n * (int64_t)c10::elementSize(t)).view(t); }

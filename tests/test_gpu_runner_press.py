@@ -11,6 +11,7 @@ from fastcache_amd.engine.kv_runner import PagedKVRunner
 from fastcache_amd.kernels import KVPressCompressor
 from fastcache_amd.presses import (ExpectedAttentionPress, KnormPress, ObservedAttentionPress, RandomPress,
                                    SimLayerKVPress, SnapKVPress, StreamingLLMPress, ThinKPress, TOVAPress)
+from fastcache_amd.utils.context import get_context, reset_context
 from oracle import paged as opaged
 from oracle import pipeline as opipe
 from oracle import presses as opress
@@ -465,3 +466,20 @@ def test_uploaded_tables_and_lengths(dev, rows, width):
     torch.cuda.synchronize()
     n = min(768, rows * width)
     assert torch.equal(buf[:n].cpu(), src[:n]) and bool((buf[n:] == -1).all())
+
+
+def test_numbers_for_a_pool_on_the_host(dev):
+    """A runner whose pool lies in host memory gets its tables and decode inputs there, by a copy: no kernel writes them."""
+    runner = PagedKVRunner(1, 1, 128, num_blocks=4, dtype=torch.float16, device="cpu", image_token_len=0)
+    a, b = Sequence(list(range(300))), Sequence(list(range(40, 47)))
+    a.block_table, b.block_table = [2, 1], [3]
+    ids, positions = runner.prepare_decode([a, b])
+    try:
+        ctx = get_context()
+        torch.cuda.synchronize()
+        assert all(t.device.type == "cpu" for t in (ids, positions, ctx.slot_mapping, ctx.context_lens, ctx.block_tables))
+        assert ids.tolist() == [299, 46] and ctx.block_tables.tolist() == [[2, 1], [3, -1]]
+        assert positions.tolist() == ctx.context_lens.tolist() == [a.kv_cache_len, b.kv_cache_len]
+        assert runner.preare_block_tables([b, a]).tolist() == [[3, -1], [2, 1]]
+    finally:
+        reset_context()
