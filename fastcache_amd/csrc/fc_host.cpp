@@ -452,7 +452,8 @@ int decode_turn(const at::Tensor& t, const c10::hip::HIPStream& stream) {
 // ---- one attention layer of a decode step ---------------------------------------------------------------------------------
 // decode_layer(q, k, v, k_cache, v_cache, slot_mapping, context_lens, block_tables, scale, q_heads, kv_heads, head_dim,
 //              workspace or None, out or None, arrivals or None) -> out [n, q_heads * head_dim], or None when the arguments
-// are not the plain decode step (the caller's general path then serves or refuses them).  arrivals: FC_DECODE_ARRIVALS zeros.
+// are not the plain decode step (the caller's general path then serves or refuses them).  arrivals: FC_DECODE_ARRIVALS zeros,
+// counted on only beside the workspace they come with: a launch whose partial results lie elsewhere may run beside theirs.
 PyObject* py_decode_layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return guarded([&]() -> PyObject* {
     need_args(nargs, 15, "decode_layer");
@@ -508,11 +509,12 @@ PyObject* py_decode_layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::Tensor ws;
     void* wsp = nullptr;
     int64_t ws_bytes = 0;
+    bool callers = false;        // the workspace is
     if (need > 0) {
       if (args[12] != Py_None) ws = tensor(args[12], "workspace");
+      callers = ws.defined() && ws.device() == dev && ws.scalar_type() == at::kByte && ws.is_contiguous() && ws.numel() >= need;
       // the allocator hands blocks out per stream, so a workspace of this call is safe with any number of them
-      if (!ws.defined() || ws.device() != dev || ws.scalar_type() != at::kByte || !ws.is_contiguous() || ws.numel() < need)
-        ws = at::empty({need}, q.options().dtype(at::kByte));
+      if (!callers) ws = at::empty({need}, q.options().dtype(at::kByte));
       wsp = ws.data_ptr();
       ws_bytes = ws.numel();
     }
@@ -528,13 +530,13 @@ PyObject* py_decode_layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(q.get_device());
     const int32_t *sp = (const int32_t*)slots.const_data_ptr(), *lp = (const int32_t*)lens.const_data_ptr();
-    if (args[14] != Py_None) {
+    if (callers && args[14] != Py_None) {
       const at::Tensor& arr = tensor(args[14], "arrivals");
       if (arr.device() != dev || arr.scalar_type() != at::kInt || !arr.is_contiguous() || arr.numel() < FC_DECODE_ARRIVALS)
         fail("decode_layer: arrivals must be contiguous int32 words on the device of q");
       check(fc_decode_layer_arrivals(&kv, &vv, q.const_data_ptr(), k.const_data_ptr(), stride[0], v.const_data_ptr(), stride[1], sp,
                                      out.data_ptr(), (int32_t)hq, lp, (float)scale, wsp, ws_bytes,
-                                     ws_bytes ? (uint32_t*)arr.data_ptr() : nullptr, (void*)stream.stream()),
+                                     (uint32_t*)arr.data_ptr(), (void*)stream.stream()),
             "fc_decode_layer");
     } else {
       check(fc_decode_layer_turn(&kv, &vv, q.const_data_ptr(), k.const_data_ptr(), stride[0], v.const_data_ptr(), stride[1], sp,

@@ -101,7 +101,13 @@ class BucketedDecodeGraphs:
         # heads on 4, 9 sequences of 100 to 248 tokens)
         for i, layer in enumerate(self.layers):
             to = out[i]
-            o = layer(q[i], k[i], v[i], out=to) if getattr(layer.forward, "__func__", None) is Attention.forward else layer(q[i], k[i], v[i])
+            # the columns' last workgroups merge their ranges, told by counters that belong to the graphs: a layer has them for
+            # this call, and eager calls, which may run beside a replay, count on their stream's own
+            layer.arrivals = self._scratch[1]
+            try:
+                o = layer(q[i], k[i], v[i], out=to) if getattr(layer.forward, "__func__", None) is Attention.forward else layer(q[i], k[i], v[i])
+            finally:
+                layer.arrivals = None
             if o.data_ptr() != to.data_ptr():      # another module's, or a forward hook's
                 to.copy_(o)
 
@@ -118,11 +124,10 @@ class BucketedDecodeGraphs:
         v = torch.zeros_like(k)
         outputs = torch.zeros_like(q)
         workspace = ops.decode_attn_workspace(bsz, a.num_heads, self.max_num_blocks * block_size, dev)
-        # the columns' last workgroups merge their ranges, told by counters that belong to the graphs like the workspace does
-        arrivals = torch.zeros(_lib.DECODE_ARRIVALS, dtype=torch.int32, device=dev)
-        self._scratch = (workspace, arrivals)       # the layers' own references end with the next capture
+        # (the layers' own references end with the next capture)
+        self._scratch = (workspace, torch.zeros(_lib.DECODE_ARRIVALS, dtype=torch.int32, device=dev))
         for layer in self.layers:
-            layer.workspace, layer.arrivals = workspace, arrivals
+            layer.workspace = workspace
         self.graph_bs = [b for b in [1, 2, 4, 8] + list(range(16, bsz + 1, 16)) if b <= bsz]
         if self.graph_bs[-1] != bsz:
             self.graph_bs.append(bsz)

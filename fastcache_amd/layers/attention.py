@@ -67,7 +67,7 @@ class Attention(nn.Module):
         self.num_heads, self.head_dim, self.scale, self.num_kv_heads = num_heads, head_dim, scale, num_kv_heads
         self.k_cache = self.v_cache = torch.tensor([])
         self.workspace: Optional[torch.Tensor] = None   # set by a graph runner that owns the scratch memory
-        self.arrivals: Optional[torch.Tensor] = None    # with it, int32 zeros for the kernels that merge a column's ranges
+        self.arrivals: Optional[torch.Tensor] = None    # during its calls: zeros for the kernels that merge a column's ranges
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """q ``[N, Hq*D]``, k and v ``[N, Hkv*D]`` -> ``[N, Hq*D]``, in ``out`` where one is given."""

@@ -729,3 +729,50 @@ def test_graphs_keep_their_scratch_when_the_layers_are_captured_again(dev):
         reset_context()
     assert all(torch.equal(o.view(torch.int16), outs[0].view(torch.int16)) for o in outs)
     assert all(bool((t == 255).all()) for t in others)
+
+
+def test_eager_calls_on_captured_layers_leave_the_graphs_counters_alone(dev):
+    """The layers of bucketed graphs called eagerly, with a batch of the graphs' size and with a larger one, whose partial
+    results do not fit the graphs' workspace: both may run beside a replay, so neither may count on the graphs' words (which hold
+    numbers here that would have no workgroup of a column merge it)."""
+    from fastcache_amd.engine.decode_graph import BucketedDecodeGraphs
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    Hq, Hkv, lens, dtype = 14, 2, [700, 513, 600, 900, 257, 800], torch.bfloat16
+    case = synth.make_paged_case(seed=63, num_layers=1, batch=6, num_kv_heads=Hkv, seq_lens=[n + 1 for n in lens], dtype=dtype)
+    pool, tables = case.kv_cache.to(dev), case.table_tensor(dev)
+    layers = [Attention(Hq, 128, 128 ** -0.5, Hkv) for _ in range(2)]
+    for a in layers:
+        a.k_cache, a.v_cache = pool[0, 0], pool[1, 0]
+    fresh, layer = layers
+    graphs = BucketedDecodeGraphs([layer], 2, tables.shape[1], dtype, dev)
+    graphs.capture_cudagraph()
+    workspace, arrivals = graphs._scratch
+    assert bool((arrivals == 0).all()) and layer.workspace is workspace
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(6, h * 128, generator=g).to(dtype).to(dev) for h in (Hq, Hkv, Hkv))
+    with torch.inference_mode():
+        arrivals.fill_(1 << 20)
+    try:
+        for given in (None, arrivals):          # by the layer as it is, and handed to it
+            for n in (2, 6):
+                if given is not None and n == 2:
+                    continue                    # counters that come with the workspace they are for are counted on
+                layer.arrivals = given
+                set_context(False, slot_mapping=torch.full((n,), -1, dtype=torch.int32, device=dev),
+                            context_lens=torch.tensor(lens[:n], dtype=torch.int32, device=dev), block_tables=tables[:n])
+                got, want = layer(q[:n], k[:n], v[:n]), fresh(q[:n], k[:n], v[:n])
+                torch.cuda.synchronize()
+                assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+                assert bool((arrivals == 1 << 20).all())
+        layer.arrivals = None
+        with torch.inference_mode():
+            arrivals.zero_()
+        set_context(False, slot_mapping=torch.full((2,), -1, dtype=torch.int32, device=dev),
+                    context_lens=torch.tensor(lens[:2], dtype=torch.int32, device=dev), block_tables=tables[:2])
+        for _ in range(3):
+            replayed = graphs.run(q[None, :2], k[None, :2], v[None, :2]).clone()
+            assert torch.equal(replayed[0].view(torch.int16), layer(q[:2], k[:2], v[:2]).view(torch.int16))
+        assert bool((arrivals == 0).all())
+    finally:
+        reset_context()
