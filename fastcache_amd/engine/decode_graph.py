@@ -73,6 +73,13 @@ class DecodeGraph:
         return self.out
 
 
+def _takes_out(layer) -> bool:
+    """Whether ``layer(...)`` ends in ``Attention.forward``: any callable may stand for a layer, also one that is no module or
+    has a ``__call__`` or ``forward`` of its own."""
+    return (isinstance(layer, Attention) and type(layer).__call__ is torch.nn.Module.__call__
+            and getattr(layer.forward, "__func__", None) is Attention.forward)
+
+
 class BucketedDecodeGraphs:
     """One captured decode step per batch bucket, replayed with host-patched static buffers: the
     protocol of ``capture_cudagraph`` / ``reset_graph_vars`` / the decode branch of ``run_model``
@@ -105,11 +112,11 @@ class BucketedDecodeGraphs:
             # this call, and eager calls, which may run beside a replay, count on their stream's own
             layer.arrivals = self._scratch[1]
             try:
-                o = layer(q[i], k[i], v[i], out=to) if getattr(layer.forward, "__func__", None) is Attention.forward else layer(q[i], k[i], v[i])
+                o = layer(q[i], k[i], v[i], out=to) if _takes_out(layer) else layer(q[i], k[i], v[i])
             finally:
                 layer.arrivals = None
-            if o.data_ptr() != to.data_ptr():      # another module's, or a forward hook's
-                to.copy_(o)
+            if o is not to:      # another layer's, or a forward hook's
+                out[i] = o
 
     @torch.inference_mode()
     def capture_cudagraph(self):

@@ -765,6 +765,8 @@ def test_eager_calls_on_captured_layers_leave_the_graphs_counters_alone(dev):
                 torch.cuda.synchronize()
                 assert torch.equal(got.view(torch.int16), want.view(torch.int16))
                 assert bool((arrivals == 1 << 20).all())
+                to = torch.empty_like(want)
+                assert fresh(q[:n], k[:n], v[:n], out=to) is to and torch.equal(to.view(torch.int16), want.view(torch.int16))
         layer.arrivals = None
         with torch.inference_mode():
             arrivals.zero_()

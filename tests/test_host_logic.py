@@ -602,3 +602,30 @@ def test_snapkv_rows_route_is_the_split_rules():
     assert route(4, 2, 2, 8, 36865, 32, 0, 36865)[0] == -1
     assert route(4, 2, 1, 17, 600, 32, 0, 600)[0] == -1          # 17 blocks
     assert route(2000, 1, 1, 4, 36865, 32, 1, 36865)[0] == 0     # whole columns need no selection of their own
+
+
+def test_any_callable_is_a_layer_of_bucketed_graphs():
+    """What a captured step calls: plain functions, layers with a ``__call__`` or a ``forward`` of their own (none of which
+    knows of an output to write to), and results that are no tensor of the output's shape."""
+    from fastcache_amd.engine.decode_graph import BucketedDecodeGraphs
+    from fastcache_amd.layers import Attention
+
+    class Called(Attention):
+        def __call__(self, q, k, v):
+            return q + 1
+
+    class Own(Attention):
+        def forward(self, q, k, v):
+            return q + 2
+
+    patched = Attention(1, 128, 1.0, 1)
+    patched.forward = lambda q, k, v: q + 3
+    layers = [lambda q, k, v: q, Called(1, 128, 1.0, 1), Own(1, 128, 1.0, 1), patched, lambda q, k, v: 4.0,
+              lambda q, k, v: q[:1].double()]
+    graphs = BucketedDecodeGraphs(layers, 2, 1, torch.float32, "cpu")
+    graphs._scratch = (None, None)
+    q = torch.randn(len(layers), 2, 128)
+    out = torch.empty_like(q)
+    graphs._model(q, q, q, out)
+    want = torch.stack([q[0], q[1] + 1, q[2] + 2, q[3] + 3, torch.full((2, 128), 4.0), q[5, :1].expand(2, -1)])
+    assert torch.equal(out, want)
