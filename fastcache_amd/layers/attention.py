@@ -62,12 +62,15 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
 class Attention(nn.Module):
     """Same constructor and cache attributes as the reference layer; ``forward`` serves decode steps."""
 
+    # set by a graph runner during its calls: zeros for the kernels that merge a column's ranges (of the class, so that layers
+    # saved before it was there, or set up without this constructor, have it)
+    arrivals: Optional[torch.Tensor] = None
+
     def __init__(self, num_heads, head_dim, scale, num_kv_heads):
         super().__init__()
         self.num_heads, self.head_dim, self.scale, self.num_kv_heads = num_heads, head_dim, scale, num_kv_heads
         self.k_cache = self.v_cache = torch.tensor([])
         self.workspace: Optional[torch.Tensor] = None   # set by a graph runner that owns the scratch memory
-        self.arrivals: Optional[torch.Tensor] = None    # during its calls: zeros for the kernels that merge a column's ranges
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """q ``[N, Hq*D]``, k and v ``[N, Hkv*D]`` -> ``[N, Hq*D]``, in ``out`` where one is given."""

@@ -629,3 +629,23 @@ def test_any_callable_is_a_layer_of_bucketed_graphs():
     graphs._model(q, q, q, out)
     want = torch.stack([q[0], q[1] + 1, q[2] + 2, q[3] + 3, torch.full((2, 128), 4.0), q[5, :1].expand(2, -1)])
     assert torch.equal(out, want)
+
+
+def test_a_layer_saved_without_counters_reaches_its_decode_step(monkeypatch):
+    """The attributes of a layer as they were saved before it could be given counters: the native call gets None."""
+    import types
+    from fastcache_amd import _lib
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    saved = {k: v for k, v in Attention(1, 128, 1.0, 1).__dict__.items() if k != "arrivals"}
+    layer = Attention.__new__(Attention)
+    layer.__setstate__(saved)
+    calls = []
+    monkeypatch.setattr(_lib, "host", lambda: types.SimpleNamespace(decode_layer=lambda *a: calls.append(a) or a[0]))
+    t = torch.zeros(1, dtype=torch.int32)
+    set_context(False, slot_mapping=t, context_lens=t, block_tables=t[None])
+    try:
+        q = torch.randn(1, 128)
+        assert layer(q, q, q) is q and calls[0][-1] is None
+    finally:
+        reset_context()
