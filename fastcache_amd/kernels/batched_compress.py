@@ -102,7 +102,7 @@ class BatchedGEMMCompressor(nn.Module):
                     ops.copy_tokens(sv[p], dv[p], seg_start, n, dst)
             else:
                 w = [self._weights(seg + kind, k0.dtype, k0.device, (l0, l1)) for kind in "kv"]
-                ops.ccm_mlp_kv(sv, dv, w, cf, seg_start, n, dst)
+                ops.ccm_mlp_planes(sv, dv, w, cf, seg_start, n, dst)
             dst += self._seg_len(n)
         return [(out[0][i], out[1][i]) for i in range(L)]
 
@@ -141,9 +141,9 @@ class BatchedGEMMCompressor(nn.Module):
             for seg, n_max, (st, ct, dt), same in plan:
                 w = [self._weights(seg + kind, kv_cache.dtype, dev, (l0, l1)) for kind in "kv"]
                 if same:
-                    ops.ccm_mlp_kv(views, dviews, w, cf, st, ct, dt)
+                    ops.ccm_mlp_planes(views, dviews, w, cf, st, ct, dt)
                 else:
-                    ops.ccm_mlp_kv_ragged(views, dviews, w, cf, st, ct, dt, n_max, self.min_seq_len)
+                    ops.ccm_mlp_planes_ragged(views, dviews, w, cf, st, ct, dt, n_max, self.min_seq_len)
             return dsts
         for s0, n, seg in ((0, img, "i"), (img, seq_len - img, "t")):
             if n == 0:
@@ -154,7 +154,7 @@ class BatchedGEMMCompressor(nn.Module):
                         ops.copy_tokens(view, dview, s0, n, dst)
             else:
                 w = [self._weights(seg + kind, kv_cache.dtype, kv_cache.device, (l0, l1)) for kind in "kv"]
-                ops.ccm_mlp_kv(views, dviews, w, cf, s0, n, dst)
+                ops.ccm_mlp_planes(views, dviews, w, cf, s0, n, dst)
             dst += self._seg_len(n)
         return dst
 

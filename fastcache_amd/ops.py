@@ -481,6 +481,30 @@ def ccm_mlp_kv_ragged(srcs, dsts, weights, cf: int, seg_start: torch.Tensor, seg
           "fc_ccm_mlp_kv_ragged")
 
 
+def _planes_alike(views) -> bool:
+    """Whether the views of two planes differ in their place only (``base``, the first field)."""
+    return bytes(views[0])[8:] == bytes(views[1])[8:]
+
+
+def ccm_mlp_planes(srcs, dsts, weights, cf: int, seg_start: int, seg_len: int, dst_start: int) -> None:
+    """``ccm_mlp_kv``, or a call per plane for planes of different strides or lengths (outputs that are tensors apart)."""
+    if _planes_alike(srcs) and _planes_alike(dsts):
+        ccm_mlp_kv(srcs, dsts, weights, cf, seg_start, seg_len, dst_start)
+    else:
+        for p in range(2):
+            ccm_mlp(srcs[p], dsts[p], weights[p], cf, seg_start, seg_len, dst_start)
+
+
+def ccm_mlp_planes_ragged(srcs, dsts, weights, cf: int, seg_start: torch.Tensor, seg_len: torch.Tensor,
+                          dst_start: torch.Tensor, max_seg_len: int, min_rows: int) -> None:
+    """``ccm_mlp_kv_ragged``, or a call per plane, as ``ccm_mlp_planes``."""
+    if _planes_alike(srcs) and _planes_alike(dsts):
+        ccm_mlp_kv_ragged(srcs, dsts, weights, cf, seg_start, seg_len, dst_start, max_seg_len, min_rows)
+    else:
+        for p in range(2):
+            ccm_mlp_ragged(srcs[p], dsts[p], weights[p], cf, seg_start, seg_len, dst_start, max_seg_len, min_rows)
+
+
 def expected_attention_score(keys: FcKvView, values: FcKvView, mean_query: torch.Tensor,
                              cov_query: Optional[torch.Tensor], n_sink: int = 4, use_vnorm: bool = True,
                              epsilon: float = 0.0, score_stride: Optional[int] = None) -> torch.Tensor:

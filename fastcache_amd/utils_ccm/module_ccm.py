@@ -208,7 +208,7 @@ class _CCMBase(nn.Module):
                         ops.copy_tokens(view, dview, s0, n, dst)
             else:
                 w = [self._layer_weights(g, l0, l1, kv_cache.dtype, kv_cache.device) for g in (gk, gv)]
-                ops.ccm_mlp_kv(views, dviews, w, cf, s0, n, dst)
+                ops.ccm_mlp_planes(views, dviews, w, cf, s0, n, dst)
             dst += self._segment_len(n)
         return dst
 
@@ -238,9 +238,9 @@ class _CCMBase(nn.Module):
         for gk, gv, n_max, (starts, counts, dsts), same in plan:
             w = [self._layer_weights(g, l0, l1, kv_cache.dtype, dev) for g in (gk, gv)]
             if same:
-                ops.ccm_mlp_kv(views, dviews, w, cf, starts, counts, dsts)
+                ops.ccm_mlp_planes(views, dviews, w, cf, starts, counts, dsts)
             else:
-                ops.ccm_mlp_kv_ragged(views, dviews, w, cf, starts, counts, dsts, n_max, self.min_seq_len)
+                ops.ccm_mlp_planes_ragged(views, dviews, w, cf, starts, counts, dsts, n_max, self.min_seq_len)
         return dst
 
     def _forward_layers(self, kv_cache: Sequence[LayerKV], segments) -> Optional[List[LayerKV]]:

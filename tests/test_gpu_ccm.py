@@ -372,3 +372,37 @@ def test_ccm_mlp_both_planes_in_one_call(dev, lens, block_size, cf, dense):
     v = _lib.paged_view(planes[1], tables, mk(lens), S - 1)
     with pytest.raises(_lib.FastcacheError, match="differ in more than their place"):
         ops.ccm_mlp_kv([src[0], v], dst, w, cf, 0, S - 1, 0)
+
+
+@pytest.mark.parametrize("lens", [[333, 333], [333, 70, 4]])
+@pytest.mark.parametrize("batched", [True, False])
+def test_planes_of_different_geometry_are_compressed_apart(dev, lens, batched):
+    """``paged_forward`` into K and V outputs that are tensors of their own, of other strides and lengths, as a K output and a
+    V output of one tensor; and a list whose V tensors hold more tokens than K's, of which the compressor takes as many."""
+    from types import SimpleNamespace
+    from fastcache_amd.kernels import BatchedGEMMCompressor
+    from fastcache_amd.utils_ccm import KVCacheLinearDecoupleCompressor
+    L, H, B, S, cf, img, dtype = 2, 3, len(lens), max(lens), 5, 41, torch.bfloat16
+    cfg = SimpleNamespace(text_config=SimpleNamespace(num_hidden_layers=L, num_key_value_heads=H, hidden_size=H * 128,
+                                                      head_dim=128, num_attention_heads=H))
+    torch.manual_seed(12)
+    comp = KVCacheLinearDecoupleCompressor(cfg, compression_factor=cf).to(dev).to(dtype).eval()
+    if batched:
+        orig, comp = comp, BatchedGEMMCompressor(num_layers=L, num_heads=H, head_dim=128, compression_factor=cf)
+        comp.load_from_original_compressor(orig)
+    case = synth.make_paged_case(seed=9, num_layers=L, batch=B, num_kv_heads=H, seq_lens=lens, dtype=dtype)
+    pool, tables, n = case.kv_cache.to(dev), case.table_tensor(dev), torch.tensor(lens, dtype=torch.int32, device=dev)
+    C = max(comp.paged_compressed_len(x, [img, x - img]) for x in lens)
+    run = lambda out: comp.paged_forward(pool, tables, n, S, [img, S - img], out=out, host_lens=lens)
+    want = torch.zeros(2, L, B, H, C, 128, dtype=dtype, device=dev)
+    apart = (torch.zeros(L, B, H, C + 7, 128, dtype=dtype, device=dev), torch.zeros(L, B, C, H, 128, dtype=dtype, device=dev).transpose(2, 3))
+    assert run(want) == run(apart)
+    for a, b in ((apart[0][:, :, :, :C], want[0]), (apart[1], want[1])):
+        assert torch.equal(a.contiguous().view(torch.int16), b.view(torch.int16))
+    assert not bool(apart[0][:, :, :, C:].any()) and bool(want[0, :, 0, :, :C].any())
+    kv = [(torch.randn(B, H, 90, 128, device=dev).to(dtype), torch.randn(B, H, 97, 128, device=dev).to(dtype)) for _ in range(L)]
+    if batched:
+        got = comp(kv, it_len=[img, 90 - img])
+        ref = comp([(k, v[:, :, :90].contiguous()) for k, v in kv], it_len=[img, 90 - img])
+        for x, y in zip(got, ref):
+            assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(x, y))
