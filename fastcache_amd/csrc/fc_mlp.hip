@@ -567,10 +567,16 @@ __global__ __launch_bounds__(ML_THREADS, ML_WAVES / 4) void mlp_list_kernel(KvVi
 // What the MLP leaves of a segment (the launch's, or with the arrays each sequence's own): the seg_len % cf remainder tokens, or
 // the whole segment of a sequence too short to compress, copied to their place behind the compressed rows.  One workgroup per
 // (sequence, plane and layer) and heads_per_wg heads, whose rows are one list, tokens ascending; ML_TAIL rows per pass, all
-// loaded before any is stored (destination token <= source token).  A workgroup per head was mostly the starting of workgroups,
-// a row or two each: 24 sequences x 32 heads x 64 layers and planes 60 us, 12 like this, 8 sequences 27, 6; 4 heads the same.
-// (Several rows per thread lose: the table reads of a thread's rows wait for each other, 10 to 20 us.)
+// loaded before any is stored (destination token <= source token).  A workgroup per head is mostly the starting of workgroups
+// where a head has a row or two, all heads in one workgroup a chain of passes where it has many, each a table read, a barrier
+// and a memory latency: ML_TAIL_ROWS rows a workgroup, in powers of two of heads (3 heads of 18 tokens 36, 4 33, 8 sequences) and
+// two heads at least.  us, 32 heads x 64 layers and planes, a workgroup per head / like this / 32 heads in one: 1 token of 1
+// sequence 6.2 / 3.2 / 3.1, of 24 58 / 7.0 / 7.0; 4 tokens 6.4 / 4.1 / 5.0, 62 / 26 / 27; 18 8.5 / 6.3 / 14, 129 / 107 / 108;
+// 60 19 / 14 / 50, 316 / 312 / 344; 130 32 / 25 / 102, 666 / 674 / 734; 200 43 / 34 / 155, 1007 / 1004 / 1115; 4 heads, 200 tokens
+// of 1 sequence 18 / 11 / 19.  (Several rows per thread lose: the table reads of a thread's rows wait for each other, 10 to
+// 20 us.)
 #define ML_TAIL 32
+#define ML_TAIL_ROWS 64
 __global__ __launch_bounds__(16 * ML_TAIL) void mlp_tail_copy_kernel(KvView src, KvView dst, MlPlanes a, int cf, int min_rows, int c_max,
                                                             const int* __restrict__ seg_start_v,
                                                             const int* __restrict__ seg_len_v,
@@ -777,7 +783,8 @@ static int ml_planes(const char* who, const fc_kv_view* const src[2], const fc_k
   return FC_OK;
 }
 
-// remainders and pass-through segments; nothing to move when a pass-through segment already lies at its place
+// remainders and pass-through segments (of the arrays' segments seg_len is the longest); nothing to move when a pass-through
+// segment already lies at its place
 static void ml_tails(const fc_kv_view* const src[2], const fc_kv_view* const dst[2], const MlPlanes& a, int planes, int cf,
                      int min_rows, int c, const int32_t* seg_start_v, const int32_t* seg_len_v, const int32_t* dst_start_v,
                      int seg_start, int seg_len, int dst_start, hipStream_t st) {
@@ -785,7 +792,11 @@ static void ml_tails(const fc_kv_view* const src[2], const fc_kv_view* const dst
   for (int p = 0; p < planes; ++p)
     same = same && src[p]->base == dst[p]->base && src[p]->block_tables == dst[p]->block_tables &&
            src[p]->stride_layer == dst[p]->stride_layer && src[p]->stride_batch == dst[p]->stride_batch;
-  const int heads = src[0]->num_kv_heads, per = heads < 32 ? heads : 32;
+  // what a sequence leaves at most: a remainder, or a segment of too few rows
+  const int64_t most = seg_len_v ? std::min<int64_t>(seg_len, std::max<int64_t>(min_rows, 1) * cf - 1) : seg_len - (int64_t)c * cf;
+  int want = 2;
+  while (want < 32 && want * most < ML_TAIL_ROWS) want *= 2;
+  const int heads = src[0]->num_kv_heads, per = heads < want ? heads : want;
   hipLaunchKernelGGL(mlp_tail_copy_kernel, dim3((heads + per - 1) / per, src[0]->batch, planes * src[0]->num_layers),
                      dim3(16 * ML_TAIL), 0, st, fc_make_view(src[0]), fc_make_view(dst[0]), a, cf, min_rows, c, seg_start_v, seg_len_v, dst_start_v,
                      seg_start, seg_len, dst_start, same, per);
@@ -834,7 +845,7 @@ static int ml_ragged(const char* who, const fc_kv_view* const src[2], const fc_k
   if (c > 0 && c >= min_rows &&
       (rc = ml_launch(who, src[0], dst[0], a, planes, cf, 0, c, 0, seg_start, seg_len, dst_start, min_rows, st)))
     return rc;
-  ml_tails(src, dst, a, planes, cf, min_rows, c, seg_start, seg_len, dst_start, 0, 0, 0, st);
+  ml_tails(src, dst, a, planes, cf, min_rows, c, seg_start, seg_len, dst_start, 0, max_seg_len, 0, st);
   FC_CHECK_LAUNCH(who);
   return FC_OK;
 }

@@ -406,3 +406,28 @@ def test_planes_of_different_geometry_are_compressed_apart(dev, lens, batched):
         ref = comp([(k, v[:, :, :90].contiguous()) for k, v in kv], it_len=[img, 90 - img])
         for x, y in zip(got, ref):
             assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(x, y))
+
+
+@pytest.mark.parametrize("H,lens,cf,min_rows", [
+    (33, [1, 3, 2], 2, 2),                  # up to 3 tokens: 32 heads a workgroup, one in the second
+    (7, [33, 1, 12, 0], 3, 12),             # up to 33: 2 heads a workgroup, more passes than one, the last of one head
+    (5, [260, 17, 90], 4, 100),             # whole segments longer than the rows of a workgroup
+    (40, [64, 63, 9], 64, 2),
+])
+def test_segments_too_short_to_compress_are_copied_whatever_their_length(dev, H, lens, cf, min_rows):
+    """Segments of too few rows, heads shared out over workgroups by the length they may have: the rows of every sequence at
+    their place, nothing else touched."""
+    L, B, S, dtype = 2, len(lens), 300, torch.float16
+    case = synth.make_paged_case(seed=14, num_layers=L, batch=B, num_kv_heads=H, seq_lens=[S] * B, dtype=dtype)
+    pool, tables = case.kv_cache.to(dev), case.table_tensor(dev)
+    mk = lambda xs: torch.tensor(xs, dtype=torch.int32, device=dev)
+    starts, dsts = [30 + 2 * b for b in range(B)], [b for b in range(B)]
+    want = case.kv_cache.clone()
+    for b, n in enumerate(lens):
+        at = lambda s: torch.tensor([case.block_tables[b][(s + i) // 256] * 256 + (s + i) % 256 for i in range(n)], dtype=torch.long)
+        flat, old = want.view(2, L, -1, H, 128), case.kv_cache.view(2, L, -1, H, 128)
+        flat[:, :, at(dsts[b])] = old[:, :, at(starts[b])]
+    views = [_lib.paged_view(pool[p], tables, mk([S] * B), S) for p in range(2)]
+    w = [tuple(torch.zeros(s, dtype=dtype, device=dev) for s in ((L, 128, 128 * cf), (L, 128), (L, 128, 128), (L, 128), (L, 128, 128), (L, 128)))] * 2
+    ops.ccm_mlp_kv_ragged(views, views, w, cf, mk(starts), mk(lens), mk(dsts), max(lens), min_rows)
+    assert torch.equal(pool.cpu().view(torch.int16), want.view(torch.int16))
