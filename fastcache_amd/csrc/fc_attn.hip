@@ -1156,13 +1156,22 @@ static bool da_tile_in_page(const fc_kv_view* v) {
 // 2000 1030 -> 1054).  Smaller groups leave those to the split kernel, which holds them whole as well (12 captured layers, this /
 // that: 32 heads, 10 of 100 to 250 186 / 165, 14 of 250 247 / 220, 16 of 500 342 / 333; 32 heads on 8, 48 of 100 to 500
 // 287 / 289, of 500 373 / 337, 40 of 700 445 / 394, 36 of 100 to 700 301 / 315).
-// Groups of 3 and 4: 2 tiles 572 -> 487 (96 of 1000), 3 635 -> 587, 4 748 -> 715, 802 -> 743, one
-// 693 -> 697; 5 730 -> 799, 921 -> 1027.  Smaller groups: 2 tiles 588 -> 551 (64 of 2000), 675 -> 533; 3 to 6 where the
-// workgroups are seven eighths of the compute units with ranges 85 % full, or three quarters and whole columns (32 heads, 12
-// captured layers, or 28 eager ones): 6 sequences of 800 288 -> 234, 1 of 8000 445 -> 374, 2 of 5000 413 -> 393, 8 of 1300
-// 383 -> 343, 7 of 120 to 1200 691 -> 701; 4 of 1400 707 -> 666, 2 of 3000 609 -> 561; else 4 of 170 to 1700 657 -> 672, 622 -> 645,
-// 5 of 900 245 -> 254, 3 of 2500 634 -> 722, 5 of 1400 616 -> 703; more tiles: 8 of 2000 462 -> 472, 4 of 4000 459 -> 479, 2 of 8000
-// 553 -> 535.
+// Up to 4 heads a group, where the split kernel holds columns of up to 1024 tokens whole and appends inside: us a captured layer,
+// split kernel / this (eager layers of these sizes: the same shares), lengths equal | a tenth to all of the longest.
+// Two tiles always: 32 heads, 2 of 2048 21.0 / 19.8 | 20.1 / 19.0, on 8 kv heads 8 of 2048 25.4 / 22.6 | 21.5 / 20.1.
+// Groups of 3 and 4, 3 and 4 tiles: on 8 kv heads 8 of 2560 27.9 / 25.8 | 22.9 / 21.5, of 4096 34.0 / 32.0 | 31.0 / 28.8, 24 of
+// 1024 30.4 / 26.1 | 26.9 / 23.1, 16 of 2048 34.0 / 32.4 | 30.1 / 28.5, 4 of 6144 30.4 / 27.3 | 26.6 / 23.2, 12 of 1280
+// 24.2 / 23.4 | 19.4 / 20.0; but 4 tiles of few ranges that are not full and leave a quarter of the compute units idle do not
+// pay: 12 of 1792 26.8 / 27.1 | 24.0 / 25.3.  5 and 6 tiles: 12 of 2304 31.9 / 32.4 | 25.8 / 28.3, 20 of 1536 31.9 / 32.4 |
+// 27.3 / 30.2.
+// Groups of 1 and 2, 3 to 6 tiles: whole columns that fill three quarters of the compute units, 32 heads, 6 of 1024 26.6 / 25.2 |
+// 24.7 / 24.0, of 1280 33.9 / 30.2 | 28.5 / 26.5, of 1536 37.8 / 35.0 | 33.9 / 33.1, 8 of 1280 36.1 / 35.0 | 28.9 / 28.4, but of
+// 1536 with one head a group 41.1 / 40.6 | 34.4 / 36.0; ranges 85 % full, seven eighths of the compute units busy, where two of
+// three hold: 3 tiles, 7 ranges or more, two heads a group or all units busy: 32 heads, 1 of 5120 26.1 / 24.3, of 8192
+// 37.2 / 32.3, of 10240 39.7 / 37.8, 2 of 3072 26.0 / 25.6 | 26.8 / 26.4, on 16 kv heads 3 of 3584 25.8 / 25.0 | 22.4 / 22.4, 2 of
+// 7168 31.7 / 30.2 | 29.4 / 28.6; else 4 of 1792 28.4 / 29.4 | 26.4 / 27.8, of 2304 33.5 / 35.1 | 27.8 / 30.6, 2 of 4608
+// 36.1 / 36.8 | 29.6 / 30.9, on 16 3 of 5632 33.6 / 35.3 | 28.9 / 30.9; 8 heads, 5 of 4096 23.7 / 24.7 | 20.7 / 21.4, of 5632
+// 29.0 / 30.5 | 23.6 / 25.9.
 #define DC_ONE 768
 #define DC_TILES_FEW 6
 #define DC_TILES_SOME 4
@@ -1190,8 +1199,12 @@ static int da_column_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_h
   for (int m = 2; m <= most; ++m) {
     const long long ranges = (k->max_seq_len + m * chunk - 1) / (m * chunk), wgs = cols * ranges;
     if (wgs > slots) continue;
-    const bool full = ranges == 1 ? 4 * wgs >= 3 * slots : 8 * wgs >= 7 * slots && 20ll * k->max_seq_len >= 17 * ranges * m * chunk;
-    return G > 2 || m == 2 || full ? m * chunk : 0;
+    const bool busy = 8 * wgs >= 7 * slots, all = wgs == slots;
+    const auto full = [&](int percent) { return 100ll * k->max_seq_len >= percent * ranges * m * chunk; };
+    if (m == 2 || G > 4) return m * chunk;
+    if (G > 2) return m == 3 || busy || ranges == 1 || ranges > 3 || full(90) ? m * chunk : 0;
+    if (ranges == 1) return 4 * wgs >= 3 * slots && (m < DC_TILES_FEW || G == 2 || !busy) ? m * chunk : 0;
+    return busy && full(85) && (m == 3) + (ranges >= 7) + (all || G == 2) >= 2 ? m * chunk : 0;
   }
   return 0;
 }

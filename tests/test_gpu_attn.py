@@ -274,7 +274,7 @@ def test_decode_attention_empty_rows(dev):
     (torch.float16, 8, 1, ([3900, 1535, 1536, 1537, 100, 3072, 3073] * 10)[:65], -1),    # 8 heads a group: 1536
     (torch.bfloat16, 32, 4, ([700, 511, 512, 1, 600] * 14)[:70], -1),                    # two rounds of whole columns
     (torch.float16, 8, 8, ([1200, 1030, 257, 1279, 64, 1025, 800, 1] * 4)[:28], -1),      # 5 tiles a wavefront, whole columns
-    (torch.bfloat16, 8, 4, ([2700, 2815, 1407, 1408, 1409, 1] * 6)[:32], 0),               # 6, two ranges
+    (torch.bfloat16, 8, 4, ([2700, 2815, 1407, 1408, 1409, 1] * 6)[:32], 0),               # two heads a group, chunks that append
 ])
 def test_attention_layer_appends_and_attends(dev, dtype, Hq, Hkv, lens, slot_at):
     """``Attention.forward`` of a decode step against the oracle on a cache the oracle appended to: every launch form the
@@ -778,3 +778,48 @@ def test_eager_calls_on_captured_layers_leave_the_graphs_counters_alone(dev):
         assert bool((arrivals == 0).all())
     finally:
         reset_context()
+
+
+def _launches(run, *names):
+    """Names of the launches of ``run`` that contain one of ``names``.  A profile now and then holds nothing: the next one is
+    asked, and that none holds any fails."""
+    for _ in range(8):
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
+            run()
+            torch.cuda.synchronize()
+        found = [e.name for e in prof.events() if any(n in e.name for n in names)]
+        if found:
+            return found
+    pytest.fail(f"no profile holds any of {names}")
+
+
+@pytest.mark.parametrize("Hq,Hkv,B,pages,column", [
+    (32, 32, 4, 6, True), (32, 32, 4, 7, False), (32, 32, 2, 18, False),      # ranges of 3 tiles for all compute units; of 4, 5
+    (8, 8, 4, 20, True), (8, 8, 5, 18, False), (16, 8, 5, 18, True),          # 7 ranges of 3 tiles; 6, one and two heads a group
+    (8, 8, 4, 32, True), (8, 8, 4, 28, False), (16, 8, 4, 28, True), (16, 8, 16, 11, False),      # 8 and 7 ranges of 4 tiles; 2 of 6
+    (32, 32, 6, 6, True), (32, 32, 8, 6, False), (32, 16, 16, 6, True),       # whole columns of 6 tiles
+    (32, 8, 12, 7, False), (32, 8, 12, 8, True), (32, 8, 12, 5, True), (32, 8, 16, 7, True)])
+def test_which_kernel_takes_columns_of_several_tiles(dev, Hq, Hkv, B, pages, column):
+    """Ranges of 3 and more tiles a wavefront for groups of up to 4 heads, on both sides of the rule between the column and
+    the split kernel: which of them runs, and the oracle's values."""
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    dtype, hi = torch.bfloat16, pages * 256 - 1
+    lens = [hi - (hi * 9 * b) // (10 * B) for b in range(B)]
+    case = synth.make_paged_case(seed=91, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=[n + 1 for n in lens], dtype=dtype)
+    g = torch.Generator().manual_seed(2)
+    q, k, v = (torch.randn(B, h * 128, generator=g).to(dtype) for h in (Hq, Hkv, Hkv))
+    tables, lens_t = case.table_tensor("cpu"), torch.tensor(lens, dtype=torch.int32)
+    slots = torch.tensor([t[n // 256] * 256 + n % 256 for t, n in zip(case.block_tables, lens)], dtype=torch.int32)
+    ref = oattn.decode_attention(q.view(B, Hq, 128), case.kv_cache[0, 0], case.kv_cache[1, 0], lens_t, tables, 128 ** -0.5)
+    layer, on_gpu = Attention(Hq, 128, 128 ** -0.5, Hkv), case.kv_cache[:, 0].to(dev)
+    layer.k_cache, layer.v_cache = on_gpu[0], on_gpu[1]
+    set_context(False, slot_mapping=slots.to(dev), context_lens=lens_t.to(dev), block_tables=tables.to(dev))
+    q, k, v = q.to(dev), k.to(dev), v.to(dev)
+    try:
+        got = layer(q, k, v).cpu()
+        names = _launches(lambda: layer(q, k, v), "decode_column_kernel<", "decode_attn_kernel<")
+    finally:
+        reset_context()
+    assert ["decode_column_kernel<" in n for n in names] == [column]
+    assert float((got.view(B, Hq, 128).float() - ref.float()).abs().max()) < 4e-3      # as above
