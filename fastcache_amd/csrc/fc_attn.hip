@@ -1249,9 +1249,19 @@ static int da_split_chunk(const fc_kv_view* k, const fc_kv_view* v, int num_q_he
   return chunk;
 }
 
-// One workgroup a column of the split kernel: no merge, and where it may append (its kv head's rows, one table) one launch a layer.
-static bool da_split_whole(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
-  return k->max_seq_len > 0 && k->max_seq_len <= da_split_chunk(k, v, num_q_heads) && da_tile_in_page(k) && da_tile_in_page(v);
+// What a launch of this shape is, decided once a call: the column kernel, or the split kernel in chunks or with whole columns (no
+// merge).
+struct DaPlan {
+  int column;      // tokens a workgroup of the column kernel, 0: the split kernel
+  int chunk;       // ... of the split kernel
+  bool whole;      // the split kernel holds every sequence in one chunk
+};
+static DaPlan da_plan(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
+  DaPlan p{da_column_chunk(k, v, num_q_heads), 0, false};
+  if (p.column) return p;
+  p.chunk = da_split_chunk(k, v, num_q_heads);
+  p.whole = k->max_seq_len > 0 && k->max_seq_len <= p.chunk && da_tile_in_page(k) && da_tile_in_page(v);
+  return p;
 }
 
 static int da_merge(const char* who, const fc_kv_view* k_cache, const float* part_o, const float* part_ml,
@@ -1267,11 +1277,11 @@ static int da_merge(const char* who, const fc_kv_view* k_cache, const float* par
   return FC_OK;
 }
 
-// Checks and launches shared by the entry points; `workspace` is a device address.
+// Checks and launches shared by the entry points; `workspace` is a device address, `plan` the caller's where it has one.
 static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_view* v_cache, int32_t layer,
                       const void* q, void* out, int32_t num_q_heads, const int32_t* context_lens, float scale,
                       void* workspace, int64_t workspace_bytes, void* stream, const DaAppend* append = nullptr,
-                      int turn = -1, uint32_t* arrivals = nullptr) {
+                      int turn = -1, uint32_t* arrivals = nullptr, const DaPlan* plan = nullptr) {
   int rc;
   if ((rc = fc_check_view(k_cache, who)) || (rc = fc_check_view(v_cache, who))) return rc;
   FC_REQUIRE(k_cache->dtype == v_cache->dtype && k_cache->num_layers == v_cache->num_layers &&
@@ -1283,7 +1293,8 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
   FC_REQUIRE(num_q_heads > 0 && num_q_heads % k_cache->num_kv_heads == 0, FC_EINVAL,
              "%s: num_q_heads %d not a multiple of num_kv_heads %d", who, num_q_heads, k_cache->num_kv_heads);
   FC_REQUIRE(q && out && context_lens, FC_EINVAL, "%s: null pointer", who);
-  const int column = da_column_chunk(k_cache, v_cache, num_q_heads);
+  const DaPlan shape = plan ? *plan : da_plan(k_cache, v_cache, num_q_heads);
+  const int column = shape.column;
   const int csplits = column ? (k_cache->max_seq_len + column - 1) / column : 0;
   // one workgroup per column needs no workspace; a caller that appends in the same call has asked whether one is needed
   FC_REQUIRE(workspace || (csplits == 1 && append), FC_EINVAL, "%s: null workspace", who);
@@ -1333,7 +1344,7 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
              (long long)workspace_bytes, (long long)need);
   const int B = k_cache->batch, Hkv = k_cache->num_kv_heads, G = num_q_heads / Hkv;
   const int gt = da_group_tile(G), gtiles = (G + gt - 1) / gt;
-  const int chunk = da_split_chunk(k_cache, v_cache, num_q_heads);
+  const int chunk = shape.chunk;
   const int splits = (k_cache->max_seq_len + chunk - 1) / chunk;
   float* part_o = (float*)workspace;
   float* part_ml = part_o + (int64_t)B * num_q_heads * (splits > 0 ? splits : 1) * FC_HEAD_DIM;
@@ -1344,7 +1355,7 @@ static int da_enqueue(const char* who, const fc_kv_view* k_cache, const fc_kv_vi
   if (splits > 0) {
     FC_REQUIRE(Hkv * gtiles <= 65535 && B <= 65535, FC_EUNSUPPORTED, "%s: grid too large", who);
     dim3 grid(splits, Hkv * gtiles, B);
-    const bool fast = da_tile_in_page(k_cache) && da_tile_in_page(v_cache), whole = da_split_whole(k_cache, v_cache, num_q_heads);
+    const bool fast = da_tile_in_page(k_cache) && da_tile_in_page(v_cache), whole = shape.whole;
     const DaAppend ap = append ? *append : DaAppend{nullptr, nullptr, 0, 0, nullptr};
 #define DA_LAUNCH(DT, GTV, FA, WH, AP)                                                                                   \
   do {                                                                                                          \
@@ -1388,18 +1399,20 @@ extern "C" int fc_decode_attn(const fc_kv_view* k_cache, const fc_kv_view* v_cac
 // of 100 to 1200 863 -> 842 (861 where the slots past the first 64 were asked for in their turn); chunks of 7 heads a group
 // lose (90 of 100 to 1000 541 -> 550).  Every workgroup looks at the slots of the whole batch: above 128 sequences that costs
 // more than the launch (6 layers: 256 of 60 to 250 inside 1044, apart 911; 200 of 100 to 250 880, 779; 128 of 60 to 120 405, 406).
-static bool da_split_appends(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
+static bool da_split_appends(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads, const DaPlan& p) {
   const int G = num_q_heads / k->num_kv_heads;
-  return k->batch <= 2 * FC_WAVE && G <= 8 && da_tile_in_page(k) && da_tile_in_page(v) && (G <= 4 || da_split_whole(k, v, num_q_heads));
+  return k->batch <= 2 * FC_WAVE && G <= 8 && da_tile_in_page(k) && da_tile_in_page(v) && (G <= 4 || p.whole);
 }
 
 // Append and attention of one layer.  The workgroup of a column appends its own head's row, so the fused form needs
-// one workgroup per kv head (groups of up to 16 query heads, 8 for whole columns of the split kernel) and both caches on one block table; otherwise the rows
-// go in first, in a launch of their own.
-static bool da_appends_inside(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
+// one workgroup per kv head (groups of up to 16 query heads, 8 for whole columns of the split kernel) and both caches on one
+// block table; otherwise the rows go in first, in a launch of their own.
+static bool da_one_table(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads) {
   return num_q_heads / k->num_kv_heads <= DC_HEADS && k->block_tables && k->block_tables == v->block_tables &&
-         k->table_stride == v->table_stride && k->block_size == v->block_size &&
-         k->max_seq_len > 0 && (da_column_chunk(k, v, num_q_heads) > 0 || da_split_appends(k, v, num_q_heads));
+         k->table_stride == v->table_stride && k->block_size == v->block_size && k->max_seq_len > 0;
+}
+static bool da_appends_inside(const fc_kv_view* k, const fc_kv_view* v, int num_q_heads, const DaPlan& p) {
+  return da_one_table(k, v, num_q_heads) && (p.column > 0 || da_split_appends(k, v, num_q_heads, p));
 }
 
 extern "C" int64_t fc_decode_layer_workspace_bytes(const fc_kv_view* k_cache, const fc_kv_view* v_cache,
@@ -1407,8 +1420,7 @@ extern "C" int64_t fc_decode_layer_workspace_bytes(const fc_kv_view* k_cache, co
   if (!k_cache || !v_cache || num_q_heads <= 0 || k_cache->num_kv_heads <= 0 || k_cache->batch <= 0 ||
       num_q_heads % k_cache->num_kv_heads || k_cache->block_size <= 0 || v_cache->block_size <= 0)
     return -1;
-  if (da_appends_inside(k_cache, v_cache, num_q_heads) &&
-      da_column_chunk(k_cache, v_cache, num_q_heads) >= k_cache->max_seq_len)
+  if (da_one_table(k_cache, v_cache, num_q_heads) && da_column_chunk(k_cache, v_cache, num_q_heads) >= k_cache->max_seq_len)
     return 0;
   return fc_decode_attn_workspace_bytes(k_cache->batch, num_q_heads, k_cache->max_seq_len);
 }
@@ -1442,10 +1454,11 @@ static int da_layer(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const 
   const int eb = fc_elem_bytes(k_cache->dtype);
   FC_REQUIRE((((uintptr_t)k_new | (uintptr_t)v_new | (uint64_t)(k_stride * eb) | (uint64_t)(v_stride * eb)) & 15) == 0, FC_EINVAL,
              "%s: new rows not 16-byte aligned", who);
-  if (da_appends_inside(k_cache, v_cache, num_q_heads)) {
+  const DaPlan plan = da_plan(k_cache, v_cache, num_q_heads);
+  if (da_appends_inside(k_cache, v_cache, num_q_heads, plan)) {
     const DaAppend ap = {(const char*)k_new, (const char*)v_new, k_stride * eb, v_stride * eb, slot_mapping};
     return da_enqueue(who, k_cache, v_cache, 0, q, out, num_q_heads, context_lens, scale, workspace, workspace_bytes,
-                      stream, &ap, turn, arrivals);
+                      stream, &ap, turn, arrivals, &plan);
   }
   // what the attention would refuse is refused before the rows are written
   FC_REQUIRE(q && out && context_lens && workspace, FC_EINVAL, "%s: null pointer", who);
@@ -1454,7 +1467,8 @@ static int da_layer(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const 
   if ((rc = fc_store_kv_slots(k_new, k_stride, v_new, v_stride, k_cache->base, v_cache->base, slot_mapping, k_cache->batch,
                               (int32_t)row, k_cache->dtype, stream)))
     return rc;
-  return da_enqueue(who, k_cache, v_cache, 0, q, out, num_q_heads, context_lens, scale, workspace, workspace_bytes, stream);
+  return da_enqueue(who, k_cache, v_cache, 0, q, out, num_q_heads, context_lens, scale, workspace, workspace_bytes, stream, nullptr,
+                    -1, nullptr, &plan);
 }
 
 extern "C" int fc_decode_layer_turn(const fc_kv_view* k_cache, const fc_kv_view* v_cache, const void* q, const void* k_new,
