@@ -549,6 +549,19 @@ def test_infinite_values_stay_infinite(dev, dtype, Hq, Hkv, wide, lens):
     assert bool(((got - ref)[..., rest].abs() <= torch.finfo(dtype).eps * ref[..., rest].abs() + 1e-5).all())
 
 
+def _launches(run, *names):
+    """Names of the launches of ``run`` that contain one of ``names``.  A profile now and then holds nothing: the next one is
+    asked, and that none holds any fails."""
+    for _ in range(8):
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
+            run()
+            torch.cuda.synchronize()
+        found = [e.name for e in prof.events() if any(n in e.name for n in names)]
+        if found:
+            return found
+    pytest.fail(f"no profile holds any of {names}")
+
+
 @pytest.mark.parametrize("Hq,Hkv,lens,plain,merges", [
     (14, 2, [700, 0, 255, 513], True, 0),         # columns of several ranges: their last workgroup merges
     (4, 2, [100, 256, 31], True, 0),              # one range a column
@@ -580,15 +593,9 @@ def test_bucket_graphs_hold_one_launch_per_layer(dev, Hq, Hkv, lens, plain, merg
                 context_lens=torch.tensor(lens, dtype=torch.int32, device=dev), block_tables=tables)
     try:
         got = []
-        for _ in range(6):        # a profile now and then holds nothing of a graph that ran in it
-            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
-                got.append(graphs.run(q, k, v).clone())
-                torch.cuda.synchronize()
-            names = [e.name for e in prof.events()]
-            if any("decode_column_kernel<" in n for n in names):
-                assert sum("decode_column_kernel<" in n for n in names) == L
-                assert sum("decode_merge_kernel" in n for n in names) == merges
-                break
+        names = _launches(lambda: got.append(graphs.run(q, k, v).clone()), "decode_column_kernel", "decode_attn_kernel", "decode_merge_kernel")
+        assert sum("decode_column_kernel" in n for n in names) == L and not any("decode_attn_kernel" in n for n in names)
+        assert sum("decode_merge_kernel" in n for n in names) == merges
         for _ in range(3):
             with torch.inference_mode():
                 graphs.graph_vars["outputs"].fill_(float("nan"))
@@ -674,14 +681,8 @@ def test_more_columns_than_compute_units(dev, dtype, Hq, Hkv, B, most, launches)
     q, k, v = q.to(dev), k.to(dev), v.to(dev)
     try:
         got = [layer(q, k, v).cpu()]
-        for _ in range(4):        # a profile now and then holds nothing
-            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
-                got.append(layer(q, k, v))
-                torch.cuda.synchronize()
-            names = [e.name for e in prof.events() if any(n in e.name for n in ("decode_", "store_slots"))]
-            if names:
-                assert len(names) == launches, names
-                break
+        names = _launches(lambda: got.append(layer(q, k, v)), "decode_", "store_slots")
+        assert len(names) == launches, names
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             held = layer(q, k, v)
@@ -778,19 +779,6 @@ def test_eager_calls_on_captured_layers_leave_the_graphs_counters_alone(dev):
         assert bool((arrivals == 0).all())
     finally:
         reset_context()
-
-
-def _launches(run, *names):
-    """Names of the launches of ``run`` that contain one of ``names``.  A profile now and then holds nothing: the next one is
-    asked, and that none holds any fails."""
-    for _ in range(8):
-        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
-            run()
-            torch.cuda.synchronize()
-        found = [e.name for e in prof.events() if any(n in e.name for n in names)]
-        if found:
-            return found
-    pytest.fail(f"no profile holds any of {names}")
 
 
 @pytest.mark.parametrize("Hq,Hkv,B,pages,column", [
