@@ -199,7 +199,8 @@ def refuse_capture() -> None:
 
 
 def upload_rows(rows, ref: torch.Tensor):
-    """Lists of Python ints as int32 tensors on the device of ``ref``: one copy, through pinned memory and without waiting."""
+    """Lists of Python ints as int32 tensors on the device of ``ref``: one upload, as a kernel's arguments or, above 3 KB, through
+    pinned memory, without waiting."""
     refuse_capture()
     return host().upload_tables([], tuple([r if type(r) is list else list(r) for r in rows]), ref)[1:]
 

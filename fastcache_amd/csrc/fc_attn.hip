@@ -3,8 +3,8 @@
 //
 // Attention is HBM-bound (one pass over K and V, ~1 FLOP per byte per query head), so the kernel is
 // organised around keeping loads in flight.  A workgroup owns one (sequence, kv head, chunk of
-// 256..1024 tokens, a multiple of 32 the host picks per launch) and serves all query heads of the group from the same K/V bytes; each of its four
-// wavefronts streams two 32-token K tiles and then the matching V tiles from global memory straight
+// 256..1024 tokens, a multiple of 32 the host picks per launch) and serves all query heads of the group from the same K/V bytes;
+// each of its four wavefronts streams its 32-token K tiles and then the matching V tiles from global memory straight
 // into a private two-stage LDS ring (global_load_lds, rows XOR-swizzled), 16 KB per wavefront in
 // flight, no workgroup barrier between a load and its use.
 //   phase 1  logits: one v_mfma_f32_32x32x16 block per tile, query heads as (zero-padded) rows;
@@ -12,9 +12,9 @@
 //   phase 3  sum of p * V rows from LDS: on the VALU, 8 output dims per lane, 16 partial sums folded through
 //            LDS; for 8 heads per workgroup on the matrix pipe with V read transposed from LDS (there an infinity in V
 //            gives NaN: the second half of its probability is zero or negative);
-// Each chunk writes (max, sum, unnormalised output) to the workspace; a second kernel merges the
-// chunks of a sequence.  Grid sizes depend only on the view's max_seq_len, never on the lengths on
-// the device, so both launches can be replayed from a graph while the lengths grow.
+// Each chunk writes (max, sum, unnormalised output) to the workspace and a second kernel merges the chunks of a sequence; where a
+// chunk holds every sequence whole, it writes the output itself.  Grid sizes depend only on the view's max_seq_len, never on the
+// lengths on the device, so the launches can be replayed from a graph while the lengths grow.
 #include <type_traits>
 #include "fc_common.h"
 #include <atomic>
@@ -83,7 +83,8 @@ struct DaAppend {                 // the step's new rows, one per sequence (k_ne
 // it back (true is returned), whichever sequence of the batch it belongs to (a table may be listed twice with lengths one
 // apart, or a page be shared): nobody depends on another workgroup's write.  The sequence's own row is also written by its last
 // workgroup, since it usually lies right behind the range.  Workgroups that write one row write the same bytes.
-// slot: of sequence `lane` (negative: none), TWO: slot2 of sequence 64 + `lane`, asked for with it, ktbl: table entry tbl0 + `lane` of sequence b; both planes use one table.
+// slot: of sequence `lane` (negative: none), TWO: slot2 of sequence 64 + `lane`, asked for with it, ktbl: table entry tbl0 + `lane`
+// of sequence b; both planes use one table.
 template <bool TWO>
 __device__ __forceinline__ bool da_append_rows(const KvView& kc, const KvView& vc, const DaAppend& ap, const char* kbase,
                                                const char* vbase, int slot, int slot2, int ktbl, int tbl0, int b, int h, int nb, int t0, int end,
@@ -522,7 +523,7 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 // A step of a few sequences is latency, not bandwidth: three users of 300 to 900 tokens move 3.4 MB a layer, and the
 // split kernel spent 11.3 us on it, the merge 3.3 and the append 1.9, each behind the one before (bf16, 28 query heads on
 // 4).  Here a workgroup of eight wavefronts owns a range of a (sequence, kv head) column, the whole context where that is
-// short: the wavefronts take the 32-token tiles in turn, K and V of the first tile (and K of the second) are requested
+// short: the wavefronts take the 32-token tiles in turn, K and V of a wavefront's first two tiles are requested
 // at once instead of K before V, every wavefront carries its own running softmax and no phase waits for the workgroup,
 // and the eight are merged through LDS.  The step's new K and V rows may be appended by the same workgroups (k_new).
 // The ranges of a column are merged by a launch of their own or (TURN) by the workgroup of the column that arrives last.
@@ -530,7 +531,8 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 //                           comes straight from memory; the lane then owns ONE head and 8 keys of the tile, so maxima
 //                           and sums run over its registers and two lane exchanges;
 //   O^T[dim][head] = V^T P^T: the probabilities are already the B operand (keys in the order the accumulator gives
-//                           them); V goes through the wavefront's 8 KB of LDS and is read transposed, 2 bytes at a time.
+//                           them); V goes straight to the wavefront's 16 KB of LDS, two tiles, and is read transposed by
+//                           the hardware (ds_read_b64_tr_b16).
 // Probabilities enter as a sum of 16-bit operands in the cache dtype: two for groups of 5 and more heads (as in the split
 // kernel), three for up to 4 heads, where the split kernel multiplies in fp32: three bf16 operands hold all 24 bits, three
 // fp16 operands all bits of a probability down to 2^-15, and what they drop is below 2^-39 of the tile's largest
