@@ -592,10 +592,17 @@ def test_bucket_graphs_hold_one_launch_per_layer(dev, Hq, Hkv, lens, plain, merg
     set_context(False, slot_mapping=torch.full((B,), -1, dtype=torch.int32, device=dev),
                 context_lens=torch.tensor(lens, dtype=torch.int32, device=dev), block_tables=tables)
     try:
-        got = []
-        names = _launches(lambda: got.append(graphs.run(q, k, v).clone()), "decode_column_kernel", "decode_attn_kernel", "decode_merge_kernel")
-        assert sum("decode_column_kernel" in n for n in names) == L and not any("decode_attn_kernel" in n for n in names)
-        assert sum("decode_merge_kernel" in n for n in names) == merges
+        got, kinds = [], ("decode_column_kernel", "decode_attn_kernel", "decode_merge_kernel")
+        step = torch.empty_like(q)                   # the calls a capture records, made eagerly
+        names = _launches(lambda: graphs._model(q, k, v, step), *kinds)
+        assert [sum(kind in n for n in names) for kind in kinds] == [L, 0, merges]
+        got.append(step)
+        for _ in range(3):        # and the graph's launches, of which a profile may hold nothing, but never others
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
+                got.append(graphs.run(q, k, v).clone())
+                torch.cuda.synchronize()
+            held = [sum(kind in e.name for e in prof.events()) for kind in kinds]
+            assert held[0] <= L and held[1] == 0 and held[2] <= merges
         for _ in range(3):
             with torch.inference_mode():
                 graphs.graph_vars["outputs"].fill_(float("nan"))
