@@ -818,3 +818,58 @@ def test_which_kernel_takes_columns_of_several_tiles(dev, Hq, Hkv, B, pages, col
         reset_context()
     assert ["decode_column_kernel<" in n for n in names] == [column]
     assert float((got.view(B, Hq, 128).float() - ref.float()).abs().max()) < 4e-3      # as above
+
+
+@pytest.mark.parametrize("Hq,Hkv,B", [(32, 32, 17), (32, 16, 33), (24, 8, 65)])     # 1, 2 and 3 heads a group; of 3, 768 tokens
+def test_whole_columns_are_summed_as_accurately_as_chunks(dev, Hq, Hkv, B):
+    """Columns that one workgroup holds whole, on values whose sums grow for half of the context and cancel in the other half,
+    so that the errors of the fp32 sums show in the rounded result.  A tile's products are summed by themselves: 0.54 to 0.60 of
+    the distance from 64 bits that fp32 sums of 256 tokens at a time, merged, have (0.82 to 1.0 as one sum over all tiles of a
+    wavefront, which on values that do not cancel is up to 1.1 of it); the bound lies between."""
+    from fastcache_amd.layers import Attention
+    from fastcache_amd.utils.context import reset_context, set_context
+    S = 768 if Hq // Hkv == 3 else 1024
+    lens, dtype, half = [S, S] + [8] * (B - 2), torch.float16, S // 2
+    case = synth.make_paged_case(seed=95, num_layers=1, batch=B, num_kv_heads=Hkv, seq_lens=[S, S] + [8] * (B - 2), dtype=dtype)
+    g = torch.Generator().manual_seed(4)
+    kd = torch.randn(2, S, Hkv, 128, generator=g).to(dtype)
+    kd[:, half:] = kd[:, :half]                                         # the second half weighs what the first does
+    vd = torch.empty(2, S, Hkv, 128, dtype=dtype)
+    vd[:, :half] = (torch.randn(2, half, Hkv, 128, generator=g) * 256).to(dtype)
+    vd[:, half:] = -vd[:, :half] + (0.25 * torch.randint(-1, 2, (2, half, Hkv, 128), generator=g)).to(dtype)
+    pool = case.kv_cache[:, 0]
+    for b in range(2):
+        for t in range(0, S, 256):
+            pool[0, case.block_tables[b][t // 256]], pool[1, case.block_tables[b][t // 256]] = kd[b, t:t + 256], vd[b, t:t + 256]
+    q, k, v = ((torch.randn(B, h * 128, generator=g) * 0.5).to(dtype) for h in (Hq, Hkv, Hkv))
+    layer, on_gpu = Attention(Hq, 128, 128 ** -0.5, Hkv), pool.to(dev)
+    layer.k_cache, layer.v_cache = on_gpu[0], on_gpu[1]
+    set_context(False, slot_mapping=torch.full((B,), -1, dtype=torch.int32, device=dev),
+                context_lens=torch.tensor(lens, dtype=torch.int32, device=dev), block_tables=case.table_tensor(dev))
+    q_d, k_d, v_d = q.to(dev), k.to(dev), v.to(dev)
+    try:
+        got = layer(q_d, k_d, v_d).cpu()[:2].view(2, Hkv, Hq // Hkv, 128).double()
+        names = _launches(lambda: layer(q_d, k_d, v_d), "decode_")
+    finally:
+        reset_context()
+    assert len(names) == 1 and "decode_attn_kernel" in names[0]
+    logits = torch.matmul(q[:2].view(2, Hkv, Hq // Hkv, 128).double(), kd.permute(0, 2, 3, 1).contiguous().double()) * 128 ** -0.5
+    p64 = logits.softmax(-1)
+    exact = torch.matmul(p64, vd.permute(0, 2, 1, 3).contiguous().double())
+    e = (logits - logits.amax(-1, keepdim=True)).exp().float()           # chunks of 256: one sum a token slot of 16, then those
+    acc = torch.zeros(2, Hkv, Hq // Hkv, 128)
+    for c in range(0, S, 256):
+        slots = torch.zeros(16, 2, Hkv, Hq // Hkv, 128)
+        for t in range(256):
+            s = (t // 32 % 4) * 4 + t % 4
+            slots[s] = (slots[s].double() + e[..., c + t, None].double() * vd[:, c + t, :, None].double()).float()       # one rounding
+        part = torch.zeros_like(acc)
+        for s in slots:
+            part += s
+        acc += part
+    chunks = (acc / e.double().sum(-1, keepdim=True).float()).to(dtype).double()
+    err, ref = float((got - exact).norm()), float((chunks - exact).norm())
+    # what rounding the result leaves is the same for all: the rest of the errors is compared
+    last = float((exact.to(dtype).double() - exact).norm()) ** 2
+    ratio = ((err ** 2 - last) / (ref ** 2 - last)) ** 0.5
+    assert ratio < 0.7, ratio
