@@ -73,6 +73,11 @@ class BatchedGEMMCompressor(nn.Module):
         w = hit[1]
         return w if layers is None else tuple(t[layers[0]:layers[1]] for t in w)
 
+    def _plane_weights(self, seg: str, ref: torch.Tensor, layers: Tuple[int, int]):
+        """What ``ops.ccm_mlp_planes`` takes for the weights of (K, V): a function of the plane, and whether both are packed."""
+        return (lambda p: self._weights(seg + "kv"[p], ref.dtype, ref.device, layers),
+                all(seg + kind in self._packed for kind in "kv"))
+
     # -- segments ---------------------------------------------------------------------------------
     def _seg_len(self, n: int) -> int:
         c = n // self.compression_factor
@@ -101,8 +106,7 @@ class BatchedGEMMCompressor(nn.Module):
                 for p in range(2):
                     ops.copy_tokens(sv[p], dv[p], seg_start, n, dst)
             else:
-                w = [self._weights(seg + kind, k0.dtype, k0.device, (l0, l1)) for kind in "kv"]
-                ops.ccm_mlp_planes(sv, dv, w, cf, seg_start, n, dst)
+                ops.ccm_mlp_planes(sv, dv, *self._plane_weights(seg, k0, (l0, l1)), cf, seg_start, n, dst)
             dst += self._seg_len(n)
         return [(out[0][i], out[1][i]) for i in range(L)]
 
@@ -126,7 +130,6 @@ class BatchedGEMMCompressor(nn.Module):
         views = [_lib.paged_view(kv_cache[p][l0:l1], block_tables, seq_lens, seq_len) for p in range(2)]
         dviews = views if out is None else [_lib.dense_view(out[p][l0:l1]) for p in range(2)]
         if host_lens is not None and len(set(host_lens)) > 1:
-            dev = kv_cache.device
             imgs = [min(int(it_len[0]), n) if it_len[0] > 0 else 0 for n in host_lens]
             dsts = [0] * len(imgs)
             plan = []      # all uploads before the first launch: one that is refused leaves the cache as it was
@@ -139,11 +142,11 @@ class BatchedGEMMCompressor(nn.Module):
                 plan.append((seg, max(counts), [xs[0] for xs in where] if same else _lib.upload_rows(where, kv_cache), same))
                 dsts = [d + self._seg_len(n) for d, n in zip(dsts, counts)]
             for seg, n_max, (st, ct, dt), same in plan:
-                w = [self._weights(seg + kind, kv_cache.dtype, dev, (l0, l1)) for kind in "kv"]
+                w = self._plane_weights(seg, kv_cache, (l0, l1))
                 if same:
-                    ops.ccm_mlp_planes(views, dviews, w, cf, st, ct, dt)
+                    ops.ccm_mlp_planes(views, dviews, *w, cf, st, ct, dt)
                 else:
-                    ops.ccm_mlp_planes_ragged(views, dviews, w, cf, st, ct, dt, n_max, self.min_seq_len)
+                    ops.ccm_mlp_planes_ragged(views, dviews, *w, cf, st, ct, dt, n_max, self.min_seq_len)
             return dsts
         for s0, n, seg in ((0, img, "i"), (img, seq_len - img, "t")):
             if n == 0:
@@ -153,8 +156,7 @@ class BatchedGEMMCompressor(nn.Module):
                     for view, dview in zip(views, dviews):
                         ops.copy_tokens(view, dview, s0, n, dst)
             else:
-                w = [self._weights(seg + kind, kv_cache.dtype, kv_cache.device, (l0, l1)) for kind in "kv"]
-                ops.ccm_mlp_planes(views, dviews, w, cf, s0, n, dst)
+                ops.ccm_mlp_planes(views, dviews, *self._plane_weights(seg, kv_cache, (l0, l1)), cf, s0, n, dst)
             dst += self._seg_len(n)
         return dst
 

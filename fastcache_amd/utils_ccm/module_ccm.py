@@ -128,6 +128,11 @@ class _CCMBase(nn.Module):
         w = self._weights(group, dtype, device)
         return w if (l0, l1) == (0, w[0].shape[0]) else tuple(t[l0:l1] for t in w)
 
+    def _plane_weights(self, groups, l0: int, l1: int, kv_cache: torch.Tensor):
+        """What ``ops.ccm_mlp_planes`` takes for the weights of (K, V): a function of the plane, and whether both are packed."""
+        return (lambda p: self._layer_weights(groups[p], l0, l1, kv_cache.dtype, kv_cache.device),
+                all(g in self._stacked for g in groups))
+
     def _apply(self, fn, *a, **kw):  # .cuda() / .half() invalidate the stacked copies
         self._stacked = {}
         return super()._apply(fn, *a, **kw)
@@ -207,8 +212,7 @@ class _CCMBase(nn.Module):
                     for view, dview in zip(views, dviews):
                         ops.copy_tokens(view, dview, s0, n, dst)
             else:
-                w = [self._layer_weights(g, l0, l1, kv_cache.dtype, kv_cache.device) for g in (gk, gv)]
-                ops.ccm_mlp_planes(views, dviews, w, cf, s0, n, dst)
+                ops.ccm_mlp_planes(views, dviews, *self._plane_weights((gk, gv), l0, l1, kv_cache), cf, s0, n, dst)
             dst += self._segment_len(n)
         return dst
 
@@ -218,7 +222,6 @@ class _CCMBase(nn.Module):
         same for all of them (the image in front of texts of different lengths) is the uniform call, whose launch need
         not provide for different lengths (20 sequences of 32 layers x 32 heads x 576 tokens, factor 2: 880 us, 950)."""
         cf, (l0, l1) = self.compression_factor, layer_range
-        dev = kv_cache.device
         by_len = {n: self._paged_segments(n, it_len) for n in set(lens)}
         per_seq = [by_len[n] for n in lens]
         dst = [0] * len(lens)
@@ -236,11 +239,11 @@ class _CCMBase(nn.Module):
             plan.append((gk, gv, n_max, [xs[0] for xs in where] if same else _lib.upload_rows(where, kv_cache), same))
             dst = [d + self._segment_len(g[3]) for d, g in zip(dst, segs)]
         for gk, gv, n_max, (starts, counts, dsts), same in plan:
-            w = [self._layer_weights(g, l0, l1, kv_cache.dtype, dev) for g in (gk, gv)]
+            w = self._plane_weights((gk, gv), l0, l1, kv_cache)
             if same:
-                ops.ccm_mlp_planes(views, dviews, w, cf, starts, counts, dsts)
+                ops.ccm_mlp_planes(views, dviews, *w, cf, starts, counts, dsts)
             else:
-                ops.ccm_mlp_planes_ragged(views, dviews, w, cf, starts, counts, dsts, n_max, self.min_seq_len)
+                ops.ccm_mlp_planes_ragged(views, dviews, *w, cf, starts, counts, dsts, n_max, self.min_seq_len)
         return dst
 
     def _forward_layers(self, kv_cache: Sequence[LayerKV], segments) -> Optional[List[LayerKV]]:

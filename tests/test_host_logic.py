@@ -649,3 +649,32 @@ def test_a_layer_saved_without_counters_reaches_its_decode_step(monkeypatch):
         assert layer(q, q, q) is q and calls[0][-1] is None
     finally:
         reset_context()
+
+
+@pytest.mark.parametrize("batched", [True, False])
+@pytest.mark.parametrize("lens", [[90, 90], [90, 41]])
+def test_a_first_pass_launches_k_before_it_packs_v(monkeypatch, batched, lens):
+    """Weights that are not packed yet: K's launch goes out before V's weights are packed, per segment; with both at hand the
+    planes are one launch."""
+    from types import SimpleNamespace
+    from fastcache_amd import _lib, ops
+    from fastcache_amd.utils_ccm import KVCacheLinearDecoupleCompressor
+    cfg = SimpleNamespace(text_config=SimpleNamespace(num_hidden_layers=2, num_key_value_heads=1, hidden_size=128))
+    comp = KVCacheLinearDecoupleCompressor(cfg, compression_factor=2).eval()
+    if batched:
+        orig, comp = comp, BatchedGEMMCompressor(num_layers=2, num_heads=1, head_dim=128, compression_factor=2)
+        comp.load_from_original_compressor(orig)
+    events, inner = [], comp._weights
+    monkeypatch.setattr(comp, "_weights", lambda g, *a: (events.append("pack" if g not in packed else "hit"), packed.add(g), inner(g, *a))[2])
+    packed = set()
+    monkeypatch.setattr(_lib, "paged_view", lambda *a: _lib.FcKvView(num_layers=2))
+    monkeypatch.setattr(_lib, "upload_rows", lambda rows, ref: tuple(rows))
+    for name in ("ccm_mlp", "ccm_mlp_ragged", "ccm_mlp_kv", "ccm_mlp_kv_ragged"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name: events.append("both" if "_kv" in name else "plane"))
+    pool = torch.zeros(2, 2, 1, 256, 1, 128)
+    args = (pool, None, None, max(lens), [41, max(lens) - 41])
+    comp.paged_forward(*args, host_lens=lens)
+    assert events == ["pack", "plane", "pack", "plane"] * 2
+    events.clear()
+    comp.paged_forward(*args, host_lens=lens)
+    assert events == ["hit", "hit", "both"] * 2
