@@ -76,7 +76,7 @@ class BatchedGEMMCompressor(nn.Module):
     def _plane_weights(self, seg: str, ref: torch.Tensor, layers: Tuple[int, int]):
         """What ``ops.ccm_mlp_planes`` takes for the weights of (K, V): a function of the plane, and whether both are packed."""
         return (lambda p: self._weights(seg + "kv"[p], ref.dtype, ref.device, layers),
-                all(seg + kind in self._packed for kind in "kv"))
+                seg + "k" in self._packed and seg + "v" in self._packed)
 
     # -- segments ---------------------------------------------------------------------------------
     def _seg_len(self, n: int) -> int:

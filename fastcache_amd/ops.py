@@ -481,15 +481,15 @@ def ccm_mlp_kv_ragged(srcs, dsts, weights, cf: int, seg_start: torch.Tensor, seg
           "fc_ccm_mlp_kv_ragged")
 
 
-def _planes_alike(views) -> bool:
-    """Whether the views of two planes differ in their place only (``base``, the first field)."""
-    return bytes(views[0])[8:] == bytes(views[1])[8:]
+def _planes_alike(srcs, dsts) -> bool:
+    """Whether the views of two planes differ in their place only (``base``, the first field); in place they are one pool's."""
+    return srcs is dsts or all(bytes(k)[8:] == bytes(v)[8:] for k, v in (srcs, dsts))
 
 
 def ccm_mlp_planes(srcs, dsts, weights, packed: bool, cf: int, seg_start: int, seg_len: int, dst_start: int) -> None:
     """``ccm_mlp_kv``, or a call per plane: for planes of different strides or lengths (outputs that are tensors apart), and
     where the weights are not ``packed`` yet, V's of which are made while K's launch runs.  ``weights``: a function of the plane."""
-    if packed and _planes_alike(srcs) and _planes_alike(dsts):
+    if packed and _planes_alike(srcs, dsts):
         ccm_mlp_kv(srcs, dsts, [weights(p) for p in range(2)], cf, seg_start, seg_len, dst_start)
     else:
         for p in range(2):
@@ -499,7 +499,7 @@ def ccm_mlp_planes(srcs, dsts, weights, packed: bool, cf: int, seg_start: int, s
 def ccm_mlp_planes_ragged(srcs, dsts, weights, packed: bool, cf: int, seg_start: torch.Tensor, seg_len: torch.Tensor,
                           dst_start: torch.Tensor, max_seg_len: int, min_rows: int) -> None:
     """``ccm_mlp_kv_ragged``, or a call per plane, as ``ccm_mlp_planes``."""
-    if packed and _planes_alike(srcs) and _planes_alike(dsts):
+    if packed and _planes_alike(srcs, dsts):
         ccm_mlp_kv_ragged(srcs, dsts, [weights(p) for p in range(2)], cf, seg_start, seg_len, dst_start, max_seg_len, min_rows)
     else:
         for p in range(2):

@@ -131,7 +131,7 @@ class _CCMBase(nn.Module):
     def _plane_weights(self, groups, l0: int, l1: int, kv_cache: torch.Tensor):
         """What ``ops.ccm_mlp_planes`` takes for the weights of (K, V): a function of the plane, and whether both are packed."""
         return (lambda p: self._layer_weights(groups[p], l0, l1, kv_cache.dtype, kv_cache.device),
-                all(g in self._stacked for g in groups))
+                groups[0] in self._stacked and groups[1] in self._stacked)
 
     def _apply(self, fn, *a, **kw):  # .cuda() / .half() invalidate the stacked copies
         self._stacked = {}
