@@ -447,7 +447,8 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
     for (int i = nj; i < 2 * nj; ++i) {
       wait_item(i);
       // Of whole columns a tile's products are summed by themselves: one chain of 64 of them was further from 64 bits than chunks of
-      // 256 tokens merged (1024 tokens of 1 head a group, logits of deviation 1 / 3: 1.09 to 1.10 / 1.03 to 1.04 of their error, now 0.98 / 1.00).
+      // 256 tokens merged (1024 tokens of 1 head a group, logits of deviation 1 / 3: 1.09 to 1.10 / 1.03 to 1.04 of their error,
+      // now 0.98 / 1.00).
       if constexpr (WHOLE) {
         float own[GT][8] = {};
         pv(wave + 4 * (i - nj), i & 1, own);
