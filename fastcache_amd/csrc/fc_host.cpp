@@ -340,7 +340,9 @@ PyObject* py_snapkv_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::Tensor ok = at::empty({B, H, n, D}, k.options()), ov = at::empty({B, H, n, D}, k.options());
     const fc_kv_view kv = dense_view(k, 1, 0), vv = dense_view(v, 1, 0), dk = dense_view(ok, 1, 0), dv = dense_view(ov, 1, 0);
     const int32_t nsplit = fc_snapkv_select_splits(&kv, (int32_t)hq, (int32_t)W);
-    const int64_t bytes = fc_snapkv_select_workspace_bytes(1, (int32_t)B, (int32_t)hq, (int32_t)H, (int32_t)W, (int32_t)S, nsplit);
+    const int64_t bytes = !lse && fc_snapkv_once_pays(&kv, (int32_t)hq, (int32_t)W, (int32_t)S)
+                              ? std::max(fc_snapkv_once_workspace_bytes(&kv, (int32_t)hq, (int32_t)W), B * H * S * 4)
+                              : fc_snapkv_select_workspace_bytes(1, (int32_t)B, (int32_t)hq, (int32_t)H, (int32_t)W, (int32_t)S, nsplit);
     at::Tensor ws = at::empty({bytes}, k.options().dtype(at::kByte));
     const at::Tensor idx = gather_apart(k, n);
     check(fc_snapkv_press_into(&kv, &vv, &dk, &dv, q.const_data_ptr(), lse, (int32_t)hq, (int32_t)W, (int32_t)ksz,
@@ -784,7 +786,7 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::Tensor q;
     int64_t W = 0, ksz = 0, causal = 0, hq = 0;
     int32_t nsplit = 1;
-    bool one = true;
+    bool one = true, once = false;
     double scale = 0, out_scale = 0;
     const bool norms_apart = args[7] == Py_False;
     if (args[7] != Py_None && !norms_apart) {
@@ -804,7 +806,8 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       hq = q.size(2);
       nsplit = fc_snapkv_rows_route(&kv, (int32_t)hq, (int32_t)W, fits, (int32_t)as_int(item(7)));
       if (nsplit < 0) Py_RETURN_NONE;
-      one = nsplit == 0;
+      once = fc_snapkv_once_pays(&kv, (int32_t)hq, (int32_t)W, (int32_t)as_int(item(7))) != 0;
+      one = nsplit == 0 && !once;
     }
     const int32_t *counts = nullptr, *order = nullptr;
     at::Tensor numbers;      // kept until the launches are enqueued
@@ -826,10 +829,15 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     void* stream = stream_of(pool);
     const int64_t idx_bytes = cols * width * 4;
     if (!one) {
-      const int64_t ws = fc_snapkv_select_workspace_bytes((int32_t)L, (int32_t)B, (int32_t)hq, (int32_t)H, (int32_t)W, (int32_t)S, nsplit);
+      const int64_t ws = once ? fc_snapkv_once_workspace_bytes(&kv, (int32_t)hq, (int32_t)W)
+                              : fc_snapkv_select_workspace_bytes((int32_t)L, (int32_t)B, (int32_t)hq, (int32_t)H, (int32_t)W, (int32_t)S, nsplit);
       Scratch mem(Scratch::room(idx_bytes) + ws, pool);
       int32_t* idx = (int32_t*)mem.take(idx_bytes);
-      check(fc_snapkv_select(&kv, q.const_data_ptr(), nullptr, (int32_t)hq, (int32_t)W, (int32_t)ksz, (int32_t)causal,
+      if (once)
+        check(fc_snapkv_select_once(&kv, q.const_data_ptr(), (int32_t)hq, (int32_t)W, (int32_t)ksz, (int32_t)causal, (float)scale,
+                                    (float)out_scale, (int32_t)width, counts, idx, (int32_t)width, 0, mem.take(ws), ws, stream),
+              "fc_snapkv_select_once");
+      else check(fc_snapkv_select(&kv, q.const_data_ptr(), nullptr, (int32_t)hq, (int32_t)W, (int32_t)ksz, (int32_t)causal,
                              (float)scale, (float)out_scale, (int32_t)width, counts, idx, (int32_t)width, nsplit,
                              mem.take(ws), ws, stream),
             "fc_snapkv_select");

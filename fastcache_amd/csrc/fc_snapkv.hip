@@ -30,6 +30,7 @@
 //
 // Table entries of a live sequence must be allocated blocks: a negative entry inside the sequence
 // reads block 0 instead of faulting.
+#include "fc_once.h"
 #include "fc_press.h"
 #include "fc_tail.h"
 
@@ -1062,8 +1063,78 @@ extern "C" int64_t fc_snapkv_select_workspace_bytes(int32_t num_layers, int32_t 
   return fc_snapkv_split_workspace_bytes(num_layers, batch, num_q_heads, num_kv_heads, window, max_seq_len, nsplit);
 }
 
+extern "C" int32_t fc_snapkv_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len) {
+  return fc_once_pays(keys, num_q_heads, window, mean_len) ? 1 : 0;
+}
+
+static int64_t sk_once_room(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) {   // the per-key sums
+  return ((int64_t)fc_once_groups(keys, num_q_heads, window) * keys->num_layers * keys->batch * keys->num_kv_heads *
+              keys->max_seq_len * (int64_t)sizeof(float) + 255) / 256 * 256;
+}
+
+extern "C" int64_t fc_snapkv_once_workspace_bytes(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) {
+  if (!fc_once_takes(keys, num_q_heads, window)) return -1;
+  return sk_once_room(keys, num_q_heads, window) +
+         fc_once_workspace_bytes(keys->num_layers, keys->batch, num_q_heads, keys->num_kv_heads, window, keys->max_seq_len);
+}
+
+// Every logit formed once (fc_once.hip), then the selection.  The views are checked, a.k, a.n_kept and a.index_stride as well.
+static int snapkv_once_impl(const char* who, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                            const fc_kv_view* out_v, const void* queries, int32_t num_q_heads, int32_t window,
+                            int32_t kernel_size, int32_t causal_window, float scale, ColumnSelect a, int32_t workgroups,
+                            void* workspace, int64_t workspace_bytes, void* stream) {
+  FC_REQUIRE(queries && workspace, FC_EINVAL, "%s: null pointer", who);
+  FC_REQUIRE(((uintptr_t)queries & 15) == 0 && ((uintptr_t)workspace & 15) == 0, FC_EINVAL,
+             "%s: queries / workspace not 16-byte aligned", who);
+  FC_REQUIRE(num_q_heads > 0 && num_q_heads % keys->num_kv_heads == 0, FC_EINVAL,
+             "%s: num_q_heads %d not a multiple of num_kv_heads %d", who, num_q_heads, keys->num_kv_heads);
+  FC_REQUIRE(window > 0, FC_EINVAL, "%s: window must be positive", who);
+  FC_REQUIRE(kernel_size >= 1 && (kernel_size & 1) && kernel_size <= 63, FC_EINVAL,
+             "%s: kernel_size %d must be odd and <= 63", who, kernel_size);
+  FC_REQUIRE(workgroups >= 0, FC_EINVAL, "%s: workgroups %d", who, workgroups);
+  const int64_t need = fc_snapkv_once_workspace_bytes(keys, num_q_heads, window);
+  FC_REQUIRE(need >= 0, FC_EUNSUPPORTED,
+             "%s: fp16/bf16 caches of at most %d tokens, at most 16 blocks of 32 window queries per kv head, pages of 64*2^n "
+             "tokens or a dense view", who, SO_CHUNKS_MAX * SO_KEYS);
+  FC_REQUIRE(workspace_bytes >= need, FC_EINVAL, "%s: workspace of %lld bytes, %lld needed", who, (long long)workspace_bytes,
+             (long long)need);
+  const int rc = fc_once_sums(who, keys, queries, num_q_heads, window, causal_window, scale, (float*)workspace, keys->max_seq_len,
+                              (char*)workspace + sk_once_room(keys, num_q_heads, window), workgroups, stream);
+  if (rc) return rc;
+  a.in = (const float*)workspace;
+  a.addends = fc_once_groups(keys, num_q_heads, window);
+  a.addend_stride = (long long)keys->num_layers * keys->batch * keys->num_kv_heads * keys->max_seq_len;
+  return fc_column_select(who, CS_SUMS, keys, values, out_k, out_v, a, (hipStream_t)stream);
+}
+
+extern "C" int fc_snapkv_select_once(const fc_kv_view* keys, const void* queries, int32_t num_q_heads, int32_t window,
+                                     int32_t kernel_size, int32_t causal_window, float scale, float out_scale, int32_t k,
+                                     const int32_t* n_kept, int32_t* indices, int32_t index_stride, int32_t workgroups,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* who = "fc_snapkv_select_once";
+  const int rc = fc_check_view(keys, who);
+  if (rc) return rc;
+  FC_REQUIRE(indices && index_stride >= 0 && index_stride <= keys->max_seq_len, FC_EINVAL, "%s: null indices or index_stride %d",
+             who, index_stride);
+  FC_REQUIRE(n_kept || (k > window && k <= index_stride), FC_EINVAL, "%s: k=%d must exceed the window (%d) and fit %d", who, k,
+             window, index_stride);
+  if (keys->max_seq_len == 0) return FC_OK;
+  ColumnSelect a{};
+  a.stride = keys->max_seq_len;
+  a.k = k;
+  a.n_kept = n_kept;
+  a.window = window;
+  a.ksz = kernel_size;
+  a.out_mul = out_scale / (float)kernel_size;
+  a.indices = indices;
+  a.index_stride = index_stride;
+  return snapkv_once_impl(who, keys, keys, nullptr, nullptr, queries, num_q_heads, window, kernel_size, causal_window, scale, a,
+                          workgroups, workspace, workspace_bytes, stream);
+}
+
 // Scores every column (split over nsplit workgroups, or whole with nsplit 1) into the workspace, then selects: the
-// window and the k - window best of the other keys.
+// window and the k - window best of the other keys.  A hook (out_k given) whose workspace has the room takes one pass over the
+// keys where that is faster.
 static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
                               const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
                               int32_t window, int32_t kernel_size, int32_t causal_window, float scale, float out_scale,
@@ -1086,6 +1157,10 @@ static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_
   a.indices = indices;
   a.index_stride = index_stride;
   a.parts = out_k && !indices ? fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, keys->max_seq_len, k) : 0;
+  if (out_k && !lse && num_q_heads > 0 && num_q_heads % keys->num_kv_heads == 0 && fc_once_pays(keys, num_q_heads, window, stride) &&
+      workspace_bytes >= fc_snapkv_once_workspace_bytes(keys, num_q_heads, window))
+    return snapkv_once_impl(who, keys, values, out_k, out_v, queries, num_q_heads, window, kernel_size, causal_window, scale, a, 0,
+                            workspace, workspace_bytes, stream);
   if (nsplit > 1) {
     const float* raw = nullptr;
     if ((rc = snapkv_split_sums(who, keys, queries, lse, num_q_heads, window, kernel_size, causal_window, scale, stride,

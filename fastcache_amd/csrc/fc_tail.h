@@ -6,6 +6,8 @@
 struct ColumnSelect {
   const float* in;      // [layer][batch][kv head][stride]: scores (SRC 0) or per-key sums (SRC 1)
   int stride;
+  int addends;          // arrays of sums (SRC 1) that are added, addend_stride floats apart (0: one)
+  long long addend_stride;
   int k;                // kept positions per row when n_kept is null
   const int* n_kept;    // [batch] in device memory, or null
   int window;           // the last `window` positions of a sequence are kept and not entered (0: all are entered)

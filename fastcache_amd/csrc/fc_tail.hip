@@ -105,6 +105,10 @@ __global__ __launch_bounds__(THREADS, KPT > 16 ? 4 : 1) void column_select_kerne
       auto fetch = [&](int e0) {
 #pragma unroll
         for (int g = 0; g <= G; ++g) v[g] = in[min(max(sg.beg + (e0 + g) * 64 - hw + lane, 0), n - 1)];
+        for (int q = 1; q < a.addends; ++q) {
+#pragma unroll
+          for (int g = 0; g <= G; ++g) v[g] += in[q * a.addend_stride + min(max(sg.beg + (e0 + g) * 64 - hw + lane, 0), n - 1)];
+        }
       };
       fetch(0);
 #pragma unroll

@@ -200,7 +200,8 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     tensor is passed through unchecked for callers that have validated the counts themselves.
 
     ``rows_only``: for callers that want the moved rows alone; scores and indices stay scratch (no window fill, no
-    padding of the index rows) and None is returned."""
+    padding of the index rows) and None is returned.  One pass over the keys, selection and compaction take the one launch's
+    place where they are faster (:func:`snapkv_once_pays`)."""
     order = None
     if n_kept is not None and not isinstance(n_kept, torch.Tensor):
         counts = [int(c) for c in n_kept]
@@ -235,6 +236,12 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     dev = queries.device
+    if rows_only and lse is None and values is not None:
+        mean = keys.max_seq_len if host_lens is None else sum(host_lens) // len(host_lens)
+        if snapkv_once_pays(keys, Hq, window, mean):
+            idx = _select_once(keys, queries, kernel_size, k, causal_window, scale, out_scale, _i32(n_kept, "n_kept", dev), 0)
+            compact(keys, values, keys, values, idx, n_kept=n_kept)
+            return None
     stride = keys.max_seq_len
     scores = torch.empty((L, B, H, stride), dtype=torch.float32, device=dev)
     row_max = torch.empty((L, B, H), dtype=torch.float32, device=dev)
@@ -271,13 +278,32 @@ def snapkv_rows_route(keys: FcKvView, num_q_heads: int, window: int, fits: bool,
     return int(fn("fc_snapkv_rows_route")(C.byref(keys), num_q_heads, window, int(fits), mean_len))
 
 
+def snapkv_once_pays(keys: FcKvView, num_q_heads: int, window: int, mean_len: int) -> bool:
+    """Whether scoring in one pass over the keys, then selection and compaction, is the fastest press of sequences of that
+    mean length (the rule and its measurements stand at ``fc_once_pays``)."""
+    return bool(fn("fc_snapkv_once_pays")(C.byref(keys), num_q_heads, window, mean_len))
+
+
+def _select_once(keys, queries, kernel_size, k, causal_window, scale, out_scale, n_kept, workgroups):
+    L, B, Hq, W, _ = queries.shape
+    nbytes = int(fn("fc_snapkv_once_workspace_bytes")(C.byref(keys), Hq, W))
+    ws = torch.empty(max(nbytes, 0), dtype=torch.uint8, device=queries.device)
+    idx = torch.empty((L, B, keys.num_kv_heads, k), dtype=torch.int32, device=queries.device)
+    check(fn("fc_snapkv_select_once")(C.byref(keys), queries.data_ptr(), Hq, W, kernel_size, int(causal_window), scale, out_scale, k,
+                                      ptr(n_kept), idx.data_ptr(), k, workgroups, ws.data_ptr(), nbytes, current_stream()),
+          "fc_snapkv_select_once")
+    return idx
+
+
 def snapkv_select(keys: FcKvView, queries: torch.Tensor, window: int, kernel_size: int, k: int,
                   causal_window: bool = True, reduction: str = "mean", scale: Optional[float] = None,
                   lse: Optional[torch.Tensor] = None, n_kept: Optional[torch.Tensor] = None,
-                  splits: Optional[int] = None) -> torch.Tensor:
+                  splits: Optional[int] = None, mean_len: Optional[int] = None,
+                  workgroups: Optional[int] = None) -> torch.Tensor:
     """The indices ``snapkv_score`` + ``topk_select`` give for counts above the window, without a score tensor:
     int32 ``[L, B, Hkv, k]`` (entries past a row's count ``n_kept[b]`` are left as they are).  ``splits``: key ranges per
-    column; default :func:`snapkv_select_splits`."""
+    column; default :func:`snapkv_select_splits`.  With ``mean_len`` (the sequences' mean length) one pass over the keys is
+    taken instead where it pays, with ``workgroups`` (at most so many, 0 for the usual number) in any case."""
     queries = queries.contiguous()
     _lib.require_gpu(queries, "queries")
     L, B, Hq, W, D = queries.shape
@@ -295,6 +321,11 @@ def snapkv_select(keys: FcKvView, queries: torch.Tensor, window: int, kernel_siz
             raise FastcacheError(f"lse must be fp32 [L={L}, B={B}, Hq={Hq}, W={W}], got {lse.dtype} {tuple(lse.shape)}")
         lse = lse.contiguous()
     n_kept = _i32(n_kept, "n_kept", dev)
+    if workgroups is not None or (mean_len is not None and lse is None and snapkv_once_pays(keys, Hq, W, mean_len)):
+        if lse is not None:
+            raise FastcacheError("one pass over the keys forms the log-sum-exp itself")
+        return _select_once(keys, queries, kernel_size, k, causal_window, 1.0 / math.sqrt(D) if scale is None else scale,
+                            1.0 / (W * (Hq // H)) if reduction == "mean" else 1.0, n_kept, workgroups or 0)
     nsplit = snapkv_select_splits(keys, Hq, W) if splits is None else splits
     nbytes = int(fn("fc_snapkv_select_workspace_bytes")(L, B, Hq, H, W, S, nsplit))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)

@@ -227,6 +227,17 @@ int fc_snapkv_select(const fc_kv_view* keys, const void* queries, const float* l
                      int32_t window, int32_t kernel_size, int32_t causal_window, float scale, float out_scale,
                      int32_t k, const int32_t* n_kept, int32_t* indices, int32_t index_stride, int32_t nsplit,
                      void* workspace, int64_t workspace_bytes, void* stream);
+/* The same selection with one pass over the keys (the exponentials wait in registers for the queries' totals) for sequences of
+ * up to 12 288 tokens and up to 16 blocks of 32 window queries per kv head.  fc_snapkv_once_pays: 1 where that is faster than
+ * what the two functions above lead to, for sequences of that mean length; workspace: fc_snapkv_once_workspace_bytes, -1 where
+ * the shape is not taken.  workgroups: at most so many, 0 for two per compute unit.  fc_snapkv_press_into does it by itself
+ * where it pays and its workspace has that room. */
+int32_t fc_snapkv_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len);
+int64_t fc_snapkv_once_workspace_bytes(const fc_kv_view* keys, int32_t num_q_heads, int32_t window);
+int fc_snapkv_select_once(const fc_kv_view* keys, const void* queries, int32_t num_q_heads, int32_t window,
+                          int32_t kernel_size, int32_t causal_window, float scale, float out_scale, int32_t k,
+                          const int32_t* n_kept, int32_t* indices, int32_t index_stride, int32_t workgroups,
+                          void* workspace, int64_t workspace_bytes, void* stream);
 int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
                          const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
                          int32_t window, int32_t kernel_size, int32_t causal_window, float scale, float out_scale,

@@ -86,6 +86,47 @@ def test_one_launch_presses_validate_on_the_host():
     assert press(*args(f32, f32, 100, 100)) == -2 and b"fp16/bf16" in err()
 
 
+def test_select_in_one_pass_validates_on_the_host():
+    """fc_snapkv_select_once refuses what it cannot take before any launch, fc_snapkv_once_workspace_bytes says so."""
+    err = lambda: _lib.fn("fc_last_error")()
+    B, call, room = ctypes.byref, _lib.fn("fc_snapkv_select_once"), _lib.fn("fc_snapkv_once_workspace_bytes")
+    k = _dense_view(1024)
+    need = room(B(k), 8, 64)
+    args = lambda v=k, q=16, hq=8, W=64, ksz=7, keep=100, wgs=0, ws=16, nbytes=need: call(
+        B(v), q, hq, W, ksz, 1, 0.1, 1.0, keep, None, 16, keep, wgs, ws, nbytes, None)
+    assert need > 0 and args(nbytes=need - 1) == -1 and b"workspace" in err()
+    assert args(q=None) == -1 and args(q=24) == -1 and args(hq=7, keep=200) in (-1, -2) and args(ksz=4) == -1
+    assert args(keep=64) == -1 and b"exceed the window" in err()
+    assert args(wgs=-1) == -1 and b"workgroups" in err()
+    long, f32 = _dense_view(12289), _dense_view(1024, dtype=0)
+    for v, hq, W in ((long, 8, 64), (f32, 8, 64), (k, 8, 64 * 40)):
+        assert room(B(v), hq, W) == -1
+    assert args(v=long) == -2 and args(v=f32) == -2
+
+
+def test_one_pass_pays_where_it_can_run():
+    """The rule never asks for a shape that the kernel does not take, a hook's columns of more than 8192 keys keep their sweeps,
+    and so do batches whose columns fill the chip."""
+    B = ctypes.byref
+
+    def pays(L, batch, H, hq, S, W, mean=None, paged=True, **kw):
+        v = _lib.FcKvView(**dict(dict(dtype=2, num_layers=L, batch=batch, num_kv_heads=H, max_seq_len=S, block_size=256 if paged else 1,
+                                      block_tables=1 if paged else None, stride_token=H * 128), **kw))
+        got = _lib.fn("fc_snapkv_once_pays")(B(v), hq, W, S if mean is None else mean)
+        assert not got or _lib.fn("fc_snapkv_once_workspace_bytes")(B(v), hq, W) > 0
+        return got
+
+    assert pays(1, 4, 8, 32, 4096, 64, paged=False) and not pays(1, 4, 8, 32, 250, 64, paged=False)
+    assert not pays(1, 1, 8, 32, 8193, 64, paged=False) and pays(1, 1, 8, 32, 8192, 64, paged=False)
+    assert pays(36, 1, 8, 32, 4096, 64) and not pays(36, 8, 8, 32, 4096, 64) and not pays(28, 13, 4, 28, 2300, 32, mean=1200)
+    assert pays(28, 3, 4, 28, 1000, 64) and not pays(28, 16, 4, 28, 4096, 64)
+    assert not pays(36, 1, 8, 32, 4096, 64, dtype=0) and not pays(36, 1, 8, 32, 1000, 64, block_size=48)
+    assert not pays(36, 1, 8, 32, 1000, 64, stride_token=1 << 24) and not pays(1, 1, 1, 17, 4096, 32, paged=False)
+    for L, batch, H, hq, W in ((36, 2, 8, 32, 32), (28, 5, 4, 28, 64), (32, 16, 32, 32, 32), (1, 8, 32, 32, 64), (1, 64, 8, 32, 64)):
+        for S in (1, 33, 450, 4096, 4097, 9216, 9217, 12289, 40000):
+            pays(L, batch, H, hq, S, W, paged=L > 1)
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "nope.so")

@@ -988,6 +988,55 @@ def test_snapkv_select_ragged(dev, S):
         assert not bool((diff & ((sc - kth).abs() > 2e-4 * kth.abs())).any())
 
 
+@pytest.mark.parametrize("Hq,H,W,causal", [(2, 2, 32, True), (4, 2, 64, False), (6, 2, 33, True), (14, 2, 32, True), (8, 2, 64, True),
+                                           (14, 2, 64, False), (8, 1, 64, True)])        # 1, 4, 6, 7, 8, 14, 16 blocks
+@pytest.mark.parametrize("dtype,large", [(torch.bfloat16, 1), (torch.float16, 4)])      # (four times as large: with offsets)
+def test_snapkv_select_in_one_pass(dev, Hq, H, W, causal, dtype, large):
+    """One pass over the keys keeps what the oracle's scores keep, up to keys at the threshold (fp32 sums of either are within
+    1e-5 of each other, scores a power of e apart): lengths around the 256 keys of a chunk, its halves and its quarters; and
+    the same positions whatever number of workgroups runs, also when one workgroup is handed many chunks of a column."""
+    L, ksz = 2, 5
+    lens = [1100, 513, 512, 385, 257, 256 + W, 129 + W, W + ksz + 1, W, 20]
+    S, keep = max(lens), [max(n // 3, W + 1) if n > W else n for n in lens]
+    case = synth.make_paged_case(seed=Hq + W, num_layers=L, batch=len(lens), num_kv_heads=H, seq_lens=lens, dtype=dtype,
+                                 num_q_heads=Hq, window=W, keep_dense=True)
+    pool, q = (case.kv_cache * large).to(dev), case.queries * large
+    kview = _lib.paged_view(pool[0], case.table_tensor(dev), case.lens_tensor(dev), S)
+    n_kept = torch.tensor(keep, dtype=torch.int32, device=dev)
+    out = [ops.snapkv_select(kview, q.to(dev), W, ksz, max(keep), causal, "sum", n_kept=n_kept, workgroups=n).cpu().long()
+           for n in (0, 1, 2, 9, 40)]
+    for b, (n, kk) in enumerate(zip(lens, keep)):
+        got = out[0][:, b, :, :kk]
+        assert all(torch.equal(o[:, b, :, :kk], got) for o in out[1:])
+        tail = min(W, n)
+        assert bool((got[..., 1:] > got[..., :-1]).all()) and bool((got[..., -tail:] == torch.arange(n - tail, n)).all())
+        if n <= W:
+            continue
+        for l in range(L):
+            sc = opress.snapkv_score(q[l, b:b + 1], case.dense_k[l, b:b + 1, :, :n] * large, W, ksz, causal, "sum")[0]
+            want = opress.topk_lowest_index(sc, kk)
+            kth = sc.gather(-1, want).min(-1, keepdim=True).values
+            diff = (torch.zeros_like(sc, dtype=torch.bool).scatter_(-1, got[l], True) ^
+                    torch.zeros_like(sc, dtype=torch.bool).scatter_(-1, want, True))
+            assert not bool((diff & ((sc - kth).abs() > 2e-4 * kth.abs())).any()), (b, l)
+
+
+def test_snapkv_select_in_one_pass_of_one_dense_layer(dev):
+    """The same from a dense layer, whose every column has the view's length, against the sweeps' selection."""
+    B, Hq, H, W, S, keep = 3, 8, 2, 64, 2049, 700
+    g = torch.Generator(device=dev).manual_seed(1)
+    k = torch.randn(1, B, H, S, 128, generator=g, device=dev).to(torch.bfloat16)
+    q = torch.randn(1, B, Hq, W, 128, generator=g, device=dev).to(torch.bfloat16)
+    kview = _lib.dense_view(k)
+    scores = ops.snapkv_score(kview, q, W, 7, True, "sum", splits=1).cpu()
+    want = opress.topk_lowest_index(scores, keep)
+    kth = scores.gather(-1, want).min(-1, keepdim=True).values
+    for n in (0, 1):
+        got = ops.snapkv_select(kview, q, W, 7, keep, True, "sum", workgroups=n).cpu().long()
+        diff = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, got, True) ^ torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, want, True)
+        assert not bool((diff & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+
+
 @pytest.mark.parametrize("lens", [[300, 1500, 64, 900, 900], [40, 2000]])
 def test_snapkv_press_longest_columns_first(dev, lens):
     """Sequence lengths known on the host order the launch's columns; the results are those of the launch as it comes."""
