@@ -226,6 +226,11 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   }
   const unsigned ring_lds = __builtin_amdgcn_readfirstlane(fc_lds_addr(smem)) + wave * (2 * DA_TILEB);
   char* ring = smem + wave * (2 * DA_TILEB);
+  // Where this workgroup alone reads its columns' bytes, the loads leave no line in the L2 (bf16, us a pass: 8 layers of
+  // 16 x 1024..4096 tokens, 32/8 heads, 449 -> 416; 90 x 128..2048 over 16 layers, 32/32 heads, 4654 -> 4250; batches that
+  // stay in the memory-side cache 1.00 to 0.9 times as long).  Workgroups that share a group of heads find the bytes there:
+  // 4 layers of 16 x 4096..8192, 128/4 heads, 591 -> 715 with such loads.
+  const bool alone = gtiles == 1;
 
   // Tile `tile` of the chunk into this wavefront's stage: eight wave-loads of four rows.  Lane i
   // writes LDS chunk i of the 64 chunks of those rows and fetches the global chunk (i & 15) ^ (row & 15)
@@ -245,11 +250,13 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
       }
       const char* g = base + tb * 2;
       const unsigned tok_bytes = (unsigned)v.stride_token * 2;
+      const auto lane_off = [&](int r) { return (unsigned)min(r, rmax) * tok_bytes + ((sub ^ (r & 15)) << 4); };
+      if (alone) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int r = 4 * u + rg;
-        const unsigned lo = (unsigned)min(r, rmax) * tok_bytes + ((sub ^ (r & 15)) << 4);
-        fc_load_lds(g, lo, dst + u * 1024);
+        for (int u = 0; u < 8; ++u) fc_load_lds_once(g, lane_off(4 * u + rg), dst + u * 1024);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) fc_load_lds(g, lane_off(4 * u + rg), dst + u * 1024);
       }
     } else {
       long long off[8];
