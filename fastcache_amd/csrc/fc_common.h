@@ -260,6 +260,11 @@ __device__ __forceinline__ void fc_load_lds_once(const char* g_uniform, unsigned
                : "memory", "m0");
 }
 #pragma clang diagnostic pop
+// 16 bytes to / from global memory, non-temporal likewise
+typedef unsigned fc_once4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void fc_store_once(void* p, const uint4& v) {
+  __builtin_nontemporal_store((fc_once4){v.x, v.y, v.z, v.w}, reinterpret_cast<fc_once4*>(p));
+}
 
 // Wait until at most N vector-memory operations of this wave are outstanding and all its LDS
 // operations are done, then synchronise the workgroup.

@@ -696,7 +696,12 @@ __global__ __launch_bounds__(256) void quant_rows_fast_kernel(QzPair io, long lo
 }
 
 // ---- flat passes, 8 output elements (one 16- or 8-byte access on each side) per thread ---------------------------
-// store 8 values in the output dtype
+// store 8 values in the output dtype.  16-bit outputs are written non-temporally: these passes are bound by the memory and
+// write two to four times what they read, and a dirty line that does not wait in the L2 costs the stream nothing (compress and
+// back, bf16, us a pass: int8 8 x 8 x 4000 keys 67.0 -> 62.6, nf4 4 x 32 x 4000 147 -> 112, fp8 8 x 32 x 4000 387 -> 374; tiny
+// ones the same).  An element-wise pass over the values right behind takes as long in all or less (int8 114.0 -> 107.4, nf4 223
+// -> 208) but for outputs about the size of the L2 (16 MB a plane: 34.9 -> 36.1).  The codes stay ordinary stores (72.4 us
+// against 74.2 so): a thread's 8 bytes are half of what a wide store takes.  32-bit outputs too: two pieces 32 bytes apart.
 template <int ODT>
 __device__ __forceinline__ void qz_store8(char* out, long long i8, const float (&y)[8]) {
   if constexpr (ODT == FC_F32) {
@@ -704,7 +709,7 @@ __device__ __forceinline__ void qz_store8(char* out, long long i8, const float (
     o[0] = make_uint4(__float_as_uint(y[0]), __float_as_uint(y[1]), __float_as_uint(y[2]), __float_as_uint(y[3]));
     o[1] = make_uint4(__float_as_uint(y[4]), __float_as_uint(y[5]), __float_as_uint(y[6]), __float_as_uint(y[7]));
   } else {
-    reinterpret_cast<uint4*>(out)[i8] = qz_pack<ODT>(y);
+    fc_store_once(reinterpret_cast<uint4*>(out) + i8, qz_pack<ODT>(y));
   }
 }
 
@@ -716,7 +721,7 @@ __device__ __forceinline__ void qz_store8(char* out, long long i8, const float (
       typedef float f2 __attribute__((ext_vector_type(2)));
       typedef __bf16 b2 __attribute__((ext_vector_type(2)));
       const auto two = [&](int j) { return __builtin_bit_cast(unsigned, __builtin_convertvector((f2){y[j], y[j + 1]}, b2)); };
-      reinterpret_cast<uint4*>(out)[i8] = make_uint4(two(0), two(2), two(4), two(6));
+      fc_store_once(reinterpret_cast<uint4*>(out) + i8, make_uint4(two(0), two(2), two(4), two(6)));
       return;
     }
   }
