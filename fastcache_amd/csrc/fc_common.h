@@ -265,6 +265,16 @@ typedef unsigned fc_once4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void fc_store_once(void* p, const uint4& v) {
   __builtin_nontemporal_store((fc_once4){v.x, v.y, v.z, v.w}, reinterpret_cast<fc_once4*>(p));
 }
+template <bool ONCE>
+__device__ __forceinline__ fc_once4 fc_load16(const char* p) {
+  if (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const fc_once4*>(p));
+  return *reinterpret_cast<const fc_once4*>(p);
+}
+template <bool ONCE>
+__device__ __forceinline__ void fc_store16(char* p, fc_once4 v) {
+  if (ONCE) __builtin_nontemporal_store(v, reinterpret_cast<fc_once4*>(p));
+  else *reinterpret_cast<fc_once4*>(p) = v;
+}
 
 // Wait until at most N vector-memory operations of this wave are outstanding and all its LDS
 // operations are done, then synchronise the workgroup.

@@ -3,8 +3,10 @@
 // One workgroup per (K|V, layer, sequence, kv head) column (per pair of heads for 512-byte fp32 rows), walked by
 // cp_walk in ascending chunks, which makes the in-place case (dst aliases src) safe.  Different heads, layers and
 // K/V planes touch disjoint bytes, so columns need no ordering between each other.
+#include <type_traits>
 #include "fc_rows.h"
 
+#define CP_ONCE_TOKEN 4096   // bytes of a token over all heads
 #define CP_THREADS 256
 
 // GATHER: src token = indices[j]; otherwise src token = src_start + j.
@@ -67,8 +69,16 @@ __global__ __launch_bounds__(CP_THREADS) void compact_kernel(KvView sk, KvView s
   const char* slayer = src_layers ? src_layers[l] : src.base + (long long)l * src.stride_layer * EB;
   const char* sbase = slayer + (long long)h * src.stride_head * EB + sub * 16;
   char* dbase = dst.base + ((long long)l * dst.stride_layer + (long long)h * dst.stride_head) * EB + sub * 16;
-  cp_walk<EB, HG, CP_THREADS>(src, dst, stbl, s_lds, dtbl, d_lds, b, S, n, sbase, dbase, src.base + sub * 16, dst_start,
-                              [&](int j) { return GATHER ? idx[j] : src_start + j; });
+  const auto walk = [&](auto once) {
+    cp_walk<EB, HG, CP_THREADS, decltype(once)::value>(src, dst, stbl, s_lds, dtbl, d_lds, b, S, n, sbase, dbase,
+                                                       src.base + sub * 16, dst_start,
+                                                       [&](int j) { return GATHER ? idx[j] : src_start + j; });
+  };
+  // Non-temporal for large planes whose tokens are 4 KB or more: there a SnapKV press of a pool, compaction included, takes
+  // 1032 us instead of 1063 (2 x 3000 tokens, 32 layers of 32 bf16 heads) and a Knorm press 253 instead of 279 (1 x 3000, 36
+  // layers of 8 fp32 heads); with tokens of 1 KB 729 instead of 721 (9 x 2000, 28 layers of 4 bf16 heads).
+  if (cp_once(src, EB) && src.num_kv_heads * FC_HEAD_DIM * EB >= CP_ONCE_TOKEN) walk(std::true_type{});
+  else walk(std::false_type{});
 }
 
 // Copies and gathers between buffers that cannot overlap need no order among their rows, and a copy is fastest on

@@ -1,11 +1,13 @@
 // The tail that the one-launch presses share: selection of a column's kept positions from its scores in LDS and the
 // in-place compaction of its K and V rows.
 #pragma once
+#include <type_traits>
 #include "fc_rows.h"
 #include "fc_select.h"
 
 // Keys per thread that the lean tail's selection keeps in registers; longer rows are selected from LDS.
 #define KP_KPT 16
+#define KP_ONCE_KEYS 1280
 
 // What the one-launch press kernels end with: the kk best of the column's S scores in LDS (0 < kk <= S, clamped by the
 // caller), their positions to the index row and to LDS, and the kept K and V rows moved to the front of the column.
@@ -51,16 +53,24 @@ __device__ __forceinline__ void kp_select_and_move(const KvView& kv, const KvVie
     const bool v_ok = cp_fill_pages<EB, THREADS>(vv, vtbl, vcol, S, ptbl + CP_PT);
     paged_walk = k_ok && v_ok;
   }
-  if (paged_walk) {
-    const CpPages kp = {ptbl, kv.block_shift, (unsigned)(kv.stride_token * EB)};
-    const CpPages vp = {ptbl + CP_PT, vv.block_shift, (unsigned)(vv.stride_token * EB)};
-    cp_walk_pages<EB, THREADS>(kp, vp, kk, sel);
-  } else {   // the general ordered walk, K then V
-    cp_walk<EB, 1, THREADS>(kv, kv, ktbl, k_lds, ktbl, k_lds, b, S, kk, kcol + sub * 16, kcol + sub * 16,
-                            kv.base + sub * 16, 0, [&](int j) { return sel[j]; });
-    cp_walk<EB, 1, THREADS>(vv, vv, vtbl, v_lds, vtbl, v_lds, b, S, kk, vcol + sub * 16, vcol + sub * 16,
-                            vv.base + sub * 16, 0, [&](int j) { return sel[j]; });
-  }
+  const auto move = [&](auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+    if (paged_walk) {
+      const CpPages kp = {ptbl, kv.block_shift, (unsigned)(kv.stride_token * EB)};
+      const CpPages vp = {ptbl + CP_PT, vv.block_shift, (unsigned)(vv.stride_token * EB)};
+      cp_walk_pages<EB, THREADS, ONCE>(kp, vp, kk, sel);
+    } else {   // the general ordered walk, K then V
+      cp_walk<EB, 1, THREADS, ONCE>(kv, kv, ktbl, k_lds, ktbl, k_lds, b, S, kk, kcol + sub * 16, kcol + sub * 16,
+                                    kv.base + sub * 16, 0, [&](int j) { return sel[j]; });
+      cp_walk<EB, 1, THREADS, ONCE>(vv, vv, vtbl, v_lds, vtbl, v_lds, b, S, kk, vcol + sub * 16, vcol + sub * 16,
+                                    vv.base + sub * 16, 0, [&](int j) { return sel[j]; });
+    }
+  };
+  // Behind SnapKV's scoring a short column's key rows are still in the L2 or near it: from KP_ONCE_KEYS keys on only (us,
+  // plain -> ONCE: 49 x 600 keys, 28 layers, 28/4 heads, 779 -> 794, 37 x 800 677 -> 703; 12 x 1500, 36 layers, 32/8 heads, 1107 ->
+  // 1086, 4 x 4000 1279 -> 1187).
+  if (cp_once(kv, EB) && (!LEAN || kv.max_seq_len >= KP_ONCE_KEYS)) move(std::true_type{});
+  else move(std::false_type{});
 }
 
 // the sequence's block-table rows of both views into LDS (when they fit); the caller synchronises

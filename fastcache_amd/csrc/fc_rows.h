@@ -12,6 +12,16 @@
 
 typedef unsigned cp_u32x4 __attribute__((ext_vector_type(4)));   // native vector: arrays of it stay in registers
 
+// Whether a walk's loads and stores are to leave no lines in the caches (ONCE below).  Where both planes of the view are
+// larger than what the memory-side cache (256 MB) keeps from one pass to the next, that makes the walk's streams faster;
+// below, the rows would be fetched from memory instead.  Measured on Knorm presses of a pool (us, plain -> ONCE, at K + V
+// in MB, 28 to 36 layers): bf16 103 -> 111 (275), 132 -> 138 (413), 194 -> 189 and 108 -> 113 (442), 173 -> 166 (528), 353
+// -> 318 (803), 651 -> 587 (1622); fp32 117 -> 134 (344), 113 -> 116 (459), 171 -> 166 (550), 538 -> 485 (1475).
+#define CP_ONCE_BYTES (480ll << 20)
+__device__ __forceinline__ bool cp_once(const KvView& v, int eb) {
+  return 2ll * v.num_layers * v.batch * v.num_kv_heads * v.max_seq_len * (FC_HEAD_DIM * eb) >= CP_ONCE_BYTES;
+}
+
 #ifndef CP_R
 #define CP_R 8      // 16-byte loads in flight per lane and chunk
 #endif
@@ -53,8 +63,8 @@ __device__ __forceinline__ long long cp_offset(const KvView& v, const int* tbl, 
 // sbase / dbase point at the lane's 16 bytes of its head's row of token offset 0 and `safe` at 16 readable bytes
 // (read in place of rows that do not exist, so that every lane always loads).  stbl / dtbl: the sequence's block-table
 // rows in LDS when s_lds / d_lds.  Two register buffers: the loads of chunk c+1 are issued right after the barrier that
-// releases the stores of chunk c, so loads and stores overlap.
-template <int EB, int HG, int THREADS, typename SrcOf>
+// releases the stores of chunk c, so loads and stores overlap.  ONCE: non-temporal accesses, see cp_once.
+template <int EB, int HG, int THREADS, bool ONCE, typename SrcOf>
 __device__ __forceinline__ void cp_walk(const KvView& src, const KvView& dst, const int* stbl, bool s_lds,
                                         const int* dtbl, bool d_lds, int b, int S, int n, const char* sbase,
                                         char* dbase, const char* safe, int dst_start, SrcOf src_of) {
@@ -82,7 +92,7 @@ __device__ __forceinline__ void cp_walk(const KvView& src, const KvView& dst, co
       if (s >= 0 && s < S) off = cp_offset(src, stbl, s_lds, b, s);
       const bool valid = off >= 0;
       const char* p = valid ? sbase + off * EB : safe;
-      buf[u] = *reinterpret_cast<const cp_u32x4*>(p);
+      buf[u] = fc_load16<ONCE>(p);
       ok |= valid ? (1u << u) : 0u;
     }
   };
@@ -94,7 +104,7 @@ __device__ __forceinline__ void cp_walk(const KvView& src, const KvView& dst, co
       const int j = j0 + u * TPP + tg;
       long long off = -1;
       if (ok & (1u << u)) off = cp_offset(dst, dtbl, d_lds, b, dst_start + j);
-      if (off >= 0) *reinterpret_cast<cp_u32x4*>(dbase + off * EB) = buf[u];
+      if (off >= 0) fc_store16<ONCE>(dbase + off * EB, buf[u]);
       all &= off >= 0;
     }
     return (bool)__all(all);
@@ -162,7 +172,7 @@ struct CpPages {
 // Rows j = 0 .. n-1 of BOTH planes: token j <- token sel[j] (ascending, sel[j] >= j, all below the sequence length; sel
 // in LDS), in place.  A chunk's K and V rows are loaded together, the workgroup waits for them and synchronises, and
 // only then are they stored; the next chunk's loads follow the stores at once (the stores are not waited for).
-template <int EB, int THREADS>
+template <int EB, int THREADS, bool ONCE>
 __device__ __forceinline__ void cp_walk_pages(const CpPages& kp, const CpPages& vp, int n, const int* sel) {
   constexpr int LPR = FC_HEAD_DIM * EB / 16;
   constexpr int RPP = THREADS / LPR;
@@ -178,7 +188,7 @@ __device__ __forceinline__ void cp_walk_pages(const CpPages& kp, const CpPages& 
       const int j = min(j0 + u * RPP + tg, n - 1);   // rows past the end re-read the last one and are not stored
       const unsigned s = (unsigned)sel[j];
       const char* page = reinterpret_cast<const char*>((uintptr_t)pl.ptbl[s >> pl.shift]);
-      buf[u] = *reinterpret_cast<const cp_u32x4*>(page + (__umul24(s & slot_mask, pl.tok_bytes) + lane_b));
+      buf[u] = fc_load16<ONCE>(page + (__umul24(s & slot_mask, pl.tok_bytes) + lane_b));
     }
   };
   auto store_rows = [&](const CpPages& pl, const cp_u32x4 (&buf)[CP_R], int j0) {
@@ -193,7 +203,7 @@ __device__ __forceinline__ void cp_walk_pages(const CpPages& kp, const CpPages& 
 #pragma unroll
     for (int u = 0; u < CP_R; ++u) {
       char* row = base + (unsigned long long)(unsigned)(u * RPP) * pl.tok_bytes;   // wave-uniform
-      if (j0 + u * RPP + tg < n) *reinterpret_cast<cp_u32x4*>(row + dlane) = buf[u];
+      if (j0 + u * RPP + tg < n) fc_store16<ONCE>(row + dlane, buf[u]);
     }
   };
 

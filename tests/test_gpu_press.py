@@ -1052,3 +1052,46 @@ def test_snapkv_press_longest_columns_first(dev, lens):
         out.append((scores, idx, pool))
     for a, b in zip(*out):
         assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+@pytest.mark.parametrize("form", ["compact", "select_compact", "knorm_press", "snapkv_press"])
+@pytest.mark.parametrize("dtype,sizes", [(torch.bfloat16, (959, 960, 1280)), (torch.float32, (479, 480))])
+def test_rows_of_large_views_move_as_those_of_small_ones(dev, dtype, sizes, form):
+    """Views that can hold 480 MiB or more (1 layer, 32 sequences, 32 heads: from 960 bf16 or 480 fp32 tokens on; behind
+    SnapKV's scoring from 1280 tokens on too) move their rows with other loads and stores: the same kept positions, the same
+    bytes in every slot."""
+    if form == "snapkv_press" and dtype == torch.float32:
+        pytest.skip("16-bit keys only")
+    B, H, W = 32, 32, 32
+    lens = [65 + (b * 53) % 400 for b in range(B)]
+    lens[3] = 470
+    keep = [n if b % 5 == 0 else (W + 1 + n) // 2 for b, n in enumerate(lens)]   # some keep everything
+    case = synth.make_paged_case(seed=8, num_layers=1, batch=B, num_kv_heads=H, seq_lens=lens, dtype=dtype, num_q_heads=H,
+                                 window=W, device=dev, device_draw=True)
+    lens_d = case.lens_tensor(dev)
+    n_kept = torch.tensor(keep, dtype=torch.int32, device=dev)
+
+    def run(S):
+        pool = case.kv_cache.clone()
+        tables = case.table_tensor(dev, width=-(-S // case.kv_cache.shape[3]))
+        kv, vv = (_lib.paged_view(pool[p], tables, lens_d, S) for p in range(2))
+        if form == "knorm_press":
+            scores, idx = ops.knorm_press(kv, vv, max(keep), dev, n_kept=n_kept)
+        elif form == "snapkv_press":
+            scores, idx = ops.snapkv_press(kv, vv, case.queries.to(dev), W, 5, max(keep), True, "sum", seq_lens=lens_d,
+                                           n_kept=n_kept)
+        else:
+            scores = ops.knorm_score(kv, dev)
+            if form == "select_compact":
+                idx = ops.select_compact(kv, vv, scores, max(keep), n_kept=n_kept)
+            else:
+                idx = ops.topk_select(scores, max(keep), row_lens=lens_d, n_kept=n_kept, rows_per_len=H)
+                ops.compact(kv, vv, kv, vv, idx, n_kept=n_kept)
+        return pool.view(torch.uint8), idx
+
+    pool, idx = run(max(lens))
+    assert not torch.equal(pool, case.kv_cache.view(torch.uint8))
+    for S in sizes:
+        pool_s, idx_s = run(S)
+        assert torch.equal(idx, idx_s), S
+        assert torch.equal(pool, pool_s), S
