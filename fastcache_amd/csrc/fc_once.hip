@@ -38,6 +38,7 @@
 
 #define SO_WAVES 4                   // wavefronts, and blocks of 32 window queries, of a workgroup
 #define SO_THREADS (SO_WAVES * 64)
+#define SO_HOOK_KEYS 32768           // see fc_once_pays
 #define SO_SLOT (128 * 256)          // 128 keys, or the queries of a group, in LDS: rows of 256 bytes, 16-byte pieces XOR-swizzled
 #define SO_RING 4
 #define SO_NONE 0xffffffffu          // a sum that is not there yet
@@ -658,10 +659,13 @@ bool fc_once_takes(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) 
 // Whether one pass beats two sweeps.  mean_len: the sequences' mean length, the view's max_seq_len their largest.  A dense layer
 // is a hook (scoring, selection, gather), everything else a paged pass (selection in a launch of its own and compaction, against
 // whichever of key ranges and the one-launch press it would take).  us, two sweeps -> one pass; where the rule says no as well:
-//  hooks, half kept.  32 query heads on 8, window 64: 8 columns of 1000 keys 20.4 -> 19.4, of 4096 30.2 -> 24.7, of 8000 39.4 ->
-//  32.6; 32 of 700 23.4 -> 21.6, of 4096 47.5 -> 41.8, of 250 19.4 -> 19.8 (no), of 10 000 92 -> 139 (no); window 32: 8 of 700
-//  16.7 -> 18.0 (no), of 4096 27.2 -> 23.7; 64 of 2000 38.1 -> 34.3.  28 on 4, window 64 (14 blocks): 4 columns of 400 25.4 ->
-//  18.4, of 4096 39.6 -> 24.7; 16 of 2000 33.5 -> 26.2.  32 on 32, window 64: 128 of 2000 55.2 -> 48.8, of 250 18.2 -> 19.9 (no).
+//  hooks, half kept.  32 query heads on 8, window 64: 8 columns of 4096 keys 30.2 -> 24.7, of 1000 20.4 -> 19.4; window 32: 8 of
+//  700 16.7 -> 18.0 (no), of 4096 27.2 -> 23.7.  28 on 4, window 64 (14 blocks): 4 columns of 400 25.4 -> 18.4, of 4096 39.6 ->
+//  24.7; 16 of 2000 33.5 -> 26.2.  More than SO_HOOK_KEYS keys in all keep the sweeps though one pass is the faster one for many of
+//  them (32 of 4096 47.5 -> 41.8): the two forms' sums differ by their fp32 roundings, and two keys that all but tie at the
+//  threshold are then ranked the other way (in 26 of 12 800 columns of 4096 keys, 6 of 8000 of 2000; against 64 bits the sweeps
+//  are off in 25 and 6, one pass in 23 and 0), which moves the rows between them: nothing in a pass over a pool's layers,
+//  but a large share of what a hook returns for a few long columns.
 //  paged, 30 % kept.  Four blocks: 576 columns of 1000 keys 126 -> 89, 1152 of 4096 826 -> 696, 2304 of 4096 1510 -> 1378; 14: 336
 //  of 1000 173 -> 107, 1792 of 600 465 -> 369, of 4096 2314 -> 2387 (no); 5 to 8: where one workgroup per column leaves the chip
 //  part empty in its last round, 288 of 1000 89 -> 67, 576 of 4096 551 -> 500, 2304 of 4096 1763 -> 1984 (no); 32 on 32: 1024 of 1000
@@ -671,11 +675,9 @@ bool fc_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, i
   const int blocks = num_q_heads / keys->num_kv_heads * ((window + 31) / 32), n = keys->max_seq_len;
   const int64_t cols = (int64_t)keys->num_layers * keys->batch * keys->num_kv_heads;
   if (!keys->block_tables && keys->num_layers == 1) {
-    if (n > 4096)
-      return n <= 8192 && cols * so_groups(num_q_heads, keys->num_kv_heads, window) * so_chunks(n) <= (blocks > 8 ? 1100 : 600);
+    if (cols * n > SO_HOOK_KEYS || n > 8192) return false;
     if (blocks > 8) return true;
-    if (blocks > 4) return cols <= 8 || n >= (blocks == 8 ? 600 : 1500);
-    return n >= 2700 || (n >= 600 && cols * n >= (blocks == 1 ? 80000 : 40000));
+    return blocks > 4 ? cols <= 8 || n >= (blocks == 8 ? 600 : 1500) : n >= 2700;
   }
   const bool equal = 16LL * mean_len >= 15LL * n;
   if (blocks > 8) return n <= 1536 || (n <= 2304 && cols <= 1500) || (n <= 4096 && (cols < 400 || (equal && cols < 1000)));

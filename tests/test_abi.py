@@ -105,7 +105,7 @@ def test_select_in_one_pass_validates_on_the_host():
 
 
 def test_one_pass_pays_where_it_can_run():
-    """The rule never asks for a shape that the kernel does not take, a hook's columns of more than 8192 keys keep their sweeps,
+    """The rule never asks for a shape that the kernel does not take, hooks of more than 8192 keys a column or 32 768 in all keep their sweeps,
     and so do batches whose columns fill the chip."""
     B = ctypes.byref
 
@@ -116,8 +116,9 @@ def test_one_pass_pays_where_it_can_run():
         assert not got or _lib.fn("fc_snapkv_once_workspace_bytes")(B(v), hq, W) > 0
         return got
 
-    assert pays(1, 4, 8, 32, 4096, 64, paged=False) and not pays(1, 4, 8, 32, 250, 64, paged=False)
-    assert not pays(1, 1, 8, 32, 8193, 64, paged=False) and pays(1, 1, 8, 32, 8192, 64, paged=False)
+    assert pays(1, 1, 8, 32, 4096, 64, paged=False) and not pays(1, 2, 8, 32, 250, 64, paged=False)
+    assert not pays(1, 1, 8, 32, 4097, 64, paged=False) and not pays(1, 4, 8, 32, 4096, 64, paged=False)
+    assert not pays(1, 1, 3, 21, 8193, 64, paged=False) and pays(1, 1, 3, 21, 8192, 64, paged=False)
     assert pays(36, 1, 8, 32, 4096, 64) and not pays(36, 8, 8, 32, 4096, 64) and not pays(28, 13, 4, 28, 2300, 32, mean=1200)
     assert pays(28, 3, 4, 28, 1000, 64) and not pays(28, 16, 4, 28, 4096, 64)
     assert not pays(36, 1, 8, 32, 4096, 64, dtype=0) and not pays(36, 1, 8, 32, 1000, 64, block_size=48)
