@@ -200,8 +200,7 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     tensor is passed through unchecked for callers that have validated the counts themselves.
 
     ``rows_only``: for callers that want the moved rows alone; scores and indices stay scratch (no window fill, no
-    padding of the index rows) and None is returned.  One pass over the keys, selection and compaction take the one launch's
-    place where they are faster (:func:`snapkv_once_pays`)."""
+    padding of the index rows) and None is returned."""
     order = None
     if n_kept is not None and not isinstance(n_kept, torch.Tensor):
         counts = [int(c) for c in n_kept]
@@ -236,12 +235,6 @@ def snapkv_press(keys: FcKvView, values: FcKvView, queries: torch.Tensor, window
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     dev = queries.device
-    if rows_only and lse is None and values is not None:
-        mean = keys.max_seq_len if host_lens is None else sum(host_lens) // len(host_lens)
-        if snapkv_once_pays(keys, Hq, window, mean):
-            idx = _select_once(keys, queries, kernel_size, k, causal_window, scale, out_scale, _i32(n_kept, "n_kept", dev), 0)
-            compact(keys, values, keys, values, idx, n_kept=n_kept)
-            return None
     stride = keys.max_seq_len
     scores = torch.empty((L, B, H, stride), dtype=torch.float32, device=dev)
     row_max = torch.empty((L, B, H), dtype=torch.float32, device=dev)

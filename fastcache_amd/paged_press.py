@@ -147,11 +147,13 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
             return None
     kview, vview = _views(kv_cache, block_tables, seq_lens, seq_len)
     fits = window_apart and ops.snapkv_press_fits(kview, hq, window_size, width)
+    once = False      # one pass over the keys, selection and compaction: every kept position is written (window_apart)
     if rows_only and window_apart:
         route = ops.snapkv_rows_route(kview, hq, window_size, fits, sum(lens) // len(lens))
+        once = route >= 0 and ops.snapkv_once_pays(kview, hq, window_size, sum(lens) // len(lens))
     else:
         route = 0 if fits and ops.snapkv_press_preferred(kview, hq, window_size, _lib.compute_units(kv_cache.device)) else -1
-    if route == 0:
+    if route == 0 and not once:
         same = len(set(kept)) == 1 and len(set(lens)) == 1
         res = ops.snapkv_press(kview, vview, queries, window_size, kernel_size, width, causal_window, reduction,
                                seq_lens=seq_lens, n_kept=None if same else kept, host_lens=lens, rows_only=rows_only)
@@ -159,10 +161,10 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
             return None
         scores, idx = res
         return PressResult(idx, width, scores, None if same else list(kept))
-    if route > 0:
+    if once or route > 0:
         n_kept = None if len(set(kept)) == 1 and len(set(lens)) == 1 else _lib.upload_ints(kept, kv_cache)
         idx = ops.snapkv_select(kview, queries, window_size, kernel_size, width, causal_window, reduction, n_kept=n_kept,
-                                splits=route, mean_len=sum(lens) // len(lens))
+                                splits=None if once else route, workgroups=0 if once else None)
         ops.compact(kview, vview, kview, vview, idx, n_kept=n_kept)
         return None
     scores = ops.snapkv_score(kview, queries, window_size, kernel_size, causal_window, reduction,

@@ -290,6 +290,39 @@ def test_snapkv_press_refuses_what_it_cannot_take(dev):
     assert not ops.snapkv_press_fits(kv, 4, 64, 5000)
     with pytest.raises(_lib.FastcacheError, match="fc_select_compact"):
         ops.snapkv_press(kv, vv, long.queries.to(dev), 64, 7, 5000)
+    kv, vv = (_lib.paged_view(pool[p], long.table_tensor(dev), long.lens_tensor(dev), 9216) for p in range(2))
+    assert ops.snapkv_once_pays(kv, 4, 64, 9216) and not ops.snapkv_press_fits(kv, 4, 64, 2000)
+    with pytest.raises(_lib.FastcacheError, match="fc_select_compact"):
+        ops.snapkv_press(kv, vv, long.queries.to(dev), 64, 7, 2000, rows_only=True)
+
+
+@pytest.mark.parametrize("lens,k,n_kept", [
+    ([1100, 1100, 1100], 300, [64, 300, 20]),      # counts in device memory that do not exceed the window
+    ([1100, 1100, 200], 300, None),                # a sequence shorter than the kept count
+    ([1100, 1100, 50], 300, [300, 299, 90])])      # a count above the length of a sequence no longer than the window
+def test_snapkv_press_rows_only_moves_what_the_full_press_moves(dev, lens, k, n_kept):
+    """With and without the scores and indices wanted: the same bytes in every slot, whatever the counts (untouched where a
+    column has no selection to make), on shapes where one pass over the keys is the faster scoring."""
+    H, Hq, W = 2, 8, 64
+    case = synth.make_paged_case(seed=11, num_layers=2, batch=len(lens), num_kv_heads=H, seq_lens=[1100] * len(lens), dtype=torch.bfloat16,
+                                 num_q_heads=Hq, window=W)
+    lens_d = torch.tensor(lens, dtype=torch.int32, device=dev)
+    counts = None if n_kept is None else torch.tensor(n_kept, dtype=torch.int32, device=dev)
+    host = n_kept is not None and min(lens) <= W                  # counts as Python ints, checked by the call
+    pools = []
+    for rows_only in (True, False):
+        pool = case.kv_cache.to(dev)
+        kv, vv = (_lib.paged_view(pool[p], case.table_tensor(dev), lens_d, max(lens)) for p in range(2))
+        assert ops.snapkv_once_pays(kv, Hq, W, 1100)
+        ops.snapkv_press(kv, vv, case.queries.to(dev), W, 5, k, True, "sum", seq_lens=lens_d, n_kept=n_kept if host else counts,
+                         ragged=True, host_lens=lens if host else None, rows_only=rows_only)
+        pools.append(pool)
+    assert torch.equal(pools[0].view(torch.uint8), pools[1].view(torch.uint8))
+    kept = torch.zeros_like(case.kv_cache[0], dtype=torch.bool)   # slots that may have changed
+    for b, (n, c) in enumerate(zip(lens, n_kept or [k] * len(lens))):
+        for j in range(min(n, c) if min(n, c) > W else 0):
+            kept[:, case.block_tables[b][j // 256], j % 256] = True
+    assert not bool((pools[0].cpu() != case.kv_cache)[:, ~kept].any())
 
 
 def test_knorm_press_one_launch_limits_and_clamps(dev):
