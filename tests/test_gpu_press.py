@@ -291,9 +291,9 @@ def test_snapkv_press_refuses_what_it_cannot_take(dev):
     with pytest.raises(_lib.FastcacheError, match="fc_select_compact"):
         ops.snapkv_press(kv, vv, long.queries.to(dev), 64, 7, 5000)
     kv, vv = (_lib.paged_view(pool[p], long.table_tensor(dev), long.lens_tensor(dev), 9216) for p in range(2))
-    assert ops.snapkv_once_pays(kv, 4, 64, 9216) and not ops.snapkv_press_fits(kv, 4, 64, 2000)
+    assert ops.snapkv_once_pays(kv, 4, 32, 9216) and not ops.snapkv_press_fits(kv, 4, 32, 9000)
     with pytest.raises(_lib.FastcacheError, match="fc_select_compact"):
-        ops.snapkv_press(kv, vv, long.queries.to(dev), 64, 7, 2000, rows_only=True)
+        ops.snapkv_press(kv, vv, long.queries[..., :32, :].contiguous().to(dev), 32, 7, 9000, rows_only=True)
 
 
 @pytest.mark.parametrize("lens,k,n_kept", [
