@@ -714,11 +714,6 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   };
   // V rows go to LDS without registers between, 4 rows of 256 bytes an instruction; the 16-byte pieces of a row are XOR-ed
   // with the row number, so that the transposed reads of 16 rows at one place meet all banks.
-  // Where this workgroup alone reads them, whole tiles leave no line in the L2 (bf16, us a pass: 16 captured layers of 16 x 3280
-  // tokens, 28/4 heads, 465 -> 446, of 1 x 8000, 32/32 heads, 487 -> 464, of 32 x 1000..4000, 28/4 heads, 700 -> 679; 28 eager layers
-  // of 3 x 300..900 325 -> 308).  K stays: an instruction takes 64 bytes of a row, the rest of the line would be fetched
-  // again (both planes so: 464 -> 480, 700 -> 778).
-  const bool alone = gtiles == 1;
   const unsigned v_lds = __builtin_amdgcn_readfirstlane(fc_lds_addr(smem) + wave * DC_STAGES * DA_TILEB);
   unsigned vlane[4];
 #pragma unroll
@@ -726,10 +721,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   auto load_v = [&](int stage, int tile) {
     const int s0 = t0 + tile * DA_TILE, rmax = end - 1 - s0;
     const char* vg = tile_base(vc, vbase, s0, vtbl);
-    if (rmax >= DA_TILE - 1 && alone) {
-#pragma unroll
-      for (int u = 0; u < 8; ++u) fc_load_lds_once(vg + u * 4 * (unsigned long long)vtok, vlane[u & 3], v_lds + stage * DA_TILEB + u * 1024);
-    } else if (rmax >= DA_TILE - 1) {
+    if (rmax >= DA_TILE - 1) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) fc_load_lds(vg + u * 4 * (unsigned long long)vtok, vlane[u & 3], v_lds + stage * DA_TILEB + u * 1024);
     } else {
