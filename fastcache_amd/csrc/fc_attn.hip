@@ -121,6 +121,13 @@ __device__ __forceinline__ bool da_append_rows(const KvView& kc, const KvView& v
   return inside;
 }
 
+// Table entry `e` of the k-th sequence after b, round the batch (k from 0; no such sequence: -1).  A page that another sequence's
+// table names at the same place belongs to a prefix that they share, and their workgroups read the same bytes.
+__device__ __forceinline__ int da_peer_page(const KvView& v, int b, int nb, int k, int e) {
+  const int p = b + 1 + k;
+  return k < nb - 1 ? v.block_tables[(long long)(p < nb ? p : p - nb) * v.table_stride + min(e, v.table_stride - 1)] : -1;
+}
+
 // GT = query heads served per workgroup (a tile of the group, at most 8).
 // FAST = a 32-token tile never straddles two pages (dense view, or pages of 32*2^n tokens), so a tile
 // load is a wave-uniform base plus a per-lane offset.
@@ -164,10 +171,15 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   // most 33), fetched before anything waits for the sequence length: a tile's address then costs a lane read instead
   // of a table load that the tile's own loads would have to wait for.
   int ktbl = 0, vtbl = 0;
+  int peer = -1, peer2 = -1;     // the range's first page in the tables of the 128 sequences after this one
   if constexpr (FAST) {
     if (kc.block_tables) {
       const int e = min((t0 >> kc.block_shift) + lane, kc.table_stride - 1);
       ktbl = kc.block_tables[(long long)b * kc.table_stride + e];
+      if (gtiles == 1) {
+        peer = da_peer_page(kc, b, gridDim.z, lane, t0 >> kc.block_shift);
+        if ((int)gridDim.z > FC_WAVE + 1) peer2 = da_peer_page(kc, b, gridDim.z, FC_WAVE + lane, t0 >> kc.block_shift);
+      }
     }
     if (vc.block_tables) {
       const int e = min((t0 >> vc.block_shift) + lane, vc.table_stride - 1);
@@ -226,11 +238,16 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   }
   const unsigned ring_lds = __builtin_amdgcn_readfirstlane(fc_lds_addr(smem)) + wave * (2 * DA_TILEB);
   char* ring = smem + wave * (2 * DA_TILEB);
-  // Where this workgroup alone reads its columns' bytes, the loads leave no line in the L2 (bf16, us a pass: 8 layers of
-  // 16 x 1024..4096 tokens, 32/8 heads, 449 -> 416; 90 x 128..2048 over 16 layers, 32/32 heads, 4654 -> 4250; batches that
-  // stay in the memory-side cache 1.00 to 0.9 times as long).  Workgroups that share a group of heads find the bytes there:
-  // 4 layers of 16 x 4096..8192, 128/4 heads, 591 -> 715 with such loads.
-  const bool alone = gtiles == 1;
+  // Where this workgroup alone reads its columns' bytes, the loads leave no line in the L2.  Workgroups that share a group of
+  // heads find the bytes there (4 layers of 16 x 4096..8192, 128/4 heads, 591 -> 715 with such loads), and so do those of
+  // sequences that share a prefix: a range whose first page another table names loads plainly.  us a pass, 16 captured bf16
+  // layers, plain loads / such loads whatever is shared / as here: 90 x 128..2048 tokens, 32/32 heads, 4611 / 4218 / 4171, 56 x
+  // 156..1565, 32/8, 965 / 923 / 877, 90 x 200..1400, 28/4, 912 / 853 / 782; 48 x 1300..1500 in groups of eight with the first
+  // 1280 in common, 32/32, 1647 / 2429 / 1613, 16 x 4096 with 3840, 32/8, 829 / 943 / 824, 90 x 1500 with 512, 32/32, 4643 / 5012 /
+  // 3755; where one head a group reads little else, 16 x 2048 with 1792, 1088 / 1269 / 1200.  (Asked for behind the first two
+  // loads instead: 0.94 to 1.1 times this one's time with a prefix, 1.0 to 1.15 without.)
+  const int page0 = __builtin_amdgcn_readfirstlane(ktbl);
+  const bool alone = gtiles == 1 && (!FAST || !kc.block_tables || !__any(page0 >= 0 && (peer == page0 || peer2 == page0)));
 
   // Tile `tile` of the chunk into this wavefront's stage: eight wave-loads of four rows.  Lane i
   // writes LDS chunk i of the 64 chunks of those rows and fetches the global chunk (i & 15) ^ (row & 15)

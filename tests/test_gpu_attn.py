@@ -882,3 +882,45 @@ def test_whole_columns_are_summed_as_accurately_as_chunks(dev, Hq, Hkv, B):
     last = float((exact.to(dtype).double() - exact).norm()) ** 2
     ratio = ((err ** 2 - last) / (ref ** 2 - last)) ** 0.5
     assert ratio < 0.7, ratio
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("width", [4, 12])                                                  # a workgroup a column; several
+@pytest.mark.parametrize("Hq,Hkv,B,apart", [(8, 8, 33, 1), (32, 8, 33, 32), (56, 8, 33, 2),          # 1, 4 and 7 heads a group
+                                            (4, 4, 66, 65), (4, 4, 130, 129), (4, 4, 200, 128)])
+def test_sequences_that_share_a_prefix_read_what_copies_of_it_hold(dev, dtype, width, Hq, Hkv, B, apart):
+    """The split kernel loads ranges of a prefix that two tables name in another way than those of one sequence alone: the
+    same bits as from a private copy of the pages, for sequences next to each other in the batch and up to its other end,
+    and with tables padded by entries that look like another sequence's page."""
+    g = torch.Generator().manual_seed(B)
+    lens = [40 + 7 * b % 300 for b in range(B)]
+    lens[0], lens[apart] = 700, 600
+    q = torch.randn(B, Hq, 128, generator=g).to(dtype).to(dev)
+    pages = sum(-(-n // 256) for n in lens)
+    pool = torch.randn(2, 1, pages + 2, 256, Hkv, 128, generator=g).to(dtype).to(dev)
+    tables, at = torch.full((B, width), -1, dtype=torch.int32), 0
+    for b, n in enumerate(lens):
+        for i in range(-(-n // 256)):
+            tables[b, i], at = at, at + 1
+    lens_d = torch.tensor(lens, dtype=torch.int32, device=dev)
+    shared = tables.clone()
+    shared[apart, :2] = shared[0, :2]                                   # two of three pages in common
+    copied = tables.clone()
+    copied[apart, :2] = torch.tensor([pages, pages + 1], dtype=torch.int32)
+    for i in range(2):
+        pool[:, :, pages + i] = pool[:, :, int(shared[0, i])]
+    decoys = copied.clone()
+    decoys[decoys < 0] = int(copied[0, 0])
+    ws = ops.decode_attn_workspace(B, Hq, width * 256, dev)
+
+    def run(t):
+        t = t.to(dev)
+        kv = [_lib.paged_view(pool[p], t, None, width * 256) for p in range(2)]
+        return ops.decode_attn(*kv, 0, q, lens_d, 128 ** -0.5, ws).cpu()
+
+    assert all("decode_attn_kernel<" in n for n in _launches(lambda: run(shared), "decode_column_kernel<", "decode_attn_kernel<"))
+    want = run(copied)
+    assert torch.equal(run(shared).view(torch.int16), want.view(torch.int16))
+    assert torch.equal(run(decoys).view(torch.int16), want.view(torch.int16))
+    ref = oattn.decode_attention(q.cpu(), pool[0, 0].cpu(), pool[1, 0].cpu(), lens_d.cpu(), shared, 128 ** -0.5)
+    assert float((want.float() - ref.float()).abs().max()) < 4e-3      # as above
