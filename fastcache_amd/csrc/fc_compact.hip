@@ -34,6 +34,7 @@ __global__ __launch_bounds__(CP_THREADS) void compact_kernel(KvView sk, KvView s
   const KvView& src = is_v ? sv : sk;
   const KvView& dst = is_v ? dv : dk;
   const int tid = threadIdx.x, sub = tid % LPR, rg = tid / LPR;
+  const int lens = cp_lens(src);
   const int S = fc_seq_len(src, b);
   // A count read from device memory is never trusted beyond what the host validated: the index row holds
   // index_stride entries, and the destination (its block table included) max_seq_len tokens.
@@ -77,7 +78,7 @@ __global__ __launch_bounds__(CP_THREADS) void compact_kernel(KvView sk, KvView s
   // Non-temporal for large planes whose tokens are 4 KB or more: there a SnapKV press of a pool, compaction included, takes
   // 1032 us instead of 1063 (2 x 3000 tokens, 32 layers of 32 bf16 heads) and a Knorm press 253 instead of 279 (1 x 3000, 36
   // layers of 8 fp32 heads); with tokens of 1 KB 729 instead of 721 (9 x 2000, 28 layers of 4 bf16 heads).
-  if (cp_once(src, EB) && src.num_kv_heads * FC_HEAD_DIM * EB >= CP_ONCE_TOKEN) walk(std::true_type{});
+  if (src.num_kv_heads * FC_HEAD_DIM * EB >= CP_ONCE_TOKEN && cp_once(src, EB, lens)) walk(std::true_type{});
   else walk(std::false_type{});
 }
 

@@ -12,7 +12,7 @@
 // What the one-launch press kernels end with: the kk best of the column's S scores in LDS (0 < kk <= S, clamped by the
 // caller), their positions to the index row and to LDS, and the kept K and V rows moved to the front of the column.
 // The last `tail_kept` positions of the column are kept whatever their scores and are not entered in the selection
-// (SnapKV's observation window, kk > tail_kept); sc[] need not hold them.  ptbl: 2 * CP_PT words of 8 bytes in LDS.
+// (SnapKV's observation window, kk > tail_kept); sc[] need not hold them.  ptbl: 2 * CP_PT words of 8 bytes in LDS, lens: cp_lens.
 //
 // LEAN picks the forms with the fewest instructions: the selection over keys held in registers and, for a paged
 // column, the walk over page addresses precomputed in LDS (about a fifth of the vector instructions of the general
@@ -26,7 +26,7 @@ template <int EB, int THREADS, bool LEAN>
 __device__ __forceinline__ void kp_select_and_move(const KvView& kv, const KvView& vv, const int* ktbl, bool k_lds,
                                                    const int* vtbl, bool v_lds, const float* sc, int* sel,
                                                    TkArea<THREADS>& sh, unsigned long long* ptbl, int l, int b, int h,
-                                                   int S, int kk, int tail_kept, int* __restrict__ idx_row) {
+                                                   int S, int kk, int tail_kept, int* __restrict__ idx_row, int lens) {
   const int tid = threadIdx.x, sub = tid % (FC_HEAD_DIM * EB / 16);
   if (kk == S) {   // everything stays where it is
     for (int i = tid; i < S; i += THREADS) idx_row[i] = i;
@@ -69,7 +69,7 @@ __device__ __forceinline__ void kp_select_and_move(const KvView& kv, const KvVie
   // Behind SnapKV's scoring a short column's key rows are still in the L2 or near it: from KP_ONCE_KEYS keys on only (us,
   // plain -> ONCE: 49 x 600 keys, 28 layers, 28/4 heads, 779 -> 794, 37 x 800 677 -> 703; 12 x 1500, 36 layers, 32/8 heads, 1107 ->
   // 1086, 4 x 4000 1279 -> 1187).
-  if (cp_once(kv, EB) && (!LEAN || kv.max_seq_len >= KP_ONCE_KEYS)) move(std::true_type{});
+  if ((!LEAN || kv.max_seq_len >= KP_ONCE_KEYS) && cp_once(kv, EB, lens)) move(std::true_type{});
   else move(std::false_type{});
 }
 

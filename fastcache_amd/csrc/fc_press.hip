@@ -50,6 +50,7 @@ __global__ __launch_bounds__(THREADS) void knorm_press_kernel(KvView kv, KvView 
   __shared__ int ktbl[CP_TBL], vtbl[CP_TBL];
   __shared__ TkArea<THREADS> sh;
 
+  const int lens = cp_lens(kv);
   int h, b, l;
   kp_column(h, b, l, kv.num_kv_heads, kv.batch, kv.num_layers);
   const int H = kv.num_kv_heads;
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(THREADS) void knorm_press_kernel(KvView kv, KvView 
   int kk = n_kept ? n_kept[b] : k;
   kk = min(min(kk, S), index_stride);
   if (kk <= 0) return;
-  kp_select_and_move<EB, THREADS, false>(kv, vv, ktbl, k_lds, vtbl, v_lds, sc, sel, sh, nullptr, l, b, h, S, kk, 0, idx_row);
+  kp_select_and_move<EB, THREADS, false>(kv, vv, ktbl, k_lds, vtbl, v_lds, sc, sel, sh, nullptr, l, b, h, S, kk, 0, idx_row, lens);
 }
 
 // Selection and compaction of a column from scores that another kernel wrote (any press whose scores are per
@@ -108,6 +109,7 @@ __global__ __launch_bounds__(THREADS) void select_compact_kernel(KvView kv, KvVi
   int* sel = reinterpret_cast<int*>(sc + smax);
   __shared__ int ktbl[CP_TBL], vtbl[CP_TBL];
   __shared__ TkArea<THREADS> sh;
+  const int lens = cp_lens(kv);
   int h, b, l;
   kp_column(h, b, l, kv.num_kv_heads, kv.batch, kv.num_layers);
   const int tid = threadIdx.x;
@@ -129,7 +131,7 @@ __global__ __launch_bounds__(THREADS) void select_compact_kernel(KvView kv, KvVi
   kp_tables<THREADS>(kv, vv, ktbl, vtbl, b, S, k_lds, v_lds);
   __syncthreads();
   kp_select_and_move<EB, THREADS, false>(kv, vv, ktbl, k_lds, vtbl, v_lds, sc, sel, sh, nullptr, l, b, h, S, kk, 0,
-                                  indices + row_id * index_stride);
+                                  indices + row_id * index_stride, lens);
 }
 
 static int kp_check(const char* who, const fc_kv_view* keys, const fc_kv_view* values, const void* scores,

@@ -12,14 +12,30 @@
 
 typedef unsigned cp_u32x4 __attribute__((ext_vector_type(4)));   // native vector: arrays of it stay in registers
 
-// Whether a walk's loads and stores are to leave no lines in the caches (ONCE below).  Where both planes of the view are
-// larger than what the memory-side cache (256 MB) keeps from one pass to the next, that makes the walk's streams faster;
-// below, the rows would be fetched from memory instead.  Measured on Knorm presses of a pool (us, plain -> ONCE, at K + V
-// in MB, 28 to 36 layers): bf16 103 -> 111 (275), 132 -> 138 (413), 194 -> 189 and 108 -> 113 (442), 173 -> 166 (528), 353
-// -> 318 (803), 651 -> 587 (1622); fp32 117 -> 134 (344), 113 -> 116 (459), 171 -> 166 (550), 538 -> 485 (1475).
+// Whether a walk's loads and stores are to leave no lines in the caches (ONCE below).  Where K and V of the batch's sequences,
+// both planes together and by their lengths, are more than what the memory-side cache (256 MB) keeps from one pass to the
+// next, that makes the walk's streams faster; below, the rows would be fetched from memory instead.  Measured on Knorm
+// presses of a pool (us, plain -> ONCE, at K + V in MB, 28 to 36 layers): bf16 103 -> 111 (275), 132 -> 138 (413), 194 -> 189
+// and 108 -> 113 (442), 173 -> 166 (528), 353 -> 318 (803), 651 -> 587 (1622); fp32 117 -> 134 (344), 113 -> 116 (459), 171 ->
+// 166 (550), 538 -> 485 (1475).  What the tables could hold does not count (plain -> ONCE -> by the lengths): 4 sequences of
+// 150 to 925 tokens, 36 layers of 8 bf16 heads, 202 MB of a view's 545, 69 -> 86 -> 70, of 150 to 1423, 276 of 839, 105 -> 115 ->
+// 108.
+// cp_lens: the length of sequence `lane`, asked for before the launch's other work so that nobody waits for it.
 #define CP_ONCE_BYTES (480ll << 20)
-__device__ __forceinline__ bool cp_once(const KvView& v, int eb) {
-  return 2ll * v.num_layers * v.batch * v.num_kv_heads * v.max_seq_len * (FC_HEAD_DIM * eb) >= CP_ONCE_BYTES;
+__device__ __forceinline__ long long cp_token_bytes(const KvView& v, int eb) {
+  return 2ll * v.num_layers * v.num_kv_heads * (FC_HEAD_DIM * eb);
+}
+__device__ __forceinline__ int cp_lens(const KvView& v) {
+  const int b = threadIdx.x & 63;
+  return v.seq_lens && b < v.batch ? v.seq_lens[b] : v.max_seq_len;
+}
+__device__ __forceinline__ bool cp_once(const KvView& v, int eb, int len) {
+  const long long token = cp_token_bytes(v, eb);
+  if (token * v.batch * v.max_seq_len < CP_ONCE_BYTES) return false;
+  int b = threadIdx.x & 63;
+  int n = b < v.batch ? min(max(len, 0), v.max_seq_len) : 0;
+  for (b += 64; b < v.batch; b += 64) n += fc_seq_len(v, b);
+  return fc_wave_sum_uniform((float)n) * (float)token >= (float)CP_ONCE_BYTES;
 }
 
 #ifndef CP_R

@@ -614,6 +614,7 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
     // page addresses of the column for the compaction: 8-byte words behind the counters (smem is 16-byte aligned)
     const int ptbl_word = (S + press.index_stride + SK_TBL + (int)(sizeof(TkArea<THREADS>) / 4) + 1) & ~1;
     unsigned long long* ptbl = reinterpret_cast<unsigned long long*>(reinterpret_cast<int*>(smem) + ptbl_word);
+    const int lens = cp_lens(kv);
     for (int s = tid; s < SW; s += THREADS) sc[s] = out_row[s];
     const KvView& vv = press.vv;
     const int nblk_v = vv.block_shift >= 0 ? ((S - 1) >> vv.block_shift) + 1 : 0;
@@ -622,7 +623,7 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
       for (int i = tid; i < nblk_v; i += THREADS) vtbl[i] = vv.block_tables[(long long)b * vv.table_stride + i];
     __syncthreads();
     int* idx_row = press.indices + (((long long)l * kv.batch + b) * Hkv + h) * (long long)press.index_stride;
-    kp_select_and_move<2, THREADS, true>(kv, vv, tbl, tbl_lds, vtbl, v_lds, sc, sel, sh, ptbl, l, b, h, S, kk, W, idx_row);
+    kp_select_and_move<2, THREADS, true>(kv, vv, tbl, tbl_lds, vtbl, v_lds, sc, sel, sh, ptbl, l, b, h, S, kk, W, idx_row, lens);
   }
 }
 

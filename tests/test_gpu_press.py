@@ -1088,43 +1088,42 @@ def test_snapkv_press_longest_columns_first(dev, lens):
 
 
 @pytest.mark.parametrize("form", ["compact", "select_compact", "knorm_press", "snapkv_press"])
-@pytest.mark.parametrize("dtype,sizes", [(torch.bfloat16, (959, 960, 1280)), (torch.float32, (479, 480))])
-def test_rows_of_large_views_move_as_those_of_small_ones(dev, dtype, sizes, form):
-    """Views that can hold 480 MiB or more (1 layer, 32 sequences, 32 heads: from 960 bf16 or 480 fp32 tokens on; behind
-    SnapKV's scoring from 1280 tokens on too) move their rows with other loads and stores: the same kept positions, the same
-    bytes in every slot."""
+@pytest.mark.parametrize("dtype,total", [(torch.bfloat16, 30719), (torch.bfloat16, 30720), (torch.float32, 15359), (torch.float32, 15360)])
+def test_rows_of_large_batches_move_as_those_of_small_ones(dev, dtype, total, form):
+    """Batches of 480 MiB or more (1 layer, 32 sequences, 32 heads: from 30 720 bf16 or 15 360 fp32 tokens in all on; behind
+    SnapKV's scoring where sequences may have 1280 tokens too) move their rows with other loads and stores: the same kept
+    positions, the same bytes in every slot as by halves of the batch."""
     if form == "snapkv_press" and dtype == torch.float32:
         pytest.skip("16-bit keys only")
     B, H, W = 32, 32, 32
-    lens = [65 + (b * 53) % 400 for b in range(B)]
-    lens[3] = 470
+    lens = [total // B + (b * 29) % 57 * (8 if dtype == torch.bfloat16 else 4) for b in range(B)]
+    spare = sum(lens) - total
+    lens = [n - spare // B - (b < spare % B) for b, n in enumerate(lens)]
+    assert sum(lens) == total and min(lens) > W + 5 and (dtype == torch.float32 or max(lens) >= 1100)
     keep = [n if b % 5 == 0 else (W + 1 + n) // 2 for b, n in enumerate(lens)]   # some keep everything
+    S = max(max(lens), 1280)
     case = synth.make_paged_case(seed=8, num_layers=1, batch=B, num_kv_heads=H, seq_lens=lens, dtype=dtype, num_q_heads=H,
                                  window=W, device=dev, device_draw=True)
-    lens_d = case.lens_tensor(dev)
+    tables, lens_d = case.table_tensor(dev, width=-(-S // case.kv_cache.shape[3])), case.lens_tensor(dev)
     n_kept = torch.tensor(keep, dtype=torch.int32, device=dev)
+    queries = case.queries.to(dev)
 
-    def run(S):
-        pool = case.kv_cache.clone()
-        tables = case.table_tensor(dev, width=-(-S // case.kv_cache.shape[3]))
-        kv, vv = (_lib.paged_view(pool[p], tables, lens_d, S) for p in range(2))
+    def press(pool, part):
+        t, n, k, q = tables[part].contiguous(), lens_d[part].contiguous(), n_kept[part].contiguous(), queries[:, part].contiguous()
+        kv, vv = (_lib.paged_view(pool[p], t, n, S) for p in range(2))
         if form == "knorm_press":
-            scores, idx = ops.knorm_press(kv, vv, max(keep), dev, n_kept=n_kept)
-        elif form == "snapkv_press":
-            scores, idx = ops.snapkv_press(kv, vv, case.queries.to(dev), W, 5, max(keep), True, "sum", seq_lens=lens_d,
-                                           n_kept=n_kept)
-        else:
-            scores = ops.knorm_score(kv, dev)
-            if form == "select_compact":
-                idx = ops.select_compact(kv, vv, scores, max(keep), n_kept=n_kept)
-            else:
-                idx = ops.topk_select(scores, max(keep), row_lens=lens_d, n_kept=n_kept, rows_per_len=H)
-                ops.compact(kv, vv, kv, vv, idx, n_kept=n_kept)
-        return pool.view(torch.uint8), idx
+            return ops.knorm_press(kv, vv, max(keep), dev, n_kept=k)[1]
+        if form == "snapkv_press":
+            return ops.snapkv_press(kv, vv, q, W, 5, max(keep), True, "sum", seq_lens=n, n_kept=k)[1]
+        scores = ops.knorm_score(kv, dev)
+        if form == "select_compact":
+            return ops.select_compact(kv, vv, scores, max(keep), n_kept=k)
+        idx = ops.topk_select(scores, max(keep), row_lens=n, n_kept=k, rows_per_len=H)
+        ops.compact(kv, vv, kv, vv, idx, n_kept=k)
+        return idx
 
-    pool, idx = run(max(lens))
-    assert not torch.equal(pool, case.kv_cache.view(torch.uint8))
-    for S in sizes:
-        pool_s, idx_s = run(S)
-        assert torch.equal(idx, idx_s), S
-        assert torch.equal(pool, pool_s), S
+    want, got = case.kv_cache.clone(), case.kv_cache.clone()
+    idx = torch.cat([press(want, slice(0, B // 2)), press(want, slice(B // 2, B))], 1)
+    assert not torch.equal(want.view(torch.uint8), case.kv_cache.view(torch.uint8))
+    assert torch.equal(press(got, slice(0, B)), idx)
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
