@@ -143,11 +143,7 @@ __global__ __launch_bounds__(THREADS, KPT > 16 ? 4 : 1) void column_select_kerne
   }
   if (a.parts == 0) return;
   __syncthreads();
-  // This workgroup's rows of both planes: source and destination are different tensors, any order will do.  Non-temporal
-  // stores: the kept rows take no room from rows still to be gathered (Knorm hook, bf16, 32 heads, plain -> non-temporal: 2 x
-  // 1000 to 12 x 5000 keys 0.99 to 0.85 times as long, 6 x 9000, a quarter kept, 198 -> 177 us; 1.06 at worst, where a layer's
-  // 500 MB in and out just fit the caches from one pass over it to the next).  The loads stay plain: the scoring pass has
-  // left part of the rows there.
+  // this workgroup's rows of both planes: source and destination are different tensors, any order will do
   const int sub = tid % LPR, rg = tid / LPR;
   const long long kcol = ((long long)l * kv.stride_layer + (long long)h * kv.stride_head) * EB + sub * 16;
   const long long vcol = ((long long)l * vv.stride_layer + (long long)h * vv.stride_head) * EB + sub * 16;
@@ -171,8 +167,8 @@ __global__ __launch_bounds__(THREADS, KPT > 16 ? 4 : 1) void column_select_kerne
       const int j = j0 + u * RPP + rg;
       if (j >= p1) continue;
       const long long ko = fc_token_offset(dk, b, j), vo = fc_token_offset(dv, b, j);
-      if (ko >= 0 && ((kok >> u) & 1u)) fc_store16<true>(dk.base + dkcol + ko * EB, kb[u]);
-      if (vo >= 0 && ((vok >> u) & 1u)) fc_store16<true>(dv.base + dvcol + vo * EB, vb[u]);
+      if (ko >= 0 && ((kok >> u) & 1u)) *reinterpret_cast<cp_u32x4*>(dk.base + dkcol + ko * EB) = kb[u];
+      if (vo >= 0 && ((vok >> u) & 1u)) *reinterpret_cast<cp_u32x4*>(dv.base + dvcol + vo * EB) = vb[u];
     }
   }
 }
