@@ -696,36 +696,38 @@ __global__ __launch_bounds__(256) void quant_rows_fast_kernel(QzPair io, long lo
 }
 
 // ---- flat passes, 8 output elements (one 16- or 8-byte access on each side) per thread ---------------------------
-// store 8 values in the output dtype.  16-bit outputs are written non-temporally: these passes are bound by the memory and
-// write two to four times what they read, and a dirty line that does not wait in the L2 costs the stream nothing (compress and
-// back, bf16, us a pass: int8 8 x 8 x 4000 keys 67.0 -> 62.6, nf4 4 x 32 x 4000 147 -> 112, fp8 8 x 32 x 4000 387 -> 374; tiny
-// ones the same).  An element-wise pass over the values right behind takes as long in all or less (int8 114.0 -> 107.4, nf4 223
-// -> 208) but for outputs about the size of the L2 (16 MB a plane: 34.9 -> 36.1).  The codes stay ordinary stores (72.4 us
-// against 74.2 so): a thread's 8 bytes are half of what a wide store takes.  32-bit outputs too: two pieces 32 bytes apart.
+// store 8 values in the output dtype.  once: non-temporally, 16-bit outputs of QZ_ONCE_BYTES and more (below).  The codes and
+// 32-bit outputs are ordinary stores: a thread's 8 bytes are half of what a wide store takes (72.4 us against 74.2 so), two
+// pieces lie 32 bytes apart.
 template <int ODT>
-__device__ __forceinline__ void qz_store8(char* out, long long i8, const float (&y)[8]) {
+__device__ __forceinline__ void qz_store8(char* out, long long i8, const float (&y)[8], bool once) {
   if constexpr (ODT == FC_F32) {
     uint4* o = reinterpret_cast<uint4*>(out) + 2 * i8;
     o[0] = make_uint4(__float_as_uint(y[0]), __float_as_uint(y[1]), __float_as_uint(y[2]), __float_as_uint(y[3]));
     o[1] = make_uint4(__float_as_uint(y[4]), __float_as_uint(y[5]), __float_as_uint(y[6]), __float_as_uint(y[7]));
   } else {
-    fc_store_once(reinterpret_cast<uint4*>(out) + i8, qz_pack<ODT>(y));
+    uint4* o = reinterpret_cast<uint4*>(out) + i8;
+    if (once) fc_store_once(o, qz_pack<ODT>(y));
+    else *o = qz_pack<ODT>(y);
   }
 }
 
 // ... of values whose sum `any` is not NaN (so none of them is): bf16 two per instruction
 template <int ODT>
-__device__ __forceinline__ void qz_store8(char* out, long long i8, const float (&y)[8], float any) {
+__device__ __forceinline__ void qz_store8(char* out, long long i8, const float (&y)[8], float any, bool once) {
   if constexpr (ODT == FC_BF16) {
     if (any == any) {
       typedef float f2 __attribute__((ext_vector_type(2)));
       typedef __bf16 b2 __attribute__((ext_vector_type(2)));
       const auto two = [&](int j) { return __builtin_bit_cast(unsigned, __builtin_convertvector((f2){y[j], y[j + 1]}, b2)); };
-      fc_store_once(reinterpret_cast<uint4*>(out) + i8, make_uint4(two(0), two(2), two(4), two(6)));
+      const uint4 v = make_uint4(two(0), two(2), two(4), two(6));
+      uint4* o = reinterpret_cast<uint4*>(out) + i8;
+      if (once) fc_store_once(o, v);
+      else *o = v;
       return;
     }
   }
-  qz_store8<ODT>(out, i8, y);
+  qz_store8<ODT>(out, i8, y, once);
 }
 // NaN if one of the values is
 __device__ __forceinline__ float qz_sum8(const float (&y)[8]) {
@@ -760,12 +762,22 @@ struct QzRowOf {
   __device__ __forceinline__ long long operator()(long long i) const { return shift >= 0 ? i >> shift : i / d8; }
 };
 
+// Values of this many bytes in 16 bits do not wait in the caches for what reads them, and these passes, bound by the memory,
+// write two to four times what they read: without dirty lines in the L2 the stream is faster.  Smaller ones are found there,
+// by an attention layer above all.  bf16, us, ordinary stores -> non-temporal ones, K and V from codes / and one row of
+// queries against them (torch) / K and V to codes and back: int8, 65 MB a plane 35.7 -> 36.5 / 189 -> 206 / 70 -> 63, 98 MB
+// 51.3 -> 51.9 / 281 -> 297 / 106 -> 90, 131 MB 71.5 -> 67.1 / 243 -> 239 / 150 -> 124, 197 MB 103 -> 97 / 357 -> 348 / 217 -> 200;
+// nf4, 33 MB 18.2 -> 15.6 / 172 -> 186 / 38 -> 36, 98 MB 52.4 -> 55.6 / 272 -> 301 / 95 -> 87, 131 MB 76 -> 71 / 239 -> 244 /
+// 148 -> 115, 262 MB 139 -> 135 / 318 -> 316 / 272 -> 252; fp8, 131 MB 74 -> 71 / 244 -> 243 / 209 -> 185.
+#define QZ_ONCE_BYTES (120ll << 20)
+
 // out = float(code) * scale: int8 rows (KIND 0, one scale per d codes), fp8 (KIND 1 / 2 = E4M3 / E5M2, one scale)
 template <int SDT, int ODT, int KIND>
 __global__ __launch_bounds__(256) void dequantize_vec_kernel(const unsigned char* __restrict__ q,
                                                              const char* __restrict__ scale, long long n8, QzRowOf row_of,
                                                              char* __restrict__ out) {
   const float sc1 = KIND == 0 ? 0.f : qz_load<SDT>(scale, 0);
+  const bool once = n8 * 16 >= QZ_ONCE_BYTES;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256) {
     const uint2 c = reinterpret_cast<const uint2*>(q)[i];
     const float sc = KIND == 0 ? qz_load<SDT>(scale, row_of(i)) : sc1;
@@ -778,7 +790,7 @@ __global__ __launch_bounds__(256) void dequantize_vec_kernel(const unsigned char
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) y[j] *= sc;
-    qz_store8<ODT>(out, i, y, qz_sum8(y));
+    qz_store8<ODT>(out, i, y, qz_sum8(y), once);
   }
 }
 
@@ -792,6 +804,7 @@ __global__ __launch_bounds__(256) void dequantize_group4_vec_kernel(const unsign
     qz_fill_levels<TDT>(levels);
     __syncthreads();
   }
+  const bool once = n8 * 16 >= QZ_ONCE_BYTES;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n8; i += (long long)gridDim.x * 256) {
     const unsigned c = reinterpret_cast<const unsigned*>(packed)[i];
     const float sc = qz_load<SDT>(scale, row_of(i));
@@ -801,7 +814,7 @@ __global__ __launch_bounds__(256) void dequantize_group4_vec_kernel(const unsign
       const unsigned code = (c >> (4 * j)) & 15u;
       y[j] = (MODE == 0 ? (float)(int)code - 8.f : levels[code]) * sc;
     }
-    qz_store8<ODT>(out, i, y, qz_sum8(y));
+    qz_store8<ODT>(out, i, y, qz_sum8(y), once);
   }
 }
 

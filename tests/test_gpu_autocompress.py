@@ -170,6 +170,24 @@ def test_quantization_method_bit_exact(dev, dtype, kind):
         assert torch.equal(qm2.dequantize(q, s, dtype).cpu(), oa.dequantize_4bit(rq, rs, 32, kind == "nf4", dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["int8", "int4", "nf4", "fp8"])
+@pytest.mark.parametrize("rows", [491519, 491520, 491523])
+def test_large_outputs_dequantise_as_their_pieces(dev, dtype, kind, rows):
+    """Outputs of 120 MiB and more (491 520 rows of 128 values) are stored another way than smaller ones: bit for bit what
+    their halves give, NaN included."""
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.randn(1, 1, rows, 128, generator=g, device=dev).to(dtype)
+    if kind != "fp8":                  # (one NaN makes all of a tensor's float8 codes NaN)
+        x[0, 0, rows // 3] = float("nan")
+    qm = ac.QuantizationMethod(kind)
+    (q, s), _ = qm.compress(x, x)
+    got, h = qm.dequantize(q, s, dtype), rows // 2
+    want = torch.cat([qm.dequantize(q[:, :, part].contiguous(), s[:, :, part].contiguous(), dtype)
+                      for part in (slice(0, h), slice(h, rows))], 2)
+    assert got.shape == x.shape and torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 def _fp8_bits(t):
     return t.view(torch.uint8)
 
