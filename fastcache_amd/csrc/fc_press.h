@@ -7,12 +7,21 @@
 
 // Keys per thread that the lean tail's selection keeps in registers; longer rows are selected from LDS.
 #define KP_KPT 16
+
+// Whether a press of views that can hold this much is launched with the walk's ONCE form as well (FAR below), which takes it
+// where the sequences do hold it (cp_once).  A kernel of its own, since a SnapKV press of columns of 540 to 1320 keys takes 0.5 to
+// 1.6 % longer with both forms in it.  Behind SnapKV's scoring a short column's key rows are still in the L2 or near it: there
+// from KP_ONCE_KEYS keys on only (us, plain -> ONCE: 49 x 600 keys, 28 layers, 28/4 heads, 779 -> 794, 37 x 800 677 -> 703; 12 x
+// 1500, 36 layers, 32/8 heads, 1107 -> 1086, 4 x 4000 1279 -> 1187, 8 x 4096, half kept, 2045 -> 1946).
 #define KP_ONCE_KEYS 1280
+static inline bool kp_far(const fc_kv_view* v) {
+  return 2ll * v->num_layers * v->batch * v->num_kv_heads * v->max_seq_len * (FC_HEAD_DIM * fc_elem_bytes(v->dtype)) >= CP_ONCE_BYTES;
+}
 
 // What the one-launch press kernels end with: the kk best of the column's S scores in LDS (0 < kk <= S, clamped by the
 // caller), their positions to the index row and to LDS, and the kept K and V rows moved to the front of the column.
 // The last `tail_kept` positions of the column are kept whatever their scores and are not entered in the selection
-// (SnapKV's observation window, kk > tail_kept); sc[] need not hold them.  ptbl: 2 * CP_PT words of 8 bytes in LDS, lens: cp_lens.
+// (SnapKV's observation window, kk > tail_kept); sc[] need not hold them.  ptbl: 2 * CP_PT words of 8 bytes in LDS, lens: cp_lens (not LEAN).
 //
 // LEAN picks the forms with the fewest instructions: the selection over keys held in registers and, for a paged
 // column, the walk over page addresses precomputed in LDS (about a fifth of the vector instructions of the general
@@ -22,7 +31,7 @@
 // and the stand-alone selection + compaction are bound by memory latency instead: there the general walk, which has
 // the next chunk's loads in flight before the current chunk's stores are issued and never waits for a store, is the
 // faster one (cfg1: 0.282 ms against 0.294 to 0.312 ms with the lean forms), so they keep it.
-template <int EB, int THREADS, bool LEAN>
+template <int EB, int THREADS, bool LEAN, bool FAR>
 __device__ __forceinline__ void kp_select_and_move(const KvView& kv, const KvView& vv, const int* ktbl, bool k_lds,
                                                    const int* vtbl, bool v_lds, const float* sc, int* sel,
                                                    TkArea<THREADS>& sh, unsigned long long* ptbl, int l, int b, int h,
@@ -66,11 +75,13 @@ __device__ __forceinline__ void kp_select_and_move(const KvView& kv, const KvVie
                                     vv.base + sub * 16, 0, [&](int j) { return sel[j]; });
     }
   };
-  // Behind SnapKV's scoring a short column's key rows are still in the L2 or near it: from KP_ONCE_KEYS keys on only (us,
-  // plain -> ONCE: 49 x 600 keys, 28 layers, 28/4 heads, 779 -> 794, 37 x 800 677 -> 703; 12 x 1500, 36 layers, 32/8 heads, 1107 ->
-  // 1086, 4 x 4000 1279 -> 1187).
-  if ((!LEAN || kv.max_seq_len >= KP_ONCE_KEYS) && cp_once(kv, EB, lens)) move(std::true_type{});
-  else move(std::false_type{});
+  if constexpr (FAR) {
+    if (cp_once(kv, EB, LEAN ? cp_lens(kv) : lens)) {
+      move(std::true_type{});
+      return;
+    }
+  }
+  move(std::false_type{});
 }
 
 // the sequence's block-table rows of both views into LDS (when they fit); the caller synchronises

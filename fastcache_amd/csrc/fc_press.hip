@@ -38,7 +38,7 @@ __device__ __forceinline__ void kp_column(int& h, int& b, int& l, int H, int B, 
   l = (int)(col / ((long long)H * B));
 }
 
-template <int DTYPE, int THREADS>
+template <int DTYPE, int THREADS, bool FAR>
 __global__ __launch_bounds__(THREADS) void knorm_press_kernel(KvView kv, KvView vv, float* __restrict__ scores,
                                                               int score_stride, int k, const int* __restrict__ n_kept,
                                                               int* __restrict__ indices, int index_stride, int smax) {
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(THREADS) void knorm_press_kernel(KvView kv, KvView 
   __shared__ int ktbl[CP_TBL], vtbl[CP_TBL];
   __shared__ TkArea<THREADS> sh;
 
-  const int lens = cp_lens(kv);
+  const int lens = FAR ? cp_lens(kv) : 0;
   int h, b, l;
   kp_column(h, b, l, kv.num_kv_heads, kv.batch, kv.num_layers);
   const int H = kv.num_kv_heads;
@@ -95,12 +95,12 @@ __global__ __launch_bounds__(THREADS) void knorm_press_kernel(KvView kv, KvView 
   int kk = n_kept ? n_kept[b] : k;
   kk = min(min(kk, S), index_stride);
   if (kk <= 0) return;
-  kp_select_and_move<EB, THREADS, false>(kv, vv, ktbl, k_lds, vtbl, v_lds, sc, sel, sh, nullptr, l, b, h, S, kk, 0, idx_row, lens);
+  kp_select_and_move<EB, THREADS, false, FAR>(kv, vv, ktbl, k_lds, vtbl, v_lds, sc, sel, sh, nullptr, l, b, h, S, kk, 0, idx_row, lens);
 }
 
 // Selection and compaction of a column from scores that another kernel wrote (any press whose scores are per
 // (layer, sequence, kv head, token)): fc_topk_select and fc_compact of a cache onto itself in one launch.
-template <int EB, int THREADS>
+template <int EB, int THREADS, bool FAR>
 __global__ __launch_bounds__(THREADS) void select_compact_kernel(KvView kv, KvView vv, const float* __restrict__ scores,
                                                                  int score_stride, int k,
                                                                  const int* __restrict__ n_kept,
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(THREADS) void select_compact_kernel(KvView kv, KvVi
   int* sel = reinterpret_cast<int*>(sc + smax);
   __shared__ int ktbl[CP_TBL], vtbl[CP_TBL];
   __shared__ TkArea<THREADS> sh;
-  const int lens = cp_lens(kv);
+  const int lens = FAR ? cp_lens(kv) : 0;
   int h, b, l;
   kp_column(h, b, l, kv.num_kv_heads, kv.batch, kv.num_layers);
   const int tid = threadIdx.x;
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(THREADS) void select_compact_kernel(KvView kv, KvVi
   bool k_lds, v_lds;
   kp_tables<THREADS>(kv, vv, ktbl, vtbl, b, S, k_lds, v_lds);
   __syncthreads();
-  kp_select_and_move<EB, THREADS, false>(kv, vv, ktbl, k_lds, vtbl, v_lds, sc, sel, sh, nullptr, l, b, h, S, kk, 0,
+  kp_select_and_move<EB, THREADS, false, FAR>(kv, vv, ktbl, k_lds, vtbl, v_lds, sc, sel, sh, nullptr, l, b, h, S, kk, 0,
                                   indices + row_id * index_stride, lens);
 }
 
@@ -167,18 +167,21 @@ extern "C" int fc_knorm_press(const fc_kv_view* keys, const fc_kv_view* values, 
   const size_t lds = ((size_t)smax + (size_t)index_stride) * 4;
   dim3 grid(keys->num_kv_heads, keys->batch, keys->num_layers);
   hipStream_t st = (hipStream_t)stream;
-#define KP_LAUNCH(DT, TH)                                                                                        \
+#define KP_LAUNCH(DT, TH, FR)                                                                                    \
   do {                                                                                                           \
-    FC_ALLOW_LDS((knorm_press_kernel<DT, TH>), KP_MAX_LDS);                                                       \
-    hipLaunchKernelGGL((knorm_press_kernel<DT, TH>), grid, dim3(TH), lds, st, kv, vv, scores, score_stride, k,   \
-                       n_kept, indices, index_stride, smax);                                                     \
+    FC_ALLOW_LDS((knorm_press_kernel<DT, TH, FR>), KP_MAX_LDS);                                                   \
+    hipLaunchKernelGGL((knorm_press_kernel<DT, TH, FR>), grid, dim3(TH), lds, st, kv, vv, scores, score_stride,  \
+                       k, n_kept, indices, index_stride, smax);                                                  \
   } while (0)
   // Columns no more than compute units are wide whatever their length, since nothing else fills the chip (us per pass, 256
   // -> 1024 threads: 112 columns of 300 bf16 keys 50 -> 47, of 1000 74 -> 55, 224 of 1000 78 -> 64; 336 of 1000 85 -> 87).
   const bool wide = (long long)smax * FC_HEAD_DIM * fc_elem_bytes(keys->dtype) >= KP_WIDE_BYTES_PRESS ||
                     (long long)keys->num_kv_heads * keys->batch * keys->num_layers <= fc_compute_units();
-#define KP_DISPATCH(DT) \
-  if (wide) KP_LAUNCH(DT, 1024); else KP_LAUNCH(DT, 256)
+  const bool far = kp_far(keys);
+#define KP_DISPATCH(DT)                                                             \
+  if (far) { if (wide) KP_LAUNCH(DT, 1024, true); else KP_LAUNCH(DT, 256, true); } \
+  else if (wide) KP_LAUNCH(DT, 1024, false);                                       \
+  else KP_LAUNCH(DT, 256, false)
   switch (keys->dtype) {
     case FC_F32: KP_DISPATCH(FC_F32); break;
     case FC_F16: KP_DISPATCH(FC_F16); break;
@@ -202,18 +205,20 @@ extern "C" int fc_select_compact(const fc_kv_view* keys, const fc_kv_view* value
   const size_t lds = ((size_t)smax + (size_t)index_stride) * 4;
   dim3 grid(keys->num_kv_heads, keys->batch, keys->num_layers);
   hipStream_t st = (hipStream_t)stream;
-#define KP_LAUNCH(E, TH)                                                                                          \
+#define KP_LAUNCH(E, TH, FR)                                                                                     \
   do {                                                                                                           \
-    FC_ALLOW_LDS((select_compact_kernel<E, TH>), KP_MAX_LDS);                                                     \
-    hipLaunchKernelGGL((select_compact_kernel<E, TH>), grid, dim3(TH), lds, st, kv, vv, scores, score_stride, k, \
-                       n_kept, indices, index_stride, smax);                                                     \
+    FC_ALLOW_LDS((select_compact_kernel<E, TH, FR>), KP_MAX_LDS);                                                 \
+    hipLaunchKernelGGL((select_compact_kernel<E, TH, FR>), grid, dim3(TH), lds, st, kv, vv, scores, score_stride, \
+                       k, n_kept, indices, index_stride, smax);                                                  \
   } while (0)
   const bool wide = (long long)smax * FC_HEAD_DIM * fc_elem_bytes(keys->dtype) >= KP_WIDE_BYTES_SELECT;
-  if (keys->dtype == FC_F32) {
-    if (wide) KP_LAUNCH(4, 1024); else KP_LAUNCH(4, 256);
-  } else {
-    if (wide) KP_LAUNCH(2, 1024); else KP_LAUNCH(2, 256);
-  }
+  const bool far = kp_far(keys);
+#define KP_DISPATCH(E)                                                            \
+  if (far) { if (wide) KP_LAUNCH(E, 1024, true); else KP_LAUNCH(E, 256, true); } \
+  else if (wide) KP_LAUNCH(E, 1024, false);                                      \
+  else KP_LAUNCH(E, 256, false)
+  if (keys->dtype == FC_F32) { KP_DISPATCH(4); } else { KP_DISPATCH(2); }
+#undef KP_DISPATCH
 #undef KP_LAUNCH
   FC_CHECK_LAUNCH(who);
   return FC_OK;

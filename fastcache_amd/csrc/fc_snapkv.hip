@@ -60,6 +60,7 @@ struct SkCfg {
 //         (a small kernel takes the moving average afterwards, across the pieces' borders).
 // PRESS (MODE 0, at least four wavefronts): the workgroup goes on to select the column's kept positions (the
 // window always among them) and to move the kept K and V rows to the front of the column, see the end of the kernel.
+// FAR: kp_far.
 struct SkPress {
   KvView vv;            // the value plane, same geometry as the keys
   int k;                // kept positions per row when n_kept is null
@@ -77,7 +78,7 @@ __host__ __device__ constexpr int sk_press_need(int max_seq_len, int index_strid
   return 4 * max_seq_len + 4 * index_stride + 4 * SK_TBL + 4096 + 16 * CP_PT;   // + the selection's counters, page addresses
 }
 
-template <int DTYPE, int NW, bool FAST, int MODE, bool PRESS = false>
+template <int DTYPE, int NW, bool FAST, int MODE, bool PRESS = false, bool FAR = false>
 __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
     KvView kv, const char* __restrict__ q, int Hq, int W, int ksz, int causal, float c, float out_mul,
     float* __restrict__ scores, int score_stride, float* __restrict__ row_max, const float* __restrict__ lse,
@@ -614,7 +615,6 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
     // page addresses of the column for the compaction: 8-byte words behind the counters (smem is 16-byte aligned)
     const int ptbl_word = (S + press.index_stride + SK_TBL + (int)(sizeof(TkArea<THREADS>) / 4) + 1) & ~1;
     unsigned long long* ptbl = reinterpret_cast<unsigned long long*>(reinterpret_cast<int*>(smem) + ptbl_word);
-    const int lens = cp_lens(kv);
     for (int s = tid; s < SW; s += THREADS) sc[s] = out_row[s];
     const KvView& vv = press.vv;
     const int nblk_v = vv.block_shift >= 0 ? ((S - 1) >> vv.block_shift) + 1 : 0;
@@ -623,7 +623,7 @@ __global__ __launch_bounds__(NW * 64, (NW <= 8 ? 4 : 2)) void snapkv_kernel(
       for (int i = tid; i < nblk_v; i += THREADS) vtbl[i] = vv.block_tables[(long long)b * vv.table_stride + i];
     __syncthreads();
     int* idx_row = press.indices + (((long long)l * kv.batch + b) * Hkv + h) * (long long)press.index_stride;
-    kp_select_and_move<2, THREADS, true>(kv, vv, tbl, tbl_lds, vtbl, v_lds, sc, sel, sh, ptbl, l, b, h, S, kk, W, idx_row, lens);
+    kp_select_and_move<2, THREADS, true, FAR>(kv, vv, tbl, tbl_lds, vtbl, v_lds, sc, sel, sh, ptbl, l, b, h, S, kk, W, idx_row, 0);
   }
 }
 
@@ -777,20 +777,24 @@ static int snapkv_score_impl(const char* who, const fc_kv_view* keys, const void
     press.indices = press_indices;
     press.index_stride = press_index_stride;
     press.order = press_order;
-#define SK_PRESS(DT, NWV)                                                                                        \
+    const bool far = keys->max_seq_len >= KP_ONCE_KEYS && kp_far(keys);
+#define SK_PRESS_FAR(DT, NWV, FR)                                                                                 \
   do {                                                                                                         \
-    FC_ALLOW_LDS((snapkv_kernel<DT, NWV, true, 0, true>), SkCfg<NWV>::LDS);                                     \
-    hipLaunchKernelGGL((snapkv_kernel<DT, NWV, true, 0, true>), grid, dim3(NWV * 64), SkCfg<NWV>::LDS, st, kv, \
-                       q, num_q_heads, window, kernel_size, causal_window, c, out_mul, scores, score_stride,   \
+    FC_ALLOW_LDS((snapkv_kernel<DT, NWV, true, 0, true, FR>), SkCfg<NWV>::LDS);                                 \
+    hipLaunchKernelGGL((snapkv_kernel<DT, NWV, true, 0, true, FR>), grid, dim3(NWV * 64), SkCfg<NWV>::LDS, st, \
+                       kv, q, num_q_heads, window, kernel_size, causal_window, c, out_mul, scores, score_stride, \
                        row_max, lse, 1, (float*)nullptr, (float*)nullptr, press);                              \
   } while (0)
-#define SK_PRESS_NW(DT)                 \
-  if (nw == 4) SK_PRESS(DT, 4);         \
-  else if (nw == 8) SK_PRESS(DT, 8);    \
-  else SK_PRESS(DT, 16)
+#define SK_PRESS(DT, NWV) \
+  if (far) SK_PRESS_FAR(DT, NWV, true); else SK_PRESS_FAR(DT, NWV, false)
+#define SK_PRESS_NW(DT)                     \
+  if (nw == 4) { SK_PRESS(DT, 4); }         \
+  else if (nw == 8) { SK_PRESS(DT, 8); }    \
+  else { SK_PRESS(DT, 16); }
     if (keys->dtype == FC_BF16) { SK_PRESS_NW(FC_BF16); } else { SK_PRESS_NW(FC_F16); }
-#undef SK_PRESS_NW
 #undef SK_PRESS
+#undef SK_PRESS_FAR
+#undef SK_PRESS_NW
     FC_CHECK_LAUNCH(who);
     return FC_OK;
   }
