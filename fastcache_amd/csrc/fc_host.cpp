@@ -806,7 +806,7 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       hq = q.size(2);
       nsplit = fc_snapkv_rows_route(&kv, (int32_t)hq, (int32_t)W, fits, (int32_t)as_int(item(7)));
       if (nsplit < 0) Py_RETURN_NONE;
-      once = fc_snapkv_once_pays(&kv, (int32_t)hq, (int32_t)W, (int32_t)as_int(item(7))) != 0;
+      once = fc_snapkv_rows_once_pays(&kv, (int32_t)hq, (int32_t)W, (int32_t)as_int(item(7)), (int32_t)width, nsplit) != 0;
       one = nsplit == 0 && !once;
     }
     const int32_t *counts = nullptr, *order = nullptr;

@@ -6,9 +6,10 @@
 #define SO_LISTS 8           // lists the columns are shared out over, at most
 #define SO_CHUNKS_MAX 48     // chunks of the longest column
 
-// Whether the kernel takes the shape, and whether it is the faster one for sequences of that mean length.
+// Whether the kernel takes the shape, and whether it is the faster one for sequences of that mean length of which at most
+// `kept` tokens stay; whole: instead of one launch per pass.
 bool fc_once_takes(const fc_kv_view* keys, int32_t num_q_heads, int32_t window);
-bool fc_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len);
+bool fc_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len, int32_t kept, bool whole);
 int64_t fc_once_workspace_bytes(int32_t num_layers, int32_t batch, int32_t num_q_heads, int32_t num_kv_heads, int32_t window,
                                 int32_t max_seq_len);
 int fc_once_groups(const fc_kv_view* keys, int32_t num_q_heads, int32_t window);   // of four blocks of 32 window queries

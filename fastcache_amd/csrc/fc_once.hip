@@ -39,6 +39,7 @@
 #define SO_WAVES 4                   // wavefronts, and blocks of 32 window queries, of a workgroup
 #define SO_THREADS (SO_WAVES * 64)
 #define SO_HOOK_KEYS 32768           // see fc_once_pays
+#define SO_KEPT_ROWS 1100000         // likewise
 #define SO_SLOT (128 * 256)          // 128 keys, or the queries of a group, in LDS: rows of 256 bytes, 16-byte pieces XOR-swizzled
 #define SO_RING 4
 #define SO_NONE 0xffffffffu          // a sum that is not there yet
@@ -656,21 +657,41 @@ bool fc_once_takes(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) 
   return (int64_t)keys->num_layers * keys->batch * keys->num_kv_heads * groups * chunks < (1ll << 22);
 }
 
-// Whether one pass beats two sweeps.  mean_len: the sequences' mean length, the view's max_seq_len their largest.  A dense layer
-// is a hook (scoring, selection, gather), everything else a paged pass (selection in a launch of its own and compaction, against
-// whichever of key ranges and the one-launch press it would take).  us, two sweeps -> one pass; where the rule says no as well:
-//  hooks, half kept.  32 query heads on 8, window 64: 8 columns of 4096 keys 30.2 -> 24.7, of 1000 20.4 -> 19.4; window 32: 8 of
-//  700 16.7 -> 18.0 (no), of 4096 27.2 -> 23.7.  28 on 4, window 64 (14 blocks): 4 columns of 400 25.4 -> 18.4, of 4096 39.6 ->
-//  24.7; 16 of 2000 33.5 -> 26.2.  More than SO_HOOK_KEYS keys in all keep the sweeps though one pass is the faster one for many of
-//  them (32 of 4096 47.5 -> 41.8): the two forms' sums differ by their fp32 roundings, and two keys that all but tie at the
-//  threshold are then ranked the other way (in 26 of 12 800 columns of 4096 keys, 6 of 8000 of 2000; against 64 bits the sweeps
-//  are off in 25 and 6, one pass in 23 and 0), which moves the rows between them: nothing in a pass over a pool's layers,
-//  but a large share of what a hook returns for a few long columns.
-//  paged, 30 % kept.  Four blocks: 576 columns of 1000 keys 126 -> 89, 1152 of 4096 826 -> 696, 2304 of 4096 1510 -> 1378; 14: 336
-//  of 1000 173 -> 107, 1792 of 600 465 -> 369, of 4096 2314 -> 2387 (no); 5 to 8: where one workgroup per column leaves the chip
-//  part empty in its last round, 288 of 1000 89 -> 67, 576 of 4096 551 -> 500, 2304 of 4096 1763 -> 1984 (no); 32 on 32: 1024 of 1000
-//  161 -> 138, 3072 of 1500 0.95.  Lengths that differ start longest first in one launch, which takes much of the gain away.
-bool fc_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len) {
+// Whether one pass beats two sweeps.  mean_len: the sequences' mean length, the view's max_seq_len their largest.
+//
+// A dense layer is a hook (scoring, selection, gather).  us, half kept, two sweeps -> one pass; where the rule says no as well:
+//  32 query heads on 8, window 64: 8 columns of 4096 keys 30.2 -> 24.7, of 1000 20.4 -> 19.4; window 32: 8 of 700 16.7 -> 18.0
+//  (no), of 4096 27.2 -> 23.7.  28 on 4, window 64 (14 blocks): 4 columns of 400 25.4 -> 18.4, of 4096 39.6 -> 24.7; 16 of 2000
+//  33.5 -> 26.2.  More than SO_HOOK_KEYS keys in all keep the sweeps, faster or not (32 of 4096 47.5 -> 41.8): the two forms' sums
+//  differ by their fp32 roundings, and two keys that all but tie at the threshold are then ranked the other way, which moves the
+//  rows between them (26 of 12 800 columns of 4096 keys, 6 of 8000 of 2000: one in two million keys; against 64 bits the sweeps are
+//  off in 25 and 6, one pass in 23 and 0).  Within the bound one call in 60 returns other rows than the sweeps do: hooks of more
+//  keys, where it would be one in 15 and more, return what they did before there was one pass.  This is a line drawn for
+//  unchanged results, not for time or precision.
+//
+// Everything else is a paged pass (selection in a launch of its own and compaction), against what fc_snapkv_rows_route says:
+// key ranges, followed by the same launches, or (whole) one launch per column, which moves a column's kept rows while others
+// are scored.  There the kept rows of both planes count as well: beyond SO_KEPT_ROWS of them, more than the caches hold,
+// compaction as a launch is slower than what the scoring saves, unless few of a column's rows stay; lengths that differ start longest
+// first in one launch, which takes most of the gain away.  us, the other form -> one pass, at 25, 50 or 70 % kept:
+//  ranges.  4 blocks: 288 columns of 4201 keys, 25 %, 225 -> 189, 576 of 5870, 25 %, 630 -> 489, 1152 of 7629, 70 %, 2413 -> 2125;
+//  14: 336 of 1752, 50 %, 270 -> 221, 784 of 3530, 70 %, 1272 -> 1189; 8: 288 of 2527, 25 %, 190 -> 150, 576 of 4062, 50 %, 654 -> 601, of 8212
+//  1278 -> 1421 (no); 7: 112 of 964, 70 %, 60 -> 51.
+//  one launch.  4 blocks: 576 of 608, 25 %, 88 -> 67, of 2332, 70 %, 392 -> 340, 1728 of 935, 25 %, 267 -> 232, of 1951, 70 %, 706 -> 786 (no);
+//  1 and 2: 3072 of 943, 25 %, 407 -> 355, 4096 of 1941, 70 %, 1499 -> 1712 (no), 8192 of 604, 70 %, 1020 -> 1087 (no), of 724, 25 %, 855 ->
+//  741; 14: 784 of 456, 25 %, 225 -> 136, 336 of 1270, 50 %, 232 -> 165, 1456 of 1968, 70 %, 1156 -> 1181 (no); 8: 288 of 1879, 25 %, 146 -> 113,
+//  of 651, 70 %, 83 -> 76, 576 of 3245, 70 %, 558 -> 582 (no); 7: 672 of 590, 70 %, 124 -> 141 (no).
+// One round of workgroups, or two of up to 4 blocks, nearly full, is where one launch is at its best: 480 columns of 671 keys, 2 blocks,
+// 60 %, 75 -> 85, 224 of 809, 14 blocks, 60 %, 91 -> 97.
+static bool so_whole_pays(int blocks, int64_t cols, int64_t n, int64_t mean_len, int64_t kept) {
+  const bool equal = 16 * mean_len >= 15 * n, few = 3 * kept <= n;
+  if (blocks > 4 && blocks <= 8) return cols <= 112 || (equal && (few || (cols <= 340 && n >= 640)));
+  if (blocks > 8 ? n > 2304 : !equal && n > 600 && !(few && 10 * mean_len >= 9 * n)) return false;
+  const int64_t slots = fc_compute_units() * (blocks > 4 ? 1 : 2), rounds = (cols + slots - 1) / slots;
+  if (rounds <= (blocks > 4 ? 1 : 2) && 4 * cols >= 3 * rounds * slots) return few && blocks <= 4;
+  return few ? blocks > 2 || n <= 1300 || 2 * cols * kept <= 3 * SO_KEPT_ROWS : cols * kept <= SO_KEPT_ROWS;
+}
+bool fc_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len, int32_t kept, bool whole) {
   if (!fc_once_takes(keys, num_q_heads, window)) return false;
   const int blocks = num_q_heads / keys->num_kv_heads * ((window + 31) / 32), n = keys->max_seq_len;
   const int64_t cols = (int64_t)keys->num_layers * keys->batch * keys->num_kv_heads;
@@ -679,10 +700,12 @@ bool fc_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, i
     if (blocks > 8) return true;
     return blocks > 4 ? cols <= 8 || n >= (blocks == 8 ? 600 : 1500) : n >= 2700;
   }
+  if (whole && !so_whole_pays(blocks, cols, n, mean_len, kept)) return false;
   const bool equal = 16LL * mean_len >= 15LL * n;
   if (blocks > 8) return n <= 1536 || (n <= 2304 && cols <= 1500) || (n <= 4096 && (cols < 400 || (equal && cols < 1000)));
   if (n < 450) return false;
-  if (blocks > 4) return n <= 4096 && 10 * ((cols + 511) / 512 * 512) >= 14 * cols && (equal || cols <= 340);
+  const int64_t round = 2 * fc_compute_units();      // 5 to 8 blocks: where whole columns leave the chip part empty in their last round
+  if (blocks > 4) return n <= 4096 && 10 * ((cols + round - 1) / round * round) >= 14 * cols && (equal || cols <= 340);
   if (blocks > 2) return n <= 9216 && (equal || cols <= 2400);
   return equal ? n <= 4096 : n <= 768;
 }

@@ -1069,7 +1069,12 @@ extern "C" int64_t fc_snapkv_select_workspace_bytes(int32_t num_layers, int32_t 
 }
 
 extern "C" int32_t fc_snapkv_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len) {
-  return fc_once_pays(keys, num_q_heads, window, mean_len) ? 1 : 0;
+  return fc_once_pays(keys, num_q_heads, window, mean_len, 0, false) ? 1 : 0;
+}
+
+extern "C" int32_t fc_snapkv_rows_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len,
+                                            int32_t kept, int32_t route) {
+  return route >= 0 && fc_once_pays(keys, num_q_heads, window, mean_len, kept, route == 0) ? 1 : 0;
 }
 
 static int64_t sk_once_room(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) {   // the per-key sums
@@ -1162,7 +1167,7 @@ static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_
   a.indices = indices;
   a.index_stride = index_stride;
   a.parts = out_k && !indices ? fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, keys->max_seq_len, k) : 0;
-  if (out_k && !lse && num_q_heads > 0 && num_q_heads % keys->num_kv_heads == 0 && fc_once_pays(keys, num_q_heads, window, stride) &&
+  if (out_k && !lse && num_q_heads > 0 && num_q_heads % keys->num_kv_heads == 0 && fc_once_pays(keys, num_q_heads, window, stride, k, false) &&
       workspace_bytes >= fc_snapkv_once_workspace_bytes(keys, num_q_heads, window))
     return snapkv_once_impl(who, keys, values, out_k, out_v, queries, num_q_heads, window, kernel_size, causal_window, scale, a, 0,
                             workspace, workspace_bytes, stream);

@@ -272,9 +272,15 @@ def snapkv_rows_route(keys: FcKvView, num_q_heads: int, window: int, fits: bool,
 
 
 def snapkv_once_pays(keys: FcKvView, num_q_heads: int, window: int, mean_len: int) -> bool:
-    """Whether scoring in one pass over the keys, then selection and compaction, is the fastest press of sequences of that
-    mean length (the rule and its measurements stand at ``fc_once_pays``)."""
+    """Whether scoring in one pass over the keys beats two sweeps in key ranges, for sequences of that mean length (the rule
+    and its measurements stand at ``fc_once_pays``)."""
     return bool(fn("fc_snapkv_once_pays")(C.byref(keys), num_q_heads, window, mean_len))
+
+
+def snapkv_rows_once_pays(keys: FcKvView, num_q_heads: int, window: int, mean_len: int, kept: int, route: int) -> bool:
+    """Whether a press whose caller wants the moved rows alone, at most ``kept`` of a sequence, is faster by one pass over the
+    keys, selection and compaction than by ``route`` (:func:`snapkv_rows_route`)."""
+    return bool(fn("fc_snapkv_rows_once_pays")(C.byref(keys), num_q_heads, window, mean_len, kept, route))
 
 
 def _select_once(keys, queries, kernel_size, k, causal_window, scale, out_scale, n_kept, workgroups):

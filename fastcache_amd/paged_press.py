@@ -150,7 +150,7 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
     once = False      # one pass over the keys, selection and compaction: every kept position is written (window_apart)
     if rows_only and window_apart:
         route = ops.snapkv_rows_route(kview, hq, window_size, fits, sum(lens) // len(lens))
-        once = route >= 0 and ops.snapkv_once_pays(kview, hq, window_size, sum(lens) // len(lens))
+        once = ops.snapkv_rows_once_pays(kview, hq, window_size, sum(lens) // len(lens), width, route)
     else:
         route = 0 if fits and ops.snapkv_press_preferred(kview, hq, window_size, _lib.compute_units(kv_cache.device)) else -1
     if route == 0 and not once:

@@ -128,6 +128,25 @@ def test_one_pass_pays_where_it_can_run():
             pays(L, batch, H, hq, S, W, paged=L > 1)
 
 
+def test_one_pass_over_a_pool_counts_the_rows_that_stay():
+    """Against key ranges the kept rows do not matter; against the one launch a pass that keeps much, fills the chip's rounds or
+    has lengths that differ stays there, and a route that refuses the shape is not overruled."""
+    B = ctypes.byref
+
+    def pays(L, batch, H, hq, S, W, kept, route=0, mean=None):
+        v = _lib.FcKvView(dtype=2, num_layers=L, batch=batch, num_kv_heads=H, max_seq_len=S, block_size=256, block_tables=1,
+                          stride_token=H * 128)
+        return bool(_lib.fn("fc_snapkv_rows_once_pays")(B(v), hq, W, S if mean is None else mean, kept, route))
+
+    for kept in (100, 700, 1400):
+        assert pays(36, 2, 8, 32, 2000, 32, kept, route=2) and not pays(36, 2, 8, 32, 2000, 32, kept, route=-1)
+    for (L, batch, H, hq, W), S in (((36, 6, 8, 32, 32), 1951), ((32, 4, 32, 32, 32), 1941), ((28, 13, 4, 28, 64), 1968)):
+        assert not pays(L, batch, H, hq, S, W, S * 7 // 10) and pays(L, batch, H, hq, min(S, 1300), W, S // 10)
+    assert pays(36, 1, 8, 32, 651, 64, 455) and not pays(36, 2, 8, 32, 3245, 64, 2271) and not pays(28, 6, 4, 28, 590, 32, 413)
+    assert not pays(12, 5, 8, 8, 671, 64, 402) and pays(12, 5, 8, 8, 671, 64, 200) and not pays(28, 2, 4, 28, 809, 64, 200)
+    assert not pays(36, 4, 8, 32, 2939, 32, 700, mean=1270) and pays(36, 2, 8, 32, 2074, 32, 500, mean=1935)
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "nope.so")

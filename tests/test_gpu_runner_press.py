@@ -413,15 +413,18 @@ def test_rows_only_moves_the_rows_of_the_general_path(dev, monkeypatch, press, L
             assert torch.equal(got[:, :, page, :m].view(torch.int16), want[:, :, page, :m].view(torch.int16)), (b, i)
 
 
-@pytest.mark.parametrize("L,H,hq,lens", [
-    (4, 2, 8, [600, 64]),           # cut by the longest length alone, whole by the lengths of the batch
-    (4, 2, 8, [600, 590]),          # cut
-    (16, 4, 28, [1100, 333, 64, 901, 700]),
+@pytest.mark.parametrize("L,H,hq,lens,form", [
+    (4, 2, 8, [400, 64], "whole"),                              # cut by the longest length alone, whole by the lengths of the batch
+    (16, 4, 28, [1100, 333, 64, 901, 700], "whole"),
+    (3, 4, 8, [5200, 1300, 60], "ranges"),
+    (4, 2, 14, [4200, 4100], "ranges"),
+    (4, 2, 8, [600, 590], "once"),                              # instead of ranges
+    (4, 2, 8, [600, 64], "once"), (16, 4, 28, [700] * 3, "once"),      # instead of whole columns
 ])
-def test_rows_only_general_path_launches_what_the_host_module_does(dev, monkeypatch, L, H, hq, lens):
-    """Where the host module's call declines, the same rule decides between whole columns and key ranges: the calls it
-    makes instead are those of ``fc_snapkv_rows_route`` for the batch's lengths, and the pool is the same."""
-    import ctypes
+def test_rows_only_general_path_launches_what_the_host_module_does(dev, monkeypatch, L, H, hq, lens, form):
+    """Where the host module's call declines, the same rules decide between whole columns, key ranges and one pass over the keys:
+    the entry point it calls instead is the one that ``fc_snapkv_rows_route`` and ``fc_snapkv_rows_once_pays`` name for the
+    batch's lengths, both launch the same kernels, and the pool is the same."""
     from fastcache_amd import _lib, ops
     torch.manual_seed(5)
     B, W, per = len(lens), 32, -(-max(lens) // 256)
@@ -429,20 +432,42 @@ def test_rows_only_general_path_launches_what_the_host_module_does(dev, monkeypa
     tables = torch.randperm(B * per + 1, device=dev)[:B * per].view(B, per).int().contiguous()
     lens_d = torch.tensor(lens, dtype=torch.int32, device=dev)
     queries = torch.randn((L, B, hq, W, 128), device=dev).to(torch.bfloat16)
+    host = lens if len(set(lens)) > 1 else None
+    kview = _lib.paged_view(pool[0], tables, lens_d, max(lens))
+    width, mean = max(paged_press.n_kept_for(n, 0.2) for n in lens), sum(lens) // B
+    route = ops.snapkv_rows_route(kview, hq, W, ops.snapkv_press_fits(kview, hq, W, width), mean)
+    once = ops.snapkv_rows_once_pays(kview, hq, W, mean, width, route)
+    assert form == ("once" if once else "whole" if route == 0 else "ranges")
+
+    def press(p):
+        paged_press.snapkv_compress_paged(p, tables, lens_d, max(lens), queries, 0.2, window_size=W, host_lens=host, rows_only=True)
+
+    def scoring(fn):
+        """Names of the scoring kernels' launches; a profile now and then holds none"""
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA], acc_events=True) as prof:
+            fn()
+            torch.cuda.synchronize()
+        return [e.name.split("(")[0] for e in prof.events() if "snapkv_" in e.name and "kernel" in e.name]
+
     got, want = pool.clone(), pool.clone()
-    paged_press.snapkv_compress_paged(want, tables, lens_d, max(lens), queries, 0.2, window_size=W, host_lens=lens, rows_only=True)
-    called = []
-    for name in ("snapkv_press", "snapkv_select", "snapkv_score"):
-        def spy(*args, _call=getattr(ops, name), _name=name, **kwargs):
-            called.append((_name, kwargs.get("splits")))
-            return _call(*args, **kwargs)
-        monkeypatch.setattr(ops, name, spy)
+    served, plain = [], paged_press._press_rows
+    with monkeypatch.context() as m:
+        m.setattr(paged_press, "_press_rows", lambda *a, **k: served.append(plain(*a, **k)) or served[-1])
+        native = scoring(lambda: press(want))
+    assert served == [True]
+    called, fn = [], ops.fn
+    monkeypatch.setattr(ops, "fn", lambda name: called.append(name) or fn(name))
     monkeypatch.setattr(paged_press, "_press_rows", lambda *a, **k: False)
-    paged_press.snapkv_compress_paged(got, tables, lens_d, max(lens), queries, 0.2, window_size=W, host_lens=lens, rows_only=True)
-    kview = _lib.paged_view(got[0], tables, lens_d, max(lens))
-    route = _lib.fn("fc_snapkv_rows_route")(ctypes.byref(kview), hq, W, 1, sum(lens) // B)
-    assert called == [("snapkv_press", None) if route == 0 else ("snapkv_select", route)]
+    general = scoring(lambda: press(got))
+    entries = {"fc_snapkv_press", "fc_snapkv_press_ordered", "fc_snapkv_select", "fc_snapkv_select_once", "fc_snapkv_score"}
+    expected = {"once": "fc_snapkv_select_once", "ranges": "fc_snapkv_select",
+                "whole": "fc_snapkv_press_ordered" if host else "fc_snapkv_press"}[form]
+    assert [c for c in called if c in entries] == [expected]
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for names in (native, general):
+        if names:
+            assert any("snapkv_once_kernel" in n for n in names) == (form == "once")
+            assert any("snapkv_kernel" in n for n in names) == (form != "once")
 
 
 @pytest.mark.parametrize("rows,width", [(1, 1), (9, 7), (64, 1), (13, 5), (64, 4), (64, 12), (96, 8), (97, 8), (90, 40)])
