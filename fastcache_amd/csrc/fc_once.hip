@@ -333,7 +333,7 @@ __global__ __launch_bounds__(SO_THREADS, 2) void snapkv_once_kernel(SoArgs a) {
         m[i] = cb == 0 ? e[cb][i] : fmaxf(m[i], e[cb][i]);
       }
     }
-    const float mx = so_reduce<true>(m, lane);
+    const float mx = fmaxf(so_reduce<true>(m, lane), SO_NEG);   // (all of the chunk's logits may be -inf)
     const int reg = so_reg(fresh(lane)), q = place(reg) + lhalf * 4;
     __builtin_amdgcn_wave_barrier();
     wbuf[wave][q] = mx;

@@ -1070,6 +1070,26 @@ def test_snapkv_select_in_one_pass_of_one_dense_layer(dev):
         assert not bool((diff & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
 
 
+def test_snapkv_select_in_one_pass_of_keys_of_infinite_distance(dev):
+    """A chunk all of whose logits are -inf weighs nothing, as in the sweeps: the rest of the column keeps its probabilities."""
+    B, Hq, H, W, S, ksz, keep = 1, 8, 2, 32, 1400, 5, 500
+    g = torch.Generator().manual_seed(4)
+    k = torch.randn(1, B, H, S, 128, generator=g).to(torch.float16)
+    q = torch.randn(1, B, Hq, W, 128, generator=g).to(torch.float16)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[..., 256:768, 0] = float("-inf")                                  # two chunks of 256 keys, and keys of others
+    k[..., 900:1000, 0] = float("-inf")
+    kd, qd = k.to(dev), q.to(dev)
+    kview = _lib.dense_view(kd)
+    scores = ops.snapkv_score(kview, qd, W, ksz, True, "sum", splits=1).cpu()
+    assert bool(torch.isfinite(scores[..., :S - W]).all())
+    got = ops.snapkv_select(kview, qd, W, ksz, keep, True, "sum", workgroups=0).cpu().long()
+    want = opress.topk_lowest_index(scores, keep)
+    kth = scores.gather(-1, want).min(-1, keepdim=True).values
+    diff = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, got, True) ^ torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, want, True)
+    assert not bool((diff & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+
+
 @pytest.mark.parametrize("lens", [[300, 1500, 64, 900, 900], [40, 2000]])
 def test_snapkv_press_longest_columns_first(dev, lens):
     """Sequence lengths known on the host order the launch's columns; the results are those of the launch as it comes."""
