@@ -82,6 +82,7 @@ SIGNATURES = {
     "fc_snapkv_once_workspace_bytes": (C.c_int64, [_V, _I, _I]),
     "fc_snapkv_select_once": (C.c_int, [_V, _VP, _I, _I, _I, _I, _F, _F, _I, _VP, _VP, _I, _I, _VP, C.c_int64, _VP]),
     "fc_snapkv_press_into": (C.c_int, [_V, _V, _V, _V, _VP, _VP, _I, _I, _I, _I, _F, _F, _I, _VP, _I, _VP, C.c_int64, _VP]),
+    "fc_snapkv_press_into_once": (C.c_int, [_V, _V, _V, _V, _VP, _I, _I, _I, _I, _F, _F, _I, _VP, _I, _VP, C.c_int64, _VP]),
     "fc_snapkv_fill_window": (C.c_int, [_VP, _I, _I, _I, _I, _VP, _I, _I, _VP, _VP]),
     "fc_topk_select": (C.c_int, [_VP, _I, _I, _I, _VP, _I, _I, _I, _VP, _VP, _I, _VP]),
     "fc_compact": (C.c_int, [_V, _V, _V, _V, _VP, _I, _I, _I, _VP, _VP]),

@@ -339,17 +339,22 @@ PyObject* py_snapkv_into(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     at::Tensor ok = at::empty({B, H, n, D}, k.options()), ov = at::empty({B, H, n, D}, k.options());
     const fc_kv_view kv = dense_view(k, 1, 0), vv = dense_view(v, 1, 0), dk = dense_view(ok, 1, 0), dv = dense_view(ov, 1, 0);
-    const int32_t nsplit = fc_snapkv_select_splits(&kv, (int32_t)hq, (int32_t)W);
-    const int64_t bytes = !lse && fc_snapkv_once_pays(&kv, (int32_t)hq, (int32_t)W, (int32_t)S)
-                              ? std::max(fc_snapkv_once_workspace_bytes(&kv, (int32_t)hq, (int32_t)W), B * H * S * 4)
-                              : fc_snapkv_select_workspace_bytes(1, (int32_t)B, (int32_t)hq, (int32_t)H, (int32_t)W, (int32_t)S, nsplit);
+    const bool once = !lse && fc_snapkv_once_pays(&kv, (int32_t)hq, (int32_t)W, (int32_t)S);
+    const int32_t nsplit = once ? 0 : fc_snapkv_select_splits(&kv, (int32_t)hq, (int32_t)W);
+    const int64_t bytes = once ? fc_snapkv_once_workspace_bytes(&kv, (int32_t)hq, (int32_t)W)
+                               : fc_snapkv_select_workspace_bytes(1, (int32_t)B, (int32_t)hq, (int32_t)H, (int32_t)W, (int32_t)S, nsplit);
     at::Tensor ws = at::empty({bytes}, k.options().dtype(at::kByte));
     const at::Tensor idx = gather_apart(k, n);
-    check(fc_snapkv_press_into(&kv, &vv, &dk, &dv, q.const_data_ptr(), lse, (int32_t)hq, (int32_t)W, (int32_t)ksz,
-                               (int32_t)causal, (float)scale, (float)out_scale, (int32_t)n,
-                               idx.defined() ? idx.data_ptr<int32_t>() : nullptr, nsplit, ws.data_ptr(), bytes,
-                               stream_of(k)),
-          "fc_snapkv_press_into");
+    int32_t* apart = idx.defined() ? idx.data_ptr<int32_t>() : nullptr;
+    if (once)
+      check(fc_snapkv_press_into_once(&kv, &vv, &dk, &dv, q.const_data_ptr(), (int32_t)hq, (int32_t)W, (int32_t)ksz, (int32_t)causal,
+                                      (float)scale, (float)out_scale, (int32_t)n, apart, 0, ws.data_ptr(), bytes, stream_of(k)),
+            "fc_snapkv_press_into_once");
+    else
+      check(fc_snapkv_press_into(&kv, &vv, &dk, &dv, q.const_data_ptr(), lse, (int32_t)hq, (int32_t)W, (int32_t)ksz,
+                                 (int32_t)causal, (float)scale, (float)out_scale, (int32_t)n, apart, nsplit, ws.data_ptr(), bytes,
+                                 stream_of(k)),
+            "fc_snapkv_press_into");
     return pair(std::move(ok), std::move(ov));
   });
 }

@@ -1088,6 +1088,22 @@ extern "C" int64_t fc_snapkv_once_workspace_bytes(const fc_kv_view* keys, int32_
          fc_once_workspace_bytes(keys->num_layers, keys->batch, num_q_heads, keys->num_kv_heads, window, keys->max_seq_len);
 }
 
+// What follows the sums or scores of a column: its selection, and the gather where no indices are asked for
+static ColumnSelect sk_column(const fc_kv_view* keys, int32_t window, int32_t kernel_size, float out_scale, int32_t k,
+                              const int32_t* n_kept, int32_t* indices, int32_t index_stride) {
+  ColumnSelect a{};
+  a.stride = keys->max_seq_len;
+  a.k = k;
+  a.n_kept = n_kept;
+  a.window = window;
+  a.ksz = kernel_size;
+  a.out_mul = out_scale / (float)kernel_size;
+  a.indices = indices;
+  a.index_stride = index_stride;
+  a.parts = indices ? 0 : fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, keys->max_seq_len, k);
+  return a;
+}
+
 // Every logit formed once (fc_once.hip), then the selection.  The views are checked, a.k, a.n_kept and a.index_stride as well.
 static int snapkv_once_impl(const char* who, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
                             const fc_kv_view* out_v, const void* queries, int32_t num_q_heads, int32_t window,
@@ -1129,22 +1145,13 @@ extern "C" int fc_snapkv_select_once(const fc_kv_view* keys, const void* queries
   FC_REQUIRE(n_kept || (k > window && k <= index_stride), FC_EINVAL, "%s: k=%d must exceed the window (%d) and fit %d", who, k,
              window, index_stride);
   if (keys->max_seq_len == 0) return FC_OK;
-  ColumnSelect a{};
-  a.stride = keys->max_seq_len;
-  a.k = k;
-  a.n_kept = n_kept;
-  a.window = window;
-  a.ksz = kernel_size;
-  a.out_mul = out_scale / (float)kernel_size;
-  a.indices = indices;
-  a.index_stride = index_stride;
+  const ColumnSelect a = sk_column(keys, window, kernel_size, out_scale, k, n_kept, indices, index_stride);
   return snapkv_once_impl(who, keys, keys, nullptr, nullptr, queries, num_q_heads, window, kernel_size, causal_window, scale, a,
                           workgroups, workspace, workspace_bytes, stream);
 }
 
 // Scores every column (split over nsplit workgroups, or whole with nsplit 1) into the workspace, then selects: the
-// window and the k - window best of the other keys.  A hook (out_k given) whose workspace has the room takes one pass over the
-// keys where that is faster.
+// window and the k - window best of the other keys.
 static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
                               const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
                               int32_t window, int32_t kernel_size, int32_t causal_window, float scale, float out_scale,
@@ -1157,20 +1164,7 @@ static int snapkv_select_impl(const char* who, const fc_kv_view* keys, const fc_
              window, index_stride);
   FC_REQUIRE(index_stride <= stride && stride <= FC_SELECT_MAX_KEYS, FC_EUNSUPPORTED,
              "%s: index_stride %d, max_seq_len %d (at most %d)", who, index_stride, stride, FC_SELECT_MAX_KEYS);
-  ColumnSelect a{};
-  a.stride = stride;
-  a.k = k;
-  a.n_kept = n_kept;
-  a.window = window;
-  a.ksz = kernel_size;
-  a.out_mul = out_scale / (float)kernel_size;
-  a.indices = indices;
-  a.index_stride = index_stride;
-  a.parts = out_k && !indices ? fc_gather_parts((long long)keys->num_layers * keys->batch * keys->num_kv_heads, keys->max_seq_len, k) : 0;
-  if (out_k && !lse && num_q_heads > 0 && num_q_heads % keys->num_kv_heads == 0 && fc_once_pays(keys, num_q_heads, window, stride, k, false) &&
-      workspace_bytes >= fc_snapkv_once_workspace_bytes(keys, num_q_heads, window))
-    return snapkv_once_impl(who, keys, values, out_k, out_v, queries, num_q_heads, window, kernel_size, causal_window, scale, a, 0,
-                            workspace, workspace_bytes, stream);
+  ColumnSelect a = sk_column(keys, window, kernel_size, out_scale, k, n_kept, indices, index_stride);
   if (nsplit > 1) {
     const float* raw = nullptr;
     if ((rc = snapkv_split_sums(who, keys, queries, lse, num_q_heads, window, kernel_size, causal_window, scale, stride,
@@ -1199,12 +1193,9 @@ extern "C" int fc_snapkv_select(const fc_kv_view* keys, const void* queries, con
                             scale, out_scale, k, n_kept, indices, index_stride, nsplit, workspace, workspace_bytes, stream);
 }
 
-extern "C" int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
-                                    const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
-                                    int32_t window, int32_t kernel_size, int32_t causal_window, float scale,
-                                    float out_scale, int32_t k, int32_t* indices, int32_t nsplit, void* workspace,
-                                    int64_t workspace_bytes, void* stream) {
-  const char* who = "fc_snapkv_press_into";
+// what both forms of a hook check of their views
+static int sk_into_check(const char* who, const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                         const fc_kv_view* out_v, int32_t k) {
   int rc;
   for (const fc_kv_view* v : {keys, values, out_k, out_v})
     if ((rc = fc_check_view(v, who))) return rc;
@@ -1215,8 +1206,35 @@ extern "C" int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* va
   FC_REQUIRE(keys->max_seq_len == values->max_seq_len && k <= keys->max_seq_len && k <= out_k->max_seq_len &&
                  k <= out_v->max_seq_len,
              FC_EINVAL, "%s: k=%d exceeds a view's max_seq_len", who, k);
+  return FC_OK;
+}
+
+extern "C" int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                                    const fc_kv_view* out_v, const void* queries, const float* lse, int32_t num_q_heads,
+                                    int32_t window, int32_t kernel_size, int32_t causal_window, float scale,
+                                    float out_scale, int32_t k, int32_t* indices, int32_t nsplit, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
+  const char* who = "fc_snapkv_press_into";
+  int rc = sk_into_check(who, keys, values, out_k, out_v, k);
+  if (rc) return rc;
   rc = snapkv_select_impl(who, keys, values, out_k, out_v, queries, lse, num_q_heads, window, kernel_size, causal_window,
                           scale, out_scale, k, nullptr, indices, k, nsplit, workspace, workspace_bytes, stream);
+  return rc || !indices ? rc : fc_compact(keys, values, out_k, out_v, indices, k, keys->num_kv_heads, k, nullptr, stream);
+}
+
+extern "C" int fc_snapkv_press_into_once(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                                         const fc_kv_view* out_v, const void* queries, int32_t num_q_heads, int32_t window,
+                                         int32_t kernel_size, int32_t causal_window, float scale, float out_scale, int32_t k,
+                                         int32_t* indices, int32_t workgroups, void* workspace, int64_t workspace_bytes,
+                                         void* stream) {
+  const char* who = "fc_snapkv_press_into_once";
+  int rc = sk_into_check(who, keys, values, out_k, out_v, k);
+  if (rc) return rc;
+  FC_REQUIRE(k > window, FC_EINVAL, "%s: k=%d must exceed the window (%d)", who, k, window);
+  if (keys->max_seq_len == 0) return FC_OK;
+  const ColumnSelect a = sk_column(keys, window, kernel_size, out_scale, k, nullptr, indices, k);
+  rc = snapkv_once_impl(who, keys, values, out_k, out_v, queries, num_q_heads, window, kernel_size, causal_window, scale, a,
+                        workgroups, workspace, workspace_bytes, stream);
   return rc || !indices ? rc : fc_compact(keys, values, out_k, out_v, indices, k, keys->num_kv_heads, k, nullptr, stream);
 }
 

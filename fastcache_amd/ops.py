@@ -286,7 +286,7 @@ def snapkv_rows_once_pays(keys: FcKvView, num_q_heads: int, window: int, mean_le
 def _select_once(keys, queries, kernel_size, k, causal_window, scale, out_scale, n_kept, workgroups):
     L, B, Hq, W, _ = queries.shape
     nbytes = int(fn("fc_snapkv_once_workspace_bytes")(C.byref(keys), Hq, W))
-    ws = torch.empty(max(nbytes, 0), dtype=torch.uint8, device=queries.device)
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=queries.device)      # (-1: refused by the call, with the reason)
     idx = torch.empty((L, B, keys.num_kv_heads, k), dtype=torch.int32, device=queries.device)
     check(fn("fc_snapkv_select_once")(C.byref(keys), queries.data_ptr(), Hq, W, kernel_size, int(causal_window), scale, out_scale, k,
                                       ptr(n_kept), idx.data_ptr(), k, workgroups, ws.data_ptr(), nbytes, current_stream()),
@@ -301,8 +301,8 @@ def snapkv_select(keys: FcKvView, queries: torch.Tensor, window: int, kernel_siz
                   workgroups: Optional[int] = None) -> torch.Tensor:
     """The indices ``snapkv_score`` + ``topk_select`` give for counts above the window, without a score tensor:
     int32 ``[L, B, Hkv, k]`` (entries past a row's count ``n_kept[b]`` are left as they are).  ``splits``: key ranges per
-    column; default :func:`snapkv_select_splits`.  With ``mean_len`` (the sequences' mean length) one pass over the keys is
-    taken instead where it pays, with ``workgroups`` (at most so many, 0 for the usual number) in any case."""
+    column; default :func:`snapkv_select_splits`, or with ``mean_len`` (the sequences' mean length) one pass over the keys where
+    that pays.  ``workgroups`` asks for the one pass (by at most so many workgroups, 0 for the usual number) in any case."""
     queries = queries.contiguous()
     _lib.require_gpu(queries, "queries")
     L, B, Hq, W, D = queries.shape
@@ -320,9 +320,9 @@ def snapkv_select(keys: FcKvView, queries: torch.Tensor, window: int, kernel_siz
             raise FastcacheError(f"lse must be fp32 [L={L}, B={B}, Hq={Hq}, W={W}], got {lse.dtype} {tuple(lse.shape)}")
         lse = lse.contiguous()
     n_kept = _i32(n_kept, "n_kept", dev)
-    if workgroups is not None or (mean_len is not None and lse is None and snapkv_once_pays(keys, Hq, W, mean_len)):
-        if lse is not None:
-            raise FastcacheError("one pass over the keys forms the log-sum-exp itself")
+    if workgroups is not None and (lse is not None or splits is not None):
+        raise FastcacheError("one pass over the keys forms the log-sum-exp itself and has no key ranges")
+    if workgroups is not None or (mean_len is not None and lse is None and splits is None and snapkv_once_pays(keys, Hq, W, mean_len)):
         return _select_once(keys, queries, kernel_size, k, causal_window, 1.0 / math.sqrt(D) if scale is None else scale,
                             1.0 / (W * (Hq // H)) if reduction == "mean" else 1.0, n_kept, workgroups or 0)
     nsplit = snapkv_select_splits(keys, Hq, W) if splits is None else splits

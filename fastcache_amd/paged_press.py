@@ -164,7 +164,7 @@ def snapkv_compress_paged(kv_cache: torch.Tensor, block_tables: torch.Tensor, se
     if once or route > 0:
         n_kept = None if len(set(kept)) == 1 and len(set(lens)) == 1 else _lib.upload_ints(kept, kv_cache)
         idx = ops.snapkv_select(kview, queries, window_size, kernel_size, width, causal_window, reduction, n_kept=n_kept,
-                                splits=None if once else route, workgroups=0 if once else None)
+                                **({"workgroups": 0} if once else {"splits": route}))
         ops.compact(kview, vview, kview, vview, idx, n_kept=n_kept)
         return None
     scores = ops.snapkv_score(kview, queries, window_size, kernel_size, causal_window, reduction,

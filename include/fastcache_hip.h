@@ -231,8 +231,8 @@ int fc_snapkv_select(const fc_kv_view* keys, const void* queries, const float* l
  * up to 12 288 tokens and up to 16 blocks of 32 window queries per kv head.  fc_snapkv_once_pays: 1 where that is faster than
  * the two sweeps in key ranges, for sequences of that mean length; fc_snapkv_rows_once_pays: where a press of which only the
  * moved rows are wanted and at most `kept` tokens of a sequence stay is faster by it than by `route` (fc_snapkv_rows_route);
- * workspace: fc_snapkv_once_workspace_bytes, -1 where the shape is not taken.  workgroups: at most so many, 0 for two per compute unit.  fc_snapkv_press_into does it by itself
- * where it pays and its workspace has that room. */
+ * workspace: fc_snapkv_once_workspace_bytes, -1 where the shape is not taken.  workgroups: at most so many, 0 for two per
+ * compute unit.  fc_snapkv_press_into_once is fc_snapkv_press_into by it, with the same workspace. */
 int32_t fc_snapkv_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len);
 int32_t fc_snapkv_rows_once_pays(const fc_kv_view* keys, int32_t num_q_heads, int32_t window, int32_t mean_len, int32_t kept,
                                  int32_t route);
@@ -246,6 +246,10 @@ int fc_snapkv_press_into(const fc_kv_view* keys, const fc_kv_view* values, const
                          int32_t window, int32_t kernel_size, int32_t causal_window, float scale, float out_scale,
                          int32_t k, int32_t* indices, int32_t nsplit, void* workspace, int64_t workspace_bytes,
                          void* stream);
+int fc_snapkv_press_into_once(const fc_kv_view* keys, const fc_kv_view* values, const fc_kv_view* out_k,
+                              const fc_kv_view* out_v, const void* queries, int32_t num_q_heads, int32_t window,
+                              int32_t kernel_size, int32_t causal_window, float scale, float out_scale, int32_t k,
+                              int32_t* indices, int32_t workgroups, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * Sets the window entries scores[l][b][h][S_b-W .. S_b) to the maximum over

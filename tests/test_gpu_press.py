@@ -1,4 +1,6 @@
 """GPU parity: Knorm scoring, top-k selection and in-place paged compaction vs the CPU oracle."""
+import ctypes
+
 import pytest
 import torch
 
@@ -855,8 +857,9 @@ def test_layer_hooks_in_one_call(dev, dtype, B, H, S):
 @pytest.mark.parametrize("Hq,H,W", [(8, 2, 64), (14, 2, 64), (7, 1, 32), (4, 4, 32)])     # 8, 14, 7 and 1 blocks of queries
 @pytest.mark.parametrize("S", [129, 191, 192, 193, 320, 449, 1100])
 def test_snapkv_hook_of_one_tile_a_range(dev, Hq, H, W, S):
-    """Short columns cut down to single tiles of 64 keys, the last one of one key, of all, or of window keys only: the
-    selection is that of the scores of whole columns but for keys near the threshold (other partial sums), window kept."""
+    """Short columns cut down to single tiles of 64 keys, the last one of one key, of all, or of window keys only, and the same
+    hooks as ``SnapKVPress`` serves them (most in one pass over the keys): the selection is that of the scores of whole columns
+    but for keys near the threshold (other partial sums), window kept."""
     keep, ksz = W + (S - W) // 3, 5
     g = torch.Generator().manual_seed(S + Hq)
     k = torch.randn(1, H, S, 128, generator=g).to(torch.float16)
@@ -864,18 +867,37 @@ def test_snapkv_hook_of_one_tile_a_range(dev, Hq, H, W, S):
     pos = torch.arange(S)
     v[..., 0], v[..., 1] = (pos % 256).to(v.dtype), (pos // 256).to(v.dtype)
     kd, vd, q = k.to(dev), v.to(dev), torch.randn(1, Hq, W, 128, generator=g).to(torch.float16).to(dev)
-    assert S < 200 or ops.snapkv_select_splits(_lib.dense_view(kd), Hq, W) > 1
-    press = SnapKVPress(1.0 - (keep + 0.5) / S, window_size=W, kernel_size=ksz)
-    ok, ov = (t.cpu() for t in press.compress(None, torch.zeros(1, S, 1), kd, vd, None, {"queries": q}))
-    idx = ov[..., 0].long() + 256 * ov[..., 1].long()
-    assert torch.equal(ok, opress.gather_tokens(k, idx)) and bool((idx[..., 1:] > idx[..., :-1]).all())
-    assert bool((idx[..., -W:] == pos[-W:]).all())
+    splits = ops.snapkv_select_splits(_lib.dense_view(kd), Hq, W)
+    assert S < 200 or splits > 1
+    views = [_lib.dense_view(x) for x in (kd, vd)]
+    room = _lib.fn("fc_snapkv_select_workspace_bytes")(1, 1, Hq, H, W, S, splits)
+
+    def ranges(nbytes):      # the sweeps whatever the workspace could hold
+        out = [torch.empty(1, H, keep, 128, dtype=k.dtype, device=dev) for _ in range(2)]
+        outs = [_lib.dense_view(x) for x in out]
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        _lib.check(_lib.fn("fc_snapkv_press_into")(*(ctypes.byref(x) for x in views + outs), q.data_ptr(), None, Hq, W, ksz, 1, 128 ** -0.5, 1.0 / W,
+                                                   keep, None, splits, ws.data_ptr(), nbytes, _lib.current_stream()), "fc_snapkv_press_into")
+        return [x.cpu() for x in out]
+
+    def press(_):            # what the rule picks
+        hook = SnapKVPress(1.0 - (keep + 0.5) / S, window_size=W, kernel_size=ksz)
+        return [x.cpu() for x in hook.compress(None, torch.zeros(1, S, 1), kd, vd, None, {"queries": q})]
+
     scores = ops.snapkv_score(_lib.dense_view(kd), q[None], W, ksz, splits=1)[0].cpu()
     want = opress.topk_lowest_index(scores, keep)
     kth = scores.gather(-1, want).min(-1, keepdim=True).values
-    got = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, idx, True)
-    ref = torch.zeros_like(got).scatter_(-1, want, True)
-    assert not bool(((got ^ ref) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+    ref = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, want, True)
+    for form, nbytes in ((ranges, room), (ranges, room + (8 << 20)), (press, 0)):
+        ok, ov = form(nbytes)
+        idx = ov[..., 0].long() + 256 * ov[..., 1].long()
+        assert torch.equal(ok, opress.gather_tokens(k, idx)) and bool((idx[..., 1:] > idx[..., :-1]).all())
+        assert bool((idx[..., -W:] == pos[-W:]).all())
+        got = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, idx, True)
+        assert not bool(((got ^ ref) & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+        if form is ranges:
+            swept = idx if nbytes == room else swept
+            assert torch.equal(idx, swept)
 
 
 @pytest.mark.parametrize("S", [500, 1000, 2000, 4096, 8000, 8681, 12320, 16000, 20000])     # one of each selection size
@@ -1088,6 +1110,19 @@ def test_snapkv_select_in_one_pass_of_keys_of_infinite_distance(dev):
     kth = scores.gather(-1, want).min(-1, keepdim=True).values
     diff = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, got, True) ^ torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, want, True)
     assert not bool((diff & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+
+
+def test_snapkv_select_says_what_the_one_pass_takes(dev):
+    """Asked for by its number of workgroups: shapes beyond it and arguments of the other form are refused by what is wrong."""
+    k, q = torch.zeros(1, 1, 1, 12289, 128, dtype=torch.float16, device=dev), torch.zeros(1, 1, 4, 32, 128, dtype=torch.float16, device=dev)
+    kview = _lib.dense_view(k)
+    with pytest.raises(_lib.FastcacheError, match="at most 12288 tokens"):
+        ops.snapkv_select(kview, q, 32, 5, 100, workgroups=0)
+    kview = _lib.dense_view(k[:, :, :, :1000])
+    with pytest.raises(_lib.FastcacheError, match="key ranges"):
+        ops.snapkv_select(kview, q, 32, 5, 100, workgroups=0, splits=2)
+    with pytest.raises(_lib.FastcacheError, match="log-sum-exp"):
+        ops.snapkv_select(kview, q, 32, 5, 100, workgroups=0, lse=torch.zeros(1, 1, 4, 32, device=dev))
 
 
 @pytest.mark.parametrize("lens", [[300, 1500, 64, 900, 900], [40, 2000]])
