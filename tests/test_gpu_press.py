@@ -1076,9 +1076,13 @@ def test_snapkv_select_in_one_pass(dev, Hq, H, W, causal, dtype, large):
             assert not bool((diff & ((sc - kth).abs() > 2e-4 * kth.abs())).any()), (b, l)
 
 
-def test_snapkv_select_in_one_pass_of_one_dense_layer(dev):
-    """The same from a dense layer, whose every column has the view's length, against the sweeps' selection."""
-    B, Hq, H, W, S, keep = 3, 8, 2, 64, 2049, 700
+@pytest.mark.parametrize("B,Hq,H,W,S", [(3, 8, 2, 64, 2049),
+                                         (2, 28, 4, 64, 8193), (1, 4, 4, 32, 12288),      # looks at more than 32 chunks
+                                         (80, 8, 2, 64, 4300), (160, 8, 2, 64, 1900)])    # many turns: one list, two
+def test_snapkv_select_in_one_pass_of_one_dense_layer(dev, B, Hq, H, W, S):
+    """The same from a dense layer, whose every column has the view's length, against the sweeps' selection: chunks shared out
+    over every number of lists."""
+    keep = S // 3
     g = torch.Generator(device=dev).manual_seed(1)
     k = torch.randn(1, B, H, S, 128, generator=g, device=dev).to(torch.bfloat16)
     q = torch.randn(1, B, Hq, W, 128, generator=g, device=dev).to(torch.bfloat16)
@@ -1086,10 +1090,36 @@ def test_snapkv_select_in_one_pass_of_one_dense_layer(dev):
     scores = ops.snapkv_score(kview, q, W, 7, True, "sum", splits=1).cpu()
     want = opress.topk_lowest_index(scores, keep)
     kth = scores.gather(-1, want).min(-1, keepdim=True).values
-    for n in (0, 1):
-        got = ops.snapkv_select(kview, q, W, 7, keep, True, "sum", workgroups=n).cpu().long()
-        diff = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, got, True) ^ torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, want, True)
-        assert not bool((diff & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+    out = [ops.snapkv_select(kview, q, W, 7, keep, True, "sum", workgroups=n).cpu().long() for n in (0, 1, 33)]
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    diff = torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, out[0], True) ^ torch.zeros_like(scores, dtype=torch.bool).scatter_(-1, want, True)
+    assert not bool((diff & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
+
+
+@pytest.mark.parametrize("Hq,H,W", [(4, 2, 32), (8, 2, 64), (14, 2, 64)])       # 2, 8 and 14 blocks
+@pytest.mark.parametrize("S", [4097, 8192, 8193, 9216, 12288])
+@pytest.mark.parametrize("dtype,large", [(torch.bfloat16, 1), (torch.float16, 4)])      # (four times as large: with offsets)
+def test_snapkv_select_in_one_pass_of_long_columns(dev, Hq, H, W, S, dtype, large):
+    """Up to 48 chunks of 256 keys, beyond 32 in a second round of looks, among short sequences: what the oracle's scores keep,
+    up to keys at the threshold, and the same whatever number of workgroups runs."""
+    ksz = 5
+    lens = [300, S, W + ksz + 1, S - 255]
+    keep = [max(n // 3, W + 1) for n in lens]
+    case = synth.make_paged_case(seed=S + W, num_layers=1, batch=len(lens), num_kv_heads=H, seq_lens=lens, dtype=dtype,
+                                 num_q_heads=Hq, window=W, keep_dense=True)
+    pool, q = (case.kv_cache * large).to(dev), case.queries * large
+    kview = _lib.paged_view(pool[0], case.table_tensor(dev), case.lens_tensor(dev), S)
+    n_kept = torch.tensor(keep, dtype=torch.int32, device=dev)
+    out = [ops.snapkv_select(kview, q.to(dev), W, ksz, max(keep), True, "sum", n_kept=n_kept, workgroups=n).cpu().long()
+           for n in (0, 1, 9)]
+    for b, (n, kk) in enumerate(zip(lens, keep)):
+        got = out[0][0, b, :, :kk]
+        assert all(torch.equal(o[0, b, :, :kk], got) for o in out[1:])
+        sc = opress.snapkv_score(q[0, b:b + 1], case.dense_k[0, b:b + 1, :, :n] * large, W, ksz, True, "sum")[0]
+        want = opress.topk_lowest_index(sc, kk)
+        kth = sc.gather(-1, want).min(-1, keepdim=True).values
+        diff = torch.zeros_like(sc, dtype=torch.bool).scatter_(-1, got, True) ^ torch.zeros_like(sc, dtype=torch.bool).scatter_(-1, want, True)
+        assert not bool((diff & ((sc - kth).abs() > 2e-4 * kth.abs())).any()), b
 
 
 def test_snapkv_select_in_one_pass_of_keys_of_infinite_distance(dev):
