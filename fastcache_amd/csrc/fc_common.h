@@ -246,13 +246,9 @@ __device__ __forceinline__ void fc_load_lds(const char* g_uniform, unsigned lane
                "s"(g_uniform)
                : "memory", "m0");
 }
-// The same two for bytes that nothing reads again before the caches have turned over: non-temporal, so that the stream
+// The second one for bytes that nothing reads again before the caches have turned over: non-temporal, so that the stream
 // takes no room in the L2.  What another workgroup reads too, or what the next launch finds in the memory-side cache
 // (256 MB), is fetched again at a cost: the callers say where that line lies.
-__device__ __forceinline__ void fc_load_lds_once(const char* g, unsigned lds_base) {
-  lds_base = __builtin_amdgcn_readfirstlane(lds_base);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds_base), "v"(g) : "memory", "m0");
-}
 __device__ __forceinline__ void fc_load_lds_once(const char* g_uniform, unsigned lane_off, unsigned lds_base) {
   lds_base = __builtin_amdgcn_readfirstlane(lds_base);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(lane_off),

@@ -77,7 +77,9 @@ __global__ __launch_bounds__(CP_THREADS) void compact_kernel(KvView sk, KvView s
   };
   // Non-temporal for large planes whose tokens are 4 KB or more: there a SnapKV press of a pool, compaction included, takes
   // 1032 us instead of 1063 (2 x 3000 tokens, 32 layers of 32 bf16 heads) and a Knorm press 253 instead of 279 (1 x 3000, 36
-  // layers of 8 fp32 heads); with tokens of 1 KB 729 instead of 721 (9 x 2000, 28 layers of 4 bf16 heads).
+  // layers of 8 fp32 heads); with tokens of 1 KB 729 instead of 721 (9 x 2000, 28 layers of 4 bf16 heads), 403 and 407 (1 x 9000);
+  // of 2 KB, 36 layers of 8 bf16 heads, 604 and 615 (2 x 7000), 1890 and 1911 (2 x 16 000), 1697 and 1700 (1 x 30 011, a fifth
+  // kept): 0 to 2 % of passes whose compaction is a launch of its own, not taken.
   if (src.num_kv_heads * FC_HEAD_DIM * EB >= CP_ONCE_TOKEN && cp_once(src, EB, lens)) walk(std::true_type{});
   else walk(std::false_type{});
 }

@@ -664,10 +664,10 @@ bool fc_once_takes(const fc_kv_view* keys, int32_t num_q_heads, int32_t window) 
 //  (no), of 4096 27.2 -> 23.7.  28 on 4, window 64 (14 blocks): 4 columns of 400 25.4 -> 18.4, of 4096 39.6 -> 24.7; 16 of 2000
 //  33.5 -> 26.2.  More than SO_HOOK_KEYS keys in all keep the sweeps, faster or not (32 of 4096 47.5 -> 41.8): the two forms' sums
 //  differ by their fp32 roundings, and two keys that all but tie at the threshold are then ranked the other way, which moves the
-//  rows between them (26 of 12 800 columns of 4096 keys, 6 of 8000 of 2000: one in two million keys; against 64 bits the sweeps are
-//  off in 25 and 6, one pass in 23 and 0).  Within the bound one call in 60 returns other rows than the sweeps do: hooks of more
-//  keys, where it would be one in 15 and more, return what they did before there was one pass.  This is a line drawn for
-//  unchanged results, not for time or precision.
+//  rows between them (26 of 12 800 columns of 4096 keys, 4 of 8000 of 2000, one in two to four million keys; against 64 bits
+//  the sweeps are off in 25 and 6, one pass in 23 and 6).  Within the bound one call in 60 to 100 returns other rows than the
+//  sweeps do; hooks of more keys, where it would be one in 15 and more, return what they did before there was one pass.  This
+//  is a line drawn for unchanged results, not for time or precision.
 //
 // Everything else is a paged pass (selection in a launch of its own and compaction), against what fc_snapkv_rows_route says:
 // key ranges, followed by the same launches, or (whole) one launch per column, which moves a column's kept rows while others
