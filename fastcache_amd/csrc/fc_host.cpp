@@ -817,7 +817,7 @@ PyObject* py_press_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int32_t *counts = nullptr, *order = nullptr;
     at::Tensor numbers;      // kept until the launches are enqueued
     if (args[5] != Py_None) {
-      const bool ordered = args[6] != Py_None;
+      const bool ordered = args[6] != Py_None && one;      // (the one launch's columns start in that order)
       if (!PyList_Check(args[5]) || PyList_GET_SIZE(args[5]) != B || (ordered && (!PyList_Check(args[6]) || PyList_GET_SIZE(args[6]) != B)))
         fail("press_rows: one count per sequence expected");
       Packed pk((ordered ? 2 : 1) * B * 4, pool.device());

@@ -1142,6 +1142,30 @@ def test_snapkv_select_in_one_pass_of_keys_of_infinite_distance(dev):
     assert not bool((diff & ((scores - kth).abs() > 2e-4 * kth.abs())).any())
 
 
+@pytest.mark.parametrize("B,Hq,H,W,S", [(1, 8, 2, 64, 1100), (2, 14, 2, 64, 700), (3, 8, 2, 32, 500)])      # one pass, one pass, the sweeps
+def test_snapkv_hook_in_a_captured_graph(dev, B, Hq, H, W, S):
+    """A hook's launches, recorded once and replayed on other inputs between eager calls: every replay keeps what the eager call
+    keeps (the one pass sets up its lists and sums anew every time)."""
+    press = SnapKVPress(0.5, window_size=W, kernel_size=5)
+    g = torch.Generator(device=dev).manual_seed(3)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device=dev).to(torch.bfloat16)
+    k, v, q = draw(B, H, S, 128), draw(B, H, S, 128), draw(B, Hq, W, 128)
+    hidden = torch.zeros(B, S, 1)
+    press.compress(None, hidden, k, v, None, {"queries": q})
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = press.compress(None, hidden, k, v, None, {"queries": q})
+    for _ in range(4):
+        for x in (k, v, q):
+            x.copy_(draw(*x.shape))
+        graph.replay()
+        eager = press.compress(None, hidden, k, v, None, {"queries": q})
+        torch.cuda.synchronize()
+        for a, b in zip(held, eager):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 def test_snapkv_select_says_what_the_one_pass_takes(dev):
     """Asked for by its number of workgroups: shapes beyond it and arguments of the other form are refused by what is wrong."""
     k, q = torch.zeros(1, 1, 1, 12289, 128, dtype=torch.float16, device=dev), torch.zeros(1, 1, 4, 32, 128, dtype=torch.float16, device=dev)
