@@ -241,7 +241,7 @@ __global__ __launch_bounds__(DA_THREADS, 2) void decode_attn_kernel(KvView kc, K
   // Where this workgroup alone reads its columns' bytes, the loads leave no line in the L2.  Workgroups that share a group of
   // heads find the bytes there (4 layers of 16 x 4096..8192, 128/4 heads, 591 -> 715 with such loads), and so do those of
   // sequences that share a prefix: a range whose first page another table names loads plainly.  us a pass, 16 captured bf16
-  // layers, plain loads / such loads whatever is shared / as here: 90 x 128..2048 tokens, 32/32 heads, 4611 / 4218 / 4171, 56 x
+  // layers on the same caches step after step, plain loads / such loads whatever is shared / as here: 90 x 128..2048 tokens, 32/32 heads, 4611 / 4218 / 4171, 56 x
   // 156..1565, 32/8, 965 / 923 / 877, 90 x 200..1400, 28/4, 912 / 853 / 782; 48 x 1300..1500 in groups of eight with the first
   // 1280 in common, 32/32, 1647 / 2429 / 1613, 16 x 4096 with 3840, 32/8, 829 / 943 / 824, 90 x 1500 with 512, 32/32, 4643 / 5012 /
   // 3755; where one head a group reads little else, 16 x 2048 with 1792, 1088 / 1269 / 1200.  (Asked for behind the first two
