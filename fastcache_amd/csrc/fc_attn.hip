@@ -587,6 +587,7 @@ __global__ __launch_bounds__(FC_HEAD_DIM) void decode_merge_kernel(const float* 
 // of the wavefronts is shorter than a merge.  us a layer, 16 captured layers of columns of 270 to 375 tokens, merged -> alone:
 // 4 columns 9.5 -> 8.1 to 8.7, 48 10.9 -> 8.9 to 9.6; of 400 9.5 -> 9.4, of 500 10.0 -> 10.6.
 #define DC_ALONE 128
+#define DC_ONCE_BYTES (16ll << 20)                                 // K and V; 16 layers of it are what the memory-side cache holds
 #define DC_STAGES 2                                                // V tiles of a wavefront in LDS or on their way
 #define DC_MERGE 8                                                // partial rows in flight per thread of the merge
 #define DC_PART (DC_WAVES * DC_STAGES * DA_TILEB)                   // V stages, then the partial outputs
@@ -733,11 +734,13 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   // with the row number, so that the transposed reads of 16 rows at one place meet all banks.
   // Of groups of up to 4 heads whole tiles leave no line in the L2 (us a pass, 16 captured bf16 layers, plain -> so: 32/8 heads, 4 x
   // 4000 tokens 339 -> 322, the first 3840 in common 256 -> 250, 24 x 700..768, 512 in common, 267 -> 250, 1 x 8000 282 -> 275, 32/32,
-  // 1 x 8000 505 -> 478, 8/8, 8 x 2048 306 -> 306; 0.94 to 0.98 times as fast where nothing but a cache of less than 256 MB is read from
-  // one step to the next).  Larger groups gain less and read a shared prefix from there: 28/4, 16 x 3900..4096 545 -> 513, but
-  // with 3840 in common 340 -> 367, 12 x 1800..2000 with 1792 231 -> 238, so they load plainly; asking the tables first costs the
-  // launch its start (28 eager layers of 3 x 300..900 305 plain, 297 so, 313 asked).  K stays: an instruction takes 64 bytes of a
-  // row, the rest of the line would be fetched again (16 x 3280, 28/4, 464 -> 480, 32 x 1000..4000 700 -> 778).
+  // 1 x 8000 486 -> 462, 8/8, 4 x 1000 198.5 -> 197.5), where the batch may hold DC_ONCE_BYTES a layer.  Less stays in the
+  // memory-side cache from step to step: 32/8, 1 x 300 147 -> 157, 1 x 1000 175 -> 183, 32/32, 1 x 300 155 -> 159.  Larger groups
+  // gain less and read a shared prefix from there: 28/4, 16 x 3900..4096 545 -> 513, but with 3840 in common 340 -> 367, 12 x
+  // 1800..2000 with 1792 231 -> 238, so they load plainly; asking the tables first costs the launch its start (28 eager layers of 3
+  // x 300..900 305 plain, 297 so, 313 asked).  K stays: an instruction takes 64 bytes of a row, the rest of the line would be
+  // fetched again (16 x 3280, 28/4, 464 -> 480, 32 x 1000..4000 700 -> 778).
+  const bool once = TERMS == 3 && (long long)gridDim.y * kc.max_seq_len * kc.num_kv_heads * (4 * FC_HEAD_DIM) >= DC_ONCE_BYTES;
   const unsigned v_lds = __builtin_amdgcn_readfirstlane(fc_lds_addr(smem) + wave * DC_STAGES * DA_TILEB);
   unsigned vlane[4];
 #pragma unroll
@@ -745,7 +748,7 @@ __global__ __launch_bounds__(DC_THREADS, 2) void decode_column_kernel(KvView kc,
   auto load_v = [&](int stage, int tile) {
     const int s0 = t0 + tile * DA_TILE, rmax = end - 1 - s0;
     const char* vg = tile_base(vc, vbase, s0, vtbl);
-    if (TERMS == 3 && rmax >= DA_TILE - 1) {
+    if (once && rmax >= DA_TILE - 1) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) fc_load_lds_once(vg + u * 4 * (unsigned long long)vtok, vlane[u & 3], v_lds + stage * DA_TILEB + u * 1024);
     } else if (rmax >= DA_TILE - 1) {
